@@ -129,10 +129,12 @@ def draw(rng):
   limit = 5e12 if case["dtype"] == "bfloat16" else 3e11
   while work(case)["flops"] > limit:
     step = case.get("group", 1)
-    smaller = case["images"] // 2 // step * step
-    if smaller < step:
-      case["experts"] = max(4, case["experts"] // 2)
-    case["images"] = max(step, smaller)
+    if case["images"] > step:
+      case["images"] = max(step, case["images"] // 2 // step * step)
+    elif step > 1:
+      case["images"] = case["group"] = step // 2
+    else:
+      case["tokens" if "tokens" in case else "layers"] //= 2
   return case
 
 
