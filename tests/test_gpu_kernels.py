@@ -811,6 +811,48 @@ def test_expert_mlp_rows_per_expert(K, dtype, E):
     assert (to_np(out[e, n:]) == 7.0).all()
 
 
+@pytest.mark.parametrize("E,R,D,M", [
+    (5, 65, 1024, 512),      # one row past a 64-row tile; 32 x 32 and 32 x 64 tiles
+    (24, 130, 384, 512),     # 32 x 128 and 64 x 64 tiles
+    (16, 257, 320, 640),     # 128 x 64 tiles, one row past the second; columns end inside a tile
+    (12, 400, 512, 768),     # 64 x 128 and 128 x 128 tiles
+    (8, 52, 96, 3072),       # long k over few rows, k not a multiple of 64 in the first product
+    (3, 33, 136, 264),       # k that ends inside a 32-wide step
+    (70, 3, 64, 200),        # more experts than rows, one short row tile each
+])
+def test_expert_mlp_small_tiles(K, E, R, D, M):
+  """bfloat16 products over few rows per expert (the small tiles, chosen by size) against a float32
+  restatement with the same rounding points; ragged rows bit for bit against the dense call,
+  nothing written past a count, and rows gathered from the items bit for bit as well."""
+  rng = np.random.default_rng(E * 1000 + R)
+  bf = torch.bfloat16
+  mk = lambda scale, *s: to_dev(O.cast(rng.standard_normal(s).astype(np.float32) * scale, O.BF16), O.BF16)
+  T = R + 7
+  items, w0, b0 = mk(1, T, D), mk(D ** -0.5, E, D, M), mk(0.1, E, M)
+  w1, b1 = mk(M ** -0.5, E, M, D), mk(0.1, E, D)
+  x_rows = torch.from_numpy(rng.integers(0, T, (E, R)).astype(np.int32)).to(dev())
+  x = items[x_rows.long()]
+  dense = K.expert_mlp(x, w0, b0, w1, b1)
+  for e in range(E):
+    h = ((x[e].float() @ w0[e].float()).to(bf).float() + b0[e].float()).to(bf)
+    h = torch.nn.functional.gelu(h.float(), approximate="tanh").to(bf)
+    y = ((h.float() @ w1[e].float()).to(bf).float() + b1[e].float()).to(bf)
+    np.testing.assert_allclose(to_np(dense[e]), to_np(y), rtol=2e-2, atol=2e-2, err_msg=f"expert {e}")
+  rows = rng.integers(0, R + 1, E).astype(np.int32)
+  rows[:3] = [R, 0, 1]
+  bad = x_rows.clone()
+  for e, n in enumerate(rows):
+    bad[e, n:] = 2 ** 30                                  # never followed
+  ragged, gathered = torch.full_like(dense, 7.0), torch.full_like(dense, 7.0)
+  K.expert_mlp(x, w0, b0, w1, b1, out=ragged, rows_per_expert=to_dev(rows))
+  for e, n in enumerate(rows):
+    assert torch.equal(ragged[e, :n], dense[e, :n]), f"expert {e}"
+    assert (to_np(ragged[e, n:]) == 7.0).all(), f"expert {e} wrote past its rows"
+  if K.expert_mlp_can_gather(bf, D, T):
+    K.expert_mlp(items, w0, b0, w1, b1, out=gathered, rows_per_expert=to_dev(rows), x_rows=bad)
+    assert torch.equal(gathered, ragged)
+
+
 def test_expert_mlp_planned_launch_random_fill(K):
   """bf16 expert products over packed rows with a die-balanced launch plan: random row
   counts (empty, one row, tile boundaries, full), expert counts below and above the

@@ -8,6 +8,7 @@
 
 #include "gemm_bf16_wide.h"
 #include "gemm_bf16_w8.h"
+#include "gemm_bf16_rows.h"
 #include "gemm_f32.h"
 #include "compact_rows.h"
 
@@ -306,7 +307,7 @@ static_assert(kStatusWords * sizeof(int32_t) <= kStatusBytes, "status block");
 //  kDownHalf: 128 x 256 tiles, two per CU (static launches the tile-walking kernels do not
 //    cover, where whole rounds of 256 x 256 tiles would waste a tenth or more).
 //  kDownPlain: 256 x 256 tiles, one workgroup per tile.
-enum DownKernel { kDownShared, kDownEightWaves, kDownNarrow, kDownWide, kDownHalf, kDownPlain };
+enum DownKernel { kDownShared, kDownEightWaves, kDownNarrow, kDownWide, kDownHalf, kDownPlain, kDownForced };
 using CfgDownNarrow = W8Cfg<6>;
 
 bool down_prefers_half_tiles(int E, int R, int N) {
@@ -321,6 +322,7 @@ bool down_prefers_half_tiles(int E, int R, int N) {
 
 // Launch plans of the two ragged products of an MLP: geometry, bytes, one planning launch.
 struct MlpPlans {
+  int up_rows = -1, down_rows = -1;      // tile of gemm_bf16_rows_kernel (kRowsTiles), -1: not taken
   GemmGeom up, down;
   DownKernel down_kernel = kDownPlain;
   int down_bm = CfgDown::BM;
@@ -328,7 +330,8 @@ struct MlpPlans {
   size_t streamk_bytes = 0;              // exchange memory of kDownShared
 };
 
-MlpPlans mlp_plans(int E, int R, int D, int M, bool ragged) {
+// (`items`: rows of the matrix of items that the first product gathers from, 0 if it does not.)
+MlpPlans mlp_plans(int E, int R, int D, int M, bool ragged, long long items) {
   MlpPlans m;
   m.up = gemm_geometry<CfgUp>(E, R, M, D);
   // Ragged launches are planned whenever the geometry allows: with whole experts per
@@ -351,44 +354,65 @@ MlpPlans mlp_plans(int E, int R, int D, int M, bool ragged) {
       E, R, D, M, rows, bytes(square) ? planned : nullptr) && M / CfgDownPersistent::BK % kStreamKGranule == 0;
   const bool wide_ok = wide_gemm_ok(E, R, D, M, nullptr, nullptr, nullptr, 0) && (!ragged || bytes(wide));
   constexpr double kNumCu = kCusPerXcd * kNumXcd;
-  // Time in units of one 256 x 256 tile of the four-wave kernel on one CU, fitted to alternating
-  // bench runs of the layer configurations (B/16 layer, Soft MoE layer, L/16 layer at capacity
-  // 0.5, B/16 model): the shared kernel pays for its tiles (the padding of the last row tile
-  // of a batch included) plus the exchange; the eight-wave kernel runs whole rounds at 0.95
-  // per tile (two waves per SIMD, 16 x 16 x 32 MFMAs); its 192-column form whole rounds of
-  // tiles three quarters the size at 0.97 of the time per flop, taken only where it wins by
-  // 3 % (Soft MoE: 512 tiles = 2 rounds instead of 1.5 shared ones, 417 -> 397 us for the
-  // MLP; the B/16 model's 13 rounds against 10: 0.2 ms slower); the wide kernel's tile is 1.5
-  // of them at 1.04 of the time per flop, in whole rounds.
+  // Microseconds of the large-tile kernels, fitted to alternating bench runs of the layer
+  // configurations (B/16 layer, Soft MoE layer, L/16 layer at capacity 0.5, B/16 model) in units
+  // of one 256 x 256 tile of the four-wave kernel on one CU: the eight-wave kernel runs whole
+  // rounds at 0.95 per tile (two waves per SIMD, 16 x 16 x 32 MFMAs); its 192-column form whole
+  // rounds of tiles three quarters the size at 0.97 of the time per flop, taken only where it wins
+  // by 3 % (Soft MoE: 512 tiles = 2 rounds, 417 -> 397 us for the MLP; the B/16 model's 13 rounds
+  // against 10: 0.2 ms slower); the wide kernel's tile is 1.5 of them at 1.04 of the time per
+  // flop, in whole rounds; the shared kernel pays for its tiles at 1.12 (32x32x16 MFMAs) and
+  // 60 us for the chain of sums through memory (50 - 75 us whatever the size: 196 rows of one
+  // expert took 80 us).
+  const double unit = 0.025 * M;
   const GemmGeom narrow = gemm_geometry<CfgDownNarrow>(E, R, D, M);
   const bool eight_ok = w8_gemm_ok<8>(E, R, D, M, rows, bytes(square) ? planned : nullptr);
   const bool narrow_ok = w8_gemm_ok<6>(E, R, D, M, rows, bytes(narrow) ? planned : nullptr);
-  const double t_wide = 1.5 * 1.04 * std::ceil((double)wide.tiles / kNumCu);
-  // the shared form balances a partial round but runs 32x32x16 MFMAs and exchanges sums: on the
-  // L/16 half-capacity layer (0.8 tiles per CU) it measures 2 % behind eight waves
-  const double t_shared = 1.12 * (double)square.tiles / kNumCu + 0.1;
-  const double t_eight = 0.95 * std::ceil((double)square.tiles / kNumCu);
-  const double t_narrow = 0.75 * 0.97 * std::ceil((double)narrow.tiles / kNumCu);
-  double t_best = 1e300;
-  m.down_kernel = !ragged && down_prefers_half_tiles(E, R, D) ? kDownHalf : kDownPlain;
+  const double t_wide = unit * 1.5 * 1.04 * std::ceil((double)wide.tiles / kNumCu);
+  const double t_shared = unit * 1.12 * (double)square.tiles / kNumCu + 60;
+  const double t_eight = unit * 0.95 * std::ceil((double)square.tiles / kNumCu);
+  const double t_narrow = unit * 0.75 * 0.97 * std::ceil((double)narrow.tiles / kNumCu);
+  const bool half = !ragged && down_prefers_half_tiles(E, R, D);
+  m.down_kernel = half ? kDownHalf : kDownPlain;
+  double t_best = 1e30;
   if (wide_ok) { m.down_kernel = kDownWide; t_best = t_wide; }
   if (shared_ok && t_shared <= t_best) { m.down_kernel = kDownShared; t_best = t_shared; }
   if (eight_ok && t_eight <= t_best) { m.down_kernel = kDownEightWaves; t_best = t_eight; }
   if (narrow_ok && t_narrow < 0.97 * t_best) { m.down_kernel = kDownNarrow; t_best = t_narrow; }
+  // Few rows: the small tiles of gemm_bf16_rows.h where their estimate is below that of the large
+  // ones (shapes that only the register-staged kernel would take always).
+  double rows_us = 0;
+  if (rows_gemm_ok(R, M, D, items)) {
+    const int tile = best_rows_tile(E, R, M, D, &rows_us);
+    if (!m.up.fast || rows_us < product_us(kFirstProductTile, E, R, M, D)) m.up_rows = tile;
+  }
+  if (rows_gemm_ok(R, D, M, 0)) {
+    const int tile = best_rows_tile(E, R, D, M, &rows_us);
+    if (t_best > 1e29 && square.fast)
+      t_best = unit * (half ? 0.5 * 1.05 * std::ceil((double)E * ((R + 127) / 128) * ((D + 255) / 256) / kNumCu)
+                            : std::ceil((double)square.tiles / kNumCu));
+    if (rows_us < 5 + t_best) m.down_rows = tile;
+  }
   // (VMOE_SECOND_PRODUCT=shared|eight|narrow|wide in the environment overrides the choice
   // where the named kernel applies: the switch behind the figures that the model above was
   // fitted to)
   if (const char* force = getenv("VMOE_SECOND_PRODUCT")) {
+    const DownKernel chosen = m.down_kernel;
+    m.down_kernel = kDownForced;
     if (strcmp(force, "shared") == 0 && shared_ok) m.down_kernel = kDownShared;
     if (strcmp(force, "eight") == 0 && eight_ok) m.down_kernel = kDownEightWaves;
     if (strcmp(force, "narrow") == 0 && narrow_ok) m.down_kernel = kDownNarrow;
     if (strcmp(force, "wide") == 0 && wide_ok) m.down_kernel = kDownWide;
+    if (m.down_kernel == kDownForced) m.down_kernel = chosen;
+    else m.down_rows = -1;
   }
   m.down = m.down_kernel == kDownWide ? wide : m.down_kernel == kDownNarrow ? narrow : square;
   m.down_bm = m.down_kernel == kDownWide ? WideCfg::BM : CfgDown::BM;
   static_assert(CfgDownNarrow::BM == CfgDown::BM, "row tiles of the narrow kernel");
   m.down_bytes = bytes(m.down);
-  if (m.down_kernel == kDownShared)
+  if (m.up_rows >= 0) m.up_bytes = 0;
+  if (m.down_rows >= 0) m.down_bytes = 0;
+  if (m.down_kernel == kDownShared && m.down_rows < 0)
     m.streamk_bytes = align256(StreamKWorkspace<CfgDownPersistent>::kBytes);
   return m;
 }
@@ -432,7 +456,8 @@ extern "C" size_t vmoe_expert_mlp_workspace_bytes(const VmoeExpertMlpParams* p) 
   const size_t b = p->dtype == VMOE_BF16 ? 2 : 4;
   size_t bytes = align256((size_t)p->E * p->R * p->M * b);  // hidden activations
   if (p->dtype == VMOE_BF16) {   // status words, launch plans of the ragged products, stream-K exchange
-    const MlpPlans m = mlp_plans(p->E, p->R, p->D, p->M, p->rows_per_expert != nullptr);
+    const MlpPlans m = mlp_plans(p->E, p->R, p->D, p->M, p->rows_per_expert != nullptr,
+                                  p->x_rows != nullptr ? p->num_items : 0);
     bytes += kStatusBytes + m.up_bytes + m.down_bytes + m.streamk_bytes;
   }
   if (p->dtype == VMOE_BF16) {
@@ -464,7 +489,8 @@ MlpWorkspace mlp_workspace(const VmoeExpertMlpParams* p) {
   if (p->dtype == VMOE_BF16) {
     w.status = reinterpret_cast<int32_t*>(ws);
     ws += kStatusBytes;
-    w.m = mlp_plans(p->E, p->R, p->D, p->M, p->rows_per_expert != nullptr);
+    w.m = mlp_plans(p->E, p->R, p->D, p->M, p->rows_per_expert != nullptr,
+                                  p->x_rows != nullptr ? p->num_items : 0);
     if (w.m.up_bytes) w.plan_up = reinterpret_cast<int4*>(ws);
     ws += w.m.up_bytes;
     if (w.m.down_bytes) w.plan_down = reinterpret_cast<int4*>(ws);
@@ -529,7 +555,15 @@ static int run_expert_mlp(const VmoeExpertMlpParams* p, vmoe_stream_t stream_, b
     int32_t* status = w.status;
     static_assert(std::is_same<CfgUp, GemmCfg<128, 256, 2, 2, 32, 3, 2>>::value,
                   "launch_gemm_bf16_first runs CfgUp's geometry");
-    if (tanh_gelu)
+    // A call that plans one product only: the other one checks that plan as well (guard).
+    const PlanRef no_plan{nullptr, 0, 0};
+    if (m.up_rows >= 0) {
+      auto up = tanh_gelu ? launch_gemm_bf16_rows<kEpiBiasGeluTanh> : launch_gemm_bf16_rows<kEpiBiasGeluErf>;
+      rc = up(m.up_rows, (const bf16_t*)p->x, (const bf16_t*)w0t, (const bf16_t*)p->b0, (bf16_t*)hidden,
+              p->E, p->R, p->M, p->D, stream, p->rows_per_expert, p->x_rows, p->num_items,
+              plan_down != nullptr ? plan_ref_of(m.down, plan_down, m.down_bm, p->E, p->R) : no_plan,
+              clear, SK::kFlags, status);
+    } else if (tanh_gelu)
       rc = launch_gemm_bf16_first<kEpiBiasGeluTanh>((const bf16_t*)p->x, (const bf16_t*)w0t,
                                                     (const bf16_t*)p->b0, (bf16_t*)hidden, p->E,
                                                     p->R, p->M, p->D, stream, p->rows_per_expert,
@@ -540,6 +574,11 @@ static int run_expert_mlp(const VmoeExpertMlpParams* p, vmoe_stream_t stream_, b
                                                    p->R, p->M, p->D, stream, p->rows_per_expert,
                                                    plan_up, p->x_rows, p->num_items, clear, SK::kFlags, status);
     if (rc != VMOE_OK) return rc;
+    if (m.down_rows >= 0)
+      return launch_gemm_bf16_rows<kEpiBias>(
+          m.down_rows, (const bf16_t*)hidden, (const bf16_t*)w1t, (const bf16_t*)p->b1, (bf16_t*)p->out,
+          p->E, p->R, p->D, p->M, stream, p->rows_per_expert, nullptr, 0,
+          plan_up != nullptr ? plan_ref_of(m.up, plan_up, CfgUp::BM, p->E, p->R) : no_plan, nullptr, 0, status);
     switch (m.down_kernel) {
       case kDownShared:
         return launch_gemm_bf16_persistent<CfgDownPersistent, kEpiBias>(

@@ -1690,11 +1690,14 @@ GemmGeom gemm_geometry(int batch, int R, int N, int Kd) {
 
 // The plan of a launch with geometry g as its kernel takes it (tag: what the planner wrote
 // for the same geometry, batch count and rows per batch).
-template <typename Cfg>
-PlanRef plan_ref(const GemmGeom& g, const int4* plan, int batch, int R) {
+inline PlanRef plan_ref_of(const GemmGeom& g, const int4* plan, int bm, int batch, int R) {
   if (plan == nullptr) return PlanRef{nullptr, 0, 0};
   const int blocks = (int)(g.ragged_slots * kNumXcd);
-  return PlanRef{plan, blocks, plan_tag(Cfg::BM, g.tiles_n, g.panel_rows, blocks, batch, R)};
+  return PlanRef{plan, blocks, plan_tag(bm, g.tiles_n, g.panel_rows, blocks, batch, R)};
+}
+template <typename Cfg>
+PlanRef plan_ref(const GemmGeom& g, const int4* plan, int batch, int R) {
+  return plan_ref_of(g, plan, Cfg::BM, batch, R);
 }
 
 // `plan`, if given, was filled by plan_ragged_tiles_kernel for this product's geometry.
