@@ -7,13 +7,17 @@ PyTorch is used for device memory and streams only.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 from ctypes import c_float, c_int32, c_size_t, c_void_p
 
 import torch
 
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "libvmoe_hip.so")
+_HOST_PATH = os.path.join(os.path.dirname(_LIB_PATH), "_vmoe_host.so")
 _lib = None
+_host = None
 
 F32, BF16 = 0, 1
 GELU_TANH, GELU_ERF = 0, 1
@@ -57,6 +61,21 @@ def lib() -> ctypes.CDLL:
   return _lib
 
 
+def host():
+  """The native host side (csrc/host.cpp), failing loudly if it has not been built."""
+  global _host
+  if _host is None:
+    lib()
+    if not os.path.exists(_HOST_PATH):
+      raise VmoeError(f"{_HOST_PATH} is missing: build it with `python -m vmoe_amd.csrc.build`.")
+    loader = importlib.machinery.ExtensionFileLoader("_vmoe_host", _HOST_PATH)
+    mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_vmoe_host", loader))
+    loader.exec_module(mod)
+    mod.set_error(VmoeError)
+    _host = mod
+  return _host
+
+
 def check(code: int, what: str) -> None:
   if code != 0:
     msg = lib().vmoe_error_string(code).decode()
@@ -81,8 +100,16 @@ def ptr(t) -> c_void_p:
   return c_void_p(t.data_ptr())
 
 
+_raw_stream, _current_device = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
+
+
+def raw_stream() -> int:
+  """torch.cuda.current_stream().cuda_stream, without the Stream object around it (3 us)."""
+  return _raw_stream(_current_device())
+
+
 def stream() -> c_void_p:
-  return c_void_p(torch.cuda.current_stream().cuda_stream)
+  return c_void_p(raw_stream())
 
 
 class GateTopkParams(ctypes.Structure):
@@ -249,6 +276,13 @@ def set_timing_sink(sink) -> None:
   ``sink[name]`` for the caller to read after synchronising.  None disables."""
   global _timing_sink
   _timing_sink = sink
+
+
+def timed(name: str) -> bool:
+  """Whether a timing sink wants entry point ``name`` bracketed: its wrapper then makes the
+  call from Python (call and call_blocks); otherwise it goes through the native host side."""
+  only = getattr(_timing_sink, "only", None)
+  return _timing_sink is not None and (only is None or name in only)
 
 
 def call2(name: str, first: ctypes.Structure, second: ctypes.Structure) -> None:

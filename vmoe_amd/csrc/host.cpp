@@ -1,0 +1,352 @@
+// Host side of the layers: the same calls of the C ABI that vmoe_amd/kernels.py makes through
+// ctypes, as functions on torch tensors that allocate their results and fill the parameter blocks
+// natively.
+//
+// Why.  A small call is as long as its host work: the sparse layer on one image spends 60 us in
+// kernels, and its twenty allocations, forty pointer checks and seven parameter blocks cost 150 us
+// of Python (3 us for torch.cuda.current_stream alone, five times a layer).  Here an entry point
+// costs its allocations (0.7 us each) and its launch.
+//
+// Every function takes the raw stream first and raises vmoe_amd._hip.VmoeError on an error code, a
+// tensor that is not on the GPU or one that is not contiguous.  Nothing is kept between calls.
+#include <torch/extension.h>
+
+#include <optional>
+#include <string>
+#include <tuple>
+
+#include "vmoe_hip.h"
+
+namespace {
+
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+
+PyObject* vmoe_error = nullptr;      // vmoe_amd._hip.VmoeError
+
+[[noreturn]] void raise_error(const std::string& text) {
+  PyErr_SetString(vmoe_error != nullptr ? vmoe_error : PyExc_RuntimeError, text.c_str());
+  throw py::error_already_set();
+}
+
+void check(int code, const char* what) {
+  if (code != VMOE_OK)
+    raise_error(std::string(what) + " failed: " + vmoe_error_string(code) + " (code " + std::to_string(code) + ")");
+}
+
+void* ptr(const Tensor& t) {
+  if (!t.is_cuda()) raise_error("tensor is not on a ROCm device; there is no CPU fallback");
+  if (!t.is_contiguous()) raise_error("tensor must be contiguous");
+  return t.data_ptr();
+}
+void* ptr(const OptTensor& t) { return t.has_value() ? ptr(*t) : nullptr; }
+template <typename T> T* ptr_as(const Tensor& t) { return static_cast<T*>(ptr(t)); }
+template <typename T> T* ptr_as(const OptTensor& t) { return static_cast<T*>(ptr(t)); }
+
+vmoe_stream_t stream_of(int64_t raw) { return reinterpret_cast<vmoe_stream_t>(raw); }
+
+int dtype_code(at::ScalarType t) {
+  if (t == at::kFloat) return VMOE_F32;
+  if (t == at::kBFloat16) return VMOE_BF16;
+  PyErr_SetString(PyExc_TypeError, "Unsupported dtype; the kernels cover float32 and bfloat16.");
+  throw py::error_already_set();
+}
+int dtype_code(const Tensor& t) { return dtype_code(t.scalar_type()); }
+
+Tensor empty(at::IntArrayRef sizes, at::ScalarType type, const Tensor& like) {
+  return at::empty(sizes, like.options().dtype(type).requires_grad(false));
+}
+Tensor i32(at::IntArrayRef sizes, const Tensor& like) { return empty(sizes, at::kInt, like); }
+Tensor f32(at::IntArrayRef sizes, const Tensor& like) { return empty(sizes, at::kFloat, like); }
+
+Tensor as_f32(const Tensor& t) {     // .to(float32).contiguous() of the wrappers
+  return t.scalar_type() == at::kFloat && t.is_contiguous() ? t : t.to(at::kFloat).contiguous();
+}
+
+Tensor cast(int64_t stream, const Tensor& x_, at::ScalarType type) {
+  if (x_.scalar_type() == type) return x_;
+  const Tensor x = x_.contiguous();
+  Tensor out = empty(x.sizes(), type, x);
+  if (x.numel() > 0) {
+    VmoeCastParams p{ptr(x), ptr(out), (size_t)x.numel(), dtype_code(x), dtype_code(type)};
+    check(vmoe_cast(&p, stream_of(stream)), "vmoe_cast");
+  }
+  return out;
+}
+
+std::tuple<OptTensor, Tensor, Tensor, OptTensor> gate_topk(
+    int64_t stream, const Tensor& x_, const Tensor& w_, int64_t k, const OptTensor& bias_, bool want_gates,
+    bool want_logits) {
+  const Tensor x = x_.contiguous(), w = w_.to(x_.scalar_type()).contiguous();
+  const int64_t G = x.size(0), S = x.size(1), D = x.size(2), E = w.size(1);
+  OptTensor bias = bias_;
+  if (bias.has_value()) bias = as_f32(*bias);
+  OptTensor gates, logits;
+  if (want_gates) gates = empty({G, S, E}, x.scalar_type(), x);
+  if (want_logits) logits = f32({G, S, E}, x);
+  Tensor val = f32({G, S, k}, x), idx = i32({G, S, k}, x);
+  VmoeGateTopkParams p{};
+  p.x = ptr(x); p.w = ptr(w); p.logit_bias = ptr_as<float>(bias); p.gates = ptr(gates);
+  p.topk_val = ptr_as<float>(val); p.topk_idx = ptr_as<int32_t>(idx);
+  p.num_items = (int32_t)(G * S); p.D = (int32_t)D; p.E = (int32_t)E; p.K = (int32_t)k;
+  p.dtype = dtype_code(x); p.logits = ptr_as<float>(logits);
+  check(vmoe_gate_topk(&p, stream_of(stream)), "vmoe_gate_topk");
+  return {gates, val, idx, logits};
+}
+
+// -> indices, token_slot, slot_token, fill and, with gates, the three losses of the router.
+std::tuple<Tensor, Tensor, Tensor, Tensor, OptTensor, OptTensor, OptTensor> route_assign(
+    int64_t stream, const OptTensor& val_, const Tensor& idx_, int64_t E, int64_t C, bool batch_priority,
+    const OptTensor& gates_, double w_gshard, double w_importance) {
+  const Tensor idx = idx_.contiguous();
+  OptTensor val = val_, gates = gates_;
+  if (val.has_value()) val = as_f32(*val);
+  const int64_t G = idx.size(0), S = idx.size(1), K = idx.size(2);
+  Tensor indices = i32({G, S, K, 2}, idx), token_slot = i32({G, S, K}, idx);
+  Tensor slot_token = i32({E * G * C}, idx), fill = i32({G, E}, idx);
+  VmoeRouteAssignParams p{};
+  p.topk_val = ptr_as<float>(val); p.topk_idx = ptr_as<int32_t>(idx); p.indices = ptr_as<int32_t>(indices);
+  p.token_slot = ptr_as<int32_t>(token_slot); p.slot_token = ptr_as<int32_t>(slot_token);
+  p.fill = ptr_as<int32_t>(fill);
+  p.G = (int32_t)G; p.S = (int32_t)S; p.E = (int32_t)E; p.K = (int32_t)K; p.C = (int32_t)C;
+  p.batch_priority = batch_priority;
+  OptTensor imp, gsh, aux;
+  if (!gates.has_value()) {
+    check(vmoe_route_assign(&p, stream_of(stream)), "vmoe_route_assign");
+  } else {
+    gates = gates->contiguous();
+    if (gates->dim() != 3 || gates->size(0) != G || gates->size(1) != S || gates->size(2) != E) {
+      PyErr_SetString(PyExc_ValueError, "gates do not have the shape (G, S, num_experts)");
+      throw py::error_already_set();
+    }
+    imp = f32({G}, idx); gsh = f32({G}, idx); aux = f32({G}, idx);
+    VmoeRouterMetricsParams m{};
+    m.gates = ptr(gates); m.top1_idx = ptr_as<int32_t>(idx); m.importance_loss = ptr_as<float>(imp);
+    m.gshard_loss = ptr_as<float>(gsh); m.auxiliary_loss = ptr_as<float>(aux);
+    m.gshard_loss_weight = (float)w_gshard; m.importance_loss_weight = (float)w_importance;
+    m.G = (int32_t)G; m.S = (int32_t)S; m.E = (int32_t)E; m.top1_stride = (int32_t)K; m.dtype = dtype_code(*gates);
+    check(vmoe_route_assign_metrics(&p, &m, stream_of(stream)), "vmoe_route_assign_metrics");
+  }
+  return {indices, token_slot, slot_token, fill, imp, gsh, aux};
+}
+
+// The expert MLP; with `fill` and `token_slot` the packed rows are computed here as well.
+// -> out, workspace, byte offset of the status words in it (-1: none), token_row,
+//    rows_per_expert, row_token, whether the call ran on a plan that the compaction wrote.
+std::tuple<Tensor, Tensor, int64_t, OptTensor, OptTensor, OptTensor, bool> expert_mlp(
+    int64_t stream, const Tensor& x_, const OptTensor& w0, const OptTensor& b0, const OptTensor& w1,
+    const OptTensor& b1, const OptTensor& w0t, const OptTensor& w1t, bool tanh_gelu,
+    const OptTensor& workspace_, const OptTensor& out_, const OptTensor& rows_per_expert,
+    const OptTensor& x_rows, const OptTensor& fill, const OptTensor& token_slot, int64_t capacity,
+    bool plan_apart) {
+  const Tensor x = x_.contiguous();
+  const bool compact = fill.has_value();
+  VmoeCompactRowsParams c{};
+  OptTensor token_row, rows = rows_per_expert, row_token = x_rows;
+  if (compact) {
+    c.G = (int32_t)fill->size(0); c.E = (int32_t)fill->size(1); c.C = (int32_t)capacity;
+    c.S = (int32_t)token_slot->size(1); c.K = (int32_t)token_slot->size(2);
+    token_row = i32({c.G, c.S, c.K}, *fill);
+    rows = i32({c.E}, *fill);
+    row_token = i32({c.E, c.G * capacity}, *fill);
+    c.fill = ptr_as<int32_t>(fill); c.token_slot = ptr_as<int32_t>(token_slot);
+    c.token_row = ptr_as<int32_t>(token_row); c.rows_per_expert = ptr_as<int32_t>(rows);
+    c.row_token = ptr_as<int32_t>(row_token);
+  }
+  VmoeExpertMlpParams p{};
+  int64_t E, R, D;
+  if (row_token.has_value()) {
+    E = row_token->size(0); R = row_token->size(1);
+    p.num_items = (int32_t)x.size(0); D = x.size(1);
+  } else {
+    E = x.size(0); R = x.size(1); D = x.size(2);
+  }
+  p.E = (int32_t)E; p.R = (int32_t)R; p.D = (int32_t)D;
+  p.M = (int32_t)(w0.has_value() ? w0->size(2) : w0t->size(1));
+  Tensor out = out_.has_value() ? *out_ : empty({E, R, D}, x.scalar_type(), x);
+  p.x = ptr(x); p.w0 = ptr(w0); p.b0 = ptr(b0); p.w1 = ptr(w1); p.b1 = ptr(b1); p.w0t = ptr(w0t); p.w1t = ptr(w1t);
+  p.out = ptr(out); p.dtype = dtype_code(x); p.gelu = tanh_gelu ? VMOE_GELU_TANH : VMOE_GELU_ERF;
+  p.rows_per_expert = ptr_as<int32_t>(rows); p.x_rows = ptr_as<int32_t>(row_token);
+  const size_t need = vmoe_expert_mlp_workspace_bytes(&p);
+  Tensor workspace = workspace_.has_value() && workspace_->nbytes() >= need
+                         ? *workspace_ : empty({(int64_t)need}, at::kByte, x);
+  p.workspace = ptr(workspace);
+  p.workspace_bytes = workspace.nbytes();
+  const int32_t* status = nullptr;
+  check(vmoe_expert_mlp_status(&p, &status), "vmoe_expert_mlp_status");
+  const int64_t status_at = status == nullptr ? -1 : (const char*)status - (const char*)p.workspace;
+  if (compact) {
+    int rc = VMOE_E_UNSUPPORTED;
+    if (p.dtype == VMOE_BF16 && !plan_apart) rc = vmoe_compact_rows_planned(&c, &p, stream_of(stream));
+    if (rc == VMOE_OK) {
+      check(vmoe_expert_mlp_planned(&p, stream_of(stream)), "vmoe_expert_mlp_planned");
+      return {out, workspace, status_at, token_row, rows, row_token, true};
+    }
+    if (rc != VMOE_E_UNSUPPORTED) check(rc, "vmoe_compact_rows_planned");
+    const Tensor prefix = i32({c.G, c.E}, *fill);
+    c.prefix = ptr_as<int32_t>(prefix);
+    check(vmoe_compact_rows(&c, stream_of(stream)), "vmoe_compact_rows");
+  }
+  check(vmoe_expert_mlp(&p, stream_of(stream)), "vmoe_expert_mlp");
+  return {out, workspace, status_at, token_row, rows, row_token, false};
+}
+
+Tensor dispatch(int64_t stream, const Tensor& x_, const Tensor& token_slot, const OptTensor& slot_token,
+                const OptTensor& out_, int64_t num_slots) {
+  const Tensor x = x_.contiguous();
+  const int64_t D = x.size(1);
+  if (slot_token.has_value()) num_slots = slot_token->numel();
+  Tensor out = out_.has_value() ? *out_ : empty({num_slots, D}, x.scalar_type(), x);
+  VmoeDispatchParams p{ptr(x), ptr_as<int32_t>(token_slot), ptr_as<int32_t>(slot_token), ptr(out),
+                       (int32_t)x.size(0), (int32_t)num_slots, (int32_t)token_slot.size(-1), (int32_t)D,
+                       dtype_code(x)};
+  check(vmoe_dispatch(&p, stream_of(stream)), "vmoe_dispatch");
+  return out;
+}
+
+Tensor combine(int64_t stream, const Tensor& y_, const Tensor& token_slot, const Tensor& weights_,
+               const OptTensor& out_) {
+  const Tensor y = y_.contiguous(), weights = as_f32(weights_);
+  const int64_t D = y.size(1), T = token_slot.size(0);
+  Tensor out = out_.has_value() ? *out_ : empty({T, D}, y.scalar_type(), y);
+  VmoeCombineParams p{ptr(y), ptr_as<int32_t>(token_slot), ptr_as<float>(weights), ptr(out), (int32_t)T,
+                      (int32_t)y.size(0), (int32_t)token_slot.size(1), (int32_t)D, dtype_code(y)};
+  check(vmoe_combine(&p, stream_of(stream)), "vmoe_combine");
+  return out;
+}
+
+// -> (x, layer_norm(x)): x the residual itself without a branch.
+std::tuple<Tensor, OptTensor> add_layer_norm(int64_t stream, const Tensor& residual_, const OptTensor& branch_,
+                                             const OptTensor& scale_, const OptTensor& bias_, double eps,
+                                             std::optional<at::ScalarType> out_type, bool write_residual) {
+  const Tensor residual = residual_.contiguous();
+  OptTensor branch = branch_, scale = scale_, bias = bias_, sum, norm;
+  const int64_t D = residual.size(-1);
+  if (branch.has_value()) {
+    if (branch->sizes() != residual.sizes()) {
+      PyErr_SetString(PyExc_ValueError, "branch and residual have different shapes");
+      throw py::error_already_set();
+    }
+    branch = branch->contiguous();
+    if (write_residual) sum = at::empty_like(residual);
+  }
+  if (scale.has_value()) scale = as_f32(*scale);
+  if (bias.has_value()) bias = as_f32(*bias);
+  if (out_type.has_value()) norm = empty(residual.sizes(), *out_type, residual);
+  if (!sum.has_value() && !norm.has_value()) return {residual, norm};
+  VmoeAddLayerNormParams p{ptr_as<float>(residual), ptr(branch), ptr_as<float>(scale), ptr_as<float>(bias),
+                           ptr_as<float>(sum), ptr(norm), (size_t)(residual.numel() / D), (int32_t)D, (float)eps,
+                           branch.has_value() ? dtype_code(*branch) : 0,
+                           out_type.has_value() ? dtype_code(*out_type) : 0};
+  check(vmoe_add_layer_norm(&p, stream_of(stream)), "vmoe_add_layer_norm");
+  return {sum.has_value() ? *sum : residual, norm};
+}
+
+Tensor attention(int64_t stream, const Tensor& q, const Tensor& k, const Tensor& v, double scale) {
+  const int64_t B = q.size(0), Sq = q.size(1), H = q.size(2), hd = q.size(3);
+  for (const Tensor* t : {&q, &k, &v}) {
+    if (!t->is_cuda()) raise_error("tensor is not on a ROCm device; there is no CPU fallback");
+    if (t->stride(3) != 1 || t->stride(2) != hd)
+      raise_error("attention operands need contiguous (H, hd) trailing axes");
+  }
+  Tensor out = empty({B, Sq, H * hd}, q.scalar_type(), q);
+  VmoeAttentionParams p{q.data_ptr(), k.data_ptr(), v.data_ptr(), ptr(out), q.stride(0), q.stride(1), k.stride(0),
+                        k.stride(1), v.stride(0), v.stride(1), (int32_t)B, (int32_t)H, (int32_t)Sq,
+                        (int32_t)k.size(1), (int32_t)hd, (float)scale, dtype_code(q)};
+  check(vmoe_attention(&p, stream_of(stream)), "vmoe_attention");
+  return out;
+}
+
+int w_code(const Tensor& w) {
+  switch (w.scalar_type()) {
+    case at::kFloat: return VMOE_W_F32;
+    case at::kBFloat16: return VMOE_W_BF16;
+    case at::kBool: return VMOE_W_BOOL;
+    default: break;
+  }
+  PyErr_SetString(PyExc_TypeError, "Unsupported weight dtype");
+  throw py::error_already_set();
+}
+
+// Dense dispatch (G, S, E, C) x (G, S, D) -> (E*G*C, D), or combine -> (G, S, D).
+Tensor einsum(int64_t stream, const Tensor& w_, const Tensor& data_, at::ScalarType out_type, bool is_dispatch) {
+  const Tensor w = w_.contiguous(), data = data_.contiguous();
+  const int64_t G = w.size(0), S = w.size(1), E = w.size(2), C = w.size(3), D = data.size(-1);
+  Tensor out = is_dispatch ? empty({E * G * C, D}, out_type, data) : empty({G, S, D}, out_type, data);
+  VmoeEinsumParams p{ptr(w), ptr(data), ptr(out), (int32_t)G, (int32_t)S, (int32_t)E, (int32_t)C, (int32_t)D,
+                     w_code(w), dtype_code(data), dtype_code(out_type)};
+  if (is_dispatch) check(vmoe_einsum_dispatch(&p, stream_of(stream)), "vmoe_einsum_dispatch");
+  else check(vmoe_einsum_combine(&p, stream_of(stream)), "vmoe_einsum_combine");
+  return out;
+}
+
+// -> dispatch weights, combine weights, the (5,) scalars of the weights, the prepared slot
+// parameters (`prepared`, if given, is what an earlier call with the same mu, scale and shapes left).
+std::tuple<Tensor, Tensor, Tensor, Tensor> soft_route_stats(int64_t stream, const Tensor& x_, const Tensor& mu_,
+                                                            double scale, const OptTensor& prepared) {
+  const Tensor x = x_.contiguous(), mu = mu_.to(x_.scalar_type()).contiguous();
+  const int64_t G = x.size(0), S = x.size(1), D = x.size(2), N = mu.size(1);
+  Tensor dw = empty({G, S, N}, x.scalar_type(), x), cw = empty({G, S, N}, x.scalar_type(), x);
+  Tensor buf = f32({G * 4 + 8}, x);
+  VmoeSoftRouteParams p{};
+  p.x = ptr(x); p.mu = ptr(mu); p.scale = (float)scale; p.dispatch_w = ptr(dw); p.combine_w = ptr(cw);
+  p.G = (int32_t)G; p.S = (int32_t)S; p.D = (int32_t)D; p.N = (int32_t)N; p.dtype = dtype_code(x);
+  Tensor ws = prepared.has_value() ? *prepared
+                                   : empty({std::max<int64_t>(16, vmoe_soft_route_workspace_bytes(&p))}, at::kByte, x);
+  p.workspace = ptr(ws); p.workspace_bytes = ws.nbytes(); p.workspace_prepared = prepared.has_value();
+  VmoeSoftStatsParams st{p.combine_w, p.dispatch_w, ptr_as<float>(buf), ptr_as<float>(buf) + G * 4, p.G, p.S, p.N, p.dtype};
+  check(vmoe_soft_route_stats(&p, &st, stream_of(stream)), "vmoe_soft_route_stats");
+  return {dw, cw, buf.slice(0, G * 4, G * 4 + 5), ws};
+}
+
+// -> dy (data) or dweights (weights) of combine.
+Tensor combine_backward_data(int64_t stream, const Tensor& dout_, const Tensor& token_slot, const Tensor& weights_,
+                             const OptTensor& slot_token, int64_t num_slots) {
+  const Tensor dout = dout_.contiguous(), weights = as_f32(weights_);
+  Tensor dy = empty({num_slots, dout.size(1)}, dout.scalar_type(), dout);
+  VmoeCombineBackwardParams p{};
+  p.dout = ptr(dout); p.token_slot = ptr_as<int32_t>(token_slot); p.weights = ptr_as<float>(weights);
+  p.slot_token = ptr_as<int32_t>(slot_token); p.dy = ptr(dy);
+  p.num_items = (int32_t)dout.size(0); p.num_slots = (int32_t)num_slots; p.K = (int32_t)token_slot.size(-1);
+  p.D = (int32_t)dout.size(1); p.dtype = dtype_code(dout);
+  check(vmoe_combine_backward_data(&p, stream_of(stream)), "vmoe_combine_backward_data");
+  return dy;
+}
+
+Tensor combine_backward_weights(int64_t stream, const Tensor& dout_, const Tensor& y_, const Tensor& token_slot) {
+  const Tensor dout = dout_.contiguous(), y = y_.contiguous();
+  Tensor dw = f32({dout.size(0), token_slot.size(-1)}, dout);
+  VmoeCombineBackwardParams p{};
+  p.dout = ptr(dout); p.y = ptr(y); p.token_slot = ptr_as<int32_t>(token_slot); p.dweights = ptr_as<float>(dw);
+  p.num_items = (int32_t)dout.size(0); p.num_slots = (int32_t)y.size(0); p.K = (int32_t)token_slot.size(-1);
+  p.D = (int32_t)dout.size(1); p.dtype = dtype_code(dout);
+  check(vmoe_combine_backward_weights(&p, stream_of(stream)), "vmoe_combine_backward_weights");
+  return dw;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_vmoe_host, m) {
+  m.def("set_error", [](py::object e) { vmoe_error = e.release().ptr(); });
+  m.def("cast", [](int64_t s, const Tensor& x, py::object t) {
+    return cast(s, x, torch::python::detail::py_object_to_dtype(std::move(t)));
+  });
+  m.def("gate_topk", &gate_topk);
+  m.def("route_assign", &route_assign);
+  m.def("expert_mlp", &expert_mlp);
+  m.def("dispatch", &dispatch);
+  m.def("combine", &combine);
+  m.def("add_layer_norm", [](int64_t s, const Tensor& r, const OptTensor& b, const OptTensor& sc, const OptTensor& bi,
+                             double eps, py::object t, bool w) {
+    std::optional<at::ScalarType> type;
+    if (!t.is_none()) type = torch::python::detail::py_object_to_dtype(std::move(t));
+    return add_layer_norm(s, r, b, sc, bi, eps, type, w);
+  });
+  m.def("attention", &attention);
+  m.def("einsum", [](int64_t s, const Tensor& w, const Tensor& d, py::object t, bool dispatch_) {
+    return einsum(s, w, d, torch::python::detail::py_object_to_dtype(std::move(t)), dispatch_);
+  });
+  m.def("soft_route_stats", &soft_route_stats);
+  m.def("combine_backward_data", &combine_backward_data);
+  m.def("combine_backward_weights", &combine_backward_weights);
+}

@@ -2,6 +2,10 @@
 
 Each function maps to one entry point of include/vmoe_hip.h.  Tensors must live
 on a ROCm device and are used as raw device pointers on torch's current stream.
+
+The calls on the layers' paths go through the native host side (csrc/host.cpp), which allocates
+and fills the parameter blocks in C++; the ctypes calls below them are what a timing sink brackets
+(_hip.timed), and what the entry points off those paths use.
 """
 from __future__ import annotations
 
@@ -38,6 +42,10 @@ def gate_topk(x: torch.Tensor, w: torch.Tensor, num_selected_experts: int,
     x = torch.nn.functional.pad(x, (0, pad))
     w = torch.nn.functional.pad(w, (0, 0, 0, pad))
     D += pad
+  if not H.timed("vmoe_gate_topk"):
+    gates, val, idx, logits = H.host().gate_topk(H.raw_stream(), x, w, K, logit_bias, return_gates,
+                                                 return_logits)
+    return (gates, val, idx, logits) if return_logits else (gates, val, idx)
   gates = torch.empty((G, S, E), dtype=x.dtype, device=x.device) if return_gates else None
   val = _f32(G, S, K, device=x.device)
   idx = _i32(G, S, K, device=x.device)
@@ -104,6 +112,10 @@ def route_assign(topk_val: Optional[torch.Tensor], topk_idx: torch.Tensor, num_e
   With ``metrics=(gates (G,S,E), gshard_loss_weight, importance_loss_weight)`` the router's
   losses are computed in the same launch and a fifth result
   ``(importance_loss, gshard_loss, auxiliary_loss)`` is returned (what router_metrics gives)."""
+  if not H.timed("vmoe_route_assign" if metrics is None else "vmoe_route_assign_metrics"):
+    out = H.host().route_assign(H.raw_stream(), topk_val, topk_idx, num_experts, capacity,
+                                bool(batch_priority), *(metrics or (None, 0.0, 0.0)))
+    return out[:4] if metrics is None else out[:4] + (out[4:],)
   G, S, K = topk_idx.shape
   dev = topk_idx.device
   topk_idx = topk_idx.contiguous()
@@ -183,6 +195,8 @@ def dispatch(x: torch.Tensor, token_slot: torch.Tensor, slot_token: Optional[tor
              out: Optional[torch.Tensor] = None, num_slots: Optional[int] = None) -> torch.Tensor:
   """x (T,D), token_slot (T,K), slot_token (NS,) -> (NS, D).  With slot_token None (and
   num_slots given) unclaimed rows are left as allocated instead of zeroed."""
+  if not H.timed("vmoe_dispatch"):
+    return H.host().dispatch(H.raw_stream(), x, token_slot, slot_token, out, num_slots or 0)
   T, D = x.shape
   K = token_slot.shape[-1]
   NS = slot_token.numel() if slot_token is not None else int(num_slots)
@@ -198,6 +212,8 @@ def dispatch(x: torch.Tensor, token_slot: torch.Tensor, slot_token: Optional[tor
 def combine(y: torch.Tensor, token_slot: torch.Tensor, weights: torch.Tensor,
             out: Optional[torch.Tensor] = None) -> torch.Tensor:
   """y (NS,D), token_slot (T,K), weights (T,K) f32 -> (T, D)."""
+  if not H.timed("vmoe_combine"):
+    return H.host().combine(H.raw_stream(), y, token_slot, weights, out)
   NS, D = y.shape
   T, K = token_slot.shape
   y = y.contiguous()
@@ -214,6 +230,9 @@ def combine_backward_data(dout: torch.Tensor, token_slot: torch.Tensor, weights:
                           slot_token: Optional[torch.Tensor], num_slots: int) -> torch.Tensor:
   """dout (T,D) -> dy (NS,D): dy[slot(t,k)] = w[t,k] * dout[t]; unclaimed slots are zero when
   slot_token is given, unwritten otherwise."""
+  if not H.timed("vmoe_combine_backward_data"):
+    return H.host().combine_backward_data(H.raw_stream(), dout, token_slot, weights, slot_token,
+                                          num_slots)
   T, D = dout.shape
   Kk = token_slot.shape[-1]
   dout = dout.contiguous()
@@ -229,6 +248,8 @@ def combine_backward_data(dout: torch.Tensor, token_slot: torch.Tensor, weights:
 def combine_backward_weights(dout: torch.Tensor, y: torch.Tensor,
                              token_slot: torch.Tensor) -> torch.Tensor:
   """dout (T,D), y (NS,D) -> dweights (T,K) f32: <dout[t], y[slot(t,k)]>, 0 where dropped."""
+  if not H.timed("vmoe_combine_backward_weights"):
+    return H.host().combine_backward_weights(H.raw_stream(), dout, y, token_slot)
   T, D = dout.shape
   Kk = token_slot.shape[-1]
   dout, y = dout.contiguous(), y.contiguous()
@@ -274,6 +295,19 @@ def expert_mlp(x: torch.Tensor, w0, b0, w1, b1, w0t=None, w1t=None, approximate_
   With ``compact=(fill (G,E), token_slot (G,S,K), capacity)`` x is the (T,D) matrix of items
   and the packed rows are computed here, in the launch that plans the products (what
   compact_rows gives is returned as well): -> (out, (token_row, rows_per_expert, row_token))."""
+  if H._timing_sink is None or not any(map(H.timed, _MLP_CALLS)):
+    global _last_planned
+    fill, token_slot, capacity = compact or (None, None, 0)
+    out, workspace, at, token_row, rows, row_token, planned = H.host().expert_mlp(
+        H.raw_stream(), x, w0, b0, w1, b1, w0t, w1t, approximate_gelu, workspace, out,
+        rows_per_expert, x_rows, fill, token_slot, capacity,
+        bool(os.environ.get("VMOE_PLAN_SEPARATE_LAUNCH")))
+    _note_status_words(workspace, at)
+    if compact is None:
+      return out
+    if planned:
+      _last_planned = (x, w0, b0, w1, b1, w0t, w1t, approximate_gelu, out, workspace, rows, row_token)
+    return out, (token_row, rows, row_token)
   maps = None
   if compact is not None:
     fill, token_slot, capacity = compact
@@ -283,26 +317,23 @@ def expert_mlp(x: torch.Tensor, w0, b0, w1, b1, w0t=None, w1t=None, approximate_
     rows_per_expert = _i32(E, device=fill.device)
     x_rows = _i32(E, G * capacity, device=fill.device)
     maps = (token_row, rows_per_expert, x_rows)
-  num_items = 0
   if x_rows is not None:
     E, R = x_rows.shape
-    num_items, D = x.shape
+    D = x.shape[1]
   else:
     E, R, D = x.shape
-  M = (w0.shape[2] if w0 is not None else w0t.shape[1])
   x = x.contiguous()
   if out is None:
     out = torch.empty((E, R, D), dtype=x.dtype, device=x.device)
-  p = H.ExpertMlpParams(H.ptr(x), H.ptr(w0), H.ptr(b0), H.ptr(w1), H.ptr(b1), H.ptr(w0t),
-                        H.ptr(w1t), H.ptr(out), None, 0, E, R, D, M, H.dtype_code(x.dtype),
-                        H.GELU_TANH if approximate_gelu else H.GELU_ERF, H.ptr(rows_per_expert),
-                        H.ptr(x_rows), num_items)
+  p = _expert_mlp_params(x, w0, b0, w1, b1, w0t, w1t, approximate_gelu, out, rows_per_expert, x_rows)
   need = H.lib().vmoe_expert_mlp_workspace_bytes(H.ctypes.byref(p))
   if workspace is None or workspace.numel() * workspace.element_size() < need:
     workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
   p.workspace = H.ptr(workspace)
   p.workspace_bytes = workspace.numel() * workspace.element_size()
-  _note_status_words(p, workspace)
+  addr = ctypes.c_void_p()
+  H.check(H.lib().vmoe_expert_mlp_status(ctypes.byref(p), ctypes.byref(addr)), "vmoe_expert_mlp_status")
+  _note_status_words(workspace, addr.value - workspace.data_ptr() if addr.value else -1)
   if compact is None:
     H.call("vmoe_expert_mlp", p)
     return out
@@ -315,8 +346,7 @@ def expert_mlp(x: torch.Tensor, w0, b0, w1, b1, w0t=None, w1t=None, approximate_
     rc = H.call_blocks("vmoe_compact_rows_planned", c, p, accept=(_E_UNSUPPORTED,))
   if rc == 0:
     H.call("vmoe_expert_mlp_planned", p)
-    global _last_planned
-    _last_planned = (p, (x, w0, b0, w1, b1, w0t, w1t, out, workspace) + maps)
+    _last_planned = (x, w0, b0, w1, b1, w0t, w1t, approximate_gelu, out, workspace, maps[1], maps[2])
   else:
     c.prefix = H.ptr(_i32(G, E, device=fill.device))
     H.call("vmoe_compact_rows", c)
@@ -324,34 +354,44 @@ def expert_mlp(x: torch.Tensor, w0, b0, w1, b1, w0t=None, w1t=None, approximate_
   return out, maps
 
 
+_MLP_CALLS = ("vmoe_expert_mlp", "vmoe_expert_mlp_planned", "vmoe_compact_rows",
+              "vmoe_compact_rows_planned")
 _last_planned = None
 
 
+def _expert_mlp_params(x, w0, b0, w1, b1, w0t, w1t, approximate_gelu, out, rows_per_expert, x_rows):
+  """The parameter block of a call, its workspace still to be named."""
+  E, R, D = out.shape
+  M = w0.shape[2] if w0 is not None else w0t.shape[1]
+  return H.ExpertMlpParams(H.ptr(x), H.ptr(w0), H.ptr(b0), H.ptr(w1), H.ptr(b1), H.ptr(w0t),
+                           H.ptr(w1t), H.ptr(out), None, 0, E, R, D, M, H.dtype_code(x.dtype),
+                           H.GELU_TANH if approximate_gelu else H.GELU_ERF,
+                           H.ptr(rows_per_expert), H.ptr(x_rows),
+                           0 if x_rows is None else x.shape[0])
+
+
 def expert_mlp_replay_planned() -> torch.Tensor:
-  """Issues vmoe_expert_mlp_planned again with the parameter block of the most recent
+  """Issues vmoe_expert_mlp_planned again on the tensors of the most recent
   expert_mlp(compact=...) call that planned its launches (same routing, same buffers: what a
   serving loop or a graph of the experts alone does) and returns that call's output tensor."""
   if _last_planned is None:
     raise RuntimeError("no planned expert_mlp call to repeat")
-  p, keep = _last_planned
+  *call, workspace, rows, row_token = _last_planned
+  p = _expert_mlp_params(*call, rows, row_token)
+  p.workspace = H.ptr(workspace)
+  p.workspace_bytes = workspace.numel() * workspace.element_size()
   H.call("vmoe_expert_mlp_planned", p)
-  return keep[7]
+  return call[-1]
 
 
-_last_status_words: Optional[torch.Tensor] = None
+_last_status_words = None       # (workspace, byte offset of its status words) of the last call
 
 
-def _note_status_words(p, workspace: torch.Tensor) -> None:
-  """Remembers where the status words of this call's workspace are (vmoe_expert_mlp_status)."""
+def _note_status_words(workspace: torch.Tensor, offset: int) -> None:
+  """Remembers where the status words of this call's workspace are (vmoe_expert_mlp_status);
+  offset < 0: the call keeps none."""
   global _last_status_words
-  addr = ctypes.c_void_p()
-  H.check(H.lib().vmoe_expert_mlp_status(ctypes.byref(p), ctypes.byref(addr)), "vmoe_expert_mlp_status")
-  if not addr.value:
-    _last_status_words = None
-    return
-  off = addr.value - workspace.data_ptr()
-  flat = workspace.view(torch.uint8).reshape(-1)
-  _last_status_words = flat[off:off + 4 * H.MLP_STATUS_WORDS].view(torch.int32)
+  _last_status_words = None if offset < 0 else (workspace, offset)
 
 
 def expert_mlp_status() -> Optional[Tuple[int, int]]:
@@ -360,7 +400,9 @@ def expert_mlp_status() -> Optional[Tuple[int, int]]:
   call on that workspace did not produce the product it should have."""
   if _last_status_words is None:
     return None
-  words = _last_status_words.cpu()
+  workspace, at = _last_status_words
+  flat = workspace.view(torch.uint8).reshape(-1)
+  words = flat[at:at + 4 * H.MLP_STATUS_WORDS].view(torch.int32).cpu()
   return int(words[H.MLP_STATUS_ABANDONED_WAITS]), int(words[H.MLP_STATUS_PLAN_MISMATCHES])
 
 
@@ -391,6 +433,14 @@ def soft_route(x: torch.Tensor, mu: torch.Tensor, scale: float, return_logits: b
   tensors, last in the result), from the same call."""
   G, S, D = x.shape
   N = mu.shape[1]
+  key = (G, S, D, N, x.dtype, float(scale), str(x.device))
+  if with_stats and not return_logits and not H.timed("vmoe_soft_route_stats"):
+    dw, cw, stats, ws = H.host().soft_route_stats(
+        H.raw_stream(), x, mu, float(scale), prepared.get(key) if prepared is not None else None)
+    if prepared is not None and key not in prepared:
+      prepared.clear()
+      prepared[key] = ws
+    return dw, cw, stats.unbind()
   x = x.contiguous()
   mu = mu.to(x.dtype).contiguous()
   dw = torch.empty((G, S, N), dtype=x.dtype, device=x.device)
@@ -398,7 +448,6 @@ def soft_route(x: torch.Tensor, mu: torch.Tensor, scale: float, return_logits: b
   logits = torch.empty_like(dw) if return_logits else None
   p = H.SoftRouteParams(H.ptr(x), H.ptr(mu), float(scale), H.ptr(dw), H.ptr(cw), H.ptr(logits),
                         None, 0, G, S, D, N, H.dtype_code(x.dtype), 0)
-  key = (G, S, D, N, x.dtype, float(scale), str(x.device))
   ws = prepared.get(key) if prepared is not None else None
   if ws is None:
     need = H.lib().vmoe_soft_route_workspace_bytes(H.ctypes.byref(p))
@@ -447,6 +496,8 @@ def _w_code(w: torch.Tensor) -> int:
 
 def einsum_dispatch(w: torch.Tensor, data: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
   """w (G,S,E,C), data (G,S,D) -> (E*G*C, D) in the expert buffer's row order."""
+  if not H.timed("vmoe_einsum_dispatch"):
+    return H.host().einsum(H.raw_stream(), w, data, out_dtype, True)
   G, S, E, C = w.shape
   D = data.shape[-1]
   w = w.contiguous()
@@ -461,6 +512,8 @@ def einsum_dispatch(w: torch.Tensor, data: torch.Tensor, out_dtype: torch.dtype)
 
 def einsum_combine(w: torch.Tensor, data: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
   """w (G,S,E,C), data (E*G*C, D) -> (G,S,D)."""
+  if not H.timed("vmoe_einsum_combine"):
+    return H.host().einsum(H.raw_stream(), w, data, out_dtype, False)
   G, S, E, C = w.shape
   D = data.shape[-1]
   w = w.contiguous()
@@ -476,6 +529,8 @@ def cast(x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
   """float32 <-> bfloat16 with the library's conversion kernel."""
   if x.dtype == dtype:
     return x
+  if not H.timed("vmoe_cast"):
+    return H.host().cast(H.raw_stream(), x, dtype)
   x = x.contiguous()
   out = torch.empty(x.shape, dtype=dtype, device=x.device)
   if x.numel():
@@ -495,6 +550,9 @@ def add_layer_norm(residual: torch.Tensor, branch: Optional[torch.Tensor],
   """
   if residual.dtype != torch.float32:
     raise TypeError(f"residual must be float32, got {residual.dtype}")
+  if not H.timed("vmoe_add_layer_norm"):
+    return H.host().add_layer_norm(H.raw_stream(), residual, branch, scale, bias, eps, out_dtype,
+                                   write_residual)
   residual = residual.contiguous()
   D = residual.shape[-1]
   rows = residual.numel() // D
@@ -536,6 +594,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float) -
   """softmax(q k^T * scale) v per (image, head).  q (B, Sq, H, hd), k, v (B, Sk, H, hd):
   views are fine as long as heads and head columns are contiguous (e.g. slices of a
   packed projection output).  Returns (B, Sq, H * hd)."""
+  if not H.timed("vmoe_attention"):
+    return H.host().attention(H.raw_stream(), q, k, v, scale)
   B, Sq, heads, hd = q.shape
   Sk = k.shape[1]
   for t in (q, k, v):

@@ -66,11 +66,13 @@ def require_no_grad(what: str, *tensors) -> None:
   """The gating, routing and expert kernels are forward-only (inference).  Called with
   the parameters and inputs of such a module: raises instead of silently cutting the
   graph when autograd is recording and one of them requires a gradient."""
-  if torch.is_grad_enabled() and any(
-      isinstance(t, torch.Tensor) and t.requires_grad for t in tensors):
-    raise NotImplementedError(
-        f"{what} has no backward pass (inference path): call it under torch.no_grad() or "
-        "detach its parameters and inputs.")
+  if not torch.is_grad_enabled():
+    return
+  for t in tensors:
+    if isinstance(t, torch.Tensor) and t.requires_grad:
+      raise NotImplementedError(
+          f"{what} has no backward pass (inference path): call it under torch.no_grad() or "
+          "detach its parameters and inputs.")
 
 
 def make_rngs(rngs, device):
@@ -97,6 +99,7 @@ class ParamCache:
   def __init__(self, limit: int = 16):
     self._entries = {}
     self._limit = limit
+    self._latest = {}       # tag -> (weak references to the tensors, versions, value) last returned
 
   @staticmethod
   def _ident(t: torch.Tensor):
@@ -105,6 +108,20 @@ class ParamCache:
 
   def get(self, tensors, tag, build):
     tensors = tuple(tensors)
+    # The tensors of the last call with this tag, unmodified: what a layer that runs over and over
+    # finds (0.3 us per tensor; the identities below take 1 us each).
+    latest = self._latest.get(tag)
+    if latest is not None and len(latest[0]) == len(tensors):
+      for t, ref, version in zip(tensors, latest[0], latest[1]):
+        if ref() is not t or t._version != version:
+          break
+      else:
+        return latest[2]
+    value = self._find(tensors, tag, build)
+    self._latest[tag] = (tuple(weakref.ref(t) for t in tensors), tuple(t._version for t in tensors), value)
+    return value
+
+  def _find(self, tensors, tag, build):
     idents = [self._ident(t) for t in tensors]
     key = (tuple(i[1] for i in idents), tag)
     versions = tuple(t._version for t in tensors)

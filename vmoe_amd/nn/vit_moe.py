@@ -24,8 +24,8 @@ class MlpBlock(module.Module):
   ``{'Dense_0': {'kernel': (D, M), 'bias': (M,)}, 'Dense_1': {'kernel': (M, D), 'bias': (D,)}}``;
   under sparse_moe_spmd every leaf gains a leading expert axis.
 
-  The bf16 kernels read the weights K-contiguous; the transposed copies are made
-  once per parameter tensor and cached.
+  The bf16 kernels read the weights K-contiguous; the transposed copies (and the biases in the
+  compute dtype) are made once per set of parameter tensors and cached.
   """
   _fields = dict(mlp_dim=module._REQUIRED, dtype=None, out_dim=None, dropout_rate=0.0,
                  deterministic=False, approximate_gelu=True)
@@ -49,8 +49,24 @@ class MlpBlock(module.Module):
     return {"params": {"Dense_0": {"kernel": k0.to(dev), "bias": b0.to(dev)},
                        "Dense_1": {"kernel": k1.to(dev), "bias": b1.to(dev)}}}
 
-  def _pack(self, w: Array, dtype) -> Array:
-    return self._packed.get((w,), dtype, lambda: K.pack_expert_weights(K.cast(w, dtype)))
+  def _weights(self, p, dtype, stacked: bool = True):
+    """Keyword arguments of kernels.expert_mlp that hold the parameters ``p`` in the compute
+    dtype and the kernels' layout, made once per set of parameter tensors.  ``stacked``: the
+    leaves have a leading expert axis (else they are one MLP's)."""
+    leaves = [p[layer].get(leaf) for layer in ("Dense_0", "Dense_1") for leaf in ("kernel", "bias")]
+    present = [t for t in leaves if t is not None]
+    module.require_no_grad("MlpBlock", *present)
+
+    def build():
+      w0, b0, w1, b1 = (t if t is None else K.cast(t if stacked else t[None], dtype) for t in leaves)
+      if dtype == torch.bfloat16:    # the matrix-core kernels read the weights K-contiguous
+        return dict(w0=None, b0=b0, w1=None, b1=b1, w0t=K.pack_expert_weights(w0),
+                    w1t=K.pack_expert_weights(w1))
+      return dict(w0=w0, b0=b0, w1=w1, b1=b1)      # float32 reads the reference's layout
+    if dtype != torch.bfloat16 and all(t.dtype == dtype for t in present):
+      return build()                               # nothing to derive
+    # (which biases are there is part of the tag: the tensors alone do not say whose they are)
+    return self._packed.get(present, (dtype, stacked, leaves[1] is None, leaves[3] is None), build)
 
   supports_packed_rows = True
 
@@ -58,18 +74,9 @@ class MlpBlock(module.Module):
     """inputs (E, R, D) with parameters stacked on axis 0 -> (E, R, D).  With
     rows_per_expert (E,) int32 only that many leading rows of each expert are
     computed; the other rows of the result are not written."""
-    p = variables["params"]
     dtype = self.dtype or inputs.dtype
-    w0, b0 = p["Dense_0"]["kernel"], p["Dense_0"].get("bias")
-    w1, b1 = p["Dense_1"]["kernel"], p["Dense_1"].get("bias")
-    module.require_no_grad("MlpBlock", inputs, w0, b0, w1, b1)
-    x = K.cast(inputs, dtype)
-    cast = lambda t: None if t is None else K.cast(t, dtype)
-    if dtype == torch.bfloat16:
-      return K.expert_mlp(x, None, cast(b0), None, cast(b1), w0t=self._pack(w0, dtype),
-                          w1t=self._pack(w1, dtype), approximate_gelu=self.approximate_gelu,
-                          rows_per_expert=rows_per_expert)
-    return K.expert_mlp(x, cast(w0), cast(b0), cast(w1), cast(b1),
+    module.require_no_grad("MlpBlock", inputs)
+    return K.expert_mlp(K.cast(inputs, dtype), **self._weights(variables["params"], dtype),
                         approximate_gelu=self.approximate_gelu, rows_per_expert=rows_per_expert)
 
   def can_gather(self, items: Array) -> bool:
@@ -83,18 +90,9 @@ class MlpBlock(module.Module):
     """items (T, D); row_token (E, R) int32 names the item in row r of expert e,
     rows_per_expert (E,) how many rows each expert has -> (E, R, D).  The first product
     reads its rows straight from ``items``: the dispatched buffer is never built."""
-    p = variables["params"]
     dtype = self.dtype or items.dtype
-    w0, b0 = p["Dense_0"]["kernel"], p["Dense_0"].get("bias")
-    w1, b1 = p["Dense_1"]["kernel"], p["Dense_1"].get("bias")
-    module.require_no_grad("MlpBlock", items, w0, b0, w1, b1)
-    cast = lambda t: None if t is None else K.cast(t, dtype)
-    if dtype != torch.bfloat16:      # float32 reads the kernels in the reference's layout
-      return K.expert_mlp(K.cast(items, dtype), cast(w0), cast(b0), cast(w1), cast(b1),
-                          approximate_gelu=self.approximate_gelu, rows_per_expert=rows_per_expert,
-                          x_rows=row_token)
-    return K.expert_mlp(K.cast(items, dtype), None, cast(b0), None, cast(b1),
-                        w0t=self._pack(w0, dtype), w1t=self._pack(w1, dtype),
+    module.require_no_grad("MlpBlock", items)
+    return K.expert_mlp(K.cast(items, dtype), **self._weights(variables["params"], dtype),
                         approximate_gelu=self.approximate_gelu, rows_per_expert=rows_per_expert,
                         x_rows=row_token)
 
@@ -104,27 +102,21 @@ class MlpBlock(module.Module):
     items (T, D), fill (G, E) and token_slot (G, S, K) of the slot assignment -> (outputs
     (E, G * capacity, D), (token_row, rows_per_expert, row_token)).  The renumbering of the
     assignments shares a launch with the planning of the two products."""
-    p = variables["params"]
     dtype = self.dtype or items.dtype
-    w0, b0 = p["Dense_0"]["kernel"], p["Dense_0"].get("bias")
-    w1, b1 = p["Dense_1"]["kernel"], p["Dense_1"].get("bias")
-    module.require_no_grad("MlpBlock", items, w0, b0, w1, b1)
-    cast = lambda t: None if t is None else K.cast(t, dtype)
-    if dtype != torch.bfloat16:
-      return K.expert_mlp(K.cast(items, dtype), cast(w0), cast(b0), cast(w1), cast(b1),
-                          approximate_gelu=self.approximate_gelu,
-                          compact=(fill, token_slot, capacity))
-    return K.expert_mlp(K.cast(items, dtype), None, cast(b0), None, cast(b1),
-                        w0t=self._pack(w0, dtype), w1t=self._pack(w1, dtype),
+    module.require_no_grad("MlpBlock", items)
+    return K.expert_mlp(K.cast(items, dtype), **self._weights(variables["params"], dtype),
                         approximate_gelu=self.approximate_gelu,
                         compact=(fill, token_slot, capacity))
 
   def apply(self, variables, inputs: Array) -> Array:
     """Single MLP: inputs (..., D)."""
-    stacked = vmoe_amd.moe._tree_map(lambda t: t[None], variables)
-    lead = inputs.shape[:-1]
-    out = self.apply_experts(stacked, inputs.reshape(1, -1, inputs.shape[-1]))
-    return out.reshape(*lead, out.shape[-1])
+    dtype = self.dtype or inputs.dtype
+    module.require_no_grad("MlpBlock", inputs)
+    x = K.cast(inputs, dtype)
+    out = K.expert_mlp(x.reshape(1, -1, x.shape[-1]),
+                       **self._weights(variables["params"], dtype, stacked=False),
+                       approximate_gelu=self.approximate_gelu)
+    return out.view(*inputs.shape[:-1], out.shape[-1])
 
 
 class MlpMoeBlock(module.Module):
@@ -284,14 +276,21 @@ class MultiHeadDotProductAttention(module.Module):
       p["key_ln"] = {"scale": torch.ones((hd,), device=dev)}
     return {"params": p}
 
-  def _proj_weights(self, p, names, dtype):
-    """(sum of H * hd, D) weight and bias of the named input projections, packed once."""
+  def _proj_weights(self, p, groups, dtype):
+    """For each group of input projections one (sum of H * hd, D) weight and its bias, then the
+    output projection's weight and bias: packed once per set of parameter tensors."""
     def build():
-      w = torch.cat([p[n]["kernel"].reshape(p[n]["kernel"].shape[0], -1).t() for n in names])
-      b = torch.cat([p[n]["bias"].reshape(-1) for n in names])
-      return w.to(dtype).contiguous(), b.to(dtype).contiguous()
-    tensors = [p[n][leaf] for n in names for leaf in ("kernel", "bias")]
-    return self._packed.get(tensors, (dtype, names), build)
+      packed = []
+      for names in groups:
+        w = torch.cat([p[n]["kernel"].reshape(p[n]["kernel"].shape[0], -1).t() for n in names])
+        b = torch.cat([p[n]["bias"].reshape(-1) for n in names])
+        packed += [w.to(dtype).contiguous(), b.to(dtype).contiguous()]
+      w = p["out"]["kernel"]
+      packed += [w.reshape(w.shape[0] * w.shape[1], -1).t().to(dtype).contiguous(),
+                 p["out"]["bias"].to(dtype)]
+      return packed
+    tensors = [p[n][leaf] for n in ("query", "key", "value", "out") for leaf in ("kernel", "bias")]
+    return self._packed.get(tensors, (dtype, groups), build)
 
   def apply(self, variables, inputs_q: Array, inputs_kv: Optional[Array] = None) -> Array:
     p = variables["params"]
@@ -305,12 +304,10 @@ class MultiHeadDotProductAttention(module.Module):
     xq = inputs_q.to(dtype)
     linear = torch.nn.functional.linear
     if inputs_kv is inputs_q:
-      w, b = self._proj_weights(p, ("query", "key", "value"), dtype)
-      qkv = linear(xq, w, b).view(B, Sq, 3, H, hd)
-      q, k, v = qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2]
+      w, b, wo, bo = self._proj_weights(p, (("query", "key", "value"),), dtype)
+      q, k, v = linear(xq, w, b).view(B, Sq, 3, H, hd).unbind(2)
     else:
-      wq, bq = self._proj_weights(p, ("query",), dtype)
-      wkv, bkv = self._proj_weights(p, ("key", "value"), dtype)
+      wq, bq, wkv, bkv, wo, bo = self._proj_weights(p, (("query",), ("key", "value")), dtype)
       q = linear(xq, wq, bq).view(B, Sq, H, hd)
       kv = linear(inputs_kv.to(dtype), wkv, bkv).view(B, Sk, 2, H, hd)
       k, v = kv[:, :, 0], kv[:, :, 1]
@@ -323,10 +320,6 @@ class MultiHeadDotProductAttention(module.Module):
       ctx = torch.nn.functional.scaled_dot_product_attention(
           q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2))     # (B, H, Sq, hd)
       ctx = ctx.transpose(1, 2).reshape(B, Sq, H * hd)
-    wo, bo = self._packed.get(
-        (p["out"]["kernel"], p["out"]["bias"]), (dtype, "out"),
-        lambda: (p["out"]["kernel"].reshape(H * hd, -1).t().to(dtype).contiguous(),
-                 p["out"]["bias"].to(dtype)))
     return linear(ctx, wo, bo)
 
 
