@@ -499,6 +499,45 @@ def test_soft_route(K, G, S, D, n, p, dtype):
   np.testing.assert_allclose(to_np(cw).sum(2), 1.0, atol=atol)
 
 
+@pytest.mark.parametrize("G,S,D,N,dtype", [
+    (3, 65, 64, 256, O.BF16),      # 16-row tiles, one row past the fourth
+    (128, 65, 64, 160, O.BF16),    # 64-row tiles
+    (256, 33, 1024, 128, O.BF16),  # 32-row tiles, widest model width
+    (2, 17, 40, 17, O.BF16),       # slots that are no whole piece, width padded to whole steps
+    (1, 1, 8, 1, O.BF16),
+    (4, 196, 736, 74, O.BF16),
+    (2, 300, 512, 520, O.BF16),    # more logits than a workgroup per group could hold
+    (5, 49, 512, 48, O.F32),
+    (2, 31, 102, 33, O.F32),       # rows at unaligned addresses
+    (3, 130, 960, 74, O.F32),
+    (140, 64, 48, 164, O.F32),     # 64-row tiles
+])
+def test_soft_route_row_tiles(K, G, S, D, N, dtype):
+  """Shapes whose routing runs over row tiles: logits against float64 within the dtype's
+  tolerance, both softmaxes against the float64 softmaxes of the returned logits, the monitoring
+  sums against the returned weights; with prepared slot parameters bit for bit the same."""
+  rng = np.random.default_rng(G * S + N)
+  x = O.cast(rng.standard_normal((G, S, D)), dtype)
+  mu = O.cast(rng.standard_normal((D, N)) / np.sqrt(D), dtype)
+  scale = 1.5
+  dw, cw, lg = (to_np(t) for t in K.soft_route(to_dev(x, dtype), to_dev(mu, dtype), scale, return_logits=True))
+  x64, mu64 = x.astype(np.float64), mu.astype(np.float64)
+  want = np.einsum("gsd,dn->gsn", x64 / np.sqrt((x64 ** 2).sum(-1, keepdims=True) + 1e-6),
+                   scale * mu64 / np.sqrt((mu64 ** 2).sum(0) + 1e-6))
+  # bfloat16: both operands and the logit are rounded, 2^-9 each, on a sum of unit vectors' products
+  assert np.abs(lg - want).max() <= (3 * 2.0 ** -9 * scale if dtype == O.BF16 else 2e-6 * scale)
+  _check_soft_weights_against_own_logits(lg, dw, cw, dtype, f"G={G} S={S} D={D} N={N}")
+  prepared = {}
+  for _ in range(2):
+    dw2, cw2, scalars = K.soft_route(to_dev(x, dtype), to_dev(mu, dtype), scale, prepared=prepared, with_stats=True)
+    np.testing.assert_array_equal(to_np(dw2), dw)
+    np.testing.assert_array_equal(to_np(cw2), cw)
+  d, c = dw.astype(np.float64), cw.astype(np.float64)
+  np.testing.assert_allclose([float(v) for v in scalars][:4],
+                             [c.min(axis=2).mean(), c.max(axis=2).mean(), d.min(axis=1).mean(), d.max(axis=1).mean()],
+                             rtol=3e-6)
+
+
 def _check_soft_weights_against_own_logits(lg, dw, cw, dtype, tag):
   """The two softmaxes themselves.  Against the oracle the weights carry the difference of the
   logits (a bfloat16 logit that rounds the other way moves a weight by exp(step) - 1, which is

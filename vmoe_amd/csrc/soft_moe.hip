@@ -1,12 +1,11 @@
 // Soft MoE routing and dense (einsum) dispatch / combine for gfx950.
 //
-// soft_route replaces vmoe/projects/soft_moe/router.py:57-96: one workgroup per
-// group normalises the item rows, multiplies them with the unit-norm slot
-// parameters on the matrix cores, keeps the (S x N) logits of the group in LDS
-// and takes both softmaxes (over items for the dispatch weights, over slots for
-// the combine weights) from that one copy.  The bfloat16 kernel for the model
-// widths up to 768 splits the waves of a workgroup into two roles
-// (soft_route_roles_kernel).
+// soft_route replaces vmoe/projects/soft_moe/router.py:57-96: item rows are normalised, multiplied
+// with the unit-norm slot parameters on the matrix cores, and both softmaxes (over items for the
+// dispatch weights, over slots for the combine weights) are taken from the logits.  bfloat16 with up
+// to 128 slots and the model widths up to 768 runs one workgroup per group whose waves have two roles
+// (soft_route_roles_kernel, logits in LDS); everything else runs over row tiles
+// (soft_route_tiles.h); rows too wide for those take soft_route_kernel.
 //
 // einsum_dispatch / einsum_combine replace EinsumDispatcher.dispatch/.combine
 // (vmoe/moe.py:148-161) for dense weights, including the expert-buffer row
@@ -19,11 +18,13 @@
 
 #include "vmoe_common.h"
 #include "einsum_bf16.h"
+#include "soft_route_tiles.h"
 
 namespace vmoe {
 namespace {
 
-constexpr float kNormEps = 1e-6f;
+using soft::kLog2e;
+using soft::kNormEps;
 
 __device__ __forceinline__ float load_any(const void* p, size_t i, int dtype) {
   return dtype == VMOE_F32 ? reinterpret_cast<const float*>(p)[i]
@@ -42,24 +43,28 @@ __device__ __forceinline__ void store_any(void* p, size_t i, float v, int dtype)
 // Unit-normalise the columns of mu (D, N) and apply the scale when it belongs to
 // mu.  bf16: writes muT (N, D) so that a column's k run is contiguous;
 // f32: writes (D, N).
-// frag_ksw > 0 (bf16, D = 32 * frag_ksw): the order in which soft_route_roles_kernel's
-// consumer waves hold the parameters, [slot / 32][slot % 32 / 16][d / 32][lane][d % 8]
-// with lane = (d % 32 / 8) * 16 + slot % 16, so that every fragment load of a wave is
-// 1 KB of consecutive memory; the grid then covers the slots up to a multiple of 32 and
-// the ones past N are zeros.
+// frag_steps > 0: the order in which the matrix cores take the parameters,
+// [slot / 16][step][lane][V] with V = 16 bytes of values, a step 4 V wide and
+// lane = (d % 4V / V) * 16 + slot % 16 (float32: (d % 4) * 16 + slot % 16), so that every fragment load of a wave is 1 KB of
+// consecutive memory; the grid then covers the slots up to a multiple of 16 (32 for
+// soft_route_roles_kernel) and the steps the widths up to frag_steps * 4 V: what lies past N and D
+// is zero.
 template <typename T>
 __global__ __launch_bounds__(256) void soft_prep_mu_kernel(const T* __restrict__ mu,
                                                            T* __restrict__ out, float scale,
                                                            int scale_mu, int D, int N,
-                                                           int frag_ksw = 0) {
+                                                           int frag_steps = 0) {
   __shared__ float red[256];
+  constexpr int V = 16 / (int)sizeof(T);
   const int n = blockIdx.x, tid = threadIdx.x;
+  const int Dp = frag_steps > 0 ? frag_steps * 4 * V : D;
   auto frag_index = [&](int d) -> size_t {
-    const int lane = ((d & 31) >> 3) * 16 + (n & 15);
-    return ((((size_t)(n >> 5) * 2 + ((n & 31) >> 4)) * frag_ksw + (d >> 5)) * 64 + lane) * 8 + (d & 7);
+    const int dd = d % (4 * V);        // float32: four values 4 apart per lane, see soft_route_tiles.h
+    const int q = sizeof(T) == 2 ? dd / V : dd % 4, v = sizeof(T) == 2 ? dd % V : dd / 4;
+    return (((size_t)(n >> 4) * frag_steps + d / (4 * V)) * 64 + q * 16 + (n & 15)) * V + v;
   };
   if (n >= N) {     // padding slots of the fragment order
-    for (int d = tid; d < D; d += 256) Elt<T>::store(out + frag_index(d), 0.f);
+    for (int d = tid; d < Dp; d += 256) Elt<T>::store(out + frag_index(d), 0.f);
     return;
   }
   float s = 0.f;
@@ -75,10 +80,10 @@ __global__ __launch_bounds__(256) void soft_prep_mu_kernel(const T* __restrict__
   }
   const float inv = 1.0f / sqrtf(red[0] + kNormEps);
   const float sc = Elt<T>::round(scale);
-  for (int d = tid; d < D; d += 256) {
-    float v = Elt<T>::round(Elt<T>::load(mu + (size_t)d * N + n) * inv);
+  for (int d = tid; d < Dp; d += 256) {
+    float v = d < D ? Elt<T>::round(Elt<T>::load(mu + (size_t)d * N + n) * inv) : 0.f;
     if (scale_mu) v = Elt<T>::round(v * sc);
-    if (frag_ksw > 0) Elt<T>::store(out + frag_index(d), v);
+    if (frag_steps > 0) Elt<T>::store(out + frag_index(d), v);
     else if (sizeof(T) == 2) Elt<T>::store(out + (size_t)n * D + d, v);
     else Elt<T>::store(out + (size_t)d * N + n, v);
   }
@@ -219,288 +224,11 @@ __global__ __launch_bounds__(256) void soft_route_kernel(
   }
 }
 
-// bfloat16 soft routing, fast path (N <= 128 slots, D <= 32 * 2 * KSW).
-//
-// One workgroup of eight waves per group, with the unit-norm slot parameters held
-// in registers for the whole kernel: wave w keeps the B fragments of 16 slots for
-// the whole contraction (v_mfma_f32_16x16x32_bf16).  The item rows then stream
-// through once, 32 at a time: each wave loads four whole rows (coalesced), takes
-// their norms from its registers, and writes the normalised rows into an LDS tile
-// while the loads of the next 64 rows are already in flight; every wave multiplies
-// the tile with its slots, and the logits of the group collect in LDS as
-// bfloat16.  Both softmaxes (over slots for the combine weights, over items for
-// the dispatch weights) are taken from that one copy, so memory sees the items
-// once and each weight once.
 constexpr int kSrThreads = 512;
-constexpr int kSrRows = 32;
 
-// Model widths the register-resident fast path is instantiated for.
-inline bool soft_fast_width(int D) { return D == 256 || D == 384 || D == 512 || D == 768 || D == 1024; }
+// Model widths that soft_route_roles_kernel is instantiated for.
+inline bool soft_roles_width(int D) { return D == 256 || D == 384 || D == 512 || D == 768; }
 
-struct SoftLds {
-  size_t xs, part, red, cmx, csum, lg, total;
-};
-inline SoftLds soft_lds_layout(int D, int SP, int NP) {
-  SoftLds l;
-  l.xs = 0;
-  l.part = l.xs + (size_t)kSrRows * (D + 8) * 2;
-  l.red = l.part;
-  l.cmx = l.red + kSrThreads * sizeof(float);
-  l.csum = l.cmx + 128 * sizeof(float);
-  l.lg = l.csum + 128 * sizeof(float);
-  l.total = l.lg + (size_t)SP * (NP + 8) * 2;
-  return l;
-}
-
-// exp(l - mx) / sum as exp2(l * log2e - mx * log2e) * (1 / sum) with the hardware
-// exp2 and reciprocal: relative error ~1e-6, against 4e-3 for the bfloat16 result.
-constexpr float kLog2e = 1.4426950408889634f;
-
-template <int KSW>
-__global__ __launch_bounds__(kSrThreads) void soft_route_bf16_kernel(
-    const bf16_t* __restrict__ x, const bf16_t* __restrict__ muw, bf16_t* __restrict__ dispatch_w,
-    bf16_t* __restrict__ combine_w, bf16_t* __restrict__ logits_out, float scale, int scale_x, int S,
-    int D, int N, int SP, int NP, SoftLds L) {
-  constexpr int CP = (KSW + 7) / 8;   // 16-byte pieces of an item row per lane of a half wave
-  extern __shared__ __align__(16) unsigned char smem[];
-  bf16_t* xs = reinterpret_cast<bf16_t*>(smem + L.xs);
-  float* red = reinterpret_cast<float*>(smem + L.red);
-  float* cmx = reinterpret_cast<float*>(smem + L.cmx);
-  float* csum = reinterpret_cast<float*>(smem + L.csum);
-  bf16_t* lg = reinterpret_cast<bf16_t*>(smem + L.lg);
-  const int LDX = D + 8, LDW = NP + 8;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int m = lane & 31, h = lane >> 5;
-  const int g = blockIdx.x;
-  const bf16_t* xg = x + (size_t)g * S * D;
-  const float sc = bf16r(scale);
-  const int row_chunks = D / 8, row_tiles = SP / kSrRows;
-  const int r16 = lane & 15, kq = lane >> 4;   // 16x16x32 fragment: row / column, k quarter
-  const bool mma_on = wave * 16 < NP;
-
-  // Slot parameters of this wave: slots wave*16 .. +16, every k step (D == 32 * KSW).
-  bf16x8 bfr[KSW];
-  {
-    const bf16_t* brow = muw + (size_t)min(wave * 16 + r16, N - 1) * D + kq * 8;
-#pragma unroll
-    for (int i = 0; i < KSW; ++i)
-      bfr[i] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(brow + i * 32));
-  }
-
-  // Combine weights of the item rows [s_begin, s_end): softmax over the N slots.
-  // Half wave = one row, lane = four consecutive slots; two rows per half wave at a
-  // time so that the two shuffle chains overlap.
-  auto combine_rows = [&](int s_begin, int s_end) {
-    for (int s0 = s_begin + wave * 4; s0 < s_end; s0 += 32) {
-      const int c = m * 4;
-      float l[2][4], mx[2];
-#pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        const int s = s0 + 2 * r + h;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) l[r][u] = -INFINITY;
-        if (s < s_end && c < N) {
-          const uint2 pr = *reinterpret_cast<const uint2*>(lg + (size_t)s * LDW + c);
-          l[r][0] = bf_lo(pr.x); l[r][1] = bf_hi(pr.x); l[r][2] = bf_lo(pr.y); l[r][3] = bf_hi(pr.y);
-        }
-        mx[r] = fmaxf(fmaxf(l[r][0], l[r][1]), fmaxf(l[r][2], l[r][3]));
-      }
-#pragma unroll
-      for (int o = 16; o > 0; o >>= 1)
-#pragma unroll
-        for (int r = 0; r < 2; ++r) mx[r] = fmaxf(mx[r], __shfl_xor(mx[r], o, kWave));
-      float e[2][4], sum[2];
-#pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        const float mb = mx[r] * kLog2e;
-        sum[r] = 0.f;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          e[r][u] = __builtin_amdgcn_exp2f(fmaf(l[r][u], kLog2e, -mb));   // exp2(-inf) = 0 past N
-          sum[r] += e[r][u];
-        }
-      }
-#pragma unroll
-      for (int o = 16; o > 0; o >>= 1)
-#pragma unroll
-        for (int r = 0; r < 2; ++r) sum[r] += __shfl_xor(sum[r], o, kWave);
-#pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        const int s = s0 + 2 * r + h;
-        const float rs = __builtin_amdgcn_rcpf(sum[r]);
-        if (s < s_end && c < N)
-          *reinterpret_cast<uint2*>(combine_w + ((size_t)g * S + s) * N + c) = make_uint2(
-              pack_bf16x2(e[r][0] * rs, e[r][1] * rs), pack_bf16x2(e[r][2] * rs, e[r][3] * rs));
-      }
-    }
-  };
-
-  // Four item rows per wave and tile, one row per half wave at a time (rows
-  // wave*4 + 2*i + h); rows past S re-read row S-1 and are written as zeros.
-  auto load_rows = [&](uint4 (&raw)[2][CP], int t) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int r = min(t * kSrRows + wave * 4 + 2 * i + h, S - 1);
-#pragma unroll
-      for (int ps = 0; ps < CP; ++ps) {
-        const int c = min(ps * 32 + m, row_chunks - 1);
-        raw[i][ps] = *reinterpret_cast<const uint4*>(xg + (size_t)r * D + c * 8);
-      }
-    }
-  };
-
-  // One tile of 32 item rows, held in raw; its registers then take the tile after next.
-  auto tile = [&](uint4 (&raw)[2][CP], int t) {
-    // norms from the registers, normalised rows into the LDS tile
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      float sq = 0.f;
-#pragma unroll
-      for (int ps = 0; ps < CP; ++ps) {
-        const uint32_t w4[4] = {raw[i][ps].x, raw[i][ps].y, raw[i][ps].z, raw[i][ps].w};
-        float tsum = 0.f;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float lo = bf_lo(w4[q]), hi = bf_hi(w4[q]);
-          tsum = fmaf(lo, lo, tsum);
-          tsum = fmaf(hi, hi, tsum);
-        }
-        if (ps * 32 + m < row_chunks) sq += tsum;
-      }
-#pragma unroll
-      for (int o = 16; o > 0; o >>= 1) sq += __shfl_xor(sq, o, kWave);
-      const int lrow = wave * 4 + 2 * i + h;
-      const float inv = t * kSrRows + lrow < S ? 1.0f / sqrtf(sq + kNormEps) : 0.f;
-#pragma unroll
-      for (int ps = 0; ps < CP; ++ps) {
-        const int c = ps * 32 + m;
-        const uint32_t w4[4] = {raw[i][ps].x, raw[i][ps].y, raw[i][ps].z, raw[i][ps].w};
-        uint32_t o4[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          float lo = bf_lo(w4[q]) * inv, hi = bf_hi(w4[q]) * inv;
-          if (scale_x) { lo = bf16r(lo) * sc; hi = bf16r(hi) * sc; }
-          o4[q] = pack_bf16x2(lo, hi);
-        }
-        if (c < row_chunks)
-          *reinterpret_cast<uint4*>(xs + (size_t)lrow * LDX + c * 8) = make_uint4(o4[0], o4[1], o4[2], o4[3]);
-      }
-    }
-    wait_lgkmcnt0();
-    raw_barrier();
-    if (t + 2 < row_tiles) load_rows(raw, t + 2);
-    // the logits of the previous tile are complete: their combine weights fill the
-    // time the loads are in flight
-    if (t > 0) combine_rows((t - 1) * kSrRows, min(t * kSrRows, S));
-
-    if (mma_on) {
-      floatx4 acc[2];
-#pragma unroll
-      for (int rh = 0; rh < 2; ++rh)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) acc[rh][v] = 0.f;
-      const bf16_t* arow = xs + (size_t)r16 * LDX + kq * 8;
-#pragma unroll
-      for (int i = 0; i < KSW; ++i) {
-        const int ko = i * 32;
-#pragma unroll
-        for (int rh = 0; rh < 2; ++rh) {
-          const bf16x8 af = __builtin_bit_cast(
-              bf16x8, *reinterpret_cast<const uint4*>(arow + (size_t)rh * 16 * LDX + ko));
-          acc[rh] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bfr[i], acc[rh], 0, 0, 0);
-        }
-        // bound how many fragment reads the scheduler hoists (register pressure)
-        if ((i & 3) == 3) __builtin_amdgcn_sched_barrier(0);
-      }
-      mfma_result_fence();
-      const int col = wave * 16 + r16;
-#pragma unroll
-      for (int rh = 0; rh < 2; ++rh)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int row = t * kSrRows + rh * 16 + kq * 4 + v;
-          lg[(size_t)row * LDW + col] = f2bf(acc[rh][v]);
-        }
-    }
-    wait_lgkmcnt0();
-    raw_barrier();
-  };
-
-  uint4 raw0[2][CP], raw1[2][CP];
-  load_rows(raw0, 0);
-  if (row_tiles > 1) load_rows(raw1, 1);
-  for (int t = 0; t < row_tiles; t += 2) {
-    tile(raw0, t);
-    if (t + 1 < row_tiles) tile(raw1, t + 1);
-  }
-  __syncthreads();
-  combine_rows((row_tiles - 1) * kSrRows, S);
-
-  // Thread -> (16-byte piece c of a weights row, rows s = sr, sr + rpp, ...).
-  const int lchunks = N / 8, rpp = kSrThreads / lchunks;
-  const int sr = tid / lchunks, pc = tid - sr * lchunks;
-  if (logits_out != nullptr && sr < rpp) {
-    for (int s = sr; s < S; s += rpp)
-      *reinterpret_cast<uint4*>(logits_out + ((size_t)g * S + s) * N + pc * 8) =
-          *reinterpret_cast<const uint4*>(lg + (size_t)s * LDW + pc * 8);
-  }
-
-  // Dispatch weights: softmax over the S items of each slot.  For the maxima and
-  // sums a column is shared by RG threads that take every RG-th row and meet in LDS.
-  {
-    const int RG = kSrThreads / NP;
-    const int n = tid % NP, rg = tid / NP;
-    const bool act = rg < RG;
-    float mx = -INFINITY;
-    if (act)
-#pragma unroll 8
-      for (int s = rg; s < S; s += RG) mx = fmaxf(mx, bf2f(lg[(size_t)s * LDW + n]));
-    red[tid] = mx;
-    __syncthreads();
-    if (act) {
-      mx = -INFINITY;
-      for (int q = 0; q < RG; ++q) mx = fmaxf(mx, red[q * NP + n]);
-    }
-    __syncthreads();
-    const float mb = mx * kLog2e;
-    float sum = 0.f;
-    if (act)
-#pragma unroll 8
-      for (int s = rg; s < S; s += RG)
-        sum += __builtin_amdgcn_exp2f(fmaf(bf2f(lg[(size_t)s * LDW + n]), kLog2e, -mb));
-    red[tid] = sum;
-    __syncthreads();
-    if (act && rg == 0) {
-      sum = 0.f;
-      for (int q = 0; q < RG; ++q) sum += red[q * NP + n];
-      cmx[n] = mb;
-      csum[n] = __builtin_amdgcn_rcpf(sum);
-    }
-    __syncthreads();
-    if (sr < rpp) {
-      float cm[8], cr[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        cm[u] = cmx[pc * 8 + u];
-        cr[u] = csum[pc * 8 + u];
-      }
-#pragma unroll 4
-      for (int s = sr; s < S; s += rpp) {
-        const uint4 rawl = *reinterpret_cast<const uint4*>(lg + (size_t)s * LDW + pc * 8);
-        const uint32_t w4[4] = {rawl.x, rawl.y, rawl.z, rawl.w};
-        uint32_t o4[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const float lo = __builtin_amdgcn_exp2f(fmaf(bf_lo(w4[u]), kLog2e, -cm[2 * u])) * cr[2 * u];
-          const float hi = __builtin_amdgcn_exp2f(fmaf(bf_hi(w4[u]), kLog2e, -cm[2 * u + 1])) * cr[2 * u + 1];
-          o4[u] = pack_bf16x2(lo, hi);
-        }
-        *reinterpret_cast<uint4*>(dispatch_w + ((size_t)g * S + s) * N + pc * 8) =
-            make_uint4(o4[0], o4[1], o4[2], o4[3]);
-      }
-    }
-  }
-}
 
 // Reductions over the 32 lanes of a half wave: four DPP steps inside a row of 16 lanes
 // (quad_perm [1,0,3,2], quad_perm [2,3,0,1], row_half_mirror, row_mirror), then one exchange
@@ -546,15 +274,15 @@ __device__ __forceinline__ float half_wave_max(float v) {
   return fmaxf(v, __shfl_xor(v, 16, kWave));
 }
 
-// soft_route_bf16_kernel with the waves of a workgroup in two roles (N <= 128 slots,
-// D = 32 * KSW <= 768).  In the single-role kernel every wave normalises rows (VALU), then
+// bfloat16 routing with up to 128 slots, one workgroup of eight waves per group (D = 32 * KSW <= 768),
+// its waves in two roles.  With one role every wave normalises rows (VALU), then
 // every wave multiplies (LDS reads and matrix cores), then every wave takes the row
 // softmax (VALU): the units take turns.  Here waves 0..3 only fetch and normalise item rows
 // (tile t + 1 into one of two LDS tiles) while waves 4..7, each with the unit-norm
 // parameters of 32 slots in registers, multiply tile t and take the combine weights of
-// tile t - 1; one barrier per tile hands the tiles over.  A consumer wave reads an item
-// tile once for 32 slots (the single-role kernel: once per 16), so the LDS reads halve as
-// well.  The arithmetic per element is that of soft_route_bf16_kernel.
+// tile t - 1; one barrier per tile hands the tiles over.  The logits of the group collect in LDS
+// as bfloat16; both softmaxes (over slots for the combine weights, over items for the dispatch
+// weights) are taken from that one copy, so memory sees the items once and each weight once.
 struct SoftPipeLds {
   size_t xs, red, cmx, csum, lg, total;
 };
@@ -1119,11 +847,11 @@ int check_einsum(const VmoeEinsumParams* p, bool dispatch) {
 
 
 // Monitoring scalars of the Soft MoE router (vmoe/projects/soft_moe/router.py:119-125),
-// per group: sum over items of the min / max over slots of the combine weights, and
+// per group, for rows of more than 1024 values or pieces: sum over items of the min / max over slots of the combine weights, and
 // sum over slots of the min / max over items of the dispatch weights.  The caller
 // sums the (G, 4) partials and divides by the counts.
 template <typename T>
-__global__ __launch_bounds__(256) void soft_stats_kernel(const T* __restrict__ combine_w,
+__global__ __launch_bounds__(256) void soft_stats_wide_kernel(const T* __restrict__ combine_w,
                                                          const T* __restrict__ dispatch_w,
                                                          float* __restrict__ partial, int S, int N) {
   __shared__ float red[4][4];
@@ -1173,89 +901,6 @@ __global__ __launch_bounds__(256) void soft_stats_kernel(const T* __restrict__ c
   if (tid < 4) partial[(size_t)g * 4 + tid] = red[0][tid] + red[1][tid] + red[2][tid] + red[3][tid];
 }
 
-template <typename T> __device__ __forceinline__ void unpack16(uint4 q, float* v);
-template <> __device__ __forceinline__ void unpack16<float>(uint4 q, float* v) {
-  v[0] = __builtin_bit_cast(float, q.x); v[1] = __builtin_bit_cast(float, q.y);
-  v[2] = __builtin_bit_cast(float, q.z); v[3] = __builtin_bit_cast(float, q.w);
-}
-template <> __device__ __forceinline__ void unpack16<bf16_t>(uint4 q, float* v) {
-  v[0] = bf_lo(q.x); v[1] = bf_hi(q.x); v[2] = bf_lo(q.y); v[3] = bf_hi(q.y);
-  v[4] = bf_lo(q.z); v[5] = bf_hi(q.z); v[6] = bf_lo(q.w); v[7] = bf_hi(q.w);
-}
-
-// The same sums with 16-byte loads when a row is a power-of-two number NC <= 64 of
-// 16-byte chunks.  blockIdx.y = 0 takes the combine weights (a row's chunks sit in NC
-// adjacent lanes, so the row minimum is a lane exchange), blockIdx.y = 1 the dispatch
-// weights (a thread keeps one chunk column over all its rows; the 256 / NC threads of
-// a column meet in LDS).
-template <typename T>
-__global__ __launch_bounds__(256) void soft_stats_vec_kernel(const T* __restrict__ combine_w,
-                                                             const T* __restrict__ dispatch_w,
-                                                             float* __restrict__ partial, int S, int N) {
-  constexpr int V = 16 / sizeof(T);
-  __shared__ float lds_min[256 * V];
-  __shared__ float lds_max[256 * V];
-  __shared__ float red[4][2];
-  const int g = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int NC = N / V;
-  const int total = S * NC;
-  float sum_min = 0.f, sum_max = 0.f;
-  if (blockIdx.y == 0) {
-    const uint4* src = reinterpret_cast<const uint4*>(combine_w + (size_t)g * S * N);
-    const int rounds = (total + 255) / 256;
-    for (int k = 0; k < rounds; ++k) {
-      const int i = k * 256 + tid;
-      float mn = INFINITY, mx = -INFINITY;
-      if (i < total) {
-        float v[V];
-        unpack16<T>(src[i], v);
-#pragma unroll
-        for (int j = 0; j < V; ++j) { mn = fminf(mn, v[j]); mx = fmaxf(mx, v[j]); }
-      }
-      for (int o = 1; o < NC; o <<= 1) {
-        mn = fminf(mn, __shfl_xor(mn, o, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-      }
-      if (i < total && (lane & (NC - 1)) == 0) { sum_min += mn; sum_max += mx; }
-    }
-  } else {
-    const uint4* src = reinterpret_cast<const uint4*>(dispatch_w + (size_t)g * S * N);
-    float mn[V], mx[V];
-#pragma unroll
-    for (int j = 0; j < V; ++j) { mn[j] = INFINITY; mx[j] = -INFINITY; }
-    for (int i = tid; i < total; i += 256) {
-      float v[V];
-      unpack16<T>(src[i], v);
-#pragma unroll
-      for (int j = 0; j < V; ++j) { mn[j] = fminf(mn[j], v[j]); mx[j] = fmaxf(mx[j], v[j]); }
-    }
-    // thread t holds chunk column t % NC; LDS as [t / NC][column * V + j]
-#pragma unroll
-    for (int j = 0; j < V; ++j) {
-      lds_min[(tid / NC) * N + (tid % NC) * V + j] = mn[j];
-      lds_max[(tid / NC) * N + (tid % NC) * V + j] = mx[j];
-    }
-    __syncthreads();
-    const int parts = 256 / NC;
-    for (int c = tid; c < N; c += 256) {
-      float a = INFINITY, b = -INFINITY;
-      for (int q = 0; q < parts; ++q) { a = fminf(a, lds_min[q * N + c]); b = fmaxf(b, lds_max[q * N + c]); }
-      sum_min += a;
-      sum_max += b;
-    }
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    sum_min += __shfl_xor(sum_min, o, 64);
-    sum_max += __shfl_xor(sum_max, o, 64);
-  }
-  if (lane == 0) { red[wave][0] = sum_min; red[wave][1] = sum_max; }
-  __syncthreads();
-  if (tid < 2)
-    partial[(size_t)g * 4 + blockIdx.y * 2 + tid] = red[0][tid] + red[1][tid] + red[2][tid] + red[3][tid];
-}
-
 // Sums the (G, 4) partials over the groups in index order and scales them to means;
 // stats[4] is the router's auxiliary loss, which is always zero.
 __global__ __launch_bounds__(256) void soft_stats_finish_kernel(const float* __restrict__ partial,
@@ -1283,9 +928,10 @@ using namespace vmoe;
 
 extern "C" size_t vmoe_soft_route_workspace_bytes(const VmoeSoftRouteParams* p) {
   if (p == nullptr || p->D < 1 || p->N < 1) return 0;
-  // float32: (D, N) floats; bfloat16: the slots padded to a multiple of 32
-  const size_t padded = (size_t)p->D * ((p->N + 31) / 32 * 32) * 2;
-  return std::max((size_t)p->D * p->N * sizeof(float), padded);
+  // The slot parameters in fragment order: the slots padded to a multiple of 32, the width to 64
+  // (float32) or 128 (bfloat16).
+  const size_t size = p->dtype == VMOE_BF16 ? 2 : 4, wide = 256 / size;
+  return (p->D + wide - 1) / wide * wide * ((p->N + 31) / 32 * 32) * size;
 }
 
 // vmoe_soft_route; with `stats_partial` the routing launch also writes the (G, 4) partial
@@ -1309,58 +955,55 @@ static int soft_route_launch(const VmoeSoftRouteParams* p, vmoe_stream_t stream_
   hipStream_t stream = as_stream(stream_);
   // router.py:79-82: the scale multiplies whichever of the two operands is smaller.
   const int scale_x = ((int64_t)p->G * p->S * p->D < (int64_t)p->D * p->N) ? 1 : 0;
-  const SoftLds L = soft_lds_layout(p->D, SP, NP);
-  if (p->dtype == VMOE_BF16 && p->N <= 128 && p->N % 8 == 0 && soft_fast_width(p->D) && L.total <= 160 * 1024 && aligned16(p->dispatch_w) && aligned16(p->combine_w) &&
+  // Two roles per workgroup where the slot parameters of 32 slots fit a wave's registers
+  // (D <= 768) and two item tiles fit LDS beside the logits (tiles of 32 rows, else 16): 43 us for 256
+  // groups of 196 items x 768 and 128 slots, 84 for the row tiles of soft_route_tiles.h, which take
+  // everything else (D = 1024: 36 us for 64 such groups, 60 for a workgroup per group).
+  // (VMOE_SOFT_ROUTE_SINGLE_ROLE=1 in the environment keeps the row tiles: the switch behind the
+  // before / after figures)
+  const int tile_rows = soft_pipe_lds_layout(p->D, SP, NP, 32).total <= 160 * 1024 ? 32 : 16;
+  const SoftPipeLds PL = soft_pipe_lds_layout(p->D, SP, NP, tile_rows);
+  if (p->dtype == VMOE_BF16 && p->N <= 128 && p->N % 8 == 0 && soft_roles_width(p->D) && PL.total <= 160 * 1024 &&
+      getenv("VMOE_SOFT_ROUTE_SINGLE_ROLE") == nullptr && aligned16(p->dispatch_w) && aligned16(p->combine_w) &&
       (p->logits == nullptr || aligned16(p->logits))) {
-    // Two roles per workgroup where the slot parameters of 32 slots fit a wave's registers
-    // (D <= 768) and two item tiles fit LDS beside the logits (tiles of 32 rows, else 16).
-    // (VMOE_SOFT_ROUTE_SINGLE_ROLE=1 in the environment keeps the single-role kernel: the
-    // switch behind the before / after figures)
-    const int tile_rows = soft_pipe_lds_layout(p->D, SP, NP, 32).total <= 160 * 1024 ? 32 : 16;
-    const SoftPipeLds PL = soft_pipe_lds_layout(p->D, SP, NP, tile_rows);
-    if (p->D <= 768 && PL.total <= 160 * 1024 && getenv("VMOE_SOFT_ROUTE_SINGLE_ROLE") == nullptr) {
-      using Kern = void (*)(const bf16_t*, const bf16_t*, bf16_t*, bf16_t*, bf16_t*, float, int, int,
-                            int, int, int, SoftPipeLds, float*);
-      // (the partial sums come out of the register-resident dispatch softmax only)
-      // (VMOE_SOFT_STATS_SEPARATE=1 in the environment keeps the separate launches: the switch
-      // behind the before / after figures)
-      float* partial_out = SP <= 32 * kTailRows && getenv("VMOE_SOFT_STATS_SEPARATE") == nullptr
-                               ? stats_partial : nullptr;
-      if (wrote_partial != nullptr) *wrote_partial = partial_out != nullptr;
-      auto pick = [&](auto ksw) -> Kern {
-        constexpr int K = decltype(ksw)::value;
-        if (tile_rows == 32)
-          return scale_x ? soft_route_roles_kernel<K, 32, true> : soft_route_roles_kernel<K, 32, false>;
-        return scale_x ? soft_route_roles_kernel<K, 16, true> : soft_route_roles_kernel<K, 16, false>;
-      };
-      Kern kern = p->D == 768   ? pick(std::integral_constant<int, 24>{})
-                  : p->D == 512 ? pick(std::integral_constant<int, 16>{})
-                  : p->D == 384 ? pick(std::integral_constant<int, 12>{})
-                                : pick(std::integral_constant<int, 8>{});
-      hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), PL.total);
-      if (e != hipSuccess) return (int)e;
-      if (!p->workspace_prepared)
-        hipLaunchKernelGGL(soft_prep_mu_kernel<bf16_t>, dim3(NP), dim3(256), 0, stream,
-                           (const bf16_t*)p->mu, (bf16_t*)p->workspace, p->scale, !scale_x, p->D, p->N,
-                           p->D / 32);
-      hipLaunchKernelGGL(kern, dim3(p->G), dim3(kSrThreads), PL.total, stream, (const bf16_t*)p->x,
-                         (const bf16_t*)p->workspace, (bf16_t*)p->dispatch_w, (bf16_t*)p->combine_w,
-                         (bf16_t*)p->logits, p->scale, p->S, p->D, p->N, SP, NP, PL, partial_out);
-      return launch_status();
-    }
-    if (!p->workspace_prepared)
-      hipLaunchKernelGGL(soft_prep_mu_kernel<bf16_t>, dim3(p->N), dim3(256), 0, stream,
-                         (const bf16_t*)p->mu, (bf16_t*)p->workspace, p->scale, !scale_x, p->D, p->N);
-    auto kern = p->D == 1024 ? soft_route_bf16_kernel<32>
-                : p->D == 768 ? soft_route_bf16_kernel<24>
-                : p->D == 512 ? soft_route_bf16_kernel<16>
-                : p->D == 384 ? soft_route_bf16_kernel<12>
-                              : soft_route_bf16_kernel<8>;
-    hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), L.total);
+    using Kern = void (*)(const bf16_t*, const bf16_t*, bf16_t*, bf16_t*, bf16_t*, float, int, int,
+                          int, int, int, SoftPipeLds, float*);
+    // (the partial sums come out of the register-resident dispatch softmax only)
+    // (VMOE_SOFT_STATS_SEPARATE=1 in the environment keeps the separate launches: the switch
+    // behind the before / after figures)
+    float* partial_out = SP <= 32 * kTailRows && getenv("VMOE_SOFT_STATS_SEPARATE") == nullptr
+                             ? stats_partial : nullptr;
+    if (wrote_partial != nullptr) *wrote_partial = partial_out != nullptr;
+    auto pick = [&](auto ksw) -> Kern {
+      constexpr int K = decltype(ksw)::value;
+      if (tile_rows == 32)
+        return scale_x ? soft_route_roles_kernel<K, 32, true> : soft_route_roles_kernel<K, 32, false>;
+      return scale_x ? soft_route_roles_kernel<K, 16, true> : soft_route_roles_kernel<K, 16, false>;
+    };
+    Kern kern = p->D == 768   ? pick(std::integral_constant<int, 24>{})
+                : p->D == 512 ? pick(std::integral_constant<int, 16>{})
+                : p->D == 384 ? pick(std::integral_constant<int, 12>{})
+                              : pick(std::integral_constant<int, 8>{});
+    hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), PL.total);
     if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL(kern, dim3(p->G), dim3(kSrThreads), L.total, stream, (const bf16_t*)p->x,
+    if (!p->workspace_prepared)
+      hipLaunchKernelGGL(soft_prep_mu_kernel<bf16_t>, dim3(NP), dim3(256), 0, stream,
+                         (const bf16_t*)p->mu, (bf16_t*)p->workspace, p->scale, !scale_x, p->D, p->N,
+                         p->D / 32);
+    hipLaunchKernelGGL(kern, dim3(p->G), dim3(kSrThreads), PL.total, stream, (const bf16_t*)p->x,
                        (const bf16_t*)p->workspace, (bf16_t*)p->dispatch_w, (bf16_t*)p->combine_w,
-                       (bf16_t*)p->logits, p->scale, scale_x, p->S, p->D, p->N, SP, NP, L);
+                       (bf16_t*)p->logits, p->scale, p->S, p->D, p->N, SP, NP, PL, partial_out);
+  } else if (p->dtype == VMOE_BF16 ? soft::tiles_ok<bf16_t>(p->S, p->D, p->N)
+                                       : soft::tiles_ok<float>(p->S, p->D, p->N)) {
+    auto run = [&](auto zero) -> int {
+      using T = decltype(zero);
+      if (!p->workspace_prepared)
+        hipLaunchKernelGGL(soft_prep_mu_kernel<T>, dim3((p->N + 15) / 16 * 16), dim3(256), 0, stream, (const T*)p->mu,
+                           (T*)p->workspace, p->scale, !scale_x, p->D, p->N, soft::padded_steps<T>(p->D));
+      return soft::launch_tiles<T>((const T*)p->x, p->workspace, (T*)p->dispatch_w, (T*)p->combine_w, (T*)p->logits,
+                                   p->scale, scale_x, p->G, p->S, p->D, p->N, stream);
+    };
+    return p->dtype == VMOE_BF16 ? run(bf16_t{}) : run(float{});
   } else if (lds > 160 * 1024) {
     return VMOE_E_UNSUPPORTED;
   } else if (p->dtype == VMOE_BF16) {
@@ -1418,27 +1061,22 @@ extern "C" int vmoe_soft_router_stats(const VmoeSoftStatsParams* p, vmoe_stream_
     return VMOE_E_NULL;
   if (p->G < 1 || p->S < 1 || p->N < 1) return VMOE_E_SHAPE;
   if (p->dtype != VMOE_BF16 && p->dtype != VMOE_F32) return VMOE_E_DTYPE;
-  const int vec = p->dtype == VMOE_BF16 ? 8 : 4;
-  const int nc = p->N / vec;
-  const bool wide = p->N % vec == 0 && nc <= 64 && (nc & (nc - 1)) == 0 &&
-                    aligned16(p->combine_w) && aligned16(p->dispatch_w) && p->G <= 65535 * 32;
   hipStream_t s = as_stream(stream);
-  if (wide && p->dtype == VMOE_BF16)
-    hipLaunchKernelGGL(soft_stats_vec_kernel<bf16_t>, dim3(p->G, 2), dim3(256), 0, s,
-                       (const bf16_t*)p->combine_w, (const bf16_t*)p->dispatch_w, p->partial, p->S,
-                       p->N);
-  else if (wide)
-    hipLaunchKernelGGL(soft_stats_vec_kernel<float>, dim3(p->G, 2), dim3(256), 0, s,
-                       (const float*)p->combine_w, (const float*)p->dispatch_w, p->partial, p->S,
-                       p->N);
-  else if (p->dtype == VMOE_BF16)
-    hipLaunchKernelGGL(soft_stats_kernel<bf16_t>, dim3(p->G), dim3(256), 0, s,
-                       (const bf16_t*)p->combine_w, (const bf16_t*)p->dispatch_w, p->partial, p->S,
-                       p->N);
-  else
-    hipLaunchKernelGGL(soft_stats_kernel<float>, dim3(p->G), dim3(256), 0, s,
-                       (const float*)p->combine_w, (const float*)p->dispatch_w, p->partial, p->S,
-                       p->N);
+  int rc = p->dtype == VMOE_BF16
+                     ? soft::launch_stats<bf16_t>((const bf16_t*)p->combine_w, (const bf16_t*)p->dispatch_w, p->partial,
+                                                  p->G, p->S, p->N, s)
+                     : soft::launch_stats<float>((const float*)p->combine_w, (const float*)p->dispatch_w, p->partial,
+                                                 p->G, p->S, p->N, s);
+  if (rc == VMOE_E_UNSUPPORTED) {
+    if (p->dtype == VMOE_BF16)
+      hipLaunchKernelGGL(soft_stats_wide_kernel<bf16_t>, dim3(p->G), dim3(256), 0, s, (const bf16_t*)p->combine_w,
+                         (const bf16_t*)p->dispatch_w, p->partial, p->S, p->N);
+    else
+      hipLaunchKernelGGL(soft_stats_wide_kernel<float>, dim3(p->G), dim3(256), 0, s, (const float*)p->combine_w,
+                         (const float*)p->dispatch_w, p->partial, p->S, p->N);
+    rc = launch_status();
+  }
+  if (rc != VMOE_OK) return rc;
   hipLaunchKernelGGL(soft_stats_finish_kernel, dim3(1), dim3(256), 0, s, p->partial, p->stats, p->G,
                      1.0f / ((float)p->G * (float)p->S), 1.0f / ((float)p->G * (float)p->N));
   return launch_status();
