@@ -644,6 +644,43 @@ def test_einsum_dispatch_combine(K, G, S, E, C, D, wdtype, ddtype):
   assert_close(to_np(out), O.cast(d.combine(y), out_dtype), tol, "einsum combine")
 
 
+@pytest.mark.parametrize("G,S,E,C,D,offset", [
+    (8, 196, 128, 2, 768, 0),    # the Soft MoE router's default capacity: 256 slots
+    (3, 256, 1, 129, 72, 0),     # one past the 128-slot form; an odd row length
+    (2, 257, 5, 1, 64, 0),       # one past 256 items: the items halved between waves
+    (9, 512, 4, 128, 136, 0),    # the longest contraction of both directions
+    (2, 513, 3, 171, 40, 0),     # one past it: the generic kernel
+    (4, 31, 7, 63, 200, 0),      # 441 slots, a lone partial row tile
+    (5, 300, 19, 1, 96, 3),      # weights at an address that is a multiple of 2 only
+    (8, 16, 8, 2, 8, 1),
+    (1, 1, 1, 1, 8, 0),
+])
+def test_einsum_bf16_long_rows(K, G, S, E, C, D, offset):
+  """bfloat16 dispatch / combine over contractions of any length and rows of weights that start
+  anywhere.  Products are exact in float32, so against the float32 oracle the result is off by its own
+  rounding to bfloat16 (half of the last of 8 bits: 2**-8 of the value) and the roundings of both sums (2**-24 of the sum of
+  magnitudes per term each)."""
+  rng = np.random.default_rng(G * S + E)
+  N = E * C
+  w = O.cast(O.softmax(rng.standard_normal((G, S, N)).astype(np.float32) * 2), O.BF16)
+  x = O.cast(rng.standard_normal((G, S, D)), O.BF16)
+  y = O.cast(rng.standard_normal((E, G * C, D)), O.BF16)
+  buf = torch.empty(w.size + offset, dtype=torch.bfloat16, device="cuda")
+  wd = buf[offset:].view(G, S, E, C)
+  wd.copy_(to_dev(w.reshape(G, S, E, C), O.BF16))
+  d = O.EinsumDispatcher(w.reshape(G, S, E, C), w.reshape(G, S, E, C))
+
+  def check(got, want, mag, terms, what):
+    err = np.abs(got.astype(np.float64) - want)
+    bound = 2.0 ** -8 * np.abs(want) + 2 * terms * 2.0 ** -24 * mag + 1e-30
+    assert (err <= bound).all(), (what, float((err / bound).max()))
+
+  got = to_np(K.einsum_dispatch(wd, to_dev(x, O.BF16), torch.bfloat16)).reshape(E, G * C, D)
+  check(got, d.dispatch(x).astype(np.float64), d.dispatch(np.abs(x)), S, "dispatch")
+  got = to_np(K.einsum_combine(wd, to_dev(y, O.BF16).view(E * G * C, D), torch.bfloat16))
+  check(got, d.combine(y).astype(np.float64), d.combine(np.abs(y)), N, "combine")
+
+
 def test_einsum_golden_and_bool_weights(K, goldens):
   data = np.asarray(goldens["dispatcher_data"]["data"], np.float32)
   for case in ("dispatcher_experts_divide_groups", "dispatcher_groups_divide_experts"):

@@ -25,7 +25,6 @@ namespace ein {
 constexpr int kTileD = 64;                  // data / output columns per tile
 constexpr int kStageLd = kTileD + 8;        // row pitch of the staged output (elements)
 constexpr int kStageElems = 32 * kStageLd;  // one wave's staging region
-constexpr int kThreads = 256;
 
 // Rotation of the 16-byte k chunks of tile row c.  Rows are a multiple of 256
 // bytes long, so the rotation alone decides the bank group: 16 consecutive rows
@@ -44,6 +43,32 @@ __device__ __forceinline__ void load_block(uint4 (&r)[8], const bf16_t* __restri
     r[i] = make_uint4(0, 0, 0, 0);
     if (rowidx[i] >= 0 && col < D)
       r[i] = *reinterpret_cast<const uint4*>(data + (size_t)rowidx[i] * D + col);
+  }
+}
+
+// Eight consecutive values at p, of which n belong to the row (the rest reads as zero).  p need not
+// be aligned: rows of weights start wherever E*C puts them, and a 16-byte global load takes any
+// address of its element type.
+__device__ __forceinline__ uint4 load_row_piece(const bf16_t* __restrict__ p, int n) {
+  uint4 r = make_uint4(0, 0, 0, 0);
+  if (n >= 8) {
+    __builtin_memcpy(&r, p, 16);
+  } else if (n > 0) {
+    uint32_t v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = i < n ? p[i] : 0u;
+    r = make_uint4(v[0] | v[1] << 16, v[2] | v[3] << 16, v[4] | v[5] << 16, v[6] | v[7] << 16);
+  }
+  return r;
+}
+
+// load_block for rows of any length N (weights).
+__device__ __forceinline__ void load_weight_block(uint4 (&r)[8], const bf16_t* __restrict__ w,
+                                                  const int (&rowidx)[8], int col, int N) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    r[i] = make_uint4(0, 0, 0, 0);
+    if (rowidx[i] >= 0 && col < N) r[i] = load_row_piece(w + (size_t)rowidx[i] * N + col, N - col);
   }
 }
 
@@ -86,6 +111,24 @@ __device__ __forceinline__ void stage_tile(const floatx16 (&acc)[2], bf16_t* so,
     }
 }
 
+constexpr int kXchElems = 32 * kWave;       // a wave's accumulators in float32
+
+// Sums over the two halves of k: the second half's waves leave theirs in xch, the first half's (first)
+// add them.  Every wave of the workgroup calls it.  True for the waves that hold the result.
+__device__ __forceinline__ bool join_halves(floatx16 (&acc)[2], float* xch, bool first, int lane) {
+  if (!first) {
+#pragma unroll
+    for (int v = 0; v < 32; ++v) xch[v * kWave + lane] = acc[v / 16][v % 16];
+  }
+  wait_lgkmcnt0();
+  raw_barrier();
+  if (first) {
+#pragma unroll
+    for (int v = 0; v < 32; ++v) acc[v / 16][v % 16] += xch[v * kWave + lane];
+  }
+  return first;
+}
+
 // Staged rows -> global rows orow[p] (row p*8 + lane/8 of the wave tile), 16 bytes per lane.
 __device__ __forceinline__ void store_staged(const bf16_t* so, bf16_t* __restrict__ out,
                                              const int (&orow)[4], int lane, int d0, int D) {
@@ -109,19 +152,22 @@ __device__ __forceinline__ bool map_group(int G, int per_group, int& g, int& rem
 }
 
 // out[slot(g, n), :] = sum_s w[g, s, n] * data[g, s, :]   (n = e*C + c)
-// A workgroup owns 128 buffer rows n of one group (wave = 32 of them) and a run
-// of column tiles; S <= 16 * KSMAX.  W_BLOCKS: the weights (k-major as well) go
-// through the same transposing LDS tile, 64 buffer rows at a time; otherwise
-// (E*C not a multiple of 8, or unaligned) each lane gathers its values one by one.
-template <int KSMAX, bool W_BLOCKS>
-__global__ __launch_bounds__(kThreads, 2) void einsum_dispatch_bf16_kernel(
+// A workgroup owns 128 buffer rows n of one group and a run of column tiles; the weights (k-major as
+// well) go through the same transposing LDS tile, 64 buffer rows at a time, and stay in registers.
+// S <= 16 * KSMAX * KSPLIT: a wave holds the weights of 32 rows x 16 * KSMAX items, and with KSPLIT = 2
+// four more waves hold those of the other half of the items and hand their sums over in LDS (a wave
+// with all of 512 items in registers spills).
+template <int KSMAX, int KSPLIT>
+__global__ __launch_bounds__(KSPLIT * 256, 2) void einsum_dispatch_bf16_kernel(
     const bf16_t* __restrict__ w, const bf16_t* __restrict__ data, bf16_t* __restrict__ out, int G,
     int S, int E, int C, int D, int KS, int KCP, int d_splits, int n_blocks, int tiles_per_split) {
   extern __shared__ __align__(16) unsigned char smem[];
   bf16_t* bt = reinterpret_cast<bf16_t*>(smem);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) & 3;
+  const int ks0 = (tid >> 8) * KSMAX;            // first k step (16 items) of this wave
   const int m = lane & 31, h = lane >> 5;
   bf16_t* so = reinterpret_cast<bf16_t*>(smem + bt_bytes(KCP)) + wave * kStageElems;
+  float* xch = reinterpret_cast<float*>(smem + bt_bytes(KCP) + 4 * kStageElems * sizeof(bf16_t)) + wave * kXchElems;
   int g, rem;
   if (!map_group(G, d_splits * n_blocks, g, rem)) return;
   const int nb = rem / d_splits, ds = rem - nb * d_splits;
@@ -136,12 +182,12 @@ __global__ __launch_bounds__(kThreads, 2) void einsum_dispatch_bf16_kernel(
   const int t0 = ds * tiles_per_split, t1 = min(t0 + tiles_per_split, total_tiles);
   uint4 pre0[8], pre1[8];
 
-  // Weights of this wave's 32 buffer rows, all k, kept in registers.
+  // Weights of this wave's 32 buffer rows and its share of k, kept in registers.
   bf16x8 wf[KSMAX];
-  if constexpr (W_BLOCKS) {
+  {
     uint4 wa[8], wb[8];
-    load_block(wa, w, rowidx, nb * 128 + cc * 8, N);
-    load_block(wb, w, rowidx, nb * 128 + 64 + cc * 8, N);
+    load_weight_block(wa, w, rowidx, nb * 128 + cc * 8, N);
+    load_weight_block(wb, w, rowidx, nb * 128 + 64 + cc * 8, N);
     load_block(pre0, data, rowidx, t0 * kTileD + cc * 8, D);
     if (t0 + 1 < t1) load_block(pre1, data, rowidx, (t0 + 1) * kTileD + cc * 8, D);
 #pragma unroll
@@ -153,29 +199,11 @@ __global__ __launch_bounds__(kThreads, 2) void einsum_dispatch_bf16_kernel(
         const int c = (wave & 1) * 32 + m;
 #pragma unroll
         for (int ks = 0; ks < KSMAX; ++ks)
-          if (ks < KS) wf[ks] = read_frag(bt, c, (wave & 1) ? rc1 : rc0, 2 * ks + h, KCP);
+          if (ks0 + ks < KS) wf[ks] = read_frag(bt, c, (wave & 1) ? rc1 : rc0, 2 * (ks0 + ks) + h, KCP);
       }
       wait_lgkmcnt0();
       raw_barrier();
     }
-  } else {
-    const int n = nb * 128 + wave * 32 + m;
-    const bf16_t* wg = w + (size_t)g * S * N;
-#pragma unroll
-    for (int ks = 0; ks < KSMAX; ++ks) {
-      uint32_t pk[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int k = ks * 16 + h * 8 + 2 * q;
-        uint32_t lo = 0, hi = 0;
-        if (n < N && k < S) lo = wg[(size_t)k * N + n];
-        if (n < N && k + 1 < S) hi = wg[(size_t)(k + 1) * N + n];
-        pk[q] = lo | (hi << 16);
-      }
-      wf[ks] = __builtin_bit_cast(bf16x8, make_uint4(pk[0], pk[1], pk[2], pk[3]));
-    }
-    load_block(pre0, data, rowidx, t0 * kTileD + cc * 8, D);
-    if (t0 + 1 < t1) load_block(pre1, data, rowidx, (t0 + 1) * kTileD + cc * 8, D);
   }
 
   int orow[4];
@@ -199,16 +227,18 @@ __global__ __launch_bounds__(kThreads, 2) void einsum_dispatch_bf16_kernel(
       for (int v = 0; v < 16; ++v) acc[jj][v] = 0.f;
 #pragma unroll
     for (int ks = 0; ks < KSMAX; ++ks) {
-      if (ks < KS) {
-        const bf16x8 f0 = read_frag(bt, m, rc0, 2 * ks + h, KCP);
-        const bf16x8 f1 = read_frag(bt, 32 + m, rc1, 2 * ks + h, KCP);
+      if (ks0 + ks < KS) {
+        const bf16x8 f0 = read_frag(bt, m, rc0, 2 * (ks0 + ks) + h, KCP);
+        const bf16x8 f1 = read_frag(bt, 32 + m, rc1, 2 * (ks0 + ks) + h, KCP);
         acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f0, wf[ks], acc[0], 0, 0, 0);
         acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f1, wf[ks], acc[1], 0, 0, 0);
       }
     }
     mfma_result_fence();
-    stage_tile(acc, so, m, h);
-    store_staged(so, out, orow, lane, t * kTileD, D);
+    if (KSPLIT == 1 || join_halves(acc, xch, ks0 == 0, lane)) {
+      stage_tile(acc, so, m, h);
+      store_staged(so, out, orow, lane, t * kTileD, D);
+    }
     wait_lgkmcnt0();
     raw_barrier();
   };
@@ -218,18 +248,27 @@ __global__ __launch_bounds__(kThreads, 2) void einsum_dispatch_bf16_kernel(
   }
 }
 
-// out[g, s, :] = sum_n w[g, s, n] * data[slot(g, n), :]   (n = e*C + c, N = E*C <= 128)
-// A workgroup owns 256 item rows of one group (wave = 64 of them, as two 32-row
-// tiles computed one after the other) and a run of column tiles.
-__global__ __launch_bounds__(kThreads, 2) void einsum_combine_bf16_kernel(
+// out[g, s, :] = sum_n w[g, s, n] * data[slot(g, n), :]   (n = e*C + c)
+// A workgroup owns 128 * ROWT item rows of one group (wave = ROWT 32-row tiles, computed one after the
+// other) and a run of column tiles.  N <= 16 * KSMAX * KSPLIT, KSPLIT as above.
+//
+// The weights of a wave's items stay in registers, so the longer a row of them, the fewer items per
+// wave: up to 128 slots two tiles, up to 256 one, up to 512 one with the slots halved between waves.
+// 64 groups of 196 items with 256 slots of width 768 (the Soft MoE router's default capacity): 24 us,
+// 2.4 TB/s of its 59 MB, where the float32 kernel that took every row of more than 128 slots needs 144.
+template <int KSMAX, int ROWT, int KSPLIT>
+__global__ __launch_bounds__(KSPLIT * 256, 2) void einsum_combine_bf16_kernel(
     const bf16_t* __restrict__ w, const bf16_t* __restrict__ data, bf16_t* __restrict__ out, int G,
     int S, int E, int C, int D, int KS, int d_splits, int row_blocks, int tiles_per_split) {
-  constexpr int KSMAX = 8, KCP = 16;
+  static_assert(KSPLIT == 1 || ROWT == 1, "the exchange region holds one row tile per wave");
+  constexpr int KCP = 2 * KSMAX * KSPLIT;
   extern __shared__ __align__(16) unsigned char smem[];
   bf16_t* bt = reinterpret_cast<bf16_t*>(smem);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) & 3;
+  const int ks0 = (tid >> 8) * KSMAX;            // first k step (16 slots) of this wave
   const int m = lane & 31, h = lane >> 5;
   bf16_t* so = reinterpret_cast<bf16_t*>(smem + bt_bytes(KCP)) + wave * kStageElems;
+  float* xch = reinterpret_cast<float*>(smem + bt_bytes(KCP) + 4 * kStageElems * sizeof(bf16_t)) + wave * kXchElems;
   int g, rem;
   if (!map_group(G, d_splits * row_blocks, g, rem)) return;
   const int rb = rem / d_splits, ds = rem - rb * d_splits;
@@ -248,25 +287,24 @@ __global__ __launch_bounds__(kThreads, 2) void einsum_combine_bf16_kernel(
   load_block(pre0, data, rowidx, t0 * kTileD + cc * 8, D);
   if (t0 + 1 < t1) load_block(pre1, data, rowidx, (t0 + 1) * kTileD + cc * 8, D);
 
-  // Combine weights of this wave's two 32-row tiles, all k, straight from memory
+  // Combine weights of this wave's 32-row tiles and its share of k, straight from memory
   // (k is the fast index of w here).
-  const int row_base = rb * 256 + wave * 64;
-  bf16x8 wf[2][KSMAX];
+  const int row_base = (rb * 4 + wave) * ROWT * 32;
+  bf16x8 wf[ROWT][KSMAX];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < ROWT; ++i) {
     const int s = row_base + i * 32 + m;
 #pragma unroll
     for (int ks = 0; ks < KSMAX; ++ks) {
-      const int k = ks * 16 + h * 8;
+      const int k = (ks0 + ks) * 16 + h * 8;
       uint4 raw = make_uint4(0, 0, 0, 0);
-      if (s < S && k < N) raw = *reinterpret_cast<const uint4*>(w + ((size_t)g * S + s) * N + k);
+      if (s < S && k < N) raw = load_row_piece(w + ((size_t)g * S + s) * N + k, N - k);
       wf[i][ks] = __builtin_bit_cast(bf16x8, raw);
     }
   }
-  const bool tile_on[2] = {row_base < S, row_base + 32 < S};
-  int orow[2][4];
+  int orow[ROWT][4];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < ROWT; ++i)
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
       const int s = row_base + i * 32 + p * 8 + (lane >> 3);
@@ -280,8 +318,8 @@ __global__ __launch_bounds__(kThreads, 2) void einsum_combine_bf16_kernel(
     raw_barrier();
     if (t + 2 < t1) load_block(pre, data, rowidx, (t + 2) * kTileD + cc * 8, D);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      if (tile_on[i]) {
+    for (int i = 0; i < ROWT; ++i) {
+      if (KSPLIT > 1 || row_base + i * 32 < S) {    // (halves that join meet at a barrier)
         floatx16 acc[2];
 #pragma unroll
         for (int jj = 0; jj < 2; ++jj)
@@ -289,16 +327,18 @@ __global__ __launch_bounds__(kThreads, 2) void einsum_combine_bf16_kernel(
           for (int v = 0; v < 16; ++v) acc[jj][v] = 0.f;
 #pragma unroll
         for (int ks = 0; ks < KSMAX; ++ks) {
-          if (ks < KS) {
-            const bf16x8 f0 = read_frag(bt, m, rc0, 2 * ks + h, KCP);
-            const bf16x8 f1 = read_frag(bt, 32 + m, rc1, 2 * ks + h, KCP);
+          if (ks0 + ks < KS) {
+            const bf16x8 f0 = read_frag(bt, m, rc0, 2 * (ks0 + ks) + h, KCP);
+            const bf16x8 f1 = read_frag(bt, 32 + m, rc1, 2 * (ks0 + ks) + h, KCP);
             acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f0, wf[i][ks], acc[0], 0, 0, 0);
             acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f1, wf[i][ks], acc[1], 0, 0, 0);
           }
         }
         mfma_result_fence();
-        stage_tile(acc, so, m, h);
-        store_staged(so, out, orow[i], lane, t * kTileD, D);
+        if (KSPLIT == 1 || join_halves(acc, xch, ks0 == 0, lane)) {
+          stage_tile(acc, so, m, h);
+          store_staged(so, out, orow[i], lane, t * kTileD, D);
+        }
       }
     }
     wait_lgkmcnt0();
@@ -321,33 +361,40 @@ inline void split_columns(int D, int64_t groups_x_blocks, int& d_splits, int& ti
   d_splits = (tiles + tiles_per_split - 1) / tiles_per_split;
 }
 
-inline bool dispatch_fast_ok(const VmoeEinsumParams* p) {
+constexpr int kMaxContraction = 512;   // 32 k steps; eight waves' threads transpose eight k each
+
+inline bool all_bf16(const VmoeEinsumParams* p) {
   return p->w_dtype == VMOE_W_BF16 && p->data_dtype == VMOE_BF16 && p->out_dtype == VMOE_BF16 &&
-         p->D % 8 == 0 && aligned16(p->data) && aligned16(p->out) && p->S <= 256;
+         p->D % 8 == 0 && aligned16(p->data) && aligned16(p->out);
 }
 
+inline bool dispatch_fast_ok(const VmoeEinsumParams* p) { return all_bf16(p) && p->S <= kMaxContraction; }
+
 inline bool combine_fast_ok(const VmoeEinsumParams* p) {
-  const int64_t N = (int64_t)p->E * p->C;
-  return p->w_dtype == VMOE_W_BF16 && p->data_dtype == VMOE_BF16 && p->out_dtype == VMOE_BF16 &&
-         p->D % 8 == 0 && aligned16(p->data) && aligned16(p->out) && aligned16(p->w) &&
-         N % 8 == 0 && N <= 128;
+  return all_bf16(p) && (int64_t)p->E * p->C <= kMaxContraction;
+}
+
+inline size_t lds_bytes(int KCP, int k_split) {
+  return (size_t)kTileD * KCP * 16 + 4 * kStageElems * sizeof(bf16_t) +
+         (k_split > 1 ? 4 * kXchElems * sizeof(float) : 0);
 }
 
 inline int launch_dispatch_fast(const VmoeEinsumParams* p, hipStream_t stream) {
   const int N = p->E * p->C;
-  const int KS = (p->S + 15) / 16, KCP = KS <= 8 ? 16 : 32;
+  const int KS = (p->S + 15) / 16, KCP = KS <= 8 ? 16 : KS <= 16 ? 32 : 64;
+  const int k_split = KS <= 16 ? 1 : 2;
   const int n_blocks = (N + 127) / 128;
   int d_splits, tiles_per_split;
-  split_columns(p->D, (int64_t)p->G * n_blocks, d_splits, tiles_per_split);
+  split_columns(p->D, (int64_t)p->G * n_blocks * k_split, d_splits, tiles_per_split);
   const int64_t blocks = (int64_t)((p->G + kNumXcd - 1) / kNumXcd) * kNumXcd * d_splits * n_blocks;
   if (blocks >= INT32_MAX) return VMOE_E_OVERFLOW;
-  const size_t lds = (size_t)kTileD * KCP * 16 + 4 * kStageElems * sizeof(bf16_t);
-  const bool w_blocks = N % 8 == 0 && aligned16(p->w);
-  auto kern = KS <= 13 ? (w_blocks ? einsum_dispatch_bf16_kernel<13, true>
-                                   : einsum_dispatch_bf16_kernel<13, false>)
-                       : (w_blocks ? einsum_dispatch_bf16_kernel<16, true>
-                                   : einsum_dispatch_bf16_kernel<16, false>);
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kThreads), lds, stream,
+  const size_t lds = lds_bytes(KCP, k_split);
+  auto kern = KS <= 13   ? einsum_dispatch_bf16_kernel<13, 1>
+              : KS <= 16 ? einsum_dispatch_bf16_kernel<16, 1>
+                         : einsum_dispatch_bf16_kernel<16, 2>;
+  hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
+  if (e != hipSuccess) return (int)e;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(k_split * 256), lds, stream,
                      (const bf16_t*)p->w, (const bf16_t*)p->data, (bf16_t*)p->out, p->G, p->S, p->E,
                      p->C, p->D, KS, KCP, d_splits, n_blocks, tiles_per_split);
   return launch_status();
@@ -355,14 +402,21 @@ inline int launch_dispatch_fast(const VmoeEinsumParams* p, hipStream_t stream) {
 
 inline int launch_combine_fast(const VmoeEinsumParams* p, hipStream_t stream) {
   const int N = p->E * p->C;
-  const int KS = (N + 15) / 16;
-  const int row_blocks = (p->S + 255) / 256;
+  const int KS = (N + 15) / 16, KCP = KS <= 8 ? 16 : KS <= 16 ? 32 : 64;
+  const int k_split = KS <= 16 ? 1 : 2;
+  const int rows = KS <= 8 ? 256 : 128;
+  const int row_blocks = (p->S + rows - 1) / rows;
   int d_splits, tiles_per_split;
-  split_columns(p->D, (int64_t)p->G * row_blocks, d_splits, tiles_per_split);
+  split_columns(p->D, (int64_t)p->G * row_blocks * k_split, d_splits, tiles_per_split);
   const int64_t blocks = (int64_t)((p->G + kNumXcd - 1) / kNumXcd) * kNumXcd * d_splits * row_blocks;
   if (blocks >= INT32_MAX) return VMOE_E_OVERFLOW;
-  const size_t lds = (size_t)kTileD * 16 * 16 + 4 * kStageElems * sizeof(bf16_t);
-  hipLaunchKernelGGL(einsum_combine_bf16_kernel, dim3((unsigned)blocks), dim3(kThreads), lds, stream,
+  const size_t lds = lds_bytes(KCP, k_split);
+  auto kern = KS <= 8    ? einsum_combine_bf16_kernel<8, 2, 1>
+              : KS <= 16 ? einsum_combine_bf16_kernel<16, 1, 1>
+                         : einsum_combine_bf16_kernel<16, 1, 2>;
+  hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
+  if (e != hipSuccess) return (int)e;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(k_split * 256), lds, stream,
                      (const bf16_t*)p->w, (const bf16_t*)p->data, (bf16_t*)p->out, p->G, p->S, p->E,
                      p->C, p->D, KS, d_splits, row_blocks, tiles_per_split);
   return launch_status();
