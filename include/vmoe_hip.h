@@ -176,6 +176,15 @@ typedef struct {
 } VmoeTopItemsParams;
 int vmoe_top_items_per_expert(const VmoeTopItemsParams* p, vmoe_stream_t stream);
 
+/* The same with the monitoring scalars of vmoe/moe.py:681-692 per group (p->sel_minmax is
+ * required): items_minmax (2, G) int32, the fewest and most experts that took an item;
+ * gate_minmax (2, G) in p->dtype, the smallest and largest selected gate; ratios
+ * (floor(log2 E) + 2, G) float32, the share of items taken by at least 1, 2, 4, ..., 2^floor(log2 E)
+ * and E experts.  rows_per_expert (optional, (E,) int32) is set to G*C, what vmoe_expert_mlp takes
+ * beside slot_token as x_rows when C <= S (every slot is filled). */
+int vmoe_top_items_metrics(const VmoeTopItemsParams* p, int32_t* items_minmax, void* gate_minmax,
+                           float* ratios, int32_t* rows_per_expert, vmoe_stream_t stream);
+
 /* Builds the two slot maps from hand-made (expert, position) indices, as
  * vmoe/moe.py:190-197 and :202-206 interpret them: entries with expert >= E or
  * position >= C are dropped.  Negative entries are counted in

@@ -219,6 +219,76 @@ def test_top_items_per_expert_vs_oracle(moe, G, S, E, C, dtype, ties):
   assert_close(to_np(got_comb), ref.combine(expert_out), rtol, "combine")
 
 
+@pytest.mark.parametrize("G,S,E,C,dtype,ties", [
+    (2, 511, 5, 100, O.BF16, False),    # 512 keys: the smallest group ranked by counting
+    (1, 1024, 9, 1024, O.BF16, True),   # everything is taken, a few long segments of equal gates
+    (1, 8191, 3, 60, O.BF16, False),    # the largest
+    (3, 65, 300, 7, O.BF16, False),     # ranks of 32 items turned around at a time; a last block of one
+    (1, 3, 20000, 2, O.F32, False),     # one item at a time
+    (1, 1, 1, 1, O.BF16, False),
+])
+def test_top_items_per_expert_edges(moe, G, S, E, C, dtype, ties):
+  test_top_items_per_expert_vs_oracle(moe, G, S, E, C, dtype, ties)
+
+
+def test_top_items_per_expert_bfloat16_gates_out_of_range(moe):
+  """A column with a negative zero, a negative gate or a gate above 1 takes the sort, the others the
+  counting rank."""
+  g = O.cast(np.tile(np.linspace(0, 1, 600, dtype=np.float32)[:, None], (1, 4)), O.BF16).copy()
+  g[300, 0], g[301, 1], g[302, 2] = -0.0, -1.0, 1.5
+  d, m = moe.get_top_items_per_expert_dispatcher(to_dev(g[None], O.BF16), name="einsum", capacity=590)
+  _, dw, want = O.top_items_per_expert_einsum(g, 590)
+  np.testing.assert_array_equal(to_np(d.dispatch_weights)[0].astype(bool), dw)
+  for k, v in want.items():
+    assert float(m[k][0]) == pytest.approx(float(v), rel=1e-6), k
+
+
+@pytest.mark.parametrize("G,S,E,D,M,C,dtype", [
+    (2, 196, 8, 64, 96, 50, O.BF16),
+    (3, 49, 12, 32, 64, 5, O.F32),
+    (1, 70, 5, 40, 48, 20, O.BF16),      # a width the first product does not gather
+])
+def test_experts_choice_layer_equals_dispatch_and_combine(G, S, E, D, M, C, dtype):
+  """The layer, whose experts fetch their items themselves, against dispatch -> experts -> combine."""
+  from vmoe_amd.nn import vit_moe
+  rng = np.random.default_rng(S)
+  x = to_dev(O.cast(rng.standard_normal((G, S, D)), dtype), dtype)
+  mlp = {"Dense_0": {"kernel": to_dev(O.cast(rng.standard_normal((E, D, M)) / np.sqrt(D), dtype), dtype),
+                     "bias": to_dev(O.cast(rng.standard_normal((E, M)) * .1, dtype), dtype)},
+         "Dense_1": {"kernel": to_dev(O.cast(rng.standard_normal((E, M, D)) / np.sqrt(M), dtype), dtype),
+                     "bias": to_dev(O.cast(rng.standard_normal((E, D)) * .1, dtype), dtype)}}
+  router = {"dense": {"kernel": to_dev((rng.standard_normal((D, E)) / np.sqrt(D)).astype(np.float32))}}
+  layer = vit_moe.MlpMoeBlock(mlp_dim=M, num_experts=E, group_size=S, deterministic=True, dtype=tdtype(dtype),
+                              router=dict(name="NoisyTopItemsPerExpertRouter",
+                                          dispatcher=dict(name="einsum", capacity=C)))
+  out, _ = layer.apply({"params": {"Router": router, "Mlp": mlp}}, x)
+  dispatcher, _ = layer.create_router().apply({"params": router}, x)
+  expert = vit_moe.MlpBlock(mlp_dim=M, deterministic=True, dtype=tdtype(dtype))
+  want = dispatcher.combine(expert.apply_experts({"params": mlp}, dispatcher.dispatch(x)))
+  assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("K_", [1, 3, 4, 8, 9, 64, 65, 256, 257])
+@pytest.mark.parametrize("dtype", [O.F32, O.BF16])
+def test_combine_any_number_of_choices(K_, dtype):
+  """Sums in choice order with one rounding per choice (the product of two float32 values is exact in
+  float64), whatever the number of choices."""
+  from vmoe_amd import kernels as K
+  rng = np.random.default_rng(K_)
+  T, D, slots = 21, 40, 50
+  y = O.cast(rng.standard_normal((slots, D)), dtype)
+  ts = np.where(rng.random((T, K_)) < 0.3, rng.integers(0, slots, (T, K_)), -1).astype(np.int32)
+  ts[3] = -1
+  ts[4] = rng.integers(0, slots, K_)
+  w = rng.standard_normal((T, K_)).astype(np.float32)
+  want = np.zeros((T, D), np.float32)
+  for k in range(K_):
+    on = ts[:, k] >= 0
+    want[on] = want[on] + w[on, k:k + 1].astype(np.float64) * y[ts[on, k]]
+  got = to_np(K.combine(to_dev(y, dtype), to_dev(ts), to_dev(w)))
+  np.testing.assert_array_equal(got, O.cast(want, dtype))
+
+
 def test_top_items_per_expert_capacity_factor_and_errors(moe):
   gates = torch.softmax(torch.randn((2, 64, 8), device=dev()), -1)
   d, _ = moe.get_top_items_per_expert_dispatcher(gates, name="einsum", capacity_factor=1.0)

@@ -21,7 +21,8 @@ namespace {
 
 constexpr int kRowsPerBlock = 8;   // item rows (or slot rows) moved by one workgroup
 constexpr int kMoveThreads = 256;
-constexpr int kMaxK = 8;           // choices per item held in LDS; larger K takes the generic kernels
+constexpr int kMaxK = 8;           // dispatch: choices per item held in LDS; larger K takes the generic kernel
+constexpr int kListedK = 256;      // combine: the same
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
@@ -145,8 +146,8 @@ __global__ __launch_bounds__(kMoveThreads) void combine_kernel(
     const float* __restrict__ weights, uint4* __restrict__ out, int num_items, int num_slots,
     int K, int cpr, uint32_t magic) {
   constexpr int N = Chunk<T>::n;
-  __shared__ int32_t slots[kRowsPerBlock * kMaxK];
-  __shared__ float wts[kRowsPerBlock * kMaxK];
+  __shared__ int32_t slots[kRowsPerBlock * 2];
+  __shared__ float wts[kRowsPerBlock * 2];
   const int tid = threadIdx.x;
   const int t0 = blockIdx.x * kRowsPerBlock;
   if (tid < kRowsPerBlock * K) {
@@ -179,17 +180,76 @@ __global__ __launch_bounds__(kMoveThreads) void combine_kernel(
         acc[j] = __fadd_rn(p0, p1);
       }
     } else {
+      const int slot = slots[r];
+      float a[N];
+      if (slot >= 0) Chunk<T>::unpack(load_stream(y + (size_t)slot * cpr + ch), a);
 #pragma unroll
-      for (int j = 0; j < N; ++j) acc[j] = 0.f;
-      for (int k = 0; k < K; ++k) {
-        const int slot = slots[r * K + k];
-        if (slot < 0) continue;
-        const float w = wts[r * K + k];
-        float a[N];
-        Chunk<T>::unpack(load_stream(y + (size_t)slot * cpr + ch), a);
-#pragma unroll
-        for (int j = 0; j < N; ++j) acc[j] = __fadd_rn(acc[j], __fmul_rn(w, a[j]));
+      for (int j = 0; j < N; ++j) acc[j] = slot >= 0 ? __fadd_rn(0.f, __fmul_rn(wts[r], a[j])) : 0.f;
+    }
+    store_stream(out + (size_t)(t0 + r) * cpr + ch, Chunk<T>::pack(acc));
+  }
+}
+
+// The same for more choices than two, of which few are kept (experts choice: K = E, an item is taken
+// by two of 32 experts).  A wave lists an item's kept choices in order (a ballot per 64 of them), then
+// the workgroup's rows are walked as in combine_kernel, four reads in flight before their sums, which
+// are taken in choice order with fused multiply-adds.  12 544 items x 768 with 32 choices, 25 600 kept: 13 us
+// (4.7 TB/s), 38 for a wave per item that reads one row after the other.
+template <typename T>
+__global__ __launch_bounds__(kMoveThreads) void combine_listed_kernel(
+    const uint4* __restrict__ y, const int32_t* __restrict__ token_slot,
+    const float* __restrict__ weights, uint4* __restrict__ out, int num_items, int num_slots,
+    int K, int cpr, uint32_t magic) {
+  constexpr int N = Chunk<T>::n;
+  extern __shared__ __align__(16) unsigned char smem[];
+  int32_t* slots = reinterpret_cast<int32_t*>(smem);                       // (kRowsPerBlock, K)
+  float* wts = reinterpret_cast<float*>(smem) + kRowsPerBlock * K;
+  __shared__ int32_t kept[kRowsPerBlock];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int t0 = blockIdx.x * kRowsPerBlock;
+  for (int r = wave; r < kRowsPerBlock; r += kMoveThreads / kWave) {
+    int n = 0;
+    for (int k0 = 0; k0 < K && t0 + r < num_items; k0 += kWave) {
+      const int k = k0 + lane;
+      const size_t at = (size_t)(t0 + r) * K + k;
+      const int slot = k < K ? checked_slot(token_slot[at], num_slots) : -1;
+      const float w = k < K ? weights[at] : 0.f;
+      const uint64_t on = __ballot(slot >= 0);
+      if (slot >= 0) {
+        const int i = r * K + n + __popcll(on & ((1ull << lane) - 1));
+        slots[i] = slot;
+        wts[i] = w;
       }
+      n += __popcll(on);
+    }
+    if (lane == 0) kept[r] = n;
+  }
+  __syncthreads();
+  const int total = kRowsPerBlock * cpr;
+  for (int idx = tid; idx < total; idx += kMoveThreads) {
+    const int r = div_chunks(idx, magic);
+    const int ch = idx - r * cpr;
+    if (t0 + r >= num_items) continue;
+    const int n = kept[r];
+    const int32_t* sl = slots + r * K;
+    const float* wt = wts + r * K;
+    float acc[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) acc[j] = 0.f;
+    for (int i = 0; i < n; i += 4) {
+      uint4 v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (i + q < n) v[q] = load_stream(y + (size_t)sl[i + q] * cpr + ch);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (i + q < n) {
+          const float w = wt[i + q];
+          float a[N];
+          Chunk<T>::unpack(v[q], a);
+#pragma unroll
+          for (int j = 0; j < N; ++j) acc[j] = fmaf(w, a[j], acc[j]);
+        }
     }
     store_stream(out + (size_t)(t0 + r) * cpr + ch, Chunk<T>::pack(acc));
   }
@@ -217,7 +277,7 @@ __global__ __launch_bounds__(kMoveThreads) void combine_generic_kernel(
       float a[N];
       Chunk<T>::unpack(y[(size_t)slot * cpr + ch], a);
 #pragma unroll
-      for (int j = 0; j < N; ++j) acc[j] = __fadd_rn(acc[j], __fmul_rn(w, a[j]));
+      for (int j = 0; j < N; ++j) acc[j] = fmaf(w, a[j], acc[j]);
     }
     out[(size_t)t * cpr + ch] = Chunk<T>::pack(acc);
   }
@@ -379,16 +439,15 @@ extern "C" int vmoe_combine(const VmoeCombineParams* p, vmoe_stream_t stream) {
   if (rc != VMOE_OK) return rc;
   const int cpr = (int)((size_t)p->D * (p->dtype == VMOE_BF16 ? 2 : 4) / 16);
   const bool bf16 = p->dtype == VMOE_BF16;
-  if (p->K <= kMaxK && kRowsPerBlock * cpr < 65536) {
+  if (p->K <= kListedK && kRowsPerBlock * cpr < 65536) {
     const int blocks = (p->num_items + kRowsPerBlock - 1) / kRowsPerBlock;
-    if (bf16)
-      hipLaunchKernelGGL(combine_kernel<bf16_t>, dim3(blocks), dim3(kMoveThreads), 0,
-                         as_stream(stream), (const uint4*)p->y, p->token_slot, p->weights,
-                         (uint4*)p->out, p->num_items, p->num_slots, p->K, cpr, chunk_magic(cpr));
-    else
-      hipLaunchKernelGGL(combine_kernel<float>, dim3(blocks), dim3(kMoveThreads), 0,
-                         as_stream(stream), (const uint4*)p->y, p->token_slot, p->weights,
-                         (uint4*)p->out, p->num_items, p->num_slots, p->K, cpr, chunk_magic(cpr));
+    const bool listed = p->K > 2;
+    const size_t lds = listed ? (size_t)kRowsPerBlock * p->K * 8 : 0;
+    auto kern = listed ? (bf16 ? combine_listed_kernel<bf16_t> : combine_listed_kernel<float>)
+                       : (bf16 ? combine_kernel<bf16_t> : combine_kernel<float>);
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(kMoveThreads), lds, as_stream(stream), (const uint4*)p->y,
+                       p->token_slot, p->weights, (uint4*)p->out, p->num_items, p->num_slots, p->K, cpr,
+                       chunk_magic(cpr));
   } else {
     const int blocks = (p->num_items + 3) / 4;
     if (bf16)

@@ -209,6 +209,31 @@ XLA_FFI_DEFINE_HANDLER_SYMBOL(VmoeTopItemsPerExpert, TopItemsPerExpertImpl,
                               ffi::Ffi::Bind().Ctx<Stream>().Arg<Any>().Ret<S32>().Ret<S32>().Ret<S32>()
                                   .Ret<F32>().Ret<F32>().Attr<int32_t>("capacity"));
 
+// The same and items_minmax (2,G), gate_minmax (2,G) of the gates' type, ratios (floor(log2 E) + 2, G),
+// rows_per_expert (E,)
+static ffi::Error TopItemsMetricsImpl(hipStream_t stream, Any gates, S32Out indices, S32Out token_slot,
+                                      S32Out slot_token, F32Out weights, F32Out sel_minmax,
+                                      S32Out items_minmax, AnyOut gate_minmax, F32Out ratios,
+                                      S32Out rows_per_expert, int32_t capacity) {
+  VmoeTopItemsParams p{};
+  p.gates = gates.untyped_data();
+  p.indices = indices->typed_data();
+  p.token_slot = token_slot->typed_data();
+  p.slot_token = slot_token->typed_data();
+  p.weights = weights->typed_data();
+  p.sel_minmax = sel_minmax->typed_data();
+  p.G = Dim(gates, 0); p.S = Dim(gates, 1); p.E = Dim(gates, 2);
+  p.C = capacity;
+  p.dtype = DType(gates.element_type());
+  return Status(vmoe_top_items_metrics(&p, items_minmax->typed_data(), gate_minmax->untyped_data(),
+                                       ratios->typed_data(), rows_per_expert->typed_data(), stream),
+                "vmoe_top_items_metrics");
+}
+XLA_FFI_DEFINE_HANDLER_SYMBOL(VmoeTopItemsMetrics, TopItemsMetricsImpl,
+                              ffi::Ffi::Bind().Ctx<Stream>().Arg<Any>().Ret<S32>().Ret<S32>().Ret<S32>()
+                                  .Ret<F32>().Ret<F32>().Ret<S32>().Ret<Any>().Ret<F32>().Ret<S32>()
+                                  .Attr<int32_t>("capacity"));
+
 // indices (G,S,K,2) -> token_slot (G,S,K), slot_token (E*G*C,), num_duplicates (1,), num_invalid (1,)
 static ffi::Error IndicesToSlotsImpl(hipStream_t stream, S32 indices, S32Out token_slot,
                                      S32Out slot_token, S32Out num_duplicates, S32Out num_invalid,

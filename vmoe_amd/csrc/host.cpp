@@ -130,6 +130,27 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, OptTensor, OptTensor, OptTensor> rout
   return {indices, token_slot, slot_token, fill, imp, gsh, aux};
 }
 
+// Experts-choice routing with its monitoring scalars -> indices, token_slot, slot_token, weights,
+// fewest / most experts per item, smallest / largest selected gate, shares of items (num, G), rows
+// per expert.
+std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> top_items_metrics(
+    int64_t stream, const Tensor& gates_, int64_t C) {
+  const Tensor gates = gates_.contiguous();
+  const int64_t G = gates.size(0), S = gates.size(1), E = gates.size(2);
+  int64_t num = 2;
+  while (E >> (num - 1)) ++num;
+  Tensor indices = i32({G, S, E, 2}, gates), token_slot = i32({G, S, E}, gates);
+  Tensor slot_token = i32({E * G * C}, gates), weights = f32({G, S, E}, gates), sel = f32({G, E, 2}, gates);
+  Tensor items = i32({2, G}, gates), gate = empty({2, G}, gates.scalar_type(), gates);
+  Tensor ratios = f32({num, G}, gates), rows = i32({E}, gates);
+  VmoeTopItemsParams p{ptr(gates), ptr_as<int32_t>(indices), ptr_as<int32_t>(token_slot),
+                       ptr_as<int32_t>(slot_token), ptr_as<float>(weights), ptr_as<float>(sel), (int32_t)G,
+                       (int32_t)S, (int32_t)E, (int32_t)C, dtype_code(gates)};
+  check(vmoe_top_items_metrics(&p, ptr_as<int32_t>(items), ptr(gate), ptr_as<float>(ratios),
+                               ptr_as<int32_t>(rows), stream_of(stream)), "vmoe_top_items_metrics");
+  return {indices, token_slot, slot_token, weights, items, gate, ratios, rows};
+}
+
 // The expert MLP; with `fill` and `token_slot` the packed rows are computed here as well.
 // -> out, workspace, byte offset of the status words in it (-1: none), token_row,
 //    rows_per_expert, row_token, whether the call ran on a plan that the compaction wrote.
@@ -333,6 +354,7 @@ PYBIND11_MODULE(_vmoe_host, m) {
   });
   m.def("gate_topk", &gate_topk);
   m.def("route_assign", &route_assign);
+  m.def("top_items_metrics", &top_items_metrics);
   m.def("expert_mlp", &expert_mlp);
   m.def("dispatch", &dispatch);
   m.def("combine", &combine);

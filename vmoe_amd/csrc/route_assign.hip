@@ -354,38 +354,57 @@ __global__ __launch_bounds__(kRouteThreads) void route_assign_metrics_kernel(
 
 // Experts-choice routing (vmoe/moe.py:655-694): every expert takes the C items
 // with its largest gates (jax.lax.top_k over the transposed gates: descending,
-// equal gates -> lower item index first).  One workgroup per (expert, group)
-// sorts the S keys (descending-gate order bits << 32 | item) of that column in
-// LDS; the rank of an item is its position, kept when rank < C.  The outputs are
-// those of the slot-assignment kernel with one "choice" per expert (K = E), so
-// the same dispatch / combine kernels serve both routing schemes.
+// equal gates -> lower item index first).  The outputs are those of the
+// slot-assignment kernel with one "choice" per expert (K = E), so the same
+// dispatch / combine kernels serve both routing schemes.
+//
+// Two launches.  top_items_kernel ranks a column: one workgroup per (expert, group).
+// Written from there, the item-major outputs would be three scattered stores per (item,
+// expert), 4 or 8 bytes of a line each; so it leaves the ranks inside token_slot, each
+// block of `chunk` items transposed (expert-major: runs of up to 256 bytes), and
+// top_items_emit_kernel turns a block's ranks around in LDS and writes whole rows.
+// 8 groups of 1 568 items, 32 experts, bfloat16: 35 us with scattered stores and the sort,
+// 11 + 13 us this way (bound by latency).
+struct TopItemsMetrics {
+  int32_t* items_minmax;   // (2, G): fewest and most experts per item
+  int32_t* counts;         // (num, G): items taken by at least 1, 2, 4, ... experts, and by all
+  int num;
+  int32_t* rows;           // (E,): G * C, or null
+};
+
+// Bins of the counting rank over every bfloat16 from 1 down to 0.
+constexpr int kGateBins = 16384;
+static_assert(kGateBins > 0x3F80 && kGateBins % (kRouteThreads * 4) == 0, "whole 16-byte pieces per thread");
+inline __host__ __device__ bool rank_by_counting(int SP, bool bf16) { return bf16 && SP >= 512; }
+
 template <typename T, int R>
 __global__ __launch_bounds__(kRouteThreads) void top_items_kernel(
-    const T* __restrict__ gates, int32_t* __restrict__ indices, int32_t* __restrict__ token_slot,
-    int32_t* __restrict__ slot_token, float* __restrict__ weights, float* __restrict__ sel_minmax,
-    int G, int S, int E, int C, int SP) {
+    const T* __restrict__ gates, int32_t* __restrict__ token_slot, int32_t* __restrict__ slot_token,
+    float* __restrict__ sel_minmax, TopItemsMetrics m, int G, int S, int E, int C, int SP, int chunk) {
   extern __shared__ __align__(16) unsigned char smem[];
   uint64_t* keys = reinterpret_cast<uint64_t*>(smem);
   const int tid = threadIdx.x;
   const int e = blockIdx.x, g = blockIdx.y;
   const T* col = gates + (size_t)g * S * E + e;
   const int last = (C < S ? C : S) - 1;
-  // Rank r of the column holds item s: the outputs of that (item, expert) pair.
-  auto emit = [&](int r, int s) {
-    const size_t o = ((size_t)g * S + s) * E + e;
-    int slot = -1;
-    if (r < C) {
-      slot = slot_row(e, g, r, G, E, C);
-      slot_token[slot] = g * S + s;
+  if (e == 0 && m.counts != nullptr) {      // what the next launch adds to
+    if (tid < m.num) m.counts[(size_t)tid * G + g] = 0;
+    if (tid == 0) {
+      m.items_minmax[g] = INT32_MAX;
+      m.items_minmax[G + g] = 0;
     }
-    indices[2 * o] = e;
-    indices[2 * o + 1] = r;
-    token_slot[o] = slot;
-    const T gate = col[(size_t)s * E];
-    weights[o] = Elt<T>::load(&gate);
-    if (sel_minmax != nullptr) {
-      if (r == last) sel_minmax[((size_t)g * E + e) * 2] = Elt<T>::load(&gate);
-      if (r == 0) sel_minmax[((size_t)g * E + e) * 2 + 1] = Elt<T>::load(&gate);
+  }
+  if (g == 0 && tid == 0 && m.rows != nullptr) m.rows[e] = G * C;
+  // Rank r of the column holds item s.
+  auto emit = [&](int r, int s) {
+    const int s0 = s & ~(chunk - 1);
+    const int rows = min(chunk, S - s0);
+    token_slot[((size_t)g * S + s0) * E + (size_t)e * rows + (s - s0)] = r;
+    if (r < C) slot_token[slot_row(e, g, r, G, E, C)] = g * S + s;
+    if (sel_minmax != nullptr && (r == last || r == 0)) {
+      const float gate = Elt<T>::load(col + (size_t)s * E);
+      if (r == last) sel_minmax[((size_t)g * E + e) * 2] = gate;
+      if (r == 0) sel_minmax[((size_t)g * E + e) * 2 + 1] = gate;
     }
   };
   if constexpr (R == 0) {
@@ -399,20 +418,180 @@ __global__ __launch_bounds__(kRouteThreads) void top_items_kernel(
     for (int r = tid; r < S; r += kRouteThreads) emit(r, (int)(uint32_t)keys[r]);
   } else {
     const int nact = SP / R;
-    uint64_t key[R];
+    uint32_t bits[R];
+    bool countable = true;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int s = tid * R + r;
-      key[r] = (tid < nact && s < S)
-                   ? bpr_key64(__builtin_bit_cast(uint32_t, Elt<T>::load(col + (size_t)s * E)), s)
-                   : ~0ull;
+      bits[r] = (tid < nact && s < S) ? __builtin_bit_cast(uint32_t, Elt<T>::load(col + (size_t)s * E)) : 0u;
+      countable = countable && bits[r] <= 0x3F800000u;       // 0 .. 1: not negative, not NaN
     }
-    bitonic_sort_regs<R, uint64_t>(key, keys, SP, tid, nact);
+    // Gates of a bfloat16 softmax take at most 0x3F81 values: rank by histogram, prefix, scatter
+    // into the bins' segments and a count inside the item's own segment (see route_assign_group),
+    // in place of 66 compare-exchange steps at 2 048 keys.  Below 512 keys clearing the bins costs
+    // what the sort does.
+    if (rank_by_counting(SP, sizeof(T) == 2) && __syncthreads_and(countable)) {
+      uint32_t* hist = reinterpret_cast<uint32_t*>(smem);    // items per bin, then the bins' cursors
+      uint32_t* seg = hist + kGateBins;                      // S items, bin by bin
+      constexpr int kPieces = kGateBins / kRouteThreads / 4; // 16-byte pieces of a thread's bins
+      uint4* hist4 = reinterpret_cast<uint4*>(hist);
 #pragma unroll
-    for (int r = 0; r < R; ++r)
-      if (tid < nact && tid * R + r < S) emit(tid * R + r, (int)(uint32_t)key[r]);
+      for (int i = 0; i < kPieces; ++i) hist4[i * kRouteThreads + tid] = make_uint4(0, 0, 0, 0);
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (tid < nact && tid * R + r < S) atomicAdd(&hist[0x3F80u - (bits[r] >> 16)], 1u);
+      __syncthreads();
+      {
+        uint4 c[kPieces];
+        uint32_t sum = 0;
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i) {
+          c[i] = hist4[tid * kPieces + i];
+          sum += c[i].x + c[i].y + c[i].z + c[i].w;
+        }
+        const int lane = tid & 63, wave = tid >> 6;
+        uint32_t incl = sum;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+          const uint32_t o = __shfl_up(incl, d, kWave);
+          if (lane >= d) incl += o;
+        }
+        __shared__ uint32_t wave_total[kRouteThreads / 64];
+        if (lane == 63) wave_total[wave] = incl;
+        __syncthreads();
+        uint32_t at = incl - sum;
+        for (int w = 0; w < wave; ++w) at += wave_total[w];
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i) {
+          const uint4 v = c[i];
+          hist4[tid * kPieces + i] = make_uint4(at, at + v.x, at + v.x + v.y, at + v.x + v.y + v.z);
+          at += v.x + v.y + v.z + v.w;
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (tid < nact && tid * R + r < S)
+          seg[atomicAdd(&hist[0x3F80u - (bits[r] >> 16)], 1u)] = (uint32_t)(tid * R + r);
+      __syncthreads();
+      // A bin's cursor now stands at its end, which is where the next bin starts.
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int s = tid * R + r;
+        if (tid < nact && s < S) {
+          const uint32_t bin = 0x3F80u - (bits[r] >> 16);
+          const uint32_t first = bin > 0 ? hist[bin - 1] : 0u, end = hist[bin];
+          uint32_t lower = 0;
+          for (uint32_t q = first; q < end; ++q) lower += seg[q] < (uint32_t)s ? 1u : 0u;
+          emit((int)(first + lower), s);
+        }
+      }
+    } else {
+      uint64_t key[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int s = tid * R + r;
+        key[r] = (tid < nact && s < S) ? bpr_key64(bits[r], s) : ~0ull;
+      }
+      bitonic_sort_regs<R, uint64_t>(key, keys, SP, tid, nact);
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (tid < nact && tid * R + r < S) emit(tid * R + r, (int)(uint32_t)key[r]);
+    }
   }
   for (int c = S + tid; c < C; c += kRouteThreads) slot_token[slot_row(e, g, c, G, E, C)] = -1;
+}
+
+// Items `chunk` at a time (a power of two up to 64): ranks -> indices, token_slot, weights, and the
+// counts of the monitoring scalars (integer atomics: the order of the workgroups does not matter).
+template <typename T>
+__global__ __launch_bounds__(256) void top_items_emit_kernel(
+    const T* __restrict__ gates, int32_t* __restrict__ indices, int32_t* __restrict__ token_slot,
+    float* __restrict__ weights, TopItemsMetrics m, int G, int S, int E, int C, int chunk, int chunks) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  int32_t* rank = reinterpret_cast<int32_t*>(smem);     // (E, chunk + 1): one word of padding per expert
+  __shared__ int32_t taken[64];
+  const int tid = threadIdx.x;
+  const int g = blockIdx.x / chunks, s0 = (blockIdx.x - g * chunks) * chunk;
+  const int rows = min(chunk, S - s0);
+  const size_t base = ((size_t)g * S + s0) * E;
+  const int n = rows * E;
+  if (tid < 64) taken[tid] = 0;
+  if (chunk > 1)
+    for (int i = tid; i < n; i += 256) {
+      const int e = i / rows;
+      rank[e * (chunk + 1) + (i - e * rows)] = token_slot[base + i];
+    }
+  __syncthreads();
+  int mine = 0;      // chunk == 1: experts that took the workgroup's one item
+  for (int i = tid; i < n; i += 256) {
+    const int o = i / E, e = i - o * E;
+    const int r = chunk > 1 ? rank[e * (chunk + 1) + o] : token_slot[base + i];
+    *reinterpret_cast<int2*>(indices + 2 * (base + i)) = make_int2(e, r);
+    token_slot[base + i] = r < C ? slot_row(e, g, r, G, E, C) : -1;
+    weights[base + i] = Elt<T>::load(gates + base + i);
+    mine += r < C ? 1 : 0;
+  }
+  if (m.counts == nullptr) return;
+  if (chunk > 1) {
+    if (tid < rows) {
+      int c = 0;
+      for (int e = 0; e < E; ++e) c += rank[e * (chunk + 1) + tid] < C ? 1 : 0;
+      taken[tid] = c;
+    }
+  } else {
+    atomicAdd(&taken[0], mine);
+  }
+  __syncthreads();
+  if (tid >= 64) return;
+  const bool on = tid < rows;
+  const int c = on ? taken[tid] : 0;
+  int lo = on ? c : INT32_MAX, hi = c;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    lo = min(lo, __shfl_xor(lo, d, kWave));
+    hi = max(hi, __shfl_xor(hi, d, kWave));
+  }
+  if (tid == 0) {
+    atomicMin(&m.items_minmax[g], lo);
+    atomicMax(&m.items_minmax[G + g], hi);
+  }
+  for (int i = 0; i < m.num; ++i) {
+    const int at_least = i < m.num - 1 ? 1 << i : E;
+    const int cnt = __popcll(__ballot(on && c >= at_least));
+    if (tid == 0 && cnt > 0) atomicAdd(&m.counts[(size_t)i * G + g], cnt);
+  }
+}
+
+// Counts -> shares of the group, in place; the smallest and largest selected gate of every group (a
+// NaN among them stays one).
+template <typename T>
+__global__ __launch_bounds__(64) void top_items_finish_kernel(const float* __restrict__ sel_minmax,
+                                                              T* __restrict__ gate_minmax,
+                                                              TopItemsMetrics m, int G, int S, int E) {
+  const int g = blockIdx.x, lane = threadIdx.x;
+  auto lower = [](float a, float b) { return (b < a || b != b) ? b : a; };
+  auto upper = [](float a, float b) { return (b > a || b != b) ? b : a; };
+  const float* sel = sel_minmax + (size_t)g * E * 2;
+  float lo = sel[0], hi = sel[1];
+  for (int e = lane; e < E; e += 64) {
+    lo = lower(lo, sel[2 * e]);
+    hi = upper(hi, sel[2 * e + 1]);
+  }
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    lo = lower(lo, __shfl_xor(lo, d, kWave));
+    hi = upper(hi, __shfl_xor(hi, d, kWave));
+  }
+  if (lane == 0) {
+    Elt<T>::store(gate_minmax + g, lo);
+    Elt<T>::store(gate_minmax + G + g, hi);
+  }
+  if (lane < m.num) {
+    int32_t* at = m.counts + (size_t)lane * G + g;
+    *reinterpret_cast<float*>(at) = (float)*at / (float)S;
+  }
 }
 
 __global__ __launch_bounds__(256) void fill_i32_kernel(int32_t* p, size_t n, int32_t v) {
@@ -639,7 +818,52 @@ extern "C" int vmoe_densify(const VmoeDensifyParams* p, vmoe_stream_t stream) {
   return launch_status();
 }
 
-extern "C" int vmoe_top_items_per_expert(const VmoeTopItemsParams* p, vmoe_stream_t stream) {
+template <typename T>
+static int launch_top_items(const VmoeTopItemsParams* p, const TopItemsMetrics& m, T* gate_minmax,
+                            vmoe_stream_t stream) {
+  const int SP = pow2ceil(p->S < 2 ? 2 : p->S);
+  const int R = keys_per_thread(SP);
+  const T* gates = (const T*)p->gates;
+  size_t lds = (size_t)SP * 8;
+  if (R > 0 && rank_by_counting(SP, sizeof(T) == 2)) {
+    const size_t counting = ((size_t)kGateBins + p->S) * 4;
+    if (counting > lds) lds = counting;
+  }
+  if (lds > 160 * 1024) return VMOE_E_UNSUPPORTED;
+  int chunk = 64;      // items per workgroup of the second launch: their ranks take up to 64 KB of LDS
+  while (chunk > 1 && (size_t)p->E * (chunk + 1) * 4 > 64 * 1024) chunk >>= 1;
+  const int chunks = (p->S + chunk - 1) / chunk;
+  const size_t emit_lds = chunk > 1 ? (size_t)p->E * (chunk + 1) * 4 : 0;
+  auto launch = [&](auto kern) -> int {
+    hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
+    if (e != hipSuccess) return (int)e;
+    hipLaunchKernelGGL(kern, dim3(p->E, p->G), dim3(kRouteThreads), lds, as_stream(stream), gates,
+                       p->token_slot, p->slot_token, p->sel_minmax, m, p->G, p->S, p->E, p->C, SP, chunk);
+    return launch_status();
+  };
+  int rc;
+  switch (R) {
+    case 1: rc = launch(top_items_kernel<T, 1>); break;
+    case 2: rc = launch(top_items_kernel<T, 2>); break;
+    case 4: rc = launch(top_items_kernel<T, 4>); break;
+    case 8: rc = launch(top_items_kernel<T, 8>); break;
+    default: rc = launch(top_items_kernel<T, 0>); break;
+  }
+  if (rc != VMOE_OK) return rc;
+  hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(top_items_emit_kernel<T>), emit_lds);
+  if (e != hipSuccess) return (int)e;
+  hipLaunchKernelGGL(top_items_emit_kernel<T>, dim3((unsigned)(p->G * chunks)), dim3(256), emit_lds,
+                     as_stream(stream), gates, p->indices, p->token_slot, p->weights, m, p->G, p->S, p->E,
+                     p->C, chunk, chunks);
+  rc = launch_status();
+  if (rc != VMOE_OK || m.counts == nullptr) return rc;
+  hipLaunchKernelGGL(top_items_finish_kernel<T>, dim3((unsigned)p->G), dim3(64), 0, as_stream(stream),
+                     p->sel_minmax, gate_minmax, m, p->G, p->S, p->E);
+  return launch_status();
+}
+
+static int top_items(const VmoeTopItemsParams* p, const TopItemsMetrics& m, void* gate_minmax,
+                     vmoe_stream_t stream) {
   if (p == nullptr || p->gates == nullptr || p->indices == nullptr || p->token_slot == nullptr ||
       p->slot_token == nullptr || p->weights == nullptr)
     return VMOE_E_NULL;
@@ -648,37 +872,22 @@ extern "C" int vmoe_top_items_per_expert(const VmoeTopItemsParams* p, vmoe_strea
   if (p->G > 65535) return VMOE_E_UNSUPPORTED;
   if ((int64_t)p->E * p->G * p->C >= INT32_MAX || (int64_t)p->G * p->S * p->E >= INT32_MAX)
     return VMOE_E_OVERFLOW;
-  const int SP = pow2ceil(p->S < 2 ? 2 : p->S);
-  const int R = keys_per_thread(SP);
-  const size_t lds = (size_t)SP * 8;
-  if (lds > 160 * 1024) return VMOE_E_UNSUPPORTED;
-  dim3 grid(p->E, p->G);
-  auto launch = [&](auto kern, auto* gates) -> int {
-    hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
-    if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL(kern, grid, dim3(kRouteThreads), lds, as_stream(stream), gates, p->indices,
-                       p->token_slot, p->slot_token, p->weights, p->sel_minmax, p->G, p->S, p->E,
-                       p->C, SP);
-    return launch_status();
-  };
-  if (p->dtype == VMOE_BF16) {
-    const bf16_t* gates = (const bf16_t*)p->gates;
-    switch (R) {
-      case 1: return launch(top_items_kernel<bf16_t, 1>, gates);
-      case 2: return launch(top_items_kernel<bf16_t, 2>, gates);
-      case 4: return launch(top_items_kernel<bf16_t, 4>, gates);
-      case 8: return launch(top_items_kernel<bf16_t, 8>, gates);
-      default: return launch(top_items_kernel<bf16_t, 0>, gates);
-    }
-  }
-  const float* gates = (const float*)p->gates;
-  switch (R) {
-    case 1: return launch(top_items_kernel<float, 1>, gates);
-    case 2: return launch(top_items_kernel<float, 2>, gates);
-    case 4: return launch(top_items_kernel<float, 4>, gates);
-    case 8: return launch(top_items_kernel<float, 8>, gates);
-    default: return launch(top_items_kernel<float, 0>, gates);
-  }
+  return p->dtype == VMOE_BF16 ? launch_top_items<bf16_t>(p, m, (bf16_t*)gate_minmax, stream)
+                               : launch_top_items<float>(p, m, (float*)gate_minmax, stream);
+}
+
+extern "C" int vmoe_top_items_per_expert(const VmoeTopItemsParams* p, vmoe_stream_t stream) {
+  return top_items(p, TopItemsMetrics{}, nullptr, stream);
+}
+
+extern "C" int vmoe_top_items_metrics(const VmoeTopItemsParams* p, int32_t* items_minmax, void* gate_minmax,
+                                      float* ratios, int32_t* rows_per_expert, vmoe_stream_t stream) {
+  if (p == nullptr || p->sel_minmax == nullptr || items_minmax == nullptr || gate_minmax == nullptr ||
+      ratios == nullptr)
+    return VMOE_E_NULL;
+  TopItemsMetrics m{items_minmax, reinterpret_cast<int32_t*>(ratios), 2, rows_per_expert};
+  while (p->E >> (m.num - 1)) ++m.num;     // floor(log2 E) + 2
+  return top_items(p, m, gate_minmax, stream);
 }
 
 // Launches the row compaction with `prefix` as the (G, E) scratch of its two-launch form.

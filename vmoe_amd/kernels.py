@@ -160,6 +160,28 @@ def top_items_per_expert(gates: torch.Tensor, capacity: int):
   return indices, token_slot, slot_token, weights, sel
 
 
+def top_items_metrics(gates: torch.Tensor, capacity: int):
+  """gates (G,S,E) -> indices (G,S,E,2), token_slot (G,S,E), slot_token (E*G*C,), weights
+  (G,S,E) float32 and the monitoring scalars per group: items (2,G) int32, the fewest and most
+  experts of an item; gate (2,G) in the gates' dtype, the smallest and largest selected gate;
+  ratios (floor(log2 E) + 2, G) float32, the share of items taken by at least 1, 2, 4, ... and E
+  experts; and rows_per_expert (E,) int32 = G * capacity."""
+  if not H.timed("vmoe_top_items_metrics"):
+    return H.host().top_items_metrics(H.raw_stream(), gates, capacity)
+  G, S, E = gates.shape
+  dev = gates.device
+  gates = gates.contiguous()
+  indices, token_slot = _i32(G, S, E, 2, device=dev), _i32(G, S, E, device=dev)
+  slot_token, items, rows = _i32(E * G * capacity, device=dev), _i32(2, G, device=dev), _i32(E, device=dev)
+  weights, sel = _f32(G, S, E, device=dev), _f32(G, E, 2, device=dev)
+  gate = torch.empty((2, G), dtype=gates.dtype, device=dev)
+  ratios = _f32(E.bit_length() + 1, G, device=dev)
+  p = H.TopItemsParams(H.ptr(gates), H.ptr(indices), H.ptr(token_slot), H.ptr(slot_token),
+                       H.ptr(weights), H.ptr(sel), G, S, E, capacity, H.dtype_code(gates.dtype))
+  H.call_blocks("vmoe_top_items_metrics", p, H.ptr(items), H.ptr(gate), H.ptr(ratios), H.ptr(rows))
+  return indices, token_slot, slot_token, weights, items, gate, ratios, rows
+
+
 def indices_to_slots(indices: torch.Tensor, num_experts: int, capacity: int):
   """indices (G,S,K,2) -> token_slot (G,S,K), slot_token (E*G*C,), counters (2,) [dups, invalid]."""
   G, S, K, _ = indices.shape

@@ -210,12 +210,12 @@ class ExpertIndicesDispatcher(BaseDispatcher):
 
   # Packed rows.  The reference's buffer gives every (group, expert) pair `capacity`
   # rows, filled or not, and the experts run over all of them.  When the fill counts
-  # are known (dispatchers made by the routers), the same buffer can hold each
+  # (or the packed rows themselves) are known (dispatchers made by the routers), the same buffer can hold each
   # expert's items in its first rows instead; experts that accept a row count per
   # expert then skip the rest.  dispatch_packed / combine_packed are the pair used
   # by sparse_moe_spmd for that; dispatch / combine keep the reference layout.
   def supports_packed(self) -> bool:
-    return self.fill is not None
+    return self.fill is not None or self._packed_maps is not None
 
   def _packed(self):
     if self._packed_maps is None:
@@ -599,24 +599,24 @@ def _get_top_items_per_expert_einsum_dispatcher(gates: Array, capacity: int, **d
   G, S, E = g3.shape
   if capacity > S:   # jax.lax.top_k(operand, k) requires k <= the operand's last dimension
     raise ValueError(f"capacity = {capacity} exceeds the group size {S}")
-  indices, token_slot, slot_token, weights, sel = K.top_items_per_expert(g3, capacity)
+  indices, token_slot, slot_token, weights, items, gate, ratios, rows = K.top_items_metrics(g3, capacity)
   inner = ExpertIndicesDispatcher(
       indices=indices, combine_weights=weights, num_experts=E, capacity=capacity,
       _slots=(token_slot, slot_token))
   inner._weights_f32 = weights
+  # Every slot holds an item, so the buffer is its own packed form: an expert that gathers its rows
+  # (21 of 350 us of the B/16 layer on 64 images) needs no dispatched copy.
+  inner.set_packed_maps((token_slot, rows, slot_token.view(E, G * capacity)))
   dispatcher = _SparseEinsumDispatcher(inner, gates.dtype, **dispatcher_kwargs)
   # Metrics useful for monitoring training (moe.py:681-692).
-  per_item = (token_slot >= 0).sum(dim=2, dtype=torch.int32)            # (G, S)
   metrics = {
-      "num_experts_per_item_min": per_item.amin(dim=1),
-      "num_experts_per_item_max": per_item.amax(dim=1),
-      "min_selected_gate": sel[:, :, 0].amin(dim=1).to(gates.dtype),
-      "max_selected_gate": sel[:, :, 1].amax(dim=1).to(gates.dtype),
+      "num_experts_per_item_min": items[0],
+      "num_experts_per_item_max": items[1],
+      "min_selected_gate": gate[0],
+      "max_selected_gate": gate[1],
   }
-  log2_num_experts = int(math.log2(E))
-  for t in [2**i for i in range(log2_num_experts + 1)] + [E]:
-    metrics[f"ratio_processed_items_by_at_least_{t}_experts"] = (
-        (per_item >= t).sum(dim=1).to(torch.float32) / S)
+  for i, t in enumerate([2**i for i in range(E.bit_length())] + [E]):
+    metrics[f"ratio_processed_items_by_at_least_{t}_experts"] = ratios[i]
   if not batched:
     return _SingleGroupView(dispatcher), {k: v[0] for k, v in metrics.items()}
   return dispatcher, metrics
