@@ -127,6 +127,41 @@ def test_gate_topk_float32_split_k_form(K, monkeypatch, n, D, E):
       np.testing.assert_allclose(to_np(g_s), to_np(g_d), rtol=1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("n,D,E,k", [(1, 64, 8, 8), (31, 128, 16, 1), (32, 192, 32, 2), (33, 768, 24, 3),
+                                     (1568, 768, 32, 2), (196, 1024, 8, 2), (65, 1088, 32, 2),
+                                     (97, 2112, 8, 1), (255 * 32, 768, 32, 2), (255 * 32 + 1, 768, 32, 2)])
+def test_gate_topk_bf16_split_k_form(K, monkeypatch, n, D, E, k):
+  """bfloat16 gating over fewer tiles of 32 items than CUs deals k to the waves of a tile's workgroup
+  in slices of 128 (one slice, a half one, exactly one round of eight, more): against the oracle, and
+  against the direct loads (VMOE_GATE_DIRECT_LOADS=1) bit for bit where every partial sum is exact."""
+  rng = np.random.default_rng(n + D)
+  xi = rng.integers(-2, 3, (1, n, D)).astype(np.float32)          # exact in bfloat16, sums below 2^24
+  wi = rng.integers(-2, 3, (D, E)).astype(np.float32) / 64
+  b = (rng.integers(-8, 9, E) / 4).astype(np.float32)
+  xr = O.cast(rng.standard_normal((1, n, D)), O.BF16)
+  wr = O.cast(rng.standard_normal((D, E)) / np.sqrt(D), O.BF16)
+  for x, w, exact in ((xi, wi, True), (xr, wr, False)):
+    xd, wd = to_dev(x, O.BF16), to_dev(w, O.BF16)
+    g_s, v_s, i_s = K.gate_topk(xd, wd, k, logit_bias=to_dev(b))
+    _, v_n, i_n = K.gate_topk(xd, wd, k, logit_bias=to_dev(b), return_gates=False)
+    g_p, _, _ = K.gate_topk(xd, wd, k)
+    monkeypatch.setenv("VMOE_GATE_DIRECT_LOADS", "1")
+    g_d, v_d, i_d = K.gate_topk(xd, wd, k, logit_bias=to_dev(b))
+    monkeypatch.delenv("VMOE_GATE_DIRECT_LOADS")
+    np.testing.assert_array_equal(to_np(i_s), to_np(i_n))
+    np.testing.assert_array_equal(to_np(v_s), to_np(v_n))
+    want_v, want_i = O.top_k(to_np(g_s), k)
+    np.testing.assert_array_equal(to_np(i_s), want_i)
+    np.testing.assert_array_equal(to_np(v_s), want_v)
+    # (2e-2 as above: one rounding of a bfloat16 logit)
+    assert_close(to_np(g_s), O.router_gates(x, w, O.BF16, b), 2e-2, "gates")
+    assert_close(to_np(g_p), O.router_gates(x, w, O.BF16), 2e-2, "gates without bias")
+    if exact:
+      np.testing.assert_array_equal(to_np(g_s), to_np(g_d))
+      np.testing.assert_array_equal(to_np(i_s), to_np(i_d))
+      np.testing.assert_array_equal(to_np(v_s), to_np(v_d))
+
+
 def test_gate_topk_streaming_and_direct_loads_agree(K, monkeypatch):
   """The two forms of the bfloat16 gating kernel (item rows through LDS by DMA, or by direct
   loads: VMOE_GATE_DIRECT_LOADS=1) add the same products in a different order of k: equal

@@ -14,9 +14,11 @@
 // that each lane holds half of one item's row: softmax and top-K are serial per
 // lane, with one xor-32 shuffle per reduction to join the two halves.
 // bfloat16 with up to 32 experts and no logits output takes gate_topk_stream_kernel,
-// which fetches the item rows with coalesced DMA requests into LDS instead.
+// which fetches the item rows with coalesced DMA requests into LDS instead, or, with fewer
+// tiles than CUs, gate_topk_split_kernel.
 // (VMOE_GATE_DIRECT_LOADS=1 in the environment keeps the direct loads: the switch behind
 // the before / after figures.)
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
@@ -421,6 +423,75 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_kernel(
   }
 }
 
+// Softmax and top-K of a 32 x 32 tile of finished logits (row pitch 33) by one wave: a lane holds
+// half (h) of item row0 + m.
+__device__ __forceinline__ void finish_tile32(const float* st, bf16_t* __restrict__ gates,
+                                              float* __restrict__ topk_val, int32_t* __restrict__ topk_idx,
+                                              int row0, int num_items, int E, int K, int m, int h) {
+  constexpr int EP = 32, CNT = EP / 2;
+  const int row = row0 + m;
+  const int n0 = h * CNT;
+  float g[CNT];
+  float mx = -INFINITY;
+#pragma unroll
+  for (int j = 0; j < CNT; ++j) {
+    const float v = st[m * (EP + 1) + n0 + j];
+    g[j] = (n0 + j < E) ? v : -INFINITY;
+    mx = fmaxf(mx, g[j]);
+  }
+  mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+  float sum = 0.f;
+#pragma unroll
+  for (int j = 0; j < CNT; ++j) {
+    g[j] = (n0 + j < E) ? expf(g[j] - mx) : 0.f;
+    sum += g[j];
+  }
+  sum += __shfl_xor(sum, 32, kWave);
+#pragma unroll
+  for (int j = 0; j < CNT; ++j) g[j] = bf16r(g[j] / sum);
+  const bool row_ok = row < num_items;
+  if (gates != nullptr && row_ok) {
+    bf16_t* grow = gates + (size_t)row * E + n0;
+    if ((reinterpret_cast<uintptr_t>(gates) & 15u) == 0) {
+#pragma unroll
+      for (int j = 0; j < CNT; j += 8) {
+        if (n0 + j < E) {
+          uint32_t pk[4];
+#pragma unroll
+          for (int t = 0; t < 4; ++t) pk[t] = pack_bf16x2(g[j + 2 * t], g[j + 2 * t + 1]);
+          *reinterpret_cast<uint4*>(grow + j) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < CNT; ++j)
+        if (n0 + j < E) Elt<bf16_t>::store(grow + j, g[j]);
+    }
+  }
+  uint64_t taken = 0;
+  for (int kk = 0; kk < K; ++kk) {
+    uint64_t best = 0;
+#pragma unroll
+    for (int j = 0; j < CNT; ++j) {
+      const int n = n0 + j;
+      if (n < E && !(taken >> j & 1ull)) {
+        uint64_t key = ((uint64_t)orderable(g[j]) << 32) | (uint32_t)(0xFFFFFFFFu - (uint32_t)n);
+        best = key > best ? key : best;
+      }
+    }
+    const uint32_t olo = __shfl_xor((uint32_t)best, 32, kWave);
+    const uint32_t ohi = __shfl_xor((uint32_t)(best >> 32), 32, kWave);
+    const uint64_t other = ((uint64_t)ohi << 32) | olo;
+    best = other > best ? other : best;
+    const int n_star = (int)(0xFFFFFFFFu - (uint32_t)best);
+    if (n_star >= n0 && n_star < n0 + CNT) taken |= 1ull << (n_star - n0);
+    if (h == 0 && row_ok) {
+      topk_val[(size_t)row * K + kk] = inv_orderable((uint32_t)(best >> 32));
+      topk_idx[(size_t)row * K + kk] = n_star;
+    }
+  }
+}
+
 // Streaming form of the bfloat16 kernel for up to 32 experts (the routers' common case).
 // The item rows are the whole traffic (77 MB on the headline layer, 0.05 MB of router
 // kernel), so they are fetched the way a copy kernel fetches: every DMA request of a wave
@@ -582,70 +653,96 @@ __global__ __launch_bounds__(WAVES * kWave, 1) void gate_topk_stream_kernel(
         st[rl * (EP + 1) + m] = v;
       }
     }
-    constexpr int CNT = EP / 2;
-    const int row = row0 + m;
-    const int n0 = h * CNT;
-    float g[CNT];
-    float mx = -INFINITY;
-#pragma unroll
-    for (int j = 0; j < CNT; ++j) {
-      const float v = st[m * (EP + 1) + n0 + j];
-      g[j] = (n0 + j < E) ? v : -INFINITY;
-      mx = fmaxf(mx, g[j]);
-    }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
-    float sum = 0.f;
-#pragma unroll
-    for (int j = 0; j < CNT; ++j) {
-      g[j] = (n0 + j < E) ? expf(g[j] - mx) : 0.f;
-      sum += g[j];
-    }
-    sum += __shfl_xor(sum, 32, kWave);
-#pragma unroll
-    for (int j = 0; j < CNT; ++j) g[j] = bf16r(g[j] / sum);
-    const bool row_ok = row < num_items;
-    if (gates != nullptr && row_ok) {
-      bf16_t* grow = gates + (size_t)row * E + n0;
-      if ((reinterpret_cast<uintptr_t>(gates) & 15u) == 0) {
-#pragma unroll
-        for (int j = 0; j < CNT; j += 8) {
-          if (n0 + j < E) {
-            uint32_t pk[4];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) pk[t] = pack_bf16x2(g[j + 2 * t], g[j + 2 * t + 1]);
-            *reinterpret_cast<uint4*>(grow + j) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
-          }
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < CNT; ++j)
-          if (n0 + j < E) Elt<bf16_t>::store(grow + j, g[j]);
-      }
-    }
-    uint64_t taken = 0;
-    for (int kk = 0; kk < K; ++kk) {
-      uint64_t best = 0;
-#pragma unroll
-      for (int j = 0; j < CNT; ++j) {
-        const int n = n0 + j;
-        if (n < E && !(taken >> j & 1ull)) {
-          uint64_t key = ((uint64_t)orderable(g[j]) << 32) | (uint32_t)(0xFFFFFFFFu - (uint32_t)n);
-          best = key > best ? key : best;
-        }
-      }
-      const uint32_t olo = __shfl_xor((uint32_t)best, 32, kWave);
-      const uint32_t ohi = __shfl_xor((uint32_t)(best >> 32), 32, kWave);
-      const uint64_t other = ((uint64_t)ohi << 32) | olo;
-      best = other > best ? other : best;
-      const int n_star = (int)(0xFFFFFFFFu - (uint32_t)best);
-      if (n_star >= n0 && n_star < n0 + CNT) taken |= 1ull << (n_star - n0);
-      if (h == 0 && row_ok) {
-        topk_val[(size_t)row * K + kk] = inv_orderable((uint32_t)(best >> 32));
-        topk_idx[(size_t)row * K + kk] = n_star;
-      }
-    }
+    finish_tile32(st, gates, topk_val, topk_idx, row0, num_items, E, K, m, h);
   }
 #endif
+}
+
+// bfloat16, up to 32 experts, fewer tiles of items than CUs: a workgroup per tile of 32 items, the k
+// range dealt to its waves in slices of 128, so that a launch is one trip to memory.  A wave loads its
+// rows' slices in fragment order and, at the same time, an 8 (k) x 8 (expert) block of the router kernel
+// per lane, which it transposes into its own piece of LDS (no barrier before the products); the waves'
+// logits meet in LDS, added in wave order, and wave 0 finishes the tile.  gate_topk_kernel walks all of
+// k in one wave per tile on a quarter of the workgroups, and stages the router kernel in two rounds.
+// Bound by that trip and by wave 0's serial epilogue.  D = 768, 7 to 255 tiles: 7.8 us against 13.6 of
+// gate_topk_kernel; D = 1024: 8.5 against 15.5.
+constexpr int kSplitWaves = 8;
+constexpr int kSplitSlice = 128;                       // k per wave and round
+constexpr int kSplitStride = kSplitSlice + 8;          // elements per expert of a staged slice
+constexpr int kSplitWaveBytes = 32 * kSplitStride * 2; // also holds the wave's 32 x 33 logits
+
+__global__ __launch_bounds__(kSplitWaves * kWave, 1) void gate_topk_split_kernel(
+    const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const float* __restrict__ bias,
+    bf16_t* __restrict__ gates, float* __restrict__ topk_val, int32_t* __restrict__ topk_idx,
+    int num_items, int D, int E, int K) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  constexpr int EP = 32;
+  static_assert(kSplitWaveBytes >= 32 * (EP + 1) * (int)sizeof(float), "the logits fit a wave's piece");
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  const int m = lane & 31, h = lane >> 5;
+  const int row0 = blockIdx.x * 32;
+  const bf16_t* xrow = x + (size_t)min(row0 + m, num_items - 1) * D;
+  bf16_t* wl = reinterpret_cast<bf16_t*>(smem + wave * kSplitWaveBytes);
+  const int kb = lane >> 2, nb = lane & 3;             // this lane's block of the router kernel
+
+  floatx16 acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+  for (int k0 = wave * kSplitSlice; k0 < D; k0 += waves * kSplitSlice) {
+    uint4 wraw[8], a[2][4];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int k = k0 + kb * 8 + i;
+      wraw[i] = make_uint4(0, 0, 0, 0);
+      if (k < D && nb * 8 < E) wraw[i] = *reinterpret_cast<const uint4*>(w + (size_t)k * E + nb * 8);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int kg = k0 + u * 64 + h * 32 + j * 8;
+        a[u][j] = make_uint4(0, 0, 0, 0);
+        if (kg < D) a[u][j] = *reinterpret_cast<const uint4*>(xrow + kg);
+      }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
+      uint32_t o[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t hi = reinterpret_cast<const uint32_t*>(&wraw[2 * q + 1])[j >> 1];
+        const uint32_t lo = reinterpret_cast<const uint32_t*>(&wraw[2 * q])[j >> 1];
+        o[q] = __builtin_amdgcn_perm(hi, lo, sel);
+      }
+      *reinterpret_cast<uint4*>(wl + (nb * 8 + j) * kSplitStride + kb * 8) = make_uint4(o[0], o[1], o[2], o[3]);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // the other lanes' blocks are read from here on
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint4 b = *reinterpret_cast<const uint4*>(wl + m * kSplitStride + u * 64 + h * 32 + j * 8);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[u][j]),
+                                                      __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
+      }
+    mfma_result_fence();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // and overwritten from here on
+  }
+  float* st = reinterpret_cast<float*>(wl);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) st[((i >> 2) * 8 + h * 4 + (i & 3)) * (EP + 1) + m] = acc[i];
+  __syncthreads();
+  for (int e = threadIdx.x; e < 32 * EP; e += blockDim.x) {
+    const int n = e & (EP - 1), at = (e >> 5) * (EP + 1) + n;
+    float v = reinterpret_cast<const float*>(smem)[at];
+    for (int ww = 1; ww < waves; ++ww) v += reinterpret_cast<const float*>(smem + ww * kSplitWaveBytes)[at];
+    v = bf16r(v);
+    if (bias != nullptr && n < E) v = bf16r(v + bias[n]);
+    reinterpret_cast<float*>(smem)[at] = v;
+  }
+  __syncthreads();
+  if (wave == 0)
+    finish_tile32(reinterpret_cast<const float*>(smem), gates, topk_val, topk_idx, row0, num_items, E, K, m, h);
 }
 
 // Top-K of given float32 gates, one wave per item, E <= 1024.
@@ -734,10 +831,23 @@ int launch_gate(const VmoeGateTopkParams* p, hipStream_t stream) {
   if constexpr (sizeof(T) == 2) {
     const size_t stream_w = ((size_t)32 * (p->D + 8) * 2 + 1023) / 1024 * 1024;
     const size_t ring3 = (size_t)kStreamWaves * 3 * kStreamChunkBytes, ring2 = (size_t)kStreamWaves * 2 * kStreamChunkBytes;
-    const bool stream_ok = nt == 1 && p->logits == nullptr && p->E % 8 == 0 && aligned16(p->w) &&
-                           p->D % 64 == 0 && (int64_t)p->num_items * p->D * 2 < ((int64_t)1 << 32) &&
-                           num_tiles >= 256 && stream_w + ring2 <= lds_cu &&
-                           getenv("VMOE_GATE_DIRECT_LOADS") == nullptr;
+    const bool simple = nt == 1 && p->logits == nullptr && p->E % 8 == 0 && aligned16(p->w) &&
+                        p->D % 64 == 0 && getenv("VMOE_GATE_DIRECT_LOADS") == nullptr;
+    const bool stream_ok = simple && (int64_t)p->num_items * p->D * 2 < ((int64_t)1 << 32) &&
+                           num_tiles >= 256 && stream_w + ring2 <= lds_cu;
+    // Fewer tiles than CUs: the waves of a tile share its k range (255 tiles x 768: 8.0 us against 13.8
+    // with direct loads).  Beyond, a CU runs two such workgroups, each with its own copy of the router
+    // kernel, and the streaming form is level (300 to 512 tiles: 10.5 both) or faster (1 152: 24 to 15).
+    if (simple && num_tiles < 256) {
+      const int swaves = std::min((p->D + kSplitSlice - 1) / kSplitSlice, kSplitWaves);
+      const size_t split_lds = (size_t)swaves * kSplitWaveBytes;
+      hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(gate_topk_split_kernel), split_lds);
+      if (e != hipSuccess) return (int)e;
+      hipLaunchKernelGGL(gate_topk_split_kernel, dim3(num_tiles), dim3(swaves * kWave), split_lds, stream,
+                         (const bf16_t*)p->x, (const bf16_t*)p->w, p->logit_bias, (bf16_t*)p->gates,
+                         p->topk_val, p->topk_idx, p->num_items, p->D, p->E, p->K);
+      return launch_status();
+    }
     if (stream_ok) {
       const bool three = stream_w + ring3 <= lds_cu;
       const size_t stream_lds = stream_w + (three ? ring3 : ring2);
