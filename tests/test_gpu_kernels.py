@@ -233,6 +233,7 @@ ROUTE_CASES = [
     (3, 1025, 4, 1, 300, False),     # two keys per thread
     (2, 2304, 32, 2, 72, True),      # four
     (1, 5000, 4, 2, 700, True),      # eight
+    (2, 2900, 6, 3, 1100, False),    # 8 700 choices: more than the 8 192 held in registers
 ]
 
 

@@ -66,8 +66,7 @@ __device__ __forceinline__ uint4 load_row_piece(const bf16_t* __restrict__ p, in
 
 // load_block for rows of any length N (weights).  Rows of whole pieces take a loop without the tail's
 // branch: a wait at every join of that branch keeps one load in flight instead of eight (256 groups of
-// 196 items x 128 slots x 768: dispatch 32.9 us with it, 32.1
-// without, combine 40.6 and 39.8).
+// 196 items x 128 slots x 768: dispatch 32.9 us with it, 32.1 without, combine 40.6 and 39.8).
 __device__ __forceinline__ void load_weight_block(uint4 (&r)[8], const bf16_t* __restrict__ w,
                                                   const int (&rowidx)[8], int col, int N) {
   if (N % 8 == 0) {
