@@ -574,6 +574,28 @@ def test_soft_route_row_tiles(K, G, S, D, N, dtype):
                              rtol=3e-6)
 
 
+@pytest.mark.parametrize("G,S,D,N", [(64, 196, 64, 256), (16, 65, 1024, 128), (32, 100, 320, 44)])
+def test_soft_route_row_tiles_round_like_float32_softmaxes(K, G, S, D, N):
+  """Logits up to about 160 (items near slots, scale 200): both softmaxes take their exponentials and
+  quotients in float32, so hardly a bfloat16 weight rounds away from the float64 softmax of the kernel's
+  own logits.  Bound: exponential, sum and quotient are within 4 * 2^-24 of a weight together (l - max is
+  exact there), and a weight rounds the other way only within that of a rounding boundary, of which there
+  is one per 2^-8 of a weight at the densest: 2 * 2^-22 / 2^-8 of the weights.  An exponential that rounds
+  max * log2(e) first is off by 2^-18 there, and 3e-4 of the weights of the first shape differ."""
+  gen = torch.Generator(device=dev()).manual_seed(D)
+  normal = lambda *shape: torch.randn(shape, generator=gen, device=dev())
+  mu = (normal(D, N) * D ** -0.5).to(torch.bfloat16)
+  near = mu.float().t()[torch.arange(G * S, device=dev()).reshape(G, S) % N]
+  x = (near * D ** 0.5 * 0.7 + normal(G, S, D)).to(torch.bfloat16)
+  dw, cw, lg = K.soft_route(x, mu, 200.0, return_logits=True)
+  assert float(lg.float().max()) > 64
+  for got, axis in ((dw, 1), (cw, 2)):
+    want = torch.softmax(lg.double(), axis)
+    counted = want > 1e-18          # (below, l itself is rounded on the way to l - max)
+    share = float((got != want.to(torch.bfloat16))[counted].double().mean())
+    assert share <= 2.0 ** -13, (axis, share)
+
+
 def _check_soft_weights_against_own_logits(lg, dw, cw, dtype, tag):
   """The two softmaxes themselves.  Against the oracle the weights carry the difference of the
   logits (a bfloat16 logit that rounds the other way moves a weight by exp(step) - 1, which is

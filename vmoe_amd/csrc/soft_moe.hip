@@ -23,8 +23,8 @@
 namespace vmoe {
 namespace {
 
-using soft::kLog2e;
 using soft::kNormEps;
+constexpr float kLog2e = 1.4426950408889634f;
 
 __device__ __forceinline__ float load_any(const void* p, size_t i, int dtype) {
   return dtype == VMOE_F32 ? reinterpret_cast<const float*>(p)[i]

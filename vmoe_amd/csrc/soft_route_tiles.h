@@ -27,7 +27,6 @@ namespace vmoe {
 namespace soft {
 
 constexpr float kNormEps = 1e-6f;
-constexpr float kLog2e = 1.4426950408889634f;
 
 // A 16-byte piece of a row: V values, and the k steps that one piece per lane covers: 4 V k per step.
 // bfloat16: a lane holds 8 consecutive k of row lane % 16, from (lane / 16) * 8 on.  float32: k = 4 j +
@@ -49,12 +48,6 @@ template <> struct Piece<bf16_t> {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, slots),
                                                    __builtin_bit_cast(bf16x8, rows), acc, 0, 0, 0);
   }
-  // exp(l - mx) and 1 / sum with the hardware exp2 and reciprocal: ~1e-6 relative, against 4e-3
-  // for the bfloat16 result.
-  __device__ static __forceinline__ float exp(float l, float mx) {
-    return __builtin_amdgcn_exp2f(fmaf(l, kLog2e, -mx * kLog2e));
-  }
-  __device__ static __forceinline__ float inverse(float s) { return __builtin_amdgcn_rcpf(s); }
 };
 template <> struct Piece<float> {
   static constexpr int V = 4;
@@ -74,8 +67,6 @@ template <> struct Piece<float> {
     for (int t = 0; t < 4; ++t) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t], b[t], acc, 0, 0, 0);
     return acc;
   }
-  __device__ static __forceinline__ float exp(float l, float mx) { return expf(l - mx); }
-  __device__ static __forceinline__ float inverse(float s) { return 1.0f / s; }
 };
 
 // k steps of a width, padded to whole groups of four (the loop's prefetch distance).
@@ -324,15 +315,14 @@ __global__ __launch_bounds__(64 * logits_waves(RB), PIECES > 4 ? 1 : !PAIR && PI
         float v[V];
         read(p, v);
 #pragma unroll
-        for (int j = 0; j < V; ++j) sum += P::exp(v[j], mx);
+        for (int j = 0; j < V; ++j) sum += expf(v[j] - mx);
       }
       for (int o = span >> 1; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
-      const float inv = P::inverse(sum);
       for (int p = sl; p < slot_pieces; p += span) {
         float v[V], e[V];
         read(p, v);
 #pragma unroll
-        for (int j = 0; j < V; ++j) e[j] = P::exp(v[j], mx) * inv;
+        for (int j = 0; j < V; ++j) e[j] = expf(v[j] - mx) / sum;
         if (!live) continue;
         if (VEC) {
           *reinterpret_cast<uint4*>(combine_w + base + p * V) = P::pack(e);
@@ -424,10 +414,10 @@ __global__ __launch_bounds__(kColThreads) void soft_columns_kernel(T* __restrict
 #pragma unroll
         for (int u = 0; u < U; ++u)
           if (r0 + u * lanes < S) m = fmaxf(m, v[u][j]);
-        float s = mx[j] == m ? sum[j] : sum[j] * P::exp(mx[j], m);
+        float s = mx[j] == m ? sum[j] : sum[j] * expf(mx[j] - m);
 #pragma unroll
         for (int u = 0; u < U; ++u)
-          if (r0 + u * lanes < S) s += P::exp(v[u][j], m);
+          if (r0 + u * lanes < S) s += expf(v[u][j] - m);
         mx[j] = m;
         sum[j] = s;
       }
@@ -442,13 +432,13 @@ __global__ __launch_bounds__(kColThreads) void soft_columns_kernel(T* __restrict
   }
   __syncthreads();
   // The row lanes of a column are joined in two steps: `parts` threads per column first, each with
-  // every parts-th lane, then one; its first row lane's place takes the maximum and inverse sum.
+  // every parts-th lane, then one; its first row lane's place takes the maximum and the sum.
   auto join = [&](int c, int first, int step, int end) {
     float m = -INFINITY, s = 0.f;
     for (int l = first; l < end; l += step) m = fmaxf(m, lds[l * width + c]);
     for (int l = first; l < end; l += step) {
       const float ml = lds[l * width + c];
-      if (ml > -INFINITY) s += lds2[l * width + c] * P::exp(ml, m);     // (a lane may have had no row)
+      if (ml > -INFINITY) s += lds2[l * width + c] * expf(ml - m);      // (a lane may have had no row)
     }
     return make_float2(m, s);
   };
@@ -464,13 +454,13 @@ __global__ __launch_bounds__(kColThreads) void soft_columns_kernel(T* __restrict
   for (int c = tid; c < width; c += kColThreads) {
     const float2 ms = join(c, 0, 1, parts > 1 ? parts : lanes);
     lds[c] = ms.x;
-    lds2[c] = P::inverse(ms.y);
+    lds2[c] = ms.y;
   }
   __syncthreads();
   if (!on) return;
-  float m[V], inv[V];
+  float m[V], total[V];
 #pragma unroll
-  for (int j = 0; j < V; ++j) { m[j] = lds[col * V + j]; inv[j] = lds2[col * V + j]; }
+  for (int j = 0; j < V; ++j) { m[j] = lds[col * V + j]; total[j] = lds2[col * V + j]; }
   for (int r0 = rl; r0 < S; r0 += U * lanes) {
     float v[U][V];
 #pragma unroll
@@ -479,7 +469,7 @@ __global__ __launch_bounds__(kColThreads) void soft_columns_kernel(T* __restrict
     for (int u = 0; u < U; ++u) {
       if (r0 + u * lanes >= S) continue;
 #pragma unroll
-      for (int j = 0; j < V; ++j) v[u][j] = P::exp(v[u][j], m[j]) * inv[j];
+      for (int j = 0; j < V; ++j) v[u][j] = expf(v[u][j] - m[j]) / total[j];
       T* p = dw + (size_t)(r0 + u * lanes) * N;
       if constexpr (VEC) *reinterpret_cast<uint4*>(p) = P::pack(v[u]);
       else Elt<T>::store(p, v[u][0]);
