@@ -596,6 +596,25 @@ def test_soft_route_row_tiles_round_like_float32_softmaxes(K, G, S, D, N):
     assert share <= 2.0 ** -13, (axis, share)
 
 
+@pytest.mark.parametrize("G,S,D,N,dtype", [(3, 65, 64, 256, O.BF16), (2, 5, 40, 17, O.BF16), (2, 300, 1024, 128, O.BF16),
+                                           (2, 31, 100, 33, O.F32)])
+def test_soft_route_row_tiles_keep_nan(K, G, S, D, N, dtype):
+  """A NaN item: NaN combine weights of that item alone, NaN dispatch weights of every item of its group
+  (the softmax over items meets it in every slot), the other groups as without it."""
+  rng = np.random.default_rng(S)
+  x = O.cast(rng.standard_normal((G, S, D)), dtype)
+  mu = to_dev(O.cast(rng.standard_normal((D, N)) / np.sqrt(D), dtype), dtype)
+  clean = [to_np(t) for t in K.soft_route(to_dev(x, dtype), mu, 1.0)]
+  x[1, S // 2] = np.nan
+  dw, cw = (to_np(t) for t in K.soft_route(to_dev(x, dtype), mu, 1.0))
+  assert np.isnan(dw[1]).all() and np.isnan(cw[1, S // 2]).all()
+  others = np.arange(S) != S // 2
+  np.testing.assert_array_equal(cw[1, others], clean[1][1, others])
+  for g in set(range(G)) - {1}:
+    np.testing.assert_array_equal(dw[g], clean[0][g])
+    np.testing.assert_array_equal(cw[g], clean[1][g])
+
+
 def _check_soft_weights_against_own_logits(lg, dw, cw, dtype, tag):
   """The two softmaxes themselves.  Against the oracle the weights carry the difference of the
   logits (a bfloat16 logit that rounds the other way moves a weight by exp(step) - 1, which is

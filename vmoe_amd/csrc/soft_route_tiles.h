@@ -414,10 +414,13 @@ __global__ __launch_bounds__(kColThreads) void soft_columns_kernel(T* __restrict
 #pragma unroll
         for (int u = 0; u < U; ++u)
           if (r0 + u * lanes < S) m = fmaxf(m, v[u][j]);
-        float s = mx[j] == m ? sum[j] : sum[j] * expf(mx[j] - m);
+        // (a column of nothing but -infinity or NaN so far keeps the maximum -infinity: its
+        // exponentials are 0 and NaN, not exp(-inf + inf))
+        const float from = m > -INFINITY ? m : 0.f;
+        float s = mx[j] == m ? sum[j] : sum[j] * expf(mx[j] - from);
 #pragma unroll
         for (int u = 0; u < U; ++u)
-          if (r0 + u * lanes < S) s += expf(v[u][j] - m);
+          if (r0 + u * lanes < S) s += expf(v[u][j] - from);
         mx[j] = m;
         sum[j] = s;
       }
@@ -436,10 +439,8 @@ __global__ __launch_bounds__(kColThreads) void soft_columns_kernel(T* __restrict
   auto join = [&](int c, int first, int step, int end) {
     float m = -INFINITY, s = 0.f;
     for (int l = first; l < end; l += step) m = fmaxf(m, lds[l * width + c]);
-    for (int l = first; l < end; l += step) {
-      const float ml = lds[l * width + c];
-      if (ml > -INFINITY) s += lds2[l * width + c] * expf(ml - m);      // (a lane may have had no row)
-    }
+    const float from = m > -INFINITY ? m : 0.f;       // (every lane's sum counts: a NaN item spoils its column)
+    for (int l = first; l < end; l += step) s += lds2[l * width + c] * expf(lds[l * width + c] - from);
     return make_float2(m, s);
   };
   const int parts = min(lanes, kColThreads / width);
