@@ -1,12 +1,14 @@
 """Host-side logic of the drop-in surface that needs no GPU: name resolution of routers
 (vmoe/utils.py:59-109, vmoe/nn/vit_moe.py:76-88), capacity arithmetic, the public
 factories, and the refusal to run forward-only kernels under autograd."""
+import weakref
+
 import numpy as np
 import pytest
 import torch
 
 from vmoe_amd import moe, utils
-from vmoe_amd.nn import routing, vit_moe
+from vmoe_amd.nn import module, routing, vit_moe
 from vmoe_amd.projects.soft_moe import router as soft_router
 
 
@@ -102,3 +104,41 @@ def test_forward_only_modules_refuse_autograd():
     with pytest.raises(Exception) as info:
       mlp.apply_experts({"params": params}, torch.zeros((1, 4, 16)))
     assert not isinstance(info.value, NotImplementedError)
+
+
+@pytest.mark.parametrize("other", [
+    lambda t: torch.full((2, 3), 5.0),                       # same shape
+    lambda t: torch.full((4, 5), 5.0),
+    lambda t: t.data.to(torch.bfloat16),
+    lambda t: t.data.t(),                                    # same address, other strides
+    lambda t: t.data.view(3, 2),
+], ids=["same-shape", "shape", "dtype", "transposed", "reshaped"])
+def test_param_cache_sees_data_assignment(other):
+  """``p.data = other`` raises no version counter: the address and the layout tell."""
+  p = torch.nn.Parameter(torch.arange(6.0).view(2, 3))
+  cache = module.ParamCache()
+  derive = lambda: cache.get((p,), "t", lambda: p.detach().clone())
+  for _ in range(2):
+    assert torch.equal(derive(), p)
+  p.data = other(p)
+  for _ in range(2):
+    got = derive()
+    assert got.dtype == p.dtype and torch.equal(got, p)
+
+
+def test_param_cache_holds_what_its_limit_allows():
+  """Derived values live as long as their entries; in-place edits and other tensors are noticed."""
+  cache = module.ParamCache(limit=1)
+  p, q = torch.zeros(3), torch.ones(3)
+  derive = lambda t, tag: cache.get((t,), tag, lambda: t + 1)
+  first = weakref.ref(derive(p, "a"))
+  assert first() is derive(p, "a")
+  derive(q, "b")                                             # the limit of one: the first entry goes
+  assert first() is None
+  assert derive(p, "a").tolist() == [1, 1, 1]
+  p.add_(1)
+  assert derive(p, "a").tolist() == [2, 2, 2]
+  assert derive(q, "a").tolist() == [2, 2, 2]
+  with pytest.raises(ZeroDivisionError):                     # a build that fails leaves nothing behind
+    cache.get((p,), "c", lambda: 1 // 0)
+  assert cache.get((p,), "c", lambda: 7) == 7

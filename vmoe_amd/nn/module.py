@@ -92,46 +92,46 @@ class ParamCache:
 
   An entry is valid while the very tensors it was built from are alive and
   unmodified: they are identified by object (views by their base tensor, offset,
-  shape and strides), held weakly, and their version counters are compared.  An
+  shape and strides), held weakly, and their version counters, addresses and layouts
+  are compared (``t.data = other`` changes those without a new version).  An
   address alone does not identify a tensor: the allocator hands a freed block
   to the next tensor of that size."""
 
   def __init__(self, limit: int = 16):
     self._entries = {}
     self._limit = limit
-    self._latest = {}       # tag -> (weak references to the tensors, versions, value) last returned
+    self._latest = {}       # tag -> (weak references to the tensors, their states, to the entry) last asked for
+
+  class _Entry:
+    __slots__ = ("bases", "states", "value", "__weakref__")
 
   @staticmethod
-  def _ident(t: torch.Tensor):
-    base = t._base if t._base is not None else t
-    return base, (id(base), t.storage_offset(), tuple(t.shape), tuple(t.stride()), t.dtype)
+  def _state(t: torch.Tensor):
+    return t._version, t.data_ptr(), t.shape, t.stride(), t.dtype, t.device
 
   def get(self, tensors, tag, build):
     tensors = tuple(tensors)
     # The tensors of the last call with this tag, unmodified: what a layer that runs over and over
-    # finds (0.3 us per tensor; the identities below take 1 us each).
+    # finds (1 us per tensor; the bases and keys below take as long again).
     latest = self._latest.get(tag)
     if latest is not None and len(latest[0]) == len(tensors):
-      for t, ref, version in zip(tensors, latest[0], latest[1]):
-        if ref() is not t or t._version != version:
+      state = self._state
+      for t, ref, known in zip(tensors, latest[0], latest[1]):
+        if ref() is not t or state(t) != known:
           break
       else:
-        return latest[2]
-    value = self._find(tensors, tag, build)
-    self._latest[tag] = (tuple(weakref.ref(t) for t in tensors), tuple(t._version for t in tensors), value)
-    return value
-
-  def _find(self, tensors, tag, build):
-    idents = [self._ident(t) for t in tensors]
-    key = (tuple(i[1] for i in idents), tag)
-    versions = tuple(t._version for t in tensors)
-    hit = self._entries.get(key)
-    if hit is not None:
-      refs, vers, value = hit
-      if vers == versions and all(r() is i[0] for r, i in zip(refs, idents)):
-        return value
-    value = build()
-    if len(self._entries) >= self._limit:
-      self._entries.clear()
-    self._entries[key] = (tuple(weakref.ref(i[0]) for i in idents), versions, value)
-    return value
+        entry = latest[2]()
+        if entry is not None:
+          return entry.value
+    states = [self._state(t) for t in tensors]
+    bases = [t._base if t._base is not None else t for t in tensors]
+    key = (tuple((id(b), t.storage_offset()) + s[2:] for b, t, s in zip(bases, tensors, states)), tag)
+    entry = self._entries.get(key)
+    if entry is None or entry.states != states or not all(r() is b for r, b in zip(entry.bases, bases)):
+      entry = self._Entry()
+      entry.bases, entry.states, entry.value = tuple(map(weakref.ref, bases)), states, build()
+      if len(self._entries) >= self._limit:
+        self._entries.clear()
+      self._entries[key] = entry
+    self._latest[tag] = (tuple(map(weakref.ref, tensors)), states, weakref.ref(entry))
+    return entry.value
