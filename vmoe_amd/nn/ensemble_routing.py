@@ -83,7 +83,7 @@ class NoisyTopExpertsPerItemEnsembleRouter(routing.NoisyTopExpertsPerItemRouter)
     if tuple(kernel.shape) != (hidden_size, M, E // M):
       raise ValueError(f"Router kernel has shape {tuple(kernel.shape)}, expected "
                        f"{(hidden_size, M, E // M)}")
-    kernel = routing._cast_kernel(self, kernel, self.dtype or inputs.dtype)   # once for all members
+    kernel = self._cast_kernel(kernel, self.dtype or inputs.dtype)   # once for all members
     rngs = module.make_rngs(rngs, inputs.device)   # one stream, split over the members in order
     x = inputs.reshape(num_groups, group_size // M, M, hidden_size)
     gates_full, per_member = None, []

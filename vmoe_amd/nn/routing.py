@@ -74,7 +74,7 @@ class NoisyTopExpertsPerItemRouter(module.Module):
     module.require_no_grad(type(self).__name__, inputs, kernel)
     dtype = self.dtype or inputs.dtype
     x = K.cast(inputs, dtype)
-    w = _cast_kernel(self, kernel, dtype)
+    w = self._cast_kernel(kernel, dtype)
     if self.deterministic or self.noise_std == 0.0:
       gates, val, idx = K.gate_topk(x, w, self.num_selected_experts, logit_bias=self.logit_bias)
       if not with_metrics:
@@ -105,6 +105,14 @@ class NoisyTopExpertsPerItemRouter(module.Module):
         "load_loss": load_loss,
     }
     return gates_noisy, metrics, (val, idx)
+
+  def _cast_kernel(self, kernel: Array, dtype) -> Array:
+    """The router kernel in the compute dtype; the cast of a parameter tensor is
+    done once and reused until the tensor changes."""
+    if kernel.dtype == dtype:
+      return kernel
+    cache = self.__dict__.setdefault("_kernel_cache", module.ParamCache())
+    return cache.get((kernel,), dtype, lambda: K.cast(kernel, dtype))
 
   def _create_dispatcher(self, gates_dispatch: Array, topk=None, _metrics=None):
     dispatcher_kwargs = dict(**(self.dispatcher or {}))
@@ -148,11 +156,11 @@ class NoisyTopItemsPerExpertRouter(module.Module):
     module.require_no_grad(type(self).__name__, inputs, kernel)
     dtype = self.dtype or inputs.dtype
     if self.deterministic or self.noise_std == 0.0:
-      gates, _, _ = K.gate_topk(K.cast(inputs, dtype), _cast_kernel(self, kernel, dtype), 1)
+      gates, _, _ = K.gate_topk(K.cast(inputs, dtype), K.cast(kernel, dtype), 1)
       return gates
     # vmoe/nn/routing.py:226-232
     noise_std = (1.0 / self.num_experts) * self.noise_std
-    _, _, _, logits = K.gate_topk(K.cast(inputs, dtype), _cast_kernel(self, kernel, dtype), 1,
+    _, _, _, logits = K.gate_topk(K.cast(inputs, dtype), K.cast(kernel, dtype), 1,
                                   return_gates=False, return_logits=True)
     noise = _gating_noise(rngs, logits.shape, logits.device)
     gates_noisy, _ = K.noisy_gates(logits, noise, noise_std, 1, return_load_loss=False)
@@ -166,15 +174,6 @@ class NoisyTopItemsPerExpertRouter(module.Module):
     if use_bfloat16:
       dispatcher = vmoe_amd.moe.Bfloat16Dispatcher(dispatcher)
     return dispatcher, metrics
-
-
-def _cast_kernel(router: module.Module, kernel: Array, dtype) -> Array:
-  """The router kernel in the compute dtype; the cast of a parameter tensor is
-  done once and reused until the tensor changes."""
-  if kernel.dtype == dtype:
-    return kernel
-  cache = router.__dict__.setdefault("_kernel_cache", module.ParamCache())
-  return cache.get((kernel,), dtype, lambda: K.cast(kernel, dtype))
 
 
 def _gating_noise(rngs, shape, device) -> Array:

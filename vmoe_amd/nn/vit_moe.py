@@ -24,8 +24,8 @@ class MlpBlock(module.Module):
   ``{'Dense_0': {'kernel': (D, M), 'bias': (M,)}, 'Dense_1': {'kernel': (M, D), 'bias': (D,)}}``;
   under sparse_moe_spmd every leaf gains a leading expert axis.
 
-  The bf16 kernels read the weights K-contiguous; the transposed copies (and the biases in the
-  compute dtype) are made once per set of parameter tensors and cached.
+  The bf16 kernels read the weights K-contiguous; the transposed copies are made
+  once per parameter tensor and cached.
   """
   _fields = dict(mlp_dim=module._REQUIRED, dtype=None, out_dim=None, dropout_rate=0.0,
                  deterministic=False, approximate_gelu=True)
@@ -51,22 +51,17 @@ class MlpBlock(module.Module):
 
   def _weights(self, p, dtype, stacked: bool = True):
     """Keyword arguments of kernels.expert_mlp that hold the parameters ``p`` in the compute
-    dtype and the kernels' layout, made once per set of parameter tensors.  ``stacked``: the
-    leaves have a leading expert axis (else they are one MLP's)."""
-    leaves = [p[layer].get(leaf) for layer in ("Dense_0", "Dense_1") for leaf in ("kernel", "bias")]
-    present = [t for t in leaves if t is not None]
-    module.require_no_grad("MlpBlock", *present)
-
-    def build():
-      w0, b0, w1, b1 = (t if t is None else K.cast(t if stacked else t[None], dtype) for t in leaves)
-      if dtype == torch.bfloat16:    # the matrix-core kernels read the weights K-contiguous
-        return dict(w0=None, b0=b0, w1=None, b1=b1, w0t=K.pack_expert_weights(w0),
-                    w1t=K.pack_expert_weights(w1))
-      return dict(w0=w0, b0=b0, w1=w1, b1=b1)      # float32 reads the reference's layout
-    if dtype != torch.bfloat16 and all(t.dtype == dtype for t in present):
-      return build()                               # nothing to derive
-    # (which biases are there is part of the tag: the tensors alone do not say whose they are)
-    return self._packed.get(present, (dtype, stacked, leaves[1] is None, leaves[3] is None), build)
+    dtype and the kernels' layout.  ``stacked``: the leaves have a leading expert axis (else
+    they are one MLP's).  Only the transposed copies are kept, one per kernel tensor: a bias is
+    cast on every call, which sees edits that raise no version counter (``b.data.add_``)."""
+    w0, b0, w1, b1 = (p[layer].get(leaf) for layer in ("Dense_0", "Dense_1") for leaf in ("kernel", "bias"))
+    module.require_no_grad("MlpBlock", w0, b0, w1, b1)
+    cast = lambda t: None if t is None else K.cast(t if stacked else t[None], dtype)
+    if dtype != torch.bfloat16:      # float32 reads the reference's layout
+      return dict(w0=cast(w0), b0=cast(b0), w1=cast(w1), b1=cast(b1))
+    # the matrix-core kernels read the weights K-contiguous
+    pack = lambda w, tag: self._packed.get((w,), (tag, stacked), lambda: K.pack_expert_weights(cast(w)))
+    return dict(w0=None, b0=cast(b0), w1=None, b1=cast(b1), w0t=pack(w0, "w0t"), w1t=pack(w1, "w1t"))
 
   supports_packed_rows = True
 
