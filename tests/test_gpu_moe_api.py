@@ -952,6 +952,26 @@ def test_packed_rows_path_equals_reference_layout(moe, dtype, bf16_dispatcher, n
   assert int(rows.sum()) < E * G * buf.shape[1] // G          # capacity 0.75: some slots stay empty
 
 
+@pytest.mark.parametrize("dtype", [O.F32, O.BF16])
+def test_experts_refuse_items_of_two_axes(moe, dtype):
+  """Items (G, S, H, W) pass the dispatchers, which move whole rows, but an MLP over one axis has no
+  meaning for them: ValueError, whatever the product of the axes."""
+  from vmoe_amd.nn import routing, vit_moe
+  G, S, H, W, E, M = 2, 32, 8, 16, 4, 32
+  x = torch.randn((G, S, H, W), device=dev()).to(tdtype(dtype))
+  router = routing.NoisyTopExpertsPerItemRouter(num_experts=E, num_selected_experts=2, deterministic=True,
+                                                dispatcher=dict(name="indices", capacity_factor=1.0,
+                                                                batch_priority=False))
+  dispatcher, _ = router.apply({"params": {"dense": {"kernel": torch.randn((H * W, E), device=dev())}}},
+                               x.view(G, S, H * W))
+  mlp = moe.sparse_moe_spmd(vit_moe.MlpBlock, variable_axes={"params": 0})(mlp_dim=M, dtype=tdtype(dtype))
+  for width in (H, W, H * W):
+    params = {f"Dense_{i}": {"kernel": torch.zeros((E, *((width, M) if i == 0 else (M, width))), device=dev()),
+                             "bias": torch.zeros((E, M if i == 0 else width), device=dev())} for i in range(2)}
+    with pytest.raises(ValueError, match="axes"):
+      mlp.apply({"params": params}, dispatcher, x)
+
+
 # ------------------------------------------------------------------ gradients of dispatch / combine
 @pytest.mark.parametrize("dtype", [O.F32, O.BF16])
 def test_dispatch_combine_gradients(moe, dtype):

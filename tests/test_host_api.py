@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from vmoe_amd import kernels, moe, utils
+from vmoe_amd import _hip, kernels, moe, utils
 from vmoe_amd.nn import module, routing, vit_moe
 from vmoe_amd.projects.soft_moe import router as soft_router
 
@@ -188,3 +188,66 @@ def test_experts_choice_router_kernel_follows_edits_without_a_version(monkeypatc
     router.apply({"params": {"dense": {"kernel": kernel}}}, torch.zeros((1, 8, 16)))
     assert torch.equal(seen[-1], kernel.to(torch.bfloat16))
     kernel.data.add_(1)
+
+
+def _bad_calls():
+  """(name, call): every tensor of a call with an axis too many or too few, then with too few values or
+  the wrong width; shapes that one another's wrapper accepts are in `good`."""
+  i32, f32 = (lambda *s: torch.zeros(s, dtype=torch.int32)), (lambda *s: torch.zeros(s))
+  mlp = dict(x=f32(2, 6, 8), w0=f32(2, 8, 16), b0=f32(2, 16), w1=f32(2, 16, 8), b1=f32(2, 8))
+  packed = dict(x=f32(2, 6, 8), w0=None, b0=f32(2, 16), w1=None, b1=f32(2, 8), w0t=f32(2, 16, 8), w1t=f32(2, 8, 16))
+  gathered = dict(mlp, x=f32(12, 8), x_rows=i32(2, 6), rows_per_expert=i32(2))
+  good = [
+      ("gate_topk", dict(x=f32(2, 6, 8), w=f32(8, 4), num_selected_experts=2, logit_bias=f32(4)),
+       dict(x=[(12, 8), (1, 2, 6, 8)], w=[(8, 4, 1), (4, 4)], logit_bias=[(3,)])),
+      ("route_assign", dict(topk_val=f32(2, 6, 2), topk_idx=i32(2, 6, 2), num_experts=4, capacity=3, batch_priority=True),
+       dict(topk_idx=[(12, 2), (1, 2, 6, 2)], topk_val=[(2, 6, 1)])),
+      ("top_items_metrics", dict(gates=f32(2, 6, 4), capacity=3), dict(gates=[(12, 4), (2, 6, 2, 2)])),
+      ("dispatch", dict(x=f32(6, 8), token_slot=i32(6, 2), slot_token=i32(9)),
+       dict(x=[(6,), (6, 2, 8), (7, 8)], token_slot=[(), (5, 2)], out=[(9, 7)])),
+      ("combine", dict(y=f32(9, 8), token_slot=i32(6, 2), weights=f32(6, 2)),
+       dict(y=[(9,), (9, 2, 8)], token_slot=[(12,), (2, 3, 2)], weights=[(6, 1)], out=[(6, 7)])),
+      ("einsum_dispatch", dict(w=f32(2, 6, 3, 2), data=f32(2, 6, 8), out_dtype=torch.float32),
+       dict(w=[(2, 6, 6), (2, 6, 3, 2, 1)], data=[(), (2, 5, 8)])),
+      ("einsum_combine", dict(w=f32(2, 6, 3, 2), data=f32(12, 8), out_dtype=torch.float32),
+       dict(w=[(2, 6, 6), (2, 6, 3, 2, 1)], data=[(), (11, 8)])),
+      ("combine_backward_data", dict(dout=f32(6, 8), token_slot=i32(6, 2), weights=f32(6, 2), slot_token=i32(9), num_slots=9),
+       dict(dout=[(6,), (6, 2, 8)], token_slot=[(), (5, 2)], weights=[(5, 2)], slot_token=[(8,)])),
+      ("combine_backward_weights", dict(dout=f32(6, 8), y=f32(9, 8), token_slot=i32(6, 2)),
+       dict(dout=[(6,), (6, 2, 8)], y=[(9,), (9, 2, 4), (9, 7)], token_slot=[(), (5, 2)])),
+      ("add_layer_norm", dict(residual=f32(6, 8), branch=f32(6, 8), scale=f32(8), bias=f32(8), eps=1e-6, out_dtype=torch.float32),
+       dict(residual=[()], branch=[(6, 4)], scale=[(7,)], bias=[(7,)])),
+      ("attention", dict(q=f32(2, 5, 3, 64), k=f32(2, 7, 3, 64), v=f32(2, 7, 3, 64), scale=0.125),
+       dict(q=[(2, 5, 192), (1, 2, 5, 3, 64)], k=[(2, 7, 192), (1, 7, 3, 64), (2, 7, 2, 64)],
+            v=[(2, 7, 192), (1, 7, 3, 64), (2, 6, 3, 64)])),
+      ("soft_route", dict(x=f32(2, 6, 8), mu=f32(8, 4), scale=1.0, with_stats=True),
+       dict(x=[(12, 8), (1, 2, 6, 8)], mu=[(8, 2, 2), (7, 4)])),
+      ("expert_mlp", mlp, dict(x=[(12, 8), (2, 3, 2, 8), (2, 6, 4)], w0=[(8, 16), (1, 8, 16), (2, 4, 16)],
+                               w1=[(16, 8), (1, 16, 8), (2, 8, 8), (2, 16, 4)], b0=[(16,)], b1=[(8,)], out=[(2, 6, 7)])),
+      ("expert_mlp", packed, dict(x=[(2, 3, 2, 8)], w0t=[(16, 8), (2, 16, 4), (1, 16, 8)], w1t=[(8, 16), (2, 4, 16), (2, 8, 8)])),
+      ("expert_mlp", gathered, dict(x=[(1, 12, 8), (12,)], x_rows=[(12,), (1, 2, 6)], rows_per_expert=[(1,)])),
+  ]
+  for name, args, bad in good:
+    for arg, shapes in bad.items():
+      like = args.get(arg)
+      for shape in shapes:
+        t = torch.zeros(shape, dtype=torch.float32 if like is None else like.dtype)
+        yield pytest.param(name, dict(args, **{arg: t}), id=f"{name}-{arg}-{'x'.join(map(str, shape)) or 'scalar'}")
+  for what, compact in (("fill-axes", (i32(2), i32(1, 6, 2), 3)), ("slot-axes", (i32(1, 2), i32(6, 2), 3)),
+                        ("groups", (i32(2, 2), i32(1, 6, 2), 3))):
+    yield pytest.param("expert_mlp", dict(mlp, x=f32(12, 8), compact=compact), id=f"expert_mlp-compact-{what}")
+
+
+@pytest.mark.parametrize("name,args", _bad_calls())
+def test_entry_points_refuse_tensors_of_the_wrong_shape(monkeypatch, name, args):
+  """The C ABI is told addresses and sizes: what they are taken from is checked on the host.  (Shapes are
+  looked at before anything else, so CPU tensors do here.)"""
+  monkeypatch.setattr(_hip, "raw_stream", lambda: 0)
+  with pytest.raises(ValueError):
+    getattr(kernels, name)(**args)
+
+
+def test_dispatch_needs_a_number_of_slots(monkeypatch):
+  monkeypatch.setattr(_hip, "raw_stream", lambda: 0)
+  with pytest.raises(TypeError):
+    kernels.dispatch(torch.zeros((6, 8)), torch.zeros((6, 2), dtype=torch.int32), None)

@@ -8,7 +8,9 @@
 // costs its allocations (0.7 us each) and its launch.
 //
 // Every function takes the raw stream first and raises vmoe_amd._hip.VmoeError on an error code, a
-// tensor that is not on the GPU or one that is not contiguous.  Nothing is kept between calls.
+// tensor that is not on the GPU or one that is not contiguous, and ValueError on a tensor with
+// another number of axes than its wrapper names or fewer values than the call would read or write:
+// the C ABI sees addresses and sizes only.  Nothing is kept between calls.
 #include <torch/extension.h>
 
 #include <optional>
@@ -42,6 +44,29 @@ void* ptr(const Tensor& t) {
 void* ptr(const OptTensor& t) { return t.has_value() ? ptr(*t) : nullptr; }
 template <typename T> T* ptr_as(const Tensor& t) { return static_cast<T*>(ptr(t)); }
 template <typename T> T* ptr_as(const OptTensor& t) { return static_cast<T*>(ptr(t)); }
+
+std::string shape_of(const Tensor& t) {
+  std::string s = "(";
+  for (int64_t i = 0; i < t.dim(); ++i) s += (i ? ", " : "") + std::to_string(t.size(i));
+  return s + ")";
+}
+void need_axes(const Tensor& t, int64_t axes, const char* name) {
+  if (t.dim() != axes)
+    throw py::value_error(std::string(name) + " has shape " + shape_of(t) + ", expected " + std::to_string(axes) + " axes");
+}
+void need_values(const Tensor& t, int64_t least, const char* name) {
+  if (t.numel() < least)
+    throw py::value_error(std::string(name) + " has shape " + shape_of(t) + ", expected " + std::to_string(least) + " values");
+}
+void need_values(const OptTensor& t, int64_t least, const char* name) {
+  if (t.has_value()) need_values(*t, least, name);
+}
+// Stacked weights (at least E, rows, cols).
+void need_stack(const OptTensor& t, int64_t E, int64_t rows, int64_t cols, const char* name) {
+  if (t.has_value() && (t->dim() != 3 || t->size(0) < E || t->size(1) != rows || t->size(2) != cols))
+    throw py::value_error(std::string(name) + " has shape " + shape_of(*t) + ", expected (" + std::to_string(E) + ", " +
+                          std::to_string(rows) + ", " + std::to_string(cols) + ")");
+}
 
 vmoe_stream_t stream_of(int64_t raw) { return reinterpret_cast<vmoe_stream_t>(raw); }
 
@@ -77,8 +102,12 @@ Tensor cast(int64_t stream, const Tensor& x_, at::ScalarType type) {
 std::tuple<OptTensor, Tensor, Tensor, OptTensor> gate_topk(
     int64_t stream, const Tensor& x_, const Tensor& w_, int64_t k, const OptTensor& bias_, bool want_gates,
     bool want_logits) {
+  need_axes(x_, 3, "x");
+  need_axes(w_, 2, "w");
   const Tensor x = x_.contiguous(), w = w_.to(x_.scalar_type()).contiguous();
   const int64_t G = x.size(0), S = x.size(1), D = x.size(2), E = w.size(1);
+  need_values(w, D * E, "w");
+  need_values(bias_, E, "logit_bias");
   OptTensor bias = bias_;
   if (bias.has_value()) bias = as_f32(*bias);
   OptTensor gates, logits;
@@ -98,10 +127,12 @@ std::tuple<OptTensor, Tensor, Tensor, OptTensor> gate_topk(
 std::tuple<Tensor, Tensor, Tensor, Tensor, OptTensor, OptTensor, OptTensor> route_assign(
     int64_t stream, const OptTensor& val_, const Tensor& idx_, int64_t E, int64_t C, bool batch_priority,
     const OptTensor& gates_, double w_gshard, double w_importance) {
+  need_axes(idx_, 3, "topk_idx");
   const Tensor idx = idx_.contiguous();
   OptTensor val = val_, gates = gates_;
   if (val.has_value()) val = as_f32(*val);
   const int64_t G = idx.size(0), S = idx.size(1), K = idx.size(2);
+  need_values(val, G * S * K, "topk_val");
   Tensor indices = i32({G, S, K, 2}, idx), token_slot = i32({G, S, K}, idx);
   Tensor slot_token = i32({E * G * C}, idx), fill = i32({G, E}, idx);
   VmoeRouteAssignParams p{};
@@ -135,6 +166,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, OptTensor, OptTensor, OptTensor> rout
 // per expert.
 std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> top_items_metrics(
     int64_t stream, const Tensor& gates_, int64_t C) {
+  need_axes(gates_, 3, "gates");
   const Tensor gates = gates_.contiguous();
   const int64_t G = gates.size(0), S = gates.size(1), E = gates.size(2);
   int64_t num = 2;
@@ -165,6 +197,9 @@ std::tuple<Tensor, Tensor, int64_t, OptTensor, OptTensor, OptTensor, bool> exper
   VmoeCompactRowsParams c{};
   OptTensor token_row, rows = rows_per_expert, row_token = x_rows;
   if (compact) {
+    need_axes(*fill, 2, "fill");
+    need_axes(*token_slot, 3, "token_slot");
+    need_values(*token_slot, fill->size(0) * token_slot->size(1) * token_slot->size(2), "token_slot");
     c.G = (int32_t)fill->size(0); c.E = (int32_t)fill->size(1); c.C = (int32_t)capacity;
     c.S = (int32_t)token_slot->size(1); c.K = (int32_t)token_slot->size(2);
     token_row = i32({c.G, c.S, c.K}, *fill);
@@ -176,14 +211,28 @@ std::tuple<Tensor, Tensor, int64_t, OptTensor, OptTensor, OptTensor, bool> exper
   }
   VmoeExpertMlpParams p{};
   int64_t E, R, D;
+  need_axes(x, row_token.has_value() ? 2 : 3, "x");
   if (row_token.has_value()) {
+    need_axes(*row_token, 2, "x_rows");
     E = row_token->size(0); R = row_token->size(1);
     p.num_items = (int32_t)x.size(0); D = x.size(1);
   } else {
     E = x.size(0); R = x.size(1); D = x.size(2);
   }
   p.E = (int32_t)E; p.R = (int32_t)R; p.D = (int32_t)D;
-  p.M = (int32_t)(w0.has_value() ? w0->size(2) : w0t->size(1));
+  const OptTensor& first = w0.has_value() ? w0 : w0t;
+  if (!first.has_value()) throw py::value_error("neither w0 nor w0t is given");
+  need_axes(*first, 3, w0.has_value() ? "w0" : "w0t");
+  const int64_t M = first->size(w0.has_value() ? 2 : 1);
+  need_stack(w0, E, D, M, "w0");
+  need_stack(w0t, E, M, D, "w0t");
+  need_stack(w1, E, M, D, "w1");
+  need_stack(w1t, E, D, M, "w1t");
+  need_values(b0, E * M, "b0");
+  need_values(b1, E * D, "b1");
+  need_values(rows, E, "rows_per_expert");
+  need_values(out_, E * R * D, "out");
+  p.M = (int32_t)M;
   Tensor out = out_.has_value() ? *out_ : empty({E, R, D}, x.scalar_type(), x);
   p.x = ptr(x); p.w0 = ptr(w0); p.b0 = ptr(b0); p.w1 = ptr(w1); p.b1 = ptr(b1); p.w0t = ptr(w0t); p.w1t = ptr(w1t);
   p.out = ptr(out); p.dtype = dtype_code(x); p.gelu = tanh_gelu ? VMOE_GELU_TANH : VMOE_GELU_ERF;
@@ -213,10 +262,15 @@ std::tuple<Tensor, Tensor, int64_t, OptTensor, OptTensor, OptTensor, bool> exper
 }
 
 Tensor dispatch(int64_t stream, const Tensor& x_, const Tensor& token_slot, const OptTensor& slot_token,
-                const OptTensor& out_, int64_t num_slots) {
+                const OptTensor& out_, std::optional<int64_t> slots) {
+  need_axes(x_, 2, "x");
   const Tensor x = x_.contiguous();
   const int64_t D = x.size(1);
-  if (slot_token.has_value()) num_slots = slot_token->numel();
+  if (!slot_token.has_value() && !slots.has_value()) throw py::type_error("dispatch needs slot_token or num_slots");
+  const int64_t num_slots = slot_token.has_value() ? slot_token->numel() : *slots;
+  if (token_slot.dim() < 1) need_axes(token_slot, 2, "token_slot");
+  need_values(token_slot, x.size(0) * token_slot.size(-1), "token_slot");
+  need_values(out_, num_slots * D, "out");
   Tensor out = out_.has_value() ? *out_ : empty({num_slots, D}, x.scalar_type(), x);
   VmoeDispatchParams p{ptr(x), ptr_as<int32_t>(token_slot), ptr_as<int32_t>(slot_token), ptr(out),
                        (int32_t)x.size(0), (int32_t)num_slots, (int32_t)token_slot.size(-1), (int32_t)D,
@@ -227,8 +281,12 @@ Tensor dispatch(int64_t stream, const Tensor& x_, const Tensor& token_slot, cons
 
 Tensor combine(int64_t stream, const Tensor& y_, const Tensor& token_slot, const Tensor& weights_,
                const OptTensor& out_) {
+  need_axes(y_, 2, "y");
+  need_axes(token_slot, 2, "token_slot");
   const Tensor y = y_.contiguous(), weights = as_f32(weights_);
   const int64_t D = y.size(1), T = token_slot.size(0);
+  need_values(weights, token_slot.numel(), "weights");
+  need_values(out_, T * D, "out");
   Tensor out = out_.has_value() ? *out_ : empty({T, D}, y.scalar_type(), y);
   VmoeCombineParams p{ptr(y), ptr_as<int32_t>(token_slot), ptr_as<float>(weights), ptr(out), (int32_t)T,
                       (int32_t)y.size(0), (int32_t)token_slot.size(1), (int32_t)D, dtype_code(y)};
@@ -240,6 +298,7 @@ Tensor combine(int64_t stream, const Tensor& y_, const Tensor& token_slot, const
 std::tuple<Tensor, OptTensor> add_layer_norm(int64_t stream, const Tensor& residual_, const OptTensor& branch_,
                                              const OptTensor& scale_, const OptTensor& bias_, double eps,
                                              std::optional<at::ScalarType> out_type, bool write_residual) {
+  if (residual_.dim() < 1) need_axes(residual_, 1, "residual");
   const Tensor residual = residual_.contiguous();
   OptTensor branch = branch_, scale = scale_, bias = bias_, sum, norm;
   const int64_t D = residual.size(-1);
@@ -251,6 +310,8 @@ std::tuple<Tensor, OptTensor> add_layer_norm(int64_t stream, const Tensor& resid
     branch = branch->contiguous();
     if (write_residual) sum = at::empty_like(residual);
   }
+  need_values(scale, D, "scale");
+  need_values(bias, D, "bias");
   if (scale.has_value()) scale = as_f32(*scale);
   if (bias.has_value()) bias = as_f32(*bias);
   if (out_type.has_value()) norm = empty(residual.sizes(), *out_type, residual);
@@ -264,7 +325,13 @@ std::tuple<Tensor, OptTensor> add_layer_norm(int64_t stream, const Tensor& resid
 }
 
 Tensor attention(int64_t stream, const Tensor& q, const Tensor& k, const Tensor& v, double scale) {
+  need_axes(q, 4, "q");
+  need_axes(k, 4, "k");
+  need_axes(v, 4, "v");
   const int64_t B = q.size(0), Sq = q.size(1), H = q.size(2), hd = q.size(3);
+  for (const Tensor* t : {&k, &v})
+    if (t->size(0) < B || t->size(1) < k.size(1) || t->size(2) < H)
+      throw py::value_error("keys or values of shape " + shape_of(*t) + " for queries of shape " + shape_of(q));
   for (const Tensor* t : {&q, &k, &v}) {
     if (!t->is_cuda()) raise_error("tensor is not on a ROCm device; there is no CPU fallback");
     if (t->stride(3) != 1 || t->stride(2) != hd)
@@ -291,8 +358,11 @@ int w_code(const Tensor& w) {
 
 // Dense dispatch (G, S, E, C) x (G, S, D) -> (E*G*C, D), or combine -> (G, S, D).
 Tensor einsum(int64_t stream, const Tensor& w_, const Tensor& data_, at::ScalarType out_type, bool is_dispatch) {
+  need_axes(w_, 4, "w");
+  if (data_.dim() < 1) need_axes(data_, is_dispatch ? 3 : 2, "data");
   const Tensor w = w_.contiguous(), data = data_.contiguous();
   const int64_t G = w.size(0), S = w.size(1), E = w.size(2), C = w.size(3), D = data.size(-1);
+  need_values(data, (is_dispatch ? G * S : E * G * C) * D, "data");
   Tensor out = is_dispatch ? empty({E * G * C, D}, out_type, data) : empty({G, S, D}, out_type, data);
   VmoeEinsumParams p{ptr(w), ptr(data), ptr(out), (int32_t)G, (int32_t)S, (int32_t)E, (int32_t)C, (int32_t)D,
                      w_code(w), dtype_code(data), dtype_code(out_type)};
@@ -305,8 +375,11 @@ Tensor einsum(int64_t stream, const Tensor& w_, const Tensor& data_, at::ScalarT
 // parameters (`prepared`, if given, is what an earlier call with the same mu, scale and shapes left).
 std::tuple<Tensor, Tensor, Tensor, Tensor> soft_route_stats(int64_t stream, const Tensor& x_, const Tensor& mu_,
                                                             double scale, const OptTensor& prepared) {
+  need_axes(x_, 3, "x");
+  need_axes(mu_, 2, "mu");
   const Tensor x = x_.contiguous(), mu = mu_.to(x_.scalar_type()).contiguous();
   const int64_t G = x.size(0), S = x.size(1), D = x.size(2), N = mu.size(1);
+  need_values(mu, D * N, "mu");
   Tensor dw = empty({G, S, N}, x.scalar_type(), x), cw = empty({G, S, N}, x.scalar_type(), x);
   Tensor buf = f32({G * 4 + 8}, x);
   VmoeSoftRouteParams p{};
@@ -323,7 +396,12 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> soft_route_stats(int64_t stream, cons
 // -> dy (data) or dweights (weights) of combine.
 Tensor combine_backward_data(int64_t stream, const Tensor& dout_, const Tensor& token_slot, const Tensor& weights_,
                              const OptTensor& slot_token, int64_t num_slots) {
+  need_axes(dout_, 2, "dout");
+  if (token_slot.dim() < 1) need_axes(token_slot, 2, "token_slot");
   const Tensor dout = dout_.contiguous(), weights = as_f32(weights_);
+  need_values(token_slot, dout.size(0) * token_slot.size(-1), "token_slot");
+  need_values(weights, dout.size(0) * token_slot.size(-1), "weights");
+  need_values(slot_token, num_slots, "slot_token");
   Tensor dy = empty({num_slots, dout.size(1)}, dout.scalar_type(), dout);
   VmoeCombineBackwardParams p{};
   p.dout = ptr(dout); p.token_slot = ptr_as<int32_t>(token_slot); p.weights = ptr_as<float>(weights);
@@ -335,7 +413,12 @@ Tensor combine_backward_data(int64_t stream, const Tensor& dout_, const Tensor& 
 }
 
 Tensor combine_backward_weights(int64_t stream, const Tensor& dout_, const Tensor& y_, const Tensor& token_slot) {
+  need_axes(dout_, 2, "dout");
+  need_axes(y_, 2, "y");
+  if (token_slot.dim() < 1) need_axes(token_slot, 2, "token_slot");
   const Tensor dout = dout_.contiguous(), y = y_.contiguous();
+  need_values(token_slot, dout.size(0) * token_slot.size(-1), "token_slot");
+  need_values(y, y.size(0) * dout.size(1), "y");
   Tensor dw = f32({dout.size(0), token_slot.size(-1)}, dout);
   VmoeCombineBackwardParams p{};
   p.dout = ptr(dout); p.y = ptr(y); p.token_slot = ptr_as<int32_t>(token_slot); p.dweights = ptr_as<float>(dw);
