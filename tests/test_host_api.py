@@ -251,3 +251,12 @@ def test_dispatch_needs_a_number_of_slots(monkeypatch):
   monkeypatch.setattr(_hip, "raw_stream", lambda: 0)
   with pytest.raises(TypeError):
     kernels.dispatch(torch.zeros((6, 8)), torch.zeros((6, 2), dtype=torch.int32), None)
+
+
+@pytest.mark.parametrize("shape", [(3, 0), (0,), (0, 0)])
+def test_add_layer_norm_refuses_an_empty_last_axis(monkeypatch, shape):
+  """The number of rows is a quotient: ZeroDivisionError, not a trap."""
+  monkeypatch.setattr(_hip, "raw_stream", lambda: 0)
+  for branch in (None, torch.zeros(shape)):
+    with pytest.raises(ZeroDivisionError):
+      kernels.add_layer_norm(torch.zeros(shape), branch, None, None, 1e-6, torch.float32)

@@ -299,6 +299,10 @@ std::tuple<Tensor, OptTensor> add_layer_norm(int64_t stream, const Tensor& resid
                                              const OptTensor& scale_, const OptTensor& bias_, double eps,
                                              std::optional<at::ScalarType> out_type, bool write_residual) {
   if (residual_.dim() < 1) need_axes(residual_, 1, "residual");
+  if (residual_.size(-1) == 0) {       // (the rows are counted by a division)
+    PyErr_SetString(PyExc_ZeroDivisionError, "residual has an empty last axis");
+    throw py::error_already_set();
+  }
   const Tensor residual = residual_.contiguous();
   OptTensor branch = branch_, scale = scale_, bias = bias_, sum, norm;
   const int64_t D = residual.size(-1);
