@@ -1,6 +1,8 @@
 """Host-side logic of the drop-in surface that needs no GPU: name resolution of routers
 (vmoe/utils.py:59-109, vmoe/nn/vit_moe.py:76-88), capacity arithmetic, the public
 factories, and the refusal to run forward-only kernels under autograd."""
+import threading
+import time
 import weakref
 
 import numpy as np
@@ -260,3 +262,31 @@ def test_add_layer_norm_refuses_an_empty_last_axis(monkeypatch, shape):
   for branch in (None, torch.zeros(shape)):
     with pytest.raises(ZeroDivisionError):
       kernels.add_layer_norm(torch.zeros(shape), branch, None, None, 1e-6, torch.float32)
+
+
+def test_native_host_side_releases_the_interpreter():
+  """Other Python threads run while a native call does its work (here: a copy of a transposed tensor,
+  before the call finds that it is not on the GPU)."""
+  x = torch.zeros((6000, 6000)).t()
+  started, done, ticks = threading.Event(), threading.Event(), []
+
+  def tick():
+    started.set()
+    while not done.wait(0.002):
+      ticks.append(time.perf_counter())
+
+  thread = threading.Thread(target=tick)
+  threads = torch.get_num_threads()
+  torch.set_num_threads(1)
+  try:
+    thread.start()
+    started.wait()
+    begin = time.perf_counter()
+    with pytest.raises(_hip.VmoeError, match="no CPU fallback"):
+      _hip.host().cast(0, x, torch.bfloat16)
+    end = time.perf_counter()
+  finally:
+    torch.set_num_threads(threads)
+    done.set()
+    thread.join()
+  assert sum(begin < t < end for t in ticks) >= 3, (len(ticks), end - begin)

@@ -26,10 +26,17 @@ using OptTensor = std::optional<Tensor>;
 
 PyObject* vmoe_error = nullptr;      // vmoe_amd._hip.VmoeError
 
-[[noreturn]] void raise_error(const std::string& text) {
-  PyErr_SetString(vmoe_error != nullptr ? vmoe_error : PyExc_RuntimeError, text.c_str());
-  throw py::error_already_set();
-}
+// (thrown without the interpreter's lock; set_error runs with it)
+struct VmoeFailure : py::builtin_exception {
+  using builtin_exception::builtin_exception;
+  void set_error() const override { PyErr_SetString(vmoe_error != nullptr ? vmoe_error : PyExc_RuntimeError, what()); }
+};
+struct ZeroDivision : py::builtin_exception {
+  using builtin_exception::builtin_exception;
+  void set_error() const override { PyErr_SetString(PyExc_ZeroDivisionError, what()); }
+};
+
+[[noreturn]] void raise_error(const std::string& text) { throw VmoeFailure(text); }
 
 void check(int code, const char* what) {
   if (code != VMOE_OK)
@@ -73,8 +80,7 @@ vmoe_stream_t stream_of(int64_t raw) { return reinterpret_cast<vmoe_stream_t>(ra
 int dtype_code(at::ScalarType t) {
   if (t == at::kFloat) return VMOE_F32;
   if (t == at::kBFloat16) return VMOE_BF16;
-  PyErr_SetString(PyExc_TypeError, "Unsupported dtype; the kernels cover float32 and bfloat16.");
-  throw py::error_already_set();
+  throw py::type_error("Unsupported dtype; the kernels cover float32 and bfloat16.");
 }
 int dtype_code(const Tensor& t) { return dtype_code(t.scalar_type()); }
 
@@ -146,10 +152,8 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, OptTensor, OptTensor, OptTensor> rout
     check(vmoe_route_assign(&p, stream_of(stream)), "vmoe_route_assign");
   } else {
     gates = gates->contiguous();
-    if (gates->dim() != 3 || gates->size(0) != G || gates->size(1) != S || gates->size(2) != E) {
-      PyErr_SetString(PyExc_ValueError, "gates do not have the shape (G, S, num_experts)");
-      throw py::error_already_set();
-    }
+    if (gates->dim() != 3 || gates->size(0) != G || gates->size(1) != S || gates->size(2) != E)
+      throw py::value_error("gates do not have the shape (G, S, num_experts)");
     imp = f32({G}, idx); gsh = f32({G}, idx); aux = f32({G}, idx);
     VmoeRouterMetricsParams m{};
     m.gates = ptr(gates); m.top1_idx = ptr_as<int32_t>(idx); m.importance_loss = ptr_as<float>(imp);
@@ -299,18 +303,12 @@ std::tuple<Tensor, OptTensor> add_layer_norm(int64_t stream, const Tensor& resid
                                              const OptTensor& scale_, const OptTensor& bias_, double eps,
                                              std::optional<at::ScalarType> out_type, bool write_residual) {
   if (residual_.dim() < 1) need_axes(residual_, 1, "residual");
-  if (residual_.size(-1) == 0) {       // (the rows are counted by a division)
-    PyErr_SetString(PyExc_ZeroDivisionError, "residual has an empty last axis");
-    throw py::error_already_set();
-  }
+  if (residual_.size(-1) == 0) throw ZeroDivision("residual has an empty last axis");   // (rows are a quotient)
   const Tensor residual = residual_.contiguous();
   OptTensor branch = branch_, scale = scale_, bias = bias_, sum, norm;
   const int64_t D = residual.size(-1);
   if (branch.has_value()) {
-    if (branch->sizes() != residual.sizes()) {
-      PyErr_SetString(PyExc_ValueError, "branch and residual have different shapes");
-      throw py::error_already_set();
-    }
+    if (branch->sizes() != residual.sizes()) throw py::value_error("branch and residual have different shapes");
     branch = branch->contiguous();
     if (write_residual) sum = at::empty_like(residual);
   }
@@ -356,8 +354,7 @@ int w_code(const Tensor& w) {
     case at::kBool: return VMOE_W_BOOL;
     default: break;
   }
-  PyErr_SetString(PyExc_TypeError, "Unsupported weight dtype");
-  throw py::error_already_set();
+  throw py::type_error("Unsupported weight dtype");
 }
 
 // Dense dispatch (G, S, E, C) x (G, S, D) -> (E*G*C, D), or combine -> (G, S, D).
@@ -434,28 +431,33 @@ Tensor combine_backward_weights(int64_t stream, const Tensor& dout_, const Tenso
 
 }  // namespace
 
+// Calls run without the interpreter's lock, as ctypes makes them (a launch can wait for room in the
+// queue, an allocation for the device).
+#define VMOE_DEF(name) m.def(#name, torch::wrap_pybind_function_no_gil(&name))
+
 PYBIND11_MODULE(_vmoe_host, m) {
   m.def("set_error", [](py::object e) { vmoe_error = e.release().ptr(); });
   m.def("cast", [](int64_t s, const Tensor& x, py::object t) {
-    return cast(s, x, torch::python::detail::py_object_to_dtype(std::move(t)));
+    return torch::wrap_pybind_function_no_gil(&cast)(s, x, torch::python::detail::py_object_to_dtype(std::move(t)));
   });
-  m.def("gate_topk", &gate_topk);
-  m.def("route_assign", &route_assign);
-  m.def("top_items_metrics", &top_items_metrics);
-  m.def("expert_mlp", &expert_mlp);
-  m.def("dispatch", &dispatch);
-  m.def("combine", &combine);
+  VMOE_DEF(gate_topk);
+  VMOE_DEF(route_assign);
+  VMOE_DEF(top_items_metrics);
+  VMOE_DEF(expert_mlp);
+  VMOE_DEF(dispatch);
+  VMOE_DEF(combine);
   m.def("add_layer_norm", [](int64_t s, const Tensor& r, const OptTensor& b, const OptTensor& sc, const OptTensor& bi,
                              double eps, py::object t, bool w) {
     std::optional<at::ScalarType> type;
     if (!t.is_none()) type = torch::python::detail::py_object_to_dtype(std::move(t));
-    return add_layer_norm(s, r, b, sc, bi, eps, type, w);
+    return torch::wrap_pybind_function_no_gil(&add_layer_norm)(s, r, b, sc, bi, eps, type, w);
   });
-  m.def("attention", &attention);
+  VMOE_DEF(attention);
   m.def("einsum", [](int64_t s, const Tensor& w, const Tensor& d, py::object t, bool dispatch_) {
-    return einsum(s, w, d, torch::python::detail::py_object_to_dtype(std::move(t)), dispatch_);
+    return torch::wrap_pybind_function_no_gil(&einsum)(s, w, d, torch::python::detail::py_object_to_dtype(std::move(t)),
+                                                       dispatch_);
   });
-  m.def("soft_route_stats", &soft_route_stats);
-  m.def("combine_backward_data", &combine_backward_data);
-  m.def("combine_backward_weights", &combine_backward_weights);
+  VMOE_DEF(soft_route_stats);
+  VMOE_DEF(combine_backward_data);
+  VMOE_DEF(combine_backward_weights);
 }
