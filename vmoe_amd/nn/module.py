@@ -105,25 +105,21 @@ class ParamCache:
   class _Entry:
     __slots__ = ("bases", "states", "value", "__weakref__")
 
-  @staticmethod
-  def _state(t: torch.Tensor):
-    return t._version, t.data_ptr(), t.shape, t.stride(), t.dtype, t.device
-
   def get(self, tensors, tag, build):
     tensors = tuple(tensors)
     # The tensors of the last call with this tag, unmodified: what a layer that runs over and over
-    # finds (1 us per tensor; the bases and keys below take as long again).
+    # finds (0.7 us per tensor, twice that with the bases and keys below).  An address belongs to one device.
     latest = self._latest.get(tag)
     if latest is not None and len(latest[0]) == len(tensors):
-      state = self._state
-      for t, ref, known in zip(tensors, latest[0], latest[1]):
-        if ref() is not t or state(t) != known:
+      for t, ref, (version, address, shape, stride, dtype) in zip(tensors, latest[0], latest[1]):
+        if (ref() is not t or t._version != version or t.data_ptr() != address or t.dtype is not dtype
+            or t.shape != shape or t.stride() != stride):
           break
       else:
         entry = latest[2]()
         if entry is not None:
           return entry.value
-    states = [self._state(t) for t in tensors]
+    states = [(t._version, t.data_ptr(), t.shape, t.stride(), t.dtype) for t in tensors]
     bases = [t._base if t._base is not None else t for t in tensors]
     key = (tuple((id(b), t.storage_offset()) + s[2:] for b, t, s in zip(bases, tensors, states)), tag)
     entry = self._entries.get(key)
