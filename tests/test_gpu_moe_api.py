@@ -268,6 +268,57 @@ def test_experts_choice_layer_equals_dispatch_and_combine(G, S, E, D, M, C, dtyp
   assert torch.equal(out, want)
 
 
+def _top_items_gates(G, S, E, equal):
+  """Distinct-ish softmax gates with `equal` items of gate 1/4 in every column."""
+  rng = np.random.default_rng(S + equal)
+  gates = rng.uniform(0.3, 0.9, (G, S, E)).astype(np.float32)
+  for g in range(G):
+    for e in range(E):
+      gates[g, rng.choice(S, equal, replace=False), e] = 0.25
+  return O.cast(gates, O.BF16)
+
+
+@pytest.mark.parametrize("S", [257, 600, 2048, 8192])
+@pytest.mark.parametrize("equal", [255, 256, 257, None])
+def test_top_items_per_expert_equal_gates(S, equal):
+  """Ranks of columns with a run of equal gates as long as is still counted, one longer (which are
+  sorted), and of nothing but equal gates: descending, the lower item first."""
+  from vmoe_amd import kernels as K
+  G, E = 2, 3
+  gates = _top_items_gates(G, S, E, S if equal is None else min(equal, S))
+  C = S // 2 + 1
+  indices, token_slot, slot_token, _, _ = K.top_items_per_expert(to_dev(gates, O.BF16), C)
+  order = np.argsort(-gates.astype(np.float64), axis=1, kind="stable")        # (G, S, E): item of every rank
+  rank = np.empty_like(order)
+  np.put_along_axis(rank, order, np.arange(S)[None, :, None], axis=1)
+  np.testing.assert_array_equal(to_np(indices)[..., 1], rank)
+  want = np.stack([[order[g, :C, e] + g * S for g in range(G)] for e in range(E)])
+  got = to_np(slot_token).reshape(E, G * C)
+  np.testing.assert_array_equal(np.sort(got, axis=1), np.sort(want.reshape(E, G * C), axis=1))
+
+
+def test_top_items_per_expert_equal_gates_cost_no_more_than_a_sort():
+  """A router kernel of zeros makes all gates equal: 8 191 of them take 2.8 times what distinct gates
+  take (the sort, behind the histogram); counted inside one segment they took 98 times as long."""
+  from vmoe_amd import kernels as K
+
+  def best_ms(gates):
+    gates = to_dev(gates, O.BF16)
+    times = []
+    for _ in range(6):
+      start, stop = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+      start.record()
+      for _ in range(4):
+        K.top_items_per_expert(gates, 1024)
+      stop.record()
+      stop.synchronize()
+      times.append(start.elapsed_time(stop))
+    return min(times)
+
+  distinct, equal = best_ms(_top_items_gates(4, 8191, 8, 0)), best_ms(_top_items_gates(4, 8191, 8, 8191))
+  assert equal < 12 * distinct, (equal, distinct)
+
+
 @pytest.mark.parametrize("K_", [1, 3, 4, 8, 9, 64, 65, 256, 257])
 @pytest.mark.parametrize("dtype", [O.F32, O.BF16])
 def test_combine_any_number_of_choices(K_, dtype):

@@ -399,6 +399,10 @@ struct TopItemsMetrics {
 // Bins of the counting rank over every bfloat16 from 1 down to 0.
 constexpr int kGateBins = 16384;
 static_assert(kGateBins > 0x3F80 && kGateBins % (kRouteThreads * 4) == 0, "whole 16-byte pieces per thread");
+// Items of one gate that are counted rather than sorted: with 200 of them 8 x 1 568 x 32 takes 30 us
+// (18 without, 32 sorted behind the histogram), 4 x 8 191 x 8 takes 68 (32, 90).  All gates equal,
+// counted: 166 and 3 143 us.
+constexpr uint32_t kLongestSegment = 256;
 inline __host__ __device__ bool rank_by_counting(int SP, bool bf16) { return bf16 && SP >= 512; }
 
 template <typename T, int R>
@@ -453,8 +457,10 @@ __global__ __launch_bounds__(kRouteThreads) void top_items_kernel(
     // Gates of a bfloat16 softmax take at most 0x3F81 values: rank by histogram, prefix, scatter
     // into the bins' segments and a count inside the item's own segment (see route_assign_group),
     // in place of 66 compare-exchange steps at 2 048 keys.  Below 512 keys clearing the bins costs
-    // what the sort does.
-    if (rank_by_counting(SP, sizeof(T) == 2) && __syncthreads_and(countable)) {
+    // what the sort does.  The count is quadratic in a segment: a column of equal gates (a router kernel
+    // of zeros, tokens that repeat, gates that vanish) takes the sort after all.
+    bool counted = rank_by_counting(SP, sizeof(T) == 2) && __syncthreads_and(countable);
+    if (counted) {
       uint32_t* hist = reinterpret_cast<uint32_t*>(smem);    // items per bin, then the bins' cursors
       uint32_t* seg = hist + kGateBins;                      // S items, bin by bin
       constexpr int kPieces = kGateBins / kRouteThreads / 4; // 16-byte pieces of a thread's bins
@@ -468,11 +474,12 @@ __global__ __launch_bounds__(kRouteThreads) void top_items_kernel(
       __syncthreads();
       {
         uint4 c[kPieces];
-        uint32_t sum = 0;
+        uint32_t sum = 0, longest = 0;
 #pragma unroll
         for (int i = 0; i < kPieces; ++i) {
           c[i] = hist4[tid * kPieces + i];
           sum += c[i].x + c[i].y + c[i].z + c[i].w;
+          longest = max(max(max(longest, c[i].x), max(c[i].y, c[i].z)), c[i].w);
         }
         const int lane = tid & 63, wave = tid >> 6;
         uint32_t incl = sum;
@@ -483,11 +490,11 @@ __global__ __launch_bounds__(kRouteThreads) void top_items_kernel(
         }
         __shared__ uint32_t wave_total[kRouteThreads / 64];
         if (lane == 63) wave_total[wave] = incl;
-        __syncthreads();
+        counted = !__syncthreads_or(longest > kLongestSegment);
         uint32_t at = incl - sum;
         for (int w = 0; w < wave; ++w) at += wave_total[w];
 #pragma unroll
-        for (int i = 0; i < kPieces; ++i) {
+        for (int i = 0; i < kPieces && counted; ++i) {
           const uint4 v = c[i];
           hist4[tid * kPieces + i] = make_uint4(at, at + v.x, at + v.x + v.y, at + v.x + v.y + v.z);
           at += v.x + v.y + v.z + v.w;
@@ -496,22 +503,26 @@ __global__ __launch_bounds__(kRouteThreads) void top_items_kernel(
       __syncthreads();
 #pragma unroll
       for (int r = 0; r < R; ++r)
-        if (tid < nact && tid * R + r < S)
+        if (counted && tid < nact && tid * R + r < S)
           seg[atomicAdd(&hist[0x3F80u - (bits[r] >> 16)], 1u)] = (uint32_t)(tid * R + r);
       __syncthreads();
       // A bin's cursor now stands at its end, which is where the next bin starts.
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const int s = tid * R + r;
-        if (tid < nact && s < S) {
+        if (counted && tid < nact && s < S) {
           const uint32_t bin = 0x3F80u - (bits[r] >> 16);
           const uint32_t first = bin > 0 ? hist[bin - 1] : 0u, end = hist[bin];
           uint32_t lower = 0;
-          for (uint32_t q = first; q < end; ++q) lower += seg[q] < (uint32_t)s ? 1u : 0u;
+          for (uint32_t q = first; q < end; q += 4)          // four reads in flight
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u)
+              lower += seg[min(q + u, end - 1)] < (uint32_t)s && q + u < end ? 1u : 0u;
           emit((int)(first + lower), s);
         }
       }
-    } else {
+    }
+    if (!counted) {
       uint64_t key[R];
 #pragma unroll
       for (int r = 0; r < R; ++r) {
