@@ -972,6 +972,8 @@ def test_expert_mlp_rows_per_expert(K, dtype, E):
     (8, 52, 96, 3072),       # long k over few rows, k not a multiple of 64 in the first product
     (3, 33, 136, 264),       # k that ends inside a 32-wide step
     (70, 3, 64, 200),        # more experts than rows, one short row tile each
+    (3, 1, 800, 136),        # one row that ends in the first half of the last 128-wide k stage
+    (5, 2, 40, 72),          # and rows shorter than that half
 ])
 def test_expert_mlp_small_tiles(K, E, R, D, M):
   """bfloat16 products over few rows per expert (the small tiles, chosen by size) against a float32

@@ -135,7 +135,10 @@ __global__ __launch_bounds__(Cfg::kThreads, 2) void gemm_bf16_rows_kernel(
     }
     a_off[i] = (uint32_t)r * (uint32_t)Kd * 2u + piece * 16u;
   }
-  // Addresses past an operand's end (k past Kd in its last row) read as zero.
+  // Addresses past an operand's end (k past Kd in its last row) read as zero, as long as the scalar
+  // offset itself lies inside the operand: the range check is num_records - offset, unsigned.  A second
+  // half of the last stage may start past Kd, which one row (or a few short ones) may all be: it takes
+  // the row's first half again, and its fragments are cleared like every k past Kd.
   const bf16_t* Ab = a_rows != nullptr ? A : A + (size_t)b * R * Kd;
   const uint32_t a_bytes = (uint32_t)(a_rows != nullptr ? a_items : R) * (uint32_t)Kd * 2u;
   const __amdgpu_buffer_rsrc_t a_rsrc =
@@ -146,7 +149,7 @@ __global__ __launch_bounds__(Cfg::kThreads, 2) void gemm_bf16_rows_kernel(
 #pragma unroll
     for (int h = 0; h < Cfg::KT; ++h) {
       unsigned char* s = smem + stage * Cfg::kStageBytes + h * Cfg::kHalfBytes;
-      const int k_bytes = (kt * Cfg::KT + h) * 128;
+      const int half = kt * Cfg::KT + h, k_bytes = Cfg::KT == 1 || half * 64 < Kd ? half * 128 : 0;
 #pragma unroll
       for (int i = 0; i < Cfg::kBIssues; ++i)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
