@@ -249,6 +249,14 @@ def test_entry_points_refuse_tensors_of_the_wrong_shape(monkeypatch, name, args)
     getattr(kernels, name)(**args)
 
 
+@pytest.mark.parametrize("dtype", [_hip.F32, _hip.BF16])
+@pytest.mark.parametrize("D", [8, 40, 144])
+def test_gathered_rows_of_broken_k_tiles_are_refused(dtype, D):
+  """x_rows asks for whole 32-wide k tiles at every size; refused before anything is launched."""
+  p = _hip.ExpertMlpParams(16, 16, None, 16, None, 16, 16, 16, 16, 1 << 40, 2, 6, D, 64, dtype, _hip.GELU_TANH, 16, 16, 12)
+  assert _hip.lib().vmoe_expert_mlp(_hip.ctypes.byref(p), None) == kernels._E_UNSUPPORTED
+
+
 def test_dispatch_needs_a_number_of_slots(monkeypatch):
   monkeypatch.setattr(_hip, "raw_stream", lambda: 0)
   with pytest.raises(TypeError):

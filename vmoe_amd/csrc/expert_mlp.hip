@@ -519,6 +519,8 @@ static int run_expert_mlp(const VmoeExpertMlpParams* p, vmoe_stream_t stream_, b
   const size_t need = vmoe_expert_mlp_workspace_bytes(p);
   if (p->workspace == nullptr || p->workspace_bytes < need || !aligned16(p->workspace))
     return VMOE_E_WORKSPACE;
+  // Gathered rows come in whole 32-wide k tiles (float32: check_mlp), whichever kernel takes them.
+  if (p->x_rows != nullptr && p->D % 32 != 0) return VMOE_E_UNSUPPORTED;
   hipStream_t stream = as_stream(stream_);
   const size_t b = p->dtype == VMOE_BF16 ? 2 : 4;
   const MlpWorkspace w = mlp_workspace(p);
