@@ -356,8 +356,8 @@ int vmoe_expert_mlp(const VmoeExpertMlpParams* p, vmoe_stream_t stream);
 /* vmoe_compact_rows and the planning launch of vmoe_expert_mlp in one launch (no counterpart
  * in the reference: the packed rows have none).  `mlp` is the parameter block of the MLP call
  * that follows, with its workspace and with rows_per_expert = c->rows_per_expert, x_rows =
- * c->row_token where the first product gathers its rows (only E, R, D, M, dtype, the
- * workspace and rows_per_expert are looked at here); that call is then made as
+ * c->row_token where the first product gathers its rows (only the sizes, dtype, the workspace
+ * and which row tensors are given are looked at here); that call is then made as
  * vmoe_expert_mlp_planned, which takes the launch plans in the workspace as written.
  * VMOE_E_UNSUPPORTED where the compaction needs its two-launch form (E > 256, fewer than 256
  * assignments per group, many groups of few experts) or the MLP plans nothing (float32):
@@ -368,7 +368,8 @@ int vmoe_expert_mlp(const VmoeExpertMlpParams* p, vmoe_stream_t stream);
  * counters it uses).  The plans carry a tag of the shapes they were written for; a call that
  * does not find its own tag (workspace never planned, or planned for other E, R, D, M)
  * launches kernels that do nothing, leaves `out` untouched and counts a plan mismatch in the
- * status words. */
+ * status words.  Where both products run on the small tiles for few rows there is no plan: such a
+ * call takes rows_per_expert and x_rows as they are. */
 int vmoe_compact_rows_planned(const VmoeCompactRowsParams* c, const VmoeExpertMlpParams* mlp,
                               vmoe_stream_t stream);
 int vmoe_expert_mlp_planned(const VmoeExpertMlpParams* p, vmoe_stream_t stream);

@@ -1498,6 +1498,31 @@ def test_expert_mlp_planned_is_repeatable_and_checks_its_plan(K):
   assert (to_np(out) == 7.0).all(), "a launch without a valid plan must not write"
 
 
+@pytest.mark.parametrize("G,S,E,k,C,D,M", [(1, 196, 8, 2, 52, 768, 3072), (2, 300, 5, 3, 200, 128, 192)])
+def test_expert_mlp_planned_over_few_rows(K, G, S, E, k, C, D, M):
+  """Products on the small tiles need no plan: vmoe_compact_rows_planned takes such a call all the
+  same, and expert_mlp_replay_planned repeats it, not an earlier, larger one."""
+  rng = np.random.default_rng(G * S + E)
+  mk = lambda scale, *s: to_dev(O.cast(rng.standard_normal(s) * scale, O.BF16), O.BF16)
+
+  def call(G, S, E, k, C, D, M):
+    val, idx = K.topk(to_dev(O.softmax(rng.standard_normal((G, S, E)).astype(np.float32))), k)
+    _, token_slot, _, fill = K.route_assign(val, idx, E, C, True)
+    return K.expert_mlp(mk(1, G * S, D), None, mk(0.1, E, M), None, mk(0.1, E, D), w0t=mk(D ** -0.5, E, M, D),
+                        w1t=mk(M ** -0.5, E, D, M), compact=(fill, token_slot, C))
+
+  call(4, 1568, 32, 2, 100, 256, 512)
+  out, maps = call(G, S, E, k, C, D, M)
+  want, rows = out.clone(), to_np(maps[1])
+  assert rows.sum() > 0 and not torch.isnan(want).all()
+  out.fill_(7.0)
+  assert K.expert_mlp_replay_planned() is out
+  for e in range(E):
+    np.testing.assert_array_equal(to_np(out[e, :rows[e]]), to_np(want[e, :rows[e]]), err_msg=f"expert {e}")
+    assert (to_np(out[e, rows[e]:]) == 7.0).all(), f"expert {e} wrote past its rows"
+  assert K.expert_mlp_status() == (0, 0)
+
+
 @pytest.mark.parametrize("G,S,D,N", [(6, 196, 768, 128), (3, 250, 768, 128), (2, 37, 384, 40),
                                      (4, 100, 512, 64), (2, 256, 256, 8), (1, 1, 768, 8),
                                      (2, 300, 256, 104), (2, 33, 1024, 128), (2, 64, 768, 20)])

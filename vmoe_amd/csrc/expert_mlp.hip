@@ -327,6 +327,7 @@ struct MlpPlans {
   DownKernel down_kernel = kDownPlain;
   int down_bm = CfgDown::BM;
   size_t up_bytes = 0, down_bytes = 0;   // 0: that product keeps the static tile order
+  bool planned = false;                  // vmoe_expert_mlp_planned takes the call (the small tiles need no plan)
   size_t streamk_bytes = 0;              // exchange memory of kDownShared
 };
 
@@ -410,6 +411,7 @@ MlpPlans mlp_plans(int E, int R, int D, int M, bool ragged, long long items) {
   m.down_bm = m.down_kernel == kDownWide ? WideCfg::BM : CfgDown::BM;
   static_assert(CfgDownNarrow::BM == CfgDown::BM, "row tiles of the narrow kernel");
   m.down_bytes = bytes(m.down);
+  m.planned = m.up_bytes + m.down_bytes > 0;
   if (m.up_rows >= 0) m.up_bytes = 0;
   if (m.down_rows >= 0) m.down_bytes = 0;
   if (m.down_kernel == kDownShared && m.down_rows < 0)
@@ -530,7 +532,7 @@ static int run_expert_mlp(const VmoeExpertMlpParams* p, vmoe_stream_t stream_, b
   void* streamk = w.streamk;
   const MlpPlans& m = w.m;
   unsigned char* ws = w.rest;
-  if (planned_already && w.plan_blocks == 0) return VMOE_E_UNSUPPORTED;
+  if (planned_already && !m.planned) return VMOE_E_UNSUPPORTED;
   if (w.plan_blocks > 0 && !planned_already)
     hipLaunchKernelGGL(plan_ragged_tiles_kernel, dim3(w.plan_blocks), dim3(256),
                        plan_ragged_tiles_lds(p->E), stream, p->rows_per_expert, p->E, p->R, w.ga, w.gb);
@@ -660,11 +662,12 @@ extern "C" int vmoe_compact_rows_planned(const VmoeCompactRowsParams* c,
   if (mlp->workspace == nullptr || mlp->workspace_bytes < vmoe_expert_mlp_workspace_bytes(mlp) ||
       !aligned16(mlp->workspace))
     return VMOE_E_WORKSPACE;
-  // One launch needs the one-launch form of the compaction and an MLP whose products are planned.
+  // One launch needs the one-launch form of the compaction and an MLP whose products are planned or,
+  // over few rows, need no plan.
   if (!compact_rows_fused_ok(c->G, c->S, c->E, c->K) || mlp->dtype != VMOE_BF16)
     return VMOE_E_UNSUPPORTED;
   const MlpWorkspace w = mlp_workspace(mlp);
-  if (w.plan_blocks == 0) return VMOE_E_UNSUPPORTED;
+  if (!w.m.planned) return VMOE_E_UNSUPPORTED;
   const size_t n = (size_t)c->G * c->S * c->K;
   const unsigned compact_blocks = (unsigned)((n + 255) / 256);
   hipLaunchKernelGGL(compact_rows_planned_kernel, dim3(compact_blocks + (unsigned)w.plan_blocks),
