@@ -1008,6 +1008,15 @@ def test_expert_mlp_small_tiles(K, E, R, D, M):
     assert torch.equal(gathered, ragged)
 
 
+@pytest.mark.parametrize("tile", range(8))
+def test_expert_mlp_every_small_tile(K, monkeypatch, tile):
+  """Each tile of the small-tile kernel (VMOE_ROW_TILES names one for both products) through the
+  checks above, at a shape whose row, column and k tiles all end inside and one of a row."""
+  monkeypatch.setenv("VMOE_ROW_TILES", str(tile))
+  test_expert_mlp_small_tiles(K, 3, 131, 136, 264)
+  test_expert_mlp_small_tiles(K, 9, 1, 192, 72)
+
+
 def test_expert_mlp_planned_launch_random_fill(K):
   """bf16 expert products over packed rows with a die-balanced launch plan: random row
   counts (empty, one row, tile boundaries, full), expert counts below and above the
@@ -1033,6 +1042,45 @@ def test_expert_mlp_planned_launch_random_fill(K):
         np.testing.assert_array_equal(to_np(out[e, :n]), to_np(full[e, :n]),
                                       err_msg=f"E={E} R={R} rows={rows.tolist()} expert {e}")
         assert (to_np(out[e, n:]) == 7.0).all(), f"E={E} R={R} rows={rows.tolist()} expert {e}"
+
+
+def test_expert_mlp_planned_launch_random_fill_on_large_tiles(K, monkeypatch):
+  """The same on the tiles that read a plan: these shapes choose the small ones, which need none."""
+  monkeypatch.setenv("VMOE_ROW_TILES", "off")
+  test_expert_mlp_planned_launch_random_fill(K)
+
+
+@pytest.mark.parametrize("E,R,D,M,dtype", [c for c in MLP_CASES if c[-1] == O.BF16])
+def test_expert_mlp_on_large_tiles(K, monkeypatch, E, R, D, M, dtype):
+  monkeypatch.setenv("VMOE_ROW_TILES", "off")
+  test_expert_mlp(K, E, R, D, M, dtype, True)
+
+
+def test_expert_mlp_bfloat16_seeded_shapes_on_large_tiles(K, monkeypatch):
+  """The sweep on the large tiles and, where k is no multiple of 32, the register-staged kernel."""
+  monkeypatch.setenv("VMOE_ROW_TILES", "off")
+  test_expert_mlp_bfloat16_seeded_shapes(K)
+
+
+def test_expert_mlp_operands_of_2_gib(K):
+  """An expert's rows of 2 GiB beside a k that is no multiple of 32: the register-staged kernel (every
+  other size takes a kernel that loads through LDS).  Dense, then with a count that ends inside a tile."""
+  R, D, M = 1 << 27, 8, 8
+  gen = torch.Generator(device=dev()).manual_seed(1)
+  mk = lambda scale, *s: torch.randn(s, generator=gen, device=dev(), dtype=torch.bfloat16) * scale
+  x, w0, b0, w1, b1 = mk(1, 1, R, D), mk(D ** -0.5, 1, D, M), mk(0.1, 1, M), mk(M ** -0.5, 1, M, D), mk(0.1, 1, D)
+  out = K.expert_mlp(x, w0, b0, w1, b1)
+  bf = torch.bfloat16
+  for at in (0, R // 2 - 100, R - 5000):
+    rows = x[0, at:at + 5000].float()
+    h = ((rows @ w0[0].float()).to(bf).float() + b0[0].float()).to(bf)
+    h = torch.nn.functional.gelu(h.float(), approximate="tanh").to(bf)
+    y = ((h.float() @ w1[0].float()).to(bf).float() + b1[0].float()).to(bf)
+    np.testing.assert_allclose(to_np(out[0, at:at + 5000]), to_np(y), rtol=2e-2, atol=5e-2, err_msg=f"rows from {at}")
+  n = R - 77
+  ragged = torch.full_like(out, 7.0)
+  K.expert_mlp(x, w0, b0, w1, b1, out=ragged, rows_per_expert=torch.tensor([n], dtype=torch.int32, device=dev()))
+  assert torch.equal(ragged[0, :n], out[0, :n]) and bool((ragged[0, n:] == 7.0).all())
 
 
 @pytest.mark.parametrize("E,R,D,M", [(64, 384, 1024, 128), (32, 1152, 1024, 256), (90, 384, 520, 160)])
@@ -1120,6 +1168,13 @@ def test_matrix_core_results_are_read_whole(K, E, R, D, M):
   np.testing.assert_array_equal(got, want)
 
 
+@pytest.mark.parametrize("E,R,D,M", [(2, 96, 64, 256), (3, 200, 72, 136), (2, 300, 256, 2048)])
+def test_matrix_core_results_are_read_whole_on_large_tiles(K, monkeypatch, E, R, D, M):
+  """The shapes above that choose the small tiles, on the kernels named beside them."""
+  monkeypatch.setenv("VMOE_ROW_TILES", "off")
+  test_matrix_core_results_are_read_whole(K, E, R, D, M)
+
+
 def test_gating_logits_are_read_whole(K):
   """The gating kernel's matrix-core loop under the same check: integer operands, exact
   float32 logits, all rows (27 and 31 of each 32-item tile first)."""
@@ -1203,6 +1258,7 @@ def test_expert_mlp_with_compaction_in_the_planning_launch(K, monkeypatch, G, S,
     for _ in range(2):
       got, maps = K.expert_mlp(items, None, b0, None, b1, w0t=w0t, w1t=w1t,
                                compact=(fill, token_slot, C))
+      assert (K._last_planned is not None and K._last_planned[8] is got) != separate, "wrong entry points"
       np.testing.assert_array_equal(to_np(maps[0]), to_np(token_row))
       np.testing.assert_array_equal(to_np(maps[1]), to_np(rows))
       r = to_np(rows)
@@ -1212,6 +1268,14 @@ def test_expert_mlp_with_compaction_in_the_planning_launch(K, monkeypatch, G, S,
         np.testing.assert_array_equal(rt_g[e, :r[e]], rt_w[e, :r[e]])
         np.testing.assert_array_equal(g_np[e, :r[e]], w_np[e, :r[e]])
   monkeypatch.delenv("VMOE_PLAN_SEPARATE_LAUNCH", raising=False)
+
+
+@pytest.mark.parametrize("G,S,E,k,C,D,M", [(4, 1568, 32, 2, 100, 256, 512), (2, 1568, 8, 2, 412, 128, 256),
+                                           (3, 300, 5, 3, 200, 128, 192)])
+def test_expert_mlp_with_compaction_in_the_planning_launch_on_large_tiles(K, monkeypatch, G, S, E, k, C, D, M):
+  """The shapes above choose small tiles for one product or both; here the launch plans both."""
+  monkeypatch.setenv("VMOE_ROW_TILES", "off")
+  test_expert_mlp_with_compaction_in_the_planning_launch(K, monkeypatch, G, S, E, k, C, D, M)
 
 
 def test_expert_mlp_hidden_layer_beyond_4_gib(K):
@@ -1457,8 +1521,30 @@ def test_expert_mlp_planned_is_repeatable_and_checks_its_plan(K):
   serving loop, a graph of the experts alone) gives the same output both times -- each call
   resets the exchange counters of its shared round -- and a call on a workspace whose plans
   were never written runs nothing and says so in the status words."""
+  _planned_repeats_and_checks_its_plan(K, 4, 1568, 32, 2, 100, 256, 512)
+
+
+@pytest.mark.parametrize("G,S,E,k,C,D,M,second", [
+    (4, 1568, 32, 2, 100, 256, 512, "shared"),     # 64 tiles of the second product: shared pieces on every die
+    (4, 1568, 32, 2, 100, 256, 512, "eight"),
+    (16, 1568, 8, 2, 400, 768, 1024, None),        # takes the large tiles by itself
+])
+def test_expert_mlp_planned_on_large_tiles_is_repeatable(K, monkeypatch, G, S, E, k, C, D, M, second):
+  """The same where both products read a plan, with the exchange counters of the shared round (its
+  memory is part of the workspace) and without."""
+  if second is not None:
+    monkeypatch.setenv("VMOE_ROW_TILES", "off")
+    need = {}
+    for which in ("shared", "eight"):
+      monkeypatch.setenv("VMOE_SECOND_PRODUCT", which)
+      need[which] = K.expert_mlp_workspace_bytes(E, G * C, D, M, torch.bfloat16, prepacked=True)
+    assert need["shared"] > need["eight"] + (1 << 24), "the shared kernel does not take the shape"
+    monkeypatch.setenv("VMOE_SECOND_PRODUCT", second)
+  _planned_repeats_and_checks_its_plan(K, G, S, E, k, C, D, M)
+
+
+def _planned_repeats_and_checks_its_plan(K, G, S, E, k, C, D, M):
   from vmoe_amd import _hip as H
-  G, S, E, k, C, D, M = 4, 1568, 32, 2, 100, 256, 512     # 64 tiles of the second product: shared pieces on every die
   rng = np.random.default_rng(23)
   gates = O.softmax(rng.standard_normal((G, S, E)).astype(np.float32) * 2)
   val, idx = K.topk(to_dev(gates), k)

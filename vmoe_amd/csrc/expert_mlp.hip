@@ -382,17 +382,26 @@ MlpPlans mlp_plans(int E, int R, int D, int M, bool ragged, long long items) {
   if (narrow_ok && t_narrow < 0.97 * t_best) { m.down_kernel = kDownNarrow; t_best = t_narrow; }
   // Few rows: the small tiles of gemm_bf16_rows.h where their estimate is below that of the large
   // ones (shapes that only the register-staged kernel would take always).
+  // (VMOE_ROW_TILES=off in the environment keeps the large tiles, VMOE_ROW_TILES=<index into kRowsTiles>
+  // takes that tile for both products wherever the kernel takes the operands: the switch behind the
+  // figures of the table, and what tests of the other kernels set)
+  const char* const row_tiles = getenv("VMOE_ROW_TILES");
+  const bool any_tile = row_tiles == nullptr || strcmp(row_tiles, "off") != 0;
+  const int forced = any_tile && row_tiles != nullptr ? atoi(row_tiles) : -1;
+  const bool forced_ok = forced >= 0 && forced < kNumRowsTiles;
   double rows_us = 0;
-  if (rows_gemm_ok(R, M, D, items)) {
+  if (any_tile && rows_gemm_ok(R, M, D, items)) {
     const int tile = best_rows_tile(E, R, M, D, &rows_us);
     if (!m.up.fast || rows_us < product_us(kFirstProductTile, E, R, M, D)) m.up_rows = tile;
+    if (forced_ok) m.up_rows = forced;
   }
-  if (rows_gemm_ok(R, D, M, 0)) {
+  if (any_tile && rows_gemm_ok(R, D, M, 0)) {
     const int tile = best_rows_tile(E, R, D, M, &rows_us);
     if (t_best > 1e29 && square.fast)
       t_best = unit * (half ? 0.5 * 1.05 * std::ceil((double)E * ((R + 127) / 128) * ((D + 255) / 256) / kNumCu)
                             : std::ceil((double)square.tiles / kNumCu));
     if (rows_us < 5 + t_best) m.down_rows = tile;
+    if (forced_ok) m.down_rows = forced;
   }
   // (VMOE_SECOND_PRODUCT=shared|eight|narrow|wide in the environment overrides the choice
   // where the named kernel applies: the switch behind the figures that the model above was

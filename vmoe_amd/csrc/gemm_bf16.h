@@ -1571,6 +1571,9 @@ __global__ __launch_bounds__(Cfg::kThreads, 1) void gemm_bf16_persistent_kernel(
 #endif
 }
 
+// Register-staged 128 x 128 tiles with 64-bit row addresses, for what no LDS-DMA kernel takes: an operand
+// (one expert's rows or weights) of 4 GiB and more, or of 2 GiB and more beside a k that is no multiple of
+// 32 (gemm_bf16_rows.h takes the smaller ones).
 template <int EPI>
 __global__ __launch_bounds__(256) void gemm_bf16_generic_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ Bt, const bf16_t* __restrict__ bias,
