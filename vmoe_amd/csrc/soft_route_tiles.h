@@ -672,12 +672,13 @@ inline int launch_tiles(const T* x, const void* prepared_mu, T* dispatch_w, T* c
       if (vec) return pair ? (Kern)soft_logits_kernel<T, RB, PC, true, true> : (Kern)soft_logits_kernel<T, RB, PC, true, false>;
     return pair ? (Kern)soft_logits_kernel<T, RB, PC, false, true> : (Kern)soft_logits_kernel<T, RB, PC, false, false>;
   };
+  // (64 rows and their logits of 160 slots leave a row two pieces per lane at most, 32 rows in half of LDS four)
   auto by_pieces = [&](auto rb) -> Kern {
+    constexpr int RB = decltype(rb)::value;
     if (pieces <= 1) return pick(rb, std::integral_constant<int, 1>{});
-    if (pieces <= 2) return pick(rb, std::integral_constant<int, 2>{});
-    if (pieces <= 4 || decltype(rb)::value == 4) return pick(rb, std::integral_constant<int, 4>{});
-    return pick(std::integral_constant<int, decltype(rb)::value < 4 ? decltype(rb)::value : 1>{},
-                std::integral_constant<int, 8>{});
+    if (pieces <= 2 || RB == 4) return pick(rb, std::integral_constant<int, 2>{});
+    if (pieces <= 4 || RB == 2) return pick(rb, std::integral_constant<int, RB == 4 ? 2 : 4>{});
+    return pick(rb, std::integral_constant<int, RB == 4 ? 2 : RB == 2 ? 4 : 8>{});
   };
   Kern kern = rb == 4   ? by_pieces(std::integral_constant<int, 4>{})
               : rb == 2 ? by_pieces(std::integral_constant<int, 2>{})
