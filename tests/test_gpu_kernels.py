@@ -501,14 +501,14 @@ SOFT_CASES = [
     (2, 196, 768, 128, 1, O.BF16),
     (4, 100, 256, 16, 2, O.BF16),
     (1, 2, 16, 4, 2, O.F32),          # inputs smaller than mu: the scale multiplies the inputs
-    # every model width of the register-resident bf16 path, ragged S and N
+    # every model width of the two-role bf16 kernel and one more, ragged S and N
     (3, 77, 384, 24, 1, O.BF16),
     (2, 130, 512, 8, 5, O.BF16),
     (2, 33, 1024, 128, 1, O.BF16),
     (1, 300, 256, 104, 1, O.BF16),
     (1, 20, 768, 64, 2, O.BF16),      # inputs smaller than mu on the bf16 path
-    (2, 64, 768, 20, 1, O.BF16),      # N % 8 != 0: generic path
-    (2, 64, 320, 16, 1, O.BF16),      # width outside the fast path
+    (2, 64, 768, 20, 1, O.BF16),      # N % 8 != 0: row tiles
+    (2, 64, 320, 16, 1, O.BF16),      # another width: row tiles
     # two-role kernel with 16-row item tiles (two 32-row tiles do not fit LDS beside the
     # logits): dispatch softmax from registers (S <= 256) and in three passes
     (1, 250, 768, 128, 1, O.BF16),
@@ -547,9 +547,18 @@ def test_soft_route(K, G, S, D, n, p, dtype):
     (2, 31, 102, 33, O.F32),       # rows at unaligned addresses
     (3, 130, 960, 74, O.F32),
     (140, 64, 48, 164, O.F32),     # 64-row tiles
+    (128, 33, 1096, 24, O.BF16),   # 32-row tiles, rows of three pieces per lane
+    (2, 33, 1536, 40, O.BF16),     # 16-row tiles, the same
+    (2, 33, 4096, 24, O.BF16),     # the widest rows that tiles take, eight pieces per lane
+    (3, 20, 2600, 17, O.BF16),
+    (2, 20, 2048, 36, O.F32),
+    (2, 33, 1100, 17, O.F32),
+    (2, 40, 4104, 20, O.BF16),     # wider than any tile: a workgroup per group
+    (3, 37, 2052, 12, O.F32),
+    (1, 40, 4096, 1024, O.BF16),   # or more logits beside such rows than LDS holds
 ])
 def test_soft_route_row_tiles(K, G, S, D, N, dtype):
-  """Shapes whose routing runs over row tiles: logits against float64 within the dtype's
+  """Shapes whose routing runs over row tiles (and the widths past them): logits against float64 within the dtype's
   tolerance, both softmaxes against the float64 softmaxes of the returned logits, the monitoring
   sums against the returned weights; with prepared slot parameters bit for bit the same."""
   rng = np.random.default_rng(G * S + N)
@@ -667,8 +676,8 @@ def test_soft_route_seeded_shapes(K):
 @pytest.mark.parametrize("G,S,D,N", [(5, 196, 768, 128), (2, 250, 768, 128), (3, 100, 512, 64),
                                      (2, 300, 256, 104), (2, 37, 384, 40)])
 def test_soft_route_two_roles_and_single_role_agree(K, G, S, D, N):
-  """The kernel whose waves split into producers and consumers against the single-role kernel
-  (VMOE_SOFT_ROUTE_SINGLE_ROLE=1): same arithmetic per element, different summation order in
+  """The kernel whose waves split into producers and consumers against the row tiles, whose waves have
+  one role (VMOE_SOFT_ROUTE_SINGLE_ROLE=1): same arithmetic per element, different summation order in
   the norms and softmax sums: a norm that rounds the other way moves a normalised item by one
   bfloat16 step, a logit by about as much, and a weight by up to exp(step) - 1, in few places."""
   rng = np.random.default_rng(G * S + N)
@@ -1616,7 +1625,7 @@ def test_soft_route_with_stats(K, G, S, D, N):
   """vmoe_soft_route_stats: the weights are those of vmoe_soft_route bit for bit, and the
   scalars are the means of vmoe/projects/soft_moe/router.py:119-125 of exactly those stored
   weights, whether the routing launch takes the partial sums itself (bfloat16, up to 256 items,
-  widths up to 768) or the separate launches run (the last three shapes)."""
+  widths up to 768) or the separate launch runs (the last three shapes)."""
   rng = np.random.default_rng(G * S + N)
   x = to_dev(O.cast(rng.standard_normal((G, S, D)), O.BF16), O.BF16)
   mu = to_dev(O.cast(rng.standard_normal((D, N)) / np.sqrt(D), O.BF16), O.BF16)
@@ -1633,7 +1642,10 @@ def test_soft_route_with_stats(K, G, S, D, N):
 
 
 @pytest.mark.parametrize("G,S,N,dtype", [(3, 50, 16, O.F32), (4, 196, 128, O.BF16), (2, 7, 300, O.BF16), (3, 196, 128, O.F32),
-                          (2, 9, 96, O.BF16), (5, 33, 8, O.BF16), (2, 300, 512, O.BF16)])
+                          (2, 9, 96, O.BF16), (5, 33, 8, O.BF16), (2, 300, 512, O.BF16),
+                          (2, 9, 8192, O.BF16), (3, 5, 1024, O.F32),
+                          # rows of more than 1 024 pieces, or values where they are no whole pieces
+                          (1, 5, 8200, O.BF16), (2, 9, 1030, O.BF16), (3, 20, 1025, O.F32)])
 def test_soft_router_stats(K, G, S, N, dtype):
   """The four means of vmoe/projects/soft_moe/router.py:119-125 in one kernel."""
   rng = np.random.default_rng(G + S + N)
@@ -1643,3 +1655,75 @@ def test_soft_router_stats(K, G, S, N, dtype):
   want = [cw.min(axis=2).mean(), cw.max(axis=2).mean(), dw.min(axis=1).mean(), dw.max(axis=1).mean()]
   np.testing.assert_allclose(got[:4], want, rtol=2e-6)
   assert got[4] == 0.0   # auxiliary_loss
+
+
+def _wrapper_calls():
+  """(entry points, call(K) -> the tensors that it writes) for every wrapper that has two forms."""
+  gen = torch.Generator(device=dev()).manual_seed(3)
+  bf, f32 = torch.bfloat16, torch.float32
+  mk = lambda dtype, *s: torch.randn(s, generator=gen, device=dev()).to(dtype)
+  G, S, D, E, k, C, M = 3, 98, 128, 8, 2, 28, 192
+  for dtype in (bf, f32):
+    x, w, bias = mk(dtype, G, S, D), mk(dtype, D, E), mk(f32, E)
+    yield "vmoe_gate_topk", lambda K, x=x, w=w, b=bias: K.gate_topk(x, w, k, logit_bias=b)
+    yield "vmoe_gate_topk", lambda K, x=x, w=w: K.gate_topk(x, w, k, return_logits=True)
+    gates = torch.softmax(mk(f32, G, S, E), -1).to(dtype)
+    yield "vmoe_top_items_metrics", lambda K, g=gates: K.top_items_metrics(g, 30)
+    routed = lambda K, g=gates, **kw: K.route_assign(*K.topk(g.float(), k), E, C, True, **kw)
+    yield "vmoe_route_assign", routed
+    yield "vmoe_route_assign_metrics", lambda K, r=routed, g=gates: (lambda o: (*o[:4], *o[4]))(r(K, metrics=(g, 0.3, 0.7)))
+    items, buf, weights = x.view(G * S, D), mk(dtype, E * G * C, D), mk(f32, G * S, k)
+    slots = lambda K, r=routed: (lambda o: (o[1].view(G * S, k), o[2]))(r(K))
+    yield "vmoe_dispatch", lambda K, x=items, t=slots: (K.dispatch(x, *t(K)),)
+    yield "vmoe_combine", lambda K, y=buf, t=slots, w=weights: (K.combine(y, t(K)[0], w),)
+    yield ("vmoe_combine_backward_data", lambda K, x=items, t=slots, w=weights:
+           (K.combine_backward_data(x, t(K)[0], w, t(K)[1], E * G * C),))
+    yield "vmoe_combine_backward_weights", lambda K, x=items, y=buf, t=slots: (K.combine_backward_weights(x, y, t(K)[0]),)
+    wts = mk(dtype, G, S, E, 5)
+    yield "vmoe_einsum_dispatch", lambda K, w=wts, x=x: (K.einsum_dispatch(w, x, x.dtype),)
+    yield "vmoe_einsum_combine", lambda K, w=wts, y=mk(dtype, E * G * 5, D): (K.einsum_combine(w, y, y.dtype),)
+    yield "vmoe_cast", lambda K, x=x: (K.cast(x, f32 if x.dtype == bf else bf),)
+    yield ("vmoe_add_layer_norm", lambda K, r=mk(f32, G, S, D), x=x, s=mk(f32, D), b=mk(f32, D):
+           K.add_layer_norm(r, x, s, b, 1e-6, x.dtype))
+    if dtype == bf:
+      q, kk, v = mk(bf, 2, 37, 3, 64), mk(bf, 2, 41, 3, 64), mk(bf, 2, 41, 3, 64)
+      yield "vmoe_attention", lambda K, q=q, kk=kk, v=v: (K.attention(q, kk, v, 0.125),)
+    yield ("vmoe_soft_route_stats", lambda K, x=x, mu=mk(dtype, D, 24):
+           (lambda o: (*o[:2], *o[2]))(K.soft_route(x, mu, 1.5, with_stats=True)))
+    w0, b0, w1, b1 = mk(dtype, E, D, M), mk(dtype, E, M), mk(dtype, E, M, D), mk(dtype, E, D)
+    mlp = dict(w0=w0, b0=b0, w1=w1, b1=b1)
+    if dtype == bf:
+      mlp = dict(mlp, w0=None, w1=None, w0t=w0.transpose(1, 2).contiguous(), w1t=w1.transpose(1, 2).contiguous())
+    out = lambda dtype=dtype: torch.full((E, G * C, D), 7.0, dtype=dtype, device=dev())
+    yield "vmoe_expert_mlp", lambda K, y=buf, m=mlp, o=out: (K.expert_mlp(y.view(E, G * C, D), out=o(), **m),)
+    rows = torch.tensor([0, 1, 63, 64, 65, 84, 7, 30], dtype=torch.int32, device=dev())
+    picks = torch.randint(0, G * S, (E, G * C), generator=gen, device=dev(), dtype=torch.int32)
+    yield ("vmoe_expert_mlp", lambda K, x=items, m=mlp, o=out, r=rows, p=picks:
+           (K.expert_mlp(x, out=o(), rows_per_expert=r, x_rows=p, **m),))
+
+    def packed(K, x=items, m=mlp, o=out, r=routed):
+      _, token_slot, _, fill = r(K)
+      got, (token_row, n, row_token) = K.expert_mlp(x, out=o(), compact=(fill, token_slot, C), **m)
+      return (got, token_row, n, *(row_token[e, :c] for e, c in enumerate(n.tolist())))
+    yield ("vmoe_compact_rows_planned" if dtype == bf else "vmoe_compact_rows"), packed
+
+
+def test_wrappers_make_the_same_call_from_python_and_natively(K):
+  """Each wrapper of the layers' calls is made through the native host side or, bracketed for a timing
+  sink, from Python: the same entry point with the same parameters, so the same bits."""
+  from vmoe_amd import _hip
+  for name, call in _wrapper_calls():
+    native = call(K)
+    sink = {}
+    _hip.set_timing_sink(sink)
+    try:
+      python = call(K)
+    finally:
+      _hip.set_timing_sink(None)
+    assert len(sink.get(name, ())) >= 1, (name, list(sink))
+    assert len(native) == len(python), name
+    for i, (a, b) in enumerate(zip(native, python)):
+      assert (a is None) == (b is None), (name, i)
+      if a is not None:
+        assert a.dtype == b.dtype and a.shape == b.shape and a.device == b.device, (name, i)
+        assert torch.equal(a, b), (name, i, a.dtype)
