@@ -298,3 +298,19 @@ def test_native_host_side_releases_the_interpreter():
     done.set()
     thread.join()
   assert sum(begin < t < end for t in ticks) >= 3, (len(ticks), end - begin)
+
+
+def test_expert_mlp_sizes_come_from_the_operands(monkeypatch):
+  """The parameter block of a call takes its sizes from the items, not from a caller's output buffer,
+  which may be larger or flat."""
+  from vmoe_amd import _hip as H
+  monkeypatch.setattr(H, "ptr", lambda t: None if t is None else t.data_ptr())
+  E, R, D, M = 3, 5, 16, 32
+  w0t, w1t = torch.zeros(E, M, D), torch.zeros(E, D, M)
+  for out in (torch.zeros(E, R, D), torch.zeros(E + 1, R + 2, D), torch.zeros(E * R, D)):
+    for x, x_rows in ((torch.zeros(E, R, D), None), (torch.zeros(7, D), torch.zeros(E, R, dtype=torch.int32))):
+      p = kernels._expert_mlp_params(x, None, None, None, None, w0t, w1t, True, out, None, x_rows)
+      assert (p.E, p.R, p.D, p.M, p.num_items) == (E, R, D, M, 0 if x_rows is None else 7)
+  with pytest.raises(ValueError):      # gathered items have two axes
+    kernels._expert_mlp_params(torch.zeros(7, D, 2), None, None, None, None, w0t, w1t, True, torch.zeros(E, R, D),
+                         None, torch.zeros(E, R, dtype=torch.int32))

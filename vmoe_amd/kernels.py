@@ -340,8 +340,7 @@ def expert_mlp(x: torch.Tensor, w0, b0, w1, b1, w0t=None, w1t=None, approximate_
     x_rows = _i32(E, G * capacity, device=fill.device)
     maps = (token_row, rows_per_expert, x_rows)
   if x_rows is not None:
-    E, R = x_rows.shape
-    D = x.shape[1]
+    (E, R), (_, D) = x_rows.shape, x.shape
   else:
     E, R, D = x.shape
   x = x.contiguous()
@@ -383,13 +382,16 @@ _last_planned = None
 
 def _expert_mlp_params(x, w0, b0, w1, b1, w0t, w1t, approximate_gelu, out, rows_per_expert, x_rows):
   """The parameter block of a call, its workspace still to be named."""
-  E, R, D = out.shape
+  if x_rows is not None:
+    (E, R), (items, D) = x_rows.shape, x.shape
+  else:
+    (E, R, D), items = x.shape, 0
   M = w0.shape[2] if w0 is not None else w0t.shape[1]
   return H.ExpertMlpParams(H.ptr(x), H.ptr(w0), H.ptr(b0), H.ptr(w1), H.ptr(b1), H.ptr(w0t),
                            H.ptr(w1t), H.ptr(out), None, 0, E, R, D, M, H.dtype_code(x.dtype),
                            H.GELU_TANH if approximate_gelu else H.GELU_ERF,
                            H.ptr(rows_per_expert), H.ptr(x_rows),
-                           0 if x_rows is None else x.shape[0])
+                           items)
 
 
 def expert_mlp_replay_planned() -> torch.Tensor:
