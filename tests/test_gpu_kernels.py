@@ -1618,6 +1618,24 @@ def test_expert_mlp_planned_over_few_rows(K, G, S, E, k, C, D, M):
   assert K.expert_mlp_status() == (0, 0)
 
 
+def test_expert_mlp_replay_of_items_that_are_a_view(K):
+  """A planned call on items that are not contiguous reads a copy of them; repeating it does, too."""
+  G, S, E, k, C, D, M = 4, 392, 8, 2, 100, 256, 512
+  rng = np.random.default_rng(5)
+  mk = lambda scale, *s: to_dev(O.cast(rng.standard_normal(s) * scale, O.BF16), O.BF16)
+  val, idx = K.topk(to_dev(O.softmax(rng.standard_normal((G, S, E)).astype(np.float32))), k)
+  _, token_slot, _, fill = K.route_assign(val, idx, E, C, True)
+  items = mk(1, D, G * S).t()
+  assert not items.is_contiguous()
+  out, maps = K.expert_mlp(items, None, mk(0.1, E, M), None, mk(0.1, E, D), w0t=mk(D ** -0.5, E, M, D),
+                           w1t=mk(M ** -0.5, E, D, M), compact=(fill, token_slot, C))
+  want, rows = out.clone(), to_np(maps[1])
+  out.fill_(7.0)
+  assert K.expert_mlp_replay_planned() is out
+  for e in range(E):
+    np.testing.assert_array_equal(to_np(out[e, :rows[e]]), to_np(want[e, :rows[e]]), err_msg=f"expert {e}")
+
+
 @pytest.mark.parametrize("G,S,D,N", [(6, 196, 768, 128), (3, 250, 768, 128), (2, 37, 384, 40),
                                      (4, 100, 512, 64), (2, 256, 256, 8), (1, 1, 768, 8),
                                      (2, 300, 256, 104), (2, 33, 1024, 128), (2, 64, 768, 20)])

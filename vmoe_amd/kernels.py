@@ -320,6 +320,7 @@ def expert_mlp(x: torch.Tensor, w0, b0, w1, b1, w0t=None, w1t=None, approximate_
   if H._timing_sink is None or not any(map(H.timed, _MLP_CALLS)):
     global _last_planned
     fill, token_slot, capacity = compact or (None, None, 0)
+    x = x.contiguous()          # (what a repeated call reads)
     out, workspace, at, token_row, rows, row_token, planned = H.host().expert_mlp(
         H.raw_stream(), x, w0, b0, w1, b1, w0t, w1t, approximate_gelu, workspace, out,
         rows_per_expert, x_rows, fill, token_slot, capacity,
