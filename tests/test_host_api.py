@@ -314,3 +314,24 @@ def test_expert_mlp_sizes_come_from_the_operands(monkeypatch):
   with pytest.raises(ValueError):      # gathered items have two axes
     kernels._expert_mlp_params(torch.zeros(7, D, 2), None, None, None, None, w0t, w1t, True, torch.zeros(E, R, D),
                          None, torch.zeros(E, R, dtype=torch.int32))
+
+
+def _ragged_mlp_bytes(E, R, D, M):
+  """Workspace of a bfloat16 call with row counts: a product that takes the large tiles keeps a plan in it."""
+  one = _hip.c_void_p(16)
+  p = _hip.ExpertMlpParams(one, None, None, None, None, one, one, one, None, 0, E, R, D, M, _hip.BF16, 0, one, None, 0)
+  return _hip.lib().vmoe_expert_mlp_workspace_bytes(_hip.ctypes.byref(p))
+
+
+@pytest.mark.parametrize("E,R,D,M,small", [
+    (1, 10482, 224, 832, False), (1, 10770, 288, 1088, False), (1, 12229, 288, 1152, False),
+    (3, 3411, 352, 1408, False),                              # two to six (batch, column tile) pairs
+    (1, 196, 768, 3072, True), (8, 52, 768, 3072, True)])
+def test_small_tiles_are_not_taken_where_they_would_run_on_few_dies(monkeypatch, E, R, D, M, small):
+  """gemm_bf16_rows_kernel gives all row tiles of a (batch, column tile) pair to one die: over many rows of a
+  narrow layer most dies have nothing to do, and the large tiles are the faster ones."""
+  monkeypatch.delenv("VMOE_SECOND_PRODUCT", raising=False)
+  monkeypatch.delenv("VMOE_ROW_TILES", raising=False)
+  chosen = _ragged_mlp_bytes(E, R, D, M)
+  monkeypatch.setenv("VMOE_ROW_TILES", "off")
+  assert (chosen < _ragged_mlp_bytes(E, R, D, M)) == small

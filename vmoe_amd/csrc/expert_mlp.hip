@@ -392,7 +392,7 @@ MlpPlans mlp_plans(int E, int R, int D, int M, bool ragged, long long items) {
   double rows_us = 0;
   if (any_tile && rows_gemm_ok(R, M, D, items)) {
     const int tile = best_rows_tile(E, R, M, D, &rows_us);
-    if (!m.up.fast || rows_us < product_us(kFirstProductTile, E, R, M, D)) m.up_rows = tile;
+    if (!m.up.fast || rows_us < product_us(kFirstProductTile, E, R, M, D, false)) m.up_rows = tile;
     if (forced_ok) m.up_rows = forced;
   }
   if (any_tile && rows_gemm_ok(R, D, M, 0)) {

@@ -57,9 +57,13 @@ constexpr RowsTile kFirstProductTile = {128, 256, 2, 4.7, 0.30, 45};     // gemm
 
 // Time in microseconds of a product on tiles of this kind; the memory term is what the weights
 // and rows cost where nothing of them is cached (4.4 TB/s over launches of this length).
-inline double product_us(const RowsTile& t, int batch, int R, int N, int Kd) {
-  const double tiles = (double)batch * ((R + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-  const double full = (double)kCusPerXcd * kNumXcd * t.per_cu;
+// whole_pairs: as gemm_bf16_rows_kernel deals them, all row tiles of a (batch, column tile) pair to one
+// die, whose rounds then count (a launch of two pairs runs on two dies: 10 482 rows x 832 x 224 on
+// 128 x 128 tiles take 37 us, with the large tiles 16); else the tiles fall evenly on all CUs.
+inline double product_us(const RowsTile& t, int batch, int R, int N, int Kd, bool whole_pairs) {
+  const double row_tiles = (R + t.bm - 1) / t.bm, pairs = (double)batch * ((N + t.bn - 1) / t.bn);
+  const double tiles = whole_pairs ? std::ceil(pairs / kNumXcd) * row_tiles : pairs * row_tiles;
+  const double full = (double)kCusPerXcd * t.per_cu * (whole_pairs ? 1 : kNumXcd);
   const int nk = (Kd + 63) / 64;
   auto round = [&](double on_a_cu) {
     return t.fix_us + nk * std::fmax(t.lat_us, on_a_cu * (t.bm + t.bn) * 0.128 / t.gbs);
@@ -74,7 +78,7 @@ inline double product_us(const RowsTile& t, int batch, int R, int N, int Kd) {
 inline int best_rows_tile(int batch, int R, int N, int Kd, double* us) {
   int best = -1;
   for (int i = 0; i < kNumRowsTiles; ++i) {
-    const double t = product_us(kRowsTiles[i], batch, R, N, Kd);
+    const double t = product_us(kRowsTiles[i], batch, R, N, Kd, true);
     if (best < 0 || t < *us) { best = i; *us = t; }
   }
   return best;
