@@ -42,8 +42,10 @@ struct RowsCfg {
 // Tiles that a launch may take, and what the choice between them is made from: the time of a
 // workgroup's round is fix + stages x max(lat, bytes of a 64-wide k tile of the workgroups that
 // share the CU / rate).  Fitted to a sweep over 30 shapes (1 - 64 experts, 16 - 6272 rows, widths
-// 192 - 4096) of both products; the fit is within 10 % (rms), and the tile it picks is on average
-// 4 % slower than the best one.
+// 192 - 4096) of both products.  Estimate against measured time of 30 such shapes on all eight tiles: rms 11 %
+// (first product) and 13 % (second); the tile that the choice takes, the large ones among them, is
+// on average 2.5 and 4 % slower than the fastest, 17 and 40 % at worst (577 rows x 4096 x 1024: 28.9 us
+// on 64 x 64, 20.6 on 64 x 32).
 struct RowsTile {
   int bm, bn, per_cu;
   double fix_us, lat_us, gbs;

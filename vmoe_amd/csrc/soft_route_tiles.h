@@ -11,11 +11,11 @@
 // items, in place; soft_stats_kernel takes the monitoring sums.
 //
 // What bounds it.  64 groups of 196 items x 768 and 256 slots move 39 MB, 6 us of HBM time, in three
-// short launches that are each one round of latencies (25 + 12 + 8 us): every tile reads all slot
+// short launches that are each one round of latencies (29 + 17 + 8 us): every tile reads all slot
 // parameters (390 KB through one CU's L2 port, 8 us), norms and softmaxes are serial behind their
 // loads.  The workgroup per group that this replaces walked its rows with four waves, read the items
 // again for every 128 slots and took the column softmax with one thread per slot: 536 us, and 18 for
-// the sums.  float32, 32 groups of 49 items x 512 and 48 slots: 8 + 8 + 4 us, 186 + 19 before (one
+// the sums.  float32, 32 groups of 49 items x 512 and 48 slots: 10 + 5 + 4 us, 186 + 19 before (one
 // value per lane and MFMA).
 #ifndef VMOE_SOFT_ROUTE_TILES_H_
 #define VMOE_SOFT_ROUTE_TILES_H_
