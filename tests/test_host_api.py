@@ -263,6 +263,14 @@ def test_dispatch_needs_a_number_of_slots(monkeypatch):
     kernels.dispatch(torch.zeros((6, 8)), torch.zeros((6, 2), dtype=torch.int32), None)
 
 
+@pytest.mark.parametrize("num_slots", [9, 9.0, np.float32(9)])
+def test_dispatch_takes_any_number_that_is_an_integer(monkeypatch, num_slots):
+  """int(num_slots), as a capacity computed in floating point asks for: the call gets as far as the device."""
+  monkeypatch.setattr(_hip, "raw_stream", lambda: 0)
+  with pytest.raises(_hip.VmoeError, match="ROCm device"):
+    kernels.dispatch(torch.zeros((6, 8)), torch.zeros((6, 2), dtype=torch.int32), None, num_slots=num_slots)
+
+
 @pytest.mark.parametrize("shape", [(3, 0), (0,), (0, 0)])
 def test_add_layer_norm_refuses_an_empty_last_axis(monkeypatch, shape):
   """The number of rows is a quotient: ZeroDivisionError, not a trap."""

@@ -218,7 +218,8 @@ def dispatch(x: torch.Tensor, token_slot: torch.Tensor, slot_token: Optional[tor
   """x (T,D), token_slot (T,K), slot_token (NS,) -> (NS, D).  With slot_token None (and
   num_slots given) unclaimed rows are left as allocated instead of zeroed."""
   if not H.timed("vmoe_dispatch"):
-    return H.host().dispatch(H.raw_stream(), x, token_slot, slot_token, out, num_slots)
+    return H.host().dispatch(H.raw_stream(), x, token_slot, slot_token, out,
+                             None if num_slots is None else int(num_slots))
   T, D = x.shape
   K = token_slot.shape[-1]
   NS = slot_token.numel() if slot_token is not None else int(num_slots)
