@@ -282,7 +282,7 @@ def soft_run(args, short=False):
       "vs_baseline": None, "dtype": "bf16", "data": "synthetic (seeded N(0,1) tokens and parameters)",
       "config": {"workload": cfg.name, "tokens": T, "d_model": D, "mlp_dim": M, "experts": n,
                  "slots_per_expert": p, "groups": G, "group_size": m},
-      "roofline": {"bound": "hbm", "kernel": "gemm_bf16_mixed_kernel (first product) / gemm_bf16_persistent_kernel (second product)", "achieved": achieved,
+      "roofline": {"bound": "hbm", "kernel": "gemm_bf16_mixed_kernel (first product) / gemm_bf16_w8_kernel<0, true, 6> (second product)", "achieved": achieved,
                    "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": achieved / PEAK_HBM_GBS,
                    "traffic": None, "launch_ms": mlp_ms / 2, "bytes_per_layer": bytes_mlp},
       "stage_ms": stage_ms, "host_enqueue_ms_per_step": host_ms, "wall_ms_per_step": wall_ms,
