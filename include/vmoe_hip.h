@@ -39,6 +39,8 @@ typedef void* vmoe_stream_t;
 
 enum { VMOE_F32 = 0, VMOE_BF16 = 1 };
 enum { VMOE_GELU_TANH = 0, VMOE_GELU_ERF = 1 };
+/* Added to VMOE_GELU_* of a float32 expert MLP: its products run on float32 matrix instructions. */
+enum { VMOE_MLP_F32_PRODUCTS = 256 };
 
 enum {
   VMOE_OK = 0,
@@ -308,6 +310,11 @@ int vmoe_densify(const VmoeDensifyParams* p, vmoe_stream_t stream);
  * off: for every expert e, y = gelu(x @ w0[e] + b0[e]) @ w1[e] + b1[e], all rows.
  * bf16: bf16 operands, float32 accumulate, results rounded to bf16 after each
  * matmul, after each bias add and after the GELU.
+ * float32: every operand value is taken apart into three bfloat16 values that add up to it and
+ * six of the nine products are summed in float32 on the bfloat16 matrix instructions (error
+ * against 64 bits below that of float32 instructions, other rounding).  VMOE_MLP_F32_PRODUCTS
+ * keeps float32 instructions, and with them the order of sums that outputs rounded to bfloat16
+ * further on were made with (Soft MoE's dispatcher: one output in 4 000 rounds the other way).
  * bf16 needs the kernels in K-contiguous order: pass w0t (E,M,D) / w1t (E,D,M)
  * made once by vmoe_pack_expert_weights; if they are null the call packs
  * w0/w1 into `workspace` first (extra HBM pass).  D % 8 == 0 and M % 8 == 0.
@@ -337,7 +344,8 @@ typedef struct {
   size_t workspace_bytes;
   int32_t E, R, D, M;
   int32_t dtype;
-  int32_t gelu;     /* VMOE_GELU_TANH (flax default) or VMOE_GELU_ERF */
+  int32_t gelu;     /* VMOE_GELU_TANH (flax default) or VMOE_GELU_ERF, for float32 also
+                       + VMOE_MLP_F32_PRODUCTS */
   const int32_t* rows_per_expert; /* optional (E,): only the first rows_per_expert[e] rows of
                                      expert e hold data; the other rows of x are not read
                                      for results and their rows of out are left untouched */

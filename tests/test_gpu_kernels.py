@@ -849,6 +849,86 @@ def test_expert_mlp_float32_products_on_the_dma_kernel(K, monkeypatch, E, R, D, 
   np.testing.assert_array_equal(outs["dma"][0], outs["64"][0])              # same order of k
 
 
+@pytest.mark.parametrize("E,R,D,M", [(3, 129, 96, 260), (5, 33, 100, 132), (2, 64, 800, 128), (70, 3, 36, 64)])
+def test_expert_mlp_float32_split_tiles(K, monkeypatch, E, R, D, M):
+  """Every tile of the float32 products on bfloat16 MFMAs (three bfloat16 values per operand), at
+  sizes that end inside a tile of rows, columns or k and for more experts than lanes: no further from
+  64 bits than the float32 MFMA kernel (VMOE_F32_GEMM=plain; 2-norm, a twentieth for the differing
+  order of few sums), also where the operands' scales lie 2^80 apart; ragged rows bit for bit as dense ones,
+  nothing past them; gathered rows bit for bit as rows indexed beforehand."""
+  rng = np.random.default_rng(E + R)
+  up = 2.0 ** 80
+  x = rng.standard_normal((E, R, D)).astype(np.float32)
+  w0 = (rng.standard_normal((E, D, M)) / np.sqrt(D)).astype(np.float32)
+  b0 = (rng.standard_normal((E, M)) * 0.1).astype(np.float32)
+  w1 = (rng.standard_normal((E, M, D)) / np.sqrt(M)).astype(np.float32)
+  b1 = (rng.standard_normal((E, D)) * 0.1).astype(np.float32)
+  rows = rng.integers(0, R + 1, E).astype(np.int32)
+  rows[:2] = [R, 0]
+  items = rng.standard_normal((R + 7, D)).astype(np.float32)
+  x_rows = rng.integers(0, R + 7, (E, R)).astype(np.int32)
+
+  def want(xx):
+    h = xx.astype(np.float64) @ w0.astype(np.float64) + b0[:, None]
+    h = 0.5 * h * (1 + np.tanh(np.sqrt(2 / np.pi) * (h + 0.044715 * h ** 3)))
+    return h @ w1.astype(np.float64) + b1[:, None]
+
+  exact = want(x)
+  off = lambda a: np.linalg.norm(to_np(a) - exact) / np.linalg.norm(exact)
+  rest = [to_dev(a) for a in (w0, b0, w1, b1)]
+  monkeypatch.setenv("VMOE_F32_GEMM", "plain")
+  plain = off(K.expert_mlp(to_dev(x), *rest))
+  for tile in range(6):
+    monkeypatch.setenv("VMOE_F32_GEMM", f"tile{tile}")
+    dense = K.expert_mlp(to_dev(x), *rest)
+    assert off(dense) <= 1.05 * plain, (tile, off(dense), plain)
+    scaled = K.expert_mlp(to_dev((x / up).astype(np.float32)), to_dev((w0 * up).astype(np.float32)), *rest[1:])
+    assert off(scaled) <= 1.05 * plain, (tile, off(scaled), plain)
+    ragged = torch.full((E, R, D), 7.0, device=dev())
+    K.expert_mlp(to_dev(x), *rest, out=ragged, rows_per_expert=to_dev(rows))
+    dense, ragged = to_np(dense), to_np(ragged)
+    for e, n in enumerate(rows):
+      np.testing.assert_array_equal(ragged[e, :n], dense[e, :n], err_msg=f"tile {tile}, expert {e}")
+      assert (ragged[e, n:] == 7.0).all(), f"tile {tile}, expert {e} wrote past its rows"
+    if D % 32 == 0:
+      full = to_dev(np.full(E, R, np.int32))
+      got = K.expert_mlp(to_dev(items), *rest, rows_per_expert=full, x_rows=to_dev(x_rows))
+      ref = K.expert_mlp(to_dev(items[x_rows]), *rest, rows_per_expert=full)
+      np.testing.assert_array_equal(to_np(got), to_np(ref))
+
+
+@pytest.mark.parametrize("tile", range(6))
+def test_expert_mlp_float32_split_tiles_infinities(K, monkeypatch, tile):
+  """Infinite and NaN operands, and finite ones that round to infinity in bfloat16, give what float32
+  multiplication gives (VMOE_F32_GEMM=plain): infinities of the same sign, NaN in the same places, the
+  other items bit for bit what they are without them."""
+  rng = np.random.default_rng(3)
+  E, R, D, M = 2, 70, 64, 132
+  x = rng.standard_normal((E, R, D)).astype(np.float32)
+  w0 = np.abs(rng.standard_normal((E, D, M)) / np.sqrt(D)).astype(np.float32)
+  w1 = (rng.standard_normal((E, M, D)) / np.sqrt(M)).astype(np.float32)
+  w1[:, :, ::2] = np.abs(w1[:, :, ::2])
+  w1[:, :, 1::4] *= -1
+  w1[:, :, 3::4] = -np.abs(w1[:, :, 3::4])
+  w0[1, 5] = 1e-38
+  odd = x.copy()
+  odd[0, 3, 7], odd[0, 69, 0], odd[1, 20, 63], odd[1, 33, 5] = np.inf, -np.inf, np.nan, 3.4e38
+  run = lambda a: to_np(K.expert_mlp(to_dev(a), to_dev(w0), None, to_dev(w1), None))
+  monkeypatch.setenv("VMOE_F32_GEMM", "plain")
+  want = run(odd)
+  monkeypatch.setenv("VMOE_F32_GEMM", f"tile{tile}")
+  got, clean = run(odd), run(x)
+  assert np.isinf(want[0, 3]).any() and np.isnan(want[1, 20]).all() and np.isfinite(want[1, 33]).all()
+  np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+  np.testing.assert_array_equal(np.where(np.isinf(got), got, 0), np.where(np.isinf(want), want, 0))
+  ok = np.isfinite(want)
+  assert_close(got[ok], want[ok], 1e-5, "finite values")
+  same = np.ones((E, R), bool)
+  for e, r in ((0, 3), (0, 69), (1, 20), (1, 33)):
+    same[e, r] = False
+  np.testing.assert_array_equal(got[same], clean[same])
+
+
 def test_expert_mlp_float32_seeded_shapes(K):
   """A seeded sweep of float32 expert MLPs over odd shapes (rows short of a block, widths that
   end inside a tile, k that is or is not whole 32-wide tiles, many or few experts), dense and

@@ -16,6 +16,8 @@ namespace vmoe {
 namespace {
 
 // ---------------------------------------------------------------- float32 path
+// Calls that ask for float32 products and whose shapes the DMA kernel (gemm_f32.h) does not take; also
+// what the other kernels' sums are compared with.
 // C[b] (R x N) = epi(A[b] (R x Kd) . B[b] (Kd x N) + bias[b]) with
 // v_mfma_f32_32x32x2_f32 (IEEE float32 multiply-add).  64x64 tile, 4 waves,
 // B is consumed in the reference's (in, out) order: a lane's B operand is one
@@ -105,22 +107,30 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(
   }
 }
 
+// `f32_products`: the caller asks for float32 MFMAs (VMOE_MLP_F32_PRODUCTS).
 template <int EPI>
 int launch_gemm_f32(const float* A, const float* B, const float* bias, float* C, int batch, int R,
-                    int N, int Kd, hipStream_t stream, const int32_t* rows = nullptr,
+                    int N, int Kd, hipStream_t stream, bool f32_products, const int32_t* rows = nullptr,
                     const int32_t* a_rows = nullptr, int a_items = 0) {
-  // The DMA kernel where its shapes allow: 64 x 128 tiles when they outnumber the CUs twice
-  // over, 64 x 64 otherwise.  VMOE_F32_GEMM=plain keeps the register-staged kernel below.
+  // VMOE_F32_GEMM=plain keeps the products on the register-staged kernel above (which does not gather),
+  // dma on float32 MFMAs with operands by LDS-DMA where its shapes allow, tile<index into kSplitTiles> takes
+  // that tile: the switches behind the figures, and what tests compare.
   const char* which = getenv("VMOE_F32_GEMM");
-  // (gathered rows are the DMA kernel's alone: check_mlp has made sure that it applies)
-  if (gemm_f32_dma_ok(A, B, R, N, Kd, a_items) &&
-      (a_rows != nullptr || !(which != nullptr && strcmp(which, "plain") == 0))) {
+  const bool plain = which != nullptr && strcmp(which, "plain") == 0;
+  const bool dma = f32_products || (which != nullptr && strcmp(which, "dma") == 0);
+  if (!dma && (!plain || a_rows != nullptr)) {
+    const int tile = which != nullptr && strncmp(which, "tile", 4) == 0 ? atoi(which + 4)
+                                                                       : best_split_tile(batch, R, N, Kd);
+    return launch_gemm_f32_split<EPI>(tile, A, B, bias, C, batch, R, N, Kd, stream, rows, a_rows, a_items);
+  }
+  // The DMA kernel where its shapes allow (gathered rows are its alone: check_mlp has made sure that it
+  // applies): 64 x 128 tiles when they outnumber the CUs twice over, 64 x 64 otherwise.
+  if (gemm_f32_dma_ok(A, B, R, N, Kd, a_items) && (a_rows != nullptr || !plain)) {
     const long long wide_tiles = (long long)batch * ((R + 63) / 64) * ((N + 127) / 128);
-    if (wide_tiles >= 2 * kCusPerXcd * kNumXcd && !(which != nullptr && strcmp(which, "64") == 0))
+    if (wide_tiles >= 2 * kCusPerXcd * kNumXcd)
       return launch_gemm_f32_dma<EPI, 128>(A, B, bias, C, batch, R, N, Kd, stream, rows, a_rows, a_items);
     return launch_gemm_f32_dma<EPI, 64>(A, B, bias, C, batch, R, N, Kd, stream, rows, a_rows, a_items);
   }
-  if (a_rows != nullptr) return VMOE_E_UNSUPPORTED;
   const int tiles_m = (R + kF32Tile - 1) / kF32Tile, tiles_n = (N + kF32Tile - 1) / kF32Tile;
   const long long blocks = (long long)batch * tiles_m * tiles_n;
   if (blocks > 0x7fffffffLL) return VMOE_E_OVERFLOW;
@@ -433,6 +443,8 @@ MlpPlans mlp_plans(int E, int R, int D, int M, bool ragged, long long items) {
 
 using namespace vmoe;
 
+static int gelu_of(const VmoeExpertMlpParams* p) { return p->gelu & ~VMOE_MLP_F32_PRODUCTS; }
+
 static int check_mlp(const VmoeExpertMlpParams* p) {
   if (p == nullptr || p->x == nullptr || p->out == nullptr) return VMOE_E_NULL;
   if (p->E < 1 || p->R < 1 || p->D < 1 || p->M < 1) return VMOE_E_SHAPE;
@@ -440,12 +452,13 @@ static int check_mlp(const VmoeExpertMlpParams* p) {
   if (p->x_rows != nullptr) {
     if (p->rows_per_expert == nullptr) return VMOE_E_NULL;
     if (p->num_items < 1) return VMOE_E_SHAPE;
-    // float32: the LDS-DMA kernel gathers (whole 32-wide k tiles, 16-byte aligned operands)
+    // float32 (whole 32-wide k tiles, 16-byte aligned operands)
     if (p->dtype != VMOE_BF16 &&
         !gemm_f32_dma_ok((const float*)p->x, (const float*)p->w0, p->R, p->M, p->D, p->num_items))
       return VMOE_E_UNSUPPORTED;
   }
-  if (p->gelu != VMOE_GELU_TANH && p->gelu != VMOE_GELU_ERF) return VMOE_E_DTYPE;
+  if ((p->gelu & VMOE_MLP_F32_PRODUCTS) != 0 && p->dtype != VMOE_F32) return VMOE_E_DTYPE;
+  if (gelu_of(p) != VMOE_GELU_TANH && gelu_of(p) != VMOE_GELU_ERF) return VMOE_E_DTYPE;
   if (p->dtype == VMOE_BF16) {
     if ((p->w0 == nullptr && p->w0t == nullptr) || (p->w1 == nullptr && p->w1t == nullptr))
       return VMOE_E_NULL;
@@ -545,7 +558,8 @@ static int run_expert_mlp(const VmoeExpertMlpParams* p, vmoe_stream_t stream_, b
   if (w.plan_blocks > 0 && !planned_already)
     hipLaunchKernelGGL(plan_ragged_tiles_kernel, dim3(w.plan_blocks), dim3(256),
                        plan_ragged_tiles_lds(p->E), stream, p->rows_per_expert, p->E, p->R, w.ga, w.gb);
-  const bool tanh_gelu = p->gelu == VMOE_GELU_TANH;
+  const bool tanh_gelu = gelu_of(p) == VMOE_GELU_TANH;
+  const bool f32_products = (p->gelu & VMOE_MLP_F32_PRODUCTS) != 0;
   if (p->dtype == VMOE_BF16) {
     const void* w0t = p->w0t;
     const void* w1t = p->w1t;
@@ -623,14 +637,14 @@ static int run_expert_mlp(const VmoeExpertMlpParams* p, vmoe_stream_t stream_, b
   if (tanh_gelu)
     rc = launch_gemm_f32<kEpiBiasGeluTanh>((const float*)p->x, (const float*)p->w0,
                                            (const float*)p->b0, (float*)hidden, p->E, p->R, p->M,
-                                           p->D, stream, p->rows_per_expert, p->x_rows, p->num_items);
+                                           p->D, stream, f32_products, p->rows_per_expert, p->x_rows, p->num_items);
   else
     rc = launch_gemm_f32<kEpiBiasGeluErf>((const float*)p->x, (const float*)p->w0,
                                           (const float*)p->b0, (float*)hidden, p->E, p->R, p->M,
-                                          p->D, stream, p->rows_per_expert, p->x_rows, p->num_items);
+                                          p->D, stream, f32_products, p->rows_per_expert, p->x_rows, p->num_items);
   if (rc != VMOE_OK) return rc;
   return launch_gemm_f32<kEpiBias>((const float*)hidden, (const float*)p->w1, (const float*)p->b1,
-                                   (float*)p->out, p->E, p->R, p->D, p->M, stream,
+                                   (float*)p->out, p->E, p->R, p->D, p->M, stream, f32_products,
                                    p->rows_per_expert);
 }
 

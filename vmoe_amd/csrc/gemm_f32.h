@@ -1,5 +1,6 @@
 // float32 expert products (vmoe/nn/vit_moe.py:38-45 on float32 parameters) on
-// v_mfma_f32_32x32x2_f32, operands delivered by LDS-DMA.
+// v_mfma_f32_32x32x2_f32, operands delivered by LDS-DMA.  For calls that ask for float32 products
+// (VMOE_MLP_F32_PRODUCTS); the others run on gemm_f32_split.h.
 //
 // C[b] = epilogue(A[b] (R x Kd) . B[b] (Kd x N) + bias[b]); B in the reference's (in, out)
 // order, so a lane's B operand is one scalar B[k][n] and nothing is transposed.
@@ -27,11 +28,10 @@
 // dealt to the sixteen MFMAs as {s, 16 + s} (the products of a k tile commute), so a lane's A
 // operands are 64 contiguous bytes (four 16-byte LDS reads).
 #pragma once
-#include "gemm_bf16.h"
+#include "gemm_f32_split.h"
 
 namespace vmoe {
 
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 template <int BN_>
 struct F32Cfg {

@@ -65,14 +65,19 @@ class MlpBlock(module.Module):
 
   supports_packed_rows = True
 
-  def apply_experts(self, variables, inputs: Array, rows_per_expert: Optional[Array] = None) -> Array:
+  def apply_experts(self, variables, inputs: Array, rows_per_expert: Optional[Array] = None,
+                    float32_products: bool = False) -> Array:
     """inputs (E, R, D) with parameters stacked on axis 0 -> (E, R, D).  With
     rows_per_expert (E,) int32 only that many leading rows of each expert are
-    computed; the other rows of the result are not written."""
+    computed; the other rows of the result are not written.  ``float32_products`` as in
+    kernels.expert_mlp."""
     dtype = self.dtype or inputs.dtype
     module.require_no_grad("MlpBlock", inputs)
     return K.expert_mlp(K.cast(inputs, dtype), **self._weights(variables["params"], dtype),
-                        approximate_gelu=self.approximate_gelu, rows_per_expert=rows_per_expert)
+                        approximate_gelu=self.approximate_gelu, rows_per_expert=rows_per_expert,
+                        float32_products=float32_products)
+
+  apply_experts.takes_float32_products = True
 
   def can_gather(self, items: Array) -> bool:
     """Whether apply_experts_gathered covers these items (dtype and width of the kernel)."""
