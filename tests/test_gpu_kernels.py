@@ -162,6 +162,64 @@ def test_gate_topk_bf16_split_k_form(K, monkeypatch, n, D, E, k):
       np.testing.assert_array_equal(to_np(v_s), to_np(v_d))
 
 
+@pytest.mark.parametrize("n,D,E,k,aligned", [
+    (1, 8, 1, 1, True), (31, 72, 5, 2, True), (33, 264, 12, 3, True), (300, 768, 7, 2, True),
+    (64, 1024, 33, 4, True), (65, 2056, 64, 2, True), (40, 832, 50, 2, True), (255 * 32, 64, 32, 2, False),
+    (255 * 32 + 1, 64, 12, 2, True), (8200, 320, 31, 2, True), (8200, 768, 16, 2, False), (8193, 96, 40, 4, True)])
+def test_gate_topk_bf16_any_expert_count(K, monkeypatch, n, D, E, k, aligned):
+  """bfloat16 gating with router kernels that do not come in aligned blocks of 8 x 8, with more than 32
+  experts or with widths that end inside a chunk: a workgroup per tile (fewer than 256 tiles of 32 items, k in
+  one chunk or several), the streaming form and the direct loads add in the same order, so
+  VMOE_GATE_DIRECT_LOADS=1 gives the same bits, with and without logits, bias and gates."""
+  rng = np.random.default_rng(n + E)
+  x = to_dev(O.cast(rng.standard_normal((1, n, D)), O.BF16), O.BF16)
+  w = to_dev(O.cast(rng.standard_normal(D * E + 1) / np.sqrt(D), O.BF16), O.BF16)
+  w = w[:-1].view(D, E) if aligned else w[1:].view(D, E)
+  b = to_dev(rng.standard_normal(E).astype(np.float32))
+  calls = [dict(return_logits=True), dict(logit_bias=b, return_logits=True), dict(logit_bias=b), dict(return_gates=False)]
+  got = [K.gate_topk(x, w, k, **c) for c in calls]
+  monkeypatch.setenv("VMOE_GATE_DIRECT_LOADS", "1")
+  want = [K.gate_topk(x, w, k, **c) for c in calls]
+  # (E % 8 == 0 on aligned router kernels without logits takes the forms that deal k in another order)
+  other = aligned and E % 8 == 0 and E <= 32 and D % 64 == 0
+  for c, g, r in zip(calls, got, want):
+    for a, e in zip(g, r):
+      if a is not None and not (other and "return_logits" not in c):
+        np.testing.assert_array_equal(to_np(a), to_np(e), err_msg=str(c))
+  want_v, want_i = O.top_k(to_np(got[0][0]), k)
+  np.testing.assert_array_equal(to_np(got[0][2]), want_i)
+  np.testing.assert_array_equal(to_np(got[0][1]), want_v)
+  assert_close(to_np(got[0][0]), O.router_gates(to_np(x), to_np(w), O.BF16), 2e-2, "gates")
+
+
+@pytest.mark.parametrize("n,D,E,k,aligned", [
+    (1, 4, 1, 1, True), (33, 36, 5, 3, True), (100, 832, 38, 2, True), (8200, 544, 6, 1, True), (8193, 100, 33, 4, True),
+    (45, 1028, 128, 4, True), (45, 260, 100, 2, False), (257 * 32, 64, 64, 2, True), (96, 2080, 32, 2, False),
+    (16400, 132, 12, 2, True), (33000, 64, 16, 2, True), (32800, 64, 60, 2, True)])
+def test_gate_topk_float32_any_expert_count(K, n, D, E, k, aligned):
+  """float32 gating: one to eight tiles per workgroup, the router kernel in one chunk of rows or several,
+  any number of experts, router kernels at any float address, widths that end inside a step of k."""
+  rng = np.random.default_rng(n + E)
+  x = rng.standard_normal((1, n, D)).astype(np.float32)
+  w = (rng.standard_normal(D * E + 1) / np.sqrt(D)).astype(np.float32)
+  wd = to_dev(w)
+  w, wd = (w[:-1], wd[:-1]) if aligned else (w[1:], wd[1:])
+  w, wd = w.reshape(D, E), wd.view(D, E)
+  b = rng.standard_normal(E).astype(np.float32)
+  for bias in (None, b):
+    gates, val, idx, logits = K.gate_topk(to_dev(x), wd, k, logit_bias=None if bias is None else to_dev(bias),
+                                          return_logits=True)
+    exact = x[0].astype(np.float64) @ w.astype(np.float64) + (0 if bias is None else bias)
+    np.testing.assert_allclose(to_np(logits)[0], exact, rtol=1e-5, atol=1e-5)
+    assert_close(to_np(gates), O.router_gates(x, w, O.F32, bias), 1e-5, "gates")
+    want_v, want_i = O.top_k(to_np(gates), k)
+    np.testing.assert_array_equal(to_np(idx), want_i)
+    np.testing.assert_array_equal(to_np(val), want_v)
+    g2, v2, i2 = K.gate_topk(to_dev(x), wd, k, logit_bias=None if bias is None else to_dev(bias))
+    for a, e in ((g2, gates), (v2, val), (i2, idx)):
+      np.testing.assert_array_equal(to_np(a), to_np(e))
+
+
 def test_gate_topk_streaming_and_direct_loads_agree(K, monkeypatch):
   """The two forms of the bfloat16 gating kernel (item rows through LDS by DMA, or by direct
   loads: VMOE_GATE_DIRECT_LOADS=1) add the same products in a different order of k: equal

@@ -3,11 +3,11 @@
 //
 // Replaces vmoe/nn/routing.py:73-80 and the jax.lax.top_k of vmoe/moe.py:567.
 //
-// Work split: a wave owns a tile of 32 items.  The router kernel W (D x E) is
-// staged once per workgroup in LDS (bf16: transposed to [expert][k] so that a
-// lane's MFMA B fragment is one 16-byte read; f32: kept [k][expert]).  Item rows
-// stream from HBM with 16-byte loads, 64 contiguous bytes per lane per step; in
-// bf16 they pass through two register buffers that are refilled as soon as their
+// gate_topk_kernel (bfloat16, what the forms below do not take): a wave owns a tile of 32
+// items.  The router kernel W (D x E) is staged once per workgroup in LDS, transposed to
+// [expert][k] so that a lane's MFMA B fragment is one 16-byte read.  Item rows
+// stream from HBM with 16-byte loads, 64 contiguous bytes per lane per step, through two
+// register buffers that are refilled as soon as their
 // MFMAs are issued, and the first loads go out before the router kernel is staged,
 // so that every workgroup of the launch is resident and loading from the start.
 // After the K loop the logits tile passes through a wave-private LDS tile, so
@@ -15,7 +15,8 @@
 // lane, with one xor-32 shuffle per reduction to join the two halves.
 // bfloat16 with up to 32 experts and no logits output takes gate_topk_stream_kernel,
 // which fetches the item rows with coalesced DMA requests into LDS instead, or, with fewer
-// tiles than CUs, gate_topk_split_kernel.
+// tiles than CUs, gate_topk_split_kernel; with fewer tiles than CUs and up to 64 experts also
+// gate_topk_tile_kernel.  float32 takes gate_topk_f32_kernel.
 // (VMOE_GATE_DIRECT_LOADS=1 in the environment keeps the direct loads: the switch behind
 // the before / after figures.)
 #include <algorithm>
@@ -66,45 +67,156 @@ __device__ __forceinline__ uint64_t half_wave_max_u64(uint64_t v) {
   return v;
 }
 
-// LDS row stride (in elements) of the staged router kernel.
-template <typename T> __host__ __device__ constexpr int w_stride(int kc, int epad) {
-  return sizeof(T) == 2 ? kc + 8 : epad;
+// Softmax and top-K of one item by two lanes: g holds the logits of experts h * EP / 2 ..., lane ^ 32 the
+// others.  Sums and maxima are serial per lane; the halves meet with one xor-32 shuffle each.
+template <typename T, int EP>
+__device__ __forceinline__ void finish_row(float (&g)[EP / 2], T* __restrict__ gates, float* __restrict__ topk_val, int32_t* __restrict__ topk_idx,
+                                           int row, int num_items, int E, int K, int h) {
+  constexpr int CNT = EP / 2;
+  const int n0 = h * CNT;
+  const bool row_ok = row < num_items;
+  float mx = -INFINITY;
+#pragma unroll
+  for (int j = 0; j < CNT; ++j) {
+    g[j] = (n0 + j < E) ? g[j] : -INFINITY;
+    mx = fmaxf(mx, g[j]);
+  }
+  mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+  float sum = 0.f;
+#pragma unroll
+  for (int j = 0; j < CNT; ++j) {
+    g[j] = (n0 + j < E) ? expf(g[j] - mx) : 0.f;
+    sum += g[j];
+  }
+  sum += __shfl_xor(sum, 32, kWave);
+#pragma unroll
+  for (int j = 0; j < CNT; ++j) g[j] = Elt<T>::round(g[j] / sum);
+  if (gates != nullptr && row_ok) {
+    T* grow = gates + (size_t)row * E + n0;
+    if (sizeof(T) == 2 && (E & 7) == 0 && (reinterpret_cast<uintptr_t>(gates) & 15u) == 0) {
+#pragma unroll
+      for (int j = 0; j < CNT; j += 8) {
+        if (n0 + j < E) {
+          uint32_t pk[4];
+#pragma unroll
+          for (int t = 0; t < 4; ++t) pk[t] = pack_bf16x2(g[j + 2 * t], g[j + 2 * t + 1]);
+          *reinterpret_cast<uint4*>(grow + j) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
+        }
+      }
+    } else if (sizeof(T) == 4 && (E & 3) == 0 && (reinterpret_cast<uintptr_t>(gates) & 15u) == 0) {
+#pragma unroll
+      for (int j = 0; j < CNT; j += 4)
+        if (n0 + j < E) *reinterpret_cast<float4*>(grow + j) = make_float4(g[j], g[j + 1], g[j + 2], g[j + 3]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < CNT; ++j)
+        if (n0 + j < E) Elt<T>::store(grow + j, g[j]);
+    }
+  }
+  uint64_t taken = 0;
+  for (int kk = 0; kk < K; ++kk) {
+    uint64_t best = 0;
+#pragma unroll
+    for (int j = 0; j < CNT; ++j) {
+      const int n = n0 + j;
+      if (n < E && !(taken >> j & 1ull)) {
+        uint64_t key = ((uint64_t)orderable(g[j]) << 32) | (uint32_t)(0xFFFFFFFFu - (uint32_t)n);
+        best = key > best ? key : best;
+      }
+    }
+    const uint32_t olo = __shfl_xor((uint32_t)best, 32, kWave);
+    const uint32_t ohi = __shfl_xor((uint32_t)(best >> 32), 32, kWave);
+    const uint64_t other = ((uint64_t)ohi << 32) | olo;
+    best = other > best ? other : best;
+    const int n_star = (int)(0xFFFFFFFFu - (uint32_t)best);
+    if (n_star >= n0 && n_star < n0 + CNT) taken |= 1ull << (n_star - n0);
+    if (h == 0 && row_ok) {
+      topk_val[(size_t)row * K + kk] = inv_orderable((uint32_t)(best >> 32));
+      topk_idx[(size_t)row * K + kk] = n_star;
+    }
+  }
 }
 
-template <typename T, int NT, bool LOGITS, int WAVES, bool SPLITK = false>
+// The logits output of a tile of finished logits in LDS (row pitch `pitch`), by one wave.
+__device__ __forceinline__ void store_logits(const float* st, int pitch, float* __restrict__ logits, int row0,
+                                             int num_items, int E, int lane) {
+  const int n = min(32, num_items - row0) * E;
+  float* const out = logits + (size_t)row0 * E;
+  for (int i = lane; i < n; i += kWave) {
+    const int r = i / E;
+    out[i] = st[r * pitch + i - r * E];
+  }
+}
+
+// A 32 x 32 tile of finished bfloat16 logits (row pitch 33).
+__device__ __forceinline__ void finish_tile32(const float* st, bf16_t* __restrict__ gates,
+                                              float* __restrict__ topk_val, int32_t* __restrict__ topk_idx,
+                                              int row0, int num_items, int E, int K, int m, int h) {
+  float g[16];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) g[j] = st[m * 33 + h * 16 + j];
+  finish_row<bf16_t, 32>(g, gates, topk_val, topk_idx, row0 + m, num_items, E, K, h);
+}
+
+// Stages rows k0 .. k0 + kc of a bfloat16 router kernel (D x E) of any E and alignment in LDS as
+// [expert][k]: a unit is eight k of one expert, read as eight 2-byte loads (neighbouring lanes read
+// neighbouring experts) and written as one 16-byte piece.  The loads of four units per thread are in flight
+// at once: every address is clamped into the matrix, so none waits on a branch.  Rows past D are zero;
+// experts past E are left as they are (their logits are never read).
+__device__ __forceinline__ void stage_router_any(const bf16_t* __restrict__ w, bf16_t* wl, int stride, int k0,
+                                                 int kc, int D, int E, int tid, int threads) {
+  constexpr int kBatch = 4;
+  const int units = kc / 8 * E;
+  for (int u0 = tid; u0 < units; u0 += kBatch * threads) {
+    uint32_t raw[kBatch][8];
+    int at[kBatch], left[kBatch];
+#pragma unroll
+    for (int t = 0; t < kBatch; ++t) {
+      const int u = min(u0 + t * threads, units - 1);   // (a thread past the end repeats the last unit)
+      const int kb = u / E, n = u - kb * E, k = k0 + kb * 8;
+      at[t] = n * stride + kb * 8;
+      left[t] = D - k;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) raw[t][i] = w[(size_t)min(k + i, D - 1) * E + n];
+    }
+#pragma unroll
+    for (int t = 0; t < kBatch; ++t) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) raw[t][i] = i < left[t] ? raw[t][i] : 0;
+      *reinterpret_cast<uint4*>(wl + at[t]) = make_uint4(raw[t][0] | raw[t][1] << 16, raw[t][2] | raw[t][3] << 16,
+                                                         raw[t][4] | raw[t][5] << 16, raw[t][6] | raw[t][7] << 16);
+    }
+  }
+}
+
+template <int NT, bool LOGITS, int WAVES>
 __global__ __launch_bounds__(WAVES * kWave) void gate_topk_kernel(
-    const T* __restrict__ x, const T* __restrict__ w, const float* __restrict__ bias,
-    T* __restrict__ gates, float* __restrict__ logits, float* __restrict__ topk_val,
+    const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const float* __restrict__ bias,
+    bf16_t* __restrict__ gates, float* __restrict__ logits, float* __restrict__ topk_val,
     int32_t* __restrict__ topk_idx,
     int num_items, int D, int E, int K, int KC, int num_chunks, int num_tiles, int stage_off) {
   extern __shared__ __align__(16) unsigned char smem[];
-  T* wl = reinterpret_cast<T*>(smem);
+  bf16_t* wl = reinterpret_cast<bf16_t*>(smem);
   constexpr int kGateWaves = WAVES;
   constexpr int kGateThreads = kGateWaves * kWave;
   constexpr int EP = NT * 32;
-  constexpr bool kBf16 = sizeof(T) == 2;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int m = lane & 31;
   const int h = lane >> 5;
-  const int stride = w_stride<T>(KC, EP);
-  // SPLITK (float32, few items): the four waves of a workgroup share one tile of 32 items and
-  // a quarter of D each, and meet in the logits tiles of the epilogue: a launch of a few dozen
-  // tiles is as long as its longest chain of loads and MFMAs, which this cuts in four.
-  static_assert(!SPLITK || (sizeof(T) == 4 && WAVES == 4), "split-k form");
-  const int tiles_per_iter = SPLITK ? gridDim.x : gridDim.x * kGateWaves;
+  const int stride = KC + 8;
+  const int tiles_per_iter = gridDim.x * kGateWaves;
   const int iters = (num_tiles + tiles_per_iter - 1) / tiles_per_iter;
 
   for (int it = 0; it < iters; ++it) {
-    const int tile = SPLITK ? it * tiles_per_iter + blockIdx.x
-                            : it * tiles_per_iter + blockIdx.x * kGateWaves + wave;
+    const int tile = it * tiles_per_iter + blockIdx.x * kGateWaves + wave;
     const bool active = tile < num_tiles;
     const int row0 = tile * 32;
     int r = row0 + m;
     if (r >= num_items) r = num_items - 1;
     if (r < 0) r = 0;
-    const T* xrow = x + (size_t)r * D;
+    const bf16_t* xrow = x + (size_t)r * D;
 
     floatx16 acc[NT];
 #pragma unroll
@@ -116,15 +228,15 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_kernel(
     // batch of item rows go out together, before anything waits: the blocks come back
     // first and are staged under the latency of the rows.
     constexpr int UB = 2;   // 64-k blocks per batch; two batches (16 x 16-byte loads per lane) in flight
-    uint4 wraw[kBf16 ? 8 : 1];
-    uint4 a[kBf16 ? 2 : 1][UB][4];
+    uint4 wraw[8];
+    uint4 a[2][UB][4];
     using Buf0 = std::integral_constant<int, 0>;
-    using Buf1 = std::integral_constant<int, kBf16 ? 1 : 0>;
+    using Buf1 = std::integral_constant<int, 1>;
     auto load_w_block = [&](int k0, int kb, int nb, bool in_range) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const int k = k0 + kb * 8 + i;
-        wraw[kBf16 ? i : 0] = (in_range && k < D && nb * 8 < E)
+        wraw[i] = (in_range && k < D && nb * 8 < E)
                                   ? *reinterpret_cast<const uint4*>(w + (size_t)k * E + nb * 8)
                                   : make_uint4(0, 0, 0, 0);
       }
@@ -157,7 +269,7 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_kernel(
         }
       }
     };
-    if constexpr (kBf16) {
+    {
       if (it == 0 && E % 8 == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0) {
         const int nbn = EP / 8;
         load_w_block(0, tid / nbn, tid % nbn, tid < (KC / 8) * nbn);
@@ -168,34 +280,6 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_kernel(
       }
     }
 
-    // float32: the item rows are loaded four 16-wide k steps at a time, two such batches in
-    // flight (a batch is refilled as soon as its MFMAs are issued); the first two go out before
-    // the router kernel is staged.
-    constexpr int FB = 4;
-    float4 va[kBf16 ? 1 : 2][kBf16 ? 1 : FB][2];
-    int kb_lo = 0, kb_hi = KC / 16;
-    if (SPLITK) {
-      kb_lo = wave * (KC / 16 / kGateWaves);
-      kb_hi = kb_lo + KC / 16 / kGateWaves;
-    }
-    auto load_f = [&](const int u, int k0, int kb0) {
-#pragma unroll
-      for (int t = 0; t < (kBf16 ? 1 : FB); ++t)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int kg = k0 + (kb0 + t) * 16 + h * 8 + j * 4;
-          va[u][t][j] = (kb0 + t < kb_hi && kg + 4 <= D)
-                            ? *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(xrow) + kg)
-                            : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-    };
-    if constexpr (!kBf16) {
-      if (active) {
-        load_f(0, 0, kb_lo);
-        load_f(1, 0, kb_lo + FB);
-      }
-    }
-
     for (int c = 0; c < num_chunks; ++c) {
       const int k0 = c * KC;
       if (num_chunks > 1 || it == 0) {
@@ -203,8 +287,7 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_kernel(
         // Stage W[k0 : k0+KC, :] into LDS, zero padded in both directions.  When
         // a row of W is a whole number of 16-byte vectors the loads are vector
         // loads, all independent, so the staging costs one memory round trip.
-        constexpr int VW = 16 / (int)sizeof(T);
-        if (kBf16 && E % VW == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0) {
+        if (E % 8 == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0) {
           // bf16: a thread loads an 8(k) x 8(expert) block with eight 16-byte loads,
           // transposes it in registers and writes each expert's eight consecutive k
           // as one 16-byte chunk (2-byte LDS writes made this the longest phase of
@@ -230,43 +313,20 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_kernel(
               }
             }
           }
-        } else if (E % VW == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0) {
-          const int vec_per_row = EP / VW;
-          constexpr int kBatch = 6;   // independent loads in flight per thread
-          for (int idx0 = tid; idx0 < KC * vec_per_row; idx0 += kBatch * kGateThreads) {
-            uint4 raw[kBatch];
-#pragma unroll
-            for (int u = 0; u < kBatch; ++u) {
-              const int idx = idx0 + u * kGateThreads;
-              const int k = idx / vec_per_row, n0 = (idx - k * vec_per_row) * VW;
-              raw[u] = make_uint4(0, 0, 0, 0);
-              if (idx < KC * vec_per_row && k0 + k < D && n0 < E)
-                raw[u] = *reinterpret_cast<const uint4*>(w + (size_t)(k0 + k) * E + n0);
-            }
-#pragma unroll
-            for (int u = 0; u < kBatch; ++u) {
-              const int idx = idx0 + u * kGateThreads;
-              if (idx >= KC * vec_per_row) continue;
-              const int k = idx / vec_per_row, n0 = (idx - k * vec_per_row) * VW;
-              const T* v = reinterpret_cast<const T*>(&raw[u]);
-#pragma unroll
-              for (int t = 0; t < VW; ++t) {
-                if (kBf16) wl[(n0 + t) * stride + k] = v[t]; else wl[k * stride + n0 + t] = v[t];
-              }
-            }
-          }
+        } else if constexpr (NT <= 2) {
+          stage_router_any(w, wl, stride, k0, KC, D, E, tid, kGateThreads);
         } else {
           for (int idx = tid; idx < KC * EP; idx += kGateThreads) {
             int k = idx / EP, n = idx - k * EP;
-            T v = 0;
+            bf16_t v = 0;
             if (k0 + k < D && n < E) v = w[(size_t)(k0 + k) * E + n];
-            if (kBf16) wl[n * stride + k] = v; else wl[k * stride + n] = v;
+            wl[n * stride + k] = v;
           }
         }
         __syncthreads();
       }
       if (!active) continue;
-      if constexpr (kBf16) {
+      {
         const int nkb = KC / 64;
         if (c > 0) {
           load_rows(Buf0{}, k0, 0, nkb);
@@ -278,35 +338,6 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_kernel(
           load_rows(Buf0{}, k0, kb0 + 2 * UB, nkb);
           mma_rows(Buf1{}, kb0 + UB, nkb);
           load_rows(Buf1{}, k0, kb0 + 3 * UB, nkb);
-          mfma_result_fence();
-        }
-      } else {
-        auto mma_f = [&](const int u, int kb0) {
-#pragma unroll
-          for (int t = 0; t < FB; ++t) {
-            if (kb0 + t >= kb_hi) break;
-            const int kl = (kb0 + t) * 16 + h * 8;
-            const float a[8] = {va[u][t][0].x, va[u][t][0].y, va[u][t][0].z, va[u][t][0].w,
-                                va[u][t][1].x, va[u][t][1].y, va[u][t][1].z, va[u][t][1].w};
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-#pragma unroll
-              for (int nt = 0; nt < NT; ++nt) {
-                float b = wl[(kl + i) * stride + nt * 32 + m];
-                acc[nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b, acc[nt], 0, 0, 0);
-              }
-            }
-          }
-        };
-        if (c > 0) {
-          load_f(0, k0, kb_lo);
-          load_f(1, k0, kb_lo + FB);
-        }
-        for (int kb0 = kb_lo; kb0 < kb_hi; kb0 += 2 * FB) {
-          mma_f(0, kb0);
-          load_f(0, k0, kb0 + 2 * FB);
-          mma_f(1, kb0 + FB);
-          load_f(1, k0, kb0 + 3 * FB);
           mfma_result_fence();
         }
       }
@@ -331,11 +362,8 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_kernel(
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           const int rl = (i >> 2) * 8 + h * 4 + (i & 3);
-          float v = acc[nt][i];
-          if (!SPLITK) {
-            v = Elt<T>::round(v);
-            if (bias != nullptr) v = Elt<T>::round(v + bn[nt]);
-          }
+          float v = bf16r(acc[nt][i]);
+          if (bias != nullptr) v = bf16r(v + bn[nt]);
           st[rl * (EP + 1) + nt * 32 + m] = v;
         }
     }
@@ -344,26 +372,12 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_kernel(
     const int n0 = h * CNT;
     float g[CNT];
     float mx = -INFINITY;
-    if (SPLITK) {
-      // the four waves' partial logits meet here, added in wave order; wave 0 finishes the tile
-      __syncthreads();
-      if (wave != 0) {
-        __syncthreads();          // the tiles are free again once wave 0 has read them
-        continue;
-      }
-    }
 #pragma unroll
     for (int j = 0; j < CNT; ++j) {
       float v = st[m * (EP + 1) + n0 + j];
-      if (SPLITK) {
-#pragma unroll
-        for (int ww = 1; ww < kGateWaves; ++ww) v += st[(ww * 32 + m) * (EP + 1) + n0 + j];
-        if (bias != nullptr && n0 + j < E) v += bias[n0 + j];
-      }
       g[j] = (n0 + j < E) ? v : -INFINITY;
       mx = fmaxf(mx, g[j]);
     }
-    if (SPLITK) __syncthreads();
     if (LOGITS && row < num_items) {
 #pragma unroll
       for (int j = 0; j < CNT; ++j)
@@ -378,11 +392,11 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_kernel(
     }
     sum += __shfl_xor(sum, 32, kWave);
 #pragma unroll
-    for (int j = 0; j < CNT; ++j) g[j] = Elt<T>::round(g[j] / sum);
+    for (int j = 0; j < CNT; ++j) g[j] = Elt<bf16_t>::round(g[j] / sum);
     const bool row_ok = row < num_items;
     if (gates != nullptr && row_ok) {
-      T* grow = gates + (size_t)row * E + n0;
-      if (kBf16 && (E & 7) == 0 && (reinterpret_cast<uintptr_t>(gates) & 15u) == 0) {
+      bf16_t* grow = gates + (size_t)row * E + n0;
+      if ((E & 7) == 0 && (reinterpret_cast<uintptr_t>(gates) & 15u) == 0) {
 #pragma unroll
         for (int j = 0; j < CNT; j += 8) {
           if (n0 + j < E) {
@@ -395,7 +409,7 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_kernel(
       } else {
 #pragma unroll
         for (int j = 0; j < CNT; ++j)
-          if (n0 + j < E) Elt<T>::store(grow + j, g[j]);
+          if (n0 + j < E) Elt<bf16_t>::store(grow + j, g[j]);
       }
     }
     uint64_t taken = 0;
@@ -423,71 +437,169 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_kernel(
   }
 }
 
-// Softmax and top-K of a 32 x 32 tile of finished logits (row pitch 33) by one wave: a lane holds
-// half (h) of item row0 + m.
-__device__ __forceinline__ void finish_tile32(const float* st, bf16_t* __restrict__ gates,
-                                              float* __restrict__ topk_val, int32_t* __restrict__ topk_idx,
-                                              int row0, int num_items, int E, int K, int m, int h) {
-  constexpr int EP = 32, CNT = EP / 2;
-  const int row = row0 + m;
-  const int n0 = h * CNT;
-  float g[CNT];
-  float mx = -INFINITY;
+// float32 gating on the bfloat16 matrix cores: every value is taken apart into three bfloat16 values that add
+// up to it exactly and six of the nine products are summed in float32, as in gemm_f32_split.h (hi is cut
+// off, not rounded, so that no finite value becomes infinite).  The waves of a workgroup (eight; four beyond 64
+// experts, for the registers) share TW tiles of 32 items, WAVES / TW waves to a tile, each with its share of every chunk of KC rows of the router kernel; the
+// launcher takes as many tiles per workgroup as keep the workgroups at one per CU.  The chunk is split and
+// transposed on its way into LDS, [plane][expert][k], read as eight floats of an expert per thread with
+// neighbouring lanes on neighbouring experts, whatever E and the address are.  Item rows come four 16-wide k
+// steps at a time, two such batches in flight, the first two sent before the chunk is staged.  The partial
+// logits of a tile meet in LDS, added in wave order, and its first wave finishes it.
+// Bound by the trips to memory (few items: 12 - 15 us; 2 688 items x 832, 38 experts: 73 us on float32 MFMAs with a
+// scalar staging loop, 24 here) or by the splitting and the items' bytes (17 024 x 896, 51 experts: 114 to 50;
+// 30 000 x 384, 16 experts: 21 to 19; 15 774 x 544, 6 experts: 35 to 18).
+__device__ __forceinline__ void split3_cut(float v0, float v1, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+  const uint32_t u0 = __builtin_bit_cast(uint32_t, v0), u1 = __builtin_bit_cast(uint32_t, v1);
+  hi = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
+  const float r0 = v0 - __builtin_bit_cast(float, u0 & 0xffff0000u), r1 = v1 - __builtin_bit_cast(float, u1 & 0xffff0000u);
+  mid = pack_bf16x2(r0, r1);
+  lo = pack_bf16x2(r0 - bf_lo(mid), r1 - bf_hi(mid));
+}
+
+constexpr int kNumCus = 256;
+
+template <int NT, int WAVES, int TW>
+__global__ __launch_bounds__(WAVES * kWave) void gate_topk_f32_kernel(
+    const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
+    float* __restrict__ gates, float* __restrict__ logits, float* __restrict__ topk_val,
+    int32_t* __restrict__ topk_idx, int num_items, int D, int E, int K, int KC, int num_chunks, int num_tiles) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  constexpr int KS = WAVES / TW, EP = NT * 32, kThreads = WAVES * kWave, FB = NT == 1 ? 4 : 2;
+  const int stride = KC + 8;                               // bfloat16 per expert and plane
+  bf16_t* const wl = reinterpret_cast<bf16_t*>(smem);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int part = wave % KS, m = lane & 31, h = lane >> 5;
+  float* const st = reinterpret_cast<float*>(smem) + (size_t)wave * 32 * (EP + 1);    // once W has been read
+  const int kb_lo = part * (KC / 16 / KS), kb_hi = kb_lo + KC / 16 / KS;
+
+  for (int tile0 = blockIdx.x * TW; tile0 < num_tiles; tile0 += gridDim.x * TW) {
+    const int tile = tile0 + wave / KS;
+    const int row0 = tile * 32;
+    const float* const xrow = x + (size_t)min(row0 + m, num_items - 1) * D;
+    floatx16 acc[NT];
 #pragma unroll
-  for (int j = 0; j < CNT; ++j) {
-    const float v = st[m * (EP + 1) + n0 + j];
-    g[j] = (n0 + j < E) ? v : -INFINITY;
-    mx = fmaxf(mx, g[j]);
-  }
-  mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
-  float sum = 0.f;
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-  for (int j = 0; j < CNT; ++j) {
-    g[j] = (n0 + j < E) ? expf(g[j] - mx) : 0.f;
-    sum += g[j];
-  }
-  sum += __shfl_xor(sum, 32, kWave);
+      for (int i = 0; i < 16; ++i) acc[nt][i] = 0.f;
+    float4 va[2][FB][2];
+    // (what lies past the wave's share or past D is read from the row's end and multiplied by the zero
+    // rows of W or not at all)
+    auto load_rows = [&](const int u, int k0, int kb0) {
 #pragma unroll
-  for (int j = 0; j < CNT; ++j) g[j] = bf16r(g[j] / sum);
-  const bool row_ok = row < num_items;
-  if (gates != nullptr && row_ok) {
-    bf16_t* grow = gates + (size_t)row * E + n0;
-    if ((reinterpret_cast<uintptr_t>(gates) & 15u) == 0) {
+      for (int t = 0; t < FB; ++t)
 #pragma unroll
-      for (int j = 0; j < CNT; j += 8) {
-        if (n0 + j < E) {
-          uint32_t pk[4];
+        for (int j = 0; j < 2; ++j)
+          va[u][t][j] = *reinterpret_cast<const float4*>(xrow + min(k0 + (kb0 + t) * 16 + h * 8 + j * 4, D - 4));
+    };
+    auto mma_rows = [&](const int u, int k0, int kb0) {
 #pragma unroll
-          for (int t = 0; t < 4; ++t) pk[t] = pack_bf16x2(g[j + 2 * t], g[j + 2 * t + 1]);
-          *reinterpret_cast<uint4*>(grow + j) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
+      for (int t = 0; t < FB; ++t) {
+        if (kb0 + t >= kb_hi) break;
+        const int kl = (kb0 + t) * 16 + h * 8;
+        uint32_t a[3][4];
+        const float v[8] = {va[u][t][0].x, va[u][t][0].y, va[u][t][0].z, va[u][t][0].w,
+                            va[u][t][1].x, va[u][t][1].y, va[u][t][1].z, va[u][t][1].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const bool in = k0 + kl + (i & 2) * 2 < D;       // (whole quads: D is a multiple of four)
+          split3_cut(in ? v[2 * i] : 0.f, in ? v[2 * i + 1] : 0.f, a[0][i], a[1][i], a[2][i]);
+        }
+        bf16x8 af[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+          af[p] = __builtin_bit_cast(bf16x8, make_uint4(a[p][0], a[p][1], a[p][2], a[p][3]));
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+          const bf16_t* const b = wl + (nt * 32 + m) * stride + kl;
+          bf16x8 bf[3];
+#pragma unroll
+          for (int p = 0; p < 3; ++p) bf[p] = *reinterpret_cast<const bf16x8*>(b + (size_t)p * EP * stride);
+          constexpr int ta[6] = {2, 0, 1, 1, 0, 0}, tb[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+          for (int p = 0; p < 6; ++p)
+            acc[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[ta[p]], bf[tb[p]], acc[nt], 0, 0, 0);
         }
       }
-    } else {
+    };
+    for (int c = 0; c < num_chunks; ++c) {
+      const int k0 = c * KC;
+      load_rows(0, k0, kb_lo);
+      load_rows(1, k0, kb_lo + FB);
+      __syncthreads();                            // the chunk, or the logits, before have been read
+      constexpr int kBatch = NT == 1 ? 4 : NT == 2 ? 2 : 1;    // units in flight per thread
+      const int units = KC / 8 * E;
+      for (int u0 = tid; u0 < units; u0 += kBatch * kThreads) {
+        float raw[kBatch][8];
+        int at[kBatch], left[kBatch];
 #pragma unroll
-      for (int j = 0; j < CNT; ++j)
-        if (n0 + j < E) Elt<bf16_t>::store(grow + j, g[j]);
-    }
-  }
-  uint64_t taken = 0;
-  for (int kk = 0; kk < K; ++kk) {
-    uint64_t best = 0;
+        for (int t = 0; t < kBatch; ++t) {
+          const int u = min(u0 + t * kThreads, units - 1);   // (a thread past the end repeats the last unit)
+          const int kb = u / E, n = u - kb * E, k = k0 + kb * 8;
+          at[t] = n * stride + kb * 8;
+          left[t] = D - k;
 #pragma unroll
-    for (int j = 0; j < CNT; ++j) {
-      const int n = n0 + j;
-      if (n < E && !(taken >> j & 1ull)) {
-        uint64_t key = ((uint64_t)orderable(g[j]) << 32) | (uint32_t)(0xFFFFFFFFu - (uint32_t)n);
-        best = key > best ? key : best;
+          for (int i = 0; i < 8; ++i) raw[t][i] = w[(size_t)min(k + i, D - 1) * E + n];
+        }
+#pragma unroll
+        for (int t = 0; t < kBatch; ++t) {
+          uint32_t o[3][4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            split3_cut(2 * i < left[t] ? raw[t][2 * i] : 0.f, 2 * i + 1 < left[t] ? raw[t][2 * i + 1] : 0.f,
+                       o[0][i], o[1][i], o[2][i]);
+#pragma unroll
+          for (int p = 0; p < 3; ++p)
+            *reinterpret_cast<uint4*>(wl + (size_t)p * EP * stride + at[t]) = make_uint4(o[p][0], o[p][1], o[p][2], o[p][3]);
+        }
+      }
+      __syncthreads();
+      if (tile < num_tiles) {
+        for (int kb0 = kb_lo; kb0 < kb_hi; kb0 += 2 * FB) {
+          mma_rows(0, k0, kb0);
+          if (kb0 + 2 * FB < kb_hi) load_rows(0, k0, kb0 + 2 * FB);
+          mma_rows(1, k0, kb0 + FB);
+          if (kb0 + 3 * FB < kb_hi) load_rows(1, k0, kb0 + 3 * FB);
+          mfma_result_fence();
+        }
       }
     }
-    const uint32_t olo = __shfl_xor((uint32_t)best, 32, kWave);
-    const uint32_t ohi = __shfl_xor((uint32_t)(best >> 32), 32, kWave);
-    const uint64_t other = ((uint64_t)ohi << 32) | olo;
-    best = other > best ? other : best;
-    const int n_star = (int)(0xFFFFFFFFu - (uint32_t)best);
-    if (n_star >= n0 && n_star < n0 + CNT) taken |= 1ull << (n_star - n0);
-    if (h == 0 && row_ok) {
-      topk_val[(size_t)row * K + kk] = inv_orderable((uint32_t)(best >> 32));
-      topk_idx[(size_t)row * K + kk] = n_star;
+    __syncthreads();                              // W's LDS takes the logits
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) st[((i >> 2) * 8 + h * 4 + (i & 3)) * (EP + 1) + nt * 32 + m] = acc[nt][i];
+    __syncthreads();
+    if constexpr (KS > 1) {
+      for (int e = tid; e < TW * 32 * EP; e += kThreads) {
+        const int n = e & (EP - 1), r = (e / EP) & 31;
+        float* const at = reinterpret_cast<float*>(smem) + (size_t)(e / (32 * EP)) * KS * 32 * (EP + 1) + r * (EP + 1) + n;
+        float v = at[0];
+#pragma unroll
+        for (int p = 1; p < KS; ++p) v += at[p * 32 * (EP + 1)];
+        if (bias != nullptr) v += bias[min(n, E - 1)];
+        at[0] = v;
+      }
+      __syncthreads();
+    }
+    if (part == 0 && tile < num_tiles) {
+      constexpr int CNT = EP / 2;
+      float g[CNT];
+#pragma unroll
+      for (int j = 0; j < CNT; ++j) {
+        const int n = h * CNT + j;
+        g[j] = st[m * (EP + 1) + n];
+        if (KS == 1 && bias != nullptr) g[j] += bias[min(n, E - 1)];
+      }
+      if (logits != nullptr) {
+        if (KS == 1 && bias != nullptr) {
+#pragma unroll
+          for (int j = 0; j < CNT; ++j) st[m * (EP + 1) + h * CNT + j] = g[j];
+          wait_lgkmcnt0();
+        }
+        store_logits(st, EP + 1, logits, row0, num_items, E, lane);
+      }
+      finish_row<float, EP>(g, gates, topk_val, topk_idx, row0 + m, num_items, E, K, h);
     }
   }
 }
@@ -510,7 +622,10 @@ constexpr int kStreamChunkBytes = 32 * 128;      // 32 rows x 64 bfloat16
 
 typedef __attribute__((address_space(3))) void* gate_lds_ptr_t;
 
-template <int SLOTS, int WAVES>
+// ANY: any number of experts and any alignment of w, and gate_topk_kernel's dealing of k to the products
+// (a lane's half takes 32 consecutive k of a chunk), whose sums it repeats bit for bit (11 250 items x 704,
+// 4 experts: 22 us with direct loads, 11 here; 38 060 x 256, 12 experts: 18 to 10).
+template <int SLOTS, int WAVES, bool ANY>
 __global__ __launch_bounds__(WAVES * kWave, 1) void gate_topk_stream_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const float* __restrict__ bias,
     bf16_t* __restrict__ gates, float* __restrict__ topk_val, int32_t* __restrict__ topk_idx,
@@ -569,7 +684,9 @@ __global__ __launch_bounds__(WAVES * kWave, 1) void gate_topk_stream_kernel(
   // consecutive k as one 16-byte piece (E % 8 == 0 and a 16-byte aligned w: the launcher
   // checks); experts E .. 31 are zero.  The LDS writes are written as instructions, like the
   // fragment reads below: a write the compiler can see would wait for the requests above.
-  {
+  if constexpr (ANY) {
+    stage_router_any(w, wl, stride, 0, D, D, E, tid, kThreads);
+  } else {
     const int nbn = EP / 8, nblk = (D / 8) * nbn;
     for (int b0 = 0; b0 < nblk; b0 += kThreads) {
       const int b = b0 + tid;
@@ -616,12 +733,12 @@ __global__ __launch_bounds__(WAVES * kWave, 1) void gate_topk_stream_kernel(
     // other slots), which would leave a wave with one chunk in flight.
     auto multiply = [&](int c) {
       const uint32_t sa = ring_addr + (uint32_t)((c % SLOTS) * kStreamChunkBytes + m * 128);
-      const uint32_t sw = wl_addr + (uint32_t)((m * stride + c * 64 + h * 8) * 2);
+      const uint32_t sw = wl_addr + (uint32_t)((m * stride + c * 64 + h * (ANY ? 32 : 8)) * 2);
       u32x4_t a[4], b[4];
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
-        asm volatile("ds_read_b128 %0, %1" : "=v"(a[ks]) : "v"(sa + (uint32_t)(((2 * ks + h) ^ swz) * 16)));
-        asm volatile("ds_read_b128 %0, %1" : "=v"(b[ks]) : "v"(sw + (uint32_t)(ks * 32)));
+        asm volatile("ds_read_b128 %0, %1" : "=v"(a[ks]) : "v"(sa + (uint32_t)(((ANY ? h * 4 + ks : 2 * ks + h) ^ swz) * 16)));
+        asm volatile("ds_read_b128 %0, %1" : "=v"(b[ks]) : "v"(sw + (uint32_t)(ks * (ANY ? 16 : 32))));
       }
       asm volatile("s_waitcnt lgkmcnt(0)"
                    : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]));
@@ -745,6 +862,113 @@ __global__ __launch_bounds__(kSplitWaves * kWave, 1) void gate_topk_split_kernel
     finish_tile32(reinterpret_cast<const float*>(smem), gates, topk_val, topk_idx, row0, num_items, E, K, m, h);
 }
 
+// bfloat16, fewer tiles of items than CUs, up to 64 experts (any number), any width: a workgroup of eight waves
+// per tile of 32 items.  All of them fetch the item rows and the router kernel (KC columns of each) into LDS in
+// one trip to memory; a wave per 32 experts multiplies, in gate_topk_kernel's order of k (same sums bit for
+// bit), and wave 0 finishes the tile.  gate_topk_kernel walks k in one wave per tile on a quarter of the
+// workgroups, with a scalar staging loop where E is no multiple of 8: 870 items x 1 024, 6 experts: 29 us to 9.7;
+// 3 000 x 768, 50 experts: 44 to 15.
+constexpr int kTileWaves = 8;
+
+template <int NT>
+__global__ __launch_bounds__(kTileWaves * kWave) void gate_topk_tile_kernel(
+    const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const float* __restrict__ bias,
+    bf16_t* __restrict__ gates, float* __restrict__ logits, float* __restrict__ topk_val,
+    int32_t* __restrict__ topk_idx, int num_items, int D, int E, int K, int KC, int num_chunks, int x_off) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  constexpr int EP = NT * 32, kThreads = kTileWaves * kWave, kBatch = 8;
+  bf16_t* const wl = reinterpret_cast<bf16_t*>(smem);              // [EP][KC + 8]
+  bf16_t* const xs = reinterpret_cast<bf16_t*>(smem + x_off);      // [32][KC + 8], later the logits [32][EP + 1]
+  float* const st = reinterpret_cast<float*>(smem + x_off);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int m = lane & 31, h = lane >> 5, stride = KC + 8;
+  const int row0 = blockIdx.x * 32;
+  const bool blocks8 = E % 8 == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
+  floatx16 acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+  for (int c = 0; c < num_chunks; ++c) {
+    const int k0 = c * KC, per_row = KC / 8, pieces = 32 * per_row;
+    uint4 raw[kBatch];
+    auto load_x = [&](int p0) {
+#pragma unroll
+      for (int t = 0; t < kBatch; ++t) {
+        const int p = min(p0 + t * kThreads, pieces - 1), r = p / per_row, k = k0 + (p - r * per_row) * 8;
+        raw[t] = *reinterpret_cast<const uint4*>(x + (size_t)min(row0 + r, num_items - 1) * D + min(k, D - 8));
+        if (k >= D) raw[t] = make_uint4(0, 0, 0, 0);
+      }
+    };
+    auto store_x = [&](int p0) {
+#pragma unroll
+      for (int t = 0; t < kBatch; ++t) {
+        const int p = min(p0 + t * kThreads, pieces - 1), r = p / per_row;   // (past the end: the last piece again)
+        *reinterpret_cast<uint4*>(xs + r * stride + (p - r * per_row) * 8) = raw[t];
+      }
+    };
+    load_x(tid);
+    if (c > 0) __syncthreads();                   // the chunk before has been read
+    if (blocks8) {
+      const int nbn = E / 8, nblk = per_row * nbn;
+      for (int b = tid; b < nblk; b += kThreads) {
+        const int kb = b / nbn, nb = b - kb * nbn;
+        uint4 wraw[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int k = k0 + kb * 8 + i;
+          wraw[i] = k < D ? *reinterpret_cast<const uint4*>(w + (size_t)k * E + nb * 8) : make_uint4(0, 0, 0, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
+          uint32_t o[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            o[q] = __builtin_amdgcn_perm(reinterpret_cast<const uint32_t*>(&wraw[2 * q + 1])[j >> 1],
+                                         reinterpret_cast<const uint32_t*>(&wraw[2 * q])[j >> 1], sel);
+          *reinterpret_cast<uint4*>(wl + (nb * 8 + j) * stride + kb * 8) = make_uint4(o[0], o[1], o[2], o[3]);
+        }
+      }
+    } else {
+      stage_router_any(w, wl, stride, k0, KC, D, E, tid, kThreads);
+    }
+    store_x(tid);
+    for (int p0 = tid + kBatch * kThreads; p0 < pieces; p0 += kBatch * kThreads) {
+      load_x(p0);
+      store_x(p0);
+    }
+    __syncthreads();
+    if (wave < NT) {
+      const bf16_t* const a = xs + m * stride + h * 32;
+      const bf16_t* const b = wl + (wave * 32 + m) * stride + h * 32;
+      for (int kb = 0; kb < KC; kb += 64)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(a + kb + j * 8),
+                                                        *reinterpret_cast<const bf16x8*>(b + kb + j * 8), acc, 0, 0, 0);
+      mfma_result_fence();
+    }
+  }
+  __syncthreads();                                // the rows' LDS takes the logits
+  if (wave < NT) {
+    const int n = wave * 32 + m;
+    const float bn = (bias != nullptr && n < E) ? bias[n] : 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float v = bf16r(acc[i]);
+      if (bias != nullptr) v = bf16r(v + bn);
+      st[((i >> 2) * 8 + h * 4 + (i & 3)) * (EP + 1) + n] = v;
+    }
+  }
+  __syncthreads();
+  if (wave == 1 && logits != nullptr) store_logits(st, EP + 1, logits, row0, num_items, E, lane);
+  if (wave == 0) {
+    float g[EP / 2];
+#pragma unroll
+    for (int j = 0; j < EP / 2; ++j) g[j] = st[m * (EP + 1) + h * (EP / 2) + j];
+    finish_row<bf16_t, EP>(g, gates, topk_val, topk_idx, row0 + m, num_items, E, K, h);
+  }
+}
+
 // Top-K of given float32 gates, one wave per item, E <= 1024.
 __global__ __launch_bounds__(256) void topk_kernel(const float* __restrict__ gates,
                                                    float* __restrict__ topk_val,
@@ -799,23 +1023,62 @@ __global__ __launch_bounds__(kMetricThreads) void router_metrics_kernel(
                           top1_stride, V, blockIdx.x, smem);
 }
 
-template <typename T>
-int launch_gate(const VmoeGateTopkParams* p, hipStream_t stream) {
+int launch_gate_f32(const VmoeGateTopkParams* p, hipStream_t stream) {
+  const int nt = (p->E + 31) / 32 == 3 ? 4 : (p->E + 31) / 32, ep = nt * 32;
+  const int num_tiles = (p->num_items + 31) / 32;
+  // Tiles per workgroup: one workgroup per CU as long as that leaves a wave per tile.
+  const int per_cu = (num_tiles + kNumCus - 1) / kNumCus;
+  const int waves = nt == 4 ? 4 : 8, tw = nt == 4 ? 1 : per_cu <= 1 ? 1 : per_cu <= 2 ? 2 : per_cu <= 4 ? 4 : 8;
+  const int gran = 16 * waves, dpad = (p->D + gran - 1) / gran * gran;
+  const int most = (156 * 1024 / (ep * 6) - 8) / gran * gran;        // rows of W whose planes fit
+  const int num_chunks = (dpad + most - 1) / most;
+  const int kc = ((dpad + num_chunks - 1) / num_chunks + gran - 1) / gran * gran;
+  const size_t lds = std::max((size_t)ep * (kc + 8) * 6, (size_t)waves * 32 * (ep + 1) * sizeof(float));
+  const int blocks = std::min((num_tiles + tw - 1) / tw, 1024);
+  auto run = [&](auto kern) {
+    hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
+    if (e != hipSuccess) return (int)e;
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(waves * kWave), lds, stream, (const float*)p->x, (const float*)p->w,
+                       p->logit_bias, (float*)p->gates, p->logits, p->topk_val, p->topk_idx, p->num_items, p->D, p->E,
+                       p->K, kc, num_chunks, num_tiles);
+    return launch_status();
+  };
+  if (nt == 1) {
+    switch (tw) {
+      case 1: return run(gate_topk_f32_kernel<1, 8, 1>);
+      case 2: return run(gate_topk_f32_kernel<1, 8, 2>);
+      case 4: return run(gate_topk_f32_kernel<1, 8, 4>);
+      default: return run(gate_topk_f32_kernel<1, 8, 8>);
+    }
+  }
+  if (nt == 2) {
+    switch (tw) {
+      case 1: return run(gate_topk_f32_kernel<2, 8, 1>);
+      case 2: return run(gate_topk_f32_kernel<2, 8, 2>);
+      case 4: return run(gate_topk_f32_kernel<2, 8, 4>);
+      default: return run(gate_topk_f32_kernel<2, 8, 8>);
+    }
+  }
+  return run(gate_topk_f32_kernel<4, 4, 1>);
+}
+
+int launch_gate_bf16(const VmoeGateTopkParams* p, hipStream_t stream) {
+  using T = bf16_t;
   const int nt = (p->E + 31) / 32;
   const int ep = (nt == 3 ? 4 : nt) * 32;
-  const int gran = sizeof(T) == 2 ? 64 : 16;
+  constexpr int gran = 64;
   const int dpad = (p->D + gran - 1) / gran * gran;
   // LDS: the staged router kernel (split along D when it would not fit) and,
   // behind it, a 32 x (ep + 1) float32 logits tile per wave for the epilogue.
-  const size_t budget = 88 * 1024;
+  // (33 .. 64 experts: one workgroup fits a CU either way, and a whole router kernel is staged once)
+  const size_t budget = (nt == 2 ? 120 : 88) * 1024;
   int kc = dpad;
-  while ((size_t)(sizeof(T) == 2 ? ep * (kc + 8) : kc * ep) * sizeof(T) > budget && kc > gran)
-    kc = ((kc / 2) + gran - 1) / gran * gran;
+  while ((size_t)ep * (kc + 8) * sizeof(T) > budget && kc > gran) kc = ((kc / 2) + gran - 1) / gran * gran;
   const int num_chunks = (dpad + kc - 1) / kc;
-  const size_t w_bytes = ((size_t)(sizeof(T) == 2 ? ep * (kc + 8) : kc * ep) * sizeof(T) + 15) / 16 * 16;
+  const size_t w_bytes = ((size_t)ep * (kc + 8) * sizeof(T) + 15) / 16 * 16;
   // Two workgroups of four waves per CU, each with its own staged copy of the router
   // kernel, where both copies fit in LDS; one workgroup of eight waves sharing a copy
-  // where they do not (D = 1024 in bf16), the registers allow it (up to 32 experts) and
+  // where they do not (D = 1024), the registers allow it (up to 32 experts) and
   // four-wave workgroups would not all be resident at once anyway.
   const size_t tile_bytes = (size_t)32 * (ep + 1) * sizeof(float);
   const size_t lds_cu = 160 * 1024;
@@ -828,12 +1091,14 @@ int launch_gate(const VmoeGateTopkParams* p, hipStream_t stream) {
   if (blocks > 1024) blocks = 1024;
   // bfloat16, up to 32 experts, no logits output, enough items to fill the chip: the
   // streaming kernel (coalesced DMA requests into wave-private LDS rings).
-  if constexpr (sizeof(T) == 2) {
+  {
     const size_t stream_w = ((size_t)32 * (p->D + 8) * 2 + 1023) / 1024 * 1024;
     const size_t ring3 = (size_t)kStreamWaves * 3 * kStreamChunkBytes, ring2 = (size_t)kStreamWaves * 2 * kStreamChunkBytes;
-    const bool simple = nt == 1 && p->logits == nullptr && p->E % 8 == 0 && aligned16(p->w) &&
-                        p->D % 64 == 0 && getenv("VMOE_GATE_DIRECT_LOADS") == nullptr;
-    const bool stream_ok = simple && (int64_t)p->num_items * p->D * 2 < ((int64_t)1 << 32) &&
+    const bool direct = getenv("VMOE_GATE_DIRECT_LOADS") != nullptr;
+    const bool whole = p->E % 8 == 0 && aligned16(p->w);      // the router kernel comes in blocks of 8 x 8
+    const bool simple = nt == 1 && p->logits == nullptr && whole && p->D % 64 == 0 && !direct;
+    const bool stream_ok = nt == 1 && p->logits == nullptr && p->D % 64 == 0 && !direct &&
+                           (int64_t)p->num_items * p->D * 2 < ((int64_t)1 << 32) &&
                            num_tiles >= 256 && stream_w + ring2 <= lds_cu;
     // Fewer tiles than CUs: the waves of a tile share its k range (255 tiles x 768: 8.0 us against 13.8
     // with direct loads).  Beyond, a CU runs two such workgroups, each with its own copy of the router
@@ -847,6 +1112,21 @@ int launch_gate(const VmoeGateTopkParams* p, hipStream_t stream) {
                          (const bf16_t*)p->x, (const bf16_t*)p->w, p->logit_bias, (bf16_t*)p->gates,
                          p->topk_val, p->topk_idx, p->num_items, p->D, p->E, p->K);
       return launch_status();
+    }
+    if (nt <= 2 && num_tiles < 256 && !direct) {
+      const int most = (int)((150 * 1024) / ((ep + 32) * sizeof(T)) - 8) / 64 * 64;
+      const int chunks = (dpad + most - 1) / most, tkc = ((dpad + chunks - 1) / chunks + 63) / 64 * 64;
+      const size_t x_off = (size_t)ep * (tkc + 8) * sizeof(T);
+      const size_t tile_lds = x_off + std::max((size_t)32 * (tkc + 8) * sizeof(T), tile_bytes);
+      auto trun = [&](auto kern) {
+        hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), tile_lds);
+        if (e != hipSuccess) return (int)e;
+        hipLaunchKernelGGL(kern, dim3(num_tiles), dim3(kTileWaves * kWave), tile_lds, stream, (const T*)p->x,
+                           (const T*)p->w, p->logit_bias, (T*)p->gates, p->logits, p->topk_val, p->topk_idx,
+                           p->num_items, p->D, p->E, p->K, tkc, chunks, (int)x_off);
+        return launch_status();
+      };
+      return nt == 1 ? trun(gate_topk_tile_kernel<1>) : trun(gate_topk_tile_kernel<2>);
     }
     if (stream_ok) {
       const bool three = stream_w + ring3 <= lds_cu;
@@ -863,14 +1143,10 @@ int launch_gate(const VmoeGateTopkParams* p, hipStream_t stream) {
                            (int)stream_w);
         return launch_status();
       };
-      return three ? srun(gate_topk_stream_kernel<3, 8>) : srun(gate_topk_stream_kernel<2, 8>);
+      if (!whole) return three ? srun(gate_topk_stream_kernel<3, 8, true>) : srun(gate_topk_stream_kernel<2, 8, true>);
+      return three ? srun(gate_topk_stream_kernel<3, 8, false>) : srun(gate_topk_stream_kernel<2, 8, false>);
     }
   }
-  // float32, up to 32 experts, at most two tiles of items per CU: a tile per workgroup, its k
-  // range dealt to the four waves.
-  const bool split_k = sizeof(T) == 4 && nt == 1 && waves == 4 && num_tiles <= 512 && kc % 64 == 0 &&
-                       getenv("VMOE_GATE_NO_SPLIT_K") == nullptr;
-  if (split_k) blocks = num_tiles;
   auto run = [&](auto kern) {
     hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
     if (e != hipSuccess) return (int)e;
@@ -882,22 +1158,17 @@ int launch_gate(const VmoeGateTopkParams* p, hipStream_t stream) {
   };
   // The logits output is a separate instantiation: its extra live pointer costs
   // the common one a wave of occupancy.
-  if constexpr (sizeof(T) == 4) {
-    if (split_k)
-      return p->logits != nullptr ? run(gate_topk_kernel<T, 1, true, 4, true>)
-                                  : run(gate_topk_kernel<T, 1, false, 4, true>);
-  }
   if (p->logits != nullptr) {
     switch (nt) {
-      case 1: return waves == 8 ? run(gate_topk_kernel<T, 1, true, 8>) : run(gate_topk_kernel<T, 1, true, 4>);
-      case 2: return run(gate_topk_kernel<T, 2, true, 4>);
-      default: return run(gate_topk_kernel<T, 4, true, 4>);
+      case 1: return waves == 8 ? run(gate_topk_kernel<1, true, 8>) : run(gate_topk_kernel<1, true, 4>);
+      case 2: return run(gate_topk_kernel<2, true, 4>);
+      default: return run(gate_topk_kernel<4, true, 4>);
     }
   }
   switch (nt) {
-    case 1: return waves == 8 ? run(gate_topk_kernel<T, 1, false, 8>) : run(gate_topk_kernel<T, 1, false, 4>);
-    case 2: return run(gate_topk_kernel<T, 2, false, 4>);
-    default: return run(gate_topk_kernel<T, 4, false, 4>);
+    case 1: return waves == 8 ? run(gate_topk_kernel<1, false, 8>) : run(gate_topk_kernel<1, false, 4>);
+    case 2: return run(gate_topk_kernel<2, false, 4>);
+    default: return run(gate_topk_kernel<4, false, 4>);
   }
 }
 
@@ -1001,8 +1272,8 @@ extern "C" int vmoe_gate_topk(const VmoeGateTopkParams* p, vmoe_stream_t stream)
   if (p->D % vec != 0 || !aligned16(p->x)) return VMOE_E_ALIGN;
   if ((int64_t)p->num_items * (p->D > p->E * p->K ? p->D : p->E * p->K) >= (int64_t)1 << 40)
     return VMOE_E_OVERFLOW;
-  return p->dtype == VMOE_BF16 ? launch_gate<bf16_t>(p, as_stream(stream))
-                               : launch_gate<float>(p, as_stream(stream));
+  return p->dtype == VMOE_BF16 ? launch_gate_bf16(p, as_stream(stream))
+                               : launch_gate_f32(p, as_stream(stream));
 }
 
 extern "C" int vmoe_topk(const VmoeTopkParams* p, vmoe_stream_t stream) {
