@@ -41,6 +41,8 @@ enum { VMOE_F32 = 0, VMOE_BF16 = 1 };
 enum { VMOE_GELU_TANH = 0, VMOE_GELU_ERF = 1 };
 /* Added to VMOE_GELU_* of a float32 expert MLP: its products run on float32 matrix instructions. */
 enum { VMOE_MLP_F32_PRODUCTS = 256 };
+/* Added to VMOE_GELU_* of a bfloat16 expert MLP: b0 and b1 are float32 and rounded to bfloat16 in the call. */
+enum { VMOE_MLP_F32_BIASES = 512 };
 
 enum {
   VMOE_OK = 0,
@@ -334,9 +336,9 @@ int vmoe_densify(const VmoeDensifyParams* p, vmoe_stream_t stream);
 typedef struct {
   const void* x;    /* (E, R, D) dtype */
   const void* w0;   /* (E, D, M) dtype: Mlp/Dense_0/kernel (may be null when w0t is given) */
-  const void* b0;   /* (E, M) dtype or null */
+  const void* b0;   /* (E, M) dtype (VMOE_MLP_F32_BIASES: float32) or null */
   const void* w1;   /* (E, M, D) dtype: Mlp/Dense_1/kernel (may be null when w1t is given) */
-  const void* b1;   /* (E, D) dtype or null */
+  const void* b1;   /* (E, D) like b0 or null */
   const void* w0t;  /* optional (E, M, D) dtype: w0 transposed per expert */
   const void* w1t;  /* optional (E, D, M) dtype: w1 transposed per expert */
   void* out;        /* (E, R, D) dtype */
@@ -345,7 +347,9 @@ typedef struct {
   int32_t E, R, D, M;
   int32_t dtype;
   int32_t gelu;     /* VMOE_GELU_TANH (flax default) or VMOE_GELU_ERF, for float32 also
-                       + VMOE_MLP_F32_PRODUCTS */
+                       + VMOE_MLP_F32_PRODUCTS, for bf16 + VMOE_MLP_F32_BIASES: the rounded
+                       biases then lie at the end of the workspace, written by this call or by
+                       vmoe_compact_rows_planned (vmoe_expert_mlp_planned reads them there) */
   const int32_t* rows_per_expert; /* optional (E,): only the first rows_per_expert[e] rows of
                                      expert e hold data; the other rows of x are not read
                                      for results and their rows of out are left untouched */
@@ -364,8 +368,8 @@ int vmoe_expert_mlp(const VmoeExpertMlpParams* p, vmoe_stream_t stream);
 /* vmoe_compact_rows and the planning launch of vmoe_expert_mlp in one launch (no counterpart
  * in the reference: the packed rows have none).  `mlp` is the parameter block of the MLP call
  * that follows, with its workspace and with rows_per_expert = c->rows_per_expert, x_rows =
- * c->row_token where the first product gathers its rows (only the sizes, dtype, the workspace
- * and which row tensors are given are looked at here); that call is then made as
+ * c->row_token where the first product gathers its rows (only the sizes, dtype, the workspace,
+ * which row tensors are given and float32 biases are looked at here); that call is then made as
  * vmoe_expert_mlp_planned, which takes the launch plans in the workspace as written.
  * VMOE_E_UNSUPPORTED where the compaction needs its two-launch form (E > 256, fewer than 256
  * assignments per group, many groups of few experts) or the MLP plans nothing (float32):

@@ -1731,6 +1731,46 @@ def _planned_repeats_and_checks_its_plan(K, G, S, E, k, C, D, M):
   assert (to_np(out) == 7.0).all(), "a launch without a valid plan must not write"
 
 
+@pytest.mark.parametrize("G,S,E,k,C,D,M", [(1, 49, 3, 2, 40, 64, 104), (2, 784, 8, 2, 208, 256, 512),
+                                           (16, 1568, 8, 2, 400, 768, 1024)])
+def test_expert_mlp_float32_biases(K, G, S, E, k, C, D, M):
+  """Float32 biases of a bfloat16 MLP, rounded inside the call (beside the row compaction where there is
+  one): the bits of biases rounded beforehand, for both, one of them, one in bfloat16, a strided one,
+  and after an edit that raises no version."""
+  rng = np.random.default_rng(E + D)
+  mk = lambda scale, *s: to_dev((rng.standard_normal(s) * scale).astype(np.float32))
+  bf = lambda t: t if t is None else t.to(torch.bfloat16)
+  x, xe = bf(mk(1, G * S, D)), bf(mk(1, E, G * C, D))
+  kw = dict(w0t=bf(mk(D ** -0.5, E, M, D)), w1t=bf(mk(M ** -0.5, E, D, M)))
+  val, idx = K.topk(to_dev(O.softmax(rng.standard_normal((G, S, E)).astype(np.float32))), k)
+  _, token_slot, _, fill = K.route_assign(val, idx, E, C, True)
+  rows = to_dev(rng.integers(0, G * C + 1, E).astype(np.int32))
+  b0, b1 = mk(0.3, E, M), mk(0.3, E, D)
+  strided = mk(0.3, D, E).t()
+
+  def both(p0, p1):
+    r0, r1 = bf(p0), bf(p1 if p1 is None else p1.contiguous())
+    for more in (dict(), dict(rows_per_expert=rows)):
+      got, want = (K.expert_mlp(xe, None, a, None, c, out=torch.zeros_like(xe), **kw, **more) for a, c in ((p0, p1), (r0, r1)))
+      assert torch.equal(got, want)
+    got, maps = K.expert_mlp(x, None, p0, None, p1, compact=(fill, token_slot, C), **kw)
+    want, _ = K.expert_mlp(x, None, r0, None, r1, compact=(fill, token_slot, C), **kw)
+    for e, n in enumerate(to_np(maps[1])):
+      assert torch.equal(got[e, :n], want[e, :n])
+    return got, maps
+
+  for p0, p1 in ((b0, b1), (None, b1), (b0, None), (bf(b0), b1), (b0, strided)):
+    both(p0, p1)
+  b0.data.add_(1)
+  both(b0, b1)
+  got, maps = K.expert_mlp(x, None, b0, None, b1, compact=(fill, token_slot, C), **kw)
+  want = got.clone()
+  got.zero_()
+  assert K.expert_mlp_replay_planned() is got
+  for e, n in enumerate(to_np(maps[1])):
+    assert torch.equal(got[e, :n], want[e, :n])
+
+
 @pytest.mark.parametrize("G,S,E,k,C,D,M", [(1, 196, 8, 2, 52, 768, 3072), (2, 300, 5, 3, 200, 128, 192)])
 def test_expert_mlp_planned_over_few_rows(K, G, S, E, k, C, D, M):
   """Products on the small tiles need no plan: vmoe_compact_rows_planned takes such a call all the

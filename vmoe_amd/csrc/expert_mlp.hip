@@ -282,21 +282,47 @@ __global__ __launch_bounds__(256, 1) void operand_delivery_probe_kernel(
 #endif
 }
 
-// Row compaction and the launch plans of the expert MLP's ragged products in one launch:
-// workgroups 0 .. compact_blocks - 1 renumber the assignments (compact_rows_fused_block),
-// the others plan (plan_ragged_tiles_block, row counts from the fill counts).  Neither part
-// reads what the other writes.
+// Float32 biases of a bfloat16 MLP (VMOE_MLP_F32_BIASES) to bfloat16: four values a thread of b0 and,
+// behind them, b1.
+struct BiasCast {
+  const float *b0, *b1;          // (n0), (n1), or null: nothing to do
+  bf16_t *o0, *o1;
+  size_t n0, n1;
+  unsigned blocks() const { return o0 == nullptr ? 0u : (unsigned)((n0 + n1 + 1023) / 1024); }
+};
+
+__device__ __forceinline__ void cast_biases_block(const BiasCast& c, unsigned block) {
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const size_t i = (size_t)block * 1024 + t * 256 + threadIdx.x;
+    if (i < c.n0) {
+      if (c.b0 != nullptr) c.o0[i] = f2bf(c.b0[i]);
+    } else if (i < c.n0 + c.n1) {
+      if (c.b1 != nullptr) c.o1[i - c.n0] = f2bf(c.b1[i - c.n0]);
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void cast_biases_kernel(BiasCast c) { cast_biases_block(c, blockIdx.x); }
+
+// Row compaction, the launch plans of the expert MLP's ragged products and the casts of its float32
+// biases in one launch: workgroups 0 .. compact_blocks - 1 renumber the assignments
+// (compact_rows_fused_block), the next plan_blocks plan (plan_ragged_tiles_block, row counts from the
+// fill counts), the others cast.  No part reads what another writes.  (A launch of their own for each of
+// the two casts cost 2.3 us and about 10 us of host time: the B/16 model over eight images makes 24.)
 __global__ __launch_bounds__(256) void compact_rows_planned_kernel(
     const int32_t* __restrict__ fill, const int32_t* __restrict__ token_slot,
     int32_t* __restrict__ token_row, int32_t* __restrict__ row_token,
     int32_t* __restrict__ rows_per_expert, int G, int E, int C, int per_group, int K, size_t n,
-    unsigned compact_blocks, int R, RaggedGeom ga, RaggedGeom gb) {
+    unsigned compact_blocks, unsigned plan_blocks, int R, RaggedGeom ga, RaggedGeom gb, BiasCast biases) {
   extern __shared__ int32_t tile_prefix[];
   if (blockIdx.x < compact_blocks)
     compact_rows_fused_block(fill, token_slot, token_row, row_token, rows_per_expert, G, E, C,
                              per_group, K, n, blockIdx.x);
-  else
+  else if (blockIdx.x < compact_blocks + plan_blocks)
     plan_ragged_tiles_block(nullptr, fill, G, E, R, ga, gb, blockIdx.x - compact_blocks, tile_prefix);
+  else
+    cast_biases_block(biases, blockIdx.x - compact_blocks - plan_blocks);
 }
 
 size_t align256(size_t v) { return (v + 255) / 256 * 256; }
@@ -443,7 +469,14 @@ MlpPlans mlp_plans(int E, int R, int D, int M, bool ragged, long long items) {
 
 using namespace vmoe;
 
-static int gelu_of(const VmoeExpertMlpParams* p) { return p->gelu & ~VMOE_MLP_F32_PRODUCTS; }
+static int gelu_of(const VmoeExpertMlpParams* p) {
+  return p->gelu & ~(VMOE_MLP_F32_PRODUCTS | VMOE_MLP_F32_BIASES);
+}
+static bool has_f32_biases(const VmoeExpertMlpParams* p) { return (p->gelu & VMOE_MLP_F32_BIASES) != 0; }
+// The rounded biases' part of the workspace, its last.
+static size_t bias_bytes(const VmoeExpertMlpParams* p) {
+  return has_f32_biases(p) ? align256((size_t)p->E * p->M * 2) + align256((size_t)p->E * p->D * 2) : 0;
+}
 
 static int check_mlp(const VmoeExpertMlpParams* p) {
   if (p == nullptr || p->x == nullptr || p->out == nullptr) return VMOE_E_NULL;
@@ -458,6 +491,7 @@ static int check_mlp(const VmoeExpertMlpParams* p) {
       return VMOE_E_UNSUPPORTED;
   }
   if ((p->gelu & VMOE_MLP_F32_PRODUCTS) != 0 && p->dtype != VMOE_F32) return VMOE_E_DTYPE;
+  if (has_f32_biases(p) && p->dtype != VMOE_BF16) return VMOE_E_DTYPE;
   if (gelu_of(p) != VMOE_GELU_TANH && gelu_of(p) != VMOE_GELU_ERF) return VMOE_E_DTYPE;
   if (p->dtype == VMOE_BF16) {
     if ((p->w0 == nullptr && p->w0t == nullptr) || (p->w1 == nullptr && p->w1t == nullptr))
@@ -488,7 +522,7 @@ extern "C" size_t vmoe_expert_mlp_workspace_bytes(const VmoeExpertMlpParams* p) 
     if (p->w0t == nullptr) bytes += align256((size_t)p->E * p->D * p->M * b);
     if (p->w1t == nullptr) bytes += align256((size_t)p->E * p->D * p->M * b);
   }
-  return bytes;
+  return bytes + bias_bytes(p);
 }
 
 // Where the pieces of a bfloat16 MLP's workspace lie, and what the planning launch is given.
@@ -499,6 +533,9 @@ struct MlpWorkspace {
   int4* plan_down = nullptr;
   void* streamk = nullptr;
   unsigned char* rest = nullptr;     // transposed weights, where the caller did not pack them
+  const bf16_t* b0 = nullptr;        // the biases in bfloat16: the caller's or, cast, the workspace's
+  const bf16_t* b1 = nullptr;
+  BiasCast biases{};                 // what has to be cast for that (o0 null: nothing)
   MlpPlans m;
   RaggedGeom ga{}, gb{};
   int plan_blocks = 0;               // workgroups of the planning launch (0: nothing to plan)
@@ -533,6 +570,18 @@ MlpWorkspace mlp_workspace(const VmoeExpertMlpParams* p) {
     }
   }
   w.rest = ws;
+  if (has_f32_biases(p)) {
+    unsigned char* const at = static_cast<unsigned char*>(p->workspace) + vmoe_expert_mlp_workspace_bytes(p) - bias_bytes(p);
+    w.biases = BiasCast{(const float*)p->b0, (const float*)p->b1, reinterpret_cast<bf16_t*>(at),
+                        reinterpret_cast<bf16_t*>(at + align256((size_t)p->E * p->M * 2)),
+                        (size_t)p->E * p->M, (size_t)p->E * p->D};
+    w.b0 = p->b0 != nullptr ? w.biases.o0 : nullptr;
+    w.b1 = p->b1 != nullptr ? w.biases.o1 : nullptr;
+    if (p->b0 == nullptr && p->b1 == nullptr) w.biases = BiasCast{};
+  } else if (p->dtype == VMOE_BF16) {
+    w.b0 = (const bf16_t*)p->b0;
+    w.b1 = (const bf16_t*)p->b1;
+  }
   return w;
 }
 
@@ -558,6 +607,8 @@ static int run_expert_mlp(const VmoeExpertMlpParams* p, vmoe_stream_t stream_, b
   if (w.plan_blocks > 0 && !planned_already)
     hipLaunchKernelGGL(plan_ragged_tiles_kernel, dim3(w.plan_blocks), dim3(256),
                        plan_ragged_tiles_lds(p->E), stream, p->rows_per_expert, p->E, p->R, w.ga, w.gb);
+  if (w.biases.blocks() > 0 && !planned_already)
+    hipLaunchKernelGGL(cast_biases_kernel, dim3(w.biases.blocks()), dim3(256), 0, stream, w.biases);
   const bool tanh_gelu = gelu_of(p) == VMOE_GELU_TANH;
   const bool f32_products = (p->gelu & VMOE_MLP_F32_PRODUCTS) != 0;
   if (p->dtype == VMOE_BF16) {
@@ -586,50 +637,50 @@ static int run_expert_mlp(const VmoeExpertMlpParams* p, vmoe_stream_t stream_, b
     const PlanRef no_plan{nullptr, 0, 0};
     if (m.up_rows >= 0) {
       auto up = tanh_gelu ? launch_gemm_bf16_rows<kEpiBiasGeluTanh> : launch_gemm_bf16_rows<kEpiBiasGeluErf>;
-      rc = up(m.up_rows, (const bf16_t*)p->x, (const bf16_t*)w0t, (const bf16_t*)p->b0, (bf16_t*)hidden,
+      rc = up(m.up_rows, (const bf16_t*)p->x, (const bf16_t*)w0t, w.b0, (bf16_t*)hidden,
               p->E, p->R, p->M, p->D, stream, p->rows_per_expert, p->x_rows, p->num_items,
               plan_down != nullptr ? plan_ref_of(m.down, plan_down, m.down_bm, p->E, p->R) : no_plan,
               clear, SK::kFlags, status);
     } else if (tanh_gelu)
       rc = launch_gemm_bf16_first<kEpiBiasGeluTanh>((const bf16_t*)p->x, (const bf16_t*)w0t,
-                                                    (const bf16_t*)p->b0, (bf16_t*)hidden, p->E,
+                                                    w.b0, (bf16_t*)hidden, p->E,
                                                     p->R, p->M, p->D, stream, p->rows_per_expert,
                                                     plan_up, p->x_rows, p->num_items, clear, SK::kFlags, status);
     else
       rc = launch_gemm_bf16_first<kEpiBiasGeluErf>((const bf16_t*)p->x, (const bf16_t*)w0t,
-                                                   (const bf16_t*)p->b0, (bf16_t*)hidden, p->E,
+                                                   w.b0, (bf16_t*)hidden, p->E,
                                                    p->R, p->M, p->D, stream, p->rows_per_expert,
                                                    plan_up, p->x_rows, p->num_items, clear, SK::kFlags, status);
     if (rc != VMOE_OK) return rc;
     if (m.down_rows >= 0)
       return launch_gemm_bf16_rows<kEpiBias>(
-          m.down_rows, (const bf16_t*)hidden, (const bf16_t*)w1t, (const bf16_t*)p->b1, (bf16_t*)p->out,
+          m.down_rows, (const bf16_t*)hidden, (const bf16_t*)w1t, w.b1, (bf16_t*)p->out,
           p->E, p->R, p->D, p->M, stream, p->rows_per_expert, nullptr, 0,
           plan_up != nullptr ? plan_ref_of(m.up, plan_up, CfgUp::BM, p->E, p->R) : no_plan, nullptr, 0, status);
     switch (m.down_kernel) {
       case kDownShared:
         return launch_gemm_bf16_persistent<CfgDownPersistent, kEpiBias>(
-            (const bf16_t*)hidden, (const bf16_t*)w1t, (const bf16_t*)p->b1, (bf16_t*)p->out, p->E,
+            (const bf16_t*)hidden, (const bf16_t*)w1t, w.b1, (bf16_t*)p->out, p->E,
             p->R, p->D, p->M, stream, plan_down, streamk, status);
       case kDownEightWaves:
         return launch_gemm_bf16_w8<kEpiBias, 8>((const bf16_t*)hidden, (const bf16_t*)w1t,
-                                                (const bf16_t*)p->b1, (bf16_t*)p->out, p->E, p->R,
+                                                w.b1, (bf16_t*)p->out, p->E, p->R,
                                                 p->D, p->M, stream, plan_down, nullptr, 0, status);
       case kDownNarrow:
         return launch_gemm_bf16_w8<kEpiBias, 6>((const bf16_t*)hidden, (const bf16_t*)w1t,
-                                                 (const bf16_t*)p->b1, (bf16_t*)p->out, p->E, p->R,
+                                                 w.b1, (bf16_t*)p->out, p->E, p->R,
                                                  p->D, p->M, stream, plan_down, nullptr, 0, status);
       case kDownWide:
         return launch_gemm_bf16_wide<kEpiBias>((const bf16_t*)hidden, (const bf16_t*)w1t,
-                                               (const bf16_t*)p->b1, (bf16_t*)p->out, p->E, p->R,
+                                               w.b1, (bf16_t*)p->out, p->E, p->R,
                                                p->D, p->M, stream, plan_down, nullptr, 0, status);
       case kDownHalf:
         return launch_gemm_bf16<CfgUp, kEpiBias>((const bf16_t*)hidden, (const bf16_t*)w1t,
-                                                (const bf16_t*)p->b1, (bf16_t*)p->out, p->E, p->R,
+                                                w.b1, (bf16_t*)p->out, p->E, p->R,
                                                 p->D, p->M, stream, nullptr, nullptr);
       default:
         return launch_gemm_bf16<CfgDown, kEpiBias>((const bf16_t*)hidden, (const bf16_t*)w1t,
-                                                  (const bf16_t*)p->b1, (bf16_t*)p->out, p->E, p->R,
+                                                  w.b1, (bf16_t*)p->out, p->E, p->R,
                                                   p->D, p->M, stream, p->rows_per_expert, plan_down,
                                                   nullptr, 0, nullptr, 0, status);
     }
@@ -693,10 +744,11 @@ extern "C" int vmoe_compact_rows_planned(const VmoeCompactRowsParams* c,
   if (!w.m.planned) return VMOE_E_UNSUPPORTED;
   const size_t n = (size_t)c->G * c->S * c->K;
   const unsigned compact_blocks = (unsigned)((n + 255) / 256);
-  hipLaunchKernelGGL(compact_rows_planned_kernel, dim3(compact_blocks + (unsigned)w.plan_blocks),
+  hipLaunchKernelGGL(compact_rows_planned_kernel,
+                     dim3(compact_blocks + (unsigned)w.plan_blocks + w.biases.blocks()),
                      dim3(256), plan_ragged_tiles_lds(c->E), as_stream(stream), c->fill,
                      c->token_slot, c->token_row, c->row_token, c->rows_per_expert, c->G, c->E, c->C,
-                     c->S * c->K, c->K, n, compact_blocks, mlp->R, w.ga, w.gb);
+                     c->S * c->K, c->K, n, compact_blocks, (unsigned)w.plan_blocks, mlp->R, w.ga, w.gb, w.biases);
   return launch_status();
 }
 

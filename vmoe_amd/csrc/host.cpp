@@ -191,12 +191,19 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> top_i
 // -> out, workspace, byte offset of the status words in it (-1: none), token_row,
 //    rows_per_expert, row_token, whether the call ran on a plan that the compaction wrote.
 std::tuple<Tensor, Tensor, int64_t, OptTensor, OptTensor, OptTensor, bool> expert_mlp(
-    int64_t stream, const Tensor& x_, const OptTensor& w0, const OptTensor& b0, const OptTensor& w1,
-    const OptTensor& b1, const OptTensor& w0t, const OptTensor& w1t, bool tanh_gelu,
+    int64_t stream, const Tensor& x_, const OptTensor& w0, const OptTensor& b0_, const OptTensor& w1,
+    const OptTensor& b1_, const OptTensor& w0t, const OptTensor& w1t, bool tanh_gelu,
     const OptTensor& workspace_, const OptTensor& out_, const OptTensor& rows_per_expert,
     const OptTensor& x_rows, const OptTensor& fill, const OptTensor& token_slot, int64_t capacity,
     bool plan_apart, bool f32_products) {
   const Tensor x = x_.contiguous();
+  // float32 biases of a bfloat16 MLP are rounded by the call (which asks for both in one type)
+  auto is_f32 = [&](const OptTensor& t) { return t.has_value() && t->scalar_type() == at::kFloat; };
+  const bool f32_biases = x.scalar_type() == at::kBFloat16 && (is_f32(b0_) || is_f32(b1_));
+  auto bias = [&](const OptTensor& t) -> OptTensor {
+    return f32_biases && t.has_value() ? OptTensor(as_f32(*t)) : t;
+  };
+  const OptTensor b0 = bias(b0_), b1 = bias(b1_);
   const bool compact = fill.has_value();
   VmoeCompactRowsParams c{};
   OptTensor token_row, rows = rows_per_expert, row_token = x_rows;
@@ -239,7 +246,8 @@ std::tuple<Tensor, Tensor, int64_t, OptTensor, OptTensor, OptTensor, bool> exper
   p.M = (int32_t)M;
   Tensor out = out_.has_value() ? *out_ : empty({E, R, D}, x.scalar_type(), x);
   p.x = ptr(x); p.w0 = ptr(w0); p.b0 = ptr(b0); p.w1 = ptr(w1); p.b1 = ptr(b1); p.w0t = ptr(w0t); p.w1t = ptr(w1t);
-  p.out = ptr(out); p.dtype = dtype_code(x); p.gelu = (tanh_gelu ? VMOE_GELU_TANH : VMOE_GELU_ERF) + (f32_products ? VMOE_MLP_F32_PRODUCTS : 0);
+  p.out = ptr(out); p.dtype = dtype_code(x); p.gelu = (tanh_gelu ? VMOE_GELU_TANH : VMOE_GELU_ERF) + (f32_products ? VMOE_MLP_F32_PRODUCTS : 0) +
+           (f32_biases ? VMOE_MLP_F32_BIASES : 0);
   p.rows_per_expert = ptr_as<int32_t>(rows); p.x_rows = ptr_as<int32_t>(row_token);
   const size_t need = vmoe_expert_mlp_workspace_bytes(&p);
   Tensor workspace = workspace_.has_value() && workspace_->nbytes() >= need

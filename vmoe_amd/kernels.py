@@ -320,7 +320,8 @@ def expert_mlp(x: torch.Tensor, w0, b0, w1, b1, w0t=None, w1t=None, approximate_
   compact_rows gives is returned as well): -> (out, (token_row, rows_per_expert, row_token)).
 
   ``float32_products``: float32 operands are multiplied on float32 matrix instructions instead of
-  as sums of three bfloat16 values each (for outputs that are rounded to bfloat16 further on)."""
+  as sums of three bfloat16 values each (for outputs that are rounded to bfloat16 further on).
+  The biases of a bfloat16 MLP may be float32: the call rounds them."""
   float32_products = float32_products and x.dtype == torch.float32
   if H._timing_sink is None or not any(map(H.timed, _MLP_CALLS)):
     global _last_planned
@@ -352,6 +353,8 @@ def expert_mlp(x: torch.Tensor, w0, b0, w1, b1, w0t=None, w1t=None, approximate_
   x = x.contiguous()
   if out is None:
     out = torch.empty((E, R, D), dtype=x.dtype, device=x.device)
+  if x.dtype == torch.bfloat16:
+    b0, b1 = (None if b is None else cast(b, x.dtype) for b in (b0, b1))
   p = _expert_mlp_params(x, w0, b0, w1, b1, w0t, w1t, approximate_gelu, out, rows_per_expert, x_rows)
   p.gelu += H.MLP_F32_PRODUCTS * float32_products
   need = H.lib().vmoe_expert_mlp_workspace_bytes(H.ctypes.byref(p))
@@ -408,6 +411,9 @@ def expert_mlp_replay_planned() -> torch.Tensor:
   if _last_planned is None:
     raise RuntimeError("no planned expert_mlp call to repeat")
   *call, workspace, rows, row_token = _last_planned
+  x, _, b0, _, b1 = call[:5]
+  # (rounded again: a repeated call sees what the parameters hold now)
+  call[2], call[4] = (b if b is None or b.dtype == x.dtype else cast(b, x.dtype) for b in (b0, b1))
   p = _expert_mlp_params(*call, rows, row_token)
   p.workspace = H.ptr(workspace)
   p.workspace_bytes = workspace.numel() * workspace.element_size()

@@ -659,11 +659,12 @@ def sparse_moe_spmd(target, variable_axes: Optional[Mapping[str, Any]] = None,
       return _tree_stack(per_expert)
 
     def apply(self, variables, dispatcher: BaseDispatcher, *inputs):
-      # Outputs that combine rounds to bfloat16: float32 sums in another order would round the other
-      # way in one value of 4 000 (3e-5 of a Soft MoE layer's output).
-      rounded = (isinstance(dispatcher, Bfloat16Dispatcher)
-                 and getattr(getattr(self.expert, "apply_experts", None), "takes_float32_products", False))
-      kwargs = {"float32_products": True} if rounded else {}
+      def rounded():
+        # Outputs that combine rounds to bfloat16: float32 sums in another order would round the other
+        # way in one value of 4 000 (3e-5 of a Soft MoE layer's output).
+        return ({"float32_products": True} if isinstance(dispatcher, Bfloat16Dispatcher)
+                and getattr(self.expert.apply_experts, "takes_float32_products", False) else {})
+
       supports = getattr(dispatcher, "supports_packed", None)
       if (not has_aux and len(inputs) == 1 and supports is not None and supports()
           and getattr(self.expert, "supports_packed_rows", False)
@@ -687,11 +688,11 @@ def sparse_moe_spmd(target, variable_axes: Optional[Mapping[str, Any]] = None,
         else:
           dispatched, rows_per_expert = dispatcher.dispatch_packed(x)
           outputs = self.expert.apply_experts(variables, dispatched,
-                                              rows_per_expert=rows_per_expert, **kwargs)
+                                              rows_per_expert=rows_per_expert, **rounded())
         return _tree_map(dispatcher.combine_packed, outputs)
       dispatched = [dispatcher.dispatch(x) for x in inputs]
       if hasattr(self.expert, "apply_experts"):
-        outputs = self.expert.apply_experts(variables, *dispatched, **kwargs)
+        outputs = self.expert.apply_experts(variables, *dispatched, **rounded())
       else:
         num_experts = dispatched[0].shape[0]
         outs = [self.expert.apply(_tree_index(variables, e), *[d[e] for d in dispatched])

@@ -52,8 +52,8 @@ class MlpBlock(module.Module):
   def _weights(self, p, dtype, stacked: bool = True):
     """Keyword arguments of kernels.expert_mlp that hold the parameters ``p`` in the compute
     dtype and the kernels' layout.  ``stacked``: the leaves have a leading expert axis (else
-    they are one MLP's).  Only the transposed copies are kept, one per kernel tensor: a bias is
-    cast on every call, which sees edits that raise no version counter (``b.data.add_``)."""
+    they are one MLP's).  Only the transposed copies are kept, one per kernel tensor: a float32 bias is
+    rounded in every call, which sees edits that raise no version counter (``b.data.add_``)."""
     w0, b0, w1, b1 = (p[layer].get(leaf) for layer in ("Dense_0", "Dense_1") for leaf in ("kernel", "bias"))
     module.require_no_grad("MlpBlock", w0, b0, w1, b1)
     cast = lambda t: None if t is None else K.cast(t if stacked else t[None], dtype)
@@ -61,7 +61,10 @@ class MlpBlock(module.Module):
       return dict(w0=cast(w0), b0=cast(b0), w1=cast(w1), b1=cast(b1))
     # the matrix-core kernels read the weights K-contiguous
     pack = lambda w, tag: self._packed.get((w,), (tag, stacked), lambda: K.pack_expert_weights(cast(w)))
-    return dict(w0=None, b0=cast(b0), w1=None, b1=cast(b1), w0t=pack(w0, "w0t"), w1t=pack(w1, "w1t"))
+    # (the call rounds float32 biases itself, beside its other preparations)
+    bias = lambda t: (cast(t) if t is None or not t.is_cuda or t.dtype != torch.float32
+                      else t if stacked else t[None])
+    return dict(w0=None, b0=bias(b0), w1=None, b1=bias(b1), w0t=pack(w0, "w0t"), w1t=pack(w1, "w1t"))
 
   supports_packed_rows = True
 
