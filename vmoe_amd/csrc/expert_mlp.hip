@@ -509,20 +509,25 @@ static int check_mlp(const VmoeExpertMlpParams* p) {
   return VMOE_OK;
 }
 
-extern "C" size_t vmoe_expert_mlp_workspace_bytes(const VmoeExpertMlpParams* p) {
-  if (p == nullptr || p->E < 1 || p->R < 1 || p->D < 1 || p->M < 1) return 0;
+static MlpPlans plans_of(const VmoeExpertMlpParams* p) {
+  if (p->dtype != VMOE_BF16) return MlpPlans{};
+  return mlp_plans(p->E, p->R, p->D, p->M, p->rows_per_expert != nullptr, p->x_rows != nullptr ? p->num_items : 0);
+}
+
+static size_t workspace_bytes(const VmoeExpertMlpParams* p, const MlpPlans& m) {
   const size_t b = p->dtype == VMOE_BF16 ? 2 : 4;
   size_t bytes = align256((size_t)p->E * p->R * p->M * b);  // hidden activations
   if (p->dtype == VMOE_BF16) {   // status words, launch plans of the ragged products, stream-K exchange
-    const MlpPlans m = mlp_plans(p->E, p->R, p->D, p->M, p->rows_per_expert != nullptr,
-                                  p->x_rows != nullptr ? p->num_items : 0);
     bytes += kStatusBytes + m.up_bytes + m.down_bytes + m.streamk_bytes;
-  }
-  if (p->dtype == VMOE_BF16) {
     if (p->w0t == nullptr) bytes += align256((size_t)p->E * p->D * p->M * b);
     if (p->w1t == nullptr) bytes += align256((size_t)p->E * p->D * p->M * b);
   }
   return bytes + bias_bytes(p);
+}
+
+extern "C" size_t vmoe_expert_mlp_workspace_bytes(const VmoeExpertMlpParams* p) {
+  if (p == nullptr || p->E < 1 || p->R < 1 || p->D < 1 || p->M < 1) return 0;
+  return workspace_bytes(p, plans_of(p));
 }
 
 // Where the pieces of a bfloat16 MLP's workspace lie, and what the planning launch is given.
@@ -537,6 +542,7 @@ struct MlpWorkspace {
   const bf16_t* b1 = nullptr;
   BiasCast biases{};                 // what has to be cast for that (o0 null: nothing)
   MlpPlans m;
+  bool fits = false;                 // the caller's workspace is there, aligned and large enough
   RaggedGeom ga{}, gb{};
   int plan_blocks = 0;               // workgroups of the planning launch (0: nothing to plan)
 };
@@ -545,13 +551,14 @@ MlpWorkspace mlp_workspace(const VmoeExpertMlpParams* p) {
   MlpWorkspace w;
   unsigned char* ws = static_cast<unsigned char*>(p->workspace);
   const size_t b = p->dtype == VMOE_BF16 ? 2 : 4;
+  w.m = plans_of(p);
+  const size_t need = workspace_bytes(p, w.m);
+  w.fits = p->workspace != nullptr && p->workspace_bytes >= need && aligned16(p->workspace);
   w.hidden = ws;
   ws += align256((size_t)p->E * p->R * p->M * b);
   if (p->dtype == VMOE_BF16) {
     w.status = reinterpret_cast<int32_t*>(ws);
     ws += kStatusBytes;
-    w.m = mlp_plans(p->E, p->R, p->D, p->M, p->rows_per_expert != nullptr,
-                                  p->x_rows != nullptr ? p->num_items : 0);
     if (w.m.up_bytes) w.plan_up = reinterpret_cast<int4*>(ws);
     ws += w.m.up_bytes;
     if (w.m.down_bytes) w.plan_down = reinterpret_cast<int4*>(ws);
@@ -571,7 +578,7 @@ MlpWorkspace mlp_workspace(const VmoeExpertMlpParams* p) {
   }
   w.rest = ws;
   if (has_f32_biases(p)) {
-    unsigned char* const at = static_cast<unsigned char*>(p->workspace) + vmoe_expert_mlp_workspace_bytes(p) - bias_bytes(p);
+    unsigned char* const at = static_cast<unsigned char*>(p->workspace) + need - bias_bytes(p);
     w.biases = BiasCast{(const float*)p->b0, (const float*)p->b1, reinterpret_cast<bf16_t*>(at),
                         reinterpret_cast<bf16_t*>(at + align256((size_t)p->E * p->M * 2)),
                         (size_t)p->E * p->M, (size_t)p->E * p->D};
@@ -589,14 +596,12 @@ MlpWorkspace mlp_workspace(const VmoeExpertMlpParams* p) {
 static int run_expert_mlp(const VmoeExpertMlpParams* p, vmoe_stream_t stream_, bool planned_already) {
   int rc = check_mlp(p);
   if (rc != VMOE_OK) return rc;
-  const size_t need = vmoe_expert_mlp_workspace_bytes(p);
-  if (p->workspace == nullptr || p->workspace_bytes < need || !aligned16(p->workspace))
-    return VMOE_E_WORKSPACE;
+  const MlpWorkspace w = mlp_workspace(p);
+  if (!w.fits) return VMOE_E_WORKSPACE;
   // Gathered rows come in whole 32-wide k tiles (float32: check_mlp), whichever kernel takes them.
   if (p->x_rows != nullptr && p->D % 32 != 0) return VMOE_E_UNSUPPORTED;
   hipStream_t stream = as_stream(stream_);
   const size_t b = p->dtype == VMOE_BF16 ? 2 : 4;
-  const MlpWorkspace w = mlp_workspace(p);
   void* hidden = w.hidden;
   int4* plan_up = w.plan_up;
   int4* plan_down = w.plan_down;
@@ -713,10 +718,9 @@ extern "C" int vmoe_expert_mlp_status(const VmoeExpertMlpParams* p, const int32_
   int rc = check_mlp(p);
   if (rc != VMOE_OK) return rc;
   if (p->dtype != VMOE_BF16) return VMOE_OK;       // the float32 kernels keep no such state
-  if (p->workspace == nullptr || p->workspace_bytes < vmoe_expert_mlp_workspace_bytes(p) ||
-      !aligned16(p->workspace))
-    return VMOE_E_WORKSPACE;
-  *status = mlp_workspace(p).status;
+  const MlpWorkspace w = mlp_workspace(p);
+  if (!w.fits) return VMOE_E_WORKSPACE;
+  *status = w.status;
   return VMOE_OK;
 }
 
@@ -733,14 +737,12 @@ extern "C" int vmoe_compact_rows_planned(const VmoeCompactRowsParams* c,
   if (mlp->E != c->E || (int64_t)mlp->R != (int64_t)c->G * c->C ||
       mlp->rows_per_expert != c->rows_per_expert)
     return VMOE_E_SHAPE;
-  if (mlp->workspace == nullptr || mlp->workspace_bytes < vmoe_expert_mlp_workspace_bytes(mlp) ||
-      !aligned16(mlp->workspace))
-    return VMOE_E_WORKSPACE;
+  const MlpWorkspace w = mlp_workspace(mlp);
+  if (!w.fits) return VMOE_E_WORKSPACE;
   // One launch needs the one-launch form of the compaction and an MLP whose products are planned or,
   // over few rows, need no plan.
   if (!compact_rows_fused_ok(c->G, c->S, c->E, c->K) || mlp->dtype != VMOE_BF16)
     return VMOE_E_UNSUPPORTED;
-  const MlpWorkspace w = mlp_workspace(mlp);
   if (!w.m.planned) return VMOE_E_UNSUPPORTED;
   const size_t n = (size_t)c->G * c->S * c->K;
   const unsigned compact_blocks = (unsigned)((n + 255) / 256);

@@ -73,7 +73,9 @@ inline double product_us(const RowsTile& t, int batch, int R, int N, int Kd, boo
   const double rounds = std::floor(tiles / full), rest = tiles - rounds * full;
   const double busy = rounds * round(t.per_cu) + (rest > 0 ? round(std::ceil(rest / (full / t.per_cu))) : 0);
   const double memory = 2.0 * batch * ((double)N * Kd + (double)R * (Kd + N)) / 4.4e6;
-  return 2.9 + std::pow(std::pow(busy, 4) + std::pow(memory, 4), 0.25);
+  // (their 4-norm.  A layer's calls estimate every tile of both products several times: with pow() that was
+  // 11 us of the host's 60 on one image.)
+  return 2.9 + std::sqrt(std::sqrt(busy * busy * busy * busy + memory * memory * memory * memory));
 }
 
 // The tile (index into kRowsTiles) that the table expects to be fastest.
