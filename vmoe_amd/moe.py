@@ -659,12 +659,6 @@ def sparse_moe_spmd(target, variable_axes: Optional[Mapping[str, Any]] = None,
       return _tree_stack(per_expert)
 
     def apply(self, variables, dispatcher: BaseDispatcher, *inputs):
-      def rounded():
-        # Outputs that combine rounds to bfloat16: float32 sums in another order would round the other
-        # way in one value of 4 000 (3e-5 of a Soft MoE layer's output).
-        return ({"float32_products": True} if isinstance(dispatcher, Bfloat16Dispatcher)
-                and getattr(self.expert.apply_experts, "takes_float32_products", False) else {})
-
       supports = getattr(dispatcher, "supports_packed", None)
       if (not has_aux and len(inputs) == 1 and supports is not None and supports()
           and getattr(self.expert, "supports_packed_rows", False)
@@ -688,11 +682,16 @@ def sparse_moe_spmd(target, variable_axes: Optional[Mapping[str, Any]] = None,
         else:
           dispatched, rows_per_expert = dispatcher.dispatch_packed(x)
           outputs = self.expert.apply_experts(variables, dispatched,
-                                              rows_per_expert=rows_per_expert, **rounded())
+                                              rows_per_expert=rows_per_expert)
         return _tree_map(dispatcher.combine_packed, outputs)
       dispatched = [dispatcher.dispatch(x) for x in inputs]
       if hasattr(self.expert, "apply_experts"):
-        outputs = self.expert.apply_experts(variables, *dispatched, **rounded())
+        # Soft MoE: outputs that combine rounds to bfloat16, where float32 sums in another order round the
+        # other way in one value of 4 000 (3e-5 of the layer's output).
+        rounded = (isinstance(dispatcher, Bfloat16Dispatcher)
+                   and getattr(self.expert.apply_experts, "takes_float32_products", False))
+        outputs = self.expert.apply_experts(variables, *dispatched,
+                                            **({"float32_products": True} if rounded else {}))
       else:
         num_experts = dispatched[0].shape[0]
         outs = [self.expert.apply(_tree_index(variables, e), *[d[e] for d in dispatched])
