@@ -1164,6 +1164,32 @@ def test_expert_mlp_every_small_tile(K, monkeypatch, tile):
   test_expert_mlp_small_tiles(K, 9, 1, 192, 72)
 
 
+@pytest.mark.parametrize("tile", range(8, 13))
+@pytest.mark.parametrize("E,R,D,M", [
+    (130, 64, 640, 776),     # several tiles per workgroup, column tiles and k that end inside
+    (40, 33, 768, 2048),     # one and two tiles, part of a row tile
+    (3, 128, 712, 1040),     # a full row tile where the tile has 128, else the small tiles
+    (9, 1, 640, 648),
+])
+def test_expert_mlp_tiles_walked_by_a_workgroup(K, monkeypatch, tile, E, R, D, M):
+  """The tile-walking kernel for few rows: the checks of the small tiles, and bit for bit what those
+  compute (same order of sums), also without a bias and with biases at an odd element."""
+  monkeypatch.setenv("VMOE_ROW_TILES", str(tile))
+  test_expert_mlp_small_tiles(K, E, R, D, M)
+  rng = np.random.default_rng(E)
+  mk = lambda scale, *s: to_dev(O.cast(rng.standard_normal(s).astype(np.float32) * scale, O.BF16), O.BF16)
+  x, w0, w1 = mk(1, E, R, D), mk(D ** -0.5, E, D, M), mk(M ** -0.5, E, M, D)
+  b0, b1 = mk(0.1, E * M + 1)[1:].view(E, M), mk(0.1, E * D + 1)[1:].view(E, D)
+  for biases in ((None, None), (b0, b1)):
+    for approximate in (True, False):
+      args = (x, w0, biases[0], w1, biases[1])
+      monkeypatch.setenv("VMOE_ROW_TILES", str(tile))
+      got = K.expert_mlp(*args, approximate_gelu=approximate)
+      monkeypatch.setenv("VMOE_ROW_TILES", "7")
+      want = K.expert_mlp(*args, approximate_gelu=approximate)
+      assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 def test_expert_mlp_planned_launch_random_fill(K):
   """bf16 expert products over packed rows with a die-balanced launch plan: random row
   counts (empty, one row, tile boundaries, full), expert counts below and above the

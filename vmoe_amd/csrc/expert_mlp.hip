@@ -358,7 +358,7 @@ bool down_prefers_half_tiles(int E, int R, int N) {
 
 // Launch plans of the two ragged products of an MLP: geometry, bytes, one planning launch.
 struct MlpPlans {
-  int up_rows = -1, down_rows = -1;      // tile of gemm_bf16_rows_kernel (kRowsTiles), -1: not taken
+  int up_rows = -1, down_rows = -1;      // tile of launch_gemm_bf16_rows, -1: not taken
   GemmGeom up, down;
   DownKernel down_kernel = kDownPlain;
   int down_bm = CfgDown::BM;
@@ -418,26 +418,36 @@ MlpPlans mlp_plans(int E, int R, int D, int M, bool ragged, long long items) {
   if (narrow_ok && t_narrow < 0.97 * t_best) { m.down_kernel = kDownNarrow; t_best = t_narrow; }
   // Few rows: the small tiles of gemm_bf16_rows.h where their estimate is below that of the large
   // ones (shapes that only the register-staged kernel would take always).
-  // (VMOE_ROW_TILES=off in the environment keeps the large tiles, VMOE_ROW_TILES=<index into kRowsTiles>
-  // takes that tile for both products wherever the kernel takes the operands: the switch behind the
+  // (VMOE_ROW_TILES=off in the environment keeps the large tiles, VMOE_ROW_TILES=<index into kRowsTiles, and
+  // behind them kStreamTiles> takes that tile for both products wherever the kernel takes the operands: the switch behind the
   // figures of the table, and what tests of the other kernels set)
   const char* const row_tiles = getenv("VMOE_ROW_TILES");
   const bool any_tile = row_tiles == nullptr || strcmp(row_tiles, "off") != 0;
   const int forced = any_tile && row_tiles != nullptr ? atoi(row_tiles) : -1;
-  const bool forced_ok = forced >= 0 && forced < kNumRowsTiles;
+  const auto forced_ok = [&](int Kd) {
+    return forced >= 0 && (forced < kNumRowsTiles || stream_tile_ok(forced - kNumRowsTiles, E, R, Kd, ragged));
+  };
   double rows_us = 0;
   if (any_tile && rows_gemm_ok(R, M, D, items)) {
     const int tile = best_rows_tile(E, R, M, D, &rows_us);
-    if (!m.up.fast || rows_us < product_us(kFirstProductTile, E, R, M, D, false)) m.up_rows = tile;
-    if (forced_ok) m.up_rows = forced;
+    double us = m.up.fast ? product_us(kFirstProductTile, E, R, M, D, false) : 1e30;
+    if (rows_us < us) { m.up_rows = tile; us = rows_us; }
+    const int walked = best_stream_tile(E, R, M, D, ragged, true, us);
+    if (walked >= 0) m.up_rows = walked;
+    if (forced_ok(D)) m.up_rows = forced;
   }
   if (any_tile && rows_gemm_ok(R, D, M, 0)) {
     const int tile = best_rows_tile(E, R, D, M, &rows_us);
     if (t_best > 1e29 && square.fast)
       t_best = unit * (half ? 0.5 * 1.05 * std::ceil((double)E * ((R + 127) / 128) * ((D + 255) / 256) / kNumCu)
                             : std::ceil((double)square.tiles / kNumCu));
-    if (rows_us < 5 + t_best) m.down_rows = tile;
-    if (forced_ok) m.down_rows = forced;
+    // (the model of the large tiles above counts their MFMAs; over few rows they wait for the weights:
+    // 128 experts x 128 rows x 768 x 3072 take 143 us, 5 TB/s, where it says 111)
+    double us = std::fmax(t_best, 2.0 * E * ((double)D * M + (double)R * (D + M)) / 5e6);
+    if (rows_us < 5 + t_best) { m.down_rows = tile; us = rows_us; }
+    const int walked = best_stream_tile(E, R, D, M, ragged, false, us);
+    if (walked >= 0) m.down_rows = walked;
+    if (forced_ok(M)) m.down_rows = forced;
   }
   // (VMOE_SECOND_PRODUCT=shared|eight|narrow|wide in the environment overrides the choice
   // where the named kernel applies: the switch behind the figures that the model above was

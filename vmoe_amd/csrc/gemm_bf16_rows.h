@@ -19,6 +19,7 @@
 #ifndef VMOE_GEMM_BF16_ROWS_H_
 #define VMOE_GEMM_BF16_ROWS_H_
 #include "gemm_bf16.h"
+#include "gemm_bf16_stream.h"
 
 namespace vmoe {
 
@@ -84,6 +85,61 @@ inline int best_rows_tile(int batch, int R, int N, int Kd, double* us) {
   for (int i = 0; i < kNumRowsTiles; ++i) {
     const double t = product_us(kRowsTiles[i], batch, R, N, Kd, true);
     if (best < 0 || t < *us) { best = i; *us = t; }
+  }
+  return best;
+}
+
+// The tiles of gemm_bf16_stream_kernel (VMOE_ROW_TILES counts them on behind kRowsTiles), and what the choice
+// is made from: a CU takes its tiles one after the other at step_us per 64 k, with the GELU's or the plain
+// epilogue behind each, and the launch cannot beat its weights at w_tbs plus its rows, once per column
+// tile, at a_tbs.  Fitted to 106 random shapes (4 - 128 experts, 12 - 128 rows, widths 384 - 4096; either product):
+// rms 5 % and less per tile, 30 % at worst.
+struct StreamTile {
+  int bm, bn;
+  double step_us, gelu_us, plain_us, fix_us, lat_us, w_tbs, a_tbs;
+};
+constexpr StreamTile kStreamTiles[] = {
+    {64, 192, 0.57, 3.8, 4.0, 2.0, 3.4, 8.5, 8.0},   {64, 256, 0.73, 4.1, 2.7, 2.0, 2.0, 7.3, 8.0},
+    {128, 128, 0.58, 3.3, 2.9, 3.0, 7.0, 9.0, 20.0}, {128, 256, 0.93, 6.1, 4.1, 2.0, 5.0, 6.9, 63.0},
+    {128, 192, 0.77, 4.7, 3.4, 2.0, 6.4, 9.0, 19.3}};
+constexpr int kNumStreamTiles = sizeof(kStreamTiles) / sizeof(kStreamTiles[0]);
+
+// f(StreamCfg of tile i).
+template <typename F>
+inline auto with_stream_tile(int i, F&& f) {
+  switch (i) {
+    case 0: return f(StreamCfg<64, 192, 4, 2, 3, 5>{});
+    case 1: return f(StreamCfg<64, 256, 1, 8, 3, 4>{});
+    case 2: return f(StreamCfg<128, 128, 2, 4, 3, 6>{});
+    case 3: return f(StreamCfg<128, 256, 2, 4, 3, 3>{});
+    default: return f(StreamCfg<128, 192, 4, 2, 3, 4>{});
+  }
+}
+
+inline bool stream_tile_ok(int i, int batch, int R, int Kd, bool ragged) {
+  return i >= 0 && i < kNumStreamTiles && with_stream_tile(i, [&](auto cfg) {
+    return stream_gemm_ok<decltype(cfg)>(batch, R, Kd, ragged);
+  });
+}
+
+// The tile (kNumRowsTiles + index into kStreamTiles) that should run the product in less than `us`
+// microseconds, the time of the kernel that has it otherwise, or -1.  It has to win by 8 %: the estimates of the
+// other kernels are off by 10 - 20 %, mostly upwards.  Below 24 rows most of a tile is padding and the 32-row
+// tiles win.  Over the same shapes the choice takes 8 380 us where the other kernels take 9 400 and the
+// fastest tile of all would take 8 320; 11 of 212 products get slower, by 11 % at worst.
+inline int best_stream_tile(int batch, int R, int N, int Kd, bool ragged, bool gelu, double us) {
+  if (R < 24) return -1;
+  int best = -1;
+  us *= 0.92;
+  for (int i = 0; i < kNumStreamTiles; ++i) {
+    if (!stream_tile_ok(i, batch, R, Kd, ragged)) continue;
+    const StreamTile& s = kStreamTiles[i];
+    const double units = (double)batch * ((N + s.bn - 1) / s.bn);
+    const double rounds = std::ceil(std::ceil(units / kNumXcd) / kCusPerXcd);
+    const double busy = s.fix_us + rounds * ((Kd + 63) / 64 * s.step_us + (gelu ? s.gelu_us : s.plain_us));
+    const double memory = s.lat_us + 2e-6 * Kd * ((double)batch * N / s.w_tbs + units * s.bm / s.a_tbs);
+    const double t = std::sqrt(std::sqrt(busy * busy * busy * busy + memory * memory * memory * memory));
+    if (t < us) { us = t; best = kNumRowsTiles + i; }
   }
   return best;
 }
@@ -307,7 +363,7 @@ int launch_rows_tile(const bf16_t* A, const bf16_t* Bt, const bf16_t* bias, bf16
   return launch_status();
 }
 
-// `tile`: index into kRowsTiles; waves, stages and 64-wide k tiles per stage of each.
+// `tile`: index into kRowsTiles, behind them into kStreamTiles; waves, stages and 64-wide k tiles per stage of each.
 template <int EPI>
 int launch_gemm_bf16_rows(int tile, const bf16_t* A, const bf16_t* Bt, const bf16_t* bias, bf16_t* C,
                           int batch, int R, int N, int Kd, hipStream_t stream, const int32_t* rows,
@@ -317,6 +373,11 @@ int launch_gemm_bf16_rows(int tile, const bf16_t* A, const bf16_t* Bt, const bf1
     return launch_rows_tile<decltype(cfg), EPI>(A, Bt, bias, C, batch, R, N, Kd, stream, rows, a_rows,
                                                 a_items, guard, clear, clear_count, status);
   };
+  if (tile >= kNumRowsTiles)
+    return with_stream_tile(tile - kNumRowsTiles, [&](auto cfg) {
+      return launch_gemm_bf16_stream<decltype(cfg), EPI>(A, Bt, bias, C, batch, R, N, Kd, stream, rows, a_rows,
+                                                         a_items, guard, clear, clear_count, status);
+    });
   switch (tile) {
     case 0: return run(RowsCfg<32, 32, 2, 2, 4, 2>{});
     case 1: return run(RowsCfg<64, 32, 2, 2, 3, 2>{});
