@@ -276,8 +276,10 @@ int vmoe_combine(const VmoeCombineParams* p, vmoe_stream_t stream);
  *   vmoe_combine_backward_data:     dy[slot(t,k)] = w[t,k] * dout[t]; slots no item claims
  *                                   get 0 (slot_token given) or stay untouched (null);
  *   vmoe_combine_backward_weights:  dweights[t,k] = <dout[t], y[slot(t,k)]>, 0 if dropped.
+ *   vmoe_combine_backward:          both of them, in one pass over dout for up to four choices per item.
  * The gradient of dispatch with respect to its input, dx[t] = sum_k dbuf[slot(t,k)], is
- * vmoe_combine with unit weights.  Row width as for dispatch / combine. */
+ * vmoe_dispatch_backward: vmoe_combine with unit weights (`weights` is not read).  Row width as for
+ * dispatch / combine. */
 typedef struct {
   const void* dout;           /* (num_items, D) dtype: gradient of combine's output */
   const void* y;              /* (num_slots, D) dtype: combine's input (weights gradient only) */
@@ -291,6 +293,8 @@ typedef struct {
 } VmoeCombineBackwardParams;
 int vmoe_combine_backward_data(const VmoeCombineBackwardParams* p, vmoe_stream_t stream);
 int vmoe_combine_backward_weights(const VmoeCombineBackwardParams* p, vmoe_stream_t stream);
+int vmoe_combine_backward(const VmoeCombineBackwardParams* p, vmoe_stream_t stream);
+int vmoe_dispatch_backward(const VmoeCombineParams* p, vmoe_stream_t stream);
 
 /* Dense (G,S,E,C) view of a sparse assignment, for callers that read
  * EinsumDispatcher.combine_weights / dispatch_weights (vmoe/moe.py:609-619):

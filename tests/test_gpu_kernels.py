@@ -1901,6 +1901,11 @@ def _wrapper_calls():
     yield ("vmoe_combine_backward_data", lambda K, x=items, t=slots, w=weights:
            (K.combine_backward_data(x, t(K)[0], w, t(K)[1], E * G * C),))
     yield "vmoe_combine_backward_weights", lambda K, x=items, y=buf, t=slots: (K.combine_backward_weights(x, y, t(K)[0]),)
+    yield ("vmoe_combine_backward", lambda K, x=items, y=buf, t=slots, w=weights:
+           K.combine_backward(x, y, t(K)[0], w, t(K)[1]))
+    yield "vmoe_dispatch_backward", lambda K, y=buf, t=slots: (K.dispatch_backward(y, t(K)[0]),)
+    pairs = torch.stack([torch.arange(G * S * k, device=dev()) % (E + 1), torch.arange(G * S * k, device=dev()) // 8], -1)
+    yield "vmoe_indices_to_slots", lambda K, i=pairs.view(G, S, k, 2): K.indices_to_slots(i, E, C)
     wts = mk(dtype, G, S, E, 5)
     yield "vmoe_einsum_dispatch", lambda K, w=wts, x=x: (K.einsum_dispatch(w, x, x.dtype),)
     yield "vmoe_einsum_combine", lambda K, w=wts, y=mk(dtype, E * G * 5, D): (K.einsum_combine(w, y, y.dtype),)

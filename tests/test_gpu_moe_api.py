@@ -1064,6 +1064,32 @@ def test_dispatch_combine_gradients(moe, dtype):
   assert (to_np(w.grad).reshape(G * S, K)[~kept.cpu().numpy()] == 0).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,K_,D,NS", [(1, 1, 8, 1), (37, 2, 520, 60), (130, 3, 64, 500), (50, 4, 1032, 190), (33, 5, 16, 170)])
+def test_combine_backward_is_both_gradients(moe, dtype, T, K_, D, NS):
+  """One launch (up to four choices, two beyond) against the launch per gradient, bit for bit: dropped
+  choices, unclaimed slots with and without their zeros, rows of a chunk and of several rounds; and
+  dispatch's gradient against combine with ones."""
+  from vmoe_amd import kernels as K
+  gen = torch.Generator().manual_seed(T + K_)
+  mk = lambda *s: torch.randn(s, generator=gen).to(dtype).cuda()
+  flat = torch.full((T * K_,), -1, dtype=torch.int32)
+  n = min(T * K_, NS) * 3 // 4 + 1
+  kept = torch.randperm(T * K_, generator=gen)[:n]
+  flat[kept] = torch.randperm(NS, generator=gen)[:n].int()
+  slot_token = torch.full((NS,), -1, dtype=torch.int32)
+  slot_token[flat[kept].long()] = (kept // K_).int()
+  token_slot, slot_token = flat.view(T, K_).cuda(), slot_token.cuda()
+  dout, y, w = mk(T, D), mk(NS, D), torch.rand((T, K_), generator=gen).cuda()
+  dy, dw = K.combine_backward(dout, y, token_slot, w, slot_token)
+  assert torch.equal(dy, K.combine_backward_data(dout, token_slot, w, slot_token, NS))
+  assert torch.equal(dw, K.combine_backward_weights(dout, y, token_slot))
+  dy, _ = K.combine_backward(dout, y, token_slot, w, None)
+  claimed = slot_token >= 0
+  assert torch.equal(dy[claimed], K.combine_backward_data(dout, token_slot, w, slot_token, NS)[claimed])
+  assert torch.equal(K.dispatch_backward(y, token_slot), K.combine(y, token_slot, torch.ones_like(w)))
+
+
 def test_combine_backward_data_zero_fills_unclaimed_slots(moe):
   from vmoe_amd import kernels as K
   rng = np.random.default_rng(42)

@@ -217,6 +217,10 @@ def _bad_calls():
        dict(dout=[(6,), (6, 2, 8)], token_slot=[(), (5, 2)], weights=[(5, 2)], slot_token=[(8,)])),
       ("combine_backward_weights", dict(dout=f32(6, 8), y=f32(9, 8), token_slot=i32(6, 2)),
        dict(dout=[(6,), (6, 2, 8)], y=[(9,), (9, 2, 4), (9, 7)], token_slot=[(), (5, 2)])),
+      ("combine_backward", dict(dout=f32(6, 8), y=f32(9, 8), token_slot=i32(6, 2), weights=f32(6, 2), slot_token=i32(9)),
+       dict(dout=[(6,), (6, 2, 8)], y=[(9,), (9, 7)], token_slot=[(), (5, 2)], weights=[(5, 2)], slot_token=[(8,)])),
+      ("dispatch_backward", dict(dbuf=f32(9, 8), token_slot=i32(6, 2)), dict(dbuf=[(9,), (9, 2, 8)], token_slot=[(12,), (2, 3, 2)])),
+      ("indices_to_slots", dict(indices=i32(2, 6, 2, 2), num_experts=4, capacity=3), dict(indices=[(12, 2), (2, 6, 2, 1)])),
       ("add_layer_norm", dict(residual=f32(6, 8), branch=f32(6, 8), scale=f32(8), bias=f32(8), eps=1e-6, out_dtype=torch.float32),
        dict(residual=[()], branch=[(6, 4)], scale=[(7,)], bias=[(7,)])),
       ("attention", dict(q=f32(2, 5, 3, 64), k=f32(2, 7, 3, 64), v=f32(2, 7, 3, 64), scale=0.125),

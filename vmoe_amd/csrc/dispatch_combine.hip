@@ -140,6 +140,7 @@ template <> struct Chunk<bf16_t> {
   }
 };
 
+// (`weights` null, here and in the two kernels below: every weight is one)
 template <typename T>
 __global__ __launch_bounds__(kMoveThreads) void combine_kernel(
     const uint4* __restrict__ y, const int32_t* __restrict__ token_slot,
@@ -154,7 +155,7 @@ __global__ __launch_bounds__(kMoveThreads) void combine_kernel(
     const int r = tid / K;
     const bool ok = t0 + r < num_items;
     slots[tid] = ok ? checked_slot(token_slot[(size_t)t0 * K + tid], num_slots) : -1;
-    wts[tid] = ok ? weights[(size_t)t0 * K + tid] : 0.f;
+    wts[tid] = !ok ? 0.f : weights != nullptr ? weights[(size_t)t0 * K + tid] : 1.f;
   }
   __syncthreads();
   const int total = kRowsPerBlock * cpr;
@@ -213,7 +214,7 @@ __global__ __launch_bounds__(kMoveThreads) void combine_listed_kernel(
       const int k = k0 + lane;
       const size_t at = (size_t)(t0 + r) * K + k;
       const int slot = k < K ? checked_slot(token_slot[at], num_slots) : -1;
-      const float w = k < K ? weights[at] : 0.f;
+      const float w = k >= K ? 0.f : weights != nullptr ? weights[at] : 1.f;
       const uint64_t on = __ballot(slot >= 0);
       if (slot >= 0) {
         const int i = r * K + n + __popcll(on & ((1ull << lane) - 1));
@@ -273,7 +274,7 @@ __global__ __launch_bounds__(kMoveThreads) void combine_generic_kernel(
     for (int k = 0; k < K; ++k) {
       const int slot = checked_slot(token_slot[(size_t)t * K + k], num_slots);
       if (slot < 0) continue;
-      float w = weights[(size_t)t * K + k];
+      float w = weights != nullptr ? weights[(size_t)t * K + k] : 1.f;
       float a[N];
       Chunk<T>::unpack(y[(size_t)slot * cpr + ch], a);
 #pragma unroll
@@ -389,6 +390,64 @@ __global__ __launch_bounds__(kMoveThreads) void row_dots_kernel(
   }
 }
 
+// Both in one pass: a wave per item reads its gradient row once and, for each choice, the row that combine
+// read and writes the row's gradient beside it, all reads of a chunk in flight before the first sum.  The sums of dw are
+// taken in row_dots_kernel's order, the rows are scatter_scaled_kernel's: the same bits.  16 x 1 568 items x
+// 768 bfloat16, two of 32 experts: 190 MB instead of 229, 40 us where the two launches take 22 + 22.
+constexpr int kBackwardK = 4;
+template <typename T>
+__global__ __launch_bounds__(kMoveThreads) void combine_backward_kernel(
+    const uint4* __restrict__ g, const uint4* __restrict__ y, const int32_t* __restrict__ token_slot,
+    const float* __restrict__ weights, const int32_t* __restrict__ slot_token, uint4* __restrict__ dy,
+    float* __restrict__ dw, int num_items, int num_slots, int K, int cpr) {
+  constexpr int N = Chunk<T>::n;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(
+      (int)((blockIdx.x * (unsigned)kMoveThreads + threadIdx.x) >> 6));
+  if (wave >= num_items) {
+    const int s = wave - num_items;
+    if (slot_token != nullptr && s < num_slots && slot_token[s] < 0)
+      for (int ch = lane; ch < cpr; ch += kWave) store_stream(dy + (size_t)s * cpr + ch, make_uint4(0, 0, 0, 0));
+    return;
+  }
+  int slot[kBackwardK];
+  float w[kBackwardK], acc[kBackwardK];
+#pragma unroll
+  for (int k = 0; k < kBackwardK; ++k) {
+    slot[k] = k < K ? checked_slot(token_slot[(size_t)wave * K + k], num_slots) : -1;
+    w[k] = k < K ? weights[(size_t)wave * K + k] : 0.f;
+    acc[k] = 0.f;
+  }
+  for (int ch = lane; ch < cpr; ch += kWave) {
+    const uint4 vg = load_stream(g + (size_t)wave * cpr + ch);
+    uint4 vy[kBackwardK];
+#pragma unroll
+    for (int k = 0; k < kBackwardK; ++k)
+      if (slot[k] >= 0) vy[k] = load_stream(y + (size_t)slot[k] * cpr + ch);
+    float a[N];
+    Chunk<T>::unpack(vg, a);
+#pragma unroll
+    for (int k = 0; k < kBackwardK; ++k) {
+      if (slot[k] < 0) continue;
+      float b[N];
+      Chunk<T>::unpack(vy[k], b);
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        acc[k] += a[j] * b[j];
+        b[j] = __fmul_rn(w[k], a[j]);
+      }
+      store_stream(dy + (size_t)slot[k] * cpr + ch, Chunk<T>::pack(b));
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < kBackwardK; ++k) {
+    if (k >= K) break;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) acc[k] += __shfl_xor(acc[k], o, kWave);
+    if (lane == 0) dw[(size_t)wave * K + k] = acc[k];
+  }
+}
+
 int check_move(const void* a, const void* b, const void* c, int num_items, int num_slots, int K,
                int D, int dtype) {
   if (a == nullptr || b == nullptr || c == nullptr) return VMOE_E_NULL;
@@ -433,8 +492,8 @@ extern "C" int vmoe_dispatch(const VmoeDispatchParams* p, vmoe_stream_t stream) 
   return launch_status();
 }
 
-extern "C" int vmoe_combine(const VmoeCombineParams* p, vmoe_stream_t stream) {
-  if (p == nullptr || p->weights == nullptr) return VMOE_E_NULL;
+// `weights`: p->weights, or null for unit weights.
+static int run_combine(const VmoeCombineParams* p, const float* weights, vmoe_stream_t stream) {
   int rc = check_move(p->y, p->token_slot, p->out, p->num_items, p->num_slots, p->K, p->D, p->dtype);
   if (rc != VMOE_OK) return rc;
   const int cpr = (int)((size_t)p->D * (p->dtype == VMOE_BF16 ? 2 : 4) / 16);
@@ -446,7 +505,7 @@ extern "C" int vmoe_combine(const VmoeCombineParams* p, vmoe_stream_t stream) {
     auto kern = listed ? (bf16 ? combine_listed_kernel<bf16_t> : combine_listed_kernel<float>)
                        : (bf16 ? combine_kernel<bf16_t> : combine_kernel<float>);
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(kMoveThreads), lds, as_stream(stream), (const uint4*)p->y,
-                       p->token_slot, p->weights, (uint4*)p->out, p->num_items, p->num_slots, p->K, cpr,
+                       p->token_slot, weights, (uint4*)p->out, p->num_items, p->num_slots, p->K, cpr,
                        chunk_magic(cpr));
   } else {
     const int blocks = (p->num_items + 3) / 4;
@@ -460,6 +519,16 @@ extern "C" int vmoe_combine(const VmoeCombineParams* p, vmoe_stream_t stream) {
                          (uint4*)p->out, p->num_items, p->num_slots, p->K, cpr);
   }
   return launch_status();
+}
+
+extern "C" int vmoe_combine(const VmoeCombineParams* p, vmoe_stream_t stream) {
+  if (p == nullptr || p->weights == nullptr) return VMOE_E_NULL;
+  return run_combine(p, p->weights, stream);
+}
+
+extern "C" int vmoe_dispatch_backward(const VmoeCombineParams* p, vmoe_stream_t stream) {
+  if (p == nullptr) return VMOE_E_NULL;
+  return run_combine(p, nullptr, stream);
 }
 
 extern "C" int vmoe_copy_bytes(const void* in, void* out, size_t n, vmoe_stream_t stream) {
@@ -526,5 +595,25 @@ extern "C" int vmoe_combine_backward_weights(const VmoeCombineBackwardParams* p,
     hipLaunchKernelGGL(row_dots_kernel<float>, dim3(blocks), dim3(kMoveThreads), 0,
                        as_stream(stream), (const uint4*)p->dout, (const uint4*)p->y, p->token_slot,
                        p->dweights, p->num_items, p->num_slots, p->K, cpr);
+  return launch_status();
+}
+
+extern "C" int vmoe_combine_backward(const VmoeCombineBackwardParams* p, vmoe_stream_t stream) {
+  if (p == nullptr || p->weights == nullptr || p->dy == nullptr || p->y == nullptr || p->dweights == nullptr)
+    return VMOE_E_NULL;
+  const long long waves = (long long)p->num_items + (p->slot_token != nullptr ? p->num_slots : 0);
+  // More choices (experts choice: K = E) or more waves than an int numbers: one gradient after the other.
+  if (p->K > kBackwardK || waves >= INT32_MAX) {
+    const int rc = vmoe_combine_backward_data(p, stream);
+    return rc != VMOE_OK ? rc : vmoe_combine_backward_weights(p, stream);
+  }
+  int rc = check_move(p->dout, p->token_slot, p->dy, p->num_items, p->num_slots, p->K, p->D, p->dtype);
+  if (rc != VMOE_OK) return rc;
+  if (!aligned16(p->y)) return VMOE_E_ALIGN;
+  const int cpr = (int)((size_t)p->D * (p->dtype == VMOE_BF16 ? 2 : 4) / 16);
+  auto kern = p->dtype == VMOE_BF16 ? combine_backward_kernel<bf16_t> : combine_backward_kernel<float>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)((waves + 3) / 4)), dim3(kMoveThreads), 0, as_stream(stream),
+                     (const uint4*)p->dout, (const uint4*)p->y, p->token_slot, p->weights, p->slot_token,
+                     (uint4*)p->dy, p->dweights, p->num_items, p->num_slots, p->K, cpr);
   return launch_status();
 }

@@ -369,6 +369,44 @@ static ffi::Error CombineBackwardWeightsImpl(hipStream_t stream, Any dout, Any y
 XLA_FFI_DEFINE_HANDLER_SYMBOL(VmoeCombineBackwardWeights, CombineBackwardWeightsImpl,
                               ffi::Ffi::Bind().Ctx<Stream>().Arg<Any>().Arg<Any>().Arg<S32>().Ret<F32>());
 
+// dout (G,S,D), y (E, G*C, D), token_slot, weights (G,S,K), slot_token (E*G*C,) -> dy (E, G*C, D), dweights (G,S,K) f32
+static ffi::Error CombineBackwardImpl(hipStream_t stream, Any dout, Any y, S32 token_slot, F32 weights,
+                                      S32 slot_token, AnyOut dy, F32Out dweights, bool zero_fill) {
+  VmoeCombineBackwardParams p{};
+  p.dout = dout.untyped_data();
+  p.y = y.untyped_data();
+  p.token_slot = token_slot.typed_data();
+  p.weights = weights.typed_data();
+  p.slot_token = zero_fill ? slot_token.typed_data() : nullptr;
+  p.dy = dy->untyped_data();
+  p.dweights = dweights->typed_data();
+  p.K = (int32_t)token_slot.dimensions().back();
+  p.num_items = (int32_t)(token_slot.element_count() / p.K);
+  p.D = (int32_t)dout.dimensions().back();
+  p.num_slots = (int32_t)(y.element_count() / p.D);
+  p.dtype = DType(dout.element_type());
+  return Status(vmoe_combine_backward(&p, stream), "vmoe_combine_backward");
+}
+XLA_FFI_DEFINE_HANDLER_SYMBOL(VmoeCombineBackward, CombineBackwardImpl,
+                              ffi::Ffi::Bind().Ctx<Stream>().Arg<Any>().Arg<Any>().Arg<S32>().Arg<F32>().Arg<S32>()
+                                  .Ret<Any>().Ret<F32>().Attr<bool>("zero_fill"));
+
+// dbuf (E, G*C, D), token_slot (G,S,K) -> dx (G,S,D)
+static ffi::Error DispatchBackwardImpl(hipStream_t stream, Any dbuf, S32 token_slot, AnyOut dx) {
+  VmoeCombineParams p{};
+  p.y = dbuf.untyped_data();
+  p.token_slot = token_slot.typed_data();
+  p.out = dx->untyped_data();
+  p.K = (int32_t)token_slot.dimensions().back();
+  p.num_items = (int32_t)(token_slot.element_count() / p.K);
+  p.D = (int32_t)dbuf.dimensions().back();
+  p.num_slots = (int32_t)(dbuf.element_count() / p.D);
+  p.dtype = DType(dbuf.element_type());
+  return Status(vmoe_dispatch_backward(&p, stream), "vmoe_dispatch_backward");
+}
+XLA_FFI_DEFINE_HANDLER_SYMBOL(VmoeDispatchBackward, DispatchBackwardImpl,
+                              ffi::Ffi::Bind().Ctx<Stream>().Arg<Any>().Arg<S32>().Ret<Any>());
+
 // indices (G,S,K,2), weights (G,S,K) -> combine (G,S,E,C) f32, dispatch (G,S,E,C) bool
 static ffi::Error DensifyImpl(hipStream_t stream, S32 indices, F32 weights, F32Out combine,
                               ffi::Result<ffi::Buffer<ffi::PRED>> dispatch) {

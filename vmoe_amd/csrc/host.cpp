@@ -437,6 +437,56 @@ Tensor combine_backward_weights(int64_t stream, const Tensor& dout_, const Tenso
   return dw;
 }
 
+// -> (dy, dweights) of combine.
+std::tuple<Tensor, Tensor> combine_backward(int64_t stream, const Tensor& dout_, const Tensor& y_, const Tensor& token_slot,
+                                            const Tensor& weights_, const OptTensor& slot_token) {
+  need_axes(dout_, 2, "dout");
+  need_axes(y_, 2, "y");
+  if (token_slot.dim() < 1) need_axes(token_slot, 2, "token_slot");
+  const Tensor dout = dout_.contiguous(), y = y_.contiguous(), weights = as_f32(weights_);
+  need_values(token_slot, dout.size(0) * token_slot.size(-1), "token_slot");
+  need_values(weights, dout.size(0) * token_slot.size(-1), "weights");
+  need_values(slot_token, y.size(0), "slot_token");
+  need_values(y, y.size(0) * dout.size(1), "y");
+  Tensor dy = empty({y.size(0), dout.size(1)}, dout.scalar_type(), dout);
+  Tensor dw = f32({dout.size(0), token_slot.size(-1)}, dout);
+  VmoeCombineBackwardParams p{};
+  p.dout = ptr(dout); p.y = ptr(y); p.token_slot = ptr_as<int32_t>(token_slot); p.weights = ptr_as<float>(weights);
+  p.slot_token = ptr_as<int32_t>(slot_token); p.dy = ptr(dy); p.dweights = ptr_as<float>(dw);
+  p.num_items = (int32_t)dout.size(0); p.num_slots = (int32_t)y.size(0); p.K = (int32_t)token_slot.size(-1);
+  p.D = (int32_t)dout.size(1); p.dtype = dtype_code(dout);
+  check(vmoe_combine_backward(&p, stream_of(stream)), "vmoe_combine_backward");
+  return {dy, dw};
+}
+
+// -> dx of dispatch.
+Tensor dispatch_backward(int64_t stream, const Tensor& dbuf_, const Tensor& token_slot) {
+  need_axes(dbuf_, 2, "dbuf");
+  need_axes(token_slot, 2, "token_slot");
+  const Tensor dbuf = dbuf_.contiguous();
+  const int64_t D = dbuf.size(1), T = token_slot.size(0);
+  Tensor dx = empty({T, D}, dbuf.scalar_type(), dbuf);
+  VmoeCombineParams p{ptr(dbuf), ptr_as<int32_t>(token_slot), nullptr, ptr(dx), (int32_t)T, (int32_t)dbuf.size(0),
+                      (int32_t)token_slot.size(1), (int32_t)D, dtype_code(dbuf)};
+  check(vmoe_dispatch_backward(&p, stream_of(stream)), "vmoe_dispatch_backward");
+  return dx;
+}
+
+// -> (token_slot (G, S, K), slot_token (E * G * C,), counters (2,): duplicates, invalid).
+std::tuple<Tensor, Tensor, Tensor> indices_to_slots(int64_t stream, const Tensor& indices_, int64_t E, int64_t C) {
+  need_axes(indices_, 4, "indices");
+  const Tensor indices = indices_.to(at::kInt).contiguous();
+  const int64_t G = indices.size(0), S = indices.size(1), K = indices.size(2);
+  need_values(indices, 2 * G * S * K, "indices");
+  const auto i32 = indices.options();
+  Tensor token_slot = at::empty({G, S, K}, i32), slot_token = at::empty({E * G * C}, i32), counters = at::zeros({2}, i32);
+  int32_t* const counts = ptr_as<int32_t>(counters);
+  VmoeIndicesToSlotsParams p{ptr_as<int32_t>(indices), ptr_as<int32_t>(token_slot), ptr_as<int32_t>(slot_token), counts,
+                             counts + 1, (int32_t)G, (int32_t)S, (int32_t)E, (int32_t)K, (int32_t)C};
+  check(vmoe_indices_to_slots(&p, stream_of(stream)), "vmoe_indices_to_slots");
+  return {token_slot, slot_token, counters};
+}
+
 }  // namespace
 
 // Calls run without the interpreter's lock, as ctypes makes them (a launch can wait for room in the
@@ -468,4 +518,7 @@ PYBIND11_MODULE(_vmoe_host, m) {
   VMOE_DEF(soft_route_stats);
   VMOE_DEF(combine_backward_data);
   VMOE_DEF(combine_backward_weights);
+  VMOE_DEF(combine_backward);
+  VMOE_DEF(dispatch_backward);
+  VMOE_DEF(indices_to_slots);
 }

@@ -184,6 +184,8 @@ def top_items_metrics(gates: torch.Tensor, capacity: int):
 
 def indices_to_slots(indices: torch.Tensor, num_experts: int, capacity: int):
   """indices (G,S,K,2) -> token_slot (G,S,K), slot_token (E*G*C,), counters (2,) [dups, invalid]."""
+  if not H.timed("vmoe_indices_to_slots"):
+    return H.host().indices_to_slots(H.raw_stream(), indices, int(num_experts), int(capacity))
   G, S, K, _ = indices.shape
   dev = indices.device
   indices = indices.to(torch.int32).contiguous()
@@ -281,6 +283,38 @@ def combine_backward_weights(dout: torch.Tensor, y: torch.Tensor,
                               H.ptr(dw), T, y.shape[0], Kk, D, H.dtype_code(dout.dtype))
   H.call("vmoe_combine_backward_weights", p)
   return dw
+
+
+def combine_backward(dout: torch.Tensor, y: torch.Tensor, token_slot: torch.Tensor,
+                     weights: torch.Tensor, slot_token: Optional[torch.Tensor]):
+  """-> (combine_backward_data(...), combine_backward_weights(...)), in one pass over dout."""
+  if not H.timed("vmoe_combine_backward"):
+    return H.host().combine_backward(H.raw_stream(), dout, y, token_slot, weights, slot_token)
+  T, D = dout.shape
+  Kk = token_slot.shape[-1]
+  dout, y = dout.contiguous(), y.contiguous()
+  weights = weights.to(torch.float32).contiguous()
+  dy = torch.empty((y.shape[0], D), dtype=dout.dtype, device=dout.device)
+  dw = _f32(T, Kk, device=dout.device)
+  p = H.CombineBackwardParams(H.ptr(dout), H.ptr(y), H.ptr(token_slot), H.ptr(weights),
+                              H.ptr(slot_token), H.ptr(dy), H.ptr(dw), T, y.shape[0], Kk, D,
+                              H.dtype_code(dout.dtype))
+  H.call("vmoe_combine_backward", p)
+  return dy, dw
+
+
+def dispatch_backward(dbuf: torch.Tensor, token_slot: torch.Tensor) -> torch.Tensor:
+  """dbuf (NS,D), token_slot (T,K) -> dx (T,D): dx[t] = sum_k dbuf[slot(t,k)]."""
+  if not H.timed("vmoe_dispatch_backward"):
+    return H.host().dispatch_backward(H.raw_stream(), dbuf, token_slot)
+  NS, D = dbuf.shape
+  T, Kk = token_slot.shape
+  dbuf = dbuf.contiguous()
+  dx = torch.empty((T, D), dtype=dbuf.dtype, device=dbuf.device)
+  p = H.CombineParams(H.ptr(dbuf), H.ptr(token_slot), None, H.ptr(dx), T, NS, Kk, D,
+                      H.dtype_code(dbuf.dtype))
+  H.call("vmoe_dispatch_backward", p)
+  return dx
 
 
 def densify(indices: torch.Tensor, weights: torch.Tensor, num_experts: int, capacity: int):

@@ -68,8 +68,7 @@ class _DispatchFn(torch.autograd.Function):
   @staticmethod
   def backward(ctx, grad):
     (token_slot,) = ctx.saved_tensors
-    ones = torch.ones(token_slot.shape, dtype=torch.float32, device=grad.device)
-    return K.combine(grad.contiguous(), token_slot, ones), None, None, None
+    return K.dispatch_backward(grad, token_slot), None, None, None
 
 
 class _CombineFn(torch.autograd.Function):
@@ -86,6 +85,9 @@ class _CombineFn(torch.autograd.Function):
     rows, token_slot, weights, slot_token = ctx.saved_tensors
     grad = grad.contiguous()
     d_rows = d_w = None
+    if ctx.needs_input_grad[0] and ctx.needs_input_grad[2] and grad.dtype == rows.dtype:
+      d_rows, d_w = K.combine_backward(grad, rows, token_slot, weights, slot_token)
+      return d_rows, None, d_w.to(weights.dtype), None
     if ctx.needs_input_grad[0]:
       d_rows = K.combine_backward_data(grad, token_slot, weights, slot_token, rows.shape[0])
     if ctx.needs_input_grad[2]:
