@@ -1190,6 +1190,41 @@ def test_expert_mlp_tiles_walked_by_a_workgroup(K, monkeypatch, tile, E, R, D, M
       assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
+@pytest.mark.parametrize("S,E,k,C,spread", [
+    (511, 7, 2, 60, 1.0), (513, 8, 1, 70, 1.0), (1925, 7, 4, 300, 1.0), (2048, 4, 2, 512, 0.5), (4100, 32, 2, 130, 1.0),
+    (900, 8, 2, 120, 1e-3),        # gates closer than a bin: sorted
+    (700, 8, 2, 90, 0.02),         # long bins, counted
+    (600, 4, 2, 150, 40.0),        # gates that reach 1 and 0
+])
+def test_float32_gates_ranked_by_counting(K, S, E, k, C, spread):
+  """Batch priority and experts choice over float32 gates (bins by their high halves, low halves and items
+  inside a bin) against a stable sort, equal gates and gates one bit apart among them."""
+  rng = np.random.default_rng(S)
+  G = 2
+  logits = (rng.standard_normal((G, S, E)) * spread).astype(np.float32)
+  logits[:, 5::7] = logits[:, 3:4]                              # equal gates
+  gates = O.softmax(logits).astype(np.float32)
+  gates[:, 11::13] = np.nextafter(gates[:, 11::13], np.float32(0))
+  g = to_dev(gates)
+  val, idx = K.topk(g, k)
+  for bpr in (True, False):
+    indices, token_slot, slot_token, fill = (to_np(t) for t in K.route_assign(val, idx, E, C, bpr)[:4])
+    v, i = to_np(val), to_np(idx)
+    for n in range(G):
+      order = np.argsort(-v[n, :, 0], kind="stable") if bpr else np.arange(S)
+      seen, pos = np.zeros(E, np.int64), np.zeros((S, k), np.int64)
+      for j in range(k):
+        for s in order:
+          pos[s, j] = seen[i[n, s, j]]
+          seen[i[n, s, j]] += 1
+      np.testing.assert_array_equal(indices[n, ..., 1], pos)
+  cols = K.top_items_metrics(g, C)
+  want = np.argsort(-gates, axis=1, kind="stable")              # (G, rank, E)
+  slot_token = to_np(cols[2]).reshape(E, G, C)
+  for n in range(G):
+    np.testing.assert_array_equal(slot_token[:, n], (n * S + want[n, :C]).T)
+
+
 def test_expert_mlp_planned_launch_random_fill(K):
   """bf16 expert products over packed rows with a die-balanced launch plan: random row
   counts (empty, one row, tile boundaries, full), expert counts below and above the

@@ -128,6 +128,7 @@ __device__ __forceinline__ void bitonic_sort_lds(uint64_t* keys, int SP, int tid
 
 constexpr int kHeld = 8;           // choices of a thread kept in registers
 constexpr int kRankBins = 1024;    // bins of the counting rank: gates from 1 down to 2^-8
+constexpr uint32_t kLongestBin = 512;
 
 template <int R>
 __device__ __forceinline__ void route_assign_group(
@@ -183,26 +184,29 @@ __device__ __forceinline__ void route_assign_group(
         bits[r] = (tid < nact && s < S) ? __builtin_bit_cast(uint32_t, val[(size_t)s * K]) : 0u;
         narrow_ok = narrow_ok && bpr_gate_is_narrow(bits[r]);
       }
-      // Narrow gates within a factor 2^8 of 1 (the largest gate of a softmax over up to 128
-      // experts always is) take at most kRankBins distinct values, in descending order as
-      // the bin number 0x3F80 - (bits >> 16) ascends: the rank of an item is then the number
-      // of items in lower bins plus the number of items of its own bin with a lower index
-      // -- a histogram, a prefix sum, a scatter into the bins' segments and a count inside
-      // the item's own segment, four barriers in all, where the bitonic sort of 2 048 keys
-      // takes 66 compare-exchange steps (15 of the kernel's 22 us on the headline layer).
+      // Gates within a factor 2^8 of 1 (the largest gate of a softmax over up to 128
+      // experts always is) fall into kRankBins bins by their high 16 bits, in descending order
+      // as the bin number 0x3F80 - (bits >> 16) ascends (narrow gates of a bin are equal): the rank of
+      // an item is then the number of items in lower bins plus the number of items of its own bin
+      // with a lower bin_key32 -- a histogram, a prefix sum, a scatter into the bins' segments and a count
+      // inside the item's own segment, four barriers in all, where the bitonic sort of 2 048 keys
+      // takes 66 compare-exchange steps (15 of the kernel's 22 us on the headline layer; float32 gates,
+      // 64-bit keys: 1 925 items x 4 of 7 experts 27 -> 17 us).
       // Every step counts, none depends on the order in which the threads arrive, so the
-      // ranks are those of the sort.  A segment as long as the group (all gates equal) costs
-      // what the sort costs.
-      bool count_ok = narrow_ok;
+      // ranks are those of the sort.  The count is quadratic in a segment: where one holds more than
+      // kLongestBin items (gates all equal, or float32 gates closer than 2^-8) the keys are sorted
+      // after all, which takes about as long as counting one of that length.
+      bool count_ok = S <= 65536;
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const uint32_t hi = bits[r] >> 16;
         if (tid < nact && tid * R + r < S) count_ok = count_ok && hi <= 0x3F80u && hi + kRankBins > 0x3F80u;
       }
-      if (__syncthreads_and(count_ok)) {
+      bool counted = __syncthreads_and(count_ok);
+      if (counted) {
         uint32_t* hist = reinterpret_cast<uint32_t*>(keys);      // items per bin, then the bins' cursors
         uint32_t* start = hist + kRankBins;                      // first rank of each bin
-        uint32_t* seg = start + kRankBins;                       // S items, bin by bin
+        uint32_t* seg = start + kRankBins;                       // S keys, bin by bin
         for (int i = tid; i < kRankBins; i += kRouteThreads) hist[i] = 0u;
         __syncthreads();
         int bin[R];
@@ -225,7 +229,7 @@ __device__ __forceinline__ void route_assign_group(
           }
           __shared__ uint32_t wave_total[kRouteThreads / 64];
           if (lane == 63) wave_total[wave] = incl;
-          __syncthreads();
+          counted = !__syncthreads_or(c > kLongestBin);
           uint32_t before = 0;
           for (int w = 0; w < wave; ++w) before += wave_total[w];
           start[tid] = before + incl - c;
@@ -234,21 +238,23 @@ __device__ __forceinline__ void route_assign_group(
         __syncthreads();
 #pragma unroll
         for (int r = 0; r < R; ++r)
-          if (tid < nact && tid * R + r < S) seg[atomicAdd(&hist[bin[r]], 1u)] = (uint32_t)(tid * R + r);
+          if (counted && tid < nact && tid * R + r < S) seg[atomicAdd(&hist[bin[r]], 1u)] = bin_key32(bits[r], tid * R + r);
         __syncthreads();
 #pragma unroll
         for (int r = 0; r < R; ++r) {
           const int item = tid * R + r;
-          if (tid < nact && item < S) {
-            const uint32_t first = start[bin[r]], end = hist[bin[r]];
+          if (counted && tid < nact && item < S) {
+            const uint32_t first = start[bin[r]], end = hist[bin[r]], mine = bin_key32(bits[r], item);
             uint32_t lower = 0;
             for (uint32_t q = first; q < end; q += 4)          // four reads in flight
 #pragma unroll
               for (uint32_t u = 0; u < 4; ++u)
-                lower += seg[min(q + u, end - 1)] < (uint32_t)item && q + u < end ? 1u : 0u;
+                lower += seg[min(q + u, end - 1)] < mine && q + u < end ? 1u : 0u;
             rank[item] = (int)(first + lower);
           }
         }
+      }
+      if (counted) {
       } else if (__syncthreads_and(narrow_ok)) {
         uint32_t key[R];
 #pragma unroll
@@ -396,14 +402,14 @@ struct TopItemsMetrics {
   int32_t* rows;           // (E,): G * C, or null
 };
 
-// Bins of the counting rank over every bfloat16 from 1 down to 0.
+// Bins of the counting rank: the high halves of the floats from 1 down to 0.
 constexpr int kGateBins = 16384;
 static_assert(kGateBins > 0x3F80 && kGateBins % (kRouteThreads * 4) == 0, "whole 16-byte pieces per thread");
 // Items of one gate that are counted rather than sorted: with 200 of them 8 x 1 568 x 32 takes 30 us
 // (18 without, 32 sorted behind the histogram), 4 x 8 191 x 8 takes 68 (32, 90).  All gates equal,
 // counted: 166 and 3 143 us.
 constexpr uint32_t kLongestSegment = 256;
-inline __host__ __device__ bool rank_by_counting(int SP, bool bf16) { return bf16 && SP >= 512; }
+inline __host__ __device__ bool rank_by_counting(int SP) { return SP >= 512; }
 
 template <typename T, int R>
 __global__ __launch_bounds__(kRouteThreads) void top_items_kernel(
@@ -454,15 +460,15 @@ __global__ __launch_bounds__(kRouteThreads) void top_items_kernel(
       bits[r] = (tid < nact && s < S) ? __builtin_bit_cast(uint32_t, Elt<T>::load(col + (size_t)s * E)) : 0u;
       countable = countable && bits[r] <= 0x3F800000u;       // 0 .. 1: not negative, not NaN
     }
-    // Gates of a bfloat16 softmax take at most 0x3F81 values: rank by histogram, prefix, scatter
+    // Gates of a softmax fall into 0x3F81 bins by their high halves: rank by histogram, prefix, scatter
     // into the bins' segments and a count inside the item's own segment (see route_assign_group),
-    // in place of 66 compare-exchange steps at 2 048 keys.  Below 512 keys clearing the bins costs
+    // in place of 66 compare-exchange steps at 2 048 keys (float32, 65 x 268 items x 16: 29 -> 23 us).  Below 512 keys clearing the bins costs
     // what the sort does.  The count is quadratic in a segment: a column of equal gates (a router kernel
     // of zeros, tokens that repeat, gates that vanish) takes the sort after all.
-    bool counted = rank_by_counting(SP, sizeof(T) == 2) && __syncthreads_and(countable);
+    bool counted = rank_by_counting(SP) && __syncthreads_and(countable);
     if (counted) {
       uint32_t* hist = reinterpret_cast<uint32_t*>(smem);    // items per bin, then the bins' cursors
-      uint32_t* seg = hist + kGateBins;                      // S items, bin by bin
+      uint32_t* seg = hist + kGateBins;                      // S keys, bin by bin
       constexpr int kPieces = kGateBins / kRouteThreads / 4; // 16-byte pieces of a thread's bins
       uint4* hist4 = reinterpret_cast<uint4*>(hist);
 #pragma unroll
@@ -504,7 +510,7 @@ __global__ __launch_bounds__(kRouteThreads) void top_items_kernel(
 #pragma unroll
       for (int r = 0; r < R; ++r)
         if (counted && tid < nact && tid * R + r < S)
-          seg[atomicAdd(&hist[0x3F80u - (bits[r] >> 16)], 1u)] = (uint32_t)(tid * R + r);
+          seg[atomicAdd(&hist[0x3F80u - (bits[r] >> 16)], 1u)] = bin_key32(bits[r], tid * R + r);
       __syncthreads();
       // A bin's cursor now stands at its end, which is where the next bin starts.
 #pragma unroll
@@ -512,12 +518,12 @@ __global__ __launch_bounds__(kRouteThreads) void top_items_kernel(
         const int s = tid * R + r;
         if (counted && tid < nact && s < S) {
           const uint32_t bin = 0x3F80u - (bits[r] >> 16);
-          const uint32_t first = bin > 0 ? hist[bin - 1] : 0u, end = hist[bin];
+          const uint32_t first = bin > 0 ? hist[bin - 1] : 0u, end = hist[bin], mine = bin_key32(bits[r], s);
           uint32_t lower = 0;
           for (uint32_t q = first; q < end; q += 4)          // four reads in flight
 #pragma unroll
             for (uint32_t u = 0; u < 4; ++u)
-              lower += seg[min(q + u, end - 1)] < (uint32_t)s && q + u < end ? 1u : 0u;
+              lower += seg[min(q + u, end - 1)] < mine && q + u < end ? 1u : 0u;
           emit((int)(first + lower), s);
         }
       }
@@ -860,7 +866,7 @@ static int launch_top_items(const VmoeTopItemsParams* p, const TopItemsMetrics& 
   const int R = keys_per_thread(SP);
   const T* gates = (const T*)p->gates;
   size_t lds = (size_t)SP * 8;
-  if (R > 0 && rank_by_counting(SP, sizeof(T) == 2)) {
+  if (R > 0 && rank_by_counting(SP)) {
     const size_t counting = ((size_t)kGateBins + p->S) * 4;
     if (counting > lds) lds = counting;
   }

@@ -51,6 +51,10 @@ VMOE_HD uint32_t bpr_key32(uint32_t gate_bits, int s) {
   return ((~orderable_bits(gate_bits)) & 0xffff0000u) | (uint32_t)s;
 }
 
+// Items whose gates (0 .. 1 and equal in their high 16 bits) share a bin of a counting rank, in the order of
+// bpr_key64: the larger low half first, equal gates by item (S <= 65536).
+VMOE_HD uint32_t bin_key32(uint32_t gate_bits, int s) { return (~gate_bits << 16) | (uint32_t)s; }
+
 // Choice k of the item with priority rank `rank` owns bit k*S + rank of its expert's
 // bitmap: K-major, so that every first choice precedes every second choice
 // (vmoe/moe.py:573-575).  The position of the choice in the expert's buffer -- the cumsum
