@@ -936,7 +936,7 @@ def test_expert_mlp_float32_split_tiles(K, monkeypatch, E, R, D, M):
   rest = [to_dev(a) for a in (w0, b0, w1, b1)]
   monkeypatch.setenv("VMOE_F32_GEMM", "plain")
   plain = off(K.expert_mlp(to_dev(x), *rest))
-  for tile in range(6):
+  for tile in range(7):
     monkeypatch.setenv("VMOE_F32_GEMM", f"tile{tile}")
     dense = K.expert_mlp(to_dev(x), *rest)
     assert off(dense) <= 1.05 * plain, (tile, off(dense), plain)
@@ -955,7 +955,7 @@ def test_expert_mlp_float32_split_tiles(K, monkeypatch, E, R, D, M):
       np.testing.assert_array_equal(to_np(got), to_np(ref))
 
 
-@pytest.mark.parametrize("tile", range(6))
+@pytest.mark.parametrize("tile", range(7))
 def test_expert_mlp_float32_split_tiles_infinities(K, monkeypatch, tile):
   """Infinite and NaN operands, and finite ones that round to infinity in bfloat16, give what float32
   multiplication gives (VMOE_F32_GEMM=plain): infinities of the same sign, NaN in the same places, the

@@ -363,20 +363,23 @@ int launch_gemm_f32_split_tile(const float* A, const float* B, const float* bias
   return launch_status();
 }
 
-// Tiles, with what a 32-wide step of k costs: `work` us of a CU's time per tile, `latency` us alone
-// on a CU (fitted to the eleven shapes above, every tile on both products).  A launch is taken to last
-// 6 + ceil(Kd / 32) x max(latency, work x tiles of the fullest CU) us, with R rows in every batch (the
-// counts are on the device; dense and ragged calls of one shape take the same tile and so the same
-// order of sums).  The tile taken is 5 % slower than the best one on average; the worst, a
-// second product whose batches are half empty, 41 us against 28 (49 on float32 MFMAs).
-struct SplitTile { int bm, bn; double work, latency; };
+// Tiles, with what they cost: a 32-wide step of k takes `work` us of a CU's time per tile, `latency` us alone on a
+// CU, a tile `fix` us besides.  A launch is taken to last 4 us plus the 4-norm of one tile's chain and the
+// fullest CU's work, with R rows in every batch (the counts are on the device; dense and ragged calls of
+// one shape take the same tile and so the same order of sums).  Tiles per CU count as halfway between
+// whole ones and even ones.  Fitted to 34 random shapes (1 - 37 experts, 26 - 7 001 rows, widths 256 - 4 096), every tile on both
+// products, rms 8 - 14 % per tile: the 68 products take 4 412 us on the tiles chosen, 4 327 on the
+// best of each, and 4 726 without the 96-row tile on constants fitted to eleven shapes (23 other shapes: 4 039, 3 877
+// and 4 154); the worst choice costs 23 %.
+struct SplitTile { int bm, bn; double work, latency, fix; };
 constexpr SplitTile kSplitTiles[] = {
-    {128, 128, 1.44, 1.55},    // two workgroups per CU
-    {64, 128, 0.73, 1.08},     // four
-    {64, 128, 0.79, 0.76},     // two groups of waves along k
-    {32, 128, 0.49, 0.78},
-    {32, 128, 0.52, 0.50},     // two groups
-    {32, 64, 0.32, 0.31},      // two groups
+    {128, 128, 1.09, 1.61, 2.7},   // two workgroups per CU
+    {64, 128, 0.59, 1.14, 2.0},    // four
+    {64, 128, 0.60, 0.84, 2.9},    // two groups of waves along k
+    {32, 128, 0.42, 0.88, 1.0},
+    {32, 128, 0.42, 0.57, 1.6},    // two groups
+    {32, 64, 0.25, 0.29, 1.0},     // two groups
+    {96, 128, 0.77, 1.39, 3.7},    // two workgroups per CU
 };
 constexpr int kNumSplitTiles = sizeof(kSplitTiles) / sizeof(kSplitTiles[0]);
 
@@ -386,8 +389,9 @@ inline int best_split_tile(int batch, int R, int N, int Kd) {
   for (int i = 0; i < kNumSplitTiles; ++i) {
     const SplitTile& t = kSplitTiles[i];
     const double per_cu = (double)batch * ((R + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) / (kCusPerXcd * kNumXcd);
-    // a few tiles per CU come in whole ones, many even out over the launch
-    const double us = 6 + (double)((Kd + 31) / 32) * std::max(t.latency, t.work * (per_cu < 4 ? std::ceil(per_cu) : per_cu + 0.5));
+    const double tiles = std::max(1.0, 0.5 * (std::ceil(per_cu) + per_cu + 0.3)), steps = (Kd + 31) / 32;
+    const double chain = steps * t.latency, busy = tiles * (steps * t.work + t.fix);
+    const double us = chain * chain * chain * chain + busy * busy * busy * busy;
     if (us < best_us) { best_us = us; best = i; }
   }
   return best;
@@ -406,7 +410,8 @@ int launch_gemm_f32_split(int tile, const float* A, const float* B, const float*
     case 2: return run(SplitCfg<64, 128, 2, 2, 32, 2, 2>{});
     case 3: return run(SplitCfg<32, 128, 1, 4, 32, 4, 1>{});
     case 4: return run(SplitCfg<32, 128, 1, 4, 32, 2, 2>{});
-    default: return run(SplitCfg<32, 64, 2, 2, 64, 2, 2>{});
+    case 5: return run(SplitCfg<32, 64, 2, 2, 64, 2, 2>{});
+    default: return run(SplitCfg<96, 128, 2, 2, 32, 2, 1>{});
   }
 }
 
