@@ -227,23 +227,33 @@ __device__ __forceinline__ void route_assign_group(
             const uint32_t o = __shfl_up(incl, d, kWave);
             if (lane >= d) incl += o;
           }
+          // A wave that saw a long bin says so in the top bit of its total (S is below it): a reduction over the
+          // workgroup (__syncthreads_or) in place of this barrier made 32 x 1 568 items x 2 of 32 16.0 us in place of 14.5.
           __shared__ uint32_t wave_total[kRouteThreads / 64];
-          if (lane == 63) wave_total[wave] = incl;
-          counted = !__syncthreads_or(c > kLongestBin);
-          uint32_t before = 0;
-          for (int w = 0; w < wave; ++w) before += wave_total[w];
+          const uint32_t long_bin = __any(c > kLongestBin) ? 0x80000000u : 0u;
+          if (lane == 63) wave_total[wave] = incl | long_bin;
+          __syncthreads();
+          uint32_t before = 0, seen = 0;
+#pragma unroll
+          for (int w = 0; w < kRouteThreads / 64; ++w) {
+            const uint32_t total = wave_total[w];
+            seen |= total;
+            before += w < wave ? total & 0x7fffffffu : 0u;
+          }
+          counted = (__builtin_amdgcn_readfirstlane((int)seen) & 0x80000000) == 0;
           start[tid] = before + incl - c;
           hist[tid] = before + incl - c;                       // cursor of the scatter
         }
         __syncthreads();
+        if (counted) {
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-          if (counted && tid < nact && tid * R + r < S) seg[atomicAdd(&hist[bin[r]], 1u)] = bin_key32(bits[r], tid * R + r);
-        __syncthreads();
+          for (int r = 0; r < R; ++r)
+            if (tid < nact && tid * R + r < S) seg[atomicAdd(&hist[bin[r]], 1u)] = bin_key32(bits[r], tid * R + r);
+          __syncthreads();
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const int item = tid * R + r;
-          if (counted && tid < nact && item < S) {
+          for (int r = 0; r < R; ++r) {
+            const int item = tid * R + r;
+            if (tid >= nact || item >= S) continue;
             const uint32_t first = start[bin[r]], end = hist[bin[r]], mine = bin_key32(bits[r], item);
             uint32_t lower = 0;
             for (uint32_t q = first; q < end; q += 4)          // four reads in flight
