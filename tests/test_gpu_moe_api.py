@@ -1065,11 +1065,11 @@ def test_dispatch_combine_gradients(moe, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("T,K_,D,NS", [(1, 1, 8, 1), (37, 2, 520, 60), (130, 3, 64, 500), (50, 4, 1032, 190), (33, 5, 16, 170)])
+@pytest.mark.parametrize("T,K_,D,NS", [(1, 1, 8, 1), (37, 2, 520, 60), (130, 3, 64, 500), (50, 4, 1032, 190), (33, 5, 16, 170), (9, 300, 16, 700)])
 def test_combine_backward_is_both_gradients(moe, dtype, T, K_, D, NS):
   """One launch (up to four choices, two beyond) against the launch per gradient, bit for bit: dropped
   choices, unclaimed slots with and without their zeros, rows of a chunk and of several rounds; and
-  dispatch's gradient against combine with ones."""
+  dispatch's gradient against combine with ones (its form for many choices too)."""
   from vmoe_amd import kernels as K
   gen = torch.Generator().manual_seed(T + K_)
   mk = lambda *s: torch.randn(s, generator=gen).to(dtype).cuda()
