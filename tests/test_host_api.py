@@ -253,6 +253,20 @@ def test_entry_points_refuse_tensors_of_the_wrong_shape(monkeypatch, name, args)
     getattr(kernels, name)(**args)
 
 
+@pytest.mark.parametrize("name", ["combine_backward", "combine_backward_weights"])
+@pytest.mark.parametrize("types", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("timed", [False, True])
+def test_gradients_of_combine_refuse_rows_of_another_type(monkeypatch, name, types, timed):
+  """The kernels read y with the width of dout's type: bfloat16 rows under a float32 gradient would be
+  read past their end."""
+  monkeypatch.setattr(_hip, "raw_stream", lambda: 0)
+  monkeypatch.setattr(_hip, "timed", lambda call: timed)
+  slots = torch.zeros((6, 2), dtype=torch.int32)
+  more = (torch.zeros((6, 2)), None) if name == "combine_backward" else ()
+  with pytest.raises(TypeError, match="dout"):
+    getattr(kernels, name)(torch.zeros((6, 8), dtype=types[0]), torch.zeros((9, 8), dtype=types[1]), slots, *more)
+
+
 @pytest.mark.parametrize("dtype", [_hip.F32, _hip.BF16])
 @pytest.mark.parametrize("D", [8, 40, 144])
 def test_gathered_rows_of_broken_k_tiles_are_refused(dtype, D):

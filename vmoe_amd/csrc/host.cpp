@@ -9,8 +9,8 @@
 //
 // Every function takes the raw stream first and raises vmoe_amd._hip.VmoeError on an error code, a
 // tensor that is not on the GPU or one that is not contiguous, and ValueError on a tensor with
-// another number of axes than its wrapper names or fewer values than the call would read or write:
-// the C ABI sees addresses and sizes only.  Nothing is kept between calls.
+// another number of axes than its wrapper names or fewer values than the call would read or write
+// (TypeError on rows of another type): the C ABI sees addresses and sizes only.  Nothing is kept between calls.
 #include <torch/extension.h>
 
 #include <optional>
@@ -67,6 +67,12 @@ void need_values(const Tensor& t, int64_t least, const char* name) {
 }
 void need_values(const OptTensor& t, int64_t least, const char* name) {
   if (t.has_value()) need_values(*t, least, name);
+}
+// Two operands that a kernel reads as one type.
+void need_type_of(const Tensor& t, const Tensor& like, const char* name, const char* like_name) {
+  if (t.scalar_type() != like.scalar_type())
+    throw py::type_error(std::string(name) + " is " + at::toString(t.scalar_type()) + ", " + like_name + " " +
+                         at::toString(like.scalar_type()));
 }
 // Stacked weights (at least E, rows, cols).
 void need_stack(const OptTensor& t, int64_t E, int64_t rows, int64_t cols, const char* name) {
@@ -428,6 +434,7 @@ Tensor combine_backward_weights(int64_t stream, const Tensor& dout_, const Tenso
   const Tensor dout = dout_.contiguous(), y = y_.contiguous();
   need_values(token_slot, dout.size(0) * token_slot.size(-1), "token_slot");
   need_values(y, y.size(0) * dout.size(1), "y");
+  need_type_of(y, dout, "y", "dout");
   Tensor dw = f32({dout.size(0), token_slot.size(-1)}, dout);
   VmoeCombineBackwardParams p{};
   p.dout = ptr(dout); p.y = ptr(y); p.token_slot = ptr_as<int32_t>(token_slot); p.dweights = ptr_as<float>(dw);
@@ -448,6 +455,7 @@ std::tuple<Tensor, Tensor> combine_backward(int64_t stream, const Tensor& dout_,
   need_values(weights, dout.size(0) * token_slot.size(-1), "weights");
   need_values(slot_token, y.size(0), "slot_token");
   need_values(y, y.size(0) * dout.size(1), "y");
+  need_type_of(y, dout, "y", "dout");
   Tensor dy = empty({y.size(0), dout.size(1)}, dout.scalar_type(), dout);
   Tensor dw = f32({dout.size(0), token_slot.size(-1)}, dout);
   VmoeCombineBackwardParams p{};

@@ -277,6 +277,8 @@ def combine_backward_weights(dout: torch.Tensor, y: torch.Tensor,
     return H.host().combine_backward_weights(H.raw_stream(), dout, y, token_slot)
   T, D = dout.shape
   Kk = token_slot.shape[-1]
+  if y.dtype != dout.dtype:
+    raise TypeError(f"y is {y.dtype}, dout {dout.dtype}")
   dout, y = dout.contiguous(), y.contiguous()
   dw = _f32(T, Kk, device=dout.device)
   p = H.CombineBackwardParams(H.ptr(dout), H.ptr(y), H.ptr(token_slot), None, None, None,
@@ -292,6 +294,8 @@ def combine_backward(dout: torch.Tensor, y: torch.Tensor, token_slot: torch.Tens
     return H.host().combine_backward(H.raw_stream(), dout, y, token_slot, weights, slot_token)
   T, D = dout.shape
   Kk = token_slot.shape[-1]
+  if y.dtype != dout.dtype:
+    raise TypeError(f"y is {y.dtype}, dout {dout.dtype}")
   dout, y = dout.contiguous(), y.contiguous()
   weights = weights.to(torch.float32).contiguous()
   dy = torch.empty((y.shape[0], D), dtype=dout.dtype, device=dout.device)
