@@ -275,6 +275,22 @@ def test_gathered_rows_of_broken_k_tiles_are_refused(dtype, D):
   assert _hip.lib().vmoe_expert_mlp(_hip.ctypes.byref(p), None) == kernels._E_UNSUPPORTED
 
 
+@pytest.mark.parametrize("name", ["vmoe_combine_backward", "vmoe_combine_backward_data", "vmoe_combine_backward_weights",
+                                  "vmoe_dispatch", "vmoe_combine", "vmoe_dispatch_backward"])
+def test_row_movers_refuse_more_rows_than_a_launch_has_waves(name):
+  """A wave per row: 2^32 - 1 threads are 2^26 - 1 rows.  (Rows and slots of eight bfloat16 values; dispatch and
+  combine take such a kernel where the rows are too wide for their others.)"""
+  n, D = (1 << 26, 8) if "backward" in name and name != "vmoe_dispatch_backward" else (1 << 26, 1 << 17)
+  if name == "vmoe_dispatch":
+    p = _hip.DispatchParams(16, 16, 16, 16, n // 2, n // 2 + 1, 2, D, _hip.BF16)
+  elif "backward_" in name or name == "vmoe_combine_backward":
+    slots = 8 if name.endswith("weights") else n // 2 + 1
+    p = _hip.CombineBackwardParams(16, 16, 16, 16, 16, 16, 16, n + 1 - slots if slots > 8 else n, slots, 2, D, _hip.BF16)
+  else:
+    p = _hip.CombineParams(16, 16, 16, 16, n, 8, 2, D, _hip.BF16)
+  assert getattr(_hip.lib(), name)(_hip.ctypes.byref(p), None) == -5      # VMOE_E_OVERFLOW
+
+
 def test_dispatch_needs_a_number_of_slots(monkeypatch):
   monkeypatch.setattr(_hip, "raw_stream", lambda: 0)
   with pytest.raises(TypeError):

@@ -26,6 +26,13 @@ constexpr int kListedK = 256;      // combine: the same
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
+// Index of the wave in its launch.  (A thread's index would need 33 bits beyond 2^26 waves; a launch holds
+// 2^32 - 1 threads, which the entry points check.)
+constexpr long long kMaxMoveBlocks = 0xffffffffLL / kMoveThreads;
+__device__ __forceinline__ int wave_of_launch() {
+  return __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kMoveThreads / kWave) + (threadIdx.x / kWave)));
+}
+
 // Streaming accesses: every row is touched once per kernel, so loads and stores
 // carry the non-temporal hint.
 __device__ __forceinline__ uint4 load_stream(const uint4* p) {
@@ -93,8 +100,7 @@ __global__ __launch_bounds__(kMoveThreads) void dispatch_generic_kernel(
     const int32_t* __restrict__ slot_token, uint4* __restrict__ out, int num_items, int num_slots,
     int K, int cpr, int item_waves) {
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(
-      (int)((blockIdx.x * (unsigned)kMoveThreads + threadIdx.x) >> 6));
+  const int wave = wave_of_launch();
   if (wave < item_waves) {
     for (int ch = lane; ch < cpr; ch += kWave) {
       const uint4 v = x[(size_t)wave * cpr + ch];
@@ -266,8 +272,7 @@ __global__ __launch_bounds__(kMoveThreads) void combine_generic_kernel(
     int K, int cpr) {
   constexpr int N = Chunk<T>::n;
   const int lane = threadIdx.x & 63;
-  const int t = __builtin_amdgcn_readfirstlane(
-      (int)((blockIdx.x * (unsigned)kMoveThreads + threadIdx.x) >> 6));
+  const int t = wave_of_launch();
   if (t >= num_items) return;
   for (int ch = lane; ch < cpr; ch += kWave) {
     float acc[N];
@@ -341,8 +346,7 @@ __global__ __launch_bounds__(kMoveThreads) void scatter_scaled_kernel(
     uint4* __restrict__ out, int num_items, int num_slots, int K, int cpr, int item_waves) {
   constexpr int N = Chunk<T>::n;
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(
-      (int)((blockIdx.x * (unsigned)kMoveThreads + threadIdx.x) >> 6));
+  const int wave = wave_of_launch();
   if (wave < item_waves) {
     for (int ch = lane; ch < cpr; ch += kWave) {
       float a[N];
@@ -371,8 +375,7 @@ __global__ __launch_bounds__(kMoveThreads) void row_dots_kernel(
     int K, int cpr) {
   constexpr int N = Chunk<T>::n;
   const int lane = threadIdx.x & 63;
-  const int t = __builtin_amdgcn_readfirstlane(
-      (int)((blockIdx.x * (unsigned)kMoveThreads + threadIdx.x) >> 6));
+  const int t = wave_of_launch();
   if (t >= num_items) return;
   for (int k = 0; k < K; ++k) {
     const int slot = checked_slot(token_slot[(size_t)t * K + k], num_slots);
@@ -404,8 +407,7 @@ __global__ __launch_bounds__(kMoveThreads) void combine_backward_kernel(
     float* __restrict__ dw, int num_items, int num_slots, int K, int cpr) {
   constexpr int N = Chunk<T>::n;
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(
-      (int)((blockIdx.x * (unsigned)kMoveThreads + threadIdx.x) >> 6));
+  const int wave = wave_of_launch();
   if (wave >= num_items) {
     const int s = wave - num_items;
     if (slot_token != nullptr && s < num_slots && slot_token[s] < 0)
@@ -486,7 +488,7 @@ extern "C" int vmoe_dispatch(const VmoeDispatchParams* p, vmoe_stream_t stream) 
   } else {
     const long long waves = (long long)p->num_items + (zero_fill ? p->num_slots : 0);
     const long long blocks = (waves + 3) / 4;
-    if (blocks > 0x7fffffffLL) return VMOE_E_OVERFLOW;
+    if (blocks > kMaxMoveBlocks) return VMOE_E_OVERFLOW;
     hipLaunchKernelGGL(dispatch_generic_kernel, dim3((unsigned)blocks), dim3(kMoveThreads), 0,
                        as_stream(stream), (const uint4*)p->x, p->token_slot, p->slot_token,
                        (uint4*)p->out, p->num_items, p->num_slots, p->K, cpr, p->num_items);
@@ -505,6 +507,7 @@ static int run_combine_form(const VmoeCombineParams* p, int cpr, vmoe_stream_t s
                        p->token_slot, p->weights, (uint4*)p->out, p->num_items, p->num_slots, p->K, cpr,
                        chunk_magic(cpr));
   } else {
+    if ((p->num_items + 3LL) / 4 > kMaxMoveBlocks) return VMOE_E_OVERFLOW;
     auto kern = combine_generic_kernel<T, UNIT>;
     hipLaunchKernelGGL(kern, dim3((p->num_items + 3) / 4), dim3(kMoveThreads), 0, as_stream(stream),
                        (const uint4*)p->y, p->token_slot, p->weights, (uint4*)p->out, p->num_items,
@@ -567,7 +570,7 @@ extern "C" int vmoe_combine_backward_data(const VmoeCombineBackwardParams* p, vm
   const int cpr = (int)((size_t)p->D * (p->dtype == VMOE_BF16 ? 2 : 4) / 16);
   const long long waves = (long long)p->num_items + (p->slot_token != nullptr ? p->num_slots : 0);
   const long long blocks = (waves + 3) / 4;
-  if (blocks > 0x7fffffffLL) return VMOE_E_OVERFLOW;
+  if (blocks > kMaxMoveBlocks) return VMOE_E_OVERFLOW;
   if (p->dtype == VMOE_BF16)
     hipLaunchKernelGGL(scatter_scaled_kernel<bf16_t>, dim3((unsigned)blocks), dim3(kMoveThreads), 0,
                        as_stream(stream), (const uint4*)p->dout, p->token_slot, p->weights,
@@ -587,13 +590,14 @@ extern "C" int vmoe_combine_backward_weights(const VmoeCombineBackwardParams* p,
   int rc = check_move(p->dout, p->token_slot, p->y, p->num_items, p->num_slots, p->K, p->D, p->dtype);
   if (rc != VMOE_OK) return rc;
   const int cpr = (int)((size_t)p->D * (p->dtype == VMOE_BF16 ? 2 : 4) / 16);
-  const int blocks = (p->num_items + 3) / 4;
+  const long long blocks = (p->num_items + 3LL) / 4;
+  if (blocks > kMaxMoveBlocks) return VMOE_E_OVERFLOW;
   if (p->dtype == VMOE_BF16)
-    hipLaunchKernelGGL(row_dots_kernel<bf16_t>, dim3(blocks), dim3(kMoveThreads), 0,
+    hipLaunchKernelGGL(row_dots_kernel<bf16_t>, dim3((unsigned)blocks), dim3(kMoveThreads), 0,
                        as_stream(stream), (const uint4*)p->dout, (const uint4*)p->y, p->token_slot,
                        p->dweights, p->num_items, p->num_slots, p->K, cpr);
   else
-    hipLaunchKernelGGL(row_dots_kernel<float>, dim3(blocks), dim3(kMoveThreads), 0,
+    hipLaunchKernelGGL(row_dots_kernel<float>, dim3((unsigned)blocks), dim3(kMoveThreads), 0,
                        as_stream(stream), (const uint4*)p->dout, (const uint4*)p->y, p->token_slot,
                        p->dweights, p->num_items, p->num_slots, p->K, cpr);
   return launch_status();
@@ -602,9 +606,8 @@ extern "C" int vmoe_combine_backward_weights(const VmoeCombineBackwardParams* p,
 extern "C" int vmoe_combine_backward(const VmoeCombineBackwardParams* p, vmoe_stream_t stream) {
   if (p == nullptr || p->weights == nullptr || p->dy == nullptr || p->y == nullptr || p->dweights == nullptr)
     return VMOE_E_NULL;
-  const long long waves = (long long)p->num_items + (p->slot_token != nullptr ? p->num_slots : 0);
-  // More choices (experts choice: K = E) or more waves than an int numbers: one gradient after the other.
-  if (p->K > kBackwardK || waves >= INT32_MAX) {
+  // More choices (experts choice: K = E): one gradient after the other.
+  if (p->K > kBackwardK) {
     const int rc = vmoe_combine_backward_data(p, stream);
     return rc != VMOE_OK ? rc : vmoe_combine_backward_weights(p, stream);
   }
@@ -612,8 +615,11 @@ extern "C" int vmoe_combine_backward(const VmoeCombineBackwardParams* p, vmoe_st
   if (rc != VMOE_OK) return rc;
   if (!aligned16(p->y)) return VMOE_E_ALIGN;
   const int cpr = (int)((size_t)p->D * (p->dtype == VMOE_BF16 ? 2 : 4) / 16);
+  const long long waves = (long long)p->num_items + (p->slot_token != nullptr ? p->num_slots : 0);
+  const long long blocks = (waves + 3) / 4;
+  if (blocks > kMaxMoveBlocks) return VMOE_E_OVERFLOW;
   auto kern = p->dtype == VMOE_BF16 ? combine_backward_kernel<bf16_t> : combine_backward_kernel<float>;
-  hipLaunchKernelGGL(kern, dim3((unsigned)((waves + 3) / 4)), dim3(kMoveThreads), 0, as_stream(stream),
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kMoveThreads), 0, as_stream(stream),
                      (const uint4*)p->dout, (const uint4*)p->y, p->token_slot, p->weights, p->slot_token,
                      (uint4*)p->dy, p->dweights, p->num_items, p->num_slots, p->K, cpr);
   return launch_status();
