@@ -956,6 +956,21 @@ def test_expert_mlp_float32_split_tiles(K, monkeypatch, E, R, D, M):
 
 
 @pytest.mark.parametrize("tile", range(7))
+def test_expert_mlp_float32_weights_at_any_address(K, monkeypatch, tile):
+  """Weights one, two and three floats past a 16-byte boundary: the bits of aligned ones."""
+  monkeypatch.setenv("VMOE_F32_GEMM", f"tile{tile}")
+  E, R, D, M = 3, 70, 100, 132
+  gen = torch.Generator().manual_seed(tile)
+  mk = lambda *s: torch.randn(s, generator=gen).to(dev())
+  x, w0, b0, w1, b1 = mk(E, R, D), mk(E, D, M), mk(E, M), mk(E, M, D), mk(E, D)
+  want = K.expert_mlp(x, w0, b0, w1, b1)
+  for shift in (1, 2, 3):
+    moved = [torch.empty(w.numel() + shift, device=dev())[shift:].view(w.shape).copy_(w) for w in (w0, b0, w1, b1)]
+    assert all(w.data_ptr() % 16 == 4 * shift for w in moved)
+    assert torch.equal(K.expert_mlp(x, *moved), want)
+
+
+@pytest.mark.parametrize("tile", range(7))
 def test_expert_mlp_float32_split_tiles_infinities(K, monkeypatch, tile):
   """Infinite and NaN operands, and finite ones that round to infinity in bfloat16, give what float32
   multiplication gives (VMOE_F32_GEMM=plain): infinities of the same sign, NaN in the same places, the

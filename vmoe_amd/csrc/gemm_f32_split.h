@@ -41,6 +41,7 @@
 namespace vmoe {
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef f32x4_t f32x4_any_t __attribute__((aligned(4)));    // weights come at any float address
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
 template <int BM_, int BN_, int WM_, int WN_, int BK_, int WGS_, int KG_>
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(Cfg::kThreads, Cfg::kWgs * Cfg::kThreads / 256) voi
       for (int j = 0; j < 4; ++j) {
         int k = k0 + b_kq[i] * 4 + j;
         if (tail) k = min(k, Kd - 1);
-        rb[i][j] = *reinterpret_cast<const f32x4_t*>(Bb + (size_t)k * N + n);
+        rb[i][j] = *reinterpret_cast<const f32x4_any_t*>(Bb + (size_t)k * N + n);
       }
     }
   };
@@ -326,7 +327,7 @@ __global__ __launch_bounds__(Cfg::kThreads, Cfg::kWgs * Cfg::kThreads / 256) voi
           }
           f32x4_t s4 = {0.f, 0.f, 0.f, 0.f};
           for (int k = 0; k < Kd; ++k) {
-            const f32x4_t bk = *reinterpret_cast<const f32x4_t*>(Bb + (size_t)k * N + ocol);
+            const f32x4_t bk = *reinterpret_cast<const f32x4_any_t*>(Bb + (size_t)k * N + ocol);
             const float av = ap[k];
 #pragma unroll
             for (int t = 0; t < 4; ++t) s4[t] = fmaf(av, bk[t], s4[t]);
