@@ -220,6 +220,47 @@ def test_gate_topk_float32_any_expert_count(K, n, D, E, k, aligned):
       np.testing.assert_array_equal(to_np(a), to_np(e))
 
 
+@pytest.mark.parametrize("n,D,E", [(45, 260, 7), (8200, 64, 16), (16400, 36, 5), (33000, 32, 32), (70, 516, 40),
+                                   (33000, 64, 33), (50, 100, 100), (33000, 36, 128)])
+@pytest.mark.parametrize("bias", [None, "finite", "infinite"])
+def test_gate_topk_float32_infinities(K, n, D, E, bias):
+  """Infinite and NaN items, an infinite router column and values that round to infinity in bfloat16 give the
+  logits of float32 multiplication, at every number of tiles per workgroup; the other items' are bit for bit what
+  they are without them.  A bias of -inf takes its expert out."""
+  rng = np.random.default_rng(n + E)
+  x = rng.standard_normal((1, n, D)).astype(np.float32)
+  w = (rng.standard_normal((D, E)) / np.sqrt(D)).astype(np.float32)
+  b = rng.standard_normal(E).astype(np.float32)
+  if bias == "infinite":
+    b[E // 2] = -np.inf
+  b = None if bias is None else b
+  run = lambda x, w: K.gate_topk(to_dev(x), to_dev(w), 1, logit_bias=None if b is None else to_dev(b), return_logits=True)
+  clean = to_np(run(x, w)[3])[0]
+  odd, rows = x.copy(), [0, 3, n // 2, n - 1]
+  odd[0, 0, 0], odd[0, 3, D - 1], odd[0, n // 2, 1], odd[0, n - 1, 2] = np.inf, -np.inf, np.nan, 3.4e38
+  with np.errstate(over="ignore", invalid="ignore"):
+    want = odd[0, rows].astype(np.float64) @ w.astype(np.float64) + (0 if b is None else b)
+  want = np.where(np.abs(want) > np.finfo(np.float32).max, np.sign(want) * np.inf, want)
+  gates, _, _, logits = (to_np(t) for t in run(odd, w))
+  got = logits[0, rows]
+  np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+  np.testing.assert_array_equal(np.where(np.isinf(got), got, 0), np.where(np.isinf(want), want, 0))
+  np.testing.assert_allclose(got[np.isfinite(want)], want[np.isfinite(want)], rtol=1e-5)
+  same = np.ones(n, bool)
+  same[rows] = False
+  np.testing.assert_array_equal(logits[0, same], clean[same])
+  assert np.isfinite(gates[0, same]).all() and (bias != "infinite" or (gates[0, same, E // 2] == 0).all())
+  # A router column of infinities: its logits are infinite, the others untouched.
+  if E > 1 and bias != "infinite":
+    column = w.copy()
+    column[D // 2, E - 1] = -np.inf
+    gates, _, _, logits = (to_np(t)[0] for t in run(x, column))
+    np.testing.assert_array_equal(logits[:, E - 1], np.where(x[0, :, D // 2] > 0, -np.inf, np.inf))
+    np.testing.assert_array_equal(logits[:, :-1], clean[:, :-1])
+    out = x[0, :, D // 2] > 0
+    assert (gates[out, E - 1] == 0).all() and np.isfinite(gates[out]).all()
+
+
 def test_gate_topk_streaming_and_direct_loads_agree(K, monkeypatch):
   """The two forms of the bfloat16 gating kernel (item rows through LDS by DMA, or by direct
   loads: VMOE_GATE_DIRECT_LOADS=1) add the same products in a different order of k: equal

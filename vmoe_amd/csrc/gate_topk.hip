@@ -69,12 +69,11 @@ __device__ __forceinline__ uint64_t half_wave_max_u64(uint64_t v) {
 
 // Softmax and top-K of one item by two lanes: g holds the logits of experts h * EP / 2 ..., lane ^ 32 the
 // others.  Sums and maxima are serial per lane; the halves meet with one xor-32 shuffle each.
-template <typename T, int EP>
-__device__ __forceinline__ void finish_row(float (&g)[EP / 2], T* __restrict__ gates, float* __restrict__ topk_val, int32_t* __restrict__ topk_idx,
-                                           int row, int num_items, int E, int K, int h) {
+// Logits -> exponentials; returns their sum.
+template <int EP>
+__device__ __forceinline__ float exponentials(float (&g)[EP / 2], int E, int h) {
   constexpr int CNT = EP / 2;
   const int n0 = h * CNT;
-  const bool row_ok = row < num_items;
   float mx = -INFINITY;
 #pragma unroll
   for (int j = 0; j < CNT; ++j) {
@@ -88,7 +87,15 @@ __device__ __forceinline__ void finish_row(float (&g)[EP / 2], T* __restrict__ g
     g[j] = (n0 + j < E) ? expf(g[j] - mx) : 0.f;
     sum += g[j];
   }
-  sum += __shfl_xor(sum, 32, kWave);
+  return sum + __shfl_xor(sum, 32, kWave);
+}
+// Exponentials and their sum -> gates and top-K.
+template <typename T, int EP>
+__device__ __forceinline__ void finish_exponentials(float (&g)[EP / 2], float sum, T* __restrict__ gates, float* __restrict__ topk_val,
+                                                    int32_t* __restrict__ topk_idx, int row, int num_items, int E, int K, int h) {
+  constexpr int CNT = EP / 2;
+  const int n0 = h * CNT;
+  const bool row_ok = row < num_items;
 #pragma unroll
   for (int j = 0; j < CNT; ++j) g[j] = Elt<T>::round(g[j] / sum);
   if (gates != nullptr && row_ok) {
@@ -135,6 +142,13 @@ __device__ __forceinline__ void finish_row(float (&g)[EP / 2], T* __restrict__ g
       topk_idx[(size_t)row * K + kk] = n_star;
     }
   }
+}
+
+template <typename T, int EP>
+__device__ __forceinline__ void finish_row(float (&g)[EP / 2], T* __restrict__ gates, float* __restrict__ topk_val, int32_t* __restrict__ topk_idx,
+                                           int row, int num_items, int E, int K, int h) {
+  const float sum = exponentials<EP>(g, E, h);
+  finish_exponentials<T, EP>(g, sum, gates, topk_val, topk_idx, row, num_items, E, K, h);
 }
 
 // The logits output of a tile of finished logits in LDS (row pitch `pitch`), by one wave.
@@ -457,6 +471,58 @@ __device__ __forceinline__ void split3_cut(float v0, float v1, uint32_t& hi, uin
   lo = pack_bf16x2(r0 - bf_lo(mid), r1 - bf_hi(mid));
 }
 
+// The infinite and NaN logits of a tile (32 rows of pitch EP + 1 in LDS; xrow: the lane's row) again, on float32
+// MFMAs, by one wave: an operand that is infinite or rounds to infinity leaves NaN in the sums of its pieces'
+// products, which the softmax's sum shows.  (A call of its own: inline, its registers cost every launch 0.4 to 2 us.
+// 196 x 768 x 8, nothing but NaN: 35 us; the check costs 0.2 us of the 12.)
+template <int NT>
+__device__ __noinline__ void retake_logits(const float* __restrict__ xrow, const float* __restrict__ w,
+                                              const float* __restrict__ bias, float* st, int D, int E, int lane) {
+  const int m = lane & 31, h = lane >> 5;
+  floatx16 acc[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[nt][i] = 0.f;
+  constexpr int kSteps = NT == 4 ? 2 : 4;         // of eight k; their loads are in flight together
+#pragma unroll 1
+  for (int k0 = 0; k0 < D; k0 += 8 * kSteps) {
+    float4 x4[kSteps];
+    float b[kSteps][4][NT];
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {            // lanes 0 - 31 take the first four k of a step, 32 - 63 the others
+      const int k = k0 + s * 8 + h * 4;
+      x4[s] = *reinterpret_cast<const float4*>(xrow + min(k, D - 4));
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) b[s][t][nt] = w[(size_t)min(k + t, D - 1) * E + min(nt * 32 + m, E - 1)];
+    }
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+      const bool in = k0 + s * 8 + h * 4 < D;
+      const float v[4] = {x4[s].x, x4[s].y, x4[s].z, x4[s].w};
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+          acc[nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? v[t] : 0.f, in ? b[s][t][nt] : 0.f, acc[nt], 0, 0, 0);
+    }
+  }
+  mfma_result_fence();
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    const int n = nt * 32 + m;
+    const float bn = bias != nullptr ? bias[min(n, E - 1)] : 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float* const at = st + ((i >> 2) * 8 + h * 4 + (i & 3)) * (NT * 32 + 1) + n;
+      if (!(*at - *at == 0.f)) *at = acc[nt][i] + bn;
+    }
+  }
+  wait_lgkmcnt0();
+}
+
 constexpr int kNumCus = 256;
 
 template <int NT, int WAVES, int TW>
@@ -566,9 +632,11 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_f32_kernel(
     }
     __syncthreads();                              // W's LDS takes the logits
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
+    for (int nt = 0; nt < NT; ++nt) {
+      const float bn = KS == 1 && bias != nullptr ? bias[min(nt * 32 + m, E - 1)] : -0.f;       // (x + -0 is x)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) st[((i >> 2) * 8 + h * 4 + (i & 3)) * (EP + 1) + nt * 32 + m] = acc[nt][i];
+      for (int i = 0; i < 16; ++i) st[((i >> 2) * 8 + h * 4 + (i & 3)) * (EP + 1) + nt * 32 + m] = acc[nt][i] + bn;
+    }
     __syncthreads();
     if constexpr (KS > 1) {
       for (int e = tid; e < TW * 32 * EP; e += kThreads) {
@@ -585,21 +653,19 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_f32_kernel(
     if (part == 0 && tile < num_tiles) {
       constexpr int CNT = EP / 2;
       float g[CNT];
+      auto read = [&]() {
 #pragma unroll
-      for (int j = 0; j < CNT; ++j) {
-        const int n = h * CNT + j;
-        g[j] = st[m * (EP + 1) + n];
-        if (KS == 1 && bias != nullptr) g[j] += bias[min(n, E - 1)];
+        for (int j = 0; j < CNT; ++j) g[j] = st[m * (EP + 1) + h * CNT + j];
+      };
+      read();
+      float sum = exponentials<EP>(g, E, h);
+      if (__builtin_expect(__any(!(sum < INFINITY)), 0)) {
+        retake_logits<NT>(xrow, w, bias, st, D, E, lane);
+        read();
+        sum = exponentials<EP>(g, E, h);
       }
-      if (logits != nullptr) {
-        if (KS == 1 && bias != nullptr) {
-#pragma unroll
-          for (int j = 0; j < CNT; ++j) st[m * (EP + 1) + h * CNT + j] = g[j];
-          wait_lgkmcnt0();
-        }
-        store_logits(st, EP + 1, logits, row0, num_items, E, lane);
-      }
-      finish_row<float, EP>(g, gates, topk_val, topk_idx, row0 + m, num_items, E, K, h);
+      if (logits != nullptr) store_logits(st, EP + 1, logits, row0, num_items, E, lane);
+      finish_exponentials<float, EP>(g, sum, gates, topk_val, topk_idx, row0 + m, num_items, E, K, h);
     }
   }
 }
