@@ -220,6 +220,28 @@ def test_gate_topk_float32_any_expert_count(K, n, D, E, k, aligned):
       np.testing.assert_array_equal(to_np(a), to_np(e))
 
 
+@pytest.mark.parametrize("n,D,E", [(4096, 768, 8), (20000, 384, 16), (900, 512, 32), (777, 832, 51), (6000, 1024, 128)])
+@pytest.mark.parametrize("features", [2, 8, None])
+def test_gate_topk_float32_keeps_float32_precision(K, n, D, E, features):
+  """Logits of items with a few non-zero features, where every product's last bits show, and of dense ones: no
+  further from 64 bits (2-norm) than a chain of float32 multiply-adds with two roundings more (where the waves'
+  partial sums meet, and where the sums of large and small products do; the error grows as the root of their number)."""
+  gen = torch.Generator(device=dev()).manual_seed(n + (features or 0))
+  x = torch.randn((n, D), generator=gen, device=dev())
+  w = torch.randn((D, E), generator=gen, device=dev()) * D ** -0.5
+  order = torch.arange(D, device=dev()).expand(n, D)
+  if features is not None:
+    order = torch.rand((n, D), generator=gen, device=dev()).argsort(-1)[:, :features].sort(-1).values
+    x = torch.zeros_like(x).scatter_(1, order, x.gather(1, order))
+  exact = x.double() @ w.double()
+  chain = torch.zeros((n, E), device=dev())
+  for i in range(order.shape[1]):
+    k = order[:, i]
+    chain = (chain.double() + x.gather(1, k[:, None]).double() * w[k].double()).float()
+  off = lambda a: ((a.double() - exact).norm() / exact.norm()).item()
+  assert off(K.gate_topk(x[None], w, 1, return_logits=True)[3][0]) <= (1 + 2 / order.shape[1]) ** 0.5 * off(chain)
+
+
 @pytest.mark.parametrize("n,D,E", [(45, 260, 7), (8200, 64, 16), (16400, 36, 5), (33000, 32, 32), (70, 516, 40),
                                    (33000, 64, 33), (50, 100, 100), (33000, 36, 128)])
 @pytest.mark.parametrize("bias", [None, "finite", "infinite"])

@@ -452,8 +452,10 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_kernel(
 }
 
 // float32 gating on the bfloat16 matrix cores: every value is taken apart into three bfloat16 values that add
-// up to it exactly and six of the nine products are summed in float32, as in gemm_f32_split.h (hi is cut
-// off, not rounded, so that no finite value becomes infinite).  The waves of a workgroup (eight; four beyond 64
+// up to it exactly and six of the nine products are summed in float32, as in gemm_f32_split.h; hi.hi in one sum
+// and the five smaller products in another, which meet once k is through: a large sum is rounded once per 16 k.
+// Off from 64 bits (2-norm, 4 096 x 768 x 8): 8.0e-8 where float32 MFMAs are off by 2.5e-7; items with two or
+// eight non-zero features 3.6e-8 and 5.3e-8, as those (with all six in one sum 4.5e-8 and 6.8e-8).  The waves of a workgroup (eight; four beyond 64
 // experts, for the registers) share TW tiles of 32 items, WAVES / TW waves to a tile, each with its share of every chunk of KC rows of the router kernel; the
 // launcher takes as many tiles per workgroup as keep the workgroups at one per CU.  The chunk is split and
 // transposed on its way into LDS, [plane][expert][k], read as eight floats of an expert per thread with
@@ -463,14 +465,6 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_kernel(
 // Bound by the trips to memory (few items: 12 - 15 us; 2 688 items x 832, 38 experts: 73 us on float32 MFMAs with a
 // scalar staging loop, 24 here) or by the splitting and the items' bytes (17 024 x 896, 51 experts: 114 to 50;
 // 30 000 x 384, 16 experts: 21 to 19; 15 774 x 544, 6 experts: 35 to 18).
-__device__ __forceinline__ void split3_cut(float v0, float v1, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
-  const uint32_t u0 = __builtin_bit_cast(uint32_t, v0), u1 = __builtin_bit_cast(uint32_t, v1);
-  hi = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
-  const float r0 = v0 - __builtin_bit_cast(float, u0 & 0xffff0000u), r1 = v1 - __builtin_bit_cast(float, u1 & 0xffff0000u);
-  mid = pack_bf16x2(r0, r1);
-  lo = pack_bf16x2(r0 - bf_lo(mid), r1 - bf_hi(mid));
-}
-
 // The infinite and NaN logits of a tile (32 rows of pitch EP + 1 in LDS; xrow: the lane's row) again, on float32
 // MFMAs, by one wave: an operand that is infinite or rounds to infinity leaves NaN in the sums of its pieces'
 // products, which the softmax's sum shows.  (A call of its own: inline, its registers cost every launch 0.4 to 2 us.
@@ -543,11 +537,11 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_f32_kernel(
     const int tile = tile0 + wave / KS;
     const int row0 = tile * 32;
     const float* const xrow = x + (size_t)min(row0 + m, num_items - 1) * D;
-    floatx16 acc[NT];
+    floatx16 acc[NT], low[NT];                    // sums of hi.hi, and of the five smaller products
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[nt][i] = 0.f;
+      for (int i = 0; i < 16; ++i) acc[nt][i] = low[nt][i] = 0.f;
     float4 va[2][FB][2];
     // (what lies past the wave's share or past D is read from the row's end and multiplied by the zero
     // rows of W or not at all)
@@ -569,7 +563,7 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_f32_kernel(
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const bool in = k0 + kl + (i & 2) * 2 < D;       // (whole quads: D is a multiple of four)
-          split3_cut(in ? v[2 * i] : 0.f, in ? v[2 * i + 1] : 0.f, a[0][i], a[1][i], a[2][i]);
+          split3(in ? v[2 * i] : 0.f, in ? v[2 * i + 1] : 0.f, a[0][i], a[1][i], a[2][i]);
         }
         bf16x8 af[3];
 #pragma unroll
@@ -581,10 +575,11 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_f32_kernel(
           bf16x8 bf[3];
 #pragma unroll
           for (int p = 0; p < 3; ++p) bf[p] = *reinterpret_cast<const bf16x8*>(b + (size_t)p * EP * stride);
-          constexpr int ta[6] = {2, 0, 1, 1, 0, 0}, tb[6] = {0, 2, 1, 0, 1, 0};
+          acc[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[0], bf[0], acc[nt], 0, 0, 0);
+          constexpr int ta[5] = {2, 0, 1, 1, 0}, tb[5] = {0, 2, 1, 0, 1};
 #pragma unroll
-          for (int p = 0; p < 6; ++p)
-            acc[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[ta[p]], bf[tb[p]], acc[nt], 0, 0, 0);
+          for (int p = 0; p < 5; ++p)
+            low[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[ta[p]], bf[tb[p]], low[nt], 0, 0, 0);
         }
       }
     };
@@ -612,7 +607,7 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_f32_kernel(
           uint32_t o[3][4];
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            split3_cut(2 * i < left[t] ? raw[t][2 * i] : 0.f, 2 * i + 1 < left[t] ? raw[t][2 * i + 1] : 0.f,
+            split3(2 * i < left[t] ? raw[t][2 * i] : 0.f, 2 * i + 1 < left[t] ? raw[t][2 * i + 1] : 0.f,
                        o[0][i], o[1][i], o[2][i]);
 #pragma unroll
           for (int p = 0; p < 3; ++p)
@@ -635,7 +630,7 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_f32_kernel(
     for (int nt = 0; nt < NT; ++nt) {
       const float bn = KS == 1 && bias != nullptr ? bias[min(nt * 32 + m, E - 1)] : -0.f;       // (x + -0 is x)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) st[((i >> 2) * 8 + h * 4 + (i & 3)) * (EP + 1) + nt * 32 + m] = acc[nt][i] + bn;
+      for (int i = 0; i < 16; ++i) st[((i >> 2) * 8 + h * 4 + (i & 3)) * (EP + 1) + nt * 32 + m] = acc[nt][i] + low[nt][i] + bn;
     }
     __syncthreads();
     if constexpr (KS > 1) {

@@ -63,14 +63,6 @@ struct SplitCfg {
   static_assert(AI >= 1 && BU >= 1, "tile");
 };
 
-// Two float32 values as three bfloat16 pairs: hi, mid, lo with hi + mid + lo == v exactly.
-__device__ __forceinline__ void split3(float v0, float v1, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
-  hi = pack_bf16x2(v0, v1);
-  const float r0 = v0 - bf_lo(hi), r1 = v1 - bf_hi(hi);
-  mid = pack_bf16x2(r0, r1);
-  lo = pack_bf16x2(r0 - bf_lo(mid), r1 - bf_hi(mid));
-}
-
 template <int EPI, typename Cfg>
 __global__ __launch_bounds__(Cfg::kThreads, Cfg::kWgs * Cfg::kThreads / 256) void gemm_f32_split_kernel(
     const float* __restrict__ A, const float* __restrict__ B, const float* __restrict__ bias,

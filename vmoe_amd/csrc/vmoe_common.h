@@ -41,6 +41,16 @@ __device__ __forceinline__ float bf_hi(uint32_t w) { return __builtin_bit_cast(f
 // Round a float32 to the nearest bfloat16 value, kept as float32.
 __device__ __forceinline__ float bf16r(float f) { return bf2f(f2bf(f)); }
 
+// Two float32 values as three bfloat16 pairs: hi, mid, lo with hi + mid + lo == v exactly.  Each is rounded to
+// nearest, so |mid| <= 2^-8 |v| and |lo| <= 2^-17 |v|: products without mid.lo, lo.mid and lo.lo are off by up to
+// 2^-24 of |a||b|, half a unit in the last place of float32 (each of the first two by 2^-25).
+__device__ __forceinline__ void split3(float v0, float v1, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+  hi = pack_bf16x2(v0, v1);
+  const float r0 = v0 - bf_lo(hi), r1 = v1 - bf_hi(hi);
+  mid = pack_bf16x2(r0, r1);
+  lo = pack_bf16x2(r0 - bf_lo(mid), r1 - bf_hi(mid));
+}
+
 template <typename T> struct Elt;
 template <> struct Elt<float> {
   static constexpr int dtype = VMOE_F32;
