@@ -969,6 +969,19 @@ def test_mlp_moe_block_router_unknown_name():
     layer.create_router()
 
 
+class _MlpBlockWithAux:
+  """MlpBlock with an auxiliary output."""
+
+  def __init__(self, **kwargs):
+    from vmoe_amd.nn import vit_moe
+    self.mlp = vit_moe.MlpBlock(**kwargs)
+
+  def apply_experts(self, variables, inputs, float32_products=False):
+    return self.mlp.apply_experts(variables, inputs, float32_products=float32_products), None
+
+  apply_experts.takes_float32_products = True
+
+
 @pytest.mark.parametrize("dtype,bf16_dispatcher", [(O.F32, False), (O.BF16, False), (O.F32, True)])
 @pytest.mark.parametrize("name", ["indices", "einsum"])
 def test_packed_rows_path_equals_reference_layout(moe, dtype, bf16_dispatcher, name):
@@ -996,6 +1009,9 @@ def test_packed_rows_path_equals_reference_layout(moe, dtype, bf16_dispatcher, n
   got = mlp.apply(mvars, dispatcher, x)
   want = dispatcher.combine(mlp.expert.apply_experts(mvars, dispatcher.dispatch(x)))
   np.testing.assert_array_equal(to_np(got), to_np(want))
+  with_aux = moe.sparse_moe_spmd(_MlpBlockWithAux, variable_axes={"params": 0}, has_aux=True)(
+      mlp_dim=M, dtype=tdtype(dtype))                                # not packed
+  np.testing.assert_array_equal(to_np(with_aux.apply(mvars, dispatcher, x)[0]), to_np(want))
   buf, rows = dispatcher.dispatch_packed(x)
   inner = dispatcher.dispatcher if bf16_dispatcher else dispatcher
   fill = getattr(inner, "_inner", inner).fill

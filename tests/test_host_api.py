@@ -377,3 +377,26 @@ def test_small_tiles_are_not_taken_where_they_would_run_on_few_dies(monkeypatch,
   chosen = _ragged_mlp_bytes(E, R, D, M)
   monkeypatch.setenv("VMOE_ROW_TILES", "off")
   assert (chosen < _ragged_mlp_bytes(E, R, D, M)) == small
+
+
+@pytest.mark.parametrize("packed", [True, False])
+@pytest.mark.parametrize("has_aux,inputs", [(True, 1), (False, 2)])
+def test_only_dispatchers_without_packed_rows_ask_for_float32_products(packed, has_aux, inputs):
+  """A layer behind a bfloat16 dispatcher with packed rows takes the same float32 products with auxiliary
+  outputs or several inputs, where its rows are not packed, as without them."""
+  class Inner:
+    supports_packed = lambda self: packed
+    dispatch = combine = lambda self, data: data
+
+  class Experts:
+    def apply_experts(self, variables, *dispatched, float32_products=False):
+      asked.append(float32_products)
+      return (dispatched[0], None) if has_aux else dispatched[0]
+
+    apply_experts.takes_float32_products = True
+
+  asked = []
+  layer = moe.sparse_moe_spmd(Experts, has_aux=has_aux)()
+  items = [torch.zeros((2, 3), dtype=torch.int32)] * inputs       # (integers pass the dispatcher uncast)
+  layer.apply({}, moe.Bfloat16Dispatcher(Inner()), *items)
+  assert asked == [not packed]

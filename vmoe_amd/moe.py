@@ -689,8 +689,9 @@ def sparse_moe_spmd(target, variable_axes: Optional[Mapping[str, Any]] = None,
       dispatched = [dispatcher.dispatch(x) for x in inputs]
       if hasattr(self.expert, "apply_experts"):
         # Soft MoE: outputs that combine rounds to bfloat16, where float32 sums in another order round the
-        # other way in one value of 4 000 (3e-5 of the layer's output).
-        rounded = (isinstance(dispatcher, Bfloat16Dispatcher)
+        # other way in one value of 4 000 (3e-5 of the layer's output).  (A dispatcher with packed rows takes
+        # the same products here, with auxiliary outputs or several inputs, as on its packed path.)
+        rounded = (isinstance(dispatcher, Bfloat16Dispatcher) and not dispatcher.supports_packed()
                    and getattr(self.expert.apply_experts, "takes_float32_products", False))
         outputs = self.expert.apply_experts(variables, *dispatched,
                                             **({"float32_products": True} if rounded else {}))
