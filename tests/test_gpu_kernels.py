@@ -970,6 +970,40 @@ def test_expert_mlp_float32_products_on_the_dma_kernel(K, monkeypatch, E, R, D, 
   np.testing.assert_array_equal(outs["dma"][0], outs["64"][0])              # same order of k
 
 
+@pytest.mark.parametrize("width", [36, 64, 100])
+@pytest.mark.parametrize("approximate", [True, False])
+def test_expert_mlp_float32_gelu(K, monkeypatch, width, approximate):
+  """The GELU of float32 MLPs through products with the identity, which are exact: tanhf where the width is no
+  multiple of 32, else within the roundings of x / (1 + 2^z) on the hardware's exp2 and reciprocal; the same as behind
+  products on float32 instructions."""
+  from scipy.special import erfc
+  x = np.concatenate([np.linspace(-14, 14, 20 * width), np.logspace(-30, 2, 10 * width),
+                      -np.logspace(-30, 2, 10 * width)]).astype(np.float32).reshape(1, 40, width)
+  eye = to_dev(np.eye(width, dtype=np.float32)[None])
+  run = lambda **kw: to_np(K.expert_mlp(to_dev(x), eye, None, eye, None, approximate_gelu=approximate, **kw))
+  monkeypatch.delenv("VMOE_F32_GEMM", raising=False)
+  got = run()
+  # (three bfloat16 values end at 2^-133: below 2^-110 a value loses its last bits)
+  np.testing.assert_allclose(got, run(float32_products=True), rtol=0, atol=2.0 ** -133)
+  monkeypatch.setenv("VMOE_F32_GEMM", "plain")
+  plain = run()
+  v = x.astype(np.float64)
+  if not approximate or width % 32 != 0:
+    np.testing.assert_array_equal(got, plain)
+  u = 2 * np.sqrt(2 / np.pi) * (v + 0.044715 * v ** 3)
+  with np.errstate(over="ignore"):
+    want = v / (1 + np.exp(-u)) if approximate else 0.5 * v * erfc(-v / np.sqrt(2))
+  # tanhf, erff: two units in the last place of a number up to one, the sum half a one, which x / 2 scales
+  bound = 2.0 ** -24 * (3 * np.abs(v) + np.abs(want))
+  if approximate and width % 32 == 0:
+    # z: three roundings and two rounded constants, each 2^-24 of |u|, which the exponential makes relative; exp2, the
+    # sum, the reciprocal and the product: 2^-24 each, twice that for the two hardware functions.  Below 2^-120 it ends.
+    bound = 2.0 ** -24 * (6 + 5 * np.abs(u)) * np.abs(want) + 2.0 ** -120
+  elif approximate:
+    bound += 2.0 ** -24 * 5 * np.abs(u) * np.abs(v) / np.cosh(np.minimum(np.abs(u) / 2, 300)) ** 2 / 4    # of tanh's argument
+  assert (np.abs(got - want) <= bound + 2.0 ** -148).all()
+
+
 @pytest.mark.parametrize("E,R,D,M", [(3, 129, 96, 260), (5, 33, 100, 132), (2, 64, 800, 128), (70, 3, 36, 64)])
 def test_expert_mlp_float32_split_tiles(K, monkeypatch, E, R, D, M):
   """Every tile of the float32 products on bfloat16 MFMAs (three bfloat16 values per operand), at

@@ -121,6 +121,11 @@ int launch_gemm_f32(const float* A, const float* B, const float* bias, float* C,
   if (!dma && (!plain || a_rows != nullptr)) {
     const int tile = which != nullptr && strncmp(which, "tile", 4) == 0 ? atoi(which + 4)
                                                                        : best_split_tile(batch, R, N, Kd);
+    // Operands that float32 instructions would take on the register-staged kernel get its tanhf.
+    if constexpr (EPI == kEpiBiasGeluTanh) {
+      if (!gemm_f32_dma_ok(A, B, R, N, Kd, a_items))
+        return launch_gemm_f32_split<kEpiBiasGeluTanhf>(tile, A, B, bias, C, batch, R, N, Kd, stream, rows, a_rows, a_items);
+    }
     return launch_gemm_f32_split<EPI>(tile, A, B, bias, C, batch, R, N, Kd, stream, rows, a_rows, a_items);
   }
   // The DMA kernel where its shapes allow (gathered rows are its alone: check_mlp has made sure that it
