@@ -95,12 +95,12 @@ def test_gate_topk_logit_bias(K):
   assert_close(to_np(gates), O.router_gates(x, w, O.BF16, b), 2e-2, "gates with bias")
 
 
-@pytest.mark.parametrize("n,D,E", [(1568, 512, 8), (45, 64, 5), (4100, 384, 32), (33, 1024, 24)])
-def test_gate_topk_float32_split_k_form(K, monkeypatch, n, D, E):
-  """float32 gating over few items deals the k range of a tile to the four waves of a workgroup
-  (partial logits added in wave order): against the one-wave-per-tile form
-  (VMOE_GATE_NO_SPLIT_K=1) bit for bit on operands whose partial sums are exact, within float32
-  rounding otherwise; logits output and logit bias included."""
+@pytest.mark.parametrize("n,D,E", [(1568, 512, 8), (45, 64, 5), (4100, 384, 32), (33, 1024, 24),
+                                   (8200, 64, 16), (16400, 36, 5), (33000, 32, 32)])      # 1, 2, 4 and 8 tiles a workgroup
+def test_gate_topk_float32_split_k_form(K, n, D, E):
+  """float32 gating deals the k range of a tile to the waves that share it, fewer the more tiles there
+  are (partial logits added in wave order): the 64-bit logits bit for bit on operands whose partial sums are
+  exact, within float32 rounding otherwise; logits output and logit bias included."""
   rng = np.random.default_rng(n + D)
   xi = rng.integers(-2, 3, (1, n, D)).astype(np.float32)
   wi = rng.integers(-2, 3, (D, E)).astype(np.float32) / 64
@@ -108,23 +108,22 @@ def test_gate_topk_float32_split_k_form(K, monkeypatch, n, D, E):
   xr = rng.standard_normal((1, n, D)).astype(np.float32)
   wr = (rng.standard_normal((D, E)) / np.sqrt(D)).astype(np.float32)
   for x, w, exact in ((xi, wi, True), (xr, wr, False)):
-    monkeypatch.delenv("VMOE_GATE_NO_SPLIT_K", raising=False)
-    g_s, v_s, i_s, l_s = K.gate_topk(to_dev(x), to_dev(w), 2, logit_bias=to_dev(b), return_logits=True)
+    gates, val, idx, logits = K.gate_topk(to_dev(x), to_dev(w), 2, logit_bias=to_dev(b), return_logits=True)
+    g_n, v_n, i_n = K.gate_topk(to_dev(x), to_dev(w), 2, logit_bias=to_dev(b))
     g_p, v_p, i_p = K.gate_topk(to_dev(x), to_dev(w), 2)
-    monkeypatch.setenv("VMOE_GATE_NO_SPLIT_K", "1")
-    g_d, v_d, i_d, l_d = K.gate_topk(to_dev(x), to_dev(w), 2, logit_bias=to_dev(b), return_logits=True)
-    monkeypatch.delenv("VMOE_GATE_NO_SPLIT_K")
     want = x[0].astype(np.float64) @ w.astype(np.float64) + b
-    np.testing.assert_allclose(to_np(l_s)[0], want, rtol=1e-5, atol=1e-5)
-    assert_close(to_np(g_p), O.router_gates(x, w, O.F32), 1e-5, "gates without bias")
     if exact:
-      np.testing.assert_array_equal(to_np(l_s), to_np(l_d))
-      np.testing.assert_array_equal(to_np(g_s), to_np(g_d))
-      np.testing.assert_array_equal(to_np(i_s), to_np(i_d))
-      np.testing.assert_array_equal(to_np(v_s), to_np(v_d))
+      np.testing.assert_array_equal(to_np(logits)[0], want)
     else:
-      np.testing.assert_allclose(to_np(l_s), to_np(l_d), rtol=1e-5, atol=1e-5)
-      np.testing.assert_allclose(to_np(g_s), to_np(g_d), rtol=1e-5, atol=1e-6)
+      np.testing.assert_allclose(to_np(logits)[0], want, rtol=1e-5, atol=1e-5)
+    assert_close(to_np(gates), O.router_gates(x, w, O.F32, b), 1e-5, "gates")
+    assert_close(to_np(g_p), O.router_gates(x, w, O.F32), 1e-5, "gates without bias")
+    for with_logits, without in ((gates, g_n), (val, v_n), (idx, i_n)):
+      np.testing.assert_array_equal(to_np(with_logits), to_np(without))
+    for g, v, i in ((gates, val, idx), (g_p, v_p, i_p)):
+      want_v, want_i = O.top_k(to_np(g), 2)
+      np.testing.assert_array_equal(to_np(i), want_i)
+      np.testing.assert_array_equal(to_np(v), want_v)
 
 
 @pytest.mark.parametrize("n,D,E,k", [(1, 64, 8, 8), (31, 128, 16, 1), (32, 192, 32, 2), (33, 768, 24, 3),
@@ -935,39 +934,44 @@ def test_compact_rows(K, G, S, E, Kk, C, bpr):
 
 
 @pytest.mark.parametrize("E,R,D,M", [
-    (8, 416, 512, 2048),      # the S/32 layer: one expert per die
-    (5, 700, 512, 1024),      # runs that begin and end inside an expert
-    (3, 1000, 512, 1536),
+    (8, 416, 512, 2048),      # one expert per die; first product 64 x 128 tiles, second 64 x 64
+    (5, 700, 512, 1024),      # 64 x 64 tiles; runs that begin and end inside an expert
+    (3, 1000, 512, 1536),     # 64 x 128 and 64 x 64
 ])
 def test_expert_mlp_float32_products_on_the_dma_kernel(K, monkeypatch, E, R, D, M):
-  """The float32 products on the LDS-DMA kernel (64 x 128 or 64 x 64 tiles, one run of the tile
-  list per die, rows past a count skipped in blocks of 32) against the register-staged kernel
-  and against the oracle; dense and over ragged rows."""
+  """Float32 products on float32 matrix instructions (float32_products=True): the LDS-DMA kernel (64 x 128 or
+  64 x 64 tiles, one run of the tile list per die, rows past a count skipped in blocks of 32)
+  against the register-staged kernel and the oracle; dense, over ragged rows and over gathered ones;
+  the same bits in a call of four times the rows, which takes 64 x 128 tiles for either product."""
+  monkeypatch.delenv("VMOE_F32_GEMM", raising=False)
   rng = np.random.default_rng(E + R)
   x = rng.standard_normal((E, R, D)).astype(np.float32)
   w0 = (rng.standard_normal((E, D, M)) / np.sqrt(D)).astype(np.float32)
   b0 = (rng.standard_normal((E, M)) * 0.1).astype(np.float32)
   w1 = (rng.standard_normal((E, M, D)) / np.sqrt(M)).astype(np.float32)
   b1 = (rng.standard_normal((E, D)) * 0.1).astype(np.float32)
-  args = [to_dev(a) for a in (x, w0, b0, w1, b1)]
+  items = rng.standard_normal((R + 7, D)).astype(np.float32)
+  x_rows = rng.integers(0, R + 7, (E, R)).astype(np.int32)
+  weights = [to_dev(a) for a in (w0, b0, w1, b1)]
   rows = rng.integers(0, R + 1, E).astype(np.int32)
   rows[:3] = [R, 0, 33]
-  want = O.mlp_block(x, w0, b0, w1, b1, O.F32)
-  outs = {}
-  for form in ("dma", "64", "plain"):
-    if form != "dma":
-      monkeypatch.setenv("VMOE_F32_GEMM", form)
-    dense = to_np(K.expert_mlp(*args))
-    ragged = torch.full((E, R, D), 7.0, dtype=torch.float32, device=dev())
-    K.expert_mlp(*args, out=ragged, rows_per_expert=to_dev(rows))
-    outs[form] = (dense, to_np(ragged))
-    assert_close(dense, want, 1e-5, f"{form}: dense")
-    for e, n in enumerate(rows):
-      np.testing.assert_array_equal(outs[form][1][e, :n], dense[e, :n], err_msg=f"{form}: expert {e}")
-      assert (outs[form][1][e, n:] == 7.0).all(), f"{form}: expert {e} wrote past its rows"
-  monkeypatch.delenv("VMOE_F32_GEMM")
-  assert_close(outs["dma"][0], outs["plain"][0], 1e-5, "dma against plain")   # other order of k
-  np.testing.assert_array_equal(outs["dma"][0], outs["64"][0])              # same order of k
+  run = lambda x, **kw: to_np(K.expert_mlp(to_dev(x), *weights, float32_products=True, **kw))
+  ragged = lambda x, **kw: run(x, out=torch.full((E, R, D), 7.0, device=dev()), rows_per_expert=to_dev(rows), **kw)
+  dense = run(x)
+  assert_close(dense, O.mlp_block(x, w0, b0, w1, b1, O.F32), 1e-5, "dense")
+  some, gathered, indexed = ragged(x), ragged(items, x_rows=to_dev(x_rows)), run(items[x_rows])
+  for e, n in enumerate(rows):
+    np.testing.assert_array_equal(some[e, :n], dense[e, :n], err_msg=f"ragged: expert {e}")
+    np.testing.assert_array_equal(gathered[e, :n], indexed[e, :n], err_msg=f"gathered: expert {e}")
+    assert (some[e, n:] == 7.0).all() and (gathered[e, n:] == 7.0).all(), f"expert {e}: written past its rows"
+  assert E * -(-4 * R // 64) * (D // 128) >= 512
+  np.testing.assert_array_equal(run(np.tile(x, (1, 4, 1))), np.tile(dense, (1, 4, 1)))    # same order of k
+  # the default products round in another order: they are not what ran above
+  assert (to_np(K.expert_mlp(to_dev(x), *weights)) != dense).any()
+  monkeypatch.setenv("VMOE_F32_GEMM", "plain")
+  plain = to_np(K.expert_mlp(to_dev(x), *weights))
+  assert_close(dense, plain, 1e-5, "against plain")                                       # other order of k
+  assert (plain != dense).any()
 
 
 @pytest.mark.parametrize("width", [36, 64, 100])
@@ -1002,6 +1006,27 @@ def test_expert_mlp_float32_gelu(K, monkeypatch, width, approximate):
   elif approximate:
     bound += 2.0 ** -24 * 5 * np.abs(u) * np.abs(v) / np.cosh(np.minimum(np.abs(u) / 2, 300)) ** 2 / 4    # of tanh's argument
   assert (np.abs(got - want) <= bound + 2.0 ** -148).all()
+
+
+def test_expert_mlp_float32_over_the_size_of_the_call(K, monkeypatch):
+  """The tile, and with it the order of float32 sums, depends on the size of the call: the same items
+  through the same experts stay as close to 64 bits at every size as float32 matrix instructions
+  are (2-norm, a twentieth for the differing order of few sums; see test_expert_mlp_float32_split_tiles)."""
+  monkeypatch.delenv("VMOE_F32_GEMM", raising=False)
+  rng = np.random.default_rng(5)
+  E, D, M, n = 8, 512, 2048, 16
+  x = rng.standard_normal((E, 784, D)).astype(np.float32)
+  w0 = (rng.standard_normal((E, D, M)) / np.sqrt(D)).astype(np.float32)
+  w1 = (rng.standard_normal((E, M, D)) / np.sqrt(M)).astype(np.float32)
+  u = x[:, :n].astype(np.float64) @ w0
+  want = (u / (1 + np.exp(-2 * np.sqrt(2 / np.pi) * (u + 0.044715 * u ** 3)))) @ w1
+  off = lambda a: np.linalg.norm(a - want) / np.linalg.norm(want)
+  run = lambda R: to_np(K.expert_mlp(to_dev(x[:, :R]), to_dev(w0), None, to_dev(w1), None))[:, :n]
+  outs = {R: run(R) for R in (16, 49, 98, 196, 392, 784)}
+  monkeypatch.setenv("VMOE_F32_GEMM", "plain")
+  most = 1.05 * off(run(n))
+  assert all(off(out) <= most for out in outs.values()), ({R: off(out) for R, out in outs.items()}, most)
+  assert len({out.tobytes() for out in outs.values()}) > 1        # (several tiles were taken)
 
 
 @pytest.mark.parametrize("E,R,D,M", [(3, 129, 96, 260), (5, 33, 100, 132), (2, 64, 800, 128), (70, 3, 36, 64)])
