@@ -318,7 +318,9 @@ int vmoe_densify(const VmoeDensifyParams* p, vmoe_stream_t stream);
  * matmul, after each bias add and after the GELU.
  * float32: every operand value is taken apart into three bfloat16 values that add up to it and
  * six of the nine products are summed in float32 on the bfloat16 matrix instructions (error
- * against 64 bits below that of float32 instructions, other rounding).  VMOE_MLP_F32_PRODUCTS
+ * against 64 bits below that of float32 instructions, other rounding).  The order of these sums
+ * depends on E, R, D and M: the same row through the same weights can differ in its last bits between
+ * calls of other sizes (dense, ragged and gathered calls of one size agree).  VMOE_MLP_F32_PRODUCTS
  * keeps float32 instructions, and with them the order of sums that outputs rounded to bfloat16
  * further on were made with (Soft MoE's dispatcher: one output in 4 000 rounds the other way).
  * bf16 needs the kernels in K-contiguous order: pass w0t (E,M,D) / w1t (E,D,M)

@@ -146,9 +146,10 @@ template <> struct Chunk<bf16_t> {
   }
 };
 
-// UNIT, here and in the two kernels below: every weight is one and none is read.  (A form of the kernel: the null
-// pointer looked at here keeps the loads of weights and slots apart, a second trip to memory before the rows:
-// 64 x 576 items x 1 024, two choices, 20.8 us, 18.6 as forms; 256 x 196 x 768: 38.0 and 36.9.)
+// UNIT, here and in the two kernels below: every weight is one and none is read.  (A form of the kernel, so
+// that combine keeps its time: a null pointer looked at here keeps the loads of weights and slots apart, a second
+// trip to memory before the rows: 64 x 576 items x 1 024, two choices, 20.8 us in place of 18.6; 256 x 196 x 768:
+// 38.0 of 36.9.)
 template <typename T, bool UNIT>
 __global__ __launch_bounds__(kMoveThreads) void combine_kernel(
     const uint4* __restrict__ y, const int32_t* __restrict__ token_slot,

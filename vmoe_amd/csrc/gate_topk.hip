@@ -29,42 +29,9 @@
 namespace vmoe {
 namespace {
 
-
 __device__ __forceinline__ float inv_orderable(uint32_t u) {
   uint32_t b = (u & 0x80000000u) ? (u & 0x7fffffffu) : ~u;
   return __builtin_bit_cast(float, b);
-}
-
-template <int MASK>
-__device__ __forceinline__ float xor_max(float v) {
-  return fmaxf(v, __shfl_xor(v, MASK, kWave));
-}
-
-__device__ __forceinline__ float half_wave_max(float v) {
-  v = fmaxf(v, __shfl_xor(v, 1, kWave));
-  v = fmaxf(v, __shfl_xor(v, 2, kWave));
-  v = fmaxf(v, __shfl_xor(v, 4, kWave));
-  v = fmaxf(v, __shfl_xor(v, 8, kWave));
-  v = fmaxf(v, __shfl_xor(v, 16, kWave));
-  return v;
-}
-__device__ __forceinline__ float half_wave_sum(float v) {
-  v += __shfl_xor(v, 1, kWave);
-  v += __shfl_xor(v, 2, kWave);
-  v += __shfl_xor(v, 4, kWave);
-  v += __shfl_xor(v, 8, kWave);
-  v += __shfl_xor(v, 16, kWave);
-  return v;
-}
-__device__ __forceinline__ uint64_t half_wave_max_u64(uint64_t v) {
-#pragma unroll
-  for (int m = 1; m < 32; m <<= 1) {
-    uint32_t lo = __shfl_xor((uint32_t)v, m, kWave);
-    uint32_t hi = __shfl_xor((uint32_t)(v >> 32), m, kWave);
-    uint64_t o = ((uint64_t)hi << 32) | lo;
-    v = o > v ? o : v;
-  }
-  return v;
 }
 
 // Softmax and top-K of one item by two lanes: g holds the logits of experts h * EP / 2 ..., lane ^ 32 the
@@ -461,9 +428,10 @@ __global__ __launch_bounds__(WAVES * kWave) void gate_topk_kernel(
 // transposed on its way into LDS, [plane][expert][k], read as eight floats of an expert per thread with
 // neighbouring lanes on neighbouring experts, whatever E and the address are.  Item rows come four 16-wide k
 // steps at a time, two such batches in flight, the first two sent before the chunk is staged.  The partial
-// logits of a tile meet in LDS, added in wave order, and its first wave finishes it.
+// logits of a tile meet in LDS, added in wave order, and its first wave finishes it.  (How many waves share a tile
+// depends on the number of items, and with it the last bits of an item's logits.)
 // Bound by the trips to memory (few items: 12 - 15 us; 2 688 items x 832, 38 experts: 73 us on float32 MFMAs with a
-// scalar staging loop, 24 here) or by the splitting and the items' bytes (17 024 x 896, 51 experts: 114 to 50;
+// scalar staging loop, 25 here) or by the splitting and the items' bytes (17 024 x 896, 51 experts: 114 to 50;
 // 30 000 x 384, 16 experts: 21 to 19; 15 774 x 544, 6 experts: 35 to 18).
 // The infinite and NaN logits of a tile (32 rows of pitch EP + 1 in LDS; xrow: the lane's row) again, on float32
 // MFMAs, by one wave: an operand that is infinite or rounds to infinity leaves NaN in the sums of its pieces'

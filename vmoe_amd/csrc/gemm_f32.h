@@ -17,7 +17,7 @@
 //     the operands is fetched into the die's L2 once for all of them;
 //   * rows beyond a ragged batch's count cost nothing: a wave skips the 32-row blocks that
 //     hold none, so a tile's time follows its live blocks.
-// With requests, fragment reads and barriers taken out the launches of the S/32 layer last
+// With requests, fragment reads and barriers taken out launches of 8 x 392 rows x 512 x 2 048 last
 // nearly as long as with them: what is left between them and the peak is the 3.4 or 1.75 tiles
 // per CU, and that the workgroups that share a CU, taking turns MFMA by MFMA, also reach their
 // prologues and epilogues together.
@@ -31,7 +31,6 @@
 #include "gemm_f32_split.h"
 
 namespace vmoe {
-
 
 template <int BN_>
 struct F32Cfg {

@@ -1,11 +1,12 @@
 // float32 expert products (vmoe/nn/vit_moe.py:38-45 on float32 parameters) on the bfloat16 matrix
-// cores: every operand value is taken apart into three bfloat16 values whose sum it is exactly.
+// cores: every operand value is taken apart into three bfloat16 values whose sum it is exactly (Henry, Tang and
+// Heinecke, "Leveraging the bfloat16 artificial intelligence datatype for higher-precision computations", 2019).
 //
 // C[b] = epilogue(A[b] (R x Kd) . B[b] (Kd x N) + bias[b]); B in the reference's (in, out) order.
 //
 // v = hi + mid + lo, each rounded to nearest from what the ones before it leave: 8 + 8 + 8 bits hold
 // a float32 significand.  Of the nine products six are taken (lo.hi, hi.lo, mid.mid, mid.hi, hi.mid,
-// hi.hi, in this order, float32 accumulators); the three left out are below 2^-25 of |a||b|, under the
+// hi.hi, in this order, float32 accumulators); the three left out add up to 2^-24 of |a||b| at most (split3), the
 // rounding of a float32 product.  One instruction adds 32 products to a sum in place of two, so there
 // are fewer roundings along k than on v_mfma_f32_32x32x2_f32: against 64 bits the MLPs of eleven
 // shapes (D 384 .. 832, M 1 408 .. 3 328, 22 .. 9 216 rows) are off by 6.8e-7 .. 1.0e-6 in place of 8.1e-7 ..
@@ -32,6 +33,9 @@
 // (spills, 320); k tiles two or four ahead (no change).
 // KG groups of four waves in a workgroup take consecutive runs of k tiles, each through its own LDS,
 // and add their sums in group order: launches of few tiles are as long as one tile's chain of k tiles.
+// The tile comes from the sizes of the call (kSplitTiles), so the order of an output's sums does too: the same item
+// through the same weights can differ in its last bits between calls over different numbers of rows or experts
+// (not between dense, ragged and gathered calls of one size), as bfloat16 MLPs can.
 // Workgroups -> tiles: the live tiles of all batches (row counts are read by every workgroup) are
 // numbered batch-major, column panel by column panel, and cut into eight equal runs, one per XCD, so that
 // the row tiles that share a column panel of weights run on one die at the same time.

@@ -59,7 +59,8 @@ std::string shape_of(const Tensor& t) {
 }
 void need_axes(const Tensor& t, int64_t axes, const char* name) {
   if (t.dim() != axes)
-    throw py::value_error(std::string(name) + " has shape " + shape_of(t) + ", expected " + std::to_string(axes) + " axes");
+    throw py::value_error(std::string(name) + " has shape " + shape_of(t) + ", expected " + std::to_string(axes) +
+                          " axes");
 }
 void need_values(const Tensor& t, int64_t least, const char* name) {
   if (t.numel() < least)
@@ -252,7 +253,8 @@ std::tuple<Tensor, Tensor, int64_t, OptTensor, OptTensor, OptTensor, bool> exper
   p.M = (int32_t)M;
   Tensor out = out_.has_value() ? *out_ : empty({E, R, D}, x.scalar_type(), x);
   p.x = ptr(x); p.w0 = ptr(w0); p.b0 = ptr(b0); p.w1 = ptr(w1); p.b1 = ptr(b1); p.w0t = ptr(w0t); p.w1t = ptr(w1t);
-  p.out = ptr(out); p.dtype = dtype_code(x); p.gelu = (tanh_gelu ? VMOE_GELU_TANH : VMOE_GELU_ERF) + (f32_products ? VMOE_MLP_F32_PRODUCTS : 0) +
+  p.out = ptr(out); p.dtype = dtype_code(x);
+  p.gelu = (tanh_gelu ? VMOE_GELU_TANH : VMOE_GELU_ERF) + (f32_products ? VMOE_MLP_F32_PRODUCTS : 0) +
            (f32_biases ? VMOE_MLP_F32_BIASES : 0);
   p.rows_per_expert = ptr_as<int32_t>(rows); p.x_rows = ptr_as<int32_t>(row_token);
   const size_t need = vmoe_expert_mlp_workspace_bytes(&p);

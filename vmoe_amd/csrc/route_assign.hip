@@ -264,8 +264,7 @@ __device__ __forceinline__ void route_assign_group(
           }
         }
       }
-      if (counted) {
-      } else if (__syncthreads_and(narrow_ok)) {
+      if (!counted && __syncthreads_and(narrow_ok)) {
         uint32_t key[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
@@ -276,7 +275,7 @@ __device__ __forceinline__ void route_assign_group(
 #pragma unroll
         for (int r = 0; r < R; ++r)
           if (tid < nact && tid * R + r < S) rank[key[r] & 0xffffu] = tid * R + r;
-      } else {
+      } else if (!counted) {
         uint64_t key[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
