@@ -1301,6 +1301,29 @@ def test_expert_mlp_every_small_tile(K, monkeypatch, tile):
   test_expert_mlp_small_tiles(K, 9, 1, 192, 72)
 
 
+@pytest.mark.parametrize("tile", [3, 5, 6, 7, 13, 14, 15, 16])
+def test_expert_mlp_medium_tiles(K, monkeypatch, tile):
+  """The tiles of the kernel for a few hundred to a few thousand rows: the checks of the small tiles with and
+  without a launch plan, at one row past a tile of each height, k and columns that end inside, and bit
+  for bit what the smallest tile computes (same order of sums), also without a bias and with biases at an
+  odd element."""
+  for E, R, D, M in [(3, 131, 136, 264), (9, 1, 192, 72), (17, 257, 320, 200), (9, 193, 96, 1032), (3, 1100, 64, 8)]:
+    monkeypatch.setenv("VMOE_ROW_TILES", str(tile))
+    test_expert_mlp_small_tiles(K, E, R, D, M)
+    rng = np.random.default_rng(E)
+    mk = lambda scale, *s: to_dev(O.cast(rng.standard_normal(s).astype(np.float32) * scale, O.BF16), O.BF16)
+    x, w0, w1 = mk(1, E, R, D), mk(D ** -0.5, E, D, M), mk(M ** -0.5, E, M, D)
+    b0, b1 = mk(0.1, E * M + 1)[1:].view(E, M), mk(0.1, E * D + 1)[1:].view(E, D)
+    for biases in ((None, None), (b0, b1)):
+      for approximate in (True, False):
+        args = (x, w0, biases[0], w1, biases[1])
+        monkeypatch.setenv("VMOE_ROW_TILES", str(tile))
+        got = K.expert_mlp(*args, approximate_gelu=approximate)
+        monkeypatch.setenv("VMOE_ROW_TILES", "0")
+        want = K.expert_mlp(*args, approximate_gelu=approximate)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 @pytest.mark.parametrize("tile", range(8, 13))
 @pytest.mark.parametrize("E,R,D,M", [
     (130, 64, 640, 776),     # several tiles per workgroup, column tiles and k that end inside

@@ -4,6 +4,7 @@
 // vit_jax.models_vit.MlpBlock (vmoe/nn/vit_moe.py:38-45): a GEMM batched over
 // the expert axis with the bias add and the GELU fused into the epilogue of the
 // first product and the bias add into the second.
+#include <algorithm>
 #include <cstring>
 
 #include "gemm_bf16_wide.h"
@@ -366,7 +367,7 @@ struct MlpPlans {
   int up_rows = -1, down_rows = -1;      // tile of launch_gemm_bf16_rows, -1: not taken
   GemmGeom up, down;
   DownKernel down_kernel = kDownPlain;
-  int down_bm = CfgDown::BM;
+  int up_bm = CfgUp::BM, down_bm = CfgDown::BM;
   size_t up_bytes = 0, down_bytes = 0;   // 0: that product keeps the static tile order
   bool planned = false;                  // vmoe_expert_mlp_planned takes the call (the small tiles need no plan)
   size_t streamk_bytes = 0;              // exchange memory of kDownShared
@@ -421,38 +422,35 @@ MlpPlans mlp_plans(int E, int R, int D, int M, bool ragged, long long items) {
   if (shared_ok && t_shared <= t_best) { m.down_kernel = kDownShared; t_best = t_shared; }
   if (eight_ok && t_eight <= t_best) { m.down_kernel = kDownEightWaves; t_best = t_eight; }
   if (narrow_ok && t_narrow < 0.97 * t_best) { m.down_kernel = kDownNarrow; t_best = t_narrow; }
-  // Few rows: the small tiles of gemm_bf16_rows.h where their estimate is below that of the large
-  // ones (shapes that only the register-staged kernel would take always).
+  // Few rows: the small tiles of gemm_bf16_rows.h and gemm_bf16_mid.h where their estimate is below that of the
+  // large ones (shapes that only the register-staged kernel would take always).
   // (VMOE_ROW_TILES=off in the environment keeps the large tiles, VMOE_ROW_TILES=<index into kRowsTiles, and
-  // behind them kStreamTiles> takes that tile for both products wherever the kernel takes the operands: the switch behind the
+  // behind them kStreamTiles and kMoreTiles> takes that tile for both products wherever the kernel takes the operands: the switch behind the
   // figures of the table, and what tests of the other kernels set)
   const char* const row_tiles = getenv("VMOE_ROW_TILES");
   const bool any_tile = row_tiles == nullptr || strcmp(row_tiles, "off") != 0;
   const int forced = any_tile && row_tiles != nullptr ? atoi(row_tiles) : -1;
-  const auto forced_ok = [&](int Kd) {
-    return forced >= 0 && (forced < kNumRowsTiles || stream_tile_ok(forced - kNumRowsTiles, E, R, Kd, ragged));
+  const auto forced_ok = [&](int N, int Kd, long long n) {
+    if (forced < 0) return false;
+    if (is_mid_tile(forced)) return mid_gemm_ok(E, R, N, Kd, n);
+    return forced < kNumRowsTiles || stream_tile_ok(forced - kNumRowsTiles, E, R, Kd, ragged);
   };
-  double rows_us = 0;
   if (any_tile && rows_gemm_ok(R, M, D, items)) {
-    const int tile = best_rows_tile(E, R, M, D, &rows_us);
-    double us = m.up.fast ? product_us(kFirstProductTile, E, R, M, D, false) : 1e30;
-    if (rows_us < us) { m.up_rows = tile; us = rows_us; }
-    const int walked = best_stream_tile(E, R, M, D, ragged, true, us);
-    if (walked >= 0) m.up_rows = walked;
-    if (forced_ok(D)) m.up_rows = forced;
+    const double us = m.up.fast ? product_us(D % 64 == 0 ? kFirstProductTile : kFirstProductK32Tile, E, R, M, D, true, false) : 1e30;
+    m.up_rows = best_tile(E, R, M, D, items, ragged, true, us);
+    if (forced_ok(M, D, items)) m.up_rows = forced;
   }
   if (any_tile && rows_gemm_ok(R, D, M, 0)) {
-    const int tile = best_rows_tile(E, R, D, M, &rows_us);
-    if (t_best > 1e29 && square.fast)
-      t_best = unit * (half ? 0.5 * 1.05 * std::ceil((double)E * ((R + 127) / 128) * ((D + 255) / 256) / kNumCu)
+    double us = 1e30;
+    if (m.down_kernel == kDownEightWaves || m.down_kernel == kDownNarrow)
+      us = product_us(m.down_kernel == kDownNarrow ? kNarrowTile : kEightWavesTile, E, R, D, M, false, false);
+    else if (t_best < 1e29)
+      us = 5 + t_best;
+    else if (square.fast)
+      us = 5 + unit * (half ? 0.5 * 1.05 * std::ceil((double)E * ((R + 127) / 128) * ((D + 255) / 256) / kNumCu)
                             : std::ceil((double)square.tiles / kNumCu));
-    // (the model of the large tiles above counts their MFMAs; over few rows they wait for the weights:
-    // 128 experts x 128 rows x 768 x 3072 take 143 us, 5 TB/s, where it says 111)
-    double us = std::fmax(t_best, 2.0 * E * ((double)D * M + (double)R * (D + M)) / 5e6);
-    if (rows_us < 5 + t_best) { m.down_rows = tile; us = rows_us; }
-    const int walked = best_stream_tile(E, R, D, M, ragged, false, us);
-    if (walked >= 0) m.down_rows = walked;
-    if (forced_ok(M)) m.down_rows = forced;
+    m.down_rows = best_tile(E, R, D, M, 0, ragged, false, us);
+    if (forced_ok(D, M, 0)) m.down_rows = forced;
   }
   // (VMOE_SECOND_PRODUCT=shared|eight|narrow|wide in the environment overrides the choice
   // where the named kernel applies: the switch behind the figures that the model above was
@@ -472,8 +470,23 @@ MlpPlans mlp_plans(int E, int R, int D, int M, bool ragged, long long items) {
   static_assert(CfgDownNarrow::BM == CfgDown::BM, "row tiles of the narrow kernel");
   m.down_bytes = bytes(m.down);
   m.planned = m.up_bytes + m.down_bytes > 0;
-  if (m.up_rows >= 0) m.up_bytes = 0;
-  if (m.down_rows >= 0) m.down_bytes = 0;
+  // What the small tiles need of a plan: no less room than the large tiles' plan, so that a planned product's
+  // workspace is large enough whichever of the two it takes.
+  const auto own_plan = [&](int tile, int N, GemmGeom& g, int& bm, size_t& plan_bytes) {
+    if (tile < 0) return;
+    const size_t large = plan_bytes;
+    plan_bytes = 0;
+    if (!is_mid_tile(tile)) return;
+    with_mid_tile(tile, [&](auto cfg) {
+      using Cfg = decltype(cfg);
+      g = tile_geometry(Cfg::BM, Cfg::BN, Cfg::kBlocksPerCu, E, R, N);
+      bm = Cfg::BM;
+    });
+    const size_t own = mid_tile_planned(E, R, bm) ? bytes(g) : 0;
+    if (own > 0) plan_bytes = std::max(own, large);
+  };
+  own_plan(m.up_rows, M, m.up, m.up_bm, m.up_bytes);
+  own_plan(m.down_rows, D, m.down, m.down_bm, m.down_bytes);
   if (m.down_kernel == kDownShared && m.down_rows < 0)
     m.streamk_bytes = align256(StreamKWorkspace<CfgDownPersistent>::kBytes);
   return m;
@@ -581,7 +594,7 @@ MlpWorkspace mlp_workspace(const VmoeExpertMlpParams* p) {
     if (w.m.streamk_bytes) w.streamk = ws;
     ws += w.m.streamk_bytes;
     if (w.plan_up != nullptr || w.plan_down != nullptr) {
-      w.ga = RaggedGeom{CfgUp::BM, w.m.up.tiles_n, w.m.up.panel_rows,
+      w.ga = RaggedGeom{w.m.up_bm, w.m.up.tiles_n, w.m.up.panel_rows,
                         w.plan_up ? (int)(w.m.up.ragged_slots * kNumXcd) : 0,
                         reinterpret_cast<PlanEntry*>(w.plan_up)};
       w.gb = RaggedGeom{w.m.down_bm, w.m.down.tiles_n, w.m.down.panel_rows,
@@ -658,7 +671,7 @@ static int run_expert_mlp(const VmoeExpertMlpParams* p, vmoe_stream_t stream_, b
     if (m.up_rows >= 0) {
       auto up = tanh_gelu ? launch_gemm_bf16_rows<kEpiBiasGeluTanh> : launch_gemm_bf16_rows<kEpiBiasGeluErf>;
       rc = up(m.up_rows, (const bf16_t*)p->x, (const bf16_t*)w0t, w.b0, (bf16_t*)hidden,
-              p->E, p->R, p->M, p->D, stream, p->rows_per_expert, p->x_rows, p->num_items,
+              p->E, p->R, p->M, p->D, stream, p->rows_per_expert, plan_up, p->x_rows, p->num_items,
               plan_down != nullptr ? plan_ref_of(m.down, plan_down, m.down_bm, p->E, p->R) : no_plan,
               clear, SK::kFlags, status);
     } else if (tanh_gelu)
@@ -675,8 +688,8 @@ static int run_expert_mlp(const VmoeExpertMlpParams* p, vmoe_stream_t stream_, b
     if (m.down_rows >= 0)
       return launch_gemm_bf16_rows<kEpiBias>(
           m.down_rows, (const bf16_t*)hidden, (const bf16_t*)w1t, w.b1, (bf16_t*)p->out,
-          p->E, p->R, p->D, p->M, stream, p->rows_per_expert, nullptr, 0,
-          plan_up != nullptr ? plan_ref_of(m.up, plan_up, CfgUp::BM, p->E, p->R) : no_plan, nullptr, 0, status);
+          p->E, p->R, p->D, p->M, stream, p->rows_per_expert, plan_down, nullptr, 0,
+          plan_up != nullptr ? plan_ref_of(m.up, plan_up, m.up_bm, p->E, p->R) : no_plan, nullptr, 0, status);
     switch (m.down_kernel) {
       case kDownShared:
         return launch_gemm_bf16_persistent<CfgDownPersistent, kEpiBias>(

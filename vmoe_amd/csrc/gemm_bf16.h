@@ -1666,21 +1666,20 @@ struct GemmGeom {
   long long ragged_slots;   // workgroups per die of a planned (ragged) launch
 };
 
-template <typename Cfg>
-GemmGeom gemm_geometry(int batch, int R, int N, int Kd) {
+// Tiles of bm x bn, per_cu workgroups of which share a CU.
+inline GemmGeom tile_geometry(int bm, int bn, int per_cu, int batch, int R, int N) {
   GemmGeom g{};
-  g.fast = !(Kd % Cfg::BK != 0 || (uint64_t)(R > N ? R : N) * Kd * 2 >= (1ull << 32));
-  if (!g.fast) return g;
-  g.tiles_m = (R + Cfg::BM - 1) / Cfg::BM;
-  g.tiles_n = (N + Cfg::BN - 1) / Cfg::BN;
+  g.fast = true;
+  g.tiles_m = (R + bm - 1) / bm;
+  g.tiles_n = (N + bn - 1) / bn;
   g.tiles = (long long)batch * g.tiles_m * g.tiles_n;
   g.tiles_per_xcd = (int)((g.tiles + kNumXcd - 1) / kNumXcd);
   // Tile order inside a batch: panels of `panel_rows` row tiles, swept column tile
   // by column tile.  The tiles that run together on one die (32 compute units)
   // then form a block of about panel_rows x (concurrent / panel_rows) tiles, whose
   // operand footprint per tile is smallest when the block's A and B bytes match.
-  const double concurrent = 32.0 * Cfg::kBlocksPerCu;
-  int panel_rows = (int)(std::sqrt(concurrent * Cfg::BN / Cfg::BM) + 0.5);
+  const double concurrent = 32.0 * per_cu;
+  int panel_rows = (int)(std::sqrt(concurrent * bn / bm) + 0.5);
   if (panel_rows < 1) panel_rows = 1;
   if (panel_rows > g.tiles_m) panel_rows = g.tiles_m;
   const int panels = (g.tiles_m + panel_rows / 2) / panel_rows > 0 ? (g.tiles_m + panel_rows / 2) / panel_rows : 1;
@@ -1689,6 +1688,12 @@ GemmGeom gemm_geometry(int batch, int R, int N, int Kd) {
   const long long share_max = ((long long)batch * g.tiles_m + kNumXcd - 1) / kNumXcd;
   g.ragged_slots = share_max * g.tiles_n;
   return g;
+}
+
+template <typename Cfg>
+GemmGeom gemm_geometry(int batch, int R, int N, int Kd) {
+  if (Kd % Cfg::BK != 0 || (uint64_t)(R > N ? R : N) * Kd * 2 >= (1ull << 32)) return GemmGeom{};
+  return tile_geometry(Cfg::BM, Cfg::BN, Cfg::kBlocksPerCu, batch, R, N);
 }
 
 // The plan of a launch with geometry g as its kernel takes it (tag: what the planner wrote

@@ -1,6 +1,7 @@
-// bf16 expert products over few rows per batch: C[b] (R x N) = epi(A[b] (R x Kd) . Bt[b]^T + bias[b]).
+// bf16 expert products over few rows per batch: C[b] (R x N) = epi(A[b] (R x Kd) . Bt[b]^T + bias[b]), and the
+// choice between the tiles of this kernel, of gemm_bf16_mid.h and of gemm_bf16_stream.h.
 //
-// What bounds them.  With a few dozen or hundred rows per expert the 128 x 256 and 256 x 256 tiles
+// What bounds them.  With a few dozen rows per expert the 128 x 256 and 256 x 256 tiles
 // of gemm_bf16.h make a handful of workgroups that each walk all of k: the second product over one
 // image (8 experts x 52 rows x 768 x 3072) was 24 tiles on 256 CUs and 86 us, for 38 MB of weights
 // that take 6 us to read.  Small tiles fill the chip; what they cost is operand bytes per flop, and
@@ -9,16 +10,17 @@
 // first product of the same layer).  Each shape therefore wants the largest tile that still
 // occupies every CU, and the tile is chosen from a table of measured constants (RowsTile below).
 //
-// One workgroup of 4 or 8 waves per tile; no launch plan (a workgroup past its batch's count leaves
-// after one scalar load).  Operands go global memory -> LDS by DMA, 8 rows x 128 bytes per request,
-// into a ring of S stages of 64 KT k; the 16-byte pieces of a row are XOR-swizzled so that fragment
+// gemm_bf16_rows_kernel: tiles of 32 x 32 to 32 x 128, one workgroup of 4 waves each; no launch plan (a workgroup past
+// its batch's count leaves after one scalar load).  Operands go global memory -> LDS by DMA, 8 rows x 128 bytes per
+// request, into a ring of S stages of 64 KT k; the 16-byte pieces of a row are XOR-swizzled so that fragment
 // reads meet no bank conflict; fragments of stage t + 1 are read while stage t is multiplied; one
-// barrier per stage.  The small tiles take 128 k per stage (KT = 2): with one row block per wave a
+// barrier per stage.  The smallest take 128 k per stage (KT = 2): with one row block per wave a
 // stage's MFMAs are shorter than the barrier and the LDS latency around them (second product of one
 // 196-token image, 32 x 32 tiles: 13.2 us with KT = 1, 9.6 with KT = 2).
 #ifndef VMOE_GEMM_BF16_ROWS_H_
 #define VMOE_GEMM_BF16_ROWS_H_
 #include "gemm_bf16.h"
+#include "gemm_bf16_mid.h"
 #include "gemm_bf16_stream.h"
 
 namespace vmoe {
@@ -40,56 +42,55 @@ struct RowsCfg {
   static_assert(S >= 2 && S * kIssues < 64, "vmcnt is a 6-bit counter");
 };
 
-// Tiles that a launch may take, and what the choice between them is made from: the time of a
-// workgroup's round is fix + stages x max(lat, bytes of a 64-wide k tile of the workgroups that
-// share the CU / rate).  Fitted to a sweep over 30 shapes (1 - 64 experts, 16 - 6272 rows, widths
-// 192 - 4096) of both products.  Estimate against measured time of 30 such shapes on all eight tiles: rms 11 %
-// (first product) and 13 % (second); the tile that the choice takes, the large ones among them, is
-// on average 2.5 and 4 % slower than the fastest, 17 and 40 % at worst (577 rows x 4096 x 1024: 28.9 us
-// on 64 x 64, 20.6 on 64 x 32).
+// Tiles that a launch may take (VMOE_ROW_TILES counts them, kStreamTiles and kMoreTiles on behind each other), and
+// what the choice between them is made from.  A workgroup's round takes fix (+ gelu) microseconds and step1 per
+// 64 k, step2 where two of them share the CU; a launch cannot beat its bytes at tbs TB/s nor its flops
+// at pflops.  Fitted to 230 random shapes, both products (1 - 128 experts, 24 - 50 000 rows, widths 192 - 1 024,
+// weights from memory): rms 6 - 12 % per tile.  The kernel that the choice takes, the tile-walking and the large ones
+// among them, is on average 1.4 % slower than the fastest; the tiles below 64 x 64
+// are gemm_bf16_rows_kernel's, the others gemm_bf16_mid_kernel's.
 struct RowsTile {
   int bm, bn, per_cu;
-  double fix_us, lat_us, gbs;
+  double fix, step1, step2, gelu, tbs, pflops;
 };
 constexpr RowsTile kRowsTiles[] = {
-    {32, 32, 2, 1.7, 0.09, 78},  {64, 32, 2, 2.0, 0.13, 79},  {32, 64, 2, 1.9, 0.14, 75},
-    {64, 64, 2, 2.1, 0.28, 66},  {32, 128, 2, 1.9, 0.29, 69}, {64, 128, 2, 2.9, 0.30, 61},
-    {128, 64, 2, 2.4, 0.30, 55}, {128, 128, 1, 5.2, 0.30, 58}};
+    {32, 32, 2, 1.41, 0.13, 0.19, 0, 4.2, 0.33},    {64, 32, 2, 1.55, 0.19, 0.30, 0, 4.2, 0.43},
+    {32, 64, 2, 1.33, 0.21, 0.31, 0.1, 4.2, 0.63},  {64, 64, 2, 1.05, 0.30, 0.37, 0.6, 4.0, 0.51},
+    {32, 128, 2, 1.14, 0.35, 0.55, 0.5, 4.3, 2.5},  {64, 128, 2, 1.20, 0.41, 0.62, 0.8, 4.4, 0.86},
+    {96, 64, 2, 1.00, 0.36, 0.50, 1.0, 4.5, 0.56},  {128, 128, 1, 1.61, 0.50, 0, 2.1, 4.4, 0.79}};
 constexpr int kNumRowsTiles = sizeof(kRowsTiles) / sizeof(kRowsTiles[0]);
-constexpr RowsTile kFirstProductTile = {128, 256, 2, 4.7, 0.30, 45};     // gemm_bf16_mixed_kernel
+constexpr RowsTile kMoreTiles[] = {
+    {96, 128, 2, 0.75, 0.60, 0.88, 1.7, 4.5, 0.91}, {128, 128, 2, 1.09, 0.65, 0.97, 2.1, 4.5, 0.92},
+    {128, 192, 1, 2.13, 0.69, 0, 2.7, 4.5, 0.89},   {256, 192, 1, 2.46, 1.11, 0, 4.6, 3.5, 0.89}};
+constexpr int kNumMoreTiles = sizeof(kMoreTiles) / sizeof(kMoreTiles[0]);
+// The large tiles in the same terms: the first product's (gemm_bf16_mixed_kernel, and gemm_bf16_kernel where k is no
+// multiple of 64), and the second one's eight waves on 256 and on 192 columns.
+constexpr RowsTile kFirstProductTile = {128, 256, 2, 2.98, 1.12, 1.66, 2.2, 4.3, 2.5};
+constexpr RowsTile kFirstProductK32Tile = {128, 256, 2, 1.28, 1.45, 2.25, 0.8, 4.3, 2.5};
+constexpr RowsTile kEightWavesTile = {256, 256, 1, 8.00, 1.23, 0, 0, 5.6, 1.87};
+constexpr RowsTile kNarrowTile = {256, 192, 1, 3.69, 0.87, 0, 0, 4.2, 1.34};
 
-// Time in microseconds of a product on tiles of this kind; the memory term is what the weights
-// and rows cost where nothing of them is cached (4.4 TB/s over launches of this length).
-// whole_pairs: as gemm_bf16_rows_kernel deals them, all row tiles of a (batch, column tile) pair to one
-// die, whose rounds then count (a launch of two pairs runs on two dies: 10 482 rows x 832 x 224 on
-// 128 x 128 tiles take 37 us, with the large tiles 16); else the tiles fall evenly on all CUs.
-inline double product_us(const RowsTile& t, int batch, int R, int N, int Kd, bool whole_pairs) {
+// Time in microseconds of a product on tiles of this kind.
+// whole_pairs: all row tiles of a (batch, column tile) pair run on one die, whose rounds then count (a launch of
+// two pairs runs on two dies); else the tiles fall evenly on the dies.
+inline double product_us(const RowsTile& t, int batch, int R, int N, int Kd, bool gelu, bool whole_pairs) {
   const double row_tiles = (R + t.bm - 1) / t.bm, pairs = (double)batch * ((N + t.bn - 1) / t.bn);
-  const double tiles = whole_pairs ? std::ceil(pairs / kNumXcd) * row_tiles : pairs * row_tiles;
-  const double full = (double)kCusPerXcd * t.per_cu * (whole_pairs ? 1 : kNumXcd);
+  const double on_die = whole_pairs ? std::ceil(pairs / kNumXcd) * row_tiles : std::ceil(pairs * row_tiles / kNumXcd);
+  const double full = (double)kCusPerXcd * t.per_cu;
+  const double fix = t.fix + (gelu ? t.gelu : 0);
   const int nk = (Kd + 63) / 64;
-  auto round = [&](double on_a_cu) {
-    return t.fix_us + nk * std::fmax(t.lat_us, on_a_cu * (t.bm + t.bn) * 0.128 / t.gbs);
-  };
-  const double rounds = std::floor(tiles / full), rest = tiles - rounds * full;
-  const double busy = rounds * round(t.per_cu) + (rest > 0 ? round(std::ceil(rest / (full / t.per_cu))) : 0);
-  const double memory = 2.0 * batch * ((double)N * Kd + (double)R * (Kd + N)) / 4.4e6;
+  const double one = fix + nk * t.step1, two = 1.35 * fix + nk * t.step2;
+  const double rounds = std::floor(on_die / full), rest = on_die - rounds * full;
+  const double busy = rounds * (t.per_cu == 2 ? two : one) + (rest > kCusPerXcd ? two : rest > 0 ? one : 0);
+  const double weights = (double)batch * N * Kd, memory = 2e-6 * (weights + (double)batch * R * (Kd + N)) / t.tbs;
+  const double matrix = 2e-9 * weights * R / t.pflops;
   // (their 4-norm.  A layer's calls estimate every tile of both products several times: with pow() that was
   // 11 us of the host's 60 on one image.)
-  return 2.9 + std::sqrt(std::sqrt(busy * busy * busy * busy + memory * memory * memory * memory));
+  const double b2 = busy * busy, m2 = memory * memory, f2 = matrix * matrix;
+  return 2 + std::sqrt(std::sqrt(b2 * b2 + m2 * m2 + f2 * f2));
 }
 
-// The tile (index into kRowsTiles) that the table expects to be fastest.
-inline int best_rows_tile(int batch, int R, int N, int Kd, double* us) {
-  int best = -1;
-  for (int i = 0; i < kNumRowsTiles; ++i) {
-    const double t = product_us(kRowsTiles[i], batch, R, N, Kd, true);
-    if (best < 0 || t < *us) { best = i; *us = t; }
-  }
-  return best;
-}
-
-// The tiles of gemm_bf16_stream_kernel (VMOE_ROW_TILES counts them on behind kRowsTiles), and what the choice
+// The tiles of gemm_bf16_stream_kernel, and what the choice
 // is made from: a CU takes its tiles one after the other at step_us per 64 k, with the GELU's or the plain
 // epilogue behind each, and the launch cannot beat its weights at w_tbs plus its rows, once per column
 // tile, at a_tbs.  Fitted to 106 random shapes (4 - 128 experts, 12 - 128 rows, widths 384 - 4096; either product):
@@ -122,33 +123,65 @@ inline bool stream_tile_ok(int i, int batch, int R, int Kd, bool ragged) {
   });
 }
 
-// The tile (kNumRowsTiles + index into kStreamTiles) that should run the product in less than `us`
-// microseconds, the time of the kernel that has it otherwise, or -1.  It has to win by 8 %: the estimates of the
-// other kernels are off by 10 - 20 %, mostly upwards.  Below 24 rows most of a tile is padding and the 32-row
-// tiles win.  Over the same shapes the choice takes 8 380 us where the other kernels take 9 400 and the
-// fastest tile of all would take 8 320; 11 of 212 products get slower, by 11 % at worst.
-inline int best_stream_tile(int batch, int R, int N, int Kd, bool ragged, bool gelu, double us) {
-  if (R < 24) return -1;
-  int best = -1;
-  us *= 0.92;
-  for (int i = 0; i < kNumStreamTiles; ++i) {
-    if (!stream_tile_ok(i, batch, R, Kd, ragged)) continue;
-    const StreamTile& s = kStreamTiles[i];
-    const double units = (double)batch * ((N + s.bn - 1) / s.bn);
-    const double rounds = std::ceil(std::ceil(units / kNumXcd) / kCusPerXcd);
-    const double busy = s.fix_us + rounds * ((Kd + 63) / 64 * s.step_us + (gelu ? s.gelu_us : s.plain_us));
-    const double memory = s.lat_us + 2e-6 * Kd * ((double)batch * N / s.w_tbs + units * s.bm / s.a_tbs);
-    const double t = std::sqrt(std::sqrt(busy * busy * busy * busy + memory * memory * memory * memory));
-    if (t < us) { us = t; best = kNumRowsTiles + i; }
-  }
-  return best;
+// Time of tile i of kStreamTiles, 1e30 where the kernel does not take the product.  (Below 24 rows most of a tile is
+// padding and the 32-row tiles win.)
+inline double stream_us(int i, int batch, int R, int N, int Kd, bool ragged, bool gelu) {
+  if (R < 24 || !stream_tile_ok(i, batch, R, Kd, ragged)) return 1e30;
+  const StreamTile& s = kStreamTiles[i];
+  const double units = (double)batch * ((N + s.bn - 1) / s.bn);
+  const double rounds = std::ceil(std::ceil(units / kNumXcd) / kCusPerXcd);
+  const double busy = s.fix_us + rounds * ((Kd + 63) / 64 * s.step_us + (gelu ? s.gelu_us : s.plain_us));
+  const double memory = s.lat_us + 2e-6 * Kd * ((double)batch * N / s.w_tbs + units * s.bm / s.a_tbs);
+  return std::sqrt(std::sqrt(busy * busy * busy * busy + memory * memory * memory * memory));
 }
+
+constexpr int kFirstMoreTile = kNumRowsTiles + kNumStreamTiles;
+inline bool is_mid_tile(int i) {
+  return i == 3 || (i >= 5 && i < kNumRowsTiles) || (i >= kFirstMoreTile && i < kFirstMoreTile + kNumMoreTiles);
+}
+// f(MidCfg of tile i).
+template <typename F>
+inline auto with_mid_tile(int i, F&& f) {
+  switch (i) {
+    case 3: return f(MidCfg<64, 64, 2, 2, 2, 2, 2>{});
+    case 5: return f(MidCfg<64, 128, 2, 2, 3, 2, 1>{});
+    case 6: return f(MidCfg<96, 64, 2, 2, 2, 2, 2>{});
+    case 7: return f(MidCfg<128, 128, 2, 4, 4, 1, 1>{});
+    case kFirstMoreTile: return f(MidCfg<96, 128, 2, 2, 2, 2, 1>{});
+    case kFirstMoreTile + 1: return f(MidCfg<128, 128, 2, 2, 2, 2, 1>{});
+    case kFirstMoreTile + 2: return f(MidCfg<128, 192, 4, 2, 3, 1, 1>{});
+    default: return f(MidCfg<256, 192, 4, 2, 2, 1, 1>{});
+  }
+}
+
+// Whether a ragged launch of a tile of gemm_bf16_mid.h has a plan: with two row tiles per die and more.  Below that
+// (batch, column tile) pairs go round the dies, which is as even.
+inline bool mid_tile_planned(int batch, int R, int bm) { return (long long)batch * ((R + bm - 1) / bm) >= 2 * kNumXcd; }
 
 // Whether the kernel takes the operands: whole 16-byte pieces, 31-bit byte offsets inside a batch.
 inline bool rows_gemm_ok(int R, int N, int Kd, long long items) {
   const uint64_t lim = 1ull << 31;
   return N % 8 == 0 && Kd % 8 == 0 && (uint64_t)R * Kd * 2 < lim && (uint64_t)N * Kd * 2 < lim &&
          (uint64_t)items * Kd * 2 < lim;
+}
+
+// The tile that should run the product in less than `us` microseconds, the time of the large tiles, or -1.
+inline int best_tile(int batch, int R, int N, int Kd, long long items, bool ragged, bool gelu, double us) {
+  int best = -1;
+  auto take = [&](int i, double t) {
+    if (t < us) { us = t; best = i; }
+  };
+  const bool mid_ok = mid_gemm_ok(batch, R, N, Kd, items);
+  auto take_tile = [&](int i, const RowsTile& t) {
+    const bool mid = is_mid_tile(i);
+    if (!mid || mid_ok)
+      take(i, product_us(t, batch, R, N, Kd, gelu, !mid || (ragged && !mid_tile_planned(batch, R, t.bm))));
+  };
+  for (int i = 0; i < kNumRowsTiles; ++i) take_tile(i, kRowsTiles[i]);
+  for (int i = 0; i < kNumMoreTiles; ++i) take_tile(kFirstMoreTile + i, kMoreTiles[i]);
+  // (8 % ahead: no tile walker where another kernel is as good)
+  for (int i = 0; i < kNumStreamTiles; ++i) take(kNumRowsTiles + i, 1.08 * stream_us(i, batch, R, N, Kd, ragged, gelu));
+  return best;
 }
 
 // `guard`: the plan of the other product of the call, where that one has a plan: a launch whose
@@ -363,16 +396,22 @@ int launch_rows_tile(const bf16_t* A, const bf16_t* Bt, const bf16_t* bias, bf16
   return launch_status();
 }
 
-// `tile`: index into kRowsTiles, behind them into kStreamTiles; waves, stages and 64-wide k tiles per stage of each.
+// `tile`: index into kRowsTiles, behind them into kStreamTiles, behind those into kMoreTiles.  `plan`: the launch
+// plan of a ragged product on a tile of gemm_bf16_mid_kernel, or none.
 template <int EPI>
 int launch_gemm_bf16_rows(int tile, const bf16_t* A, const bf16_t* Bt, const bf16_t* bias, bf16_t* C,
-                          int batch, int R, int N, int Kd, hipStream_t stream, const int32_t* rows,
+                          int batch, int R, int N, int Kd, hipStream_t stream, const int32_t* rows, const int4* plan,
                           const int32_t* a_rows, int a_items, PlanRef guard, int32_t* clear,
                           int clear_count, int32_t* status) {
   auto run = [&](auto cfg) {
     return launch_rows_tile<decltype(cfg), EPI>(A, Bt, bias, C, batch, R, N, Kd, stream, rows, a_rows,
                                                 a_items, guard, clear, clear_count, status);
   };
+  if (is_mid_tile(tile))
+    return with_mid_tile(tile, [&](auto cfg) {
+      return launch_mid_tile<decltype(cfg), EPI>(A, Bt, bias, C, batch, R, N, Kd, stream, rows, plan, a_rows,
+                                                 a_items, guard, clear, clear_count, status);
+    });
   if (tile >= kNumRowsTiles)
     return with_stream_tile(tile - kNumRowsTiles, [&](auto cfg) {
       return launch_gemm_bf16_stream<decltype(cfg), EPI>(A, Bt, bias, C, batch, R, N, Kd, stream, rows, a_rows,
@@ -382,11 +421,7 @@ int launch_gemm_bf16_rows(int tile, const bf16_t* A, const bf16_t* Bt, const bf1
     case 0: return run(RowsCfg<32, 32, 2, 2, 4, 2>{});
     case 1: return run(RowsCfg<64, 32, 2, 2, 3, 2>{});
     case 2: return run(RowsCfg<32, 64, 2, 2, 3, 2>{});
-    case 3: return run(RowsCfg<64, 64, 2, 2, 2, 2>{});
     case 4: return run(RowsCfg<32, 128, 1, 4, 4, 1>{});
-    case 5: return run(RowsCfg<64, 128, 2, 2, 3, 1>{});
-    case 6: return run(RowsCfg<128, 64, 2, 2, 3, 1>{});
-    case 7: return run(RowsCfg<128, 128, 2, 4, 4, 1>{});
   }
   return VMOE_E_UNSUPPORTED;
 }
