@@ -392,6 +392,14 @@ int vmoe_compact_rows_planned(const VmoeCompactRowsParams* c, const VmoeExpertMl
                               vmoe_stream_t stream);
 int vmoe_expert_mlp_planned(const VmoeExpertMlpParams* p, vmoe_stream_t stream);
 
+/* A dense layer alone (the projections of vmoe/nn/vit_moe.py:166-174, the patch embedding as rows):
+ *   out[e] (R, M) = x[e] (R, D) . w[e] + b0[e],  rounded once.
+ * Of the MLP's parameter block x, out, b0, E, R, D, M, dtype are read and the weights: float32 w0 (E, D, M), bf16
+ * w0t (E, M, D).  No workspace.  float32: D and M multiples of 4, products as sums of three bfloat16 values per
+ * operand (or, with gelu = VMOE_MLP_F32_PRODUCTS, VMOE_E_UNSUPPORTED); bf16: multiples of 8, operands of one e
+ * within 2 GiB; x and out 16-byte aligned.  VMOE_E_UNSUPPORTED with rows_per_expert or x_rows. */
+int vmoe_dense(const VmoeExpertMlpParams* p, vmoe_stream_t stream);
+
 /* Status words of the expert MLP calls made on p->workspace (no counterpart in the
  * reference).  *status receives the DEVICE address of VMOE_MLP_STATUS_WORDS int32 inside the
  * workspace, or null for float32 (those kernels keep no such state); nothing is launched.

@@ -373,3 +373,39 @@ def test_model_from_checkpoint_files(vit_moe, tmp_path):
   model = vit_moe.VisionTransformerMoe(**product_config(SMALL, O.F32))
   got, _ = model.apply({"params": C.to_device(sparse, dev())}, tree_to_dev(images))
   assert_close(to_np(got), want, 2e-4, "logits from restored parameters")
+
+
+# ------------------------------------------------------------------ dense layers
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,D,M", [(1, 8, 8), (63, 72, 24), (193, 136, 520), (1569, 200, 264), (2050, 776, 1000)])
+def test_dense_against_64_bits(rows, D, M, dtype):
+  """vmoe_dense at rows, k and columns that end inside its tiles: one rounding of the sum and the bias
+  (bfloat16: half a unit in the last place of eight bits, 2^-8, and float32 sums; float32: sums of D products)."""
+  from vmoe_amd import kernels as K
+  gen = torch.Generator(device=dev()).manual_seed(rows)
+  mk = lambda *s: torch.randn(s, generator=gen, device=dev()).to(dtype)
+  x, w, b = mk(rows, D), mk(D, M) * D ** -0.5, mk(M)
+  layout = w if dtype == torch.float32 else w.t().contiguous()
+  for bias in (b, None):
+    want = x.double() @ w.double() + (0 if bias is None else bias.double())
+    got = K.dense(x, layout, bias).double()
+    size = x.double().abs() @ w.double().abs() + 1
+    bound = size * D ** 0.5 * 2.0 ** -23 + (want.abs() * 2.0 ** -8 if dtype == torch.bfloat16 else 0)
+    assert bool(((got - want).abs() <= bound).all())
+
+
+def test_dense_stands_aside_where_torch_has_to_see_the_product(vit_moe):
+  """Gradients, functorch transforms and autocast take the library's product."""
+  x = torch.randn(1301, 1000, device=dev())
+  w, b = torch.randn(1000, 1000, device=dev()), torch.randn(1000, device=dev())
+  plain = vit_moe._affine(x, w, b)
+  leaf = w.clone().requires_grad_()
+  out = vit_moe._affine(x, leaf, b)
+  out.sum().backward()
+  assert torch.allclose(leaf.grad, x.sum(0)[:, None].expand(-1, 1000), rtol=1e-3, atol=1e-2)
+  # (sums of 1 000 products of unit variance in float32, in two orders)
+  assert torch.allclose(plain, out, rtol=1e-4, atol=1e-3)
+  both = torch.vmap(lambda t: vit_moe._affine(t, w, b))(x[None])
+  assert torch.allclose(plain, both[0], rtol=1e-4, atol=1e-3)
+  _, tangent = torch.func.jvp(lambda t: vit_moe._affine(t, w, b), (x,), (x,))
+  assert torch.allclose(tangent, plain - b, rtol=1e-4, atol=2e-3)

@@ -740,6 +740,29 @@ extern "C" int vmoe_expert_mlp_planned(const VmoeExpertMlpParams* p, vmoe_stream
   return run_expert_mlp(p, stream, true);
 }
 
+extern "C" int vmoe_dense(const VmoeExpertMlpParams* p, vmoe_stream_t stream_) {
+  if (p == nullptr || p->x == nullptr || p->out == nullptr) return VMOE_E_NULL;
+  if (p->E < 1 || p->R < 1 || p->D < 1 || p->M < 1) return VMOE_E_SHAPE;
+  if (p->dtype != VMOE_F32 && p->dtype != VMOE_BF16) return VMOE_E_DTYPE;
+  if ((p->dtype == VMOE_F32 ? p->w0 : p->w0t) == nullptr) return VMOE_E_NULL;
+  if (p->rows_per_expert != nullptr || p->x_rows != nullptr || (p->gelu & VMOE_MLP_F32_PRODUCTS) != 0)
+    return VMOE_E_UNSUPPORTED;
+  const int step = p->dtype == VMOE_F32 ? 4 : 8;
+  if (p->D % step != 0 || p->M % step != 0 || !aligned16(p->x) || !aligned16(p->out)) return VMOE_E_ALIGN;
+  if ((int64_t)p->E * p->R >= INT32_MAX) return VMOE_E_OVERFLOW;
+  hipStream_t stream = as_stream(stream_);
+  if (p->dtype == VMOE_F32)
+    return launch_gemm_f32_split<kEpiBias>(best_split_tile(p->E, p->R, p->M, p->D), (const float*)p->x, (const float*)p->w0,
+                                           (const float*)p->b0, (float*)p->out, p->E, p->R, p->M, p->D, stream, nullptr,
+                                           nullptr, 0);
+  if (!aligned16(p->w0t)) return VMOE_E_ALIGN;
+  if (!rows_gemm_ok(p->R, p->M, p->D, 0)) return VMOE_E_UNSUPPORTED;
+  const int tile = best_tile(p->E, p->R, p->M, p->D, 0, false, false, 1e30, false);
+  return launch_gemm_bf16_rows<kEpiBiasOnce>(tile, (const bf16_t*)p->x, (const bf16_t*)p->w0t, (const bf16_t*)p->b0,
+                                             (bf16_t*)p->out, p->E, p->R, p->M, p->D, stream, nullptr, nullptr, nullptr, 0,
+                                             PlanRef{nullptr, 0, 0}, nullptr, 0, nullptr);
+}
+
 extern "C" int vmoe_expert_mlp_status(const VmoeExpertMlpParams* p, const int32_t** status) {
   if (status == nullptr) return VMOE_E_NULL;
   *status = nullptr;

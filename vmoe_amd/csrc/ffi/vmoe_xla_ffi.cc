@@ -487,6 +487,23 @@ XLA_FFI_DEFINE_HANDLER_SYMBOL(VmoeExpertMlp, ExpertMlpImpl,
                                   .Attr<bool>("packed").Attr<bool>("has_bias").Attr<bool>("ragged")
                                   .Attr<bool>("gather").Attr<int32_t>("gelu"));
 
+// x (E,R,D), w (E,D,M) float32 or, transposed, (E,M,D) bfloat16, b (E,M) -> out (E,R,M)
+static ffi::Error DenseImpl(hipStream_t stream, Any x, Any w, Any b, AnyOut out, bool has_bias) {
+  VmoeExpertMlpParams p{};
+  p.x = x.untyped_data();
+  p.dtype = DType(x.element_type());
+  if (p.dtype == VMOE_BF16) p.w0t = w.untyped_data();
+  else p.w0 = w.untyped_data();
+  p.b0 = has_bias ? b.untyped_data() : nullptr;
+  p.out = out->untyped_data();
+  p.E = Dim(x, 0); p.R = Dim(x, 1); p.D = Dim(x, 2);
+  p.M = (int32_t)out->dimensions()[2];
+  return Status(vmoe_dense(&p, stream), "vmoe_dense");
+}
+XLA_FFI_DEFINE_HANDLER_SYMBOL(VmoeDense, DenseImpl,
+                              ffi::Ffi::Bind().Ctx<Stream>().Arg<Any>().Arg<Any>().Arg<Any>().Ret<Any>()
+                                  .Attr<bool>("has_bias"));
+
 // The MLP with its launch plans already in `workspace` (written by vmoe_compact_rows_planned
 // for the same shapes): bind `workspace` as a result that aliases the operand holding them
 // (input_output_aliases).  Operands and attributes as VmoeExpertMlp with ragged = gather = true.

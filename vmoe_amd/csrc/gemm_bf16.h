@@ -46,7 +46,8 @@
 
 namespace vmoe {
 
-enum { kEpiBias = 0, kEpiBiasGeluTanh = 1, kEpiBiasGeluErf = 2 };
+// (3 is taken by the float32 products; kEpiBiasOnce: sum and bias are rounded once, as a library's product does)
+enum { kEpiBias = 0, kEpiBiasGeluTanh = 1, kEpiBiasGeluErf = 2, kEpiBiasOnce = 4 };
 
 // f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>), in order: a loop whose
 // index is a constant in the body (register arrays, if constexpr).
@@ -86,6 +87,7 @@ __device__ __forceinline__ float apply_epilogue(float acc, float bias, bool has_
 // by a shift and a mask, instead of a conversion and a shift per element.
 template <int EPI, bool HAS_BIAS>
 __device__ __forceinline__ uint32_t epilogue_pair(float a0, float a1, float b0, float b1) {
+  if (EPI == kEpiBiasOnce) return HAS_BIAS ? pack_bf16x2(a0 + b0, a1 + b1) : pack_bf16x2(a0, a1);
   uint32_t p = pack_bf16x2(a0, a1);
   if (HAS_BIAS) p = pack_bf16x2(bf_lo(p) + b0, bf_hi(p) + b1);
   if (EPI == kEpiBiasGeluTanh) p = pack_bf16x2(gelu_tanh_fast(bf_lo(p)), gelu_tanh_fast(bf_hi(p)));

@@ -166,7 +166,9 @@ inline bool rows_gemm_ok(int R, int N, int Kd, long long items) {
 }
 
 // The tile that should run the product in less than `us` microseconds, the time of the large tiles, or -1.
-inline int best_tile(int batch, int R, int N, int Kd, long long items, bool ragged, bool gelu, double us) {
+// (walkers: whether kStreamTiles are among them)
+inline int best_tile(int batch, int R, int N, int Kd, long long items, bool ragged, bool gelu, double us,
+                     bool walkers = true) {
   int best = -1;
   auto take = [&](int i, double t) {
     if (t < us) { us = t; best = i; }
@@ -180,7 +182,7 @@ inline int best_tile(int batch, int R, int N, int Kd, long long items, bool ragg
   for (int i = 0; i < kNumRowsTiles; ++i) take_tile(i, kRowsTiles[i]);
   for (int i = 0; i < kNumMoreTiles; ++i) take_tile(kFirstMoreTile + i, kMoreTiles[i]);
   // (8 % ahead: no tile walker where another kernel is as good)
-  for (int i = 0; i < kNumStreamTiles; ++i) take(kNumRowsTiles + i, 1.08 * stream_us(i, batch, R, N, Kd, ragged, gelu));
+  for (int i = 0; walkers && i < kNumStreamTiles; ++i) take(kNumRowsTiles + i, 1.08 * stream_us(i, batch, R, N, Kd, ragged, gelu));
   return best;
 }
 
@@ -412,7 +414,9 @@ int launch_gemm_bf16_rows(int tile, const bf16_t* A, const bf16_t* Bt, const bf1
       return launch_mid_tile<decltype(cfg), EPI>(A, Bt, bias, C, batch, R, N, Kd, stream, rows, plan, a_rows,
                                                  a_items, guard, clear, clear_count, status);
     });
-  if (tile >= kNumRowsTiles)
+  if constexpr (EPI == kEpiBiasOnce) {
+    if (tile >= kNumRowsTiles) return VMOE_E_UNSUPPORTED;      // (dense layers leave the tile walkers to the MLPs)
+  } else if (tile >= kNumRowsTiles)
     return with_stream_tile(tile - kNumRowsTiles, [&](auto cfg) {
       return launch_gemm_bf16_stream<decltype(cfg), EPI>(A, Bt, bias, C, batch, R, N, Kd, stream, rows, a_rows,
                                                          a_items, guard, clear, clear_count, status);

@@ -469,6 +469,29 @@ std::tuple<Tensor, Tensor> combine_backward(int64_t stream, const Tensor& dout_,
   return {dy, dw};
 }
 
+// x (..., D) . w + b -> (..., M), rounded once: float32 w (D, M), bfloat16 w transposed (M, D).
+Tensor dense(int64_t stream, const Tensor& x_, const Tensor& w, const OptTensor& b) {
+  if (x_.dim() < 2) need_axes(x_, 2, "x");
+  need_axes(w, 2, "w");
+  need_type_of(w, x_, "w", "x");
+  if (b.has_value()) need_type_of(*b, x_, "bias", "x");
+  const Tensor x = x_.contiguous();
+  const bool f32 = x.scalar_type() == at::kFloat;
+  const int64_t D = x.size(-1), M = w.size(f32 ? 1 : 0);
+  if (w.size(f32 ? 0 : 1) != D)
+    throw py::value_error("w has shape " + shape_of(w) + ", x " + shape_of(x));
+  need_values(b, M, "bias");
+  auto sizes = x.sizes().vec();
+  sizes.back() = M;
+  Tensor out = empty(sizes, x.scalar_type(), x);
+  if (out.numel() == 0) return out;
+  VmoeExpertMlpParams p{};
+  p.x = ptr(x); (f32 ? p.w0 : p.w0t) = ptr(w); p.b0 = ptr(b); p.out = ptr(out);
+  p.E = 1; p.R = (int32_t)(x.numel() / D); p.D = (int32_t)D; p.M = (int32_t)M; p.dtype = dtype_code(x);
+  check(vmoe_dense(&p, stream_of(stream)), "vmoe_dense");
+  return out;
+}
+
 // -> dx of dispatch.
 Tensor dispatch_backward(int64_t stream, const Tensor& dbuf_, const Tensor& token_slot) {
   need_axes(dbuf_, 2, "dbuf");
@@ -521,6 +544,7 @@ PYBIND11_MODULE(_vmoe_host, m) {
     return torch::wrap_pybind_function_no_gil(&add_layer_norm)(s, r, b, sc, bi, eps, type, w);
   });
   VMOE_DEF(attention);
+  VMOE_DEF(dense);
   m.def("einsum", [](int64_t s, const Tensor& w, const Tensor& d, py::object t, bool dispatch_) {
     return torch::wrap_pybind_function_no_gil(&einsum)(s, w, d, torch::python::detail::py_object_to_dtype(std::move(t)),
                                                        dispatch_);

@@ -651,6 +651,34 @@ def add_layer_norm(residual: torch.Tensor, branch: Optional[torch.Tensor],
   return (res_out if res_out is not None else residual), norm_out
 
 
+def dense_pays(rows: int, D: int, M: int, dtype: torch.dtype) -> bool:
+  """Whether dense() is the faster one for x (rows, D) . w (D, M) beside the library's product.  bfloat16: up to
+  2.8e9 multiply-adds (1 568 x 768 x 2 304: 11.1 us either way, 1 568 x 768 x 768: 7.5 and 9.0, and 17 us less host
+  work; 3 136 x 1 024 x 3 072: 25.5 and 22.2), and over short rows (50 176 x 384 x 384: 28 and 42).  float32: from
+  1.3e9 on (3 136 x 768 x 768: 35 us and 48, 50 176: 306 and 510; 784 x 768 x 768: 16 and 13), where its error
+  against 64 bits is also the smaller one (2.9e-7 and 3.5e-7 at D = 768)."""
+  work = rows * D * M
+  if dtype == torch.bfloat16:
+    return D % 8 == 0 and M % 8 == 0 and 0 < work and (work <= 2.8e9 or D <= 384) and max(rows, M) * D < 1 << 30 and rows * M < 1 << 30
+  return dtype == torch.float32 and D % 4 == 0 and M % 4 == 0 and work >= 1.3e9 and rows < 1 << 31
+
+
+def dense(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor]) -> torch.Tensor:
+  """x (..., D) . w + b -> (..., M), rounded once.  float32: w (D, M), products as sums of three bfloat16
+  values per operand; bfloat16: w (M, D), transposed."""
+  if not H.timed("vmoe_dense"):
+    return H.host().dense(H.raw_stream(), x, w, b)
+  x = x.contiguous()
+  D, f32 = x.shape[-1], x.dtype == torch.float32
+  M = w.shape[1 if f32 else 0]
+  out = torch.empty((*x.shape[:-1], M), dtype=x.dtype, device=x.device)
+  p = H.ExpertMlpParams(x=H.ptr(x), b0=H.ptr(b) if b is not None else None, out=H.ptr(out), E=1,
+                        R=x.numel() // D, D=D, M=M, dtype=H.dtype_code(x.dtype))
+  setattr(p, "w0" if f32 else "w0t", H.ptr(w))
+  H.call("vmoe_dense", p)
+  return out
+
+
 ATTENTION_HEAD_DIM = 64
 
 

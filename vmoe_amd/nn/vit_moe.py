@@ -225,6 +225,15 @@ def _add_layer_norm(residual: Array, branch: Optional[Array], p: Mapping[str, Ar
   return x, _layer_norm(x, p, dtype, eps)
 
 
+def _affine(x: Array, w: Array, b: Array) -> Array:
+  """x (..., D) . w (D, M) + b in float32: the package's own product where it is the faster one."""
+  D, M = w.shape
+  if (x.dtype == w.dtype == b.dtype and w.is_contiguous() and b.is_contiguous()
+      and K.dense_pays(x.numel() // D, D, M, x.dtype) and module.is_plain(x, w, b)):
+    return K.dense(x, w, b)
+  return torch.addmm(b, x.reshape(-1, D), w).view(*x.shape[:-1], M)
+
+
 class IdentityLayer(module.Module):
   """vit_jax.models_vit.IdentityLayer (exists to name the pre-logits activation)."""
 
@@ -280,20 +289,29 @@ class MultiHeadDotProductAttention(module.Module):
     return {"params": p}
 
   def _proj_weights(self, p, groups, dtype):
-    """For each group of input projections one (sum of H * hd, D) weight and its bias, then the
-    output projection's weight and bias: packed once per set of parameter tensors."""
+    """For each group of input projections one weight, (D, sum of H * hd) in float32 and transposed in any
+    other type, and its bias, then the output projection's weight and bias: packed once per set of
+    parameter tensors."""
     def build():
+      layout = lambda w: (w if dtype == torch.float32 else w.t()).to(dtype).contiguous()
       packed = []
       for names in groups:
-        w = torch.cat([p[n]["kernel"].reshape(p[n]["kernel"].shape[0], -1).t() for n in names])
+        w = torch.cat([p[n]["kernel"].reshape(p[n]["kernel"].shape[0], -1) for n in names], dim=1)
         b = torch.cat([p[n]["bias"].reshape(-1) for n in names])
-        packed += [w.to(dtype).contiguous(), b.to(dtype).contiguous()]
+        packed += [layout(w), b.to(dtype).contiguous()]
       w = p["out"]["kernel"]
-      packed += [w.reshape(w.shape[0] * w.shape[1], -1).t().to(dtype).contiguous(),
-                 p["out"]["bias"].to(dtype)]
+      packed += [layout(w.reshape(w.shape[0] * w.shape[1], -1)), p["out"]["bias"].to(dtype)]
       return packed
     tensors = [p[n][leaf] for n in ("query", "key", "value", "out") for leaf in ("kernel", "bias")]
     return self._packed.get(tensors, (dtype, groups), build)
+
+  @staticmethod
+  def _project(x: Array, w: Array, b: Array) -> Array:
+    """x . w + b for a weight of _proj_weights: the package's own product where it is the faster one."""
+    D, M = w.shape if w.dtype == torch.float32 else reversed(w.shape)
+    if K.dense_pays(x.numel() // D, D, M, w.dtype) and module.is_plain(x, w, b):
+      return K.dense(x, w, b)
+    return torch.nn.functional.linear(x, w.t() if w.dtype == torch.float32 else w, b)
 
   def apply(self, variables, inputs_q: Array, inputs_kv: Optional[Array] = None) -> Array:
     p = variables["params"]
@@ -305,7 +323,7 @@ class MultiHeadDotProductAttention(module.Module):
     Sk = inputs_kv.shape[1]
     hd = p["query"]["kernel"].shape[-1]
     xq = inputs_q.to(dtype)
-    linear = torch.nn.functional.linear
+    linear = self._project
     if inputs_kv is inputs_q:
       w, b, wo, bo = self._proj_weights(p, (("query", "key", "value"),), dtype)
       q, k, v = linear(xq, w, b).view(B, Sq, 3, H, hd).unbind(2)
@@ -590,8 +608,7 @@ class VisionTransformerMoe(module.Module):
       raise ValueError(f"embedding kernel has shape {tuple(k.shape)}, expected "
                        f"{(*self.patch_size, inputs.shape[-1], self.hidden_size)}")
     rows = self._patches(inputs.float())
-    return torch.addmm(p["bias"].float(), rows.reshape(-1, rows.shape[-1]),
-                       k.float().reshape(-1, k.shape[-1])).view(*rows.shape[:3], k.shape[-1])
+    return _affine(rows, k.float().reshape(-1, k.shape[-1]), p["bias"].float())
 
   def apply(self, variables, inputs: Array, rngs=None):
     params = variables["params"]
@@ -611,8 +628,8 @@ class VisionTransformerMoe(module.Module):
       raise ValueError(f"Unknown classifier: {self.classifier!r}")
     if self.representation_size is not None:
       p = params["pre_logits"]
-      x = torch.tanh(torch.addmm(p["bias"].float(), x, p["kernel"].float()))
+      x = torch.tanh(_affine(x, p["kernel"].float(), p["bias"].float()))
     if self.num_classes:
       p = params["head"]
-      return torch.addmm(p["bias"].float(), x, p["kernel"].float()), metrics
+      return _affine(x, p["kernel"].float(), p["bias"].float()), metrics
     return x, metrics
