@@ -195,7 +195,7 @@ int vmoe_top_items_metrics(const VmoeTopItemsParams* p, int32_t* items_minmax, v
  * *num_invalid; slots targeted by more than one item are counted in
  * *num_duplicates (the reference would accumulate them; these kernels do not,
  * callers must treat a non-zero count as an error).  Both counters are device
- * int32 and must be zeroed by the caller. */
+ * int32; the call sets them. */
 typedef struct {
   const int32_t* indices; /* (G, S, K, 2) */
   int32_t* token_slot;    /* out (G, S, K) */

@@ -1195,3 +1195,51 @@ def test_soft_router_reuses_prepared_slot_parameters():
   mu2 = mu.clone() * 2.0 + 0.1                   # another tensor
   for a, b in zip(weights(layer, mu2, scale), fresh(mu2, scale)):
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("data_grad,weights_grad", [(True, True), (True, False), (False, True)])
+def test_native_gradients_are_those_of_the_python_functions(moe, monkeypatch, data_grad, weights_grad):
+  """dispatch and combine recorded natively and as Python functions: the same bits, whichever gradients are asked
+  for, through non-contiguous gradients and saved-tensor hooks."""
+  rng = np.random.default_rng(4)
+  G, S, E, C, k, D = 3, 41, 5, 9, 2, 24
+  pos = rng.permuted(np.tile(np.arange(E * C), (G, 1)), axis=1)[:, :S]            # a slot of its own for every item
+  idx = np.stack([np.stack([pos // C, pos % C], -1), np.full((G, S, 2), E)], 2)    # the second choice is dropped
+  indices = to_dev(idx.astype(np.int32))
+  base_x = torch.randn(G, S, D, device=dev()).to(torch.bfloat16)
+  base_w = torch.rand(G, S, k, device=dev())
+  seen = []
+
+  def both():
+    x, w = base_x.clone().requires_grad_(data_grad), base_w.clone().requires_grad_(weights_grad)
+    d = moe.ExpertIndicesDispatcher(indices, w, E, C)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (seen.append(t.shape), t)[1], lambda t: t):
+      out = d.combine(d.dispatch(x) * 1.5)
+    grad = torch.ones(G, D, S, device=dev(), dtype=torch.bfloat16).transpose(1, 2) * base_x
+    return [out, *torch.autograd.grad(out, [t for t in (x, w) if t.requires_grad], grad)]
+
+  native = both()
+  hooked, seen[:] = list(seen), []
+  from vmoe_amd.nn import module
+  monkeypatch.setattr(module, "is_plain_but_for_gradients", lambda *t: False)
+  python = both()
+  assert hooked == seen and seen
+  for a, b in zip(native, python):
+    assert a.dtype == b.dtype and torch.equal(a, b)
+
+
+def test_dispatcher_checks_new_maps_behind_the_dispatch(moe):
+  """Indices are checked after the dispatch has been issued: negative ones raise in every call, shared slots are
+  added up in the first."""
+  bad = torch.tensor([[[[0, 0]], [[0, -1]]]], dtype=torch.int32, device=dev())
+  d = moe.ExpertIndicesDispatcher(bad, torch.ones(1, 2, 1, device=dev()), 2, 2)
+  x = torch.randn(1, 2, 8, device=dev())
+  for _ in range(2):
+    for call in (lambda: d.dispatch(x), lambda: d.combine(torch.zeros(2, 2, 8, device=dev()))):
+      with pytest.raises(ValueError, match="negative indices"):
+        call()
+  shared = torch.zeros((1, 2, 1, 2), dtype=torch.int32, device=dev())
+  out = moe.ExpertIndicesDispatcher(shared, torch.ones(1, 2, 1, device=dev()), 2, 2).dispatch(x)
+  assert torch.equal(out[0, 0], x[0, 0] + x[0, 1])
+  with pytest.raises(NotImplementedError):
+    moe.ExpertIndicesDispatcher(shared, torch.ones(1, 2, 1, device=dev()), 2, 2).dispatch(x.requires_grad_())

@@ -3,6 +3,7 @@ from __future__ import annotations
 
 import concurrent.futures
 import os
+import shutil
 import subprocess
 import sys
 import sysconfig
@@ -51,9 +52,11 @@ def _compile_host() -> str:
   import torch
   from torch.utils import cpp_extension
   obj = os.path.join(OUT_DIR, "obj", "host.o")
-  includes = [os.path.join(ROOT, "include"), *cpp_extension.include_paths(),
+  rocm = os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(shutil.which(_hipcc()) or _hipcc()))), "include")
+  includes = [os.path.join(ROOT, "include"), *cpp_extension.include_paths(), rocm,
               sysconfig.get_paths()["include"]]
   _run(["g++", "-O2", "-std=c++17", "-fPIC", "-DTORCH_EXTENSION_NAME=_vmoe_host",
+        "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",       # (c10's stream header declares HIP's types)
         f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
         *[a for i in includes for a in ("-isystem" if "torch" in i else "-I", i)],
         "-c", os.path.join(HERE, "host.cpp"), "-o", obj], "g++ on host.cpp")
@@ -63,7 +66,7 @@ def _compile_host() -> str:
 def _link_host(obj: str) -> None:
   from torch.utils import cpp_extension
   libs = [a for d in cpp_extension.library_paths() for a in ("-L", d)]
-  _run(["g++", "-shared", obj, "-o", HOST, *libs, "-lc10", "-ltorch_cpu", "-ltorch", "-ltorch_python",
+  _run(["g++", "-shared", obj, "-o", HOST, *libs, "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python",
         "-L", OUT_DIR, "-l:libvmoe_hip.so", "-Wl,-rpath,$ORIGIN"], "linking the host module")
 
 

@@ -644,9 +644,11 @@ __global__ __launch_bounds__(64) void top_items_finish_kernel(const float* __res
   }
 }
 
-__global__ __launch_bounds__(256) void fill_i32_kernel(int32_t* p, size_t n, int32_t v) {
+// Empty slots and counters of indices_to_slots_kernel.
+__global__ __launch_bounds__(256) void clear_slots_kernel(int32_t* p, size_t n, int32_t* num_dup, int32_t* num_inv) {
   size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
+  if (i < n) p[i] = -1;
+  if (i == 0) *num_dup = *num_inv = 0;
 }
 
 __global__ __launch_bounds__(256) void indices_to_slots_kernel(
@@ -849,8 +851,8 @@ extern "C" int vmoe_indices_to_slots(const VmoeIndicesToSlotsParams* p, vmoe_str
     return VMOE_E_OVERFLOW;
   const size_t ns = (size_t)p->E * p->G * p->C;
   const size_t n = (size_t)p->G * p->S * p->K;
-  hipLaunchKernelGGL(fill_i32_kernel, dim3((unsigned)((ns + 255) / 256)), dim3(256), 0,
-                     as_stream(stream), p->slot_token, ns, -1);
+  hipLaunchKernelGGL(clear_slots_kernel, dim3((unsigned)((ns + 255) / 256)), dim3(256), 0,
+                     as_stream(stream), p->slot_token, ns, p->num_duplicates, p->num_invalid);
   hipLaunchKernelGGL(indices_to_slots_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
                      as_stream(stream), p->indices, p->token_slot, p->slot_token,
                      p->num_duplicates, p->num_invalid, p->G, p->S, p->E, p->K, p->C);

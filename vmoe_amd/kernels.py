@@ -191,7 +191,7 @@ def indices_to_slots(indices: torch.Tensor, num_experts: int, capacity: int):
   indices = indices.to(torch.int32).contiguous()
   token_slot = _i32(G, S, K, device=dev)
   slot_token = _i32(num_experts * G * capacity, device=dev)
-  counters = torch.zeros(2, dtype=torch.int32, device=dev)
+  counters = _i32(2, device=dev)
   p = H.IndicesToSlotsParams(H.ptr(indices), H.ptr(token_slot), H.ptr(slot_token),
                              H.c_void_p(counters.data_ptr()), H.c_void_p(counters.data_ptr() + 4),
                              G, S, num_experts, K, capacity)

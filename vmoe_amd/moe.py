@@ -19,7 +19,9 @@ from typing import Any, Callable, Dict, Mapping, Optional, Tuple
 
 import torch
 
+from vmoe_amd import _hip as H
 from vmoe_amd import kernels as K
+from vmoe_amd.nn import module
 
 Array = torch.Tensor
 _FLOAT_DTYPES = (torch.float32, torch.bfloat16)
@@ -95,6 +97,20 @@ class _CombineFn(torch.autograd.Function):
     return d_rows, None, d_w, None
 
 
+def _dispatch_recorded(rows, token_slot, slot_token):
+  """_DispatchFn, as a native function where nothing but autograd looks on."""
+  if H._timing_sink is None and module.is_plain_but_for_gradients(rows, token_slot, slot_token):
+    return H.host().dispatch_recorded(rows, token_slot, slot_token)
+  return _DispatchFn.apply(rows, token_slot, slot_token, slot_token.numel())
+
+
+def _combine_recorded(rows, token_slot, weights, slot_token):
+  """_CombineFn, likewise."""
+  if H._timing_sink is None and module.is_plain_but_for_gradients(rows, token_slot, weights, slot_token):
+    return H.host().combine_recorded(rows, token_slot, weights, slot_token)
+  return _CombineFn.apply(rows, token_slot, weights, slot_token)
+
+
 def _wants_grad(*tensors) -> bool:
   return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
 
@@ -127,6 +143,7 @@ class ExpertIndicesDispatcher(BaseDispatcher):
     self.fill = None                              # (G, E) kept items per (group, expert), if known
     self._packed_maps = None                      # (token_row (G,S,K), rows_per_expert (E,))
     self._rounds = None                           # per-occurrence slot maps when slots are shared
+    self._unread = None                           # (counters on their way to the host, event) of maps not yet checked
 
   @property
   def combine_weights(self) -> Array:
@@ -139,19 +156,41 @@ class ExpertIndicesDispatcher(BaseDispatcher):
   def combine_weights(self, value: Array):
     self._combine_weights = value
 
-  def _maps(self):
+  def _maps(self, settle: bool = True):
+    """The slot maps.  settle False: of maps that this call makes the counters may still be on their way (the
+    maps send nothing out of range, whatever the indices are); the caller issues the work behind them and
+    calls _settle() before it hands out a result."""
     if self._slots is None:
       if self.indices.ndim != 4 or self.indices.shape[-1] != 2:
         raise ValueError(f"indices must have shape (G, S, K, 2), got {tuple(self.indices.shape)}")
       token_slot, slot_token, counters = K.indices_to_slots(
           self.indices, self.num_experts, self.capacity)
-      dups, invalid = counters.tolist()
-      if invalid:
-        raise ValueError("ExpertIndicesDispatcher: negative indices are not supported.")
-      if dups:
-        self._rounds = self._occurrence_rounds(token_slot, slot_token.numel())
+      counters = counters.to("cpu", non_blocking=True)
+      event = torch.cuda.Event()
+      event.record()
+      self._unread = (counters, event)
       self._slots = (token_slot, slot_token)
+      if settle:
+        self._settle()
+      return token_slot, slot_token
+    self._settle()
     return self._slots
+
+  def _settle(self) -> None:
+    """Waits for the counters of new maps: negative indices raise, shared slots make rounds."""
+    unread = self._unread
+    if unread is None:
+      return
+    counters, event = unread
+    event.synchronize()
+    dups, invalid = counters.tolist()
+    if invalid:
+      self._slots = self._unread = None
+      raise ValueError("ExpertIndicesDispatcher: negative indices are not supported.")
+    if dups:
+      token_slot, slot_token = self._slots
+      self._rounds = self._occurrence_rounds(token_slot, slot_token.numel())
+    self._unread = None
 
   @staticmethod
   def _occurrence_rounds(token_slot: Array, num_slots: int):
@@ -179,8 +218,16 @@ class ExpertIndicesDispatcher(BaseDispatcher):
 
   def dispatch(self, data: Array) -> Array:
     G, S, Kk, _ = self.indices.shape
-    token_slot, slot_token = self._maps()
+    token_slot, slot_token = self._maps(settle=False)
     rows, item_shape, width = _as_rows(data, 2)
+    if self._rounds is None:
+      # (issued before the counters are read, so that the GPU has work while the host waits for them; with shared
+      # slots this result is dropped)
+      if _wants_grad(rows):
+        out = _dispatch_recorded(rows, token_slot.view(G * S, Kk), slot_token)
+      else:
+        out = K.dispatch(rows, token_slot.view(G * S, Kk), slot_token)
+      self._settle()
     if self._rounds is not None:
       if _wants_grad(rows):
         raise NotImplementedError("gradients through a dispatch with shared slots")
@@ -189,10 +236,6 @@ class ExpertIndicesDispatcher(BaseDispatcher):
         part = K.dispatch(rows, ts_r, st_r).to(torch.float32)
         acc = part if acc is None else acc + part
       out = acc.to(rows.dtype)
-    elif _wants_grad(rows):
-      out = _DispatchFn.apply(rows, token_slot.view(G * S, Kk), slot_token, slot_token.numel())
-    else:
-      out = K.dispatch(rows, token_slot.view(G * S, Kk), slot_token)
     return _from_rows(out, (self.num_experts, G * self.capacity), item_shape, width)
 
   def combine(self, data: Array) -> Array:
@@ -203,7 +246,7 @@ class ExpertIndicesDispatcher(BaseDispatcher):
     if _wants_grad(rows, cw if isinstance(cw, torch.Tensor) else None):
       # differentiable in the data and in combine_weights
       w = self.combine_weights.to(torch.float32)
-      out = _CombineFn.apply(rows, token_slot.view(G * S, Kk), w.reshape(G * S, Kk), slot_token)
+      out = _combine_recorded(rows, token_slot.view(G * S, Kk), w.reshape(G * S, Kk), slot_token)
       return _from_rows(out, (G, S), item_shape, width)
     w = self._weights_f32 if self._weights_f32 is not None else K.cast(
         self.combine_weights.contiguous(), torch.float32)

@@ -78,11 +78,16 @@ def require_no_grad(what: str, *tensors) -> None:
 def is_plain(*tensors) -> bool:
   """Whether torch operations on these tensors may be replaced by a kernel that sees nothing but their memory:
   ordinary tensors on the GPU, no gradient recorded, and no transform, mode, trace or autocast at work."""
+  if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+    return False
+  return is_plain_but_for_gradients(*tensors)
+
+
+def is_plain_but_for_gradients(*tensors) -> bool:
+  """is_plain for an operation that autograd may record."""
   for t in tensors:
     if type(t) not in (torch.Tensor, torch.nn.Parameter) or not t.is_cuda:
       return False
-  if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
-    return False
   return not (torch._C._functorch.peek_interpreter_stack() is not None
               or torch.autograd.forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack()
               or torch._C._len_torch_function_stack() or torch._C._get_tracing_state() is not None
