@@ -1243,3 +1243,26 @@ def test_dispatcher_checks_new_maps_behind_the_dispatch(moe):
   assert torch.equal(out[0, 0], x[0, 0] + x[0, 1])
   with pytest.raises(NotImplementedError):
     moe.ExpertIndicesDispatcher(shared, torch.ones(1, 2, 1, device=dev()), 2, 2).dispatch(x.requires_grad_())
+
+
+@pytest.mark.parametrize("S,E,k,capacity", [(1, 1, 1, 4), (37, 5, 2, 8), (300, 7, 3, 200)])
+def test_packed_rows_of_one_group_are_its_slots(moe, S, E, k, capacity):
+  """One group: the maps that no launch computes are those that the compaction would, and a layer's bfloat16
+  experts with float32 biases (rounded and planned in one launch) give the bits of the separate calls."""
+  from vmoe_amd import kernels as K
+  gates = torch.softmax(torch.randn(1, S, E, device=dev()), -1)
+  d = moe.get_top_experts_per_item_dispatcher(gates, "indices", num_selected_experts=k, capacity=capacity,
+                                              batch_priority=True)
+  assert d.pending_compaction() is None
+  token_row, rows, row_token = d._packed()
+  want_row, want_rows, want_token = K.compact_rows(d.fill, d._maps()[0], capacity)
+  assert torch.equal(token_row, want_row) and torch.equal(rows, want_rows)
+  for e, n in enumerate(rows.tolist()):
+    assert torch.equal(row_token[e, :n], want_token[e, :n])
+  D, M = 64, 136
+  bf = lambda *s: torch.randn(*s, device=dev()).to(torch.bfloat16)
+  x, w0, w1, b0, b1 = bf(S, D), bf(E, D, M), bf(E, M, D), bf(E, M), bf(E, D)
+  got = K.expert_mlp(x, w0, b0.float(), w1, b1.float(), rows_per_expert=rows, x_rows=row_token)
+  want = K.expert_mlp(x, w0, b0, w1, b1, rows_per_expert=want_rows, x_rows=want_token)
+  for e, n in enumerate(rows.tolist()):
+    assert torch.equal(got[e, :n], want[e, :n])

@@ -309,8 +309,6 @@ __device__ __forceinline__ void cast_biases_block(const BiasCast& c, unsigned bl
   }
 }
 
-__global__ __launch_bounds__(256) void cast_biases_kernel(BiasCast c) { cast_biases_block(c, blockIdx.x); }
-
 // Row compaction, the launch plans of the expert MLP's ragged products and the casts of its float32
 // biases in one launch: workgroups 0 .. compact_blocks - 1 renumber the assignments
 // (compact_rows_fused_block), the next plan_blocks plan (plan_ragged_tiles_block, row counts from the
@@ -326,7 +324,7 @@ __global__ __launch_bounds__(256) void compact_rows_planned_kernel(
     compact_rows_fused_block(fill, token_slot, token_row, row_token, rows_per_expert, G, E, C,
                              per_group, K, n, blockIdx.x);
   else if (blockIdx.x < compact_blocks + plan_blocks)
-    plan_ragged_tiles_block(nullptr, fill, G, E, R, ga, gb, blockIdx.x - compact_blocks, tile_prefix);
+    plan_ragged_tiles_block(fill, G, E, R, ga, gb, blockIdx.x - compact_blocks, tile_prefix);
   else
     cast_biases_block(biases, blockIdx.x - compact_blocks - plan_blocks);
 }
@@ -637,11 +635,11 @@ static int run_expert_mlp(const VmoeExpertMlpParams* p, vmoe_stream_t stream_, b
   const MlpPlans& m = w.m;
   unsigned char* ws = w.rest;
   if (planned_already && !m.planned) return VMOE_E_UNSUPPORTED;
-  if (w.plan_blocks > 0 && !planned_already)
-    hipLaunchKernelGGL(plan_ragged_tiles_kernel, dim3(w.plan_blocks), dim3(256),
-                       plan_ragged_tiles_lds(p->E), stream, p->rows_per_expert, p->E, p->R, w.ga, w.gb);
-  if (w.biases.blocks() > 0 && !planned_already)
-    hipLaunchKernelGGL(cast_biases_kernel, dim3(w.biases.blocks()), dim3(256), 0, stream, w.biases);
+  // Launch plans and bias casts in one launch (rows_per_expert are the fill counts of a single group).
+  if (!planned_already && w.plan_blocks + w.biases.blocks() > 0)
+    hipLaunchKernelGGL(compact_rows_planned_kernel, dim3((unsigned)w.plan_blocks + w.biases.blocks()), dim3(256),
+                       w.plan_blocks > 0 ? plan_ragged_tiles_lds(p->E) : 0, stream, p->rows_per_expert, nullptr, nullptr,
+                       nullptr, nullptr, 1, p->E, p->R, 1, 1, 0, 0u, (unsigned)w.plan_blocks, p->R, w.ga, w.gb, w.biases);
   const bool tanh_gelu = gelu_of(p) == VMOE_GELU_TANH;
   const bool f32_products = (p->gelu & VMOE_MLP_F32_PRODUCTS) != 0;
   if (p->dtype == VMOE_BF16) {

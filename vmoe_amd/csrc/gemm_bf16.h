@@ -300,11 +300,11 @@ __device__ __forceinline__ void plan_one(const RaggedGeom& g, const int32_t* til
 // row tiles, from which a tile-walking kernel derives the length of its die's run, and the
 // tag of the geometry the plan was written for (plan_tag).
 // One workgroup of the planning launch (block = its index among the planning workgroups).
-// With `fill` (G x batch fill counts of the slot assignment) the row counts are its column
-// sums, added up here, and `rows` is not read: the plan then does not wait for the launch
+// The row counts are the column sums of `fill` (G x batch fill counts of the slot assignment; row
+// counts themselves are those of one group), added up here: the plan does not wait for the launch
 // that writes the row counts and can share a launch with it.
 __device__ __forceinline__ void plan_ragged_tiles_block(
-    const int32_t* __restrict__ rows, const int32_t* __restrict__ fill, int G, int batch, int R,
+    const int32_t* __restrict__ fill, int G, int batch, int R,
     const RaggedGeom& ga, const RaggedGeom& gb, unsigned block, int32_t* tile_prefix) {
   // tile_prefix: 2 x (batch + 1) live row tiles before batch b, then `batch` row counts
   __shared__ int32_t wsum[2][4];
@@ -317,11 +317,7 @@ __device__ __forceinline__ void plan_ragged_tiles_block(
     const int bb = b0 + tid;
     int n = 0;
     if (bb < batch) {
-      if (fill != nullptr) {
-        for (int g = 0; g < G; ++g) n += fill[(size_t)g * batch + bb];
-      } else {
-        n = rows[bb];
-      }
+      for (int g = 0; g < G; ++g) n += fill[(size_t)g * batch + bb];
       n = min(max(n, 0), R);
       rows_here[bb] = n;
     }
@@ -364,12 +360,6 @@ __device__ __forceinline__ void plan_ragged_tiles_block(
 
 // LDS of a planning workgroup.
 inline size_t plan_ragged_tiles_lds(int batch) { return ((size_t)2 * (batch + 1) + batch) * sizeof(int32_t); }
-
-__global__ __launch_bounds__(256) void plan_ragged_tiles_kernel(
-    const int32_t* __restrict__ rows, int batch, int R, RaggedGeom ga, RaggedGeom gb) {
-  extern __shared__ int32_t tile_prefix[];
-  plan_ragged_tiles_block(rows, nullptr, 0, batch, R, ga, gb, blockIdx.x, tile_prefix);
-}
 
 // A launch plan as a product kernel is given it: the entries, the index of the header entry
 // and the tag that the header must carry (plan_tag of the launch's own geometry).
@@ -1710,7 +1700,7 @@ PlanRef plan_ref(const GemmGeom& g, const int4* plan, int batch, int R) {
   return plan_ref_of(g, plan, Cfg::BM, batch, R);
 }
 
-// `plan`, if given, was filled by plan_ragged_tiles_kernel for this product's geometry.
+// `plan`, if given, was filled by plan_ragged_tiles_block for this product's geometry.
 // `clear` / `status`: see begin_call.
 template <typename Cfg, int EPI>
 int launch_gemm_bf16(const bf16_t* A, const bf16_t* Bt, const bf16_t* bias, bf16_t* C, int batch,
@@ -1821,7 +1811,7 @@ struct StreamKWorkspace {
 };
 
 // Launches the persistent kernel; the caller checked persistent_gemm_ok.  `plan`, if
-// given, was filled by plan_ragged_tiles_kernel for gemm_geometry<Cfg> (BM, BN and
+// given, was filled by plan_ragged_tiles_block for gemm_geometry<Cfg> (BM, BN and
 // workgroups per CU decide it, not the number of stages).  `streamk`, if given, is
 // StreamKWorkspace<Cfg>::kBytes of memory: the die's last, partial round is then shared
 // along k; an earlier launch of the call has set its flags to zero (begin_call).  `status`:
