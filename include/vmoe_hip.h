@@ -481,9 +481,11 @@ int vmoe_soft_route_stats(const VmoeSoftRouteParams* route, const VmoeSoftStatsP
  *   combine:  out[g,s,:]     = sum_n w[g,s,n] * y[slot(g,n)]
  * with N = E*C and slot(g, n=e*C+c) the slot row defined at the top.
  * float32 accumulate, result rounded to out_dtype.  `w` is float32, bf16 or
- * bool (dispatch only; w_dtype = 2).
+ * bool (dispatch only; w_dtype = 2).  data_dtype may be VMOE_EINSUM_F32_AS_BF16: float32 data, each value
+ * rounded to bf16 as it is read (Bfloat16Dispatcher, vmoe/moe.py:217-227).
  */
 enum { VMOE_W_F32 = 0, VMOE_W_BF16 = 1, VMOE_W_BOOL = 2 };
+enum { VMOE_EINSUM_F32_AS_BF16 = 2 };
 typedef struct {
   const void* w;     /* (G, S, E*C) */
   const void* data;  /* dispatch: (G, S, D); combine: (E*G*C, D) */

@@ -832,6 +832,34 @@ EINSUM_CASES = [
 ]
 
 
+@pytest.mark.parametrize("G,S,E,C,D", [(2, 64, 8, 8, 64), (3, 65, 5, 13, 70), (4, 1, 2, 1, 3), (2, 130, 3, 43, 129)])
+@pytest.mark.parametrize("wdtype", [torch.float32, torch.bool])
+def test_einsum_float32_weights_in_64_bits(K, G, S, E, C, D, wdtype):
+  """The generic einsum at k tiles, rows and columns that end inside (and addresses of the types' own alignment)
+  against 64 bits; float32 data that count as rounded to bfloat16 give the bits of a cast in front."""
+  gen = torch.Generator(device=dev()).manual_seed(S)
+  w = torch.randn((G, S, E, C), generator=gen, device=dev())
+  w = w > 0 if wdtype == torch.bool else w
+  x = torch.randn((G, S, D), generator=gen, device=dev())
+  y = torch.randn((E * G * C, D), generator=gen, device=dev())
+  order = torch.arange(E * G * C, device=dev()).view(E * G * C, 1).float()       # slot rows, by a one-hot of each
+  bound = lambda a, b: a.abs() @ b.abs() * max(S, E * C) * 2.0 ** -24 + 1e-30     # n roundings of partial sums
+  wd = w.double().view(G, S, E * C)
+  eye = torch.eye(E * C, device=dev()).view(1, E * C, E, C).expand(G, -1, -1, -1)
+  rows = K.einsum_combine(eye, order, torch.float32).long().view(G, E * C)         # row of slot (g, n)
+  got = K.einsum_dispatch(w, x, torch.float32)
+  for g in range(G):
+    want, at = wd[g].t() @ x[g].double(), got[rows[g]].double()
+    assert bool(((at - want).abs() <= bound(wd[g].t(), x[g].double())).all())
+  assert torch.equal(K.einsum_dispatch(w, x, torch.float32, True), K.einsum_dispatch(w, x.bfloat16(), torch.float32))
+  if wdtype != torch.bool:
+    got = K.einsum_combine(w, y, torch.float32)
+    for g in range(G):
+      data = y[rows[g]].double()
+      assert bool(((got[g].double() - wd[g] @ data).abs() <= bound(wd[g], data)).all())
+    assert torch.equal(K.einsum_combine(w, y, torch.float32, True), K.einsum_combine(w, y.bfloat16(), torch.float32))
+
+
 @pytest.mark.parametrize("G,S,E,C,D,wdtype,ddtype", EINSUM_CASES)
 def test_einsum_dispatch_combine(K, G, S, E, C, D, wdtype, ddtype):
   rng = np.random.default_rng(G + S)

@@ -375,7 +375,9 @@ int w_code(const Tensor& w) {
 }
 
 // Dense dispatch (G, S, E, C) x (G, S, D) -> (E*G*C, D), or combine -> (G, S, D).
-Tensor einsum(int64_t stream, const Tensor& w_, const Tensor& data_, at::ScalarType out_type, bool is_dispatch) {
+// rounded: float32 data, rounded to bfloat16 as they are read.
+Tensor einsum(int64_t stream, const Tensor& w_, const Tensor& data_, at::ScalarType out_type, bool is_dispatch,
+              bool rounded) {
   need_axes(w_, 4, "w");
   if (data_.dim() < 1) need_axes(data_, is_dispatch ? 3 : 2, "data");
   const Tensor w = w_.contiguous(), data = data_.contiguous();
@@ -383,7 +385,8 @@ Tensor einsum(int64_t stream, const Tensor& w_, const Tensor& data_, at::ScalarT
   need_values(data, (is_dispatch ? G * S : E * G * C) * D, "data");
   Tensor out = is_dispatch ? empty({E * G * C, D}, out_type, data) : empty({G, S, D}, out_type, data);
   VmoeEinsumParams p{ptr(w), ptr(data), ptr(out), (int32_t)G, (int32_t)S, (int32_t)E, (int32_t)C, (int32_t)D,
-                     w_code(w), dtype_code(data), dtype_code(out_type)};
+                     w_code(w), rounded && data.scalar_type() == at::kFloat ? VMOE_EINSUM_F32_AS_BF16 : dtype_code(data),
+                     dtype_code(out_type)};
   if (is_dispatch) check(vmoe_einsum_dispatch(&p, stream_of(stream)), "vmoe_einsum_dispatch");
   else check(vmoe_einsum_combine(&p, stream_of(stream)), "vmoe_einsum_combine");
   return out;
@@ -596,9 +599,9 @@ PYBIND11_MODULE(_vmoe_host, m) {
   });
   VMOE_DEF(attention);
   VMOE_DEF(dense);
-  m.def("einsum", [](int64_t s, const Tensor& w, const Tensor& d, py::object t, bool dispatch_) {
+  m.def("einsum", [](int64_t s, const Tensor& w, const Tensor& d, py::object t, bool dispatch_, bool rounded) {
     return torch::wrap_pybind_function_no_gil(&einsum)(s, w, d, torch::python::detail::py_object_to_dtype(std::move(t)),
-                                                       dispatch_);
+                                                       dispatch_, rounded);
   });
   VMOE_DEF(soft_route_stats);
   VMOE_DEF(combine_backward_data);

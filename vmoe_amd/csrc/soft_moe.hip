@@ -26,15 +26,6 @@ namespace {
 using soft::kNormEps;
 constexpr float kLog2e = 1.4426950408889634f;
 
-__device__ __forceinline__ float load_any(const void* p, size_t i, int dtype) {
-  return dtype == VMOE_F32 ? reinterpret_cast<const float*>(p)[i]
-                           : bf2f(reinterpret_cast<const bf16_t*>(p)[i]);
-}
-__device__ __forceinline__ float load_w(const void* p, size_t i, int wdtype) {
-  if (wdtype == VMOE_W_F32) return reinterpret_cast<const float*>(p)[i];
-  if (wdtype == VMOE_W_BF16) return bf2f(reinterpret_cast<const bf16_t*>(p)[i]);
-  return reinterpret_cast<const uint8_t*>(p)[i] ? 1.f : 0.f;
-}
 __device__ __forceinline__ void store_any(void* p, size_t i, float v, int dtype) {
   if (dtype == VMOE_F32) reinterpret_cast<float*>(p)[i] = v;
   else reinterpret_cast<bf16_t*>(p)[i] = f2bf(v);
@@ -763,13 +754,50 @@ __global__ __launch_bounds__(kSrThreads) void soft_route_roles_kernel(
 // Dense einsum between per-group weights and data on the float32 matrix cores.
 //   DISPATCH: out[slot(g,mm)] = sum_s w[g,s,mm] * data[g,s,:]      (M = E*C, Kd = S)
 //   COMBINE:  out[g,mm,:]     = sum_n w[g,mm,n] * data[slot(g,n)]  (M = S,   Kd = E*C)
-template <bool DISPATCH>
+// WT, DT: types of w and data (DT VMOE_EINSUM_F32_AS_BF16: float32 rounded to bfloat16 as it is read).
+// Bound by latency: 32 groups of 49 items x 48 slots x 512 are 256 workgroups of one k tile, whose two operands have to
+// be there before anything else can happen.  A k tile is 64 values, fetched in pieces of four at any address of the
+// type's own alignment, the next one under the MFMAs of this one: 12.5 and 7.4 us (16 values of k at a time, scalar
+// loads of types looked up per value, a slot's row from three divisions per output) -> 6.5 each for that shape, the casts
+// to bfloat16 in front of them (3 and 5 us) included.  The order of sums, two values of k per MFMA, is
+// part of the result: what a Soft MoE layer rounds to bfloat16 later comes out of it.
+template <int T>
+__device__ __forceinline__ void load4(const void* p, size_t i, int n, bool whole, float (&v)[4]) {
+  if constexpr (T == VMOE_F32 || T == VMOE_EINSUM_F32_AS_BF16) {
+    typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));
+    const float* q = static_cast<const float*>(p) + i;
+    if (whole) {
+      const f4_any t = *reinterpret_cast<const f4_any*>(q);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = t[j];
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = j < n ? q[j] : 0.f;
+    }
+    if constexpr (T == VMOE_EINSUM_F32_AS_BF16)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = bf16r(v[j]);
+  } else {
+    const bf16_t* q = static_cast<const bf16_t*>(p) + i;
+    if (whole && (reinterpret_cast<uintptr_t>(q) & 7u) == 0) {
+      const uint2 t = *reinterpret_cast<const uint2*>(q);
+      v[0] = bf_lo(t.x); v[1] = bf_hi(t.x); v[2] = bf_lo(t.y); v[3] = bf_hi(t.y);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = j < n ? bf2f(q[j]) : 0.f;
+    }
+  }
+}
+
+template <bool DISPATCH, int WT, int DT>
 __global__ __launch_bounds__(256) void einsum_kernel(const void* __restrict__ w,
                                                      const void* __restrict__ data,
                                                      void* __restrict__ out, int G, int S, int E,
-                                                     int C, int D, int wdt, int ddt, int odt) {
-  __shared__ float sa[64][16 + 1];
-  __shared__ float sb[16][64 + 4];
+                                                     int C, int D, int odt) {
+  constexpr int BK = 64;
+  __shared__ float sa[64][BK + 1];
+  __shared__ __align__(16) float sb[BK][64 + 4];
+  __shared__ int out_row[64];       // row of the output of the tile's rows
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const int m = lane & 31, h = lane >> 5;
@@ -779,55 +807,60 @@ __global__ __launch_bounds__(256) void einsum_kernel(const void* __restrict__ w,
   const int Kd = DISPATCH ? S : N;
   const int row0 = blockIdx.y * 64, col0 = blockIdx.x * 64;
   const size_t wbase = (size_t)g * S * N;
+  const int slot0 = slot_row(0, g, 0, G, E, C);      // slot_row's divisions once; one more per slot
+  auto slot_of = [&](int n) { return n / C * (G * C) + slot0 + n % C; };
+  // A thread's pieces of a k tile: four weights (of one k, DISPATCH, or one row) and four columns of one k, four times.
+  const int hi = tid >> 4, lo4 = (tid & 15) * 4;
+  float va[4][4], vb[4][4];
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int r = u * 16 + hi;                       // k (DISPATCH) or row of the tile
+      const int k = DISPATCH ? k0 + r : k0 + lo4, mm = DISPATCH ? row0 + lo4 : row0 + r;
+      const int n = DISPATCH ? (k < Kd ? M - mm : 0) : (mm < M ? Kd - k : 0);
+      const size_t at = DISPATCH ? wbase + (size_t)k * N + mm : wbase + (size_t)mm * N + k;
+      if constexpr (WT == VMOE_W_BOOL) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) va[u][j] = j < n && static_cast<const uint8_t*>(w)[at + j] != 0 ? 1.f : 0.f;
+      } else {
+        load4<WT == VMOE_W_BF16 ? VMOE_BF16 : VMOE_F32>(w, at, n, n >= 4, va[u]);
+      }
+      const int kb = k0 + r, cols = kb < Kd ? D - (col0 + lo4) : 0;
+      size_t rowi = 0;
+      if (kb < Kd) rowi = DISPATCH ? (size_t)g * S + kb : (size_t)slot_of(kb);
+      load4<DT>(data, rowi * D + col0 + lo4, cols, cols >= 4, vb[u]);
+    }
+  };
   floatx16 acc;
 #pragma unroll
   for (int v = 0; v < 16; ++v) acc[v] = 0.f;
-  for (int k0 = 0; k0 < Kd; k0 += 16) {
-    float va[4], vb[4];
-    if (DISPATCH) {
-      const int kk = k0 + (tid >> 4), m4 = row0 + (tid & 15) * 4;
+  fetch(0);
+  if (tid < 64) out_row[tid] = DISPATCH ? slot_of(min(row0 + tid, N - 1)) : g * S + row0 + tid;
+  for (int k0 = 0; k0 < Kd; k0 += BK) {
+    if (k0 > 0) __syncthreads();
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        va[i] = (kk < Kd && m4 + i < M) ? load_w(w, wbase + (size_t)kk * N + m4 + i, wdt) : 0.f;
-    } else {
-      const int mm = row0 + (tid >> 2), k4 = k0 + (tid & 3) * 4;
+    for (int u = 0; u < 4; ++u) {
+      const int r = u * 16 + hi;
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        va[i] = (mm < M && k4 + i < Kd) ? load_w(w, wbase + (size_t)mm * N + k4 + i, wdt) : 0.f;
-    }
-    {
-      const int kk = k0 + (tid >> 4), n4 = col0 + (tid & 15) * 4;
-      size_t rowi = 0;
-      if (kk < Kd) rowi = DISPATCH ? (size_t)g * S + kk : (size_t)slot_row(kk / C, g, kk % C, G, E, C);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        vb[i] = (kk < Kd && n4 + i < D) ? load_any(data, rowi * D + n4 + i, ddt) : 0.f;
+      for (int j = 0; j < 4; ++j) {
+        if (DISPATCH) sa[lo4 + j][r] = va[u][j];
+        else sa[r][lo4 + j] = va[u][j];
+      }
+      *reinterpret_cast<float4*>(&sb[r][lo4]) = make_float4(vb[u][0], vb[u][1], vb[u][2], vb[u][3]);
     }
     __syncthreads();
-    if (DISPATCH) {
+    if (k0 + BK < Kd) fetch(k0 + BK);
+    for (int k = 0; k < BK && k0 + k < Kd; k += 16)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) sa[(tid & 15) * 4 + i][tid >> 4] = va[i];
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) sa[tid >> 2][(tid & 3) * 4 + i] = va[i];
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sb[tid >> 4][(tid & 15) * 4 + i] = vb[i];
-    __syncthreads();
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks)
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(sa[wm * 32 + m][ks * 2 + h],
-                                                 sb[ks * 2 + h][wn * 32 + m], acc, 0, 0, 0);
+      for (int ks = 0; ks < 8; ++ks)
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(sa[wm * 32 + m][k + ks * 2 + h], sb[k + ks * 2 + h][wn * 32 + m], acc, 0, 0, 0);
   }
   mfma_result_fence();
   const int col = col0 + wn * 32 + m;
 #pragma unroll
   for (int v = 0; v < 16; ++v) {
-    const int mm = row0 + wm * 32 + (v >> 2) * 8 + h * 4 + (v & 3);
-    if (mm < M && col < D) {
-      size_t orow = DISPATCH ? (size_t)slot_row(mm / C, g, mm % C, G, E, C) : (size_t)g * S + mm;
-      store_any(out, orow * D + col, acc[v], odt);
-    }
+    const int r = wm * 32 + (v >> 2) * 8 + h * 4 + (v & 3);
+    if (row0 + r < M && col < D) store_any(out, (size_t)out_row[r] * D + col, acc[v], odt);
   }
 }
 
@@ -837,7 +870,7 @@ int check_einsum(const VmoeEinsumParams* p, bool dispatch) {
   if (p->G > 65535) return VMOE_E_UNSUPPORTED;
   if (p->w_dtype < VMOE_W_F32 || p->w_dtype > VMOE_W_BOOL) return VMOE_E_DTYPE;
   if (!dispatch && p->w_dtype == VMOE_W_BOOL) return VMOE_E_DTYPE;
-  if ((p->data_dtype != VMOE_F32 && p->data_dtype != VMOE_BF16) ||
+  if ((p->data_dtype != VMOE_F32 && p->data_dtype != VMOE_BF16 && p->data_dtype != VMOE_EINSUM_F32_AS_BF16) ||
       (p->out_dtype != VMOE_F32 && p->out_dtype != VMOE_BF16))
     return VMOE_E_DTYPE;
   if ((int64_t)p->E * p->G * p->C >= INT32_MAX || (int64_t)p->G * p->S >= INT32_MAX)
@@ -1034,25 +1067,38 @@ extern "C" int vmoe_soft_route(const VmoeSoftRouteParams* p, vmoe_stream_t strea
   return soft_route_launch(p, stream, nullptr, nullptr);
 }
 
+template <bool DISPATCH>
+static int launch_einsum(const VmoeEinsumParams* p, hipStream_t stream) {
+  const int M = DISPATCH ? p->E * p->C : p->S;
+  const dim3 grid((p->D + 63) / 64, (M + 63) / 64, p->G);
+  auto launch = [&](auto wt, auto dt) {
+    hipLaunchKernelGGL((einsum_kernel<DISPATCH, decltype(wt)::value, decltype(dt)::value>), grid, dim3(256), 0, stream,
+                       p->w, p->data, p->out, p->G, p->S, p->E, p->C, p->D, p->out_dtype);
+    return launch_status();
+  };
+  auto with_data = [&](auto wt) {
+    if (p->data_dtype == VMOE_F32) return launch(wt, std::integral_constant<int, VMOE_F32>{});
+    if (p->data_dtype == VMOE_BF16) return launch(wt, std::integral_constant<int, VMOE_BF16>{});
+    return launch(wt, std::integral_constant<int, VMOE_EINSUM_F32_AS_BF16>{});
+  };
+  if (p->w_dtype == VMOE_W_F32) return with_data(std::integral_constant<int, VMOE_W_F32>{});
+  if (p->w_dtype == VMOE_W_BF16) return with_data(std::integral_constant<int, VMOE_W_BF16>{});
+  if constexpr (DISPATCH) return with_data(std::integral_constant<int, VMOE_W_BOOL>{});
+  return VMOE_E_DTYPE;
+}
+
 extern "C" int vmoe_einsum_dispatch(const VmoeEinsumParams* p, vmoe_stream_t stream) {
   int rc = check_einsum(p, true);
   if (rc != VMOE_OK) return rc;
   if (ein::dispatch_fast_ok(p)) return ein::launch_dispatch_fast(p, as_stream(stream));
-  const int M = p->E * p->C;
-  dim3 grid((p->D + 63) / 64, (M + 63) / 64, p->G);
-  hipLaunchKernelGGL(einsum_kernel<true>, grid, dim3(256), 0, as_stream(stream), p->w, p->data,
-                     p->out, p->G, p->S, p->E, p->C, p->D, p->w_dtype, p->data_dtype, p->out_dtype);
-  return launch_status();
+  return launch_einsum<true>(p, as_stream(stream));
 }
 
 extern "C" int vmoe_einsum_combine(const VmoeEinsumParams* p, vmoe_stream_t stream) {
   int rc = check_einsum(p, false);
   if (rc != VMOE_OK) return rc;
   if (ein::combine_fast_ok(p)) return ein::launch_combine_fast(p, as_stream(stream));
-  dim3 grid((p->D + 63) / 64, (p->S + 63) / 64, p->G);
-  hipLaunchKernelGGL(einsum_kernel<false>, grid, dim3(256), 0, as_stream(stream), p->w, p->data,
-                     p->out, p->G, p->S, p->E, p->C, p->D, p->w_dtype, p->data_dtype, p->out_dtype);
-  return launch_status();
+  return launch_einsum<false>(p, as_stream(stream));
 }
 
 extern "C" int vmoe_soft_router_stats(const VmoeSoftStatsParams* p, vmoe_stream_t stream) {

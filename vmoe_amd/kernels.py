@@ -569,10 +569,15 @@ def _w_code(w: torch.Tensor) -> int:
   raise TypeError(f"Unsupported weight dtype {w.dtype}")
 
 
-def einsum_dispatch(w: torch.Tensor, data: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
-  """w (G,S,E,C), data (G,S,D) -> (E*G*C, D) in the expert buffer's row order."""
+def _einsum_data_code(data: torch.Tensor, rounded: bool) -> int:
+  return H.EINSUM_F32_AS_BF16 if rounded and data.dtype == torch.float32 else H.dtype_code(data.dtype)
+
+
+def einsum_dispatch(w: torch.Tensor, data: torch.Tensor, out_dtype: torch.dtype, rounded: bool = False) -> torch.Tensor:
+  """w (G,S,E,C), data (G,S,D) -> (E*G*C, D) in the expert buffer's row order.  ``rounded``: float32 data are
+  rounded to bfloat16 as they are read."""
   if not H.timed("vmoe_einsum_dispatch"):
-    return H.host().einsum(H.raw_stream(), w, data, out_dtype, True)
+    return H.host().einsum(H.raw_stream(), w, data, out_dtype, True, rounded)
   G, S, E, C = w.shape
   D = data.shape[-1]
   w = w.contiguous()
@@ -580,22 +585,22 @@ def einsum_dispatch(w: torch.Tensor, data: torch.Tensor, out_dtype: torch.dtype)
   out = torch.empty((E * G * C, D), dtype=out_dtype, device=data.device)
   wv = w.view(torch.uint8) if w.dtype == torch.bool else w
   p = H.EinsumParams(H.ptr(wv), H.ptr(data), H.ptr(out), G, S, E, C, D, _w_code(w),
-                     H.dtype_code(data.dtype), H.dtype_code(out_dtype))
+                     _einsum_data_code(data, rounded), H.dtype_code(out_dtype))
   H.call("vmoe_einsum_dispatch", p)
   return out
 
 
-def einsum_combine(w: torch.Tensor, data: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
-  """w (G,S,E,C), data (E*G*C, D) -> (G,S,D)."""
+def einsum_combine(w: torch.Tensor, data: torch.Tensor, out_dtype: torch.dtype, rounded: bool = False) -> torch.Tensor:
+  """w (G,S,E,C), data (E*G*C, D) -> (G,S,D).  ``rounded`` as in einsum_dispatch."""
   if not H.timed("vmoe_einsum_combine"):
-    return H.host().einsum(H.raw_stream(), w, data, out_dtype, False)
+    return H.host().einsum(H.raw_stream(), w, data, out_dtype, False, rounded)
   G, S, E, C = w.shape
   D = data.shape[-1]
   w = w.contiguous()
   data = data.contiguous()
   out = torch.empty((G, S, D), dtype=out_dtype, device=data.device)
   p = H.EinsumParams(H.ptr(w), H.ptr(data), H.ptr(out), G, S, E, C, D, _w_code(w),
-                     H.dtype_code(data.dtype), H.dtype_code(out_dtype))
+                     _einsum_data_code(data, rounded), H.dtype_code(out_dtype))
   H.call("vmoe_einsum_combine", p)
   return out
 

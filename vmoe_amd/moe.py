@@ -326,23 +326,29 @@ class EinsumDispatcher(BaseDispatcher):
     self.einsum_precision = einsum_precision
 
   @staticmethod
-  def _result_dtype(w: Array, data: Array) -> torch.dtype:
+  def _result_dtype(w: Array, data_dtype: torch.dtype) -> torch.dtype:
     if w.dtype == torch.bool:
-      return data.dtype
-    return torch.promote_types(w.dtype, data.dtype)
+      return data_dtype
+    return torch.promote_types(w.dtype, data_dtype)
 
-  def dispatch(self, data: Array) -> Array:
+  # (as_dtype bfloat16: float32 data count as rounded to it, which the kernels do as they read)
+  def _reads_rounded(self, data: Array) -> bool:
+    return data.dtype == torch.float32 and all(
+        w is None or w.dtype == torch.float32 for w in (self.combine_weights, self.dispatch_weights))
+
+  def dispatch(self, data: Array, as_dtype: Optional[torch.dtype] = None) -> Array:
     w = self.combine_weights > 0 if self.dispatch_weights is None else self.dispatch_weights
     G, S, E, C = w.shape
     rows, item_shape, width = _as_rows(data, 2)
-    out = K.einsum_dispatch(w, rows.view(G, S, -1), self._result_dtype(w, data))
+    out = K.einsum_dispatch(w, rows.view(G, S, -1), self._result_dtype(w, as_dtype or data.dtype),
+                            as_dtype is not None)
     return _from_rows(out, (E, G * C), item_shape, width)
 
-  def combine(self, data: Array) -> Array:
+  def combine(self, data: Array, as_dtype: Optional[torch.dtype] = None) -> Array:
     w = self.combine_weights
     G, S, E, C = w.shape
     rows, item_shape, width = _as_rows(data, 2)
-    out = K.einsum_combine(w, rows, self._result_dtype(w, data))
+    out = K.einsum_combine(w, rows, self._result_dtype(w, as_dtype or data.dtype), as_dtype is not None)
     return _from_rows(out.view(G * S, -1), (G, S), item_shape, width)
 
 
@@ -441,14 +447,22 @@ class Bfloat16Dispatcher(BaseDispatcher):
   def __init__(self, dispatcher: BaseDispatcher):
     self.dispatcher = dispatcher
 
+  def _rounds_as_it_reads(self, data: Array) -> bool:
+    """Whether the inner dispatcher's kernels take the cast to bfloat16 upon themselves."""
+    return type(self.dispatcher) is EinsumDispatcher and self.dispatcher._reads_rounded(data)
+
   def dispatch(self, data: Array) -> Array:
     dtype = data.dtype
+    if self._rounds_as_it_reads(data):
+      return K.cast(self.dispatcher.dispatch(data, torch.bfloat16), dtype)
     data = _cast_to_bfloat16(data)
     data = self.dispatcher.dispatch(data)
     return K.cast(data, dtype) if data.is_floating_point() else data
 
   def combine(self, data: Array) -> Array:
     dtype = data.dtype
+    if self._rounds_as_it_reads(data):
+      return K.cast(self.dispatcher.combine(data, torch.bfloat16), dtype)
     data = _cast_to_bfloat16(data)
     data = self.dispatcher.combine(data)
     return K.cast(data, dtype) if data.is_floating_point() else data
