@@ -1152,6 +1152,30 @@ def test_expert_mlp_float32_split_tiles_infinities(K, monkeypatch, tile):
   np.testing.assert_array_equal(got[same], clean[same])
 
 
+@pytest.mark.parametrize("tile", [7, 8])
+def test_expert_mlp_float32_four_groups_along_k(K, monkeypatch, tile):
+  """The tiles whose four groups take turns: the checks above, and against 64 bits where k leaves some of the groups
+  nothing, ends inside a group's share, or ends inside a k tile; ragged rows bit for bit as well."""
+  test_expert_mlp_float32_weights_at_any_address(K, monkeypatch, tile)
+  test_expert_mlp_float32_split_tiles_infinities(K, monkeypatch, tile)
+  monkeypatch.setenv("VMOE_F32_GEMM", f"tile{tile}")
+  for E, R, D, M in [(2, 33, 4, 36), (3, 65, 100, 260), (2, 129, 36, 132), (5, 7, 288, 68), (2, 64, 1028, 64)]:
+    gen = torch.Generator(device=dev()).manual_seed(D)
+    mk = lambda *s: torch.randn(s, generator=gen, device=dev())
+    x, w0, b0, w1, b1 = mk(E, R, D), mk(E, D, M) * D ** -0.5, mk(E, M), mk(E, M, D) * M ** -0.5, mk(E, D)
+    got = K.expert_mlp(x, w0, b0, w1, b1)
+    h = torch.nn.functional.gelu(torch.bmm(x.double(), w0.double()) + b0.double()[:, None], approximate="tanh")
+    want = torch.bmm(h, w1.double()) + b1.double()[:, None]
+    # (2-norm: sums of float32 products in float32 are off by less than 2^-24 times the square root of their number)
+    assert ((got.double() - want).norm() / want.norm()).item() <= max(D, M) ** 0.5 * 2.0 ** -23
+    rows = torch.randint(0, R + 1, (E,), generator=gen, device=dev(), dtype=torch.int32)
+    rows[0] = R
+    ragged = torch.full_like(got, 7.0)
+    K.expert_mlp(x, w0, b0, w1, b1, out=ragged, rows_per_expert=rows)
+    for e, n in enumerate(rows.tolist()):
+      assert torch.equal(ragged[e, :n], got[e, :n]) and bool((ragged[e, n:] == 7.0).all())
+
+
 def test_expert_mlp_float32_seeded_shapes(K):
   """A seeded sweep of float32 expert MLPs over odd shapes (rows short of a block, widths that
   end inside a tile, k that is or is not whole 32-wide tiles, many or few experts), dense and

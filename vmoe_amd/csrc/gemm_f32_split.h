@@ -17,8 +17,8 @@
 // Why: a float32 MFMA does 256 flops a clock and CU, a bfloat16 one 4 096: 683 after six products.
 // 9 216 rows, 768 x 3 072 (both products): 359 and 379 us (115 TFLOP/s, 0.74 of the float32 peak) on
 // float32 MFMAs with operands by LDS-DMA, 240 and 229 (185) here; 51 experts x ~330 rows x 896 x 1 984: 589 and
-// 611 to 398 and 406; 8 x 392 x 512 x 2 048: 81 and 79 to 50 and 62; 23 x 22 x 576 x 2 304: 38 and 48 to
-// 23 and 28.  The large shapes run at 1.1 PFLOP/s of bfloat16 MFMAs, which is where the
+// 611 to 398 and 406; 8 x 392 x 512 x 2 048: 81 and 79 to 50 and 51; 23 x 22 x 576 x 2 304: 38 and 48 to
+// 26 and 26.  The large shapes run at 1.1 PFLOP/s of bfloat16 MFMAs, which is where the
 // bfloat16 products of this library stand at the chip's power limit.
 //
 // Structure.  A k tile is fetched into registers (16-byte loads, one k tile ahead), split there and
@@ -32,7 +32,8 @@
 // (128 x 256 tiles, eight waves: 250 and 228 us on the 9 216 rows); three 128 x 128 workgroups per CU
 // (spills, 320); k tiles two or four ahead (no change).
 // KG groups of four waves in a workgroup take consecutive runs of k tiles, each through its own LDS,
-// and add their sums in group order: launches of few tiles are as long as one tile's chain of k tiles.
+// and add their sums in group order: launches of few tiles are as long as one tile's chain of k tiles.  Two or four
+// groups of the larger tiles take turns at splitting and multiplying.
 // The tile comes from the sizes of the call (kSplitTiles), so the order of an output's sums does too: the same item
 // through the same weights can differ in its last bits between calls over different numbers of rows or experts
 // (not between dense, ragged and gathered calls of one size), as bfloat16 MLPs can.
@@ -40,6 +41,8 @@
 // numbered batch-major, column panel by column panel, and cut into eight equal runs, one per XCD, so that
 // the row tiles that share a column panel of weights run on one die at the same time.
 #pragma once
+#include <cmath>
+
 #include "gemm_bf16.h"
 
 namespace vmoe {
@@ -68,6 +71,7 @@ struct SplitCfg {
   static constexpr int kPiece = kStage > kOutBytes ? (kStage > kSumBytes ? kStage : kSumBytes)
                                                    : (kOutBytes > kSumBytes ? kOutBytes : kSumBytes);
   static constexpr int kLds = KG * kPiece;
+  static constexpr bool kTurns = KG > 2 || (KG == 2 && BM * BN >= 64 * 128);      // groups take turns (see below)
   static_assert(AI >= 1 && BU >= 1, "tile");
 };
 
@@ -257,9 +261,14 @@ __global__ __launch_bounds__(Cfg::kThreads, Cfg::kWgs * Cfg::kThreads / 256) voi
   // A group's k tiles are consecutive; where they do not divide evenly the last group's run past
   // the end, where fetch() finds zeros.
   const int nk = ((Kd + BK - 1) / BK + Cfg::KG - 1) / Cfg::KG, kt0 = group * nk;
+  // Turns: between two barriers every other group splits and the rest multiply.  (In step, all of a SIMD's waves want
+  // its vector instructions first and its matrix core then: 8 x 392 rows x 2 048 x 512 on 64 x 128 tiles and two
+  // groups 61 -> 54 us.  The smaller two-group tiles, four workgroups of which share a CU, lose 0 - 7 %; tiles
+  // without groups fall out of step by themselves, and lost as two tiles of one workgroup: 50 -> 53, 235 -> 252.)
   fetch(kt0);
+  if (Cfg::kTurns && (group & 1)) raw_barrier();
   for (int s = 0; s < nk; ++s) {
-    if (s > 0) raw_barrier();               // every wave has read the k tile before
+    if (!Cfg::kTurns && s > 0) raw_barrier();      // every wave has read the k tile before
     __builtin_amdgcn_s_setprio(2);
 #pragma unroll
     for (int u = 0; u < kUnits; ++u) stage_unit(u);
@@ -268,9 +277,11 @@ __global__ __launch_bounds__(Cfg::kThreads, Cfg::kWgs * Cfg::kThreads / 256) voi
     __builtin_amdgcn_s_setprio(0);
     raw_barrier();
     if (blocks > 0) multiply();
+    if (Cfg::kTurns) raw_barrier();
   }
+  if (Cfg::kTurns && !(group & 1)) raw_barrier();
   mfma_result_fence();
-  raw_barrier();                               // the operands' LDS is free
+  if (!Cfg::kTurns) raw_barrier();               // the operands' LDS is free
   if constexpr (Cfg::KG > 1) {
     f32x4_t* sums = reinterpret_cast<f32x4_t*>(piece);
     if (group > 0) {
@@ -282,7 +293,7 @@ __global__ __launch_bounds__(Cfg::kThreads, Cfg::kWgs * Cfg::kThreads / 256) voi
     wait_lgkmcnt0();
     raw_barrier();
     if (group > 0) return;
-#pragma unroll
+#pragma unroll 1
     for (int g = 1; g < Cfg::KG; ++g)
 #pragma unroll
       for (int i = 0; i < FM; ++i)
@@ -366,34 +377,51 @@ int launch_gemm_f32_split_tile(const float* A, const float* B, const float* bias
 }
 
 // Tiles, with what they cost: a 32-wide step of k takes `work` us of a CU's time per tile, `latency` us alone on a
-// CU, a tile `fix` us besides.  A launch is taken to last 4 us plus the 4-norm of one tile's chain and the
-// fullest CU's work, with R rows in every batch (the counts are on the device; dense and ragged calls of
-// one shape take the same tile and so the same order of sums).  Tiles per CU count as halfway between
-// whole ones and even ones.  Fitted to 34 random shapes (1 - 37 experts, 26 - 7 001 rows, widths 256 - 4 096), every tile on both
-// products, rms 8 - 14 % per tile: the 68 products take 4 412 us on the tiles chosen, 4 327 on the
-// best of each, and 4 726 without the 96-row tile on constants fitted to eleven shapes (23 other shapes: 4 039, 3 877
-// and 4 154); the worst choice costs 23 %.
-struct SplitTile { int bm, bn; double work, latency, fix; };
+// CU, a tile `fix` us besides.  A launch is taken to last the 4-norm of one tile's chain and the fullest CU's work.
+// Tiles per CU count as halfway between whole ones and even ones; four groups along k fill a CU, and are for launches
+// of a tile per CU at most (with two rounds of them the others win, and constants fitted to both miss by 12 %).
+// How many of the R rows are live stands on the device, and a dense call keeps the order of sums of a ragged
+// one of its shape, so the tile may not depend on it: it is the one with the least time for all rows and for 35 % of
+// them together.  (By the time for all rows alone a launch whose experts are half empty takes 128-row tiles where
+// 32 rows are live: 38 experts of up to 92 rows, 3328 to 832, 167 us on 96 x 128 and 116 on 32 x 64.)  Four groups
+// have to be 15 % ahead: their time is the chain's, which fewer rows do not shorten.
+// Fitted to 90 random shapes (1 - 64 experts, 16 - 9 000 rows, widths 192 - 4 096), every tile on both products, rms
+// 6 - 10 % per tile; chosen on them and on 80 ragged ones, a quarter to all of their rows live.  Before groups took
+// turns and before there were four of them the 180 products with all rows took 12 827 us and take 12 363 (4 % in the
+// geometric mean; 12 018 by the time for all rows alone, 11 792 on the best tile of each), the 160 ragged ones 12 620
+// and 11 827 (6 %; 12 182 by the time for all rows alone; 11 030).
+struct SplitTile { int bm, bn; double work, latency, fix; bool fills_cu; };
 constexpr SplitTile kSplitTiles[] = {
-    {128, 128, 1.09, 1.61, 2.7},   // two workgroups per CU
-    {64, 128, 0.59, 1.14, 2.0},    // four
-    {64, 128, 0.60, 0.84, 2.9},    // two groups of waves along k
-    {32, 128, 0.42, 0.88, 1.0},
-    {32, 128, 0.42, 0.57, 1.6},    // two groups
-    {32, 64, 0.25, 0.29, 1.0},     // two groups
-    {96, 128, 0.77, 1.39, 3.7},    // two workgroups per CU
+    {128, 128, 1.13, 1.53, 3.7, false},   // two workgroups per CU
+    {64, 128, 0.67, 1.08, 1.1, false},    // four
+    {64, 128, 0.68, 0.47, 2.0, false},    // two groups of waves along k
+    {32, 128, 0.48, 0.83, 0.4, false},
+    {32, 128, 0.49, 0.48, 1.2, false},    // two groups
+    {32, 64, 0.28, 0.23, 1.0, false},     // two groups
+    {96, 128, 0.90, 1.35, 1.9, false},    // two workgroups per CU
+    {64, 128, 0.48, 0.49, 4.1, true},     // four groups
+    {32, 64, 0.10, 0.28, 1.6, true},      // four groups
 };
 constexpr int kNumSplitTiles = sizeof(kSplitTiles) / sizeof(kSplitTiles[0]);
 
 inline int best_split_tile(int batch, int R, int N, int Kd) {
+  const int few_rows = std::max(1, (int)(0.35 * R));
   int best = 0;
   double best_us = 1e30;
   for (int i = 0; i < kNumSplitTiles; ++i) {
     const SplitTile& t = kSplitTiles[i];
-    const double per_cu = (double)batch * ((R + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) / (kCusPerXcd * kNumXcd);
-    const double tiles = std::max(1.0, 0.5 * (std::ceil(per_cu) + per_cu + 0.3)), steps = (Kd + 31) / 32;
-    const double chain = steps * t.latency, busy = tiles * (steps * t.work + t.fix);
-    const double us = chain * chain * chain * chain + busy * busy * busy * busy;
+    const double steps = (Kd + 31) / 32;
+    auto tiles_per_cu = [&](int rows) {
+      return (double)batch * ((rows + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) / (kCusPerXcd * kNumXcd);
+    };
+    if (t.fills_cu && tiles_per_cu(R) > 1) continue;
+    auto time = [&](int rows) {
+      const double per_cu = tiles_per_cu(rows);
+      const double tiles = t.fills_cu ? 1.0 : std::max(1.0, 0.5 * (std::ceil(per_cu) + per_cu + 0.3));
+      const double chain = steps * t.latency, busy = tiles * (steps * t.work + t.fix);
+      return std::sqrt(std::sqrt(chain * chain * chain * chain + busy * busy * busy * busy));
+    };
+    const double us = (t.fills_cu ? 1.15 : 1.0) * (time(R) + time(few_rows));
     if (us < best_us) { best_us = us; best = i; }
   }
   return best;
@@ -413,6 +441,8 @@ int launch_gemm_f32_split(int tile, const float* A, const float* B, const float*
     case 3: return run(SplitCfg<32, 128, 1, 4, 32, 4, 1>{});
     case 4: return run(SplitCfg<32, 128, 1, 4, 32, 2, 2>{});
     case 5: return run(SplitCfg<32, 64, 2, 2, 64, 2, 2>{});
+    case 7: return run(SplitCfg<64, 128, 2, 2, 32, 1, 4>{});
+    case 8: return run(SplitCfg<32, 64, 2, 2, 64, 1, 4>{});
     default: return run(SplitCfg<96, 128, 2, 2, 32, 2, 1>{});
   }
 }
