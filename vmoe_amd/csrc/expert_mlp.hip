@@ -434,18 +434,18 @@ MlpPlans mlp_plans(int E, int R, int D, int M, bool ragged, long long items) {
     return forced < kNumRowsTiles || stream_tile_ok(forced - kNumRowsTiles, E, R, Kd, ragged);
   };
   if (any_tile && rows_gemm_ok(R, M, D, items)) {
-    const double us = m.up.fast ? product_us(D % 64 == 0 ? kFirstProductTile : kFirstProductK32Tile, E, R, M, D, true, false) : 1e30;
+    const double us = m.up.fast ? launch_us(D % 64 == 0 ? kFirstProductTile : kFirstProductK32Tile, E, R, M, D, true, false, ragged) : 1e30;
     m.up_rows = best_tile(E, R, M, D, items, ragged, true, us);
     if (forced_ok(M, D, items)) m.up_rows = forced;
   }
   if (any_tile && rows_gemm_ok(R, D, M, 0)) {
     double us = 1e30;
     if (m.down_kernel == kDownEightWaves || m.down_kernel == kDownNarrow)
-      us = product_us(m.down_kernel == kDownNarrow ? kNarrowTile : kEightWavesTile, E, R, D, M, false, false);
+      us = launch_us(m.down_kernel == kDownNarrow ? kNarrowTile : kEightWavesTile, E, R, D, M, false, false, ragged);
     else if (t_best < 1e29)
-      us = 5 + t_best;
+      us = 5 + (ragged ? 0.7 : 1) * t_best;
     else if (square.fast)
-      us = 5 + unit * (half ? 0.5 * 1.05 * std::ceil((double)E * ((R + 127) / 128) * ((D + 255) / 256) / kNumCu)
+      us = 5 + (ragged ? 0.7 : 1) * unit * (half ? 0.5 * 1.05 * std::ceil((double)E * ((R + 127) / 128) * ((D + 255) / 256) / kNumCu)
                             : std::ceil((double)square.tiles / kNumCu));
     m.down_rows = best_tile(E, R, D, M, 0, ragged, false, us);
     if (forced_ok(D, M, 0)) m.down_rows = forced;

@@ -90,6 +90,16 @@ inline double product_us(const RowsTile& t, int batch, int R, int N, int Kd, boo
   return 2 + std::sqrt(std::sqrt(b2 * b2 + m2 * m2 + f2 * f2));
 }
 
+// The same for a launch whose live rows are counted on the device: the mean over full, 70 % full and 40 % full
+// experts.  On 80 random ragged layers, 23 % to all of their rows live, the choice by this mean takes 6 514 us for the
+// 160 products, by the time of full experts 6 566 and 39 % too long at worst instead of 18 %, on the best tile of each 6 113.
+inline double launch_us(const RowsTile& t, int batch, int R, int N, int Kd, bool gelu, bool whole_pairs, bool ragged) {
+  const double us = product_us(t, batch, R, N, Kd, gelu, whole_pairs);
+  if (!ragged) return us;
+  return (us + product_us(t, batch, (int)std::ceil(0.7 * R), N, Kd, gelu, whole_pairs) +
+          product_us(t, batch, (int)std::ceil(0.4 * R), N, Kd, gelu, whole_pairs)) / 3;
+}
+
 // The tiles of gemm_bf16_stream_kernel, and what the choice
 // is made from: a CU takes its tiles one after the other at step_us per 64 k, with the GELU's or the plain
 // epilogue behind each, and the launch cannot beat its weights at w_tbs plus its rows, once per column
@@ -177,7 +187,7 @@ inline int best_tile(int batch, int R, int N, int Kd, long long items, bool ragg
   auto take_tile = [&](int i, const RowsTile& t) {
     const bool mid = is_mid_tile(i);
     if (!mid || mid_ok)
-      take(i, product_us(t, batch, R, N, Kd, gelu, !mid || (ragged && !mid_tile_planned(batch, R, t.bm))));
+      take(i, launch_us(t, batch, R, N, Kd, gelu, !mid || (ragged && !mid_tile_planned(batch, R, t.bm)), ragged));
   };
   for (int i = 0; i < kNumRowsTiles; ++i) take_tile(i, kRowsTiles[i]);
   for (int i = 0; i < kNumMoreTiles; ++i) take_tile(kFirstMoreTile + i, kMoreTiles[i]);
