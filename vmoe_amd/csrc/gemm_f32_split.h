@@ -381,47 +381,55 @@ int launch_gemm_f32_split_tile(const float* A, const float* B, const float* bias
 // Tiles per CU count as halfway between whole ones and even ones; four groups along k fill a CU, and are for launches
 // of a tile per CU at most (with two rounds of them the others win, and constants fitted to both miss by 12 %).
 // How many of the R rows are live stands on the device, and a dense call keeps the order of sums of a ragged
-// one of its shape, so the tile may not depend on it: it is the one with the least time for all rows and for 35 % of
-// them together.  (By the time for all rows alone a launch whose experts are half empty takes 128-row tiles where
-// 32 rows are live: 38 experts of up to 92 rows, 3328 to 832, 167 us on 96 x 128 and 116 on 32 x 64.)  Four groups
-// have to be 15 % ahead: their time is the chain's, which fewer rows do not shorten.
+// one of its shape, so the tile may not depend on it.  Tiles whose groups take turns are taken where they are 5 %
+// ahead of the best of the others for all rows and for 35 % of them together: their time is the chain's, which fewer
+// rows do not shorten (18 experts of up to 88 rows, 393 in all, 2560 to 640: 53 us on four groups, 37 on 32 x 64).
 // Fitted to 90 random shapes (1 - 64 experts, 16 - 9 000 rows, widths 192 - 4 096), every tile on both products, rms
 // 6 - 10 % per tile; chosen on them and on 80 ragged ones, a quarter to all of their rows live.  Before groups took
-// turns and before there were four of them the 180 products with all rows took 12 827 us and take 12 363 (4 % in the
-// geometric mean; 12 018 by the time for all rows alone, 11 792 on the best tile of each), the 160 ragged ones 12 620
-// and 11 827 (6 %; 12 182 by the time for all rows alone; 11 030).
-struct SplitTile { int bm, bn; double work, latency, fix; bool fills_cu; };
+// turns and before there were four of them the 180 products with all rows took 12 827 us and take 12 385 (5 % in the
+// geometric mean; 11 792 on the best tile of each), the 160 ragged ones 12 620 and 12 177 (4 %; 11 030).
+struct SplitTile {
+  int bm, bn;
+  double work, latency, fix;
+  bool turns, fills_cu;
+};
 constexpr SplitTile kSplitTiles[] = {
-    {128, 128, 1.13, 1.53, 3.7, false},   // two workgroups per CU
-    {64, 128, 0.67, 1.08, 1.1, false},    // four
-    {64, 128, 0.68, 0.47, 2.0, false},    // two groups of waves along k
-    {32, 128, 0.48, 0.83, 0.4, false},
-    {32, 128, 0.49, 0.48, 1.2, false},    // two groups
-    {32, 64, 0.28, 0.23, 1.0, false},     // two groups
-    {96, 128, 0.90, 1.35, 1.9, false},    // two workgroups per CU
-    {64, 128, 0.48, 0.49, 4.1, true},     // four groups
-    {32, 64, 0.10, 0.28, 1.6, true},      // four groups
+    {128, 128, 1.09, 1.61, 2.7, false, false},   // two workgroups per CU
+    {64, 128, 0.59, 1.14, 2.0, false, false},    // four
+    {64, 128, 0.68, 0.47, 2.0, true, false},     // two groups of waves along k
+    {32, 128, 0.42, 0.88, 1.0, false, false},
+    {32, 128, 0.42, 0.57, 1.6, false, false},    // two groups
+    {32, 64, 0.25, 0.29, 1.0, false, false},     // two groups
+    {96, 128, 0.77, 1.39, 3.7, false, false},    // two workgroups per CU
+    {64, 128, 0.48, 0.49, 4.1, true, true},      // four groups
+    {32, 64, 0.10, 0.28, 1.6, true, true},       // four groups
 };
 constexpr int kNumSplitTiles = sizeof(kSplitTiles) / sizeof(kSplitTiles[0]);
 
 inline int best_split_tile(int batch, int R, int N, int Kd) {
-  const int few_rows = std::max(1, (int)(0.35 * R));
+  const double steps = (Kd + 31) / 32;
+  auto tiles_per_cu = [&](const SplitTile& t, int rows) {
+    return (double)batch * ((rows + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) / (kCusPerXcd * kNumXcd);
+  };
+  auto time = [&](const SplitTile& t, int rows) {
+    const double per_cu = tiles_per_cu(t, rows);
+    const double tiles = t.fills_cu ? 1.0 : std::max(1.0, 0.5 * (std::ceil(per_cu) + per_cu + 0.3));
+    const double chain = steps * t.latency, busy = tiles * (steps * t.work + t.fix);
+    return std::sqrt(std::sqrt(chain * chain * chain * chain + busy * busy * busy * busy));
+  };
   int best = 0;
   double best_us = 1e30;
   for (int i = 0; i < kNumSplitTiles; ++i) {
+    if (kSplitTiles[i].turns) continue;
+    const double us = time(kSplitTiles[i], R);
+    if (us < best_us) { best_us = us; best = i; }
+  }
+  const int few_rows = std::max(1, (int)(0.35 * R));
+  best_us = 0.95 * (best_us + time(kSplitTiles[best], few_rows));
+  for (int i = 0; i < kNumSplitTiles; ++i) {
     const SplitTile& t = kSplitTiles[i];
-    const double steps = (Kd + 31) / 32;
-    auto tiles_per_cu = [&](int rows) {
-      return (double)batch * ((rows + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) / (kCusPerXcd * kNumXcd);
-    };
-    if (t.fills_cu && tiles_per_cu(R) > 1) continue;
-    auto time = [&](int rows) {
-      const double per_cu = tiles_per_cu(rows);
-      const double tiles = t.fills_cu ? 1.0 : std::max(1.0, 0.5 * (std::ceil(per_cu) + per_cu + 0.3));
-      const double chain = steps * t.latency, busy = tiles * (steps * t.work + t.fix);
-      return std::sqrt(std::sqrt(chain * chain * chain * chain + busy * busy * busy * busy));
-    };
-    const double us = (t.fills_cu ? 1.15 : 1.0) * (time(R) + time(few_rows));
+    if (!t.turns || (t.fills_cu && tiles_per_cu(t, R) > 1)) continue;
+    const double us = time(t, R) + time(t, few_rows);
     if (us < best_us) { best_us = us; best = i; }
   }
   return best;
