@@ -160,6 +160,21 @@ def test_add_layer_norm_kernel(rows, D, branch_dtype, out_dtype):
                              atol=2e-5)
 
 
+@pytest.mark.parametrize("D", [256, 768, 2048])
+def test_add_layer_norm_on_either_side_of_the_caches(D):
+  """A residual stream of more than 16 MB goes past the caches, a smaller one through them: the same bits row by
+  row, also where the sum is written over the residual."""
+  from vmoe_amd import kernels as K
+  rows = 2 ** 24 // (4 * D)
+  gen = torch.Generator(device=dev()).manual_seed(D)
+  mk = lambda *s: torch.randn(*s, generator=gen, device=dev())
+  x, branch, scale, bias = mk(rows + 1, D), mk(rows + 1, D).bfloat16(), mk(D), mk(D)
+  parts = [K.add_layer_norm(x[a:b], branch[a:b], scale, bias, 1e-6, torch.bfloat16) for a, b in ((0, rows), (rows, rows + 1))]
+  whole = K.add_layer_norm(x, branch, scale, bias, 1e-6, torch.bfloat16)
+  for got, pieces in zip(whole, zip(*parts)):
+    assert torch.equal(got, torch.cat(pieces))
+
+
 @pytest.mark.parametrize("B,H,Sq,Sk,packed", [
     (2, 3, 196, 196, True), (2, 2, 197, 197, True), (3, 2, 1, 50, False), (1, 4, 33, 33, True),
     (2, 2, 300, 300, True), (1, 2, 64, 512, False), (1, 1, 40, 7, False)])

@@ -3,6 +3,8 @@
 // follows it, and softmax attention over one image's tokens.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "vmoe_common.h"
 #include "vmoe_hip.h"
 
@@ -11,6 +13,11 @@ namespace {
 
 constexpr int kLnThreads = 256;
 constexpr int kLnWaves = kLnThreads / 64;
+// Up to this size the residual stream is read and written through the caches, where the next add + norm, a few
+// products further on, finds it again; above it goes past them.  Both ways in the B/16 model, per launch and all
+// kernels of a pass: 8 images (4.8 MB) 6.4 past the caches, 5.8 through them (1 394 and 1 374 us), 24 images (14.5 MB)
+// 10.2 and 8.9 (2 180 and 2 139), 64 images (38 MB) 21.6 and 21.3 (4 148 and 4 214), 512 images 141 and 157.
+constexpr size_t kLnCachedBytes = 16u << 20;
 
 template <typename T> struct Vec4;
 template <> struct Vec4<float> {
@@ -62,7 +69,7 @@ __device__ __forceinline__ float wave_sum(float v) {
 //   norm_out = (x - mean) * rsqrt(var + eps) * scale + bias,  var = E[x^2] - E[x]^2
 // which is flax.linen.LayerNorm's arithmetic (float32 statistics, "fast variance").
 // Every element is read once and written once: HBM-bound.
-template <typename TB, typename TO, int NV>
+template <typename TB, typename TO, int NV, bool STREAM>
 __global__ __launch_bounds__(kLnThreads) void add_layer_norm_kernel(
     const float* residual, const TB* __restrict__ branch,
     const float* __restrict__ scale, const float* __restrict__ bias,
@@ -91,12 +98,15 @@ __global__ __launch_bounds__(kLnThreads) void add_layer_norm_kernel(
       const int c = lane + 64 * i;
       v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
       if (c < chunks) {
-        v[i] = Vec4<float>::load_stream(residual + base + 4 * c);
+        v[i] = STREAM ? Vec4<float>::load_stream(residual + base + 4 * c) : Vec4<float>::load(residual + base + 4 * c);
         if (branch != nullptr) {
-          const float4 b = Vec4<TB>::load_stream(branch + base + 4 * c);
+          const float4 b = STREAM ? Vec4<TB>::load_stream(branch + base + 4 * c) : Vec4<TB>::load(branch + base + 4 * c);
           v[i].x += b.x; v[i].y += b.y; v[i].z += b.z; v[i].w += b.w;
         }
-        if (residual_out != nullptr) Vec4<float>::store_stream(residual_out + base + 4 * c, v[i]);
+        if (residual_out != nullptr) {
+          if (STREAM) Vec4<float>::store_stream(residual_out + base + 4 * c, v[i]);
+          else Vec4<float>::store(residual_out + base + 4 * c, v[i]);
+        }
       }
       s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
       s2 += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
@@ -170,9 +180,14 @@ int launch_add_layer_norm(const VmoeAddLayerNormParams* p, hipStream_t stream) {
                    (reinterpret_cast<uintptr_t>(br) & 7u) == 0 &&
                    (reinterpret_cast<uintptr_t>(out) & 7u) == 0 &&
                    (sizeof(TB) == 2 || aligned16(br)) && (sizeof(TO) == 2 || aligned16(out));
-#define VMOE_LN_CASE(NV)                                                                      \
-  hipLaunchKernelGGL((add_layer_norm_kernel<TB, TO, NV>), grid, block, 0, stream, res, br,    \
-                     p->scale, p->bias, p->residual_out, out, rows, D, p->eps)
+  const bool streamed = (size_t)rows * D * sizeof(float) > kLnCachedBytes;
+  auto run = [&](auto nv, auto st) {
+    hipLaunchKernelGGL((add_layer_norm_kernel<TB, TO, decltype(nv)::value, decltype(st)::value>), grid, block, 0, stream,
+                       res, br, p->scale, p->bias, p->residual_out, out, rows, D, p->eps);
+  };
+#define VMOE_LN_CASE(NV)                                                     \
+  if (streamed) run(std::integral_constant<int, NV>{}, std::true_type{});    \
+  else run(std::integral_constant<int, NV>{}, std::false_type{})
   if (!vec) {
     hipLaunchKernelGGL((add_layer_norm_generic_kernel<TB, TO>), grid, block, 0, stream, res, br,
                        p->scale, p->bias, p->residual_out, out, rows, D, p->eps);
