@@ -424,3 +424,23 @@ def test_dense_stands_aside_where_torch_has_to_see_the_product(vit_moe):
   assert torch.allclose(plain, both[0], rtol=1e-4, atol=1e-3)
   _, tangent = torch.func.jvp(lambda t: vit_moe._affine(t, w, b), (x,), (x,))
   assert torch.allclose(tangent, plain - b, rtol=1e-4, atol=2e-3)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_dense_operands_at_odd_addresses(vit_moe, dtype):
+  """Rows, weights and biases that start inside a larger buffer, off the 16 bytes that the kernels read, give what
+  aligned copies give (float32 sums of D products in two orders, rounded to eight bits in bfloat16)."""
+  rows, D, M = 1301, 1000, 1016
+  gen = torch.Generator(device=dev()).manual_seed(1)
+  off = lambda *s: torch.randn(int(np.prod(s)) + 1, generator=gen, device=dev()).to(dtype)[1:].view(s)
+  x, w, b = off(1, rows, D), off(D, M) if dtype == torch.float32 else off(M, D), off(M)
+  assert x.data_ptr() % 16 and w.data_ptr() % 16
+  project = vit_moe.MultiHeadDotProductAttention._project
+  forms = [project] + ([vit_moe._affine] if dtype == torch.float32 else [])
+  mat = (w if dtype == torch.float32 else w.t()).double()
+  want = x.double() @ mat + b.double()
+  size = x.double().abs() @ mat.abs() + 1
+  bound = size * D ** 0.5 * 2.0 ** -23 + (want.abs() * 2.0 ** -8 if dtype == torch.bfloat16 else 0)
+  for form in forms:
+    for args in ((x, w, b), (x.clone(), w, b), (x, w.clone(), b)):
+      assert bool(((form(*args).double() - want).abs() <= bound).all())

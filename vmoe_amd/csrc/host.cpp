@@ -474,12 +474,13 @@ std::tuple<Tensor, Tensor> combine_backward(int64_t stream, const Tensor& dout_,
 }
 
 // x (..., D) . w + b -> (..., M), rounded once: float32 w (D, M), bfloat16 w transposed (M, D).
-Tensor dense(int64_t stream, const Tensor& x_, const Tensor& w, const OptTensor& b) {
+Tensor dense(int64_t stream, const Tensor& x_, const Tensor& w_, const OptTensor& b_) {
   if (x_.dim() < 2) need_axes(x_, 2, "x");
-  need_axes(w, 2, "w");
-  need_type_of(w, x_, "w", "x");
-  if (b.has_value()) need_type_of(*b, x_, "bias", "x");
-  const Tensor x = x_.contiguous();
+  need_axes(w_, 2, "w");
+  need_type_of(w_, x_, "w", "x");
+  if (b_.has_value()) need_type_of(*b_, x_, "bias", "x");
+  const Tensor x = x_.contiguous(), w = w_.contiguous();
+  const OptTensor b = b_.has_value() ? OptTensor(b_->contiguous()) : b_;
   const bool f32 = x.scalar_type() == at::kFloat;
   const int64_t D = x.size(-1), M = w.size(f32 ? 1 : 0);
   if (w.size(f32 ? 0 : 1) != D)

@@ -668,12 +668,19 @@ def dense_pays(rows: int, D: int, M: int, dtype: torch.dtype) -> bool:
   return dtype == torch.float32 and D % 4 == 0 and M % 4 == 0 and work >= 1.3e9 and rows < 1 << 31
 
 
+def dense_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
+  """Whether the operands start where dense() can read them (16 bytes; float32 weights anywhere): a view into a
+  larger buffer may not, and takes the library's product."""
+  return (x.data_ptr() | (0 if w.dtype == torch.float32 else w.data_ptr())) % 16 == 0
+
+
 def dense(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor]) -> torch.Tensor:
   """x (..., D) . w + b -> (..., M), rounded once.  float32: w (D, M), products as sums of three bfloat16
   values per operand; bfloat16: w (M, D), transposed."""
   if not H.timed("vmoe_dense"):
     return H.host().dense(H.raw_stream(), x, w, b)
-  x = x.contiguous()
+  x, w = x.contiguous(), w.contiguous()
+  b = b.contiguous() if b is not None else None
   D, f32 = x.shape[-1], x.dtype == torch.float32
   M = w.shape[1 if f32 else 0]
   out = torch.empty((*x.shape[:-1], M), dtype=x.dtype, device=x.device)

@@ -229,7 +229,8 @@ def _affine(x: Array, w: Array, b: Array) -> Array:
   """x (..., D) . w (D, M) + b in float32: the package's own product where it is the faster one."""
   D, M = w.shape
   if (x.dtype == w.dtype == b.dtype and w.is_contiguous() and b.is_contiguous()
-      and K.dense_pays(x.numel() // D, D, M, x.dtype) and module.is_plain(x, w, b)):
+      and K.dense_pays(x.numel() // D, D, M, x.dtype) and module.is_plain(x, w, b)
+      and K.dense_takes(x, w)):
     return K.dense(x, w, b)
   return torch.addmm(b, x.reshape(-1, D), w).view(*x.shape[:-1], M)
 
@@ -309,7 +310,7 @@ class MultiHeadDotProductAttention(module.Module):
   def _project(x: Array, w: Array, b: Array) -> Array:
     """x . w + b for a weight of _proj_weights: the package's own product where it is the faster one."""
     D, M = w.shape if w.dtype == torch.float32 else reversed(w.shape)
-    if K.dense_pays(x.numel() // D, D, M, w.dtype) and module.is_plain(x, w, b):
+    if K.dense_pays(x.numel() // D, D, M, w.dtype) and module.is_plain(x, w, b) and K.dense_takes(x, w):
       return K.dense(x, w, b)
     return torch.nn.functional.linear(x, w.t() if w.dtype == torch.float32 else w, b)
 
