@@ -1376,6 +1376,34 @@ def test_expert_mlp_medium_tiles(K, monkeypatch, tile):
         assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
+@pytest.mark.parametrize("second", ["eight", "narrow"])
+@pytest.mark.parametrize("rows", [1, 16, 33, 63, 64, 65, 96, 97, 127, 128, 129, 161, 193, 255, 256, 257, 449])
+def test_expert_mlp_last_tiles_of_the_large_kernels(K, monkeypatch, rows, second):
+  """The large tiles multiply the live row blocks of an expert's last tile only: every number of them, at one row
+  either side, in dense and ragged calls (experts without a row, with one tile and with several among them), bit for
+  bit what the smallest tile computes (same order of sums), and nothing written past the live rows."""
+  E, D, M = 5, 320, 456 if second == "eight" else 392
+  M += -M % 64                                             # (k of the second product: whole 64s, from 256 on)
+  rng = np.random.default_rng(rows)
+  mk = lambda scale, *s: to_dev(O.cast(rng.standard_normal(s).astype(np.float32) * scale, O.BF16), O.BF16)
+  x, w0, w1 = mk(1, E, rows, D), mk(D ** -0.5, E, D, M), mk(M ** -0.5, E, M, D)
+  b0, b1 = mk(0.1, E, M), mk(0.1, E, D)
+  counts = torch.tensor([rows, 0, min(rows, 1), (rows + 1) // 2, max(rows - 30, 0)], dtype=torch.int32, device=dev())
+
+  def run(large, live):
+    monkeypatch.setenv("VMOE_ROW_TILES", "off" if large else "0")
+    monkeypatch.setenv("VMOE_SECOND_PRODUCT", second if large else "")
+    out = torch.full((E, rows, D), 7.0, dtype=torch.bfloat16, device=dev())
+    K.expert_mlp(x, w0, b0, w1, b1, out=out, rows_per_expert=live)
+    return out
+
+  for live in (None, counts):
+    got, want = run(True, live), run(False, live)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    for e, n in enumerate(counts.tolist() if live is not None else []):
+      assert bool((got[e, n:] == 7.0).all())
+
+
 @pytest.mark.parametrize("tile", range(8, 13))
 @pytest.mark.parametrize("E,R,D,M", [
     (130, 64, 640, 776),     # several tiles per workgroup, column tiles and k that end inside

@@ -159,8 +159,9 @@ __device__ __forceinline__ void load_bias(uint2 (&bias_pk)[TN / 8], const bf16_t
 }
 
 // The staged wave tile (TM rows of TN + 8 bfloat16 at `so`) to memory as 16-byte
-// row-contiguous pieces.
-template <int EPI, int TM, int TN>
+// row-contiguous pieces.  BLOCK: rows per block of the wave, blocks of WAVES waves take turns in the tile
+// (one wave: its rows are consecutive).
+template <int EPI, int TM, int TN, int WAVES = 1, int BLOCK = 16>
 __device__ __forceinline__ void store_staged_tile(const bf16_t* so, int lane, bf16_t* __restrict__ C,
                                                   int b, int R, int live, int N, int wrow0, int wcol0) {
   constexpr int OLD = TN + 8;
@@ -169,6 +170,7 @@ __device__ __forceinline__ void store_staged_tile(const bf16_t* so, int lane, bf
   constexpr int kChunksOut = TN / 8;                  // 16-byte chunks per staged row
   constexpr int kRowsPerPass = 64 / kChunksOut;
   static_assert(64 % kChunksOut == 0, "wave tile width must divide a wave");
+  static_assert(BLOCK % kRowsPerPass == 0, "a pass stays inside a block");
   const int oc = (lane % kChunksOut) * 8;
   const int orow = lane / kChunksOut;
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -197,7 +199,7 @@ __device__ __forceinline__ void store_staged_tile(const bf16_t* so, int lane, bf
         v[t] = *reinterpret_cast<const uint4*>(so + (r0 + t * kRowsPerPass + orow) * OLD + oc);
 #pragma unroll
       for (int t = 0; t < kBatch; ++t) {
-        const int rs = r0 + t * kRowsPerPass;
+        const int rs = (r0 + t * kRowsPerPass) / BLOCK * (BLOCK * WAVES) + (r0 + t * kRowsPerPass) % BLOCK;
         const bool ok = col_ok && orow < live - (row_u + rs);
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v[t]), c_rsrc,
                                                ok ? lane_off : 0xfffffff0u,
@@ -211,7 +213,7 @@ __device__ __forceinline__ void store_staged_tile(const bf16_t* so, int lane, bf
 #pragma unroll
   for (int r0 = 0; r0 < TM; r0 += kRowsPerPass) {
     const int rl = r0 + orow;
-    const int row = wrow0 + rl;
+    const int row = wrow0 + rl / BLOCK * (BLOCK * WAVES) + rl % BLOCK;
     const int col = wcol0 + oc;
     uint4 v = *reinterpret_cast<const uint4*>(so + rl * OLD + oc);
     if (row < live && col + 8 <= N) {
@@ -711,13 +713,14 @@ __global__ __launch_bounds__(Cfg::kThreads, Cfg::kBlocksPerCu) void gemm_bf16_ke
 // written with 32x32x16 MFMAs (two slices of eight per iteration, barrier between them) took
 // 0.970 - 0.977 ms per step of the B/16 layer against 0.949 - 0.957 (three alternating pairs).
 // store_tile for sums in the layout of v_mfma_f32_16x16x32_bf16 with the B fragment first:
-// acc[i][j][v] = C[row i * 16 + lane % 16][column j * 16 + (lane / 16) * 4 + v].
-template <int EPI, int TM, int TN>
+// acc[i][j][v] = C[row i * 16 WAVES + lane % 16][column j * 16 + (lane / 16) * 4 + v]; only the wave's first
+// BLOCKS row blocks hold live rows.
+template <int EPI, int TM, int TN, int WAVES, int BLOCKS>
 __device__ __forceinline__ void store_tile16(floatx4 (&acc)[TM / 16][TN / 16], unsigned char* smem,
                                              int wave, int lane, const uint2 (&bias_pk)[TN / 16],
                                              bool has_bias, bf16_t* __restrict__ C, int b, int R,
                                              int live, int N, int wrow0, int wcol0) {
-  constexpr int FM = TM / 16, FN = TN / 16, OLD = TN + 8;
+  constexpr int FN = TN / 16, OLD = TN + 8;
   const int n16 = lane & 15, g4 = lane >> 4;
   bf16_t* so = reinterpret_cast<bf16_t*>(smem) + (size_t)wave * TM * OLD;
   auto stage = [&](auto has_bias_c) {
@@ -728,7 +731,7 @@ __device__ __forceinline__ void store_tile16(floatx4 (&acc)[TM / 16][TN / 16], u
       const uint2 bp = bias_pk[j];
       const float bv[4] = {bf_lo(bp.x), bf_hi(bp.x), bf_lo(bp.y), bf_hi(bp.y)};
 #pragma unroll
-      for (int i = 0; i < FM; ++i) {
+      for (int i = 0; i < BLOCKS; ++i) {
         const uint32_t p0 = epilogue_pair<EPI, kHasBias>(acc[i][j][0], acc[i][j][1], bv[0], bv[1]);
         const uint32_t p1 = epilogue_pair<EPI, kHasBias>(acc[i][j][2], acc[i][j][3], bv[2], bv[3]);
         *reinterpret_cast<uint2*>(so + (i * 16 + n16) * OLD + cl) = make_uint2(p0, p1);
@@ -737,7 +740,7 @@ __device__ __forceinline__ void store_tile16(floatx4 (&acc)[TM / 16][TN / 16], u
   };
   if (has_bias) stage(std::true_type{});
   else stage(std::false_type{});
-  store_staged_tile<EPI, TM, TN>(so, lane, C, b, R, live, N, wrow0, wcol0);
+  store_staged_tile<EPI, TM, TN, WAVES>(so, lane, C, b, R, live, N, wrow0, wcol0);
 }
 
 template <int EPI>
@@ -854,12 +857,12 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_mixed_kernel(
   static_assert(FN % kRing == 0, "fragment ring");
   constexpr int kBarrierUnit = FN - kLook;      // first unit that reads from the next k tile
   bf16x8 fa[2][FM], fb[kRing];
-  const int a_row_off = (wm * TM + n16) * 64;
+  const int a_row_off = (wm * 16 + n16) * 64;
   const int b_row_off = kBBase + (wn * TN + n16) * 128;
   const int swz_a = (n16 >> 1) & 3, swz_b = (n16 >> 1) & 7;
   auto read_a = [&](int buf, int kt, int i) {
     fa[buf][i] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(
-        smem + (kt & 1) * kASlot + a_row_off + i * 16 * 64 + ((g4 ^ swz_a) * 16)));
+        smem + (kt & 1) * kASlot + a_row_off + i * 32 * 64 + ((g4 ^ swz_a) * 16)));
   };
   auto read_b = [&](int buf, int kt, int j) {
     fb[buf] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(
@@ -883,10 +886,11 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_mixed_kernel(
     }
   }
 
-  // Units lo .. hi - 1 of iteration kt (fragment set par = kt & 1 as a constant); `next`: the
+  // Units lo .. hi - 1 of iteration kt over the first `nb` row blocks (fragment set par = kt & 1 as a constant); `next`: the
   // k tile kt + 1 exists, so the units from kBarrierUnit on read its first fragments; `dma`
   // requests go out under these units, spread evenly.
-  auto units = [&](auto lo_c, auto hi_c, auto par_c, int kt, auto next_c, auto dma_c) __attribute__((always_inline)) {
+  auto units = [&](auto nb_c, auto lo_c, auto hi_c, auto par_c, int kt, auto next_c, auto dma_c) __attribute__((always_inline)) {
+    constexpr int nb = decltype(nb_c)::value;
     constexpr int lo = decltype(lo_c)::value, hi = decltype(hi_c)::value, par = decltype(par_c)::value;
     constexpr bool next = decltype(next_c)::value;
     constexpr int dma = decltype(dma_c)::value;
@@ -894,26 +898,25 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_mixed_kernel(
       constexpr int j = lo + decltype(c)::value;
       constexpr int jl = j + kLook;
       constexpr bool rb = jl < FN || next;
-      constexpr bool ra = next && j >= FN - 2;
+      constexpr int i0 = 2 * (j - (FN - 2));           // A fragments of the next k tile: i0 and i0 + 1
+      constexpr bool ra = next && j >= FN - 2 && i0 < nb, ra1 = ra && i0 + 1 < nb;
       if constexpr (jl < FN) read_b(jl % kRing, kt, jl);
       else if constexpr (next) read_b(jl % kRing, kt + 1, jl - FN);
-      if constexpr (ra) {
-        read_a(par ^ 1, kt + 1, 2 * (j - (FN - 2)));
-        read_a(par ^ 1, kt + 1, 2 * (j - (FN - 2)) + 1);
-      }
+      if constexpr (ra) read_a(par ^ 1, kt + 1, i0);
+      if constexpr (ra1) read_a(par ^ 1, kt + 1, i0 + 1);
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
+      for (int i = 0; i < nb; ++i)
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j % kRing], fa[par][i], acc[i][j], 0, 0, 0);
       constexpr int u = j - lo, n = hi - lo;
       constexpr int dma_here = (u + 1) * dma / n - u * dma / n;
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       if constexpr (rb) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      if constexpr (nb > 1) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       if constexpr (ra) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      if constexpr (ra) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      if constexpr (nb > 2) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      if constexpr (ra1) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       if constexpr (dma_here > 0) __builtin_amdgcn_sched_group_barrier(0x020, dma_here, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      if constexpr (nb > 3) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
     });
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -938,18 +941,18 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_mixed_kernel(
   // Pair J = iterations 2 J and 2 J + 1 (B slot J mod 2).  B1: pair J + 1 exists; A2 / A3: k
   // tiles 2 J + 2 / 2 J + 3 exist; B2: pair J + 2 exists.  Requests and barriers as described
   // above the kernel; a barrier stands in front of the first unit that reads from the next k tile.
-  auto pair = [&](int J, auto b1_c, auto a2_c, auto a3_c, auto b2_c) __attribute__((always_inline)) {
+  auto pair = [&](auto nb, int J, auto b1_c, auto a2_c, auto a3_c, auto b2_c) __attribute__((always_inline)) {
     constexpr bool B1 = decltype(b1_c)::value, A2 = decltype(a2_c)::value;
     constexpr bool A3 = decltype(a3_c)::value, B2 = decltype(b2_c)::value;
     const int kt = 2 * J;
     if constexpr (B1) load_b_half((J + 1) & 1, J + 1, Half1{});
-    units(U0{}, UB{}, P0{}, kt, std::true_type{}, std::integral_constant<int, B1 ? 8 - kBFirst : 0>{});
+    units(nb, U0{}, UB{}, P0{}, kt, std::true_type{}, std::integral_constant<int, B1 ? 8 - kBFirst : 0>{});
     wait_vmcnt<B1 ? 8 - kBFirst : 0>();
     wait_lgkmcnt0();
     raw_barrier();
     if constexpr (A2) load_a(0, kt + 2);
-    units(UB{}, UN{}, P0{}, kt, std::true_type{}, std::integral_constant<int, A2 ? 2 : 0>{});
-    units(U0{}, UB{}, P1{}, kt + 1, std::bool_constant<A2>{}, U0{});
+    units(nb, UB{}, UN{}, P0{}, kt, std::true_type{}, std::integral_constant<int, A2 ? 2 : 0>{});
+    units(nb, U0{}, UB{}, P1{}, kt + 1, std::bool_constant<A2>{}, U0{});
     if constexpr (A2) {
       wait_vmcnt<0>();
       wait_lgkmcnt0();
@@ -957,20 +960,31 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_mixed_kernel(
     }
     if constexpr (A3) load_a(1, kt + 3);
     if constexpr (B2) load_b_half(J & 1, J + 2, Half0{});
-    units(UB{}, UN{}, P1{}, kt + 1, std::bool_constant<A2>{},
+    units(nb, UB{}, UN{}, P1{}, kt + 1, std::bool_constant<A2>{},
           std::integral_constant<int, (A3 ? 2 : 0) + (B2 ? kBFirst : 0)>{});
   };
   using T = std::true_type;
   using F = std::false_type;
   const int npairs = nk / 2;
-  for (int J = 0; J < npairs - 2; ++J) pair(J, T{}, T{}, T{}, T{});
-  pair(npairs - 2, T{}, T{}, T{}, F{});
-  pair(npairs - 1, F{}, F{}, F{}, F{});
-  wait_lgkmcnt0();
-  __syncthreads();   // all waves are done with the operand tiles: LDS is reused below
-  mfma_result_fence();
-  store_tile16<EPI, TM, TN>(acc, smem, wave, lane, bias_pk, bias != nullptr, C, b, R, live, N,
-                            row0 + wm * TM, col0 + wn * TN);
+  auto product = [&](auto nb) __attribute__((always_inline)) {
+    for (int J = 0; J < npairs - 2; ++J) pair(nb, J, T{}, T{}, T{}, T{});
+    pair(nb, npairs - 2, T{}, T{}, T{}, F{});
+    pair(nb, npairs - 1, F{}, F{}, F{}, F{});
+    wait_lgkmcnt0();
+    __syncthreads();   // all waves are done with the operand tiles: LDS is reused below
+    mfma_result_fence();
+    store_tile16<EPI, TM, TN, 2, decltype(nb)::value>(acc, smem, wave, lane, bias_pk, bias != nullptr, C, b, R, live,
+                                                      N, row0 + wm * 16, col0 + wn * TN);
+  };
+  // Row blocks of 16 go to the two waves of a column half in turn, so that a batch's last tile costs what its live
+  // rows do, to 32 rows, where it took as long as a full one: experts choice, 32 experts x 800 rows (6.25 tiles of
+  // rows each) 339 -> 332 us a layer, 32 x 3 136 rows (24.5) 954 -> 950, at the power limit, and the bfloat16 model of 512
+  // images 23.26 -> 23.20 ms.
+  const int blocks = __builtin_amdgcn_readfirstlane((live - row0 + 31) / 32);
+  if (blocks >= FM) product(std::integral_constant<int, FM>{});
+  else if (blocks == 3) product(std::integral_constant<int, 3>{});
+  else if (blocks == 2) product(std::integral_constant<int, 2>{});
+  else product(std::integral_constant<int, 1>{});
 #endif
 }
 
