@@ -400,3 +400,18 @@ def test_only_dispatchers_without_packed_rows_ask_for_float32_products(packed, h
   items = [torch.zeros((2, 3), dtype=torch.int32)] * inputs       # (integers pass the dispatcher uncast)
   layer.apply({}, moe.Bfloat16Dispatcher(Inner()), *items)
   assert asked == [not packed]
+
+
+def test_negative_indices_are_refused_in_every_thread(monkeypatch):
+  """Two threads dispatch by the same new maps before the counters of invalid indices arrive: one waits for them
+  first and raises, and so does the other."""
+  monkeypatch.setattr(moe.K, "indices_to_slots", lambda *args: (None, None, torch.tensor([0, 1])))
+  event = type("Event", (), {"record": lambda self: None, "synchronize": lambda self: None})
+  monkeypatch.setattr(torch.cuda, "Event", event)
+  dispatcher = moe.ExpertIndicesDispatcher(torch.zeros((1, 2, 1, 2), dtype=torch.int32), torch.ones((1, 2, 1)), 2, 2)
+  dispatcher._maps(settle=False)
+  for _ in range(2):
+    with pytest.raises(ValueError, match="negative indices"):
+      dispatcher._settle()
+  with pytest.raises(ValueError, match="negative indices"):
+    dispatcher._maps()

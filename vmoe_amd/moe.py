@@ -185,7 +185,7 @@ class ExpertIndicesDispatcher(BaseDispatcher):
     event.synchronize()
     dups, invalid = counters.tolist()
     if invalid:
-      self._slots = self._unread = None
+      self._slots = None        # (and not _unread: another thread's dispatch of these maps has yet to be refused)
       raise ValueError("ExpertIndicesDispatcher: negative indices are not supported.")
     if dups:
       token_slot, slot_token = self._slots
