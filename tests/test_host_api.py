@@ -415,3 +415,21 @@ def test_negative_indices_are_refused_in_every_thread(monkeypatch):
       dispatcher._settle()
   with pytest.raises(ValueError, match="negative indices"):
     dispatcher._maps()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("same", [True, False])
+def test_library_projections_get_weights_in_their_own_layout(monkeypatch, dtype, same):
+  """Where the library multiplies, it is handed contiguous (out, in) weights in every type, not transposed views;
+  the result is the projections' in the reference's order."""
+  linear, seen = torch.nn.functional.linear, []
+  monkeypatch.setattr(torch.nn.functional, "linear", lambda x, w, b: seen.append(w) or linear(x, w, b))
+  attn = vit_moe.MultiHeadDotProductAttention(num_heads=2, dtype=dtype)
+  x = torch.randn(2, 5, 16, generator=torch.Generator().manual_seed(0))
+  kv = x if same else x[:, :3].contiguous()
+  p = attn.init(0, x, kv)["params"]
+  out = attn.apply({"params": p}, x, kv)
+  assert len(seen) == (2 if same else 3) and all(w.is_contiguous() for w in seen)
+  q, k, v = (torch.einsum("bsd,dhe->bhse", t, p[n]["kernel"]) for n, t in (("query", x), ("key", kv), ("value", kv)))
+  want = torch.einsum("bhse,hed->bsd", torch.nn.functional.scaled_dot_product_attention(q, k, v), p["out"]["kernel"])
+  assert torch.allclose(out.float(), want, rtol=0, atol=1e-5 if dtype == torch.float32 else 5e-2)
