@@ -433,3 +433,40 @@ def test_library_projections_get_weights_in_their_own_layout(monkeypatch, dtype,
   q, k, v = (torch.einsum("bsd,dhe->bhse", t, p[n]["kernel"]) for n, t in (("query", x), ("key", kv), ("value", kv)))
   want = torch.einsum("bhse,hed->bsd", torch.nn.functional.scaled_dot_product_attention(q, k, v), p["out"]["kernel"])
   assert torch.allclose(out.float(), want, rtol=0, atol=1e-5 if dtype == torch.float32 else 5e-2)
+
+
+@pytest.mark.parametrize("x,w,b", [
+    ((6, 4), (4, 8), (16,)),            # a bias longer than the row
+    ((6, 4), (4, 8), (1,)),
+    ((6, 4), (4, 8), (6, 8)),
+    ((6, 4), (8, 8), (8,)),
+    ((6, 0), (0, 8), (8,)),
+])
+@pytest.mark.parametrize("timed", [False, True])
+def test_dense_refuses_what_its_sizes_do_not_cover(monkeypatch, x, w, b, timed):
+  """Widths that differ, an empty one, and biases of other sizes than a row."""
+  if timed:
+    monkeypatch.setattr(_hip, "_timing_sink", {})
+  else:
+    monkeypatch.setattr(_hip, "raw_stream", lambda: 0)
+  with pytest.raises(ValueError):
+    kernels.dense(torch.zeros(x), torch.zeros(w), torch.zeros(b))
+
+
+@pytest.mark.parametrize("bias", [(8,), (1, 8), (6, 8), (6, 1), (1,), ()])
+def test_dense_layers_spread_biases_as_the_library_does(monkeypatch, bias):
+  """A bias that is not one row of the output takes the library's product, which spreads it; one that is goes to
+  the package's."""
+  asked = []
+  monkeypatch.setattr(kernels, "dense_pays", lambda *args: True)
+  monkeypatch.setattr(kernels, "dense_takes", lambda *args: True)
+  monkeypatch.setattr(module, "is_plain", lambda *args: True)
+  monkeypatch.setattr(kernels, "dense", lambda x, w, b: asked.append(b.shape) or x @ w + b)
+  x, w, b = torch.randn(6, 4), torch.randn(4, 8), torch.randn(bias)
+  assert torch.allclose(vit_moe._affine(x, w, b), torch.addmm(b, x, w))
+  assert asked == ([(8,)] if bias == (8,) else [])
+  if bias in [(8,), (1,), ()]:
+    assert torch.allclose(vit_moe.MultiHeadDotProductAttention._project(x, w, b), x @ w + b)
+    assert len(asked) == (2 if bias == (8,) else 0)
+  with pytest.raises(RuntimeError):
+    vit_moe._affine(torch.randn(6, 8), w, b)

@@ -483,9 +483,11 @@ Tensor dense(int64_t stream, const Tensor& x_, const Tensor& w_, const OptTensor
   const OptTensor b = b_.has_value() ? OptTensor(b_->contiguous()) : b_;
   const bool f32 = x.scalar_type() == at::kFloat;
   const int64_t D = x.size(-1), M = w.size(f32 ? 1 : 0);
-  if (w.size(f32 ? 0 : 1) != D)
+  if (w.size(f32 ? 0 : 1) != D || D == 0)
     throw py::value_error("w has shape " + shape_of(w) + ", x " + shape_of(x));
-  need_values(b, M, "bias");
+  if (b.has_value() && b->numel() != M)
+    throw py::value_error("bias has shape " + shape_of(*b) + ", expected (" + std::to_string(M) + ",)");
+  if (x.numel() / D > INT32_MAX) throw py::value_error("x has shape " + shape_of(x) + ": too many rows");
   auto sizes = x.sizes().vec();
   sizes.back() = M;
   Tensor out = empty(sizes, x.scalar_type(), x);

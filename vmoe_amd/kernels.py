@@ -683,7 +683,13 @@ def dense(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor]) -> torch.
   b = b.contiguous() if b is not None else None
   D, f32 = x.shape[-1], x.dtype == torch.float32
   M = w.shape[1 if f32 else 0]
+  if w.dtype != x.dtype or (b is not None and b.dtype != x.dtype):
+    raise TypeError(f"x is {x.dtype}, w {w.dtype}, bias {None if b is None else b.dtype}")
+  if D == 0 or w.shape[0 if f32 else 1] != D or (b is not None and b.numel() != M):
+    raise ValueError(f"x has shape {tuple(x.shape)}, w {tuple(w.shape)}, bias {None if b is None else tuple(b.shape)}")
   out = torch.empty((*x.shape[:-1], M), dtype=x.dtype, device=x.device)
+  if out.numel() == 0:
+    return out
   p = H.ExpertMlpParams(x=H.ptr(x), b0=H.ptr(b) if b is not None else None, out=H.ptr(out), E=1,
                         R=x.numel() // D, D=D, M=M, dtype=H.dtype_code(x.dtype))
   setattr(p, "w0" if f32 else "w0t", H.ptr(w))

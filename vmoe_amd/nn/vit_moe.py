@@ -227,12 +227,18 @@ def _add_layer_norm(residual: Array, branch: Optional[Array], p: Mapping[str, Ar
 
 def _affine(x: Array, w: Array, b: Array) -> Array:
   """x (..., D) . w (D, M) + b in float32: the package's own product where it is the faster one."""
-  D, M = w.shape
-  if (x.dtype == w.dtype == b.dtype and w.is_contiguous() and b.is_contiguous()
-      and K.dense_pays(x.numel() // D, D, M, x.dtype) and module.is_plain(x, w, b)
+  (D, M), rows = w.shape, x.shape[:-1].numel()
+  if (_fits_dense(x, D, M, b) and x.dtype == w.dtype == b.dtype and w.is_contiguous() and b.is_contiguous()
+      and K.dense_pays(rows, D, M, x.dtype) and module.is_plain(x, w, b)
       and K.dense_takes(x, w)):
     return K.dense(x, w, b)
-  return torch.addmm(b, x.reshape(-1, D), w).view(*x.shape[:-1], M)
+  return torch.addmm(b, x.reshape(rows, x.shape[-1]), w).view(*x.shape[:-1], M)
+
+
+def _fits_dense(x: Array, D: int, M: int, b: Array) -> bool:
+  """Whether x is (..., D) and b (M,), what a weight of D x M goes with: the library refuses other widths and
+  spreads other biases, over rows or columns, and K.dense does neither."""
+  return x.shape[-1] == D and b.shape == (M,)
 
 
 class IdentityLayer(module.Module):
@@ -315,10 +321,12 @@ class MultiHeadDotProductAttention(module.Module):
   @staticmethod
   def _project(x: Array, w: Array, b: Array) -> Array:
     """x . w + b for a weight of _proj_weights: the package's own product where it is the faster one."""
-    D, M = w.shape if w.dtype == torch.float32 else reversed(w.shape)
-    if K.dense_pays(x.numel() // D, D, M, w.dtype) and module.is_plain(x, w, b) and K.dense_takes(x, w):
+    f32 = w.dtype == torch.float32
+    D, M = w.shape if f32 else reversed(w.shape)
+    if (_fits_dense(x, D, M, b) and K.dense_pays(x.shape[:-1].numel(), D, M, w.dtype)
+        and module.is_plain(x, w, b) and K.dense_takes(x, w)):
       return K.dense(x, w, b)
-    return torch.nn.functional.linear(x, w.t() if w.dtype == torch.float32 else w, b)
+    return torch.nn.functional.linear(x, w.t() if f32 else w, b)
 
   def apply(self, variables, inputs_q: Array, inputs_kv: Optional[Array] = None) -> Array:
     p = variables["params"]
