@@ -379,6 +379,17 @@ def test_small_tiles_are_not_taken_where_they_would_run_on_few_dies(monkeypatch,
   assert (chosen < _ragged_mlp_bytes(E, R, D, M)) == small
 
 
+@pytest.mark.parametrize("E,R,D,M", [(51, 729, 640, 2560), (20, 1571, 640, 2560), (28, 381, 576, 2304)])
+def test_medium_tiles_are_chosen_by_the_rounds_that_a_plan_makes_of_them(monkeypatch, E, R, D, M):
+  """A launch plan deals whole row tiles to the dies: shapes whose medium tiles would fill the chip's rounds one by one, and
+  do not as rows of column tiles, keep the large ones."""
+  monkeypatch.delenv("VMOE_SECOND_PRODUCT", raising=False)
+  monkeypatch.delenv("VMOE_ROW_TILES", raising=False)
+  chosen = _ragged_mlp_bytes(E, R, D, M)
+  monkeypatch.setenv("VMOE_ROW_TILES", "off")
+  assert chosen == _ragged_mlp_bytes(E, R, D, M)
+
+
 @pytest.mark.parametrize("packed", [True, False])
 @pytest.mark.parametrize("has_aux,inputs", [(True, 1), (False, 2)])
 def test_only_dispatchers_without_packed_rows_ask_for_float32_products(packed, has_aux, inputs):

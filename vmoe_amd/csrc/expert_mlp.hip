@@ -434,14 +434,14 @@ MlpPlans mlp_plans(int E, int R, int D, int M, bool ragged, long long items) {
     return forced < kNumRowsTiles || stream_tile_ok(forced - kNumRowsTiles, E, R, Kd, ragged);
   };
   if (any_tile && rows_gemm_ok(R, M, D, items)) {
-    const double us = m.up.fast ? launch_us(D % 64 == 0 ? kFirstProductTile : kFirstProductK32Tile, E, R, M, D, true, false, ragged) : 1e30;
+    const double us = m.up.fast ? launch_us(D % 64 == 0 ? kFirstProductTile : kFirstProductK32Tile, E, R, M, D, true, kDealTiles, ragged) : 1e30;
     m.up_rows = best_tile(E, R, M, D, items, ragged, true, us);
     if (forced_ok(M, D, items)) m.up_rows = forced;
   }
   if (any_tile && rows_gemm_ok(R, D, M, 0)) {
     double us = 1e30;
     if (m.down_kernel == kDownEightWaves || m.down_kernel == kDownNarrow)
-      us = launch_us(m.down_kernel == kDownNarrow ? kNarrowTile : kEightWavesTile, E, R, D, M, false, false, ragged);
+      us = launch_us(m.down_kernel == kDownNarrow ? kNarrowTile : kEightWavesTile, E, R, D, M, false, kDealTiles, ragged);
     else if (t_best < 1e29)
       us = 5 + (ragged ? 0.7 : 1) * t_best;
     else if (square.fast)

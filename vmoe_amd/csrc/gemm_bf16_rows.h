@@ -70,12 +70,18 @@ constexpr RowsTile kFirstProductK32Tile = {128, 256, 2, 1.28, 1.45, 2.25, 0.8, 4
 constexpr RowsTile kEightWavesTile = {256, 256, 1, 8.00, 1.23, 0, 0, 5.6, 1.87};
 constexpr RowsTile kNarrowTile = {256, 192, 1, 3.69, 0.87, 0, 0, 4.2, 1.34};
 
+// How a launch's tiles are dealt to the dies, whose rounds count: one by one (kDealTiles), all row tiles of a (batch,
+// column tile) pair to one die (kDealPairs: a launch of two pairs runs on two dies), or all column tiles of a row tile
+// (kDealRows: launch plans.  35 row tiles of seven column tiles each are 245 tiles for 256 CUs, and 35 for the 32 of a
+// die: 5 experts x 800 rows x 832 x 3 328, second product, on 128 x 128: 60.6 us, on 64 x 128 35.9).
+enum TileDeal { kDealTiles, kDealPairs, kDealRows };
+
 // Time in microseconds of a product on tiles of this kind.
-// whole_pairs: all row tiles of a (batch, column tile) pair run on one die, whose rounds then count (a launch of
-// two pairs runs on two dies); else the tiles fall evenly on the dies.
-inline double product_us(const RowsTile& t, int batch, int R, int N, int Kd, bool gelu, bool whole_pairs) {
-  const double row_tiles = (R + t.bm - 1) / t.bm, pairs = (double)batch * ((N + t.bn - 1) / t.bn);
-  const double on_die = whole_pairs ? std::ceil(pairs / kNumXcd) * row_tiles : std::ceil(pairs * row_tiles / kNumXcd);
+inline double product_us(const RowsTile& t, int batch, int R, int N, int Kd, bool gelu, TileDeal deal) {
+  const double row_tiles = (R + t.bm - 1) / t.bm, tiles_n = (N + t.bn - 1) / t.bn;
+  const double on_die = deal == kDealPairs  ? std::ceil(batch * tiles_n / kNumXcd) * row_tiles
+                        : deal == kDealRows ? std::ceil(batch * row_tiles / kNumXcd) * tiles_n
+                                            : std::ceil(batch * tiles_n * row_tiles / kNumXcd);
   const double full = (double)kCusPerXcd * t.per_cu;
   const double fix = t.fix + (gelu ? t.gelu : 0);
   const int nk = (Kd + 63) / 64;
@@ -93,11 +99,11 @@ inline double product_us(const RowsTile& t, int batch, int R, int N, int Kd, boo
 // The same for a launch whose live rows are counted on the device: the mean over full, 70 % full and 40 % full
 // experts.  On 80 random ragged layers, 23 % to all of their rows live, the choice by this mean takes 6 514 us for the
 // 160 products, by the time of full experts 6 566 and 39 % too long at worst instead of 18 %, on the best tile of each 6 113.
-inline double launch_us(const RowsTile& t, int batch, int R, int N, int Kd, bool gelu, bool whole_pairs, bool ragged) {
-  const double us = product_us(t, batch, R, N, Kd, gelu, whole_pairs);
+inline double launch_us(const RowsTile& t, int batch, int R, int N, int Kd, bool gelu, TileDeal deal, bool ragged) {
+  const double us = product_us(t, batch, R, N, Kd, gelu, deal);
   if (!ragged) return us;
-  return (us + product_us(t, batch, (int)std::ceil(0.7 * R), N, Kd, gelu, whole_pairs) +
-          product_us(t, batch, (int)std::ceil(0.4 * R), N, Kd, gelu, whole_pairs)) / 3;
+  return (us + product_us(t, batch, (int)std::ceil(0.7 * R), N, Kd, gelu, deal) +
+          product_us(t, batch, (int)std::ceil(0.4 * R), N, Kd, gelu, deal)) / 3;
 }
 
 // The tiles of gemm_bf16_stream_kernel, and what the choice
@@ -187,7 +193,8 @@ inline int best_tile(int batch, int R, int N, int Kd, long long items, bool ragg
   auto take_tile = [&](int i, const RowsTile& t) {
     const bool mid = is_mid_tile(i);
     if (!mid || mid_ok)
-      take(i, launch_us(t, batch, R, N, Kd, gelu, !mid || (ragged && !mid_tile_planned(batch, R, t.bm)), ragged));
+      take(i, launch_us(t, batch, R, N, Kd, gelu,
+                        !mid || (ragged && !mid_tile_planned(batch, R, t.bm)) ? kDealPairs : ragged ? kDealRows : kDealTiles, ragged));
   };
   for (int i = 0; i < kNumRowsTiles; ++i) take_tile(i, kRowsTiles[i]);
   for (int i = 0; i < kNumMoreTiles; ++i) take_tile(kFirstMoreTile + i, kMoreTiles[i]);
