@@ -43,6 +43,9 @@ enum { VMOE_GELU_TANH = 0, VMOE_GELU_ERF = 1 };
 enum { VMOE_MLP_F32_PRODUCTS = 256 };
 /* Added to VMOE_GELU_* of a bfloat16 expert MLP: b0 and b1 are float32 and rounded to bfloat16 in the call. */
 enum { VMOE_MLP_F32_BIASES = 512 };
+/* Every expert's rows are live (rows_per_expert all R, as experts choice makes them): a choice between
+ * kernels then goes by full experts.  Results do not depend on it. */
+enum { VMOE_MLP_FULL_ROWS = 1024 };
 
 enum {
   VMOE_OK = 0,
@@ -355,7 +358,8 @@ typedef struct {
   int32_t gelu;     /* VMOE_GELU_TANH (flax default) or VMOE_GELU_ERF, for float32 also
                        + VMOE_MLP_F32_PRODUCTS, for bf16 + VMOE_MLP_F32_BIASES: the rounded
                        biases then lie at the end of the workspace, written by this call or by
-                       vmoe_compact_rows_planned (vmoe_expert_mlp_planned reads them there) */
+                       vmoe_compact_rows_planned (vmoe_expert_mlp_planned reads them there);
+                       + VMOE_MLP_FULL_ROWS */
   const int32_t* rows_per_expert; /* optional (E,): only the first rows_per_expert[e] rows of
                                      expert e hold data; the other rows of x are not read
                                      for results and their rows of out are left untouched */

@@ -1404,6 +1404,25 @@ def test_expert_mlp_last_tiles_of_the_large_kernels(K, monkeypatch, rows, second
       assert bool((got[e, n:] == 7.0).all())
 
 
+@pytest.mark.parametrize("E,R,D,M", [(5, 800, 832, 3328), (3, 1500, 512, 2048), (12, 896, 448, 1088), (21, 140, 704, 2816),
+                                     (5, 8, 64, 136), (4, 2576, 96, 2048)])
+def test_expert_mlp_of_full_experts(K, E, R, D, M):
+  """A call that says that every row is live may take other tiles (these shapes do), and gives the same bits; so does
+  one that says it of rows that are not."""
+  rng = np.random.default_rng(R)
+  mk = lambda scale, *s: to_dev(O.cast(rng.standard_normal(s).astype(np.float32) * scale, O.BF16), O.BF16)
+  T = R + 5
+  items, w0, b0 = mk(1, T, D), mk(D ** -0.5, E, D, M), mk(0.1, E, M)
+  w1, b1 = mk(M ** -0.5, E, M, D), mk(0.1, E, D)
+  x_rows = torch.from_numpy(rng.integers(0, T, (E, R)).astype(np.int32)).to(dev())
+  for counts in ([R] * E, rng.integers(0, R + 1, E)):
+    live = torch.as_tensor(np.asarray(counts, np.int32), device=dev())
+    got, want = (torch.full((E, R, D), 7.0, dtype=torch.bfloat16, device=dev()) for _ in range(2))
+    for out, full in ((got, True), (want, False)):
+      K.expert_mlp(items, w0, b0, w1, b1, out=out, rows_per_expert=live, x_rows=x_rows, full_rows=full)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 @pytest.mark.parametrize("tile", range(8, 13))
 @pytest.mark.parametrize("E,R,D,M", [
     (130, 64, 640, 776),     # several tiles per workgroup, column tiles and k that end inside

@@ -481,3 +481,35 @@ def test_dense_layers_spread_biases_as_the_library_does(monkeypatch, bias):
     assert len(asked) == (2 if bias == (8,) else 0)
   with pytest.raises(RuntimeError):
     vit_moe._affine(torch.randn(6, 8), w, b)
+
+
+@pytest.mark.parametrize("full", [True, False])
+@pytest.mark.parametrize("gathers,takes", [(True, True), (False, True), (True, False)])
+def test_experts_hear_that_every_packed_row_is_live(full, gathers, takes):
+  """What experts choice knows about its rows reaches experts that ask for it, and only those."""
+  class Dispatcher(moe.ExpertIndicesDispatcher):
+    dispatch_packed = lambda self, data: (data, self.packed_rows()[1])
+    combine_packed = lambda self, data: data
+
+  class Experts:
+    supports_packed_rows = True
+    can_gather = lambda self, items: gathers
+
+    def apply_experts_gathered(self, variables, items, row_token, rows_per_expert, **hints):
+      asked.append(hints)
+      return items
+
+    def apply_experts(self, variables, dispatched, rows_per_expert=None, **hints):
+      asked.append(hints)
+      return dispatched
+
+    apply_experts.takes_full_rows = apply_experts_gathered.takes_full_rows = takes
+
+  asked = []
+  maps = (torch.zeros((2, 3, 1), dtype=torch.int32), torch.full((2,), 4), torch.zeros((2, 4), dtype=torch.int32))
+  dispatcher = Dispatcher(torch.zeros((2, 3, 1, 2), dtype=torch.int32), torch.ones((2, 3, 1)), 2, 2)
+  dispatcher.set_packed_maps(maps, full_rows=full)
+  wrapped = moe._SparseEinsumDispatcher(dispatcher, torch.float32)
+  for d in (dispatcher, wrapped):
+    moe.sparse_moe_spmd(Experts)().apply({}, d, torch.zeros((2, 3, 8)))
+  assert asked == [{"full_rows": True} if full and takes else {}] * 2

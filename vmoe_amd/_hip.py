@@ -21,7 +21,7 @@ _host = None
 
 F32, BF16 = 0, 1
 GELU_TANH, GELU_ERF = 0, 1
-MLP_F32_PRODUCTS, MLP_F32_BIASES = 256, 512
+MLP_F32_PRODUCTS, MLP_F32_BIASES, MLP_FULL_ROWS = 256, 512, 1024
 EINSUM_F32_AS_BF16 = 2
 MLP_STATUS_ABANDONED_WAITS, MLP_STATUS_PLAN_MISMATCHES, MLP_STATUS_WORDS = 0, 1, 2
 W_F32, W_BF16, W_BOOL = 0, 1, 2

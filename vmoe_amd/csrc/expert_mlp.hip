@@ -371,8 +371,9 @@ struct MlpPlans {
   size_t streamk_bytes = 0;              // exchange memory of kDownShared
 };
 
-// (`items`: rows of the matrix of items that the first product gathers from, 0 if it does not.)
-MlpPlans mlp_plans(int E, int R, int D, int M, bool ragged, long long items) {
+// (`items`: rows of the matrix of items that the first product gathers from, 0 if it does not.  `full`: all rows of a
+// ragged call are live.)
+MlpPlans mlp_plans(int E, int R, int D, int M, bool ragged, bool full, long long items) {
   MlpPlans m;
   m.up = gemm_geometry<CfgUp>(E, R, M, D);
   // Ragged launches are planned whenever the geometry allows: with whole experts per
@@ -428,26 +429,30 @@ MlpPlans mlp_plans(int E, int R, int D, int M, bool ragged, long long items) {
   const char* const row_tiles = getenv("VMOE_ROW_TILES");
   const bool any_tile = row_tiles == nullptr || strcmp(row_tiles, "off") != 0;
   const int forced = any_tile && row_tiles != nullptr ? atoi(row_tiles) : -1;
+  const bool partly = ragged && !full;       // how many rows are live is known on the device only
+  // (the large tiles of 80 random layers of partly filled experts, chosen as if dealt one by one and by whole row
+  // tiles: 8 692 and 8 745 us for the 160 products; of 80 of full ones: 5 349 and 5 323)
+  const TileDeal large_deal = ragged && full ? kDealRows : kDealTiles;
   const auto forced_ok = [&](int N, int Kd, long long n) {
     if (forced < 0) return false;
     if (is_mid_tile(forced)) return mid_gemm_ok(E, R, N, Kd, n);
     return forced < kNumRowsTiles || stream_tile_ok(forced - kNumRowsTiles, E, R, Kd, ragged);
   };
   if (any_tile && rows_gemm_ok(R, M, D, items)) {
-    const double us = m.up.fast ? launch_us(D % 64 == 0 ? kFirstProductTile : kFirstProductK32Tile, E, R, M, D, true, kDealTiles, ragged) : 1e30;
-    m.up_rows = best_tile(E, R, M, D, items, ragged, true, us);
+    const double us = m.up.fast ? launch_us(D % 64 == 0 ? kFirstProductTile : kFirstProductK32Tile, E, R, M, D, true, large_deal, partly) : 1e30;
+    m.up_rows = best_tile(E, R, M, D, items, ragged, partly, true, us);
     if (forced_ok(M, D, items)) m.up_rows = forced;
   }
   if (any_tile && rows_gemm_ok(R, D, M, 0)) {
     double us = 1e30;
     if (m.down_kernel == kDownEightWaves || m.down_kernel == kDownNarrow)
-      us = launch_us(m.down_kernel == kDownNarrow ? kNarrowTile : kEightWavesTile, E, R, D, M, false, kDealTiles, ragged);
+      us = launch_us(m.down_kernel == kDownNarrow ? kNarrowTile : kEightWavesTile, E, R, D, M, false, large_deal, partly);
     else if (t_best < 1e29)
-      us = 5 + (ragged ? 0.7 : 1) * t_best;
+      us = 5 + (partly ? 0.7 : 1) * t_best;
     else if (square.fast)
-      us = 5 + (ragged ? 0.7 : 1) * unit * (half ? 0.5 * 1.05 * std::ceil((double)E * ((R + 127) / 128) * ((D + 255) / 256) / kNumCu)
+      us = 5 + (partly ? 0.7 : 1) * unit * (half ? 0.5 * 1.05 * std::ceil((double)E * ((R + 127) / 128) * ((D + 255) / 256) / kNumCu)
                             : std::ceil((double)square.tiles / kNumCu));
-    m.down_rows = best_tile(E, R, D, M, 0, ragged, false, us);
+    m.down_rows = best_tile(E, R, D, M, 0, ragged, partly, false, us);
     if (forced_ok(D, M, 0)) m.down_rows = forced;
   }
   // (VMOE_SECOND_PRODUCT=shared|eight|narrow|wide in the environment overrides the choice
@@ -496,7 +501,7 @@ MlpPlans mlp_plans(int E, int R, int D, int M, bool ragged, long long items) {
 using namespace vmoe;
 
 static int gelu_of(const VmoeExpertMlpParams* p) {
-  return p->gelu & ~(VMOE_MLP_F32_PRODUCTS | VMOE_MLP_F32_BIASES);
+  return p->gelu & ~(VMOE_MLP_F32_PRODUCTS | VMOE_MLP_F32_BIASES | VMOE_MLP_FULL_ROWS);
 }
 static bool has_f32_biases(const VmoeExpertMlpParams* p) { return (p->gelu & VMOE_MLP_F32_BIASES) != 0; }
 // The rounded biases' part of the workspace, its last.
@@ -542,16 +547,17 @@ static MlpPlans plans_of(const VmoeExpertMlpParams* p) {
   if (p->dtype != VMOE_BF16) return MlpPlans{};
   struct Key {
     int E, R, D, M;
-    bool ragged;
+    bool ragged, full;
     long long items;
   };
-  const Key key = {p->E, p->R, p->D, p->M, p->rows_per_expert != nullptr, p->x_rows != nullptr ? p->num_items : 0};
-  auto plans = [&] { return mlp_plans(key.E, key.R, key.D, key.M, key.ragged, key.items); };
+  const Key key = {p->E, p->R, p->D, p->M, p->rows_per_expert != nullptr, (p->gelu & VMOE_MLP_FULL_ROWS) != 0,
+                   p->x_rows != nullptr ? p->num_items : 0};
+  auto plans = [&] { return mlp_plans(key.E, key.R, key.D, key.M, key.ragged, key.full, key.items); };
   if (getenv("VMOE_ROW_TILES") != nullptr || getenv("VMOE_SECOND_PRODUCT") != nullptr) return plans();
   thread_local Key last_key = {};
   thread_local MlpPlans last;
   if (last_key.E != key.E || last_key.R != key.R || last_key.D != key.D || last_key.M != key.M ||
-      last_key.ragged != key.ragged || last_key.items != key.items) {
+      last_key.ragged != key.ragged || last_key.full != key.full || last_key.items != key.items) {
     last = plans();
     last_key = key;
   }
@@ -784,7 +790,7 @@ extern "C" int vmoe_dense(const VmoeExpertMlpParams* p, vmoe_stream_t stream_) {
                                            nullptr, 0);
   if (!aligned16(p->w0t)) return VMOE_E_ALIGN;
   if (!rows_gemm_ok(p->R, p->M, p->D, 0)) return VMOE_E_UNSUPPORTED;
-  const int tile = best_tile(p->E, p->R, p->M, p->D, 0, false, false, 1e30, false);
+  const int tile = best_tile(p->E, p->R, p->M, p->D, 0, false, false, false, 1e30, false);
   return launch_gemm_bf16_rows<kEpiBiasOnce>(tile, (const bf16_t*)p->x, (const bf16_t*)p->w0t, (const bf16_t*)p->b0,
                                              (bf16_t*)p->out, p->E, p->R, p->M, p->D, stream, nullptr, nullptr, nullptr, 0,
                                              PlanRef{nullptr, 0, 0}, nullptr, 0, nullptr);

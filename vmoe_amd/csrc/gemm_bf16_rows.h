@@ -96,12 +96,12 @@ inline double product_us(const RowsTile& t, int batch, int R, int N, int Kd, boo
   return 2 + std::sqrt(std::sqrt(b2 * b2 + m2 * m2 + f2 * f2));
 }
 
-// The same for a launch whose live rows are counted on the device: the mean over full, 70 % full and 40 % full
+// The same for a launch whose live rows (partly: some of all) are counted on the device: the mean over full, 70 % full and 40 % full
 // experts.  On 80 random ragged layers, 23 % to all of their rows live, the choice by this mean takes 6 514 us for the
 // 160 products, by the time of full experts 6 566 and 39 % too long at worst instead of 18 %, on the best tile of each 6 113.
-inline double launch_us(const RowsTile& t, int batch, int R, int N, int Kd, bool gelu, TileDeal deal, bool ragged) {
+inline double launch_us(const RowsTile& t, int batch, int R, int N, int Kd, bool gelu, TileDeal deal, bool partly) {
   const double us = product_us(t, batch, R, N, Kd, gelu, deal);
-  if (!ragged) return us;
+  if (!partly) return us;
   return (us + product_us(t, batch, (int)std::ceil(0.7 * R), N, Kd, gelu, deal) +
           product_us(t, batch, (int)std::ceil(0.4 * R), N, Kd, gelu, deal)) / 3;
 }
@@ -182,8 +182,9 @@ inline bool rows_gemm_ok(int R, int N, int Kd, long long items) {
 }
 
 // The tile that should run the product in less than `us` microseconds, the time of the large tiles, or -1.
-// (walkers: whether kStreamTiles are among them)
-inline int best_tile(int batch, int R, int N, int Kd, long long items, bool ragged, bool gelu, double us,
+// (ragged: the rows' counts stand on the device; partly: and may be fewer than all; walkers: whether kStreamTiles are
+// among the tiles)
+inline int best_tile(int batch, int R, int N, int Kd, long long items, bool ragged, bool partly, bool gelu, double us,
                      bool walkers = true) {
   int best = -1;
   auto take = [&](int i, double t) {
@@ -194,7 +195,7 @@ inline int best_tile(int batch, int R, int N, int Kd, long long items, bool ragg
     const bool mid = is_mid_tile(i);
     if (!mid || mid_ok)
       take(i, launch_us(t, batch, R, N, Kd, gelu,
-                        !mid || (ragged && !mid_tile_planned(batch, R, t.bm)) ? kDealPairs : ragged ? kDealRows : kDealTiles, ragged));
+                        !mid || (ragged && !mid_tile_planned(batch, R, t.bm)) ? kDealPairs : ragged ? kDealRows : kDealTiles, partly));
   };
   for (int i = 0; i < kNumRowsTiles; ++i) take_tile(i, kRowsTiles[i]);
   for (int i = 0; i < kNumMoreTiles; ++i) take_tile(kFirstMoreTile + i, kMoreTiles[i]);

@@ -203,7 +203,7 @@ std::tuple<Tensor, Tensor, int64_t, OptTensor, OptTensor, OptTensor, bool> exper
     const OptTensor& b1_, const OptTensor& w0t, const OptTensor& w1t, bool tanh_gelu,
     const OptTensor& workspace_, const OptTensor& out_, const OptTensor& rows_per_expert,
     const OptTensor& x_rows, const OptTensor& fill, const OptTensor& token_slot, int64_t capacity,
-    bool plan_apart, bool f32_products) {
+    bool plan_apart, bool f32_products, bool full_rows) {
   const Tensor x = x_.contiguous();
   // float32 biases of a bfloat16 MLP are rounded by the call (which asks for both in one type)
   auto is_f32 = [&](const OptTensor& t) { return t.has_value() && t->scalar_type() == at::kFloat; };
@@ -256,7 +256,7 @@ std::tuple<Tensor, Tensor, int64_t, OptTensor, OptTensor, OptTensor, bool> exper
   p.x = ptr(x); p.w0 = ptr(w0); p.b0 = ptr(b0); p.w1 = ptr(w1); p.b1 = ptr(b1); p.w0t = ptr(w0t); p.w1t = ptr(w1t);
   p.out = ptr(out); p.dtype = dtype_code(x);
   p.gelu = (tanh_gelu ? VMOE_GELU_TANH : VMOE_GELU_ERF) + (f32_products ? VMOE_MLP_F32_PRODUCTS : 0) +
-           (f32_biases ? VMOE_MLP_F32_BIASES : 0);
+           (f32_biases ? VMOE_MLP_F32_BIASES : 0) + (full_rows ? VMOE_MLP_FULL_ROWS : 0);
   p.rows_per_expert = ptr_as<int32_t>(rows); p.x_rows = ptr_as<int32_t>(row_token);
   const size_t need = vmoe_expert_mlp_workspace_bytes(&p);
   Tensor workspace = workspace_.has_value() && workspace_->nbytes() >= need

@@ -347,7 +347,8 @@ def pack_expert_weights(w: torch.Tensor) -> torch.Tensor:
 def expert_mlp(x: torch.Tensor, w0, b0, w1, b1, w0t=None, w1t=None, approximate_gelu: bool = True,
                workspace: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None,
                rows_per_expert: Optional[torch.Tensor] = None,
-               x_rows: Optional[torch.Tensor] = None, compact=None, float32_products: bool = False):
+               x_rows: Optional[torch.Tensor] = None, compact=None, float32_products: bool = False,
+               full_rows: bool = False):
   """x (E,R,D) -> (E,R,D): gelu(x @ w0 + b0) @ w1 + b1 per expert; with rows_per_expert (E,)
   int32 only that many leading rows of every expert are computed.  With x_rows (E,R) int32,
   x is the (T,D) matrix of items and x_rows names the item of every row (gathered by the
@@ -359,6 +360,7 @@ def expert_mlp(x: torch.Tensor, w0, b0, w1, b1, w0t=None, w1t=None, approximate_
 
   ``float32_products``: float32 operands are multiplied on float32 matrix instructions instead of
   as sums of three bfloat16 values each (for outputs that are rounded to bfloat16 further on).
+  ``full_rows``: rows_per_expert are all R, which the choice between kernels may count on.
   The biases of a bfloat16 MLP may be float32: the call rounds them."""
   float32_products = float32_products and x.dtype == torch.float32
   if H._timing_sink is None or not any(map(H.timed, _MLP_CALLS)):
@@ -368,7 +370,7 @@ def expert_mlp(x: torch.Tensor, w0, b0, w1, b1, w0t=None, w1t=None, approximate_
     out, workspace, at, token_row, rows, row_token, planned = H.host().expert_mlp(
         H.raw_stream(), x, w0, b0, w1, b1, w0t, w1t, approximate_gelu, workspace, out,
         rows_per_expert, x_rows, fill, token_slot, capacity,
-        bool(os.environ.get("VMOE_PLAN_SEPARATE_LAUNCH")), float32_products)
+        bool(os.environ.get("VMOE_PLAN_SEPARATE_LAUNCH")), float32_products, full_rows)
     _note_status_words(workspace, at)
     if compact is None:
       return out
@@ -394,7 +396,7 @@ def expert_mlp(x: torch.Tensor, w0, b0, w1, b1, w0t=None, w1t=None, approximate_
   if x.dtype == torch.bfloat16:
     b0, b1 = (None if b is None else cast(b, x.dtype) for b in (b0, b1))
   p = _expert_mlp_params(x, w0, b0, w1, b1, w0t, w1t, approximate_gelu, out, rows_per_expert, x_rows)
-  p.gelu += H.MLP_F32_PRODUCTS * float32_products
+  p.gelu += H.MLP_F32_PRODUCTS * float32_products + H.MLP_FULL_ROWS * full_rows
   need = H.lib().vmoe_expert_mlp_workspace_bytes(H.ctypes.byref(p))
   if workspace is None or workspace.numel() * workspace.element_size() < need:
     workspace = torch.empty(need, dtype=torch.uint8, device=x.device)

@@ -142,6 +142,7 @@ class ExpertIndicesDispatcher(BaseDispatcher):
     self._weights_f32 = None                      # float32 copy of combine_weights, if on hand
     self.fill = None                              # (G, E) kept items per (group, expert), if known
     self._packed_maps = None                      # (token_row (G,S,K), rows_per_expert (E,))
+    self._full_rows = False                       # rows_per_expert are all G * capacity
     self._rounds = None                           # per-occurrence slot maps when slots are shared
     self._unread = None                           # (counters on their way to the host, event) of maps not yet checked
 
@@ -285,8 +286,12 @@ class ExpertIndicesDispatcher(BaseDispatcher):
     token_slot, _ = self._maps()
     return self.fill, token_slot, self.capacity
 
-  def set_packed_maps(self, maps) -> None:
-    self._packed_maps = tuple(maps)
+  def set_packed_maps(self, maps, full_rows: bool = False) -> None:
+    self._packed_maps, self._full_rows = tuple(maps), full_rows
+
+  def packed_rows_are_full(self) -> bool:
+    """Whether every packed row holds an item, as experts choice makes them."""
+    return self._full_rows
 
   def packed_rows(self):
     """-> (row_token (E, G * capacity) int32: the item (g * S + s) in every packed row,
@@ -434,8 +439,11 @@ class _SparseEinsumDispatcher(EinsumDispatcher):
   def pending_compaction(self):
     return self._inner.pending_compaction()
 
-  def set_packed_maps(self, maps) -> None:
-    self._inner.set_packed_maps(maps)
+  def set_packed_maps(self, maps, full_rows: bool = False) -> None:
+    self._inner.set_packed_maps(maps, full_rows)
+
+  def packed_rows_are_full(self) -> bool:
+    return self._inner.packed_rows_are_full()
 
   def combine_packed(self, data: Array) -> Array:
     return self._inner.combine_packed(data)
@@ -469,6 +477,10 @@ class Bfloat16Dispatcher(BaseDispatcher):
 
   def supports_packed(self) -> bool:
     fn = getattr(self.dispatcher, "supports_packed", None)
+    return bool(fn and fn())
+
+  def packed_rows_are_full(self) -> bool:
+    fn = getattr(self.dispatcher, "packed_rows_are_full", None)
     return bool(fn and fn())
 
   def dispatch_packed(self, data: Array):
@@ -674,7 +686,7 @@ def _get_top_items_per_expert_einsum_dispatcher(gates: Array, capacity: int, **d
   inner._weights_f32 = weights
   # Every slot holds an item, so the buffer is its own packed form: an expert that gathers its rows
   # (21 of 350 us of the B/16 layer on 64 images) needs no dispatched copy.
-  inner.set_packed_maps((token_slot, rows, slot_token.view(E, G * capacity)))
+  inner.set_packed_maps((token_slot, rows, slot_token.view(E, G * capacity)), full_rows=True)
   dispatcher = _SparseEinsumDispatcher(inner, gates.dtype, **dispatcher_kwargs)
   # Metrics useful for monitoring training (moe.py:681-692).
   metrics = {
@@ -735,6 +747,9 @@ def sparse_moe_spmd(target, variable_axes: Optional[Mapping[str, Any]] = None,
         gather = getattr(self.expert, "apply_experts_gathered", None)
         packed_rows = getattr(dispatcher, "packed_rows", None)
         x = inputs[0]
+        full = getattr(dispatcher, "packed_rows_are_full", None)
+        full = full is not None and full()
+        hint = lambda fn: {"full_rows": True} if full and getattr(fn, "takes_full_rows", False) else {}
         if (gather is not None and packed_rows is not None and x.ndim == 3
             and self.expert.can_gather(x)):
           # ... and fetches them from the items itself: no dispatched buffer at all.
@@ -746,11 +761,11 @@ def sparse_moe_spmd(target, variable_axes: Optional[Mapping[str, Any]] = None,
             dispatcher.set_packed_maps(maps)
           else:
             row_token, rows_per_expert = packed_rows()
-            outputs = gather(variables, x.reshape(-1, x.shape[-1]), row_token, rows_per_expert)
+            outputs = gather(variables, x.reshape(-1, x.shape[-1]), row_token, rows_per_expert, **hint(gather))
         else:
           dispatched, rows_per_expert = dispatcher.dispatch_packed(x)
-          outputs = self.expert.apply_experts(variables, dispatched,
-                                              rows_per_expert=rows_per_expert)
+          outputs = self.expert.apply_experts(variables, dispatched, rows_per_expert=rows_per_expert,
+                                              **hint(self.expert.apply_experts))
         return _tree_map(dispatcher.combine_packed, outputs)
       dispatched = [dispatcher.dispatch(x) for x in inputs]
       if hasattr(self.expert, "apply_experts"):

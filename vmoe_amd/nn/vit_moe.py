@@ -69,18 +69,18 @@ class MlpBlock(module.Module):
   supports_packed_rows = True
 
   def apply_experts(self, variables, inputs: Array, rows_per_expert: Optional[Array] = None,
-                    float32_products: bool = False) -> Array:
+                    float32_products: bool = False, full_rows: bool = False) -> Array:
     """inputs (E, R, D) with parameters stacked on axis 0 -> (E, R, D).  With
     rows_per_expert (E,) int32 only that many leading rows of each expert are
-    computed; the other rows of the result are not written.  ``float32_products`` as in
-    kernels.expert_mlp."""
+    computed; the other rows of the result are not written.  ``float32_products`` and
+    ``full_rows`` as in kernels.expert_mlp."""
     dtype = self.dtype or inputs.dtype
     module.require_no_grad("MlpBlock", inputs)
     return K.expert_mlp(K.cast(inputs, dtype), **self._weights(variables["params"], dtype),
                         approximate_gelu=self.approximate_gelu, rows_per_expert=rows_per_expert,
-                        float32_products=float32_products)
+                        float32_products=float32_products, full_rows=full_rows)
 
-  apply_experts.takes_float32_products = True
+  apply_experts.takes_float32_products = apply_experts.takes_full_rows = True
 
   def can_gather(self, items: Array) -> bool:
     """Whether apply_experts_gathered covers these items (dtype and width of the kernel)."""
@@ -89,15 +89,17 @@ class MlpBlock(module.Module):
             and K.expert_mlp_can_gather(dtype, items.shape[-1], items.numel() // items.shape[-1]))
 
   def apply_experts_gathered(self, variables, items: Array, row_token: Array,
-                             rows_per_expert: Array) -> Array:
+                             rows_per_expert: Array, full_rows: bool = False) -> Array:
     """items (T, D); row_token (E, R) int32 names the item in row r of expert e,
-    rows_per_expert (E,) how many rows each expert has -> (E, R, D).  The first product
+    rows_per_expert (E,) how many rows each expert has (``full_rows``: all R) -> (E, R, D).  The first product
     reads its rows straight from ``items``: the dispatched buffer is never built."""
     dtype = self.dtype or items.dtype
     module.require_no_grad("MlpBlock", items)
     return K.expert_mlp(K.cast(items, dtype), **self._weights(variables["params"], dtype),
                         approximate_gelu=self.approximate_gelu, rows_per_expert=rows_per_expert,
-                        x_rows=row_token)
+                        x_rows=row_token, full_rows=full_rows)
+
+  apply_experts_gathered.takes_full_rows = True
 
   def apply_experts_routed(self, variables, items: Array, fill: Array, token_slot: Array,
                            capacity: int):
