@@ -1404,6 +1404,28 @@ def test_expert_mlp_last_tiles_of_the_large_kernels(K, monkeypatch, rows, second
       assert bool((got[e, n:] == 7.0).all())
 
 
+@pytest.mark.parametrize("second", ["eight", "narrow"])
+@pytest.mark.parametrize("E", [100, 150])                   # (below and above two rounds of tiles per die: 500 and 750)
+def test_expert_mlp_short_last_tiles_of_long_launches(K, monkeypatch, E, second):
+  """Last tiles of 129 to 192 rows, whose idle waves take part in the product of a launch of few rounds and stay out of it in
+  a longer one: bit for bit what the smallest tile computes, and nothing written past the live rows."""
+  R, D, M = 161, 1280 if second == "eight" else 960, 256
+  rng = np.random.default_rng(E)
+  mk = lambda scale, *s: to_dev(O.cast(rng.standard_normal(s).astype(np.float32) * scale, O.BF16), O.BF16)
+  x, w0, w1 = mk(1, E, R, D), mk(D ** -0.5, E, D, M), mk(M ** -0.5, E, M, D)
+  b0, b1 = mk(0.1, E, M), mk(0.1, E, D)
+  counts = torch.from_numpy(rng.choice([0, 1, 128, 129, 160, 161], E).astype(np.int32)).to(dev())
+  out = []
+  for tiles, kernel in (("off", second), ("0", "")):
+    monkeypatch.setenv("VMOE_ROW_TILES", tiles)
+    monkeypatch.setenv("VMOE_SECOND_PRODUCT", kernel)
+    for live in (None, counts):
+      out.append(torch.full((E, R, D), 7.0, dtype=torch.bfloat16, device=dev()))
+      K.expert_mlp(x, w0, b0, w1, b1, out=out[-1], rows_per_expert=live)
+  assert torch.equal(out[0].view(torch.int16), out[2].view(torch.int16))
+  assert torch.equal(out[1].view(torch.int16), out[3].view(torch.int16))
+
+
 @pytest.mark.parametrize("E,R,D,M", [(5, 800, 832, 3328), (3, 1500, 512, 2048), (12, 896, 448, 1088), (21, 140, 704, 2816),
                                      (5, 8, 64, 136), (4, 2576, 96, 2048)])
 def test_expert_mlp_of_full_experts(K, E, R, D, M):

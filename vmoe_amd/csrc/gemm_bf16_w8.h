@@ -328,10 +328,13 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_w8_kernel(
       iteration(alive, nxt, 0, cur, (nk - 1) * BK, NotFirst{}, NotLast{});
       iteration(alive, nxt, BK, nxt, 0, NotFirst{}, Last{});
     };
-    // (In a batch's last tile the waves without live rows stay out of the way of the others: of 128 rows and fewer
-    // each SIMD has one wave at work, which halves the tile's MFMAs and fragment reads.  Experts choice, 32 experts x
-    // 800 rows, 3.1 tiles of rows each: 332 -> 327 us a layer.)
-    if (cur.row0 + wm * Cfg::TM >= cur.live) {
+    // (In a batch's last tile of 128 live rows and fewer the waves without live rows stay out of the way of the others:
+    // each SIMD has one wave at work at most, which halves the tile's MFMAs and fragment reads.  32 experts x 800 rows, 3.1
+    // tiles of rows each: 332 -> 327 us a layer; 6 x 108 x 2 240 x 864, this product alone: 29.8 -> 26.4.  Of 129 to 192
+    // rows two SIMDs have both of their waves at work and set the time, and with the others out of step it grows: 11 x 168 x
+    // 3 200 x 800 took 54.4 where it takes 48.6.  In launches of more than two rounds such a tile is one of many and
+    // its idle waves save power: 0.3 % of the headline layer.)
+    if (cur.row0 + wm * Cfg::TM >= cur.live && cur.live - cur.row0 <= (die_tiles > 2 * kCusPerXcd ? BM : BM / 2)) {
       k_tiles(std::false_type{});
       if (!has_next) break;
       materialize(nxt, cur);
