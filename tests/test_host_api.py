@@ -513,3 +513,29 @@ def test_experts_hear_that_every_packed_row_is_live(full, gathers, takes):
   for d in (dispatcher, wrapped):
     moe.sparse_moe_spmd(Experts)().apply({}, d, torch.zeros((2, 3, 8)))
   assert asked == [{"full_rows": True} if full and takes else {}] * 2
+
+
+@pytest.mark.parametrize("rows,D,M,pays", [
+    (1568, 768, 2304, True),                                    # either side of where multiples of 256 stop
+    (4521, 768, 2304, True), (4522, 768, 2304, False),
+    (40690, 256, 768, True), (40691, 256, 768, False),
+    (50176, 704, 2112, True), (50176, 1024, 1024, False),        # other widths do not
+    (2089, 1152, 1160, True), (2096, 1152, 1160, False),
+    (100, 1020, 768, False), (100, 768, 1020, False), (0, 768, 768, False),
+    (1 << 20, 960, 960, True), (1 << 21, 960, 960, False),       # byte offsets of 31 bits
+])
+def test_where_bfloat16_dense_layers_take_the_kernel(rows, D, M, pays):
+  assert kernels.dense_pays(rows, D, M, torch.bfloat16) == pays
+
+
+def test_kept_launch_plans_are_those_of_the_shapes_that_ask(monkeypatch):
+  """A thread keeps what it worked out for its last shapes: more of them, in any order, get their own."""
+  monkeypatch.delenv("VMOE_ROW_TILES", raising=False)
+  shapes = [(1, 1568, 768, 3072), (8, 412, 768, 3072), (32, 1600, 768, 3072), (5, 800, 832, 3328), (47, 140, 576, 2304),
+            (20, 1571, 640, 2560)]
+  monkeypatch.setenv("VMOE_SECOND_PRODUCT", "")           # (worked out anew on every call)
+  want = [_ragged_mlp_bytes(*s) for s in shapes]
+  monkeypatch.delenv("VMOE_SECOND_PRODUCT")
+  rng = np.random.default_rng(0)
+  for i in rng.integers(0, len(shapes), 200):
+    assert _ragged_mlp_bytes(*shapes[i]) == want[i]

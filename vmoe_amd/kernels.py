@@ -659,14 +659,23 @@ def add_layer_norm(residual: torch.Tensor, branch: Optional[torch.Tensor],
 
 
 def dense_pays(rows: int, D: int, M: int, dtype: torch.dtype) -> bool:
-  """Whether dense() is the faster one for x (rows, D) . w (D, M) beside the library's product.  bfloat16: up to
-  2.8e9 multiply-adds (1 568 x 768 x 2 304: 11.1 us either way, 1 568 x 768 x 768: 7.5 and 9.0, and 17 us less host
-  work; 3 136 x 1 024 x 3 072: 25.5 and 22.2), and over short rows (50 176 x 384 x 384: 28 and 42).  float32: from
-  1.3e9 on (3 136 x 768 x 768: 35 us and 48, 50 176: 306 and 510; 784 x 768 x 768: 16 and 13), where its error
-  against 64 bits is also the smaller one (2.9e-7 and 3.5e-7 at D = 768)."""
+  """Whether dense() is the faster one for x (rows, D) . w (D, M) beside the library's product.
+
+  bfloat16: the kernel's call takes 4 us of the host, the library's 18, so small models gain more than the kernels' times
+  say.  Those, kernel to library, over 1 200 shapes (D 192 .. 1 024 in steps of 64, M = D and 3 D, 49 .. 100 000 rows): 0.66 -
+  1.08 up to 2e9 multiply-adds at every width; beyond, 0.64 - 0.98 where D is 192 .. 704 and no multiple of 256, 0.85 - 1.13 at 832 ..
+  960, and at the multiples of 256, which the library knows best, 0.95 - 1.18 up to 1e10 and up to 1.37 above.  Models
+  of six blocks at 224 px, microseconds a pass on the library and here, by the multiply-adds of q, k and v: D = 768 2.8e9 885 and
+  755, 5.5e9 946 and 941, 8.3e9 1 162 and 1 147, 1.1e10 1 396 and 1 428; 1 024 4.9e9 913 and 906, 9.9e9 1 206 and 1 215, 1.5e10 1 523
+  and 1 588; 512 2.5e9 886 and 694, 4.9e9 926 and 905, 7.4e9 1 189 and 1 205; 640 2.3e10 2 606 and 2 443; 832 2.6e10 2 560 and 2 512.
+  Above 1 024 (1 088 .. 3 072) the kernels are 0.80 - 1.06 below 1e9 and 0.92 - 1.25 from there to 4e9.
+
+  float32: from 1.3e9 on (3 136 x 768 x 768: 35 us and 48, 50 176: 306 and 510; 784 x 768 x 768: 16 and 13), where its error
+  against 64 bits is also the smaller one (D = 192 .. 1 024: 1.0e-7 - 4.9e-7 and 2.3e-7 - 5.7e-7, on each of 120 shapes)."""
   work = rows * D * M
   if dtype == torch.bfloat16:
-    return D % 8 == 0 and M % 8 == 0 and 0 < work and (work <= 2.8e9 or D <= 384) and max(rows, M) * D < 1 << 30 and rows * M < 1 << 30
+    return (0 < work and (work <= 2.8e9 or (D <= 1024 and (work <= 8e9 or D % 256 != 0))) and D % 8 == 0 and M % 8 == 0
+            and max(rows, M) * D < 1 << 30 and rows * M < 1 << 30)
   return dtype == torch.float32 and D % 4 == 0 and M % 4 == 0 and work >= 1.3e9 and rows < 1 << 31
 
 
