@@ -748,8 +748,8 @@ def sparse_moe_spmd(target, variable_axes: Optional[Mapping[str, Any]] = None,
         packed_rows = getattr(dispatcher, "packed_rows", None)
         x = inputs[0]
         full = getattr(dispatcher, "packed_rows_are_full", None)
-        full = full is not None and full()
-        hint = lambda fn: {"full_rows": True} if full and getattr(fn, "takes_full_rows", False) else {}
+        hint = lambda fn: ({"full_rows": True} if full is not None and full() and getattr(fn, "takes_full_rows", False)
+                           else {})
         if (gather is not None and packed_rows is not None and x.ndim == 3
             and self.expert.can_gather(x)):
           # ... and fetches them from the items itself: no dispatched buffer at all.

@@ -228,19 +228,14 @@ def _add_layer_norm(residual: Array, branch: Optional[Array], p: Mapping[str, Ar
 
 
 def _affine(x: Array, w: Array, b: Array) -> Array:
-  """x (..., D) . w (D, M) + b in float32: the package's own product where it is the faster one."""
+  """x (..., D) . w (D, M) + b in float32: the package's own product where it is the faster one.  (The library
+  refuses other widths of x and spreads biases that are not one row of the output.)"""
   (D, M), rows = w.shape, x.shape[:-1].numel()
-  if (_fits_dense(x, D, M, b) and x.dtype == w.dtype == b.dtype and w.is_contiguous() and b.is_contiguous()
+  if (x.shape[-1] == D and b.shape == (M,) and x.dtype == w.dtype == b.dtype and w.is_contiguous() and b.is_contiguous()
       and K.dense_pays(rows, D, M, x.dtype) and module.is_plain(x, w, b)
       and K.dense_takes(x, w)):
     return K.dense(x, w, b)
   return torch.addmm(b, x.reshape(rows, x.shape[-1]), w).view(*x.shape[:-1], M)
-
-
-def _fits_dense(x: Array, D: int, M: int, b: Array) -> bool:
-  """Whether x is (..., D) and b (M,), what a weight of D x M goes with: the library refuses other widths and
-  spreads other biases, over rows or columns, and K.dense does neither."""
-  return x.shape[-1] == D and b.shape == (M,)
 
 
 class IdentityLayer(module.Module):
@@ -325,8 +320,8 @@ class MultiHeadDotProductAttention(module.Module):
     """x . w + b for a weight of _proj_weights: the package's own product where it is the faster one."""
     f32 = w.dtype == torch.float32
     D, M = w.shape if f32 else reversed(w.shape)
-    if (_fits_dense(x, D, M, b) and K.dense_pays(x.shape[:-1].numel(), D, M, w.dtype)
-        and module.is_plain(x, w, b) and K.dense_takes(x, w)):
+    if (b.numel() == M and K.dense_pays(x.numel() // D, D, M, w.dtype) and module.is_plain(x, w, b)
+        and K.dense_takes(x, w)):
       return K.dense(x, w, b)
     return torch.nn.functional.linear(x, w.t() if f32 else w, b)
 
@@ -340,21 +335,20 @@ class MultiHeadDotProductAttention(module.Module):
     Sk = inputs_kv.shape[1]
     hd = p["query"]["kernel"].shape[-1]
     xq = inputs_q.to(dtype)
-    # Which of the products are the package's own: in float32 the weight's layout follows it.
-    f32 = dtype == torch.float32
+    # In float32 a weight's layout follows the product that reads it: whether it is the package's own.
+    f32, library = dtype == torch.float32, torch.nn.functional.linear
     own = lambda rows, D, M: (f32 and K.dense_pays(rows, D, M, dtype)
                               and module.is_plain(xq, inputs_kv, *self._leaves(p)))
-    linear = lambda x, w, b, own: self._project(x, w, b) if own or not f32 else torch.nn.functional.linear(x, w, b)
-    own_out = own(B * Sq, H * hd, p["out"]["kernel"].shape[-1])
+    own_out = f32 and own(B * Sq, H * hd, p["out"]["kernel"].shape[-1])
     if inputs_kv is inputs_q:
-      own_in = own(B * Sq, D, 3 * H * hd)
+      own_in = f32 and own(B * Sq, D, 3 * H * hd)
       w, b, wo, bo = self._proj_weights(p, (("query", "key", "value"),), dtype, (own_in, own_out))
-      q, k, v = linear(xq, w, b, own_in).view(B, Sq, 3, H, hd).unbind(2)
+      q, k, v = (library if f32 and not own_in else self._project)(xq, w, b).view(B, Sq, 3, H, hd).unbind(2)
     else:
       own_q, own_kv = own(B * Sq, D, H * hd), own(B * Sk, inputs_kv.shape[-1], 2 * H * hd)
       wq, bq, wkv, bkv, wo, bo = self._proj_weights(p, (("query",), ("key", "value")), dtype, (own_q, own_kv, own_out))
-      q = linear(xq, wq, bq, own_q).view(B, Sq, H, hd)
-      kv = linear(inputs_kv.to(dtype), wkv, bkv, own_kv).view(B, Sk, 2, H, hd)
+      q = (library if f32 and not own_q else self._project)(xq, wq, bq).view(B, Sq, H, hd)
+      kv = (library if f32 and not own_kv else self._project)(inputs_kv.to(dtype), wkv, bkv).view(B, Sk, 2, H, hd)
       k, v = kv[:, :, 0], kv[:, :, 1]
     if self.normalize_qk:
       q = _layer_norm(q, p["query_ln"], dtype)
@@ -365,7 +359,8 @@ class MultiHeadDotProductAttention(module.Module):
       ctx = torch.nn.functional.scaled_dot_product_attention(
           q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2))     # (B, H, Sq, hd)
       ctx = ctx.transpose(1, 2).reshape(B, Sq, H * hd)
-    return linear(ctx, wo, bo, own_out)
+    # (a bias of more axes is spread over rows by the library)
+    return (library if bo.dim() != 1 or (f32 and not own_out) else self._project)(ctx, wo, bo)
 
 
 class MapHead(module.Module):
