@@ -541,27 +541,33 @@ static int check_mlp(const VmoeExpertMlpParams* p) {
 }
 
 // A layer's call asks three or four times (workspace, status words, compaction, launch), and the estimates behind an
-// answer take 1 - 3 us of the host; a thread keeps its last one.  (Nothing in it depends on more than the sizes; with a
-// switch in the environment it is worked out every time.)
+// answer take 1 - 3 us of the host; a thread keeps those of its last four shapes (a model's dense and sparse MLPs take
+// turns: with one shape kept, every call of a model of six blocks worked its own out).  (Nothing in an answer depends on
+// more than the sizes; with a switch in the environment it is worked out every time.)
 static MlpPlans plans_of(const VmoeExpertMlpParams* p) {
   if (p->dtype != VMOE_BF16) return MlpPlans{};
   struct Key {
-    int E, R, D, M;
-    bool ragged, full;
+    int E, R, D, M, ragged, full;
     long long items;
+    bool operator==(const Key& o) const {
+      return E == o.E && R == o.R && D == o.D && M == o.M && ragged == o.ragged && full == o.full && items == o.items;
+    }
   };
   const Key key = {p->E, p->R, p->D, p->M, p->rows_per_expert != nullptr, (p->gelu & VMOE_MLP_FULL_ROWS) != 0,
                    p->x_rows != nullptr ? p->num_items : 0};
   auto plans = [&] { return mlp_plans(key.E, key.R, key.D, key.M, key.ragged, key.full, key.items); };
   if (getenv("VMOE_ROW_TILES") != nullptr || getenv("VMOE_SECOND_PRODUCT") != nullptr) return plans();
-  thread_local Key last_key = {};
-  thread_local MlpPlans last;
-  if (last_key.E != key.E || last_key.R != key.R || last_key.D != key.D || last_key.M != key.M ||
-      last_key.ragged != key.ragged || last_key.full != key.full || last_key.items != key.items) {
-    last = plans();
-    last_key = key;
-  }
-  return last;
+  constexpr int kKept = 4;
+  thread_local Key keys[kKept] = {};      // (E 0: none)
+  thread_local MlpPlans kept[kKept];
+  thread_local int next = 0;
+  for (int i = 0; i < kKept; ++i)
+    if (keys[i] == key) return kept[i];
+  const int at = next;
+  next = (next + 1) % kKept;
+  kept[at] = plans();
+  keys[at] = key;
+  return kept[at];
 }
 
 static size_t workspace_bytes(const VmoeExpertMlpParams* p, const MlpPlans& m) {
