@@ -142,7 +142,7 @@ class ExpertIndicesDispatcher(BaseDispatcher):
     self._weights_f32 = None                      # float32 copy of combine_weights, if on hand
     self.fill = None                              # (G, E) kept items per (group, expert), if known
     self._packed_maps = None                      # (token_row (G,S,K), rows_per_expert (E,))
-    self._full_rows = False                       # rows_per_expert are all G * capacity
+    self.full_rows = False                        # every packed row holds an item (experts choice)
     self._rounds = None                           # per-occurrence slot maps when slots are shared
     self._unread = None                           # (counters on their way to the host, event) of maps not yet checked
 
@@ -287,11 +287,7 @@ class ExpertIndicesDispatcher(BaseDispatcher):
     return self.fill, token_slot, self.capacity
 
   def set_packed_maps(self, maps, full_rows: bool = False) -> None:
-    self._packed_maps, self._full_rows = tuple(maps), full_rows
-
-  def packed_rows_are_full(self) -> bool:
-    """Whether every packed row holds an item, as experts choice makes them."""
-    return self._full_rows
+    self._packed_maps, self.full_rows = tuple(maps), full_rows
 
   def packed_rows(self):
     """-> (row_token (E, G * capacity) int32: the item (g * S + s) in every packed row,
@@ -442,8 +438,9 @@ class _SparseEinsumDispatcher(EinsumDispatcher):
   def set_packed_maps(self, maps, full_rows: bool = False) -> None:
     self._inner.set_packed_maps(maps, full_rows)
 
-  def packed_rows_are_full(self) -> bool:
-    return self._inner.packed_rows_are_full()
+  @property
+  def full_rows(self) -> bool:
+    return self._inner.full_rows
 
   def combine_packed(self, data: Array) -> Array:
     return self._inner.combine_packed(data)
@@ -479,9 +476,9 @@ class Bfloat16Dispatcher(BaseDispatcher):
     fn = getattr(self.dispatcher, "supports_packed", None)
     return bool(fn and fn())
 
-  def packed_rows_are_full(self) -> bool:
-    fn = getattr(self.dispatcher, "packed_rows_are_full", None)
-    return bool(fn and fn())
+  @property
+  def full_rows(self) -> bool:
+    return getattr(self.dispatcher, "full_rows", False)
 
   def dispatch_packed(self, data: Array):
     dtype = data.dtype
@@ -747,9 +744,8 @@ def sparse_moe_spmd(target, variable_axes: Optional[Mapping[str, Any]] = None,
         gather = getattr(self.expert, "apply_experts_gathered", None)
         packed_rows = getattr(dispatcher, "packed_rows", None)
         x = inputs[0]
-        full = getattr(dispatcher, "packed_rows_are_full", None)
-        hint = lambda fn: ({"full_rows": True} if full is not None and full() and getattr(fn, "takes_full_rows", False)
-                           else {})
+        full = getattr(dispatcher, "full_rows", False)
+        hint = lambda fn: {"full_rows": True} if full and getattr(fn, "takes_full_rows", False) else {}
         if (gather is not None and packed_rows is not None and x.ndim == 3
             and self.expert.can_gather(x)):
           # ... and fetches them from the items itself: no dispatched buffer at all.
