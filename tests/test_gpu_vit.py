@@ -409,6 +409,45 @@ def test_dense_against_64_bits(rows, D, M, dtype):
     assert bool(((got - want).abs() <= bound).all())
 
 
+def _dense_of_batches(K, x, w, b):
+  """vmoe_dense on E matrices at once, through the C entry point."""
+  from vmoe_amd import _hip as H
+  f32 = x.dtype == torch.float32
+  E, R, D = x.shape
+  out = torch.full((E, R, w.shape[2 if f32 else 1]), 7.0, dtype=x.dtype, device=x.device)
+  p = H.ExpertMlpParams(x=H.ptr(x), b0=H.ptr(b), out=H.ptr(out), E=E, R=R, D=D, M=out.shape[2], dtype=H.dtype_code(x.dtype))
+  setattr(p, "w0" if f32 else "w0t", H.ptr(w))
+  H.call("vmoe_dense", p)
+  return out
+
+
+@pytest.mark.parametrize("tile", [("f32", i) for i in range(9)] + [("bf16", i) for i in (0, 1, 2, 3, 4, 5, 6, 7, 13, 14, 15, 16)])
+@pytest.mark.parametrize("rows,D,M", [(1, 8, 8), (67, 136, 264), (257, 328, 520)])
+def test_dense_on_every_tile(monkeypatch, tile, rows, D, M):
+  """Each tile that vmoe_dense may take, at rows, k and columns that end inside it, with a bias and without: one rounding of
+  the 64-bit result as above; three matrices at once are three calls bit for bit; bfloat16 tiles agree bit for bit."""
+  from vmoe_amd import kernels as K
+  kind, index = tile
+  dtype = torch.float32 if kind == "f32" else torch.bfloat16
+  monkeypatch.setenv("VMOE_F32_GEMM" if kind == "f32" else "VMOE_ROW_TILES", f"tile{index}" if kind == "f32" else str(index))
+  gen = torch.Generator(device=dev()).manual_seed(rows)
+  mk = lambda *s: torch.randn(s, generator=gen, device=dev()).to(dtype)
+  x, w, b = mk(3, rows, D), mk(3, D, M) * D ** -0.5, mk(3, M)
+  layout = w if kind == "f32" else w.transpose(1, 2).contiguous()
+  for bias in (b, None):
+    want = x.double() @ w.double() + (0 if bias is None else bias.double()[:, None])
+    got = _dense_of_batches(K, x, layout, bias)
+    bound = ((x.double().abs() @ w.double().abs() + 1) * D ** 0.5 * 2.0 ** -23
+             + (want.abs() * 2.0 ** -8 if kind == "bf16" else 0))
+    assert bool(((got.double() - want).abs() <= bound).all())
+    for e in range(3):
+      assert torch.equal(got[e], K.dense(x[e], layout[e], None if bias is None else bias[e]))
+    if kind == "bf16" and index != 0:
+      monkeypatch.setenv("VMOE_ROW_TILES", "0")
+      assert torch.equal(got, _dense_of_batches(K, x, layout, bias))
+      monkeypatch.setenv("VMOE_ROW_TILES", str(index))
+
+
 def test_dense_stands_aside_where_torch_has_to_see_the_product(vit_moe):
   """Gradients, functorch transforms and autocast take the library's product."""
   x = torch.randn(1301, 1000, device=dev())

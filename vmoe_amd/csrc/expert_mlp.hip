@@ -790,13 +790,22 @@ extern "C" int vmoe_dense(const VmoeExpertMlpParams* p, vmoe_stream_t stream_) {
   if (p->D % step != 0 || p->M % step != 0 || !aligned16(p->x) || !aligned16(p->out)) return VMOE_E_ALIGN;
   if ((int64_t)p->E * p->R >= INT32_MAX) return VMOE_E_OVERFLOW;
   hipStream_t stream = as_stream(stream_);
-  if (p->dtype == VMOE_F32)
-    return launch_gemm_f32_split<kEpiBias>(best_split_tile(p->E, p->R, p->M, p->D), (const float*)p->x, (const float*)p->w0,
-                                           (const float*)p->b0, (float*)p->out, p->E, p->R, p->M, p->D, stream, nullptr,
-                                           nullptr, 0);
+  // (the switches of the MLP's products name tiles here too: VMOE_F32_GEMM=tile<index>, VMOE_ROW_TILES=<index> but of kStreamTiles)
+  if (p->dtype == VMOE_F32) {
+    const char* const which = getenv("VMOE_F32_GEMM");
+    const int split = which != nullptr && strncmp(which, "tile", 4) == 0 ? atoi(which + 4)
+                                                                         : best_split_tile(p->E, p->R, p->M, p->D);
+    return launch_gemm_f32_split<kEpiBias>(split, (const float*)p->x, (const float*)p->w0, (const float*)p->b0,
+                                           (float*)p->out, p->E, p->R, p->M, p->D, stream, nullptr, nullptr, 0);
+  }
   if (!aligned16(p->w0t)) return VMOE_E_ALIGN;
   if (!rows_gemm_ok(p->R, p->M, p->D, 0)) return VMOE_E_UNSUPPORTED;
-  const int tile = best_tile(p->E, p->R, p->M, p->D, 0, false, false, false, 1e30, false);
+  int tile = best_tile(p->E, p->R, p->M, p->D, 0, false, false, false, 1e30, false);
+  if (const char* const row_tiles = getenv("VMOE_ROW_TILES"); row_tiles != nullptr && strcmp(row_tiles, "off") != 0) {
+    const int forced = atoi(row_tiles);
+    const bool mid = is_mid_tile(forced);
+    if (mid ? mid_gemm_ok(p->E, p->R, p->M, p->D, 0) : forced >= 0 && forced < kNumRowsTiles) tile = forced;
+  }
   return launch_gemm_bf16_rows<kEpiBiasOnce>(tile, (const bf16_t*)p->x, (const bf16_t*)p->w0t, (const bf16_t*)p->b0,
                                              (bf16_t*)p->out, p->E, p->R, p->M, p->D, stream, nullptr, nullptr, nullptr, 0,
                                              PlanRef{nullptr, 0, 0}, nullptr, 0, nullptr);
