@@ -1228,6 +1228,58 @@ def test_native_gradients_are_those_of_the_python_functions(moe, monkeypatch, da
     assert a.dtype == b.dtype and torch.equal(a, b)
 
 
+def test_native_gradients_of_a_pass_on_another_stream(moe):
+  """A forward pass on a side stream, its backward pass asked for from the default one: the nodes run on the stream
+  that recorded them, as the Python ones do, with tensors that were made there."""
+  rng = np.random.default_rng(5)
+  G, S, E, k, D = 4, 512, 8, 2, 256
+  C = S // 2
+  gates = torch.softmax(torch.from_numpy(rng.standard_normal((G, S, E)).astype(np.float32)).to(dev()), -1)
+  routed = moe.get_top_experts_per_item_dispatcher(gates, "indices", num_selected_experts=k, capacity=C, batch_priority=True)
+  indices, weights = routed.indices, routed.combine_weights.float()
+  base = torch.randn(G, S, D, device=dev()).to(torch.bfloat16)
+  grad = torch.randn(G, S, D, device=dev()).to(torch.bfloat16)
+
+  def leaves():
+    return base.clone().requires_grad_(), weights.clone().requires_grad_()
+
+  def forward(x, w):
+    d = moe.ExpertIndicesDispatcher(indices, w, E, C)
+    return d.combine(torch.tanh(d.dispatch(x)))
+
+  x, w = leaves()
+  want = torch.autograd.grad(forward(x, w), (x, w), grad)
+  side = torch.cuda.Stream()
+  for _ in range(3):
+    x, w = leaves()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+      busy = torch.randn(2048, 2048, device=dev())
+      for _ in range(20):                                   # (work in front of the pass: it is late on its stream)
+        busy = torch.tanh(busy @ busy)
+      out = forward(x, w)
+    torch.cuda.current_stream().wait_stream(side)
+    for a, b in zip(torch.autograd.grad(out, (x, w), grad), want):
+      assert torch.equal(a, b)
+
+
+def test_recorded_dispatch_and_combine_under_functorch(moe):
+  """Transforms see the Python functions, which functorch refuses with its own error, and never the native nodes."""
+  from vmoe_amd.nn import module
+  indices = torch.tensor([[[[0, 0]], [[1, 0]]]], dtype=torch.int32, device=dev())
+  x = torch.randn(1, 2, 8, device=dev())
+  d = moe.ExpertIndicesDispatcher(indices, torch.ones(1, 2, 1, device=dev()), 2, 2)
+  d.dispatch(x)
+  assert module.is_plain_but_for_gradients(x.requires_grad_())
+
+  def total(t):
+    assert not module.is_plain_but_for_gradients(t)
+    return d.combine(d.dispatch(t)).sum()
+
+  with pytest.raises(RuntimeError):
+    torch.func.grad(total)(x.detach())
+
+
 def test_dispatcher_checks_new_maps_behind_the_dispatch(moe):
   """Indices are checked after the dispatch has been issued: negative ones raise in every call, shared slots are
   added up in the first."""
