@@ -1301,10 +1301,10 @@ def test_expert_mlp_rows_per_expert(K, dtype, E):
 
 
 @pytest.mark.parametrize("E,R,D,M", [
-    (5, 65, 1024, 512),      # one row past a 64-row tile; 32 x 32 and 32 x 64 tiles
-    (24, 130, 384, 512),     # 32 x 128 and 64 x 64 tiles
-    (16, 257, 320, 640),     # 128 x 64 tiles, one row past the second; columns end inside a tile
-    (12, 400, 512, 768),     # 64 x 128 and 128 x 128 tiles
+    (5, 65, 1024, 512),      # one row past a 64-row tile
+    (24, 130, 384, 512),     # two rows past a 128-row tile, as many experts as make three rounds of the dies
+    (16, 257, 320, 640),     # one row past two 128-row tiles; columns end inside tiles of 128 and 192
+    (12, 400, 512, 768),     # rows that end inside tiles of every height
     (8, 52, 96, 3072),       # long k over few rows, k not a multiple of 64 in the first product
     (3, 33, 136, 264),       # k that ends inside a 32-wide step
     (70, 3, 64, 200),        # more experts than rows, one short row tile each
@@ -1312,8 +1312,8 @@ def test_expert_mlp_rows_per_expert(K, dtype, E):
     (5, 2, 40, 72),          # and rows shorter than that half
 ])
 def test_expert_mlp_small_tiles(K, E, R, D, M):
-  """bfloat16 products over few rows per expert (the small tiles, chosen by size) against a float32
-  restatement with the same rounding points; ragged rows bit for bit against the dense call,
+  """bfloat16 products over few rows per expert (on the tiles that the choice by size takes; the tests below name
+  them) against a float32 restatement with the same rounding points; ragged rows bit for bit against the dense call,
   nothing written past a count, and rows gathered from the items bit for bit as well."""
   rng = np.random.default_rng(E * 1000 + R)
   bf = torch.bfloat16
@@ -1346,8 +1346,9 @@ def test_expert_mlp_small_tiles(K, E, R, D, M):
 
 @pytest.mark.parametrize("tile", range(8))
 def test_expert_mlp_every_small_tile(K, monkeypatch, tile):
-  """Each tile of the small-tile kernel (VMOE_ROW_TILES names one for both products) through the
-  checks above, at a shape whose row, column and k tiles all end inside and one of a row."""
+  """Each tile of kRowsTiles (0, 1, 2 and 4 are gemm_bf16_rows_kernel's, the others gemm_bf16_mid_kernel's;
+  VMOE_ROW_TILES names one for both products) through the checks above, at a shape whose row, column and k tiles
+  all end inside and one of a row."""
   monkeypatch.setenv("VMOE_ROW_TILES", str(tile))
   test_expert_mlp_small_tiles(K, 3, 131, 136, 264)
   test_expert_mlp_small_tiles(K, 9, 1, 192, 72)
