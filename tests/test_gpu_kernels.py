@@ -1377,24 +1377,6 @@ def test_expert_mlp_medium_tiles(K, monkeypatch, tile):
         assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
-@pytest.mark.parametrize("tile", [5, 7, 13, 16])
-@pytest.mark.parametrize("E", [24, 37])                     # (pairs per die that fill chunks, and that end inside one)
-def test_expert_mlp_medium_tiles_in_chunks_of_pairs(K, monkeypatch, tile, E):
-  """Without a launch plan a die takes its (expert, column tile) pairs in chunks, row tile by row tile: bit for bit what
-  the smallest tile computes, and nothing written past the live rows."""
-  R, D, M = 300, 704, 1024
-  rng = np.random.default_rng(E)
-  mk = lambda scale, *s: to_dev(O.cast(rng.standard_normal(s).astype(np.float32) * scale, O.BF16), O.BF16)
-  x, w0, w1 = mk(1, E, R, D), mk(D ** -0.5, E, D, M), mk(M ** -0.5, E, M, D)
-  b0, b1 = mk(0.1, E, M), mk(0.1, E, D)
-  counts = torch.from_numpy(rng.choice([0, 1, 128, 129, 257, 300], E).astype(np.int32)).to(dev())
-  got, want = (torch.full((E, R, D), 7.0, dtype=torch.bfloat16, device=dev()) for _ in range(2))
-  for out, t in ((got, tile), (want, 0)):
-    monkeypatch.setenv("VMOE_ROW_TILES", str(t))
-    K.expert_mlp(x, w0, b0, w1, b1, out=out, rows_per_expert=counts)
-  assert torch.equal(got.view(torch.int16), want.view(torch.int16))
-
-
 @pytest.mark.parametrize("second", ["eight", "narrow"])
 @pytest.mark.parametrize("rows", [1, 16, 33, 63, 64, 65, 96, 97, 127, 128, 129, 161, 193, 255, 256, 257, 449])
 def test_expert_mlp_last_tiles_of_the_large_kernels(K, monkeypatch, rows, second):

@@ -10,8 +10,8 @@
 //
 // Operands go global memory -> LDS by DMA, 8 rows x 128 bytes per request, into a ring of S stages of 64 KT k,
 // XOR-swizzled as in gemm_bf16_rows.h.  The output leaves straight from registers (v_permlane16_swap, as in
-// gemm_bf16_stream.h).  Tiles are dealt to the dies as evenly as they come: dense launches as eight
-// runs of one list, ragged ones from a launch plan (whole row tiles) or, where they have none, (batch, column tile)
+// gemm_bf16_stream.h).  Tiles are dealt to the dies evenly, whatever their number: dense launches as eight
+// runs of one list, ragged ones from a launch plan or, over less than two row tiles per die, (batch, column tile)
 // pairs round the dies.  Sums run over k in the order of the other bfloat16 kernels: same bits.
 #ifndef VMOE_GEMM_BF16_MID_H_
 #define VMOE_GEMM_BF16_MID_H_
@@ -47,15 +47,7 @@ inline bool mid_gemm_ok(int batch, int R, int N, int Kd, long long items) {
 
 // `plan_ref`: the launch's own plan, or none.  `guard`: the plan of the other product of the call, where that one
 // has a plan: a launch whose plan was not written for this geometry runs nothing, and neither does this one.
-// per_die: tiles of a die (dense launches without a plan); 0: pairs go round the dies.  A die's pairs then come in
-// chunks of kPairChunk, the first row tiles of a chunk's pairs ahead of their second ones: a die hands workgroups to its
-// shader engines in turn, so that with the row tiles of a pair side by side and every second one empty all of the work
-// lands on half of its CUs.  Whole layers, row tiles side by side and in chunks: 22 experts x 136 rows x 1 024 x 4 096
-// 161.0 -> 150.6 us, 25 x 156 x 832 x 1 792 (59 % filled) 92.3 -> 88.2; of 223 random ones 11 are 3 to 9 % faster, none
-// more than 2.1 % slower, and the mean falls by 0.1 %.  11 x 148 x 896 x 3 584, half filled, gains nothing (92.8, 91.4) and
-// would take 81.9 with a chunk as large as a die's places; that one is up to 3.5 % slower for layers that are full.
-constexpr int kPairChunk = 8;
-
+// per_die: tiles of a die (dense launches without a plan); 0: pairs go round the dies.
 template <typename Cfg, int EPI>
 __global__ __launch_bounds__(Cfg::kThreads, Cfg::kBlocksPerCu * Cfg::kWaves / 4) void gemm_bf16_mid_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ Bt, const bf16_t* __restrict__ bias,
@@ -90,10 +82,8 @@ __global__ __launch_bounds__(Cfg::kThreads, Cfg::kBlocksPerCu * Cfg::kWaves / 4)
       pair = tile / tiles_m;
       tile_m = tile - pair * tiles_m;
     } else {
-      const int die_pairs = (batch * tiles_n + kNumXcd - 1) / kNumXcd, first = idx / (kPairChunk * tiles_m) * kPairChunk;
-      const int in_chunk = idx - first * tiles_m, here = min(kPairChunk, die_pairs - first);
-      tile_m = in_chunk / here;
-      pair = (first + in_chunk - tile_m * here) * kNumXcd + xcd;
+      pair = idx / tiles_m * kNumXcd + xcd;
+      tile_m = idx % tiles_m;
     }
     if (pair >= batch * tiles_n) return;
     b = pair / tiles_n;
