@@ -668,7 +668,10 @@ static int run_expert_mlp(const VmoeExpertMlpParams* p, vmoe_stream_t stream_, b
   // A plan beside the row compaction is there before the rows are; here it is 5.4 us in front of the first product.
   // Tiles that do without one go without it where eight (expert, column tile) pairs per die and more fall
   // evenly enough.  A layer, with the plan and without: 36 experts x 12 rows x 640 x 2 496 95.8 -> 87.3 us, 47 x 140 x 576 x
-  // 2 304 151.8 -> 143.3, 27 x 216 x 704 x 2 816, unbalanced, 115.4 -> 109.7; none of 23 random ones slower.
+  // 2 304 151.8 -> 143.3, 27 x 216 x 704 x 2 816, unbalanced, 115.4 -> 109.7; none of 23 random ones slower than with the plan.
+  // Without it, experts that fill the first of two row tiles only leave every second workgroup of a die empty: both
+  // products of 46 x 132 rows (110 live) x 960 x 3 136 take 185 us, and 160 with the first row tiles of eight pairs ahead of
+  // the second ones, an order that costs full experts up to 10 % of a product.
   unsigned plan_blocks = (unsigned)w.plan_blocks;
   const auto enough_pairs = [&](int tiles_n, int tile) { return !is_mid_tile(tile) || (long long)p->E * tiles_n >= 8 * kNumXcd; };
   if (!planned_already && m.up_rows >= 0 && m.down_rows >= 0 && enough_pairs(m.up.tiles_n, m.up_rows) &&

@@ -10,9 +10,9 @@
 //
 // Operands go global memory -> LDS by DMA, 8 rows x 128 bytes per request, into a ring of S stages of 64 KT k,
 // XOR-swizzled as in gemm_bf16_rows.h.  The output leaves straight from registers (v_permlane16_swap, as in
-// gemm_bf16_stream.h).  Tiles are dealt to the dies evenly, whatever their number: dense launches as eight
-// runs of one list, ragged ones from a launch plan or, over less than two row tiles per die, (batch, column tile)
-// pairs round the dies.  Sums run over k in the order of the other bfloat16 kernels: same bits.
+// gemm_bf16_stream.h).  Tiles are dealt to the dies: dense launches as eight runs of one list, which come out even;
+// ragged ones from a launch plan (whole row tiles to a die) or, over less than two row tiles per die or many (batch,
+// column tile) pairs, those pairs round the dies.  Sums run over k in the order of the other bfloat16 kernels: same bits.
 #ifndef VMOE_GEMM_BF16_MID_H_
 #define VMOE_GEMM_BF16_MID_H_
 #include "gemm_bf16.h"

@@ -671,7 +671,7 @@ def dense_pays(rows: int, D: int, M: int, dtype: torch.dtype) -> bool:
   Above 1 024 (1 088 .. 3 072) the kernels are 0.80 - 1.06 below 1e9 and 0.92 - 1.25 from there to 4e9.
 
   float32: from 1.3e9 on (3 136 x 768 x 768: 35 us and 48, 50 176: 306 and 510; 784 x 768 x 768: 16 and 13), where its error
-  against 64 bits is also the smaller one (D = 192 .. 1 024: 1.0e-7 - 4.9e-7 and 2.3e-7 - 5.7e-7, on each of 120 shapes)."""
+  against 64 bits is also the smaller one (D = 192 .. 1 024: 1.0e-7 - 4.9e-7 and 2.3e-7 - 5.7e-7, on each of 125 shapes)."""
   work = rows * D * M
   if dtype == torch.bfloat16:
     return (0 < work and (work <= 2.8e9 or (D <= 1024 and (work <= 8e9 or D % 256 != 0))) and D % 8 == 0 and M % 8 == 0
